@@ -43,27 +43,27 @@ def listed():
                     spread=spread, new=new, chunk=chunk)
     return [
         # a test run of three short requests on a model of two layers, in 32 bits: launches and host time
-        case("tiny model, 32 bits", "llama", "tiny-a", 2, 3, 8, 8, dtype="float32", spread=0.4),
+        case("tiny model in 32 bits", "llama", "tiny-a", 2, 3, 8, 8, dtype="float32", spread=0.4),
         # one user chats: single rows
-        case("chat, one user", "llama", "tinyllama-1.1b", 22, 1, 512, 128),
+        case("chat with one user", "llama", "tinyllama-1.1b", 22, 1, 512, 128),
         # the headline workload of bench.py: eight requests decode together
-        case("decode, eight requests", "llama", "tinyllama-1.1b", 22, 8, 512, 128),
+        case("decode eight requests", "llama", "tinyllama-1.1b", 22, 8, 512, 128),
         # an offline batch: 64 prompts of 512 tokens at once, then 64 rows a step
         case("offline batch of 64", "llama", "tinyllama-1.1b", 22, 64, 512, 64),
         # a document is read and one token comes back (a classification, or the wait for the first token)
         case("one prompt of 2048", "llama", "tinyllama-1.1b", 22, 1, 2048, 1),
         # serving: ragged prompts enter in portions beside requests that decode, which end one after the other
-        case("served, 24 ragged requests", "llama", "tinyllama-1.1b", 22, 24, 403, 64, spread=0.8, chunk=512),
+        case("served 24 ragged requests", "llama", "tinyllama-1.1b", 22, 24, 403, 64, spread=0.8, chunk=512),
         # the 32-bit path that answers are checked against
         case("checked in 32 bits", "llama", "tinyllama-1.1b", 22, 2, 301, 16, dtype="float32", spread=0.3),
         # a larger model with longer contexts of all lengths
-        case("8B, eight long contexts", "llama", "llama-3-8b", 32, 8, 1201, 32, spread=0.3),
+        case("8B eight long contexts", "llama", "llama-3-8b", 32, 8, 1201, 32, spread=0.3),
         # the Kasuvik decoder: a prompt, and eight requests that decode
-        case("Kasuvik, one prompt of 2048", "kasuvik", 2048, 4, 1, 2048, 1),
-        case("Kasuvik, eight requests", "kasuvik", 2048, 4, 8, 509, 64),
+        case("Kasuvik one prompt of 2048", "kasuvik", 2048, 4, 1, 2048, 1),
+        case("Kasuvik eight requests", "kasuvik", 2048, 4, 8, 509, 64),
         # the Fisesun decoder (experts): a prompt, and eight requests that decode
-        case("Fisesun, one prompt of 2048", "fisesun", 2048, 4, 1, 2048, 1),
-        case("Fisesun, eight requests", "fisesun", 2048, 4, 8, 509, 64),
+        case("Fisesun one prompt of 2048", "fisesun", 2048, 4, 1, 2048, 1),
+        case("Fisesun eight requests", "fisesun", 2048, 4, 8, 509, 64),
     ]
 
 
