@@ -12,6 +12,9 @@
 // A row's result is a fixed sequence of operations on its own keys: chunks start at absolute
 // multiples of 64, lanes map to keys and dims the same way every time.  It therefore does not
 // depend on which other rows are in the launch, nor on which physical pages hold the keys.
+//
+// 32-bit storage with head sizes 16, 32, 64 and 128, up to 16 query heads per kv head and pages of a multiple of 4 tokens
+// takes attention_f32_kernel below: the same products on the matrix cores' 32-bit instruction.
 #include <cfloat>
 
 #include "common.h"
@@ -116,6 +119,208 @@ __global__ void __launch_bounds__(kAttnWaves* kWave)
   }
 }
 
+// ---- 32-bit storage on the matrix cores (v_mfma_f32_16x16x4_f32) -----------------------------------------------------------
+// A workgroup owns 16 items, an item being one query head of one row: the heads of a kv head's group, of one row or of 16 /
+// group consecutive rows, so that the keys and values of the group are read once.  Its waves take the chunks of 64 keys in turn
+// (chunk c goes to wave c % WAVES) and meet in LDS at the end, in wave order.  Products are transposed as in the bfloat16
+// kernels, S^T = K Q^T and O^T += V^T P^T: a lane's scores are four consecutive keys of one item, which is where the second
+// product wants their probabilities, and both caches are read in 16-byte pieces.
+// A chunk in which an item sees nothing changes nothing of it, so its result does not depend on the items beside it.
+// One wave per (row, head) that reads values one token at a time (the kernel above) was bound by that chain of loads: two prompts
+// of 301 and 272 tokens and 15 decode steps behind them, 32 heads of 64: 123.6 us a launch in the mean -> 13.8 us.
+using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
+
+template <int NT>      // head size / 16
+constexpr int f32_waves() { return NT <= 4 ? 8 : 4; }      // (a wave's share of the output lies in LDS: 64 KB in all)
+
+template <int NT>
+__global__ void __launch_bounds__(f32_waves<NT>() * kWave)
+    attention_f32_kernel(const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
+                         const float* __restrict__ kcache, const float* __restrict__ vcache, const int* __restrict__ tables,
+                         int table_stride, const int* __restrict__ row_seq, const int* __restrict__ ctx_lens, int T, int nh, int nkv,
+                         int rows_per_tile, int B, float scale, int window) {
+  constexpr int WAVES = f32_waves<NT>(), hd = 16 * NT;
+  __shared__ f32x4 part_o[WAVES][16][NT * 4];
+  __shared__ float part_m[WAVES][16], part_l[WAVES][16];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int it = lane & 15, g = lane >> 4;
+  const int group = nh / nkv, kvh = blockIdx.x % nkv, r0 = blockIdx.x / nkv * rows_per_tile;
+  const int rows = T - r0 < rows_per_tile ? T - r0 : rows_per_tile;
+  const int own = it / group;                                   // the item's row within the tile
+  const bool real = it < rows * group;
+  const int row = r0 + (real ? own : 0), head = kvh * group + (real ? it % group : 0);
+  const int ctx = real ? ctx_lens[row] : 0;
+  const int first = (window > 0 && ctx > window) ? ctx - window : 0;
+  f32x4 qf[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+    qf[u] = *reinterpret_cast<const f32x4*>(q + size_t(row) * q_stride + size_t(head) * hd + 16 * u + 4 * g) * scale;
+
+  const size_t head_stride = size_t(B) * hd, page_stride = head_stride * nkv;
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[NT];
+#pragma unroll
+  for (int d = 0; d < NT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // consecutive rows of one sequence walk its keys together
+  for (int j = 0; j < rows;) {
+    const int seq = row_seq[r0 + j];
+    int end = j, most = 0, least = 0x7fffffff;                  // rows j .. end - 1 see tokens in [least, most)
+    for (; end < rows && row_seq[r0 + end] == seq; ++end) {
+      const int c = ctx_lens[r0 + end];
+      if (c <= 0) continue;
+      const int f = (window > 0 && c > window) ? c - window : 0;
+      most = c > most ? c : most;
+      least = f < least ? f : least;
+    }
+    const bool mine = real && own >= j && own < end;
+    const int* table = tables + size_t(seq) * table_stride;
+    int chunk = most > 0 ? least / kWave : 0;
+    chunk += (wave - chunk % WAVES + WAVES) % WAVES;
+    for (int c0 = chunk * kWave; c0 < most; c0 += WAVES * kWave) {
+      f32x4 kf[4][NT], vf[4][NT];
+      const float *kp[4], *vp[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {                             // tokens outside [least, most) read an inner token's place
+        int t = c0 + 16 * i + it;
+        t = t < most ? (t > least ? t : least) : most - 1;
+        kp[i] = kcache + size_t(table[t / B]) * page_stride + kvh * head_stride + size_t(t % B) * hd + 4 * g;
+        int t4 = c0 + 16 * i + 4 * g;
+        t4 = t4 < most ? (t4 > least ? t4 : least) : most - 1;
+        t4 &= ~3;
+        vp[i] = vcache + size_t(table[t4 / B]) * page_stride + kvh * head_stride + size_t(it) * B + t4 % B;
+      }
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kf[i][u] = *reinterpret_cast<const f32x4*>(kp[i] + 16 * u);
+#pragma unroll
+      for (int d = 0; d < NT; ++d)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vf[i][d] = *reinterpret_cast<const f32x4*>(vp[i] + size_t(16 * d) * B);
+      f32x4 s[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][u][e], qf[u][e], s[i], 0, 0, 0);
+      float top = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = c0 + 16 * i + 4 * g + e;
+          const bool sees = mine && t >= first && t < ctx;
+          s[i][e] = sees ? s[i][e] : -INFINITY;
+          top = fmaxf(top, s[i][e]);
+        }
+      top = fmaxf(top, __shfl_xor(top, 16, kWave));
+      top = fmaxf(top, __shfl_xor(top, 32, kWave));
+      const float m_new = fmaxf(m, top);
+      const bool some = m_new > -INFINITY;                      // the item has seen a key with a finite score
+      const float alpha = some ? expf(m - m_new) : 1.f;
+      float sum = 0.f, bad = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = c0 + 16 * i + 4 * g + e;
+          const bool sees = mine && t >= first && t < ctx;
+          s[i][e] = sees ? expf(s[i][e] - m_new) : 0.f;
+          sum += s[i][e];
+          // values outside [least, most) are a page's previous owner's: zero times a stale Inf or NaN would not be zero
+          const bool kept = t >= least && t < most;
+#pragma unroll
+          for (int d = 0; d < NT; ++d) {
+            vf[i][d][e] = kept ? vf[i][d][e] : 0.f;
+            bad = fmaf(vf[i][d][e], 0.f, bad);                  // NaN when some value is not finite
+          }
+        }
+      l = l * alpha + sum;
+      m = m_new;
+#pragma unroll
+      for (int d = 0; d < NT; ++d) o[d] *= alpha;
+      if (end - j == 1 || __ballot(bad != bad) == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int d = 0; d < NT; ++d) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][d][e], s[i][e], o[d], 0, 0, 0);
+      } else {
+        // a value that is not finite counts for the rows that see it only: row by row, the others' values zero
+        for (int r = j; r < end; ++r) {
+          const int c = ctx_lens[r0 + r], f = (window > 0 && c > window) ? c - window : 0;
+          f32x4 one[NT];
+#pragma unroll
+          for (int d = 0; d < NT; ++d) one[d] = o[d];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int t = c0 + 16 * i + 4 * g + e;
+#pragma unroll
+              for (int d = 0; d < NT; ++d)
+                one[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(t >= f && t < c ? vf[i][d][e] : 0.f, s[i][e], one[d], 0, 0, 0);
+            }
+#pragma unroll
+          for (int d = 0; d < NT; ++d) o[d] = own == r ? one[d] : o[d];
+        }
+      }
+    }
+    j = end;
+  }
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+  if (g == 0) {
+    part_m[wave][it] = m;
+    part_l[wave][it] = l;
+  }
+#pragma unroll
+  for (int d = 0; d < NT; ++d) part_o[wave][it][4 * d + g] = o[d];
+  __syncthreads();
+  for (int t = threadIdx.x; t < rows * group * NT * 4; t += WAVES * kWave) {
+    const int i = t / (NT * 4), d = t % (NT * 4), r = r0 + i / group;
+    float* to = out + size_t(r) * out_stride + size_t(kvh * group + i % group) * hd + 4 * d;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    if (ctx_lens[r] > 0) {
+      float high = part_m[0][i], total = 0.f;
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) high = fmaxf(high, part_m[w][i]);
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        const float f = part_m[w][i] > -INFINITY ? expf(part_m[w][i] - high) : 0.f;      // (a wave that saw nothing: zero)
+        if (part_m[w][i] > -INFINITY || part_l[w][i] != 0.f) {
+          total += f * part_l[w][i];
+          sum += f * part_o[w][i][d];
+        }
+      }
+      sum = sum / total;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) to[e] = sum[e];
+  }
+}
+
+// Shapes of the kernel above: a rule on the model's sizes alone, so that all rows of a model take the same one.
+bool attention_f32_takes(int nh, int nkv, int hd, int B) {
+  return (hd == 16 || hd == 32 || hd == 64 || hd == 128) && nh / nkv <= 16 && B % 4 == 0;
+}
+
+template <int NT>
+void launch_attention_f32(const float* q, int q_stride, float* out, int out_stride, const float* kcache, const float* vcache,
+                          const int* tables, int table_stride, const int* row_seq, const int* ctx_lens, int T, int nh, int nkv,
+                          int B, float scale, int window, hipStream_t s) {
+  // Few rows (decoding): one row a workgroup, whose keys nobody shares.  Many: as many rows as fill the 16 items.
+  const int per = static_cast<long long>(T) * nkv <= 512 ? 1 : 16 / (nh / nkv);
+  const unsigned blocks = static_cast<unsigned>((T + per - 1) / per) * nkv;
+  attention_f32_kernel<NT><<<blocks, f32_waves<NT>() * kWave, 0, s>>>(q, q_stride, out, out_stride, kcache, vcache, tables, table_stride,
+                                                                      row_seq, ctx_lens, T, nh, nkv, per, B, scale, window);
+}
+
 }  // namespace kvcm
 
 using namespace kvcm;
@@ -149,6 +354,15 @@ extern "C" int kvcm_attention_generic(const void* q, int dtype, int q_stride, vo
   const long long blocks = (items + kAttnWaves - 1) / kAttnWaves;
   KVCM_REQUIRE(blocks < (1ll << 31), "attention: too many rows");
   const size_t lds = sizeof(float) * kAttnWaves * hd;
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (dtype == kF32 && attention_f32_takes(nh, nkv, hd, B) && q_stride % 4 == 0 && aligned(q) && aligned(kcache) && aligned(vcache)) {
+    KVCM_REQUIRE(static_cast<long long>(T) * nkv < (1ll << 31), "attention: too many rows");
+    auto* launch = hd == 16 ? launch_attention_f32<1> : hd == 32 ? launch_attention_f32<2> : hd == 64 ? launch_attention_f32<4>
+                                                                                              : launch_attention_f32<8>;
+    launch(static_cast<const float*>(q), q_stride, static_cast<float*>(out), out_stride, static_cast<const float*>(kcache),
+           static_cast<const float*>(vcache), tables, table_stride, row_seq, ctx_lens, T, nh, nkv, B, scale, window, s);
+    return launch_status("attention_f32");
+  }
   if (dtype == kF32)
     attention_generic_kernel<float><<<dim3(static_cast<unsigned>(blocks)), kAttnWaves * kWave, lds, s>>>(
         static_cast<const float*>(q), q_stride, static_cast<float*>(out), out_stride,

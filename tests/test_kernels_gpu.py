@@ -489,6 +489,25 @@ def test_paged_attention_window_edge(ops, window):
         assert np.abs(got[r, 0] - P["Vl"][0][edge, 0]).max() > 0.1
 
 
+@pytest.mark.parametrize("nh,nkv,hd,B,window", [(4, 2, 16, 4, 0), (3, 1, 32, 8, 0), (32, 4, 64, 16, 0), (16, 1, 64, 16, 70), (8, 8, 128, 64, 0)])
+def test_paged_attention_f32_rows_do_not_depend_on_their_neighbours(ops, nh, nkv, hd, B, window):
+    # prompt rows share a workgroup's 16 places and its keys, decoded rows do not; values that no row of a context sees, or
+    # that only its later rows see, may be anything
+    P = _paged_problem(np.random.default_rng(nh + hd), [130, 5, 66, 1], nh, nkv, hd, B, all_rows=True)
+    P["Vc"][P["tables"][0, 100 // B], :, 100 % B] = np.nan
+    P["Vl"][0][100] = np.nan
+    last = (P["ctx"].max() - 1) // B
+    P["Vc"][P["tables"][0, last], :, 130 - last * B:] = np.inf                      # behind the context's end
+    got = _run_attention(ops, P, nh, nkv, hd, torch.float32, window=window)
+    ref = _ref_attention(P, nh, nkv, hd, window=window)
+    sees = np.array([s == 0 and c > 100 and (not window or c - 1 - 100 < window) for s, c in zip(P["row_seq"], P["ctx"])])
+    assert np.isnan(got[sees]).all() and np.isfinite(got[~sees]).all()
+    np.testing.assert_allclose(got[~sees], ref[~sees], atol=2e-5, rtol=0)
+    for r in (0, 63, 64, 99, 128, 129, 131, 135, 200):
+        one = dict(P, Q=P["Q"][r:r + 1], row_seq=P["row_seq"][r:r + 1], ctx=P["ctx"][r:r + 1], R=1)
+        np.testing.assert_array_equal(_run_attention(ops, one, nh, nkv, hd, torch.float32, window=window)[0], got[r])
+
+
 # -------------------------------------------------------------------------------- sampling
 def test_argmax_reference_vector(ops):
     # tests/test_kernels.cu:96-109
