@@ -1,65 +1,332 @@
-// Y[M,N] = X[M,K] * W[N,K]^T in true 32-bit: plain FMA, no matrix-core mode of lower precision.
-// Every output element is one chain of fused multiply-adds over k = 0 .. K-1 in ascending order,
-// whatever M, the tile shape or the position of the element in its tile: a row's result does not
-// depend on which other rows share the launch.  (The reference has no 32-bit path; its GEMMs are
-// cuBLAS calls with this same operand layout, src/model/llama.cpp:45-52.)
+// Y[M,N] = X[M,K] * W[N,K]^T in true 32-bit, on the matrix cores' 32-bit instruction (v_mfma_f32_16x16x4_f32: 32-bit
+// operands, 32-bit fused multiply-adds; no mode of lower precision).
+//
+// Every output element is the same sequence of operations whatever M, the kernel, the tile or the element's place in it, so a
+// row's result does not depend on which other rows share the launch.  K is cut into up to 8 segments whose length depends on K
+// alone (segment_units).  A segment is one chain of matrix instructions over its units of 32 k in ascending order, halves of 16
+// after one another, instruction m of a half taking k = 4 g + m for g = 0..3 (so that a lane's operands of a half are one
+// 16-byte load); the segments' sums are added in ascending order.  Against one chain over all of K this halves the error at K = 2048 (shorter chains).
+// (The reference has no 32-bit path; its GEMMs are cuBLAS calls with this same operand layout, src/model/llama.cpp:45-52.)
+//
+// Three kernels, by sizes:
+//   K <= 256    one chain over all of K (gemm_f32_short_kernel); the segments above are for longer sums.
+//   few rows    bound by reading W once.  A workgroup owns 16 columns, its waves one segment each, eight 16-byte loads of W a
+//               lane multiplied while the next eight are on their way; segments meet in LDS.  Two rows, K = 2048: N = 11264
+//               (92 MB) 22 us, 4.2 TB/s; N = 2048 8 us; K = 5632, N = 2048 20 us.  As 16 x 64 tiles of plain fused
+//               multiply-adds with scalar loads these took 304 us in the mean.
+//   more rows   bound by the matrix cores (157 TFLOP/s).  Tiles of 64 x 64 or 64 x 32, four waves, 32 k staged in LDS while the
+//               next 32 are on their way.  573 rows, K = 2048: N = 11264 254 us (104 TFLOP/s), N = 2048 68 us; 539 us in the
+//               mean of a layer's four products as 64 x 64 tiles of plain fused multiply-adds.
 #include "common.h"
 
 namespace kvcm {
 
-constexpr int kBN = 64, kBK = 16;
+using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 
-template <int BM>  // 64 (TM = 4 rows per thread) or 16 (TM = 1)
-__global__ void __launch_bounds__(256)
-    gemm_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N,
-                    int K, int ldx, int ldw, int ldy) {
-  constexpr int TM = BM / 16;
-  __shared__ float Xs[kBK][BM + 4];
-  __shared__ float Ws[kBK][kBN + 4];
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * kBN;
-  float acc[TM][4];
+constexpr int kUnit = 32, kSegments = 8;      // k of a unit; most segments
+
+// Units of 32 k per segment: up to 8 segments of equal length.
+__host__ __device__ __forceinline__ int segment_units(int K) {
+  const int units = (K + kUnit - 1) / kUnit;
+  return (units + kSegments - 1) / kSegments;
+}
+
+// Four consecutive k of one row, zero from K on.  VEC: rows are 16-byte aligned and K is a multiple of 4, so a piece lies
+// wholly inside or outside; the load is unconditional (from k = 0 where it would be outside) and masked afterwards.  FULL: no
+// piece lies outside.
+template <bool VEC, bool FULL = false>
+__device__ __forceinline__ f32x4 load4(const float* __restrict__ row, int k, int K) {
+  f32x4 v;
+  if constexpr (VEC && FULL) {
+    v = *reinterpret_cast<const f32x4*>(row + k);
+  } else if constexpr (VEC) {
+    v = *reinterpret_cast<const f32x4*>(row + (k < K ? k : 0));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = k < K ? v[e] : 0.f;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = row[k + e < K ? k + e : 0];
+      v[e] = k + e < K ? x : 0.f;
+    }
+  }
+  return v;
+}
+
+// ---- up to 16 * MT rows: columns 16 blockIdx.x .. + 15, wave w segment w ---------------------------------------------------
+template <int MT, bool VEC>
+__global__ void __launch_bounds__(kSegments* kWave)
+    gemm_f32_rows_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
+                         int ldx, int ldw, int ldy) {
+  __shared__ float sums[kSegments][MT][4][kWave];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * MT;
+  const int n = n0 + r < N ? n0 + r : N - 1;
+  const int seg = segment_units(K), units = (K + kUnit - 1) / kUnit;
+  const int lo = wave * seg, hi = lo + seg < units ? lo + seg : units;
+  const float* w = W + size_t(n) * ldw;
+  const float* x[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + 16 * i + r;
+    x[i] = X + size_t(m < M ? m : M - 1) * ldx;
+  }
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // D units at a time, the next D on their way meanwhile (the barriers keep the compiler from moving loads to their uses)
+  constexpr int D = MT == 1 ? 4 : MT == 2 ? 2 : 1;
+  f32x4 b[2][D][2], a[2][D][2][MT];
+  auto fetch = [&](f32x4 (&bb)[D][2], f32x4 (&aa)[D][2][MT], int u) {
+    if (VEC && u + D <= hi && (u + D) * kUnit <= K) {
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = (u + d) * kUnit + 16 * h + 4 * g;
+          bb[d][h] = load4<true, true>(w, k, K);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) aa[d][h][i] = load4<true, true>(x[i], k, K);
+        }
+    } else {
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = u + d < hi ? (u + d) * kUnit + 16 * h + 4 * g : K;      // (beyond the segment: zeros)
+          bb[d][h] = load4<VEC>(w, k, K);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) aa[d][h][i] = load4<VEC>(x[i], k, K);
+        }
+    }
+  };
+  auto multiply = [&](const f32x4 (&bb)[D][2], const f32x4 (&aa)[D][2][MT]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[d][h][i][m], bb[d][h][m], acc[i], 0, 0, 0);
+  };
+  if (lo < hi) fetch(b[0], a[0], lo);
+  for (int u = lo; u < hi; u += 2 * D) {
+    if (u + D < hi) fetch(b[1], a[1], u + D);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(b[0], a[0]);
+    if (u + D >= hi) break;
+    __builtin_amdgcn_sched_barrier(0);
+    if (u + 2 * D < hi) fetch(b[0], a[0], u + 2 * D);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(b[1], a[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sums[wave][i][e][lane] = acc[i][e];
+  __syncthreads();
+  const int segments = (units + seg - 1) / seg;
+  for (int t = threadIdx.x; t < MT * 4 * kWave; t += kSegments * kWave) {
+    const int i = t / (4 * kWave), e = t / kWave % 4, l = t % kWave;
+    float total = sums[0][i][e][l];
+    for (int s = 1; s < segments; ++s) total += sums[s][i][e][l];
+    const int m = m0 + 16 * i + 4 * (l >> 4) + e, c = n0 + (l & 15);
+    if (m < M && c < N) Y[size_t(m) * ldy + c] = total;
+  }
+}
+
+// ---- more rows: tiles of 32 TM x 32 TN, four waves of TM x TN instruction tiles each ----------------------------------------
+// LDS rows hold 32 k as eight 16-byte pieces, piece c of row r at place c ^ (r & 7): a wave's read of one piece of 16 rows
+// meets no bank twice.
+template <int TM, int TN, bool VEC>
+__global__ void __launch_bounds__(256, 2)
+    gemm_f32_tiles_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
+                          int ldx, int ldw, int ldy) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, BK = kUnit;      // (32 rows of 8 pieces: one piece a thread)
+  __shared__ f32x4 xs[2][BM * 8], ws[2][BN * 8];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int r = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int wm = (wave >> 1) * 16 * TM, wn = (wave & 1) * 16 * TN;
+  const int seg = segment_units(K);
+  const int srow = threadIdx.x >> 3, sc = threadIdx.x & 7, kc = 4 * sc;
+  const float *xr[TM], *wr[TN];
+#pragma unroll
+  for (int p = 0; p < TM; ++p) xr[p] = X + size_t(m0 + srow + 32 * p < M ? m0 + srow + 32 * p : M - 1) * ldx;
+#pragma unroll
+  for (int p = 0; p < TN; ++p) wr[p] = W + size_t(n0 + srow + 32 * p < N ? n0 + srow + 32 * p : N - 1) * ldw;
+  const int at = srow * 8 + (sc ^ (srow & 7));      // (rows 32 apart have the same place in a row)
+  f32x4 px[TM], pw[TN];
+  auto fetch = [&](int k0) {
+    if (VEC && k0 + BK <= K) {
+#pragma unroll
+      for (int p = 0; p < TM; ++p) px[p] = load4<true, true>(xr[p], k0 + kc, K);
+#pragma unroll
+      for (int p = 0; p < TN; ++p) pw[p] = load4<true, true>(wr[p], k0 + kc, K);
+    } else {
+#pragma unroll
+      for (int p = 0; p < TM; ++p) px[p] = load4<VEC>(xr[p], k0 + kc, K);
+#pragma unroll
+      for (int p = 0; p < TN; ++p) pw[p] = load4<VEC>(wr[p], k0 + kc, K);
+    }
+  };
+  auto stage = [&](int b) {
+#pragma unroll
+    for (int p = 0; p < TM; ++p) xs[b][at + 256 * p] = px[p];
+#pragma unroll
+    for (int p = 0; p < TN; ++p) ws[b][at + 256 * p] = pw[p];
+  };
+  f32x4 acc[TM][TN], total[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-  for (int k0 = 0; k0 < K; k0 += kBK) {
-    // stage X[m0 .. m0+BM) x [k0 .. k0+16) and W[n0 .. n0+64) x [k0 .. k0+16), zero outside
-    for (int e = threadIdx.x; e < BM * kBK; e += 256) {
-      const int r = e / kBK, c = e % kBK;
-      const int m = m0 + r, k = k0 + c;
-      Xs[c][r] = (m < M && k < K) ? X[size_t(m) * ldx + k] : 0.f;
+    for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  int left = seg, b = 0;      // units left in the segment
+  for (int k0 = 0; k0 < K; k0 += BK, b ^= 1) {
+    if (k0 + BK < K) fetch(k0 + BK);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4 a[TM], w[TN];
+      const int c = 4 * h + g;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int row = wm + 16 * i + r;
+        a[i] = xs[b][row * 8 + (c ^ (row & 7))];
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int row = wn + 16 * j + r;
+        w[j] = ws[b][row * 8 + (c ^ (row & 7))];
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][m], w[j][m], acc[i][j], 0, 0, 0);
     }
-    for (int e = threadIdx.x; e < kBN * kBK; e += 256) {
-      const int r = e / kBK, c = e % kBK;
-      const int n = n0 + r, k = k0 + c;
-      Ws[c][r] = (n < N && k < K) ? W[size_t(n) * ldw + k] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kBK; ++k) {
-      float a[TM], b[4];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = Xs[k][ty * TM + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Ws[k][tx * 4 + j];
+    if (--left == 0) {      // a segment ends
+      left = seg;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+        for (int j = 0; j < TN; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     }
+    if (k0 + BK < K) stage(b ^ 1);
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + ty * TM + i;
-    if (m >= M) continue;
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n < N) Y[size_t(m) * ldy + n] = acc[i][j];
+    for (int j = 0; j < TN; ++j) {
+      if (left != seg) total[i][j] += acc[i][j];      // the last segment, where it is shorter
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm + 16 * i + 4 * g + e, n = n0 + wn + 16 * j + r;
+        if (m < M && n < N) Y[size_t(m) * ldy + n] = total[i][j][e];
+      }
     }
+}
+
+// ---- K up to 256: one chain over all of K ----------------------------------------------------------------------------------
+// These launches (models of small width, low-rank factors) are bound by their latency, so they are not cut: an element is one
+// chain of fused multiply-adds over k in ascending order.  The instruction takes its four k in ascending order (checked bit
+// for bit against such a chain), lane group g holding k = 4 s + g of step s.  A wave owns T x T tiles of 16 x 16, operands
+// straight from L2.  Three rows, K = 64: 7.5 us as 16 x 64 tiles staged through LDS, 3.9 us here.
+constexpr int kShortK = 256;
+
+template <int T>
+__global__ void __launch_bounds__(256)
+    gemm_f32_short_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
+                          int ldx, int ldw, int ldy) {
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int r = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.y * 16 * T, n0 = (blockIdx.x * 4 + wave) * 16 * T;
+  if (n0 >= N) return;
+  const float *x[T], *w[T];
+  f32x4 acc[T][T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    x[i] = X + size_t(m0 + 16 * i + r < M ? m0 + 16 * i + r : M - 1) * ldx;
+    w[i] = W + size_t(n0 + 16 * i + r < N ? n0 + 16 * i + r : N - 1) * ldw;
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  constexpr int D = 16;      // steps whose loads are on their way together
+  for (int k0 = 0; k0 < K; k0 += 4 * D) {
+    float a[D][T], b[D][T];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int k = k0 + 4 * d + g;
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        a[d][i] = x[i][k < K ? k : 0];
+        b[d][i] = w[i][k < K ? k : 0];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const bool in = k0 + 4 * d + g < K;
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a[d][i] : 0.f, in ? b[d][j] : 0.f, acc[i][j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + 16 * i + 4 * g + e, n = n0 + 16 * j + r;
+        if (m < M && n < N) Y[size_t(m) * ldy + n] = acc[i][j][e];
+      }
+}
+
+template <int TM, int TN, bool VEC>
+void launch_tiles(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t s) {
+  const dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM));
+  gemm_f32_tiles_kernel<TM, TN, VEC><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+}
+
+template <bool VEC>
+void launch_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t s) {
+  // Measured at K = 2048 (us; rows kernel / tiles of 64 x 32 / of 64 x 64).  The rows kernel takes 22 for up to 256 workgroups
+  // and about 0.09 for each beyond; the tiles take 41 / 50 as long as a CU has one or two, and 0.084 / 0.165 each beyond.  So
+  // rows while the 64 x 32 tiles are few: N = 2048, 64 rows 22 / 41 / 50, 128 rows 23 / 41 / 50, 200 rows 42 / 41 / 50;
+  // N = 11264, 64 rows 64 / 53 / 54; up to 32 rows its blocks are half as long (24 rows, N = 11264: 39 / 52 / 54, N = 32000:
+  // 100 / 93 / 87), up to 16 always.  The larger tiles (half the columns' rows from L2) from three a CU on: 573 rows, N = 2048
+  // 100 / 68 / 76, N = 11264 497 / 255 / 254, N = 32000 1441 / 705 / 660; 2048 rows, N = 11264: 1764 / 841 / 764
+  // (124 TFLOP/s).  Tiles of 128 x 128 and 128 x 64 were never faster (290 and 303 at 573 rows, N = 11264).
+  if (K <= kShortK) {
+    const int t = M <= 16 ? 1 : 2;
+    const dim3 grid((N + 64 * t - 1) / (64 * t), (M + 16 * t - 1) / (16 * t));
+    if (t == 1) gemm_f32_short_kernel<1><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    else gemm_f32_short_kernel<2><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    return;
+  }
+  const long long few = (long long)((M + 63) / 64) * ((N + 31) / 32), large = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  if (M <= 16 || few < (M <= 32 ? 600 : 228)) {
+    const dim3 grid((N + 15) / 16, M <= 64 ? 1 : (M + 63) / 64);
+    if (M <= 16) gemm_f32_rows_kernel<1, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    else if (M <= 32) gemm_f32_rows_kernel<2, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    else gemm_f32_rows_kernel<4, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+  } else if (large >= 704) {
+    launch_tiles<2, 2, VEC>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+  } else {
+    launch_tiles<2, 1, VEC>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   }
 }
 
@@ -72,12 +339,9 @@ extern "C" int kvcm_gemm_f32(const float* X, const float* W, float* Y, int M, in
   if (M == 0 || N == 0) return 0;
   KVCM_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   KVCM_REQUIRE(ldx >= K && ldw >= K && ldy >= N, "gemm_f32: leading dimensions too small");
-  if (M <= 32) {
-    const dim3 grid((N + kBN - 1) / kBN, (M + 15) / 16);
-    gemm_f32_kernel<16><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
-  } else {
-    const dim3 grid((N + kBN - 1) / kBN, (M + 63) / 64);
-    gemm_f32_kernel<64><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
-  }
+  const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(W) % 16 == 0;
+  if (vec) launch_gemm_f32<true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+  else launch_gemm_f32<false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   return launch_status("gemm_f32");
 }

@@ -568,7 +568,7 @@ def skinny_splits(M, N, K):
 
 
 def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None):
-    """out[M, N] = x[M, K] @ w[N, K]^T.  float32 x float32 -> float32 (plain FMA, fixed k order), or
+    """out[M, N] = x[M, K] @ w[N, K]^T.  float32 x float32 -> float32 (32-bit multiply-adds, an order of k fixed by K), or
     bfloat16 x bfloat16 -> bfloat16 | float32 (MFMA, 32-bit accumulation).
 
     Rows below LIBRARY_GEMM_MIN_ROWS take the weight-streaming kernels (also more rows, up to 512,

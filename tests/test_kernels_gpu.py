@@ -299,6 +299,29 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(ops):
         assert torch.equal(part, full[lo:hi]), "a row's sum changed with the rows beside it"
 
 
+@pytest.mark.parametrize("N,K", [(64, 16), (130, 20), (300, 333), (2560, 2048), (520, 5632)])
+def test_gemm_f32_kernels_agree_bit_for_bit(ops, N, K):
+    # up to 16, 32 and 64 rows, tiles of 64 and of 128 (where those fill the chip): one sequence of operations for an element;
+    # in rows whose 16-byte pieces are aligned, and from an odd column on (single loads)
+    rng = np.random.default_rng(N + K)
+    M = 1700
+    x = _t(rng.normal(size=(M, K + 1)).astype(np.float32), torch.float32)
+    w = _t(rng.normal(size=(N, K)).astype(np.float32), torch.float32)
+    aligned = x[:, :K].contiguous()
+    full = torch.zeros(M, N, device=DEV)
+    ops.gemm(aligned, w, full)
+    ref = aligned.double() @ w.double().t()
+    # segments of at most K / 8 products, each addition off by half a unit in the last place of a partial sum: the errors add
+    # like a random walk of sqrt(K) steps of 2^-24 times the sums' size sqrt(K); six deviations
+    assert float((full - ref).abs().max()) <= 6 * 2.0 ** -24 * K
+    for n in (1, 15, 17, 33, 64, 65, 200):
+        part = torch.zeros(n, N, device=DEV)
+        ops.gemm(aligned[40:40 + n], w, part)
+        assert torch.equal(part, full[40:40 + n]), n
+        ops.gemm(x[40:40 + n, :K], w, part)
+        assert torch.equal(part, full[40:40 + n]), n
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (5, 100, 96), (64, 64, 64), (70, 176, 200), (200, 333, 1024), (3, 50, 20)])
 def test_gemm_bf16_equals_x_wT(ops, M, N, K, out_dtype):
