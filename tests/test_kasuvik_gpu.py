@@ -332,6 +332,31 @@ def test_delta_rule_against_the_plain_recurrence():
             np.testing.assert_allclose(got[s], want[s], atol=5e-5 * max(1.0, np.abs(want[s]).max()))
 
 
+@pytest.mark.parametrize("C,N", [(70, 16), (300, 16), (257, 8), (64, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_selective_scan_in_pieces_by_state_size(C, N, dtype):
+    """Pieces whose channels are a lane's each (8 and 16 states) or spread over lanes, with runs that end anywhere in a piece."""
+    from kvcm_amd import ops
+    rng = np.random.default_rng(C + N)
+    lengths = (129, 1, 640, 200)
+    grid = lambda a: torch.tensor(a).to(dtype).double().numpy()
+    data = [(grid(rng.normal(size=(n, C))), rng.normal(size=(n, C)), rng.normal(size=(n, C)) - 1.0, rng.normal(size=(n, 2 * N))) for n in lengths]
+    a_log, dsk, db = np.log(rng.uniform(0.3, 4.0, size=(C, N))), rng.normal(size=C), rng.normal(size=C)
+    step = Step([(i, 0, n) for i, n in enumerate(lengths)])
+    step.max_run = max(lengths)
+    cat = lambda i: dev(np.concatenate([x[i] for x in data]))
+    state, out = torch.full((4, C, N), 5.0, device=DEV), torch.empty(step.rows, C, dtype=dtype, device=DEV)
+    carry = torch.full((ops.selective_scan_carry_floats(step.rows, step.seqs, C, N),), float("nan"), device=DEV)
+    ops.selective_scan(cat(0).to(dtype), cat(2), dev(db), cat(3), 0, N, dev(a_log), dev(dsk), cat(1), out, state, step, prepare=True, carry=carry)
+    got, row = out.float().cpu().numpy(), 0
+    for x, z, dtl, bc in data:
+        want = plain.selective_scan(x, plain.softplus(dtl + db), -np.exp(a_log), bc[:, :N], bc[:, N:], dsk) * plain.silu(z)
+        # 32-bit: sums in another order; bfloat16: the result's own rounding, half a unit of 8 bits
+        tol = 3e-5 if dtype == torch.float32 else 2.0 ** -8
+        np.testing.assert_allclose(got[row:row + len(x)], want, atol=tol * max(1.0, np.abs(want).max()))
+        row += len(x)
+
+
 def test_gated_activations_and_scaled_embedding():
     from kvcm_amd import ops
     rng = np.random.default_rng(7)
