@@ -91,6 +91,43 @@ __device__ __forceinline__ uint4 keep_first_bf16(uint4 v, int n) {
   return uint4{v.x & word(0), v.y & word(1), v.z & word(2), v.w & word(3)};
 }
 
+// Four values of a row of n from place i on, zero beyond its end.  FULL: the row is 16-byte aligned and nothing lies beyond;
+// WIDE: it is aligned, and n and i are multiples of four.  Loads are unconditional, from places clamped into the row, and
+// masked value by value afterwards (a branch around a load would make each wait for the one before).
+enum RowLoad : int { kRowSingle = 0, kRowWide = 1, kRowFull = 2 };
+template <int HOW>
+__device__ __forceinline__ float4 load_four(const float* __restrict__ row, int i, int n) {
+  if constexpr (HOW == kRowFull) return *reinterpret_cast<const float4*>(row + i);
+  float4 x;
+  if constexpr (HOW == kRowWide) {
+    x = *reinterpret_cast<const float4*>(row + (i < n ? i : 0));
+  } else {
+    x.x = row[i < n ? i : 0];
+    x.y = row[i + 1 < n ? i + 1 : 0];
+    x.z = row[i + 2 < n ? i + 2 : 0];
+    x.w = row[i + 3 < n ? i + 3 : 0];
+  }
+  x.x = i < n ? x.x : 0.f;
+  x.y = i + 1 < n ? x.y : 0.f;
+  x.z = i + 2 < n ? x.z : 0.f;
+  x.w = i + 3 < n ? x.w : 0.f;
+  return x;
+}
+
+// Which head, and which of its column blocks, a workgroup of a walk over a matrix state takes (blockIdx.x of heads * col_blocks).
+// All of a head's read the same rows: where the heads allow it, one of the eight XCDs (which take workgroups in turn) gets all
+// of them, so that its L2 fetches the rows once.
+__device__ __forceinline__ void head_and_columns(int heads, int col_blocks, int& head, int& cb) {
+  const int b = blockIdx.x;
+  if (heads % 8 == 0) {
+    head = b % 8 + 8 * (b / 8 / col_blocks);
+    cb = b / 8 % col_blocks;
+  } else {
+    head = b / col_blocks;
+    cb = b % col_blocks;
+  }
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);

@@ -11,16 +11,15 @@
 // Two launches.  The first turns the projections of every row into (w, a * u, u), in parallel over rows
 // (the second step of the decay's projection included).
 // The second walks each sequence's run token by token: a value column j of S needs u^T S[:, j], updates itself
-// and sums o_j, and needs no other column, so columns are spread over lanes and workgroups.  The per-token
-// vectors (r, k, w, a*u, u, v) are staged through LDS a few tokens at a time, the next tokens' values
-// requested before the current ones are computed.  A run that starts at position 0 starts from zero
-// without reading its slot.  Tokens are taken one by one in prompts and in decoding.
+// and sums o_j, and needs no other column, so columns are spread over lanes and waves.  What bounds the walk is a token's
+// chain of dependent instructions, so a wave has few columns, its key dimension over up to 16 lanes, and a workgroup is one
+// wave: nothing is shared and nobody waits.  The per-token vectors (r, k, w, a*u, u, v) go from L2 into the lanes that use
+// them, a few tokens ahead.  A run that starts at position 0 starts from zero without reading its slot.  Tokens are taken one
+// by one in prompts and in decoding.
 #include "common.h"
 #include "kvcm_hip.h"
 
 namespace kvcm {
-
-// (tokens staged at once: a template parameter of the walk, fewer for the largest key size so that the values on their way fit the registers)
 
 // one wave per (row, head).  The decay's logit is a two-step projection whose second step runs here in 32-bit:
 // w_lin[c] = sum_j w2[c, j] * tanh(low[j]), low = the first step's output (rank values a row); w2 comes transposed,
@@ -60,110 +59,142 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The state of one head is dk x dv.  A workgroup of 256 threads owns 256 / G value columns of one head of one
-// sequence; the key dimension of a column is spread over G lanes (IPT = DKP / G entries each, DKP: dk padded
-// with zeros), so a token costs a lane IPT multiply-adds for u^T S, a sum across its G lanes, 3 IPT
-// multiply-adds for the update, IPT for o and another sum across the lanes.
-template <int DKP, int G, int TILE>
-__global__ void __launch_bounds__(256)
+// The state of one head is dk x dv.  A wave owns 64 / G * NC value columns of one head of one sequence; the key dimension of a
+// column is spread over G lanes (IPT = DKP / G entries each, DKP: dk padded with zeros), so a token costs a lane IPT
+// multiply-adds for u^T S, a sum across its G lanes, 3 IPT multiply-adds for the update, IPT for o and another sum across the
+// lanes; a lane has NC such columns.  U tokens' vectors are in registers or on their way.  Runs of a few tokens are bound by the state's own bytes instead:
+// they take workgroups of 32 columns (whole lines of the state's rows; 8 sequences of one token: 13 us as waves of 4 columns).
+// One sequence of 2,048 tokens, 32 heads of 64 x 64: 999 us with workgroups of 256 threads that staged the vectors through LDS
+// (64 workgroups on 256 CUs, ten reads of LDS and a quarter of a barrier a token), 294 us here.
+template <int DKP, int G, int NC, int U, int NT, int HOW>
+__global__ void __launch_bounds__(NT)
     delta_scan_kernel(const float* __restrict__ r, int ldr, const float* __restrict__ k, int ldk,
                       const float* __restrict__ v, int ldv, const float* __restrict__ w, const float* __restrict__ au,
                       const float* __restrict__ u, float* __restrict__ o, int ldo, float* __restrict__ state,
                       const int* __restrict__ run_start, const int* __restrict__ seq_start,
                       const int* __restrict__ state_slots, int heads, int dk, int dv, int col_blocks) {
-  constexpr int IPT = DKP / G, CB = 256 / G, W = 5 * DKP + CB;
-  constexpr int PF = (TILE * W + 255) / 256;
-  __shared__ __attribute__((aligned(16))) float tile[TILE][W];      // per token: r, k, w, a*u, u (zero beyond dk), v of these columns
-  const int s = blockIdx.y, head = blockIdx.x / col_blocks, cb = blockIdx.x % col_blocks;
-  const int g = threadIdx.x % G, j = cb * CB + threadIdx.x / G;
+  constexpr int IPT = DKP / G, LC = NT / G, CB = LC * NC, Q = IPT / 4;      // LC columns apart: a lane's NC columns
+  int head, cb;
+  head_and_columns(heads, col_blocks, head, cb);
+  const int s = blockIdx.y;
+  const int g = threadIdx.x % G, j0 = cb * CB + threadIdx.x / G;
   const int r0 = run_start[s], r1 = run_start[s + 1];
   const int slot = state_slots[s];
   if (r1 <= r0) return;
   const size_t D = size_t(heads) * dk;
-  const bool owns = j < dv;
+  bool owns[NC];
+  int j[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    owns[c] = j0 + c * LC < dv;
+    j[c] = owns[c] ? j0 + c * LC : 0;
+  }
   if (slot < 0) {
-    if (owns && g == 0)
-      for (int row = r0; row < r1; ++row) o[size_t(row) * ldo + size_t(head) * dv + j] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (owns[c] && g == 0)
+        for (int row = r0; row < r1; ++row) o[size_t(row) * ldo + size_t(head) * dv + j[c]] = 0.f;
     return;
   }
-  float* st = state + ((size_t(slot) * heads + head) * dk) * dv + (owns ? j : 0);      // [slot][head][i][j]
+  float* st = state + ((size_t(slot) * heads + head) * dk) * dv;      // [slot][head][i][j]
   const bool fresh = seq_start[s] == 0;
-  float S[IPT];
+  float S[NC][IPT];
 #pragma unroll
-  for (int il = 0; il < IPT; ++il) {
-    const int i = g * IPT + il;
-    S[il] = (i < dk && owns && !fresh) ? st[size_t(i) * dv] : 0.f;
-  }
-  float pf[PF];
-  // (loads are unconditional, from clamped places, and masked afterwards: a branch around a load would make every
-  // one of them wait for the one before)
-  auto request = [&](int t0) {      // the staged values of the tokens t0 .. t0 + tile - 1, into registers
-#pragma unroll
-    for (int q = 0; q < PF; ++q) {
-      const int e = threadIdx.x + q * 256;
-      const int t = e / W, off = e % W;
-      const int row = t0 + t < r1 ? t0 + t : r1 - 1;
-      const bool vector = off < 5 * DKP;
-      const int which = off / DKP, i = off % DKP;
-      const int jj = cb * CB + (off - 5 * DKP);
-      const bool ok = t < TILE && t0 + t < r1 && (vector ? i < dk : jj < dv);
-      const size_t col = size_t(head) * dk + (i < dk ? i : dk - 1);
-      const size_t vcol = size_t(head) * dv + ((jj >= 0 && jj < dv) ? jj : 0);
-      const float* src = !vector     ? v + size_t(row) * ldv + vcol
-                         : which == 0 ? r + size_t(row) * ldr + col
-                         : which == 1 ? k + size_t(row) * ldk + col
-                         : which == 2 ? w + size_t(row) * D + col
-                         : which == 3 ? au + size_t(row) * D + col
-                                      : u + size_t(row) * D + col;
-      const float val = *src;
-      pf[q] = ok ? val : 0.f;
-    }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int q = 0; q < PF; ++q) {
-      const int e = threadIdx.x + q * 256;
-      if (e < TILE * W) tile[e / W][e % W] = pf[q];
-    }
-  };
-  request(r0);
-  stage();
-  __syncthreads();
-  for (int t0 = r0; t0 < r1; t0 += TILE) {
-    const int nt = r1 - t0 < TILE ? r1 - t0 : TILE;
-    const bool more = t0 + TILE < r1;
-    if (more) request(t0 + TILE);
-    for (int t = 0; t < nt; ++t) {
-      const float* tv = tile[t];
-      const float vj = tv[5 * DKP + threadIdx.x / G];
-      float sa = 0.f;
-#pragma unroll
-      for (int il = 0; il < IPT; ++il) sa = fmaf(tv[4 * DKP + g * IPT + il], S[il], sa);
-      sa = group_sum<G>(sa);
-      float acc = 0.f;
-#pragma unroll
-      for (int il = 0; il < IPT; ++il) {
-        const int i = g * IPT + il;
-        float sn = tv[2 * DKP + i] * S[il];
-        sn = fmaf(-tv[3 * DKP + i], sa, sn);
-        sn = fmaf(tv[DKP + i], vj, sn);
-        S[il] = sn;
-        acc = fmaf(sn, tv[i], acc);
-      }
-      acc = group_sum<G>(acc);
-      if (owns && g == 0) o[size_t(t0 + t) * ldo + size_t(head) * dv + j] = acc;
-    }
-    __syncthreads();
-    if (more) stage();
-    __syncthreads();
-  }
-  if (owns) {
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int il = 0; il < IPT; ++il) {
       const int i = g * IPT + il;
-      if (i < dk) st[size_t(i) * dv] = S[il];
+      S[c][il] = (i < dk && owns[c] && !fresh) ? st[size_t(i) * dv + j[c]] : 0.f;
     }
+  static_assert(U <= G, "lane n of a column keeps token n's output until the U tokens are stored together");
+  const size_t col = size_t(head) * dk;
+  const float *rp = r + size_t(r0) * ldr + col, *kp = k + size_t(r0) * ldk + col, *vp = v + size_t(r0) * ldv + size_t(head) * dv;
+  const float *wp = w + size_t(r0) * D + col, *ap = au + size_t(r0) * D + col, *up = u + size_t(r0) * D + col;
+  float* op = o + size_t(r0 + g) * ldo + size_t(head) * dv;
+  float4 rv[U][Q], kv[U][Q], wv[U][Q], av[U][Q], uv[U][Q];
+  float vv[U][NC];
+  auto request = [&](int n) {      // the next row
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = g * IPT + 4 * q;
+      uv[n][q] = load_four<HOW>(up, i, dk);
+      wv[n][q] = load_four<HOW>(wp, i, dk);
+      av[n][q] = load_four<HOW>(ap, i, dk);
+      kv[n][q] = load_four<HOW>(kp, i, dk);
+      rv[n][q] = load_four<HOW>(rp, i, dk);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) vv[n][c] = vp[j[c]];
+    up += D; wp += D; ap += D; kp += ldk; rp += ldr; vp += ldv;
+  };
+  float out[NC] = {};
+  auto walk = [&](int n) {
+    float sa[NC] = {}, acc[NC] = {};
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const float ue[4] = {uv[n][q].x, uv[n][q].y, uv[n][q].z, uv[n][q].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) sa[c] = fmaf(ue[e], S[c][4 * q + e], sa[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) sa[c] = group_sum<G>(sa[c]);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const float we[4] = {wv[n][q].x, wv[n][q].y, wv[n][q].z, wv[n][q].w}, ae[4] = {av[n][q].x, av[n][q].y, av[n][q].z, av[n][q].w};
+      const float ke[4] = {kv[n][q].x, kv[n][q].y, kv[n][q].z, kv[n][q].w}, re[4] = {rv[n][q].x, rv[n][q].y, rv[n][q].z, rv[n][q].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          float sn = we[e] * S[c][4 * q + e];
+          sn = fmaf(-ae[e], sa[c], sn);
+          sn = fmaf(ke[e], vv[n][c], sn);
+          S[c][4 * q + e] = sn;
+          acc[c] = fmaf(sn, re[e], acc[c]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      acc[c] = group_sum<G>(acc[c]);
+      out[c] = g == n ? acc[c] : out[c];
+    }
+  };
+  auto store = [&]() {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (owns[c]) op[j[c]] = out[c];
+  };
+#pragma unroll
+  for (int n = 0; n < U; ++n)
+    if (r0 + n < r1) request(n);
+  int t0 = r0;
+  for (; t0 + 2 * U <= r1; t0 += U, op += size_t(U) * ldo) {
+#pragma unroll
+    for (int n = 0; n < U; ++n) {
+      walk(n);
+      request(n);
+      __builtin_amdgcn_sched_barrier(0x7);      // (loads stay here, U tokens ahead of their use; arithmetic may move)
+    }
+    if (g < U) store();
   }
+  for (; t0 < r1; t0 += U, op += size_t(U) * ldo) {
+#pragma unroll
+    for (int n = 0; n < U; ++n)
+      if (t0 + n < r1) {
+        walk(n);
+        if (t0 + n + U < r1) request(n);
+      }
+    if (g < U && t0 + g < r1) store();
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int il = 0; il < IPT; ++il) {
+      const int i = g * IPT + il;
+      if (i < dk && owns[c]) st[size_t(i) * dv + j[c]] = S[c][il];
+    }
 }
 
 }  // namespace kvcm
@@ -190,28 +221,48 @@ int kvcm_delta_prepare(const float* k, int ldk, const float* a_lin, int lda, con
 }
 
 // r, k [T, heads*dk], v [T, heads*dv] at their own strides; w, au, u [T, heads*dk] dense; o [T, >= heads*dv];
-// state [slots, heads, dk, dv]; all 32-bit.
+// state [slots, heads, dk, dv]; all 32-bit.  max_run: tokens of the longest run (what the lanes are dealt out by).
 int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* w, const float* au,
                     const float* u, float* o, int ldo, float* state, const int* run_start, const int* seq_start,
-                    const int* state_slots, int S, int heads, int dk, int dv, hipStream_t s) {
+                    const int* state_slots, int S, int heads, int dk, int dv, int max_run, hipStream_t s) {
   if (S == 0) return 0;
   KVCM_REQUIRE(S > 0 && heads > 0 && dk > 0 && dv > 0, "delta_scan: bad sizes S=%d heads=%d dk=%d dv=%d", S, heads, dk, dv);
   KVCM_REQUIRE(dk <= 256, "delta_scan: a key size of %d is not supported (up to 256)", dk);
-  KVCM_REQUIRE(static_cast<long long>(heads) * ((dv + 31) / 32) < (1ll << 31), "delta_scan: too many heads");
+  KVCM_REQUIRE(static_cast<long long>(heads) * ((dv + 3) / 4) < (1ll << 31), "delta_scan: too many heads");
   KVCM_REQUIRE(S <= 65535, "delta_scan: too many sequences for one launch (%d)", S);
   KVCM_REQUIRE(ldr >= heads * dk && ldk >= heads * dk && ldv >= heads * dv && ldo >= heads * dv, "delta_scan: row strides too small");
-#define KVCM_DELTA(DKP, G, TILE)                                                                                            \
-  {                                                                                                                    \
-    const int col_blocks = (dv + 256 / G - 1) / (256 / G);                                                             \
-    delta_scan_kernel<DKP, G, TILE><<<dim3(heads * col_blocks, S), 256, 0, s>>>(r, ldr, k, ldk, v, ldv, w, au, u, o, ldo, state, \
-                                                                          run_start, seq_start, state_slots, heads, dk, dv, \
-                                                                          col_blocks);                                  \
+  auto aligned = [](const float* p, int ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; };
+  const bool wide = dk % 4 == 0 && aligned(r, ldr) && aligned(k, ldk) && aligned(w, 0) && aligned(au, 0) && aligned(u, 0);
+#define KVCM_DELTA_AS(DKP, G, NC, U, NT, HOW)                                                                                      \
+  {                                                                                                                           \
+    const int col_blocks = (dv + NT / G * NC - 1) / (NT / G * NC);                                                                      \
+    delta_scan_kernel<DKP, G, NC, U, NT, HOW><<<dim3(heads * col_blocks, S), NT, 0, s>>>(r, ldr, k, ldk, v, ldv, w, au, u, o, ldo, \
+                                                                                     state, run_start, seq_start,             \
+                                                                                     state_slots, heads, dk, dv, col_blocks); \
   }
-  if (dk <= 16) KVCM_DELTA(16, 2, 8)
-  else if (dk <= 32) KVCM_DELTA(32, 4, 8)
-  else if (dk <= 64) KVCM_DELTA(64, 8, 8)
-  else if (dk <= 128) KVCM_DELTA(128, 8, 8)
-  else KVCM_DELTA(256, 16, 2)
+#define KVCM_DELTA(DKP, G, NC, U, NT)                                 \
+  {                                                               \
+    if (wide && dk == DKP) KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowFull) \
+    else if (wide) KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowWide)         \
+    else KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowSingle)                 \
+  }
+  // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
+  // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 294 (16 lanes) / 374 and 261 (16 lanes; 8 lanes of two columns).
+  if (max_run >= 16) {
+    if (dk <= 16) KVCM_DELTA(16, 4, 1, 4, kWave)
+    else if (dk <= 32) KVCM_DELTA(32, 8, 1, 4, kWave)
+    else if (dk <= 64 && static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024) KVCM_DELTA(64, 16, 1, 8, kWave)
+    else if (dk <= 64) KVCM_DELTA(64, 8, 2, 4, kWave)
+    else if (dk <= 128) KVCM_DELTA(128, 16, 1, 4, kWave)
+    else KVCM_DELTA(256, 16, 1, 1, kWave)
+  } else {
+    if (dk <= 16) KVCM_DELTA(16, 4, 1, 1, 128)
+    else if (dk <= 32) KVCM_DELTA(32, 8, 1, 1, 256)
+    else if (dk <= 64) KVCM_DELTA(64, 8, 1, 1, 256)
+    else if (dk <= 128) KVCM_DELTA(128, 8, 1, 1, 256)
+    else KVCM_DELTA(256, 16, 1, 1, 256)
+  }
+#undef KVCM_DELTA_AS
 #undef KVCM_DELTA
   return launch_status("delta_scan");
 }

@@ -132,7 +132,7 @@ def _declare(lib):
     lib.kvcm_gated_state_carry_floats.argtypes = [i] * 7
     fn("kvcm_scan_prepare", vp, i, vp, vp, i, i, i, vp)
     fn("kvcm_delta_prepare", vp, i, vp, i, vp, vp, i, vp, i, vp, vp, vp, vp, i, i, i, vp)
-    fn("kvcm_delta_scan", vp, i, vp, i, vp, i, vp, vp, vp, vp, i, vp, vp, vp, vp, i, i, i, i, vp)
+    fn("kvcm_delta_scan", vp, i, vp, i, vp, i, vp, vp, vp, vp, i, vp, vp, vp, vp, i, i, i, i, i, vp)
     lib.kvcm_gemm_library_workspace_bytes.restype = C.c_longlong
     lib.kvcm_gemm_library_workspace_bytes.argtypes = []
     lib.kvcm_program_new.restype = vp
@@ -1372,7 +1372,7 @@ def delta_scan(r, k, v, w, au, u, o, state, step, heads, dk, dv):
           "state must be float32 [slots, heads, dk, dv]")
     _call("kvcm_delta_scan", _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w), _ptr(au), _ptr(u),
           _ptr(o), o.stride(0), _ptr(state), _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs,
-          heads, dk, dv, _stream())
+          heads, dk, dv, int(getattr(step, "max_run", o.shape[0])), _stream())
     return o
 
 

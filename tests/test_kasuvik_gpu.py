@@ -332,6 +332,33 @@ def test_delta_rule_against_the_plain_recurrence():
             np.testing.assert_allclose(got[s], want[s], atol=5e-5 * max(1.0, np.abs(want[s]).max()))
 
 
+@pytest.mark.parametrize("d,dv", [(8, 5), (16, 16), (20, 33), (32, 32), (64, 64), (40, 64), (70, 9), (128, 128), (100, 16), (256, 8), (130, 3)])
+def test_delta_rule_by_sizes_and_run_lengths(d, dv):
+    """Every way the walk deals a state out over lanes and loads its rows (whole rows of 16-byte pieces, masked, single values),
+    with runs around the number of tokens it has on their way and around the length from which runs are long."""
+    from kvcm_amd import ops
+    rng = np.random.default_rng(d)
+    heads, lengths = (8 if d == 64 else 2), ((1, 2, 15), (16, 17, 5), (33, 1, 8), (31, 24, 70))
+    seqs = [{n: rng.normal(size=(sum(x[i] for x in lengths), heads, dv if n == "v" else d)) for n in ("r", "k", "v", "w", "a")} for i in range(3)]
+    for q in seqs:
+        q["w"], q["a"] = np.exp(-0.6 * plain.sigmoid(q["w"])), plain.sigmoid(q["a"])
+    want = [plain.delta_rule(q["r"], q["k"], q["v"], q["w"], q["a"]) for q in seqs]
+    state, at = torch.full((3, heads, d, dv), 3.0, device=DEV), [0, 0, 0]
+    for part in lengths:
+        step = Step([(i, at[i], n) for i, n in enumerate(part)])
+        step.max_run = max(part)
+        cat = lambda f: dev(np.concatenate([f(q)[at[i]:at[i] + part[i]] for i, q in enumerate(seqs)]).reshape(step.rows, -1))
+        unit = lambda q: q["k"] / np.sqrt((q["k"] ** 2).sum(-1, keepdims=True) + 1e-6)
+        o = torch.full((step.rows, heads * dv), float("nan"), device=DEV)
+        ops.delta_scan(cat(lambda q: q["r"]), cat(lambda q: q["k"]), cat(lambda q: q["v"]), cat(lambda q: q["w"]),
+                       cat(lambda q: q["a"] * unit(q)), cat(unit), o, state, step, heads, d, dv)
+        got, row = o.cpu().numpy().reshape(step.rows, heads, dv), 0
+        for i, n in enumerate(part):
+            ref = want[i][at[i]:at[i] + n]
+            np.testing.assert_allclose(got[row:row + n], ref, atol=5e-5 * max(1.0, np.abs(ref).max()))
+            row, at[i] = row + n, at[i] + n
+
+
 @pytest.mark.parametrize("C,N", [(70, 16), (300, 16), (257, 8), (64, 4)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_selective_scan_in_pieces_by_state_size(C, N, dtype):
