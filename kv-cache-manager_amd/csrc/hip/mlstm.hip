@@ -8,17 +8,16 @@
 //   o  = S'^T q / (max(|n' . q|, exp(-m')) + 1e-6)               q comes scaled by q_scale
 //
 // S, n and m start at zero (m at 0, not at minus infinity), are 32-bit and live in the request's state slot.
-// A run is walked token by token, in prompts and in decoding.  Only m_t = max(lf_t + m_(t-1), li_t) has to go first, and it
-// is a chain of one addition and one maximum a token: a launch with one lane per (sequence, head) walks it and leaves
-// (li, lf, m_(t-1), m_t) per row (for runs of 16 rows or more the two logarithms of all rows are made before that, in
-// parallel, so that no tanh or log1p sits in the chain).  The main walk needs no transcendental function in its chain: the
-// three exponentials of a token are evaluated as its values are staged.  A value column j of S needs nothing of another
-// column, so columns are spread over lanes and workgroups, the key dimension of a column over G lanes; every workgroup
-// carries n along beside its columns (n is a column of S whose value is always one) and sums n . q like any column's
-// output.  The per-token vectors (q, k, v of these columns, the three factors) are staged through LDS a few tokens at a
-// time, the next tokens' values requested before the current ones are computed.  All workgroups of a head read the old n
-// from the slot; the first one leaves the new n in scratch, and a small launch moves it to the slot afterwards, so that
-// no workgroup reads a state that another one of the same launch writes.
+// A run is walked token by token, in prompts and in decoding.  Only m_t = max(lf_t + m_(t-1), li_t) has to go first: a launch
+// with one wave per (sequence, head) scans it 64 tokens at a time (the step (lf, li): m -> max(m + lf, li) composes) and leaves
+// every row's three factors (for runs of 16 rows or more the two logarithms of all rows are made before that, in parallel).
+// The main walk needs no transcendental function.  A value column j of S needs nothing of another column, so columns are spread
+// over lanes and waves, the key dimension of a column over G lanes; every wave carries n along beside its columns (n is a
+// column of S whose value is always one) and sums n . q like any column's output.  What bounds the walk is a token's chain of
+// dependent instructions, so a wave has few columns and a workgroup is one wave: nothing is shared and nobody waits.  The
+// per-token vectors go from L2 into the lanes that use them, a few tokens ahead.  All waves of a head read the old n from the
+// slot; the first one leaves the new n in scratch, and a small launch moves it to the slot afterwards, so that no wave reads a
+// state that another one of the same launch writes.
 #include "common.h"
 #include "kvcm_hip.h"
 
@@ -26,8 +25,6 @@ namespace kvcm {
 
 __device__ __forceinline__ float soft_cap(float z, float cap) { return cap * tanhf(z / cap); }
 __device__ __forceinline__ float log_sigmoid(float z) { return z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z)); }
-
-constexpr int kGateTile = 8;
 
 // For steps with long runs the gates' logarithms of all rows are made first, in parallel: coef[row, head] = (li, lf, ., .).
 __global__ void __launch_bounds__(256)
@@ -42,152 +39,186 @@ __global__ void __launch_bounds__(256)
                      0.f, 0.f};
 }
 
-// one lane per (sequence, head): coef[row, head] = (li, lf, m before the row, m after it) for every row of the run; the
-// slot's m is read at the start (a run that starts at position 0 starts from 0) and written at the end.
+// one wave per (sequence, head): coef[row, head] = (exp(lf + m before - m), exp(li - m), exp(-m), .) for every row of the run;
+// the slot's m is read at the start (a run that starts at position 0 starts from 0) and written at the end.
 __global__ void __launch_bounds__(kWave)
     mlstm_max_kernel(const float* __restrict__ ig, int ldi, const float* __restrict__ fg, int ldf,
                      const float* __restrict__ i_bias, const float* __restrict__ f_bias, float cap, float4* __restrict__ coef,
                      float* __restrict__ m_state, const int* __restrict__ run_start, const int* __restrict__ seq_start,
-                     const int* __restrict__ state_slots, int S, int heads, int logs_ready) {
-  const int idx = blockIdx.x * kWave + threadIdx.x;
-  if (idx >= S * heads) return;
-  const int s = idx / heads, head = idx % heads;
+                     const int* __restrict__ state_slots, int heads, int logs_ready) {
+  const int s = blockIdx.x / heads, head = blockIdx.x % heads, lane = threadIdx.x;
   const int r0 = run_start[s], r1 = run_start[s + 1];
   const int slot = state_slots[s];
   if (r1 <= r0) return;
   if (slot < 0) {
-    for (int row = r0; row < r1; ++row) coef[size_t(row) * heads + head] = float4{0.f, 0.f, 0.f, 0.f};
+    for (int row = r0 + lane; row < r1; row += kWave) coef[size_t(row) * heads + head] = float4{0.f, 0.f, 0.f, 0.f};
     return;
   }
   float* mst = m_state + size_t(slot) * heads + head;
   float m = seq_start[s] == 0 ? 0.f : *mst;
   const float ib = i_bias[head], fb = f_bias[head];
-  for (int t0 = r0; t0 < r1; t0 += kGateTile) {
-    float li[kGateTile], lf[kGateTile];
+  auto request = [&](int t0) {
+    const int row = t0 + lane < r1 ? t0 + lane : r1 - 1;
+    float4 c;
+    if (logs_ready) {
+      c = coef[size_t(row) * heads + head];
+    } else {
+      c.x = soft_cap(ig[size_t(row) * ldi + head] + ib, cap);
+      c.y = log_sigmoid(soft_cap(fg[size_t(row) * ldf + head] + fb, cap));
+    }
+    return c;
+  };
+  float4 next = request(r0);
+  for (int t0 = r0; t0 < r1; t0 += kWave) {
+    const bool in = t0 + lane < r1;
+    const float li = in ? next.x : -INFINITY, lf = in ? next.y : 0.f;      // (beyond the run: m stays)
+    if (t0 + kWave < r1) next = request(t0 + kWave);
+    float a = lf, b = li;      // the steps up to this token together: m -> max(m + a, b)
 #pragma unroll
-    for (int t = 0; t < kGateTile; ++t) {      // the tile's loads first, from clamped places
-      const int row = t0 + t < r1 ? t0 + t : r1 - 1;
-      if (logs_ready) {
-        const float4 c = coef[size_t(row) * heads + head];
-        li[t] = c.x;
-        lf[t] = c.y;
-      } else {
-        li[t] = ig[size_t(row) * ldi + head];
-        lf[t] = fg[size_t(row) * ldf + head];
+    for (int d = 1; d < kWave; d <<= 1) {
+      const float pa = __shfl_up(a, d, kWave), pb = __shfl_up(b, d, kWave);
+      if (lane >= d) {
+        b = fmaxf(pb + a, b);
+        a += pa;
       }
     }
-#pragma unroll
-    for (int t = 0; t < kGateTile; ++t) {
-      if (t0 + t >= r1) break;
-      const float a = logs_ready ? li[t] : soft_cap(li[t] + ib, cap);
-      const float f = logs_ready ? lf[t] : log_sigmoid(soft_cap(lf[t] + fb, cap));
-      const float m_new = fmaxf(f + m, a);
-      coef[size_t(t0 + t) * heads + head] = float4{a, f, m, m_new};
-      m = m_new;
-    }
+    const float after = fmaxf(m + a, b);
+    float before = __shfl_up(after, 1, kWave);
+    before = lane == 0 ? m : before;
+    if (in) coef[size_t(t0 + lane) * heads + head] = float4{expf(lf + before - after), expf(li - after), expf(-after), 0.f};
+    m = __shfl(after, kWave - 1, kWave);
   }
-  *mst = m;
+  if (lane == 0) *mst = m;
 }
 
-template <int DKP, int G, int TILE>
-__global__ void __launch_bounds__(256)
+// A wave owns 64 / G * NC value columns of one head of one sequence (NC a lane); U tokens' vectors are in registers or on their way.  Runs of a
+// few tokens are bound by the state's own bytes: they take workgroups of 32 columns (whole lines of the state's rows).
+// One sequence of 2,048 tokens, 32 heads of 64 x 64: 819 us with workgroups of 256 threads that staged the vectors through LDS
+// (64 workgroups on 256 CUs), 292 us here; the maxima 214 us as one lane's chain, 27 us as a scan.
+template <int DKP, int G, int NC, int U, int NT, int HOW>
+__global__ void __launch_bounds__(NT)
     mlstm_scan_kernel(const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v,
                       int ldv, const float4* __restrict__ coef, float q_scale, float* __restrict__ o, int ldo,
                       float* __restrict__ s_state, const float* __restrict__ n_state, float* __restrict__ n_new,
                       const int* __restrict__ run_start, const int* __restrict__ seq_start,
                       const int* __restrict__ state_slots, int heads, int dk, int dv, int col_blocks) {
-  constexpr int IPT = DKP / G, CB = 256 / G, W = 2 * DKP + CB + 3;
-  constexpr int PF = (TILE * (2 * DKP + CB) + 255) / 256;
-  static_assert(TILE <= 256, "one thread stages a token's factors");
-  __shared__ __attribute__((aligned(16))) float tile[TILE][W];      // per token: q (scaled), k (zero beyond dk), v of these columns, keep, take, exp(-m)
-  const int s = blockIdx.y, head = blockIdx.x / col_blocks, cb = blockIdx.x % col_blocks;
-  const int g = threadIdx.x % G, j = cb * CB + threadIdx.x / G;
+  constexpr int IPT = DKP / G, LC = NT / G, CB = LC * NC, Q = IPT / 4;      // LC columns apart: a lane's NC columns
+  int head, cb;
+  head_and_columns(heads, col_blocks, head, cb);
+  const int s = blockIdx.y;
+  const int g = threadIdx.x % G, j0 = cb * CB + threadIdx.x / G;
   const int r0 = run_start[s], r1 = run_start[s + 1];
   const int slot = state_slots[s];
   if (r1 <= r0) return;
-  const bool owns = j < dv;
+  bool owns[NC];
+  int j[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    owns[c] = j0 + c * LC < dv;
+    j[c] = owns[c] ? j0 + c * LC : 0;
+  }
   if (slot < 0) {
-    if (owns && g == 0)
-      for (int row = r0; row < r1; ++row) o[size_t(row) * ldo + size_t(head) * dv + j] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (owns[c] && g == 0)
+        for (int row = r0; row < r1; ++row) o[size_t(row) * ldo + size_t(head) * dv + j[c]] = 0.f;
     return;
   }
-  float* st = s_state + ((size_t(slot) * heads + head) * dk) * dv + (owns ? j : 0);      // [slot][head][i][j]
+  float* st = s_state + ((size_t(slot) * heads + head) * dk) * dv;      // [slot][head][i][j]
   const float* nst = n_state + (size_t(slot) * heads + head) * dk;
   const bool fresh = seq_start[s] == 0;
-  float S[IPT], N[IPT];
+  float S[NC][IPT], N[IPT];
 #pragma unroll
   for (int il = 0; il < IPT; ++il) {
     const int i = g * IPT + il;
-    S[il] = (i < dk && owns && !fresh) ? st[size_t(i) * dv] : 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) S[c][il] = (i < dk && owns[c] && !fresh) ? st[size_t(i) * dv + j[c]] : 0.f;
     N[il] = (i < dk && !fresh) ? nst[i] : 0.f;
   }
-  constexpr int V = 2 * DKP + CB;      // the vectors of a token; its three factors follow
-  float pf[PF];
-  float4 cf;
-  auto request = [&](int t0) {      // unconditional loads from clamped places, masked afterwards
+  static_assert(U <= G, "lane n of a column keeps token n's sums until the U tokens are stored together");
+  const size_t col = size_t(head) * dk;
+  const float *qp = q + size_t(r0) * ldq + col, *kp = k + size_t(r0) * ldk + col, *vp = v + size_t(r0) * ldv + size_t(head) * dv;
+  const float4* cp = coef + size_t(r0) * heads + head;
+  float* op = o + size_t(r0 + g) * ldo + size_t(head) * dv;
+  float4 qv[U][Q], kv[U][Q], cf[U];
+  float vv[U][NC];
+  auto request = [&](int n) {      // the next row
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int e = threadIdx.x + p * 256;
-      const int t = e / V, off = e % V;
-      const int row = t0 + t < r1 ? t0 + t : r1 - 1;
-      const bool vec = off < 2 * DKP;
-      const int which = off / DKP, i = off % DKP;
-      const int jj = cb * CB + (off - 2 * DKP);
-      const bool ok = t < TILE && t0 + t < r1 && (vec ? i < dk : jj < dv);
-      const size_t col = size_t(head) * dk + (i < dk ? i : dk - 1);
-      const size_t vcol = size_t(head) * dv + ((jj >= 0 && jj < dv) ? jj : 0);
-      const float* src = !vec ? v + size_t(row) * ldv + vcol : which == 0 ? q + size_t(row) * ldq + col : k + size_t(row) * ldk + col;
-      const float val = *src;
-      pf[p] = ok ? (off < DKP ? val * q_scale : val) : 0.f;
+    for (int p = 0; p < Q; ++p) {
+      const int i = g * IPT + 4 * p;
+      kv[n][p] = load_four<HOW>(kp, i, dk);
+      qv[n][p] = load_four<HOW>(qp, i, dk);
     }
-    const int t = threadIdx.x < TILE ? threadIdx.x : TILE - 1;
-    cf = coef[size_t(t0 + t < r1 ? t0 + t : r1 - 1) * heads + head];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) vv[n][c] = vp[j[c]];
+    cf[n] = *cp;
+    kp += ldk; qp += ldq; vp += ldv; cp += heads;
   };
-  auto stage = [&]() {
+  float over[NC] = {}, under = 0.f, least = 0.f;
+  auto walk = [&](int n) {
+    const float keep = cf[n].x, take = cf[n].y;
+    float vj[NC], acc[NC] = {}, nq = 0.f;
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int e = threadIdx.x + p * 256;
-      if (e < TILE * V) tile[e / V][e % V] = pf[p];
-    }
-    if (threadIdx.x < TILE) {      // (li, lf, m before, m after) -> the token's three factors
-      tile[threadIdx.x][V] = expf(cf.y + cf.z - cf.w);
-      tile[threadIdx.x][V + 1] = expf(cf.x - cf.w);
-      tile[threadIdx.x][V + 2] = expf(-cf.w);
-    }
-  };
-  request(r0);
-  stage();
-  __syncthreads();
-  for (int t0 = r0; t0 < r1; t0 += TILE) {
-    const int nt = r1 - t0 < TILE ? r1 - t0 : TILE;
-    const bool more = t0 + TILE < r1;
-    if (more) request(t0 + TILE);
-    for (int t = 0; t < nt; ++t) {
-      const float* tv = tile[t];
-      const float keep = tv[V], take = tv[V + 1], floor_ = tv[V + 2];
-      const float vj = take * tv[2 * DKP + threadIdx.x / G];
-      float acc = 0.f, nq = 0.f;
+    for (int c = 0; c < NC; ++c) vj[c] = take * vv[n][c];
 #pragma unroll
-      for (int il = 0; il < IPT; ++il) {
-        const int i = g * IPT + il;
-        const float kd = tv[DKP + i], qd = tv[i];
-        S[il] = fmaf(keep, S[il], kd * vj);
-        N[il] = fmaf(keep, N[il], take * kd);
-        acc = fmaf(S[il], qd, acc);
+    for (int p = 0; p < Q; ++p) {
+      const float ke[4] = {kv[n][p].x, kv[n][p].y, kv[n][p].z, kv[n][p].w}, qe[4] = {qv[n][p].x, qv[n][p].y, qv[n][p].z, qv[n][p].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int il = 4 * p + e;
+        const float qd = qe[e] * q_scale;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          S[c][il] = fmaf(keep, S[c][il], ke[e] * vj[c]);
+          acc[c] = fmaf(S[c][il], qd, acc[c]);
+        }
+        N[il] = fmaf(keep, N[il], take * ke[e]);
         nq = fmaf(N[il], qd, nq);
       }
-      acc = group_sum<G>(acc);
-      nq = group_sum<G>(nq);
-      if (owns && g == 0) o[size_t(t0 + t) * ldo + size_t(head) * dv + j] = acc / (fmaxf(fabsf(nq), floor_) + 1e-6f);
     }
-    __syncthreads();
-    if (more) stage();
-    __syncthreads();
+    nq = group_sum<G>(nq);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      acc[c] = group_sum<G>(acc[c]);
+      over[c] = g == n ? acc[c] : over[c];
+    }
+    under = g == n ? nq : under;
+    least = g == n ? cf[n].z : least;
+  };
+  auto store = [&]() {
+    const float by = fmaxf(fabsf(under), least) + 1e-6f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (owns[c]) op[j[c]] = over[c] / by;
+  };
+#pragma unroll
+  for (int n = 0; n < U; ++n)
+    if (r0 + n < r1) request(n);
+  int t0 = r0;
+  for (; t0 + 2 * U <= r1; t0 += U, op += size_t(U) * ldo) {
+#pragma unroll
+    for (int n = 0; n < U; ++n) {
+      walk(n);
+      request(n);
+      __builtin_amdgcn_sched_barrier(0x7);      // (loads stay here, U tokens ahead of their use; arithmetic may move)
+    }
+    if (g < U) store();
+  }
+  for (; t0 < r1; t0 += U, op += size_t(U) * ldo) {
+#pragma unroll
+    for (int n = 0; n < U; ++n)
+      if (t0 + n < r1) {
+        walk(n);
+        if (t0 + n + U < r1) request(n);
+      }
+    if (g < U && t0 + g < r1) store();
   }
 #pragma unroll
   for (int il = 0; il < IPT; ++il) {
     const int i = g * IPT + il;
-    if (i < dk && owns) st[size_t(i) * dv] = S[il];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (i < dk && owns[c]) st[size_t(i) * dv + j[c]] = S[c][il];
     if (i < dk && cb == 0 && threadIdx.x < G) n_new[(size_t(s) * heads + head) * dk + i] = N[il];
   }
 }
@@ -222,7 +253,7 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
   KVCM_REQUIRE(S > 0 && heads > 0 && dk > 0 && dv > 0, "mlstm_scan: bad sizes S=%d heads=%d dk=%d dv=%d", S, heads, dk, dv);
   KVCM_REQUIRE(dk <= 256, "mlstm_scan: a key size of %d is not supported (up to 256)", dk);
   KVCM_REQUIRE(cap > 0.f, "mlstm_scan: the gates' cap must be positive (%g)", cap);
-  KVCM_REQUIRE(static_cast<long long>(heads) * ((dv + 15) / 16) < (1ll << 31), "mlstm_scan: too many heads");
+  KVCM_REQUIRE(static_cast<long long>(heads) * ((dv + 3) / 4) < (1ll << 31), "mlstm_scan: too many heads");
   KVCM_REQUIRE(S <= 65535 && static_cast<long long>(S) * heads * dk < (1ll << 31), "mlstm_scan: too many sequences for one launch (%d)", S);
   KVCM_REQUIRE(ldq >= heads * dk && ldk >= heads * dk && ldv >= heads * dv && ldo >= heads * dv && ldi >= heads && ldf >= heads,
                "mlstm_scan: row strides too small");
@@ -234,21 +265,41 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
     const long long n = static_cast<long long>(T) * heads;
     mlstm_gate_logs_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, n, heads);
   }
-  mlstm_max_kernel<<<(S * heads + kWave - 1) / kWave, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start,
-                                                                      seq_start, state_slots, S, heads, logs_first);
-#define KVCM_MLSTM(DKP, G, TILE)                                                                                             \
+  mlstm_max_kernel<<<S * heads, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start,
+                                               state_slots, heads, logs_first);
+  auto aligned = [](const float* p, int ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; };
+  const bool wide = dk % 4 == 0 && aligned(q, ldq) && aligned(k, ldk);
+#define KVCM_MLSTM_AS(DKP, G, NC, U, NT, HOW)                                                                                    \
   {                                                                                                                          \
-    const int col_blocks = (dv + 256 / G - 1) / (256 / G);                                                                   \
-    mlstm_scan_kernel<DKP, G, TILE><<<dim3(heads * col_blocks, S), 256, 0, s>>>(q, ldq, k, ldk, v, ldv, cf, q_scale, o, ldo,  \
-                                                                                s_state, n_state, n_new, run_start,          \
-                                                                                seq_start, state_slots, heads, dk, dv,       \
-                                                                                col_blocks);                                 \
+    const int col_blocks = (dv + NT / G * NC - 1) / (NT / G * NC);                                                                     \
+    mlstm_scan_kernel<DKP, G, NC, U, NT, HOW><<<dim3(heads * col_blocks, S), NT, 0, s>>>(q, ldq, k, ldk, v, ldv, cf, q_scale, o,  \
+                                                                                     ldo, s_state, n_state, n_new, run_start, \
+                                                                                     seq_start, state_slots, heads, dk, dv,  \
+                                                                                     col_blocks);                            \
   }
-  if (dk <= 16) KVCM_MLSTM(16, 4, 8)
-  else if (dk <= 32) KVCM_MLSTM(32, 8, 8)
-  else if (dk <= 64) KVCM_MLSTM(64, 8, 8)
-  else if (dk <= 128) KVCM_MLSTM(128, 16, 8)
-  else KVCM_MLSTM(256, 16, 4)
+#define KVCM_MLSTM(DKP, G, NC, U, NT)                                 \
+  {                                                               \
+    if (wide && dk == DKP) KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowFull) \
+    else if (wide) KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowWide)         \
+    else KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowSingle)                 \
+  }
+  // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
+  // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 292 (16 lanes) / 247 and 217 (16 lanes; 8 lanes of two columns).
+  if (max_run >= 16) {
+    if (dk <= 16) KVCM_MLSTM(16, 4, 1, 4, kWave)
+    else if (dk <= 32) KVCM_MLSTM(32, 8, 1, 4, kWave)
+    else if (dk <= 64 && static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024) KVCM_MLSTM(64, 16, 1, 8, kWave)
+    else if (dk <= 64) KVCM_MLSTM(64, 8, 2, 4, kWave)
+    else if (dk <= 128) KVCM_MLSTM(128, 16, 1, 6, kWave)
+    else KVCM_MLSTM(256, 16, 1, 4, kWave)
+  } else {
+    if (dk <= 16) KVCM_MLSTM(16, 4, 1, 1, 128)
+    else if (dk <= 32) KVCM_MLSTM(32, 8, 1, 1, 256)
+    else if (dk <= 64) KVCM_MLSTM(64, 8, 1, 1, 256)
+    else if (dk <= 128) KVCM_MLSTM(128, 16, 1, 1, 256)
+    else KVCM_MLSTM(256, 16, 1, 1, 256)
+  }
+#undef KVCM_MLSTM_AS
 #undef KVCM_MLSTM
   const int per_seq = heads * dk;
   mlstm_keep_n_kernel<<<(S * per_seq + 255) / 256, 256, 0, s>>>(n_new, n_state, run_start, state_slots, S, per_seq);

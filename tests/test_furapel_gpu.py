@@ -269,6 +269,42 @@ def test_matrix_memory_against_the_plain_recurrence(shape):
         np.testing.assert_allclose(g, w, atol=3e-5 * max(1.0, np.abs(w).max()))
 
 
+@pytest.mark.parametrize("d,dv", [(16, 6), (20, 33), (32, 32), (64, 64), (60, 5), (128, 16), (256, 8), (130, 3)])
+def test_matrix_memory_by_sizes_and_run_lengths(d, dv):
+    """Every way the walk deals a state out over lanes and loads its rows, with runs around the number of tokens it has on their
+    way, around the length from which runs are long and around the 64 tokens that the maxima are scanned by."""
+    from kvcm_amd import ops
+    rng = np.random.default_rng(d)
+    heads, cap, parts = (8 if d == 64 else 2), 12.0, ((1, 2, 15), (16, 17, 5), (63, 1, 8), (64, 24, 130), (65, 1, 1))
+    total = [sum(x[i] for x in parts) for i in range(3)]
+    # positive keys and queries: the divisor n . q has no cancellation (its relative error, and the output's, would be unbounded);
+    # then a state of up to 130 tokens and 256 products a sum stays within 3e-5 of 32-bit rounding (256 steps of 2^-24, twice)
+    data = [[np.abs(rng.normal(size=(n, heads, d))), np.abs(rng.normal(size=(n, heads, d))), rng.normal(size=(n, heads, dv)),
+             rng.normal(size=(n, heads)) * 4, rng.normal(size=(n, heads)) * 4 + 2] for n in total]
+    bi, bf = rng.normal(size=heads), rng.normal(size=heads)
+    want = []
+    for q, k, v, gi, gf in data:
+        o = np.zeros((q.shape[0], heads, dv))
+        for a in range(heads):
+            o[:, a], _ = plain.matrix_memory(q[:, a] * d ** -0.5, k[:, a], v[:, a], plain.soft_cap(gi[:, a] + bi[a], cap),
+                                             plain.log_sigmoid(plain.soft_cap(gf[:, a] + bf[a], cap)))
+        want.append(o.reshape(-1, heads * dv))
+    S = torch.full((3, heads, d, dv), 9.0, device=DEV)
+    N, M = torch.full((3, heads, d), -3.0, device=DEV), torch.full((3, heads), 50.0, device=DEV)
+    at = [0, 0, 0]
+    for part in parts:
+        st = Step([(i, at[i], n) for i, n in enumerate(part)])
+        st.max_run = max(part)
+        q, k, v, gi, gf = (dev(np.concatenate([x[j][at[i]:at[i] + part[i]] for i, x in enumerate(data)]).reshape(st.rows, -1)) for j in range(5))
+        coef, o = torch.empty(st.rows, 4 * heads, device=DEV), torch.full((st.rows, heads * dv), float("nan"), device=DEV)
+        ops.mlstm_scan(q, k, v, gi, gf, dev(bi), dev(bf), cap, d ** -0.5, coef, torch.empty(3 * heads * d, device=DEV), o, S, N, M, st, heads, d, dv)
+        row = 0
+        for i, n in enumerate(part):
+            ref = want[i][at[i]:at[i] + n]
+            np.testing.assert_allclose(o[row:row + n].cpu().numpy(), ref, atol=3e-5 * max(1.0, np.abs(ref).max()))
+            row, at[i] = row + n, at[i] + n
+
+
 def test_matrix_memory_keeps_what_an_open_gate_wrote_long_ago():
     """A recurrence that reduces to a lookup: one early token is written with its input gate wide open while every other gate
     is shut, the forget gate keeps everything; 200 tokens later a query along that key reads its value back."""
