@@ -147,6 +147,51 @@ template <> __device__ __forceinline__ float scaled_exp<bf16_t>(float v) { retur
 
 constexpr int kScanTile = 64;      // tokens whose B and C lie in LDS
 
+// Runs of one token (decoding), a lane a channel with all its states: with the states over lanes a wave's four channels each
+// fetched their step size, input and gate sixteen times and asked for four tokens; 8 rows, 4,096 channels, 16 states: 14.5 us a
+// launch, 4.5 us so (2 MB of states read and written).
+template <class T, int N>
+__global__ void __launch_bounds__(kWave)
+    scan_single_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ dt_lin, int lddt, const float* __restrict__ dt_bias,
+                       const float* __restrict__ bc, int ldbc, int off_b, int off_c, const float* __restrict__ a_log,
+                       const float* __restrict__ dskip, const float* __restrict__ z, int ldz, T* __restrict__ out, int ldo,
+                       float* __restrict__ state, const int* __restrict__ run_start, const int* __restrict__ seq_start,
+                       const int* __restrict__ state_slots, int C, int prepared) {
+  const int s = blockIdx.y, c = blockIdx.x * kWave + threadIdx.x;
+  const int r = run_start[s], slot = state_slots[s];
+  if (run_start[s + 1] <= r || c >= C) return;
+  if (slot < 0) {      // a padding sequence: its row carries nothing
+    store_f(out + size_t(r) * ldo + c, 0.f);
+    return;
+  }
+  float* at = state + (size_t(slot) * C + c) * N;
+  const float keep = seq_start[s] == 0 ? 0.f : 1.f;
+  float4 sv[N / 4], av[N / 4];
+#pragma unroll
+  for (int n = 0; n < N / 4; ++n) {
+    sv[n] = *reinterpret_cast<const float4*>(at + 4 * n);
+    av[n] = *reinterpret_cast<const float4*>(a_log + size_t(c) * N + 4 * n);
+  }
+  const float lin = dt_lin[size_t(r) * lddt + c], xx = load_f(x + size_t(r) * ldx + c), zz = z[size_t(r) * ldz + c];
+  const float v = lin + (dt_bias ? dt_bias[c] : 0.f), skip = dskip[c];
+  const float *b = bc + size_t(r) * ldbc + off_b, *cc = bc + size_t(r) * ldbc + off_c;
+  const float dt = prepared ? lin : (v > 20.f ? v : log1pf(expf(v))), dx = dt * xx;
+  float y = 0.f;
+#pragma unroll
+  for (int n = 0; n < N / 4; ++n) {
+    float se[4] = {sv[n].x, sv[n].y, sv[n].z, sv[n].w};
+    const float ae[4] = {av[n].x, av[n].y, av[n].z, av[n].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float was = keep != 0.f ? se[e] : 0.f;      // (a first token starts from zero, whatever the slot holds)
+      se[e] = fmaf(decay_exp<T>(dt * -expf(ae[e])), was, dx * b[4 * n + e]);
+      y = fmaf(se[e], cc[4 * n + e], y);
+    }
+    *reinterpret_cast<float4*>(at + 4 * n) = float4{se[0], se[1], se[2], se[3]};
+  }
+  store_f(out + size_t(r) * ldo + c, fmaf(skip, xx, y) * (prepared ? zz : zz / (1.0f + expf(-zz))));
+}
+
 template <class T, int N, bool OUT>
 __global__ void __launch_bounds__(256)
     scan_channels_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ dt, int lddt, const float* __restrict__ bc,
@@ -271,7 +316,19 @@ template <class T>
 int launch_scan(const void* x, int ldx, const float* dt_lin, int lddt, const float* dt_bias, const float* bc, int ldbc,
                 int off_b, int off_c, const float* a_log, const float* dskip, const float* z, int ldz, void* out, int ldo,
                 float* state, const int* run_start, const int* seq_start, const int* state_slots, int S, int C, int N,
-                int prepared, int phase, int chunk_len, int pieces, float* carry, float* dsum, hipStream_t s) {
+                int prepared, int phase, int chunk_len, int pieces, int max_run, float* carry, float* dsum, hipStream_t s) {
+  auto aligned = [](const float* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (phase == 0 && max_run == 1 && (N == 8 || N == 16) && aligned(state) && aligned(a_log)) {
+    const dim3 grid((C + kWave - 1) / kWave, S);
+#define KVCM_SCAN_SINGLE(N)                                                                                                    \
+  scan_single_kernel<T, N><<<grid, kWave, 0, s>>>(static_cast<const T*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, \
+                                                  a_log, dskip, z, ldz, static_cast<T*>(out), ldo, state, run_start, seq_start, \
+                                                  state_slots, C, prepared)
+    if (N == 8) KVCM_SCAN_SINGLE(8);
+    else KVCM_SCAN_SINGLE(16);
+#undef KVCM_SCAN_SINGLE
+    return launch_status("selective_scan");
+  }
   if (phase != 0 && (N == 8 || N == 16)) {
     const dim3 grid((C + 255) / 256, S, pieces);
 #define KVCM_SCAN_CHANNELS(N, OUT)                                                                                            \
@@ -326,9 +383,9 @@ extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, const floa
   auto launch = [&](int phase, int pieces, float* cr, float* ds) {
     if (dtype == kF32)
       return launch_scan<float>(x, ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, a_log, dskip, z, ldz, out, ldo, state,
-                                run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, cr, ds, s);
+                                run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, max_run, cr, ds, s);
     return launch_scan<bf16_t>(x, ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, a_log, dskip, z, ldz, out, ldo, state,
-                               run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, cr, ds, s);
+                               run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, max_run, cr, ds, s);
   };
   if (chunk_len <= 0) return launch(0, 1, nullptr, nullptr);
   // long runs in pieces of chunk_len rows: every piece from zero, the states that enter the pieces, every piece again

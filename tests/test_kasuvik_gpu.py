@@ -384,6 +384,33 @@ def test_selective_scan_in_pieces_by_state_size(C, N, dtype):
         row += len(x)
 
 
+@pytest.mark.parametrize("C,N", [(64, 16), (70, 16), (33, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_selective_scan_of_single_tokens(C, N, dtype):
+    """Decoded steps whose channels are a lane's each: from a slot with rubbish, beside a padding sequence."""
+    from kvcm_amd import ops
+    rng = np.random.default_rng(C * N)
+    grid = lambda a: torch.tensor(a).to(dtype).double().numpy()
+    n = 5
+    data = [(grid(rng.normal(size=(n, C))), rng.normal(size=(n, C)), rng.normal(size=(n, C)) - 1.0, rng.normal(size=(n, 2 * N))) for _ in range(2)]
+    a_log, dsk, db = np.log(rng.uniform(0.3, 4.0, size=(C, N))), rng.normal(size=C), rng.normal(size=C)
+    want = [plain.selective_scan(x, plain.softplus(dtl + db), -np.exp(a_log), bc[:, :N], bc[:, N:], dsk) * plain.silu(z)
+            for x, z, dtl, bc in data]
+    state = torch.full((2, C, N), float("nan"), device=DEV)
+    for t in range(n):
+        step = Step([(0, t, 1), (-1, 0, 1), (1, t, 1)])
+        step.max_run = 1
+        cat = lambda i: dev(np.stack([data[0][i][t], data[0][i][t], data[1][i][t]]))
+        out = torch.full((3, C), float("nan"), dtype=dtype, device=DEV)
+        ops.selective_scan(cat(0).to(dtype), cat(2), dev(db), cat(3), 0, N, dev(a_log), dev(dsk), cat(1), out, state, step)
+        got = out.float().cpu().numpy()
+        assert not got[1].any()
+        for k, row in ((0, 0), (1, 2)):
+            # 32-bit: sums in another order; bfloat16: the result's own rounding, half a unit of 8 bits
+            tol = 3e-5 if dtype == torch.float32 else 2.0 ** -8
+            np.testing.assert_allclose(got[row], want[k][t], atol=tol * max(1.0, np.abs(want[k]).max()))
+
+
 def test_gated_activations_and_scaled_embedding():
     from kvcm_amd import ops
     rng = np.random.default_rng(7)
