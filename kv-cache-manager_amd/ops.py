@@ -567,7 +567,16 @@ def skinny_splits(M, N, K):
     return lib().kvcm_gemm_skinny_splits(M, N, K)
 
 
-def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None):
+def _rows8_takes(M, N, K):
+    """Whether a product of at most 8 rows that nobody adds slices of runs unsplit (gemm_rows8.hip) instead of split along K
+    with a second launch that adds the slices up.  Measured (us, split and added / unsplit; 8 rows): N 2048, K 2048 8.8 / 4.1;
+    8192 x 2048 14.9 / 8.6; 2048 x 4096 10.6 / 6.9; 2048 x 5632 12.3 / 9.6; 11264 x 2048 17.7 / 12.4; 4096 x 8192 19.1 / 17.7;
+    32000 x 2048 28.6 / 27.5; beyond that each of its many short workgroups reads all rows again: 16384 x 4096 28.2 / 32.1,
+    28672 x 4096 48.9 / 52.6 (one row: 28.4 / 27.7 and 47.8 / 43.7)."""
+    return M <= FUSED_NORM_MAX_ROWS and (M <= 2 or N * K <= 66_000_000) and gemm8_supported(M, N, K)
+
+
+def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False):
     """out[M, N] = x[M, K] @ w[N, K]^T.  float32 x float32 -> float32 (32-bit multiply-adds, an order of k fixed by K), or
     bfloat16 x bfloat16 -> bfloat16 | float32 (MFMA, 32-bit accumulation).
 
@@ -575,6 +584,7 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None):
     while the library is switched off: inside a captured graph); when they split K they need
     ``scratch`` (float32, at least splits*M*N elements).  With ``keep_partial``
     the un-added partial sums are returned as PartialSums (for a fused consumer) instead of ``out``.
+    ``unsplit``: a product of at most 8 rows may run unsplit (gemm_rows8.hip), where nobody asks for its slices.
     ``tuning``: which of the library's algorithms a many-row product runs ("off" | "heuristic" | "all";
     None: this module's LIBRARY_TUNING); an engine passes its own option, so that two engines in one
     process do not change each other's.
@@ -607,6 +617,11 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None):
         ws = _library_workspace(out.device)
         _call("kvcm_gemm_library_f32out", _ptr(x), _ptr(w), _ptr(out), M, N, K, x.stride(0), w.stride(0), out.stride(0),
               _ptr(ws), ws.numel(), _stream())
+        return out
+    if (unsplit and not (keep_partial and scratch is not None) and _rows8_takes(M, N, K) and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        _call("kvcm_gemm8", _ptr(x), x.stride(0), _ptr(w), w.stride(0), M, N, K, 0, 0, 0.0, _ptr(out), _DT[out.dtype],
+              out.stride(0), 0, _stream())
         return out
     library = _library_takes(M, N, K) and out.dtype == torch.bfloat16 and out.is_contiguous()
     S = skinny_splits(M, N, K) if (not library and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0

@@ -19,7 +19,7 @@ def _linear(ctx, step, x, w, name, keep_partial=False, dtype=None):
     out = step.ws(name, (x.shape[0], w.shape[0]), dtype)
     scratch = step.scratch(name, x.shape[0], w.shape[0], w.shape[1])
     return ctx.ops.gemm(x, w, out, scratch=scratch, keep_partial=keep_partial and scratch is not None,
-                        tuning=step.tune_products)
+                        tuning=step.tune_products, unsplit=True)
 
 
 def _to_residual(ctx, step, x, w, name):
@@ -262,7 +262,7 @@ class LinearHead(Head):
         return (self._name(),) if self.params.get("tied") else ()
 
     def forward(self, step, h, out):
-        self.ctx.ops.gemm(h, self.w["table"], out, tuning=step.tune_products)
+        self.ctx.ops.gemm(h, self.w["table"], out, tuning=step.tune_products, unsplit=True)
         if float(self.params.get("scale", 1.0)) != 1.0:
             self.ctx.ops.scale_rows(out, self.params["scale"])
         if float(self.params.get("softcap") or 0.0) > 0.0:
