@@ -2,11 +2,15 @@
 // positions, on the matrix cores: a workgroup of four waves takes 64 consecutive rows of one run and one
 // query head, walks the keys those rows can see 64 at a time (first the pooled blocks from block 0, then the
 // tokens in chunks that start at absolute multiples of 64), stages each chunk's keys and values once in LDS
-// as bfloat16 and multiplies with v_mfma_f32_16x16x32_bf16: S = Q K^T (a wave: 16 rows x 64 keys), the
-// mask and a running-maximum softmax in 32-bit on the accumulators, P rounded to bfloat16 and handed over
-// through LDS as the next product's first operand, O += P V.  Which keys a row sees is decided per score
-// (window, causality, blocks wholly before the window), so a chunk that some rows of the tile do not see
-// costs them nothing but zeros; a row's chunks and their order depend on its own position only.  The first
+// as bfloat16 and multiplies with v_mfma_f32_16x16x32_bf16, transposed: S^T = K Q^T (a wave: 64 keys x 16 rows), the
+// mask and a running-maximum softmax in 32-bit on the accumulators, whose lane holds sixteen keys of one row, P rounded to
+// bfloat16, which is the second operand of O^T += V^T P^T as it lies there (a tile's 16 keys are dealt out so that a lane's
+// eight of 32 are consecutive).  Which keys a row sees is decided per score
+// (window, causality, blocks wholly before the window) in the chunks at the ends of what the tile sees, so a chunk that some
+// rows of the tile do not see costs them nothing but zeros; a row's chunks and their order depend on its own position only.
+// Bound by its vector instructions: with P handed over through LDS, a row's statistics over 16 lanes, the mask at every score
+// and divisions by the page size this took 86 us for 2,048 rows of 32 heads of 64 in a window of 512 with pooled blocks (96 us
+// with capped scores by the exact tanh); 54 us (64 us) as it is, with the same error against 64 bits.  The first
 // keep_first tokens of a sequence may stay visible beyond the window (chunks of their own, from token 0), and the
 // scores may be capped, score <- c tanh(score / c), and a bias that grows with the distance may be taken off them,
 // score <- score - slope_h * (i - j) with a slope per query head (tokens only: not beside pooled blocks); the output may be
@@ -23,6 +27,7 @@ namespace kvcm {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef float pooled_four __attribute__((ext_vector_type(4), aligned(4)));      // (pooled entries may lie at any float)
 
 constexpr int kTileRows = 64, kChunk = 64, kVtPitch = kChunk + 8;
 constexpr float kMasked = -1.0e30f;
@@ -31,9 +36,28 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return uint32_t(float_to_bf16_bits(a)) | (uint32_t(float_to_bf16_bits(b)) << 16);
 }
 
+// largest of the four lanes that share lane % 16
+__device__ __forceinline__ float quad_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// tanh for scores whose exponentials become bfloat16: its series up to 1/4 (three terms beyond x, off by less than 3e-7 of it),
+// 1 - 2 / (1 + e^(2x)) by the hardware's exp2 and reciprocal beyond (off by about 1e-7); the exact function is some thirty
+// instructions of a score's fifty.
+__device__ __forceinline__ float score_tanh(float x) {
+  const float y = x * x;
+  const float near = x * fmaf(y, fmaf(y, fmaf(y, -0.0539682540f, 0.133333333f), -0.333333333f), 1.0f);
+  const float far = fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.88539008177792681f * x)), 1.0f);
+  return y < 0.0625f ? near : far;
+}
+
 // DP: key size padded to a multiple of 32; DVT: tiles of 16 value columns
+// (bounds that keep the accumulators in ordinary registers and, at sizes up to 64, four workgroups on a CU)
 template <int DP, int DVT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DP <= 64 && DVT <= 4 ? 4 : DVT <= 8 ? 2 : 1)
     attention_window_pool_tiles_kernel(const uint16_t* __restrict__ q, int ldq, uint16_t* __restrict__ out, int ldo,
                                        const uint16_t* __restrict__ kcache, const uint16_t* __restrict__ vcache,
                                        const float* __restrict__ pk, const float* __restrict__ pv,
@@ -45,7 +69,6 @@ __global__ void __launch_bounds__(256)
   constexpr int KP = DP + 8, KS = DP / 32, DVP = DVT * 16;
   __shared__ __attribute__((aligned(16))) uint16_t Ks[kChunk][KP];
   __shared__ __attribute__((aligned(16))) uint16_t Vt[DVP][kVtPitch];
-  __shared__ __attribute__((aligned(16))) uint16_t Ps[4][16][kVtPitch];
   const int s = blockIdx.x / tiles_per_seq, tile = blockIdx.x % tiles_per_seq, head = blockIdx.y;
   const int run0 = run_start[s], run_len = run_start[s + 1] - run0;
   if (tile * kTileRows >= run_len) return;
@@ -65,33 +88,27 @@ __global__ void __launch_bounds__(256)
   const float cap2 = softcap * kLog2e;
   const float slope2 = dist_slope ? dist_slope[head] * kLog2e : 0.f;      // the bias in units of log 2, like the scores
 
-  // this wave's 16 query rows as first operands (row = lane % 16, k = 8 * (lane / 16) .. + 8 of every 32)
+  // this wave's 16 query rows as second operands (row = lane % 16, k = 8 * (lane / 16) .. + 8 of every 32)
   bf16x8 qf[KS];
+  const int my_row = wave * 16 + col;      // the row whose scores and output this lane holds
   {
-    const int row = wave * 16 + col;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int k = ks * 32 + quad * 8;
       uint4 v = {0u, 0u, 0u, 0u};
-      if (row < nrows && k < d) v = *reinterpret_cast<const uint4*>(q + size_t(r0 + row) * ldq + size_t(head) * d + k);
+      if (my_row < nrows && k < d) v = *reinterpret_cast<const uint4*>(q + size_t(r0 + my_row) * ldq + size_t(head) * d + k);
       qf[ks] = __builtin_bit_cast(bf16x8, v);
     }
   }
-  // the four rows whose scores this lane holds: 4 * quad + i of the wave's 16
-  int pos[4], seen_blocks[4], lo_pos[4];      // lo_pos: the first token of the row's window or chunk
-  float m[4], lsum[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = wave * 16 + quad * 4 + i;
-    pos[i] = row < nrows ? p0 + row : -1;
-    seen_blocks[i] = (P > 0 && window > 0 && pos[i] + 1 > window) ? (pos[i] + 1 - window) / P : 0;
-    lo_pos[i] = chunk > 0 ? pos[i] / chunk * chunk : window > 0 ? pos[i] - window + 1 : 0;
-    m[i] = kMasked;
-    lsum[i] = 0.f;
-  }
-  f32x4 o[DVT];
+  const int pos = my_row < nrows ? p0 + my_row : -1;
+  const int seen_blocks = (P > 0 && window > 0 && pos + 1 > window) ? (pos + 1 - window) / P : 0;
+  const int lo_pos = chunk > 0 ? pos / chunk * chunk : window > 0 ? pos - window + 1 : 0;      // the first token of the row's window or chunk
+  float m = kMasked;
+  f32x4 o[DVT], lsum = {0.f, 0.f, 0.f, 0.f};      // O^T: column = row, rows = dims 16 vt + 4 quad + i; the sums of P by a product with ones
 #pragma unroll
   for (int vt = 0; vt < DVT; ++vt) o[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t one2 = 0x3F803F80u;
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, uint4{one2, one2, one2, one2});
 
   const int blocks = (P > 0 && window > 0 && p_last + 1 > window) ? (p_last + 1 - window) / P : 0;      // of the tile's last row
   const int t_lo = chunk > 0 ? p0 / chunk * chunk : (window > 0 && p0 + 1 > window) ? p0 + 1 - window : 0;
@@ -100,6 +117,9 @@ __global__ void __launch_bounds__(256)
   // of their own, from token 0, between the blocks and the window (every row of the tile sees all of them)
   const int kept = keep_first < t_lo ? keep_first : t_lo;
   const int head_chunks = block_chunks + (kept + kChunk - 1) / kChunk;
+  // tokens from here to p0 are seen by every row of the tile
+  const int all_from = chunk > 0 ? p_last / chunk * chunk : window > 0 ? p_last - window + 1 : 0;
+  const int page_bits = 31 - __builtin_clz(B);      // (a page size that is a multiple of 8 and divides 64 is a power of two)
   const int first_token_chunk = t_lo / kChunk, last_token_chunk = p_last / kChunk;
   const int chunks = head_chunks + (last_token_chunk - first_token_chunk + 1);
   auto chunk_start = [&](int c) {
@@ -121,7 +141,7 @@ __global__ void __launch_bounds__(256)
       // (pages that the window has passed may have been given back: nothing outside the stretch is read)
       const int tl = t < lo ? lo : t;
       const int tc = tl <= hi ? tl : hi, kc = k < d ? k : d - 8;
-      const uint4 v = *reinterpret_cast<const uint4*>(kcache + ((size_t(table[tc / B]) * nkv + kvh) * B + tc % B) * d + kc);
+      const uint4 v = *reinterpret_cast<const uint4*>(kcache + (((size_t(table[tc >> page_bits]) * nkv + kvh) << page_bits) + (tc & (B - 1))) * d + kc);
       kreg[qq] = (t <= hi && k < d) ? v : uint4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
@@ -130,7 +150,7 @@ __global__ void __launch_bounds__(256)
       const int cc = (e / (kChunk / 8)) % DVP, piece = e % (kChunk / 8), t = c0 + piece * 8;
       const int tl = t < (lo / 8) * 8 ? (lo / 8) * 8 : t;
       const int tc = tl <= hi ? tl : (hi / 8) * 8, ccl = cc < dv ? cc : dv - 1;
-      uint4 v = *reinterpret_cast<const uint4*>(vcache + ((size_t(table[tc / B]) * nkv + kvh) * dv + ccl) * B + tc % B);
+      uint4 v = *reinterpret_cast<const uint4*>(vcache + (((size_t(table[tc >> page_bits]) * nkv + kvh) * dv + ccl) << page_bits) + (tc & (B - 1)));
       v = keep_first_bf16(v, hi + 1 - tc < 8 ? hi + 1 - tc : 8);      // beyond the stretch: whatever was there (counted from the piece that was read)
       vreg[qq] = cc < dv ? v : uint4{0u, 0u, 0u, 0u};
     }
@@ -152,31 +172,55 @@ __global__ void __launch_bounds__(256)
     }
   };
 
+  // where block b's entry (the last one's beyond the blocks) lies: in the page of its last token
+  constexpr int PVQ = (kChunk * (DVP / 4) + 255) / 256;
+  auto pooled_entry = [&](int b) {
+    b = b < blocks ? b : blocks - 1;
+    const int pgi = (b * P + P - 1) >> page_bits;
+    return (size_t(table[pgi]) * nkv + kvh) * E + (b - (pgi << page_bits) / P);
+  };
+
   for (int c = 0; c < chunks; ++c) {
     const bool pooled = c < block_chunks, early = !pooled && c < head_chunks;
     const int c0 = chunk_start(c);
     if (!pooled && c == block_chunks) request_chunk(c);      // the first chunk of tokens: nobody asked for it yet
     __syncthreads();      // the chunk before is done with Ks, Vt and Ps
-    if (pooled) {
-      for (int e = tid; e < kChunk * (DP / 8); e += 256) {
-        const int key = e / (DP / 8), k = (e % (DP / 8)) * 8, b = c0 + key;
-        uint4 v = {0u, 0u, 0u, 0u};
-        if (b < blocks && k < d) {
-          const int pgi = (b * P + P - 1) / B;
-          const float* src = pk + ((size_t(table[pgi]) * nkv + kvh) * E + (b - (pgi * B) / P)) * d + k;
-          const float4 x = *reinterpret_cast<const float4*>(src), y = *reinterpret_cast<const float4*>(src + 4);
-          v = uint4{pack_bf16(x.x, x.y), pack_bf16(x.z, x.w), pack_bf16(y.x, y.y), pack_bf16(y.z, y.w)};
+    if (pooled) {      // (loads from places clamped to the last block, masked afterwards)
+      {
+        pooled_four x[KQ][2];
+#pragma unroll
+        for (int qq = 0; qq < KQ; ++qq) {
+          const int e = tid + qq * 256, k = (e % (DP / 8)) * 8;
+          const float* src = pk + pooled_entry(c0 + (e / (DP / 8)) % kChunk) * d + (k < d ? k : d - 8);
+          x[qq][0] = *reinterpret_cast<const pooled_four*>(src);
+          x[qq][1] = *reinterpret_cast<const pooled_four*>(src + 4);
         }
-        *reinterpret_cast<uint4*>(&Ks[key][k]) = v;
+#pragma unroll
+        for (int qq = 0; qq < KQ; ++qq) {
+          const int e = tid + qq * 256, key = e / (DP / 8), k = (e % (DP / 8)) * 8;
+          uint4 v = {pack_bf16(x[qq][0].x, x[qq][0].y), pack_bf16(x[qq][0].z, x[qq][0].w), pack_bf16(x[qq][1].x, x[qq][1].y),
+                     pack_bf16(x[qq][1].z, x[qq][1].w)};
+          if (c0 + key >= blocks || k >= d) v = uint4{0u, 0u, 0u, 0u};
+          if (e < kChunk * (DP / 8)) *reinterpret_cast<uint4*>(&Ks[key][k]) = v;
+        }
       }
-      for (int e = tid; e < kChunk * DVP; e += 256) {
-        const int key = e / DVP, cc = e % DVP, b = c0 + key;
-        float x = 0.f;
-        if (b < blocks && cc < dv) {
-          const int pgi = (b * P + P - 1) / B;
-          x = pv[((size_t(table[pgi]) * nkv + kvh) * E + (b - (pgi * B) / P)) * dv + cc];
+      __builtin_amdgcn_sched_barrier(0);      // (keys, then values: both at once do not fit the registers)
+      {
+        pooled_four x[PVQ];
+#pragma unroll
+        for (int qq = 0; qq < PVQ; ++qq) {
+          const int e = tid + qq * 256, cc = (e % (DVP / 4)) * 4;
+          x[qq] = *reinterpret_cast<const pooled_four*>(pv + pooled_entry(c0 + (e / (DVP / 4)) % kChunk) * dv + (cc < dv ? cc : dv - 4));
         }
-        Vt[cc][key] = float_to_bf16_bits(x);
+#pragma unroll
+        for (int qq = 0; qq < PVQ; ++qq) {
+          const int e = tid + qq * 256, key = e / (DVP / 4), cc = (e % (DVP / 4)) * 4;
+          const float v[4] = {x[qq].x, x[qq].y, x[qq].z, x[qq].w};
+          const bool in = c0 + key < blocks && cc < dv;
+          if (e < kChunk * (DVP / 4))
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Vt[cc + i][key] = in ? float_to_bf16_bits(v[i]) : uint16_t(0);
+        }
       }
     } else {
       stage_tokens();
@@ -184,87 +228,102 @@ __global__ void __launch_bounds__(256)
     __syncthreads();
     if (!pooled && c + 1 < chunks) request_chunk(c + 1);      // on its way while this chunk is multiplied
 
-    // scores of 16 rows x 64 keys: four column tiles
-    f32x4 sc[4];
+    // scores of 64 keys x 16 rows, two groups of 32 keys as two tiles each: row r of tile t is key 8 (r / 4) + 4 t + r % 4 of
+    // the group, so that this lane's sc[g][t][i] is key 8 quad + 4 t + i of it
+    f32x4 sc[2][2];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-      sc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < 2; ++g)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8 kf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Ks[ct * 16 + col][ks * 32 + quad * 8]));
-        sc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks], kf, sc[ct], 0, 0, 0);
+      for (int t = 0; t < 2; ++t) {
+        sc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int key = g * 32 + 8 * (col / 4) + 4 * t + col % 4;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const bf16x8 kf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Ks[key][ks * 32 + quad * 8]));
+          sc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], sc[g][t], 0, 0, 0);
+        }
+      }
+    const int key0 = c0 + 8 * quad;
+    const bool all_see = !pooled && !early && c0 >= all_from && c0 + kChunk - 1 <= p0;      // (the same for the whole tile)
+    float sv[16];      // of key0 + 32 (j / 8) + j % 8
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      sv[j] = sc[j / 8][j / 4 % 2][j % 4] * f;
+      if (softcap > 0.f) sv[j] = cap2 * score_tanh(sv[j]);
+      if (dist_slope) sv[j] = fmaf(-slope2, float(pos - (key0 + j / 8 * 32 + j % 8)), sv[j]);
+    }
+    uint32_t seen = 0xFFFFu;      // bit j
+    if (!all_see) {
+      seen = 0u;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int key = key0 + j / 8 * 32 + j % 8;
+        const bool vis = pooled ? key < seen_blocks
+                         : early ? (key < kept && pos >= 0)
+                                 : (key >= t_lo && key <= pos && (key >= lo_pos || key < keep_first));
+        seen |= vis ? 1u << j : 0u;
+        sv[j] = vis ? sv[j] : kMasked;
       }
     }
-    float alpha[4];
+    float mx = kMasked;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float mx = kMasked;
-      bool vis[4];
+    for (int j = 0; j < 16; ++j) mx = fmaxf(mx, sv[j]);
+    const float m_new = fmaxf(m, quad_max(mx));
+    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        const int key = c0 + ct * 16 + col;
-        vis[ct] = pooled ? key < seen_blocks[i]
-                  : early ? (key < kept && pos[i] >= 0)
-                          : (key >= t_lo && key <= pos[i] && (key >= lo_pos[i] || key < keep_first));
-        float sv = sc[ct][i] * f;
-        if (softcap > 0.f) sv = cap2 * tanhf(sv);
-        if (dist_slope) sv = fmaf(-slope2, float(pos[i] - key), sv);
-        sv = vis[ct] ? sv : kMasked;
-        sc[ct][i] = sv;
-        mx = fmaxf(mx, sv);
-      }
-      mx = group_max<16>(mx);
-      const float m_new = fmaxf(m[i], mx);
-      alpha[i] = __builtin_amdgcn_exp2f(m[i] - m_new);
-      float add = 0.f;
+    for (int j = 0; j < 16; ++j) sv[j] = __builtin_amdgcn_exp2f(sv[j] - m_new);
+    if (!all_see) {
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        const float p = vis[ct] ? __builtin_amdgcn_exp2f(sc[ct][i] - m_new) : 0.f;
-        const uint16_t pb = float_to_bf16_bits(p);
-        Ps[wave][quad * 4 + i][ct * 16 + col] = pb;
-        add += bf16_bits_to_float(pb);      // the sum of what is multiplied, so that the weights add up to one
-      }
-      lsum[i] = lsum[i] * alpha[i] + add;
-      m[i] = m_new;
+      for (int j = 0; j < 16; ++j) sv[j] = seen >> j & 1u ? sv[j] : 0.f;
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lsum[i] *= alpha;
 #pragma unroll
     for (int vt = 0; vt < DVT; ++vt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[vt][i] *= alpha[i];
-    __syncthreads();      // Ps written by other lanes of the wave
+      for (int i = 0; i < 4; ++i) o[vt][i] *= alpha;
 #pragma unroll
-    for (int ks = 0; ks < kChunk / 32; ++ks) {
-      const bf16x8 pf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Ps[wave][col][ks * 32 + quad * 8]));
+    for (int g = 0; g < 2; ++g) {
+      const bf16x8 pf = __builtin_bit_cast(bf16x8, uint4{pack_bf16(sv[8 * g], sv[8 * g + 1]), pack_bf16(sv[8 * g + 2], sv[8 * g + 3]),
+                                                         pack_bf16(sv[8 * g + 4], sv[8 * g + 5]), pack_bf16(sv[8 * g + 6], sv[8 * g + 7])});
+      lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf, lsum, 0, 0, 0);      // (of what is multiplied, so that the weights add up to one)
 #pragma unroll
       for (int vt = 0; vt < DVT; ++vt) {
-        const bf16x8 vf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Vt[vt * 16 + col][ks * 32 + quad * 8]));
-        o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf, o[vt], 0, 0, 0);
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Vt[vt * 16 + col][g * 32 + quad * 8]));
+        o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[vt], 0, 0, 0);
       }
     }
   }
   const float sl2 = sink_logit ? sink_logit[head] * kLog2e : 0.f;
+  float l = lsum[0], factor = out_scale;
+  if (sink) {      // the head's sink (a score of 0 without a number of its own) joins the denominator, in units of log 2 too
+    const float m_all = fmaxf(m, sl2);
+    const float keep = __builtin_amdgcn_exp2f(m - m_all);
+    l = l * keep + __builtin_amdgcn_exp2f(sl2 - m_all);
+    factor *= keep;
+  }
+  if (my_row >= nrows) return;
+  float inv = factor / l;
+  if (gate && gate_heads) inv *= 1.0f / (1.0f + expf(-gate[size_t(r0 + my_row) * ldg + head]));      // one gate per head
+  uint16_t* orow = out + size_t(r0 + my_row) * ldo + size_t(head) * dv;
+  const float* grow = gate && !gate_heads ? gate + size_t(r0 + my_row) * ldg + size_t(head) * dv : nullptr;      // a gate per element
+  const bool wide = ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float l = group_sum<16>(lsum[i]), factor = out_scale;
-    if (sink) {      // the head's sink (a score of 0 without a number of its own) joins the denominator, in units of log 2 too
-      const float m_all = fmaxf(m[i], sl2);
-      const float keep = __builtin_amdgcn_exp2f(m[i] - m_all);
-      l = l * keep + __builtin_amdgcn_exp2f(sl2 - m_all);
-      factor *= keep;
+  for (int vt = 0; vt < DVT; ++vt) {
+    const int c4 = vt * 16 + 4 * quad;      // (dv is a multiple of 8: the four lie inside or outside)
+    if (c4 >= dv) continue;
+    float res[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      res[i] = o[vt][i] * inv;
+      if (grow) res[i] *= 1.0f / (1.0f + expf(-grow[c4 + i]));
     }
-    const int row = wave * 16 + quad * 4 + i;
-    if (row < nrows) {
-      float inv = factor / l;
-      if (gate && gate_heads) inv *= 1.0f / (1.0f + expf(-gate[size_t(r0 + row) * ldg + head]));      // one gate per head
+    if (wide) {
+      *reinterpret_cast<uint2*>(orow + c4) = uint2{pack_bf16(res[0], res[1]), pack_bf16(res[2], res[3])};
+    } else {
 #pragma unroll
-      for (int vt = 0; vt < DVT; ++vt) {
-        const int cc = vt * 16 + col;
-        if (cc < dv) {
-          float res = o[vt][i] * inv;
-          if (gate && !gate_heads) res *= 1.0f / (1.0f + expf(-gate[size_t(r0 + row) * ldg + size_t(head) * dv + cc]));      // a gate per element
-          out[size_t(r0 + row) * ldo + size_t(head) * dv + cc] = float_to_bf16_bits(res);
-        }
-      }
+      for (int i = 0; i < 4; ++i) orow[c4 + i] = float_to_bf16_bits(res[i]);
     }
   }
 }
