@@ -131,7 +131,7 @@ __global__ void __launch_bounds__(kAttnWaves* kWave)
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 
 template <int NT>      // head size / 16
-constexpr int f32_waves() { return NT <= 4 ? 8 : 4; }      // (a wave's share of the output lies in LDS: 64 KB in all)
+constexpr int f32_waves() { return NT <= 4 ? 8 : 4; }      // (a wave's share of the output lies in LDS: 1 KB a tile, 32 KB in all)
 
 template <int NT>
 __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
       m = m_new;
 #pragma unroll
       for (int d = 0; d < NT; ++d) o[d] *= alpha;
-      if (end - j == 1 || __ballot(bad != bad) == 0) {
+      if (rows == 1 || __ballot(bad != bad) == 0) {      // (zero times these values is zero, or nobody else is here)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll

@@ -531,6 +531,31 @@ def test_paged_attention_f32_rows_do_not_depend_on_their_neighbours(ops, nh, nkv
         np.testing.assert_array_equal(_run_attention(ops, one, nh, nkv, hd, torch.float32, window=window)[0], got[r])
 
 
+@pytest.mark.parametrize("nh,nkv,hd,B,window", [(32, 4, 64, 16, 0), (16, 4, 64, 16, 70), (10, 5, 32, 8, 0), (15, 5, 16, 4, 33), (8, 8, 128, 64, 0), (8, 8, 128, 16, 70)])
+def test_paged_attention_f32_bad_values_stay_with_their_sequence(ops, nh, nkv, hd, B, window):
+    # rows enough for tiles of several rows: a prompt, single rows of other sequences beside its last row and beside each
+    # other, another prompt; every second single row sees values that are not finite
+    rng = np.random.default_rng(nh + hd + window)
+    lens = [129, 40, 70, 5, 1, 64, 65, 90]
+    P = _paged_problem(rng, lens, nh, nkv, hd, B, all_rows=True)
+    single = [s for s in range(1, 7)]
+    rows = np.array([r for r in range(P["R"]) if P["row_seq"][r] not in single or P["ctx"][r] == lens[P["row_seq"][r]]])
+    P = dict(P, Q=P["Q"][rows], row_seq=P["row_seq"][rows], ctx=P["ctx"][rows], R=len(rows))
+    assert P["R"] * nkv > 512 and 16 // (nh // nkv) > 1
+    clean = _run_attention(ops, P, nh, nkv, hd, torch.float32, window=window)
+    bad = [1, 3, 5]
+    for s, value in zip(bad, (np.nan, np.inf, -np.inf)):
+        P["Vc"][P["tables"][s, (lens[s] - 1) // B], :, (lens[s] - 1) % B] = value
+    got = _run_attention(ops, P, nh, nkv, hd, torch.float32, window=window)
+    hit = np.isin(P["row_seq"], bad)
+    assert not np.isfinite(got[hit]).any()
+    np.testing.assert_array_equal(got[~hit], clean[~hit])
+    np.testing.assert_allclose(got[~hit], _ref_attention(P, nh, nkv, hd, window=window)[~hit], atol=2e-5, rtol=0)
+    for r in [int(r) for r in np.flatnonzero(np.isin(P["row_seq"], single))] + [0, 127, 128, P["R"] - 1]:
+        one = dict(P, Q=P["Q"][r:r + 1], row_seq=P["row_seq"][r:r + 1], ctx=P["ctx"][r:r + 1], R=1)
+        np.testing.assert_array_equal(_run_attention(ops, one, nh, nkv, hd, torch.float32, window=window)[0], got[r])
+
+
 # -------------------------------------------------------------------------------- sampling
 def test_argmax_reference_vector(ops):
     # tests/test_kernels.cu:96-109
