@@ -221,10 +221,11 @@ int kvcm_delta_prepare(const float* k, int ldk, const float* a_lin, int lda, con
 }
 
 // r, k [T, heads*dk], v [T, heads*dv] at their own strides; w, au, u [T, heads*dk] dense; o [T, >= heads*dv];
-// state [slots, heads, dk, dv]; all 32-bit.  max_run: tokens of the longest run (what the lanes are dealt out by).
+// state [slots, heads, dk, dv]; all 32-bit.  max_run: tokens of the longest run (what the lanes are dealt out by);
+// one_order: not 0: a row's sums are taken in an order that depends on the key size alone.
 int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* w, const float* au,
                     const float* u, float* o, int ldo, float* state, const int* run_start, const int* seq_start,
-                    const int* state_slots, int S, int heads, int dk, int dv, int max_run, hipStream_t s) {
+                    const int* state_slots, int S, int heads, int dk, int dv, int max_run, int one_order, hipStream_t s) {
   if (S == 0) return 0;
   KVCM_REQUIRE(S > 0 && heads > 0 && dk > 0 && dv > 0, "delta_scan: bad sizes S=%d heads=%d dk=%d dv=%d", S, heads, dk, dv);
   KVCM_REQUIRE(dk <= 256, "delta_scan: a key size of %d is not supported (up to 256)", dk);
@@ -248,10 +249,15 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
   }
   // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
   // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 294 (16 lanes) / 374 and 261 (16 lanes; 8 lanes of two columns).
+  // The lanes of a column are the order of its sums.  With one_order (32-bit storage, where a row's result depends on that row
+  // alone) they follow from the key size, whatever the runs: 8 lanes from 33 to 64, 405 / 211 us; 16 beyond, also for single
+  // tokens (8 rows, 32 heads of 128 x 128: 20 us, with 8 lanes and workgroups of 32 columns 14 us).
+  const bool few = static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024;
   if (max_run >= 16) {
     if (dk <= 16) KVCM_DELTA(16, 4, 1, 4, kWave)
     else if (dk <= 32) KVCM_DELTA(32, 8, 1, 4, kWave)
-    else if (dk <= 64 && static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024) KVCM_DELTA(64, 16, 1, 8, kWave)
+    else if (dk <= 64 && few && !one_order) KVCM_DELTA(64, 16, 1, 8, kWave)
+    else if (dk <= 64 && few) KVCM_DELTA(64, 8, 1, 4, kWave)
     else if (dk <= 64) KVCM_DELTA(64, 8, 2, 4, kWave)
     else if (dk <= 128) KVCM_DELTA(128, 16, 1, 4, kWave)
     else KVCM_DELTA(256, 16, 1, 1, kWave)
@@ -259,6 +265,7 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
     if (dk <= 16) KVCM_DELTA(16, 4, 1, 1, 128)
     else if (dk <= 32) KVCM_DELTA(32, 8, 1, 1, 256)
     else if (dk <= 64) KVCM_DELTA(64, 8, 1, 1, 256)
+    else if (dk <= 128 && one_order) KVCM_DELTA(128, 16, 1, 1, 256)
     else if (dk <= 128) KVCM_DELTA(128, 8, 1, 1, 256)
     else KVCM_DELTA(256, 16, 1, 1, 256)
   }

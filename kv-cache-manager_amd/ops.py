@@ -132,7 +132,7 @@ def _declare(lib):
     lib.kvcm_gated_state_carry_floats.argtypes = [i] * 7
     fn("kvcm_scan_prepare", vp, i, vp, vp, i, i, i, vp)
     fn("kvcm_delta_prepare", vp, i, vp, i, vp, vp, i, vp, i, vp, vp, vp, vp, i, i, i, vp)
-    fn("kvcm_delta_scan", vp, i, vp, i, vp, i, vp, vp, vp, vp, i, vp, vp, vp, vp, i, i, i, i, i, vp)
+    fn("kvcm_delta_scan", vp, i, vp, i, vp, i, vp, vp, vp, vp, i, vp, vp, vp, vp, i, i, i, i, i, i, vp)
     lib.kvcm_gemm_library_workspace_bytes.restype = C.c_longlong
     lib.kvcm_gemm_library_workspace_bytes.argtypes = []
     lib.kvcm_program_new.restype = vp
@@ -1377,8 +1377,9 @@ def delta_prepare(k, a_lin, a_bias, low, w2t, w0, w_out, au_out, u_out, heads, d
           _ptr(w2t), rank, _ptr(w0), _ptr(w_out), _ptr(au_out), _ptr(u_out), rows, heads, d, _stream())
 
 
-def delta_scan(r, k, v, w, au, u, o, state, step, heads, dk, dv):
-    """The delta-rule recurrence over the step's runs (csrc/hip/delta_rule.hip); state [slots, heads, dk, dv]."""
+def delta_scan(r, k, v, w, au, u, o, state, step, heads, dk, dv, one_order=False):
+    """The delta-rule recurrence over the step's runs (csrc/hip/delta_rule.hip); state [slots, heads, dk, dv].  ``one_order``: a
+    row's sums are taken in one order whatever else the step holds (32-bit storage), not in the one that is fastest for its runs."""
     for t, n, c in ((r, "r", heads * dk), (k, "k", heads * dk), (v, "v", heads * dv), (o, "o", heads * dv)):
         _f32rows(t, n, c)
     for t, n in ((w, "w"), (au, "au"), (u, "u")):
@@ -1387,7 +1388,7 @@ def delta_scan(r, k, v, w, au, u, o, state, step, heads, dk, dv):
           "state must be float32 [slots, heads, dk, dv]")
     _call("kvcm_delta_scan", _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w), _ptr(au), _ptr(u),
           _ptr(o), o.stride(0), _ptr(state), _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs,
-          heads, dk, dv, int(getattr(step, "max_run", o.shape[0])), _stream())
+          heads, dk, dv, int(getattr(step, "max_run", o.shape[0])), int(one_order), _stream())
     return o
 
 

@@ -131,8 +131,8 @@ class GeneralDeltaMixer(_StatefulMixer):
         decay, au, u = (step.ws(n, (T, D), torch.float32) for n in ("delta_w", "delta_au", "delta_u"))
         ops.delta_prepare(k, a, w["a_bias"], low, w["w2"], w["w0"], decay, au, u, heads, d, T)
         o = step.ws("delta_o", (T, D), torch.float32)
-        ops.delta_scan(r, k, v, decay, au, u, o, self.state("delta"), step, heads, d, d)
         gated = step.ws("delta_gated", (T, D))
+        ops.delta_scan(r, k, v, decay, au, u, o, self.state("delta"), step, heads, d, d, one_order=gated.dtype == torch.float32)
         ops.head_norm_gate(o, g, w["norm"], gated, heads, d, p["eps"])
         return linear32(self.ctx, step, gated, w["w_o"], "delta_out")
 

@@ -411,6 +411,58 @@ def test_selective_scan_of_single_tokens(C, N, dtype):
             np.testing.assert_allclose(got[row], want[k][t], atol=tol * max(1.0, np.abs(want[k]).max()))
 
 
+# One sequence of 150 tokens: whole, token by token, cut anywhere, and cut beside seven others (whose runs make steps long, and
+# their number the walk's waves many).  Steps as [(slot, first position, count)].
+_ONE = 150
+_WHOLE = [[(0, 0, _ONE)]]
+_SINGLE = [[(0, t, 1)] for t in range(_ONE)]
+_CUT = [[(0, p, n)] for p, n in ((0, 1), (1, 15), (16, 16), (32, 2), (34, 65), (99, 1), (100, 50))]
+_MIXED = ([[(0, t, 1)] + [(s, 20 * t, 20) for s in range(1, 8)] for t in range(7)] + [[(3, 140, 3), (0, 7, 70), (4, 140, 1)]]
+          + [[(0, t, 1)] for t in range(77, 90)] + [[(0, 90, 60)] + [(s, 143 if s == 3 else 141 if s == 4 else 140, 7) for s in range(1, 8)]])
+
+
+def _rows_of_first(run, data):
+    """``run(step, rows of data)`` -> outputs of one step; all schedules' outputs for the sequence in slot 0, and its state's bits."""
+    got = []
+    for schedule in (_WHOLE, _SINGLE, _CUT, _MIXED):
+        rows, call = [], run()
+        for runs in schedule:
+            step = Step(runs)
+            step.max_run = max(n for _, _, n in runs)
+            part = [torch.cat([x[s, p:p + n] for s, p, n in runs]).contiguous() for x in data]
+            out, first = call(step, *part), [s for s, _, _ in runs].index(0)
+            at = sum(n for _, _, n in runs[:first])
+            rows.append(out[at:at + runs[first][2]].clone())
+        got.append((torch.cat(rows), call(None)))
+    return got
+
+
+def _all_equal(got):
+    for out, state in got[1:]:
+        assert torch.equal(out, got[0][0])
+        assert all(torch.equal(a[0], b[0]) for a, b in zip(state, got[0][1]))
+
+
+@pytest.mark.parametrize("d", [12, 32, 64, 100, 256])
+def test_delta_rule_in_32_bits_depends_on_its_row_alone(d):
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(d)
+    heads = 24 if d == 64 else 3      # (at 64 enough heads for eight sequences to fill the chip, too few for one)
+    r, k, v, w, a = (torch.randn(8, _ONE, heads * d, generator=g).to(DEV) for _ in range(5))
+    u = torch.nn.functional.normalize(k.view(8, _ONE, heads, d), dim=-1).reshape(8, _ONE, heads * d)
+
+    def run():
+        state = torch.full((8, heads, d, d), 3.0, device=DEV)
+
+        def call(step, *x):
+            if step is None:
+                return [state]
+            o = torch.empty(step.rows, heads * d, device=DEV)
+            return ops.delta_scan(*x, o, state, step, heads, d, d, one_order=True)
+        return call
+    _all_equal(_rows_of_first(run, (r, k, v, torch.sigmoid(w), torch.sigmoid(a) * u, u)))
+
+
 def test_gated_activations_and_scaled_embedding():
     from kvcm_amd import ops
     rng = np.random.default_rng(7)
