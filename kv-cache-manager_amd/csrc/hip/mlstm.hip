@@ -9,8 +9,8 @@
 //
 // S, n and m start at zero (m at 0, not at minus infinity), are 32-bit and live in the request's state slot.
 // A run is walked token by token, in prompts and in decoding.  Only m_t = max(lf_t + m_(t-1), li_t) has to go first: a launch
-// with one wave per (sequence, head) scans it 64 tokens at a time (the step (lf, li): m -> max(m + lf, li) composes) and leaves
-// every row's three factors (for runs of 16 rows or more the two logarithms of all rows are made before that, in parallel).
+// with one wave per (sequence, head) scans it 64 tokens at a time (the step (lf, li): m -> max(m + lf, li) composes; in 32-bit
+// storage, where a row's result depends on that row alone, it takes them one by one) and leaves every row's three factors (for runs of 16 rows or more the two logarithms of all rows are made before that, in parallel).
 // The main walk needs no transcendental function.  A value column j of S needs nothing of another column, so columns are spread
 // over lanes and waves, the key dimension of a column over G lanes; every wave carries n along beside its columns (n is a
 // column of S whose value is always one) and sums n . q like any column's output.  What bounds the walk is a token's chain of
@@ -39,8 +39,12 @@ __global__ void __launch_bounds__(256)
                      0.f, 0.f};
 }
 
+__device__ __forceinline__ float lane_of(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+
 // one wave per (sequence, head): coef[row, head] = (exp(lf + m before - m), exp(li - m), exp(-m), .) for every row of the run;
-// the slot's m is read at the start (a run that starts at position 0 starts from 0) and written at the end.
+// the slot's m is read at the start (a run that starts at position 0 starts from 0) and written at the end.  IN_ORDER: token by
+// token, so that a row's factors do not depend on where its run began; 2,048 tokens: 56 us, as a scan 27 us.
+template <bool IN_ORDER>
 __global__ void __launch_bounds__(kWave)
     mlstm_max_kernel(const float* __restrict__ ig, int ldi, const float* __restrict__ fg, int ldf,
                      const float* __restrict__ i_bias, const float* __restrict__ f_bias, float cap, float4* __restrict__ coef,
@@ -73,20 +77,39 @@ __global__ void __launch_bounds__(kWave)
     const bool in = t0 + lane < r1;
     const float li = in ? next.x : -INFINITY, lf = in ? next.y : 0.f;      // (beyond the run: m stays)
     if (t0 + kWave < r1) next = request(t0 + kWave);
-    float a = lf, b = li;      // the steps up to this token together: m -> max(m + a, b)
+    float before, after;
+    if constexpr (IN_ORDER) {
+      const int n = r1 - t0 < kWave ? r1 - t0 : kWave;
+      const float entered = m;
+      after = m;
+      auto token = [&](int t) {
+        m = fmaxf(lane_of(lf, t) + m, lane_of(li, t));
+        after = lane == t ? m : after;
+      };
+      if (n == kWave) {
 #pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const float pa = __shfl_up(a, d, kWave), pb = __shfl_up(b, d, kWave);
-      if (lane >= d) {
-        b = fmaxf(pb + a, b);
-        a += pa;
+        for (int t = 0; t < kWave; ++t) token(t);
+      } else {
+        for (int t = 0; t < n; ++t) token(t);
       }
+      before = __shfl_up(after, 1, kWave);
+      before = lane == 0 ? entered : before;
+    } else {
+      float a = lf, b = li;      // the steps up to this token together: m -> max(m + a, b)
+#pragma unroll
+      for (int d = 1; d < kWave; d <<= 1) {
+        const float pa = __shfl_up(a, d, kWave), pb = __shfl_up(b, d, kWave);
+        if (lane >= d) {
+          b = fmaxf(pb + a, b);
+          a += pa;
+        }
+      }
+      after = fmaxf(m + a, b);
+      before = __shfl_up(after, 1, kWave);
+      before = lane == 0 ? m : before;
+      m = __shfl(after, kWave - 1, kWave);
     }
-    const float after = fmaxf(m + a, b);
-    float before = __shfl_up(after, 1, kWave);
-    before = lane == 0 ? m : before;
     if (in) coef[size_t(t0 + lane) * heads + head] = float4{expf(lf + before - after), expf(li - after), expf(-after), 0.f};
-    m = __shfl(after, kWave - 1, kWave);
   }
   if (lane == 0) *mst = m;
 }
@@ -247,7 +270,7 @@ extern "C" {
 int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* ig, int ldi,
                     const float* fg, int ldf, const float* i_bias, const float* f_bias, float cap, float q_scale, float* coef,
                     float* n_new, float* o, int ldo, float* s_state, float* n_state, float* m_state, const int* run_start,
-                    const int* seq_start, const int* state_slots, int S, int heads, int dk, int dv, int T, int max_run,
+                    const int* seq_start, const int* state_slots, int S, int heads, int dk, int dv, int T, int max_run, int one_order,
                     hipStream_t s) {
   if (S == 0) return 0;
   KVCM_REQUIRE(S > 0 && heads > 0 && dk > 0 && dv > 0, "mlstm_scan: bad sizes S=%d heads=%d dk=%d dv=%d", S, heads, dk, dv);
@@ -265,8 +288,9 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
     const long long n = static_cast<long long>(T) * heads;
     mlstm_gate_logs_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, n, heads);
   }
-  mlstm_max_kernel<<<S * heads, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start,
-                                               state_slots, heads, logs_first);
+  auto* maxima = one_order ? mlstm_max_kernel<true> : mlstm_max_kernel<false>;
+  maxima<<<S * heads, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, heads,
+                                     logs_first);
   auto aligned = [](const float* p, int ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; };
   const bool wide = dk % 4 == 0 && aligned(q, ldq) && aligned(k, ldk);
 #define KVCM_MLSTM_AS(DKP, G, NC, U, NT, HOW)                                                                                    \
@@ -285,10 +309,14 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
   }
   // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
   // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 292 (16 lanes) / 247 and 217 (16 lanes; 8 lanes of two columns).
+  // The lanes of a column are the order of its sums: with one_order they follow from the key size alone (8 from 33 to
+  // 64: 394 us for the one sequence).
+  const bool few = static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024;
   if (max_run >= 16) {
     if (dk <= 16) KVCM_MLSTM(16, 4, 1, 4, kWave)
     else if (dk <= 32) KVCM_MLSTM(32, 8, 1, 4, kWave)
-    else if (dk <= 64 && static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024) KVCM_MLSTM(64, 16, 1, 8, kWave)
+    else if (dk <= 64 && few && !one_order) KVCM_MLSTM(64, 16, 1, 8, kWave)
+    else if (dk <= 64 && few) KVCM_MLSTM(64, 8, 1, 8, kWave)
     else if (dk <= 64) KVCM_MLSTM(64, 8, 2, 4, kWave)
     else if (dk <= 128) KVCM_MLSTM(128, 16, 1, 6, kWave)
     else KVCM_MLSTM(256, 16, 1, 4, kWave)

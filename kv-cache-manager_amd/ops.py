@@ -109,7 +109,7 @@ def _declare(lib):
     fn("kvcm_head_norm_store", vp, i, vp, vp, vp, f, i, vp, i, i, vp, f, i, i, vp, vp, i, i, vp, vp, i, i, i, i, i, i, vp)
     fn("kvcm_gemm_heads", vp, i, i, vp, vp, i, i, vp, i, i, i, i, i, vp)
     fn("kvcm_act_rows", vp, i, i, C.c_longlong, vp, i, i, i, i, i, vp)
-    fn("kvcm_mlstm_scan", vp, i, vp, i, vp, i, vp, i, vp, i, vp, vp, f, f, vp, vp, vp, i, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, vp)
+    fn("kvcm_mlstm_scan", vp, i, vp, i, vp, i, vp, i, vp, i, vp, vp, f, f, vp, vp, vp, i, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, vp)
     fn("kvcm_moe_route", vp, i, i, C.c_longlong, i, i, i, f, vp, vp, i, vp)
     fn("kvcm_moe_table_route", vp, vp, i, i, i, vp, vp, i, vp)
     fn("kvcm_moe_up", vp, i, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
@@ -1633,10 +1633,11 @@ def act_rows(x, out, activation):
     return out
 
 
-def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, coef, n_new, o, s_state, n_state, m_state, step, heads, dk, dv):
+def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, coef, n_new, o, s_state, n_state, m_state, step, heads, dk, dv, one_order=False):
     """The matrix memory with exponential gates over the step's runs (csrc/hip/mlstm.hip).  q, k [T, heads*dk], v [T, heads*dv],
     gate_in, gate_keep [T, heads] (projections without biases): 32-bit rows; coef: float32 scratch of 4 T heads values;
-    n_new: float32 scratch of seqs heads dk values; states [slots, heads, dk, dv], [slots, heads, dk], [slots, heads]."""
+    n_new: float32 scratch of seqs heads dk values; states [slots, heads, dk, dv], [slots, heads, dk], [slots, heads].
+    ``one_order``: a row's maximum and sums are taken in one order whatever else the step holds (32-bit storage)."""
     T = o.shape[0]
     for t, n, c in ((q, "q", heads * dk), (k, "k", heads * dk), (v, "v", heads * dv), (o, "o", heads * dv), (gate_in, "gate_in", heads),
                     (gate_keep, "gate_keep", heads)):
@@ -1651,7 +1652,7 @@ def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, co
     _call("kvcm_mlstm_scan", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_in), gate_in.stride(0),
           _ptr(gate_keep), gate_keep.stride(0), _ptr(in_bias), _ptr(keep_bias), float(cap), float(q_scale), _ptr(coef), _ptr(n_new), _ptr(o),
           o.stride(0), _ptr(s_state), _ptr(n_state), _ptr(m_state), _ptr(step.run_start), _ptr(step.seq_start),
-          _ptr(step.state_slots), step.seqs, heads, dk, dv, T, int(step.max_run), _stream())
+          _ptr(step.state_slots), step.seqs, heads, dk, dv, T, int(step.max_run), int(one_order), _stream())
     return o
 
 

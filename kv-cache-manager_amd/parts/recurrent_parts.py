@@ -186,9 +186,10 @@ class MatrixMemoryMixer(_StatefulMixer):
         seqs = max(step.seqs, step.limits.max_seqs if step.limits is not None else step.seqs)
         n_new = step.flat("memory_normalizer", seqs * heads * d)
         o = step.ws("memory_o", (T, heads * dv), torch.float32)
-        ops.mlstm_scan(q, k, v, gi, gf, w["in_bias"], w["keep_bias"], p["gate_cap"], float(d) ** -0.5, coef, n_new, o,
-                       self.state("memory"), self.state("normalizer"), self.state("maximum"), step, heads, d, dv)
         gated = step.ws("memory_gated", (T, heads * dv))
+        ops.mlstm_scan(q, k, v, gi, gf, w["in_bias"], w["keep_bias"], p["gate_cap"], float(d) ** -0.5, coef, n_new, o,
+                       self.state("memory"), self.state("normalizer"), self.state("maximum"), step, heads, d, dv,
+                       one_order=gated.dtype == torch.float32)
         ops.head_norm_gate(o, g, w["norm"], gated, heads, dv, p["eps"])
         return linear32(self.ctx, step, gated, w["w_o"], "memory_out", keep_partial=True)      # the stream's next norm adds the slices
 

@@ -305,6 +305,32 @@ def test_matrix_memory_by_sizes_and_run_lengths(d, dv):
             row, at[i] = row + n, at[i] + n
 
 
+@pytest.mark.parametrize("d,dv", [(12, 5), (32, 32), (64, 64), (100, 9), (256, 8)])
+def test_matrix_memory_in_32_bits_depends_on_its_row_alone(d, dv):
+    """One sequence of 150 tokens whole, token by token, cut anywhere and beside seven others: the same bits."""
+    from kvcm_amd import ops
+    from test_kasuvik_gpu import _ONE, _all_equal, _rows_of_first
+    g = torch.Generator().manual_seed(d)
+    heads = 24 if d == 64 else 3      # (at 64 enough heads for eight sequences to fill the chip, too few for one)
+    q, k = (torch.randn(8, _ONE, heads * d, generator=g).to(DEV) for _ in range(2))
+    v = torch.randn(8, _ONE, heads * dv, generator=g).to(DEV)
+    gi, gf = (torch.randn(8, _ONE, heads, generator=g).to(DEV) * 4 + a for a in (0, 2))
+    bi, bf = torch.randn(heads, generator=g).to(DEV), torch.randn(heads, generator=g).to(DEV)
+
+    def run():
+        states = [torch.full(shape, 9.0, device=DEV) for shape in ((8, heads, d, dv), (8, heads, d), (8, heads))]
+
+        def call(step, *x):
+            if step is None:
+                return states
+            coef, o = torch.empty(step.rows, 4 * heads, device=DEV), torch.empty(step.rows, heads * dv, device=DEV)
+            ops.mlstm_scan(*x, bi, bf, 12.0, d ** -0.5, coef, torch.empty(step.seqs * heads * d, device=DEV), o, *states, step, heads, d, dv,
+                           one_order=True)
+            return o
+        return call
+    _all_equal(_rows_of_first(run, (q, k, v, gi, gf)))
+
+
 def test_matrix_memory_keeps_what_an_open_gate_wrote_long_ago():
     """A recurrence that reduces to a lookup: one early token is written with its input gate wide open while every other gate
     is shut, the forget gate keeps everything; 200 tokens later a query along that key reads its value back."""
