@@ -6,14 +6,18 @@
 //   y_c = sum_n S[c, n] * C_n + D_c * x_c;   out_c = y_c * silu(z_c)
 //
 // Everything of the recurrence is 32-bit: the state, the step size with its softplus, the decay's
-// exponential, the sums.  The states of a channel are spread over LPC lanes (a power of two, up to a whole
-// wave; NPL states a lane beyond that), so that a wave of 64 lanes walks 64 / LPC channels: the run's
+// exponential, the sums.  Runs are walked with the states of a channel spread over LPC lanes (a power of two, up to a
+// whole wave; NPL states a lane beyond that), so that a wave of 64 lanes walks 64 / LPC channels: the run's
 // tokens are taken in order, one exponential and two multiply-adds a lane and token, and the sum over a
-// channel's states crosses its lanes in a fixed tree.  What a token brings (its step size, input, gate, B
-// and C) does not depend on the state: it is requested a few tokens ahead, so that the walk waits for
-// arithmetic and not for memory.  A run that starts at position 0 starts from zero without reading its
-// slot; the state after the run's last token goes back to the slot.  Tokens are taken one by one in both
-// prompts and decoding, so a position's result does not depend on how the prompt was cut.
+// channel's states crosses its lanes in a fixed tree.  With 8 or 16 states, steps of single tokens and the pieces of
+// long runs have a channel's states in one lane instead; in 32-bit storage they are added in the same tree.
+// What a token brings (its step size, input, gate, B and C) does not depend on the state: it is requested a few
+// tokens ahead, so that the walk waits for arithmetic and not for memory.  A run that starts at position 0 starts from
+// zero without reading its slot; the state after the run's last token goes back to the slot.  Tokens are taken one by
+// one in prompts and in decoding, so in 32-bit storage a position's result does not depend on how the prompt was cut,
+// but for runs walked in pieces, where a piece's entering state comes by one multiply-add instead of one per token.
+#include <type_traits>
+
 #include "common.h"
 #include "kvcm_hip.h"
 
@@ -147,6 +151,16 @@ template <> __device__ __forceinline__ float scaled_exp<bf16_t>(float v) { retur
 
 constexpr int kScanTile = 64;      // tokens whose B and C lie in LDS
 
+// Sum over a channel's states in the order of group_sum, where the states lie over lanes: neighbours, pairs, fours, eights.
+template <int N>
+__device__ __forceinline__ float states_sum(float (&v)[N]) {
+#pragma unroll
+  for (int d = 1; d < N; d *= 2)
+#pragma unroll
+    for (int n = 0; n < N; n += 2 * d) v[n] += v[n + d];
+  return v[0];
+}
+
 // Runs of one token (decoding), a lane a channel with all its states: with the states over lanes a wave's four channels each
 // fetched their step size, input and gate sixteen times and asked for four tokens; 8 rows, 4,096 channels, 16 states: 14.5 us a
 // launch, 4.5 us so (2 MB of states read and written).
@@ -176,7 +190,7 @@ __global__ void __launch_bounds__(kWave)
   const float v = lin + (dt_bias ? dt_bias[c] : 0.f), skip = dskip[c];
   const float *b = bc + size_t(r) * ldbc + off_b, *cc = bc + size_t(r) * ldbc + off_c;
   const float dt = prepared ? lin : (v > 20.f ? v : log1pf(expf(v))), dx = dt * xx;
-  float y = 0.f;
+  float ys[N];
 #pragma unroll
   for (int n = 0; n < N / 4; ++n) {
     float se[4] = {sv[n].x, sv[n].y, sv[n].z, sv[n].w};
@@ -185,11 +199,11 @@ __global__ void __launch_bounds__(kWave)
     for (int e = 0; e < 4; ++e) {
       const float was = keep != 0.f ? se[e] : 0.f;      // (a first token starts from zero, whatever the slot holds)
       se[e] = fmaf(decay_exp<T>(dt * -expf(ae[e])), was, dx * b[4 * n + e]);
-      y = fmaf(se[e], cc[4 * n + e], y);
+      ys[4 * n + e] = fmaf(se[e], cc[4 * n + e], 0.f);      // (rounded before it is added, like a lane's own)
     }
     *reinterpret_cast<float4*>(at + 4 * n) = float4{se[0], se[1], se[2], se[3]};
   }
-  store_f(out + size_t(r) * ldo + c, fmaf(skip, xx, y) * (prepared ? zz : zz / (1.0f + expf(-zz))));
+  store_f(out + size_t(r) * ldo + c, fmaf(skip, xx, states_sum(ys)) * (prepared ? zz : zz / (1.0f + expf(-zz))));
 }
 
 template <class T, int N, bool OUT>
@@ -200,6 +214,7 @@ __global__ void __launch_bounds__(256)
                          const int* __restrict__ state_slots, int C, int chunk_len, float* __restrict__ carry,
                          float* __restrict__ dsum) {
   constexpr int U = 4, W = OUT ? 2 * N : N;
+  constexpr bool kOneOrder = std::is_same<T, float>::value;      // (32-bit results do not depend on how the states are dealt out)
   __shared__ __attribute__((aligned(16))) float tile[kScanTile][W];
   const int s = blockIdx.y, c_real = blockIdx.x * 256 + threadIdx.x;
   const bool owns = c_real < C;
@@ -241,12 +256,14 @@ __global__ void __launch_bounds__(256)
       const float step = dtv[from][u], dx = step * xv[from][u];
       const float* bt = tile[r - t0];
       dt_total += step;
-      float y = 0.f;
+      float y = 0.f, ys[N];
 #pragma unroll
       for (int n = 0; n < N; ++n) {
         S[n] = fmaf(scaled_exp<T>(step * A[n]), S[n], dx * bt[n]);
-        if (OUT) y = fmaf(S[n], bt[N + n], y);
+        if (OUT && kOneOrder) ys[n] = fmaf(S[n], bt[N + n], 0.f);
+        else if (OUT) y = fmaf(S[n], bt[N + n], y);
       }
+      if (OUT && kOneOrder) y = states_sum(ys);
       if (OUT && owns) store_f(out + size_t(r) * ldo + c, fmaf(skip, xv[from][u], y) * zv[from][u]);
     }
   };

@@ -463,6 +463,36 @@ def test_delta_rule_in_32_bits_depends_on_its_row_alone(d):
     _all_equal(_rows_of_first(run, (r, k, v, torch.sigmoid(w), torch.sigmoid(a) * u, u)))
 
 
+@pytest.mark.parametrize("C,N", [(70, 16), (300, 8), (20, 4), (33, 20)])
+def test_selective_scan_in_32_bits_depends_on_its_row_alone(C, N):
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(C)
+    x, z, dt = (torch.randn(8, _ONE, C, generator=g).to(DEV) for _ in range(3))
+    bc = torch.randn(8, _ONE, 2 * N, generator=g).to(DEV)
+    a_log, dsk, db = torch.rand(C, N, generator=g).to(DEV), torch.randn(C, generator=g).to(DEV), torch.randn(C, generator=g).to(DEV)
+
+    def run():
+        state = torch.full((8, C, N), 5.0, device=DEV)
+
+        def call(step, *p):
+            if step is None:
+                return [state]
+            x, z, dt, bc = (t.clone() for t in p)
+            out = torch.empty(step.rows, C, device=DEV)
+            return ops.selective_scan(x, dt, db, bc, 0, N, a_log, dsk, z, out, state, step, prepare=step.max_run >= 16)
+        return call
+    got = _rows_of_first(run, (x, z, dt, bc))
+    _all_equal(got)
+    # pieces that begin where the walk does: the first piece's rows, too
+    step = Step(_WHOLE[0])
+    step.max_run = _ONE
+    carry = torch.empty(ops.selective_scan_carry_floats(_ONE, 1, C, N), device=DEV)
+    out = torch.empty(_ONE, C, device=DEV)
+    ops.selective_scan(x[0].clone(), dt[0].clone(), db, bc[0], 0, N, a_log, dsk, z[0].clone(), out, torch.full((1, C, N), 5.0, device=DEV), step,
+                       prepare=True, carry=carry)
+    assert torch.equal(out[:ops.SCAN_PIECE], got[0][0][:ops.SCAN_PIECE])
+
+
 def test_gated_activations_and_scaled_embedding():
     from kvcm_amd import ops
     rng = np.random.default_rng(7)
