@@ -9,8 +9,9 @@
 // (window, causality, blocks wholly before the window) in the chunks at the ends of what the tile sees, so a chunk that some
 // rows of the tile do not see costs them nothing but zeros; a row's chunks and their order depend on its own position only.
 // Bound by its vector instructions: with P handed over through LDS, a row's statistics over 16 lanes, the mask at every score
-// and divisions by the page size this took 86 us for 2,048 rows of 32 heads of 64 in a window of 512 with pooled blocks (96 us
-// with capped scores by the exact tanh); 54 us (64 us) as it is, with the same error against 64 bits.  The first
+// and divisions by the page size this took 86 us for 2,048 rows of 32 heads of 64 in a window of 512 with pooled blocks,
+// 54 us as it is, with the same error against 64 bits (without pooled blocks 71 and 46 us, with capped scores 81 and 58 us).  The bound of four workgroups on a CU (128
+// registers) leaves heads of 64 with 76 bytes of scratch a lane.  The first
 // keep_first tokens of a sequence may stay visible beyond the window (chunks of their own, from token 0), and the
 // scores may be capped, score <- c tanh(score / c), and a bias that grows with the distance may be taken off them,
 // score <- score - slope_h * (i - j) with a slope per query head (tokens only: not beside pooled blocks); the output may be
@@ -44,14 +45,16 @@ __device__ __forceinline__ float quad_max(float v) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-// tanh for scores whose exponentials become bfloat16: its series up to 1/4 (three terms beyond x, off by less than 3e-7 of it),
-// 1 - 2 / (1 + e^(2x)) by the hardware's exp2 and reciprocal beyond (off by about 1e-7); the exact function is some thirty
-// instructions of a score's fifty.
+// tanh of a score: an odd polynomial up to 5/8 (x + x^3 p(x^2), p fitted to 4e-9 of the result), (1 - e) / (1 + e) with
+// e = 2^(-2 |x| log2 e) by the hardware's exp2 and reciprocal beyond.  As exact as tanhf, which is some thirty instructions of a
+// score's fifty: over [-12, 12] at most 1.6e-7 of the result off (tanhf 1.7e-7), 2.7e-8 on average up to 5/8 and 4e-8 beyond (the same).
 __device__ __forceinline__ float score_tanh(float x) {
   const float y = x * x;
-  const float near = x * fmaf(y, fmaf(y, fmaf(y, -0.0539682540f, 0.133333333f), -0.333333333f), 1.0f);
-  const float far = fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.88539008177792681f * x)), 1.0f);
-  return y < 0.0625f ? near : far;
+  const float p = fmaf(y, fmaf(y, fmaf(y, fmaf(y, -0.005704974f, 0.020639075f), -0.05373971f), 0.13331442f), -0.3333328f);
+  const float near = fmaf(x * y, p, x);
+  const float e = __builtin_amdgcn_exp2f(-2.88539008177792681f * fabsf(x));
+  const float far = copysignf(fmaf(-2.0f * e, __builtin_amdgcn_rcpf(1.0f + e), 1.0f), x);
+  return y < 0.390625f ? near : far;
 }
 
 // DP: key size padded to a multiple of 32; DVT: tiles of 16 value columns
@@ -184,7 +187,7 @@ __global__ void __launch_bounds__(256, DP <= 64 && DVT <= 4 ? 4 : DVT <= 8 ? 2 :
     const bool pooled = c < block_chunks, early = !pooled && c < head_chunks;
     const int c0 = chunk_start(c);
     if (!pooled && c == block_chunks) request_chunk(c);      // the first chunk of tokens: nobody asked for it yet
-    __syncthreads();      // the chunk before is done with Ks, Vt and Ps
+    __syncthreads();      // the chunk before is done with Ks and Vt
     if (pooled) {      // (loads from places clamped to the last block, masked afterwards)
       {
         pooled_four x[KQ][2];
