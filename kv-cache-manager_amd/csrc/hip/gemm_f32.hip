@@ -8,8 +8,9 @@
 // 16-byte load); the segments' sums are added in ascending order.  Against one chain over all of K this halves the error at K = 2048 (shorter chains).
 // (The reference has no 32-bit path; its GEMMs are cuBLAS calls with this same operand layout, src/model/llama.cpp:45-52.)
 //
-// Three kernels, by sizes:
-//   K <= 256    one chain over all of K (gemm_f32_short_kernel); the segments above are for longer sums.
+// By sizes:
+//   K <= 256    one chain over all of K in ascending order (the instruction takes its four k in ascending order, checked bit
+//               for bit); the segments above are for longer sums.  Tiles of 32 x 32 or 64 x 64.
 //   few rows    bound by reading W once.  A workgroup owns 16 columns, its waves one segment each, eight 16-byte loads of W a
 //               lane multiplied while the next eight are on their way; segments meet in LDS.  Two rows, K = 2048: N = 11264
 //               (92 MB) 22 us, 4.2 TB/s; N = 2048 8 us; K = 5632, N = 2048 20 us.  As 16 x 64 tiles of plain fused
@@ -141,7 +142,9 @@ __global__ void __launch_bounds__(kSegments* kWave)
 // ---- more rows: tiles of 32 TM x 32 TN, four waves of TM x TN instruction tiles each ----------------------------------------
 // LDS rows hold 32 k as eight 16-byte pieces, piece c of row r at place c ^ (r & 7): a wave's read of one piece of 16 rows
 // meets no bank twice.
-template <int TM, int TN, bool VEC>
+// ASCENDING: one chain over all of K instead, k after k: a piece's four elements then go to four pieces as they are staged, so
+// that lane group g's piece holds k = 4 m + g for m = 0..3.
+template <int TM, int TN, bool VEC, bool ASCENDING>
 __global__ void __launch_bounds__(256, 2)
     gemm_f32_tiles_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
                           int ldx, int ldw, int ldy) {
@@ -159,6 +162,9 @@ __global__ void __launch_bounds__(256, 2)
 #pragma unroll
   for (int p = 0; p < TN; ++p) wr[p] = W + size_t(n0 + srow + 32 * p < N ? n0 + srow + 32 * p : N - 1) * ldw;
   const int at = srow * 8 + (sc ^ (srow & 7));      // (rows 32 apart have the same place in a row)
+  int spread[4];                                    // ASCENDING: where a piece's elements go
+#pragma unroll
+  for (int e = 0; e < 4; ++e) spread[e] = 4 * (srow * 8 + (((sc & 4) + e) ^ (srow & 7))) + (sc & 3);
   f32x4 px[TM], pw[TN];
   auto fetch = [&](int k0) {
     if (VEC && k0 + BK <= K) {
@@ -173,11 +179,20 @@ __global__ void __launch_bounds__(256, 2)
       for (int p = 0; p < TN; ++p) pw[p] = load4<VEC>(wr[p], k0 + kc, K);
     }
   };
+  auto put = [&](f32x4* rows, int p, f32x4 v) {
+    if constexpr (ASCENDING) {
+      float* to = reinterpret_cast<float*>(rows);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) to[spread[e] + 1024 * p] = v[e];
+    } else {
+      rows[at + 256 * p] = v;
+    }
+  };
   auto stage = [&](int b) {
 #pragma unroll
-    for (int p = 0; p < TM; ++p) xs[b][at + 256 * p] = px[p];
+    for (int p = 0; p < TM; ++p) put(xs[b], p, px[p]);
 #pragma unroll
-    for (int p = 0; p < TN; ++p) ws[b][at + 256 * p] = pw[p];
+    for (int p = 0; p < TN; ++p) put(ws[b], p, pw[p]);
   };
   f32x4 acc[TM][TN], total[TM][TN];
 #pragma unroll
@@ -211,7 +226,7 @@ __global__ void __launch_bounds__(256, 2)
 #pragma unroll
           for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][m], w[j][m], acc[i][j], 0, 0, 0);
     }
-    if (--left == 0) {      // a segment ends
+    if (!ASCENDING && --left == 0) {      // a segment ends
       left = seg;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -228,7 +243,8 @@ __global__ void __launch_bounds__(256, 2)
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      if (left != seg) total[i][j] += acc[i][j];      // the last segment, where it is shorter
+      if (ASCENDING) total[i][j] = acc[i][j];
+      else if (left != seg) total[i][j] += acc[i][j];      // the last segment, where it is shorter
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int m = m0 + wm + 16 * i + 4 * g + e, n = n0 + wn + 16 * j + r;
@@ -237,68 +253,13 @@ __global__ void __launch_bounds__(256, 2)
     }
 }
 
-// ---- K up to 256: one chain over all of K ----------------------------------------------------------------------------------
-// These launches (models of small width, low-rank factors) are bound by their latency, so they are not cut: an element is one
-// chain of fused multiply-adds over k in ascending order.  The instruction takes its four k in ascending order (checked bit
-// for bit against such a chain), lane group g holding k = 4 s + g of step s.  A wave owns T x T tiles of 16 x 16, operands
-// straight from L2.  Three rows, K = 64: 7.5 us as 16 x 64 tiles staged through LDS, 3.9 us here.
+// K up to 256 (models of small width, low-rank factors): these launches are bound by their latency, so they are not cut.
 constexpr int kShortK = 256;
 
-template <int T>
-__global__ void __launch_bounds__(256)
-    gemm_f32_short_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
-                          int ldx, int ldw, int ldy) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int r = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.y * 16 * T, n0 = (blockIdx.x * 4 + wave) * 16 * T;
-  if (n0 >= N) return;
-  const float *x[T], *w[T];
-  f32x4 acc[T][T];
-#pragma unroll
-  for (int i = 0; i < T; ++i) {
-    x[i] = X + size_t(m0 + 16 * i + r < M ? m0 + 16 * i + r : M - 1) * ldx;
-    w[i] = W + size_t(n0 + 16 * i + r < N ? n0 + 16 * i + r : N - 1) * ldw;
-#pragma unroll
-    for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  constexpr int D = 16;      // steps whose loads are on their way together
-  for (int k0 = 0; k0 < K; k0 += 4 * D) {
-    float a[D][T], b[D][T];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int k = k0 + 4 * d + g;
-#pragma unroll
-      for (int i = 0; i < T; ++i) {
-        a[d][i] = x[i][k < K ? k : 0];
-        b[d][i] = w[i][k < K ? k : 0];
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const bool in = k0 + 4 * d + g < K;
-#pragma unroll
-      for (int i = 0; i < T; ++i)
-#pragma unroll
-        for (int j = 0; j < T; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a[d][i] : 0.f, in ? b[d][j] : 0.f, acc[i][j], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < T; ++i)
-#pragma unroll
-    for (int j = 0; j < T; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * i + 4 * g + e, n = n0 + 16 * j + r;
-        if (m < M && n < N) Y[size_t(m) * ldy + n] = acc[i][j][e];
-      }
-}
-
-template <int TM, int TN, bool VEC>
+template <int TM, int TN, bool VEC, bool ASCENDING>
 void launch_tiles(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t s) {
   const dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM));
-  gemm_f32_tiles_kernel<TM, TN, VEC><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+  gemm_f32_tiles_kernel<TM, TN, VEC, ASCENDING><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
 }
 
 template <bool VEC>
@@ -310,23 +271,24 @@ void launch_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int
   // 100 / 93 / 87), up to 16 always.  The larger tiles (half the columns' rows from L2) from three a CU on: 573 rows, N = 2048
   // 100 / 68 / 76, N = 11264 497 / 255 / 254, N = 32000 1441 / 705 / 660; 2048 rows, N = 11264: 1764 / 841 / 764
   // (124 TFLOP/s).  Tiles of 128 x 128 and 128 x 64 were never faster (290 and 303 at 573 rows, N = 11264).
+  // K up to 256: 32 x 32 tiles until 64 x 64 ones are one a CU.  K = 256, us, as 32 x 32 / 64 x 64 tiles: 64 x 2048 4.8 / 8.2,
+  // 300 x 2048 7.7 / 8.6, 128 x 8192 9.4 / 9.0, 1000 x 2048 16.6 / 13.7, 4000 x 2048 56 / 47 (90 TFLOP/s).  With operands straight from
+  // L2 into a wave's registers these took 33, 33, 34, 60 and 228 us, as plain fused multiply-adds from LDS 29, 29, 30, 33 and 81.
+  const long long few = (long long)((M + 63) / 64) * ((N + 31) / 32), large = (long long)((M + 63) / 64) * ((N + 63) / 64);
   if (K <= kShortK) {
-    const int t = M <= 16 ? 1 : 2;
-    const dim3 grid((N + 64 * t - 1) / (64 * t), (M + 16 * t - 1) / (16 * t));
-    if (t == 1) gemm_f32_short_kernel<1><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
-    else gemm_f32_short_kernel<2><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    if (large >= 256) launch_tiles<2, 2, VEC, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    else launch_tiles<1, 1, VEC, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
     return;
   }
-  const long long few = (long long)((M + 63) / 64) * ((N + 31) / 32), large = (long long)((M + 63) / 64) * ((N + 63) / 64);
   if (M <= 16 || few < (M <= 32 ? 600 : 228)) {
     const dim3 grid((N + 15) / 16, M <= 64 ? 1 : (M + 63) / 64);
     if (M <= 16) gemm_f32_rows_kernel<1, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
     else if (M <= 32) gemm_f32_rows_kernel<2, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
     else gemm_f32_rows_kernel<4, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
   } else if (large >= 704) {
-    launch_tiles<2, 2, VEC>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    launch_tiles<2, 2, VEC, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   } else {
-    launch_tiles<2, 1, VEC>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    launch_tiles<2, 1, VEC, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   }
 }
 

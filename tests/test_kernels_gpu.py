@@ -301,7 +301,7 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(ops):
 
 @pytest.mark.parametrize("N,K", [(64, 16), (130, 20), (300, 333), (2560, 2048), (520, 5632)])
 def test_gemm_f32_kernels_agree_bit_for_bit(ops, N, K):
-    # up to 16, 32 and 64 rows, tiles of 64 and of 128 (where those fill the chip): one sequence of operations for an element;
+    # up to 16, 32 and 64 rows, tiles of 64 x 32 and of 64 x 64 (where those fill the chip): one sequence of operations for an element;
     # in rows whose 16-byte pieces are aligned, and from an odd column on (single loads)
     rng = np.random.default_rng(N + K)
     M = 1700
@@ -320,6 +320,21 @@ def test_gemm_f32_kernels_agree_bit_for_bit(ops, N, K):
         assert torch.equal(part, full[40:40 + n]), n
         ops.gemm(x[40:40 + n, :K], w, part)
         assert torch.equal(part, full[40:40 + n]), n
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (5, 70, 3), (33, 40, 250), (16, 33, 256), (300, 65, 64), (1100, 1000, 37), (1030, 1025, 64)])
+def test_gemm_f32_of_short_rows_is_one_ascending_chain(ops, M, N, K):
+    # tiles of 32 x 32 and, from 256 of them on, of 64 x 64; rows of aligned pieces and from an odd column on
+    rng = np.random.default_rng(M + N + K)
+    x = _t(rng.normal(size=(M, K + 1)).astype(np.float32), torch.float32)
+    w = _t(rng.normal(size=(N, K)).astype(np.float32), torch.float32)
+    for rows in (x[:, :K].contiguous(), x[:, 1:]):
+        want = torch.zeros(M, N, device=DEV)
+        for k in range(K):      # a product of two 32-bit numbers is exact in 64 bits, and so is, nearly always, the rounding of the sum
+            want = (rows[:, k:k + 1].double() * w[:, k].double() + want.double()).float()
+        out = torch.zeros(M, N, device=DEV)
+        ops.gemm(rows, w, out)
+        assert torch.equal(out, want)
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
