@@ -91,27 +91,44 @@ __device__ __forceinline__ uint4 keep_first_bf16(uint4 v, int n) {
   return uint4{v.x & word(0), v.y & word(1), v.z & word(2), v.w & word(3)};
 }
 
-// Four values of a row of n from place i on, zero beyond its end.  FULL: the row is 16-byte aligned and nothing lies beyond;
-// WIDE: it is aligned, and n and i are multiples of four.  Loads are unconditional, from places clamped into the row, and
-// masked value by value afterwards (a branch around a load would make each wait for the one before).
-enum RowLoad : int { kRowSingle = 0, kRowWide = 1, kRowFull = 2 };
+// How a lane's entries of a row of n floats, four from place i on, are read.  kRowFull: nothing lies beyond the row.  kRowPart
+// (n >= 4): the four that end with the row where they would pass its end; entries before place i are then another lane's and not
+// `own`.  kRowWide: n is a multiple of four, the four are own or not as one.  kRowSingle: one by one, from places clamped
+// into the row.  Every entry read is one of the row's, so that a lane may compute with what is not its own (not finite there is
+// not finite for its owner either) and leave it out of sums and stores.  Rows may begin at any float: the hardware takes
+// 16-byte loads there.  (As four single loads, each with an address of its own, rows that are not 16-byte aligned took a walk
+// over 8 x 509 tokens of 32 heads of 64 from 215 to 1,595 us; 214 us so.)
+enum RowLoad : int { kRowSingle = 0, kRowPart = 1, kRowWide = 2, kRowFull = 3 };
 template <int HOW>
-__device__ __forceinline__ float4 load_four(const float* __restrict__ row, int i, int n) {
-  if constexpr (HOW == kRowFull) return *reinterpret_cast<const float4*>(row + i);
-  float4 x;
-  if constexpr (HOW == kRowWide) {
-    x = *reinterpret_cast<const float4*>(row + (i < n ? i : 0));
+__device__ __forceinline__ unsigned entry_place(unsigned i, unsigned e, unsigned n) {      // of entry e of the four, if it is own
+  if constexpr (HOW == kRowFull || HOW == kRowWide) return i + e;
+  if constexpr (HOW == kRowPart) return (i < n - 4 ? i : n - 4) + e;
+  return i + e < n ? i + e : n - 1;
+}
+template <int HOW>
+__device__ __forceinline__ bool entry_own(unsigned i, unsigned e, unsigned n) {
+  if constexpr (HOW == kRowFull) return true;
+  if constexpr (HOW == kRowPart) return entry_place<HOW>(i, e, n) >= i;
+  if constexpr (HOW == kRowWide) return i < n;
+  return i + e < n;
+}
+template <int HOW>
+__device__ __forceinline__ float4 load_four(const float* __restrict__ row, unsigned i, unsigned n) {
+  typedef float any_four __attribute__((ext_vector_type(4), aligned(4)));
+  if constexpr (HOW == kRowSingle) {
+    return float4{row[entry_place<HOW>(i, 0, n)], row[entry_place<HOW>(i, 1, n)], row[entry_place<HOW>(i, 2, n)], row[entry_place<HOW>(i, 3, n)]};
   } else {
-    x.x = row[i < n ? i : 0];
-    x.y = row[i + 1 < n ? i + 1 : 0];
-    x.z = row[i + 2 < n ? i + 2 : 0];
-    x.w = row[i + 3 < n ? i + 3 : 0];
+    const unsigned at = HOW == kRowWide && i >= n ? 0 : entry_place<HOW>(i, 0, n);      // (unsigned: one offset register)
+    const any_four x = *reinterpret_cast<const any_four*>(row + at);
+    return float4{x.x, x.y, x.z, x.w};
   }
-  x.x = i < n ? x.x : 0.f;
-  x.y = i + 1 < n ? x.y : 0.f;
-  x.z = i + 2 < n ? x.z : 0.f;
-  x.w = i + 3 < n ? x.w : 0.f;
-  return x;
+}
+// The same with zeros for what is not own.
+template <int HOW>
+__device__ __forceinline__ float4 load_own(const float* __restrict__ row, unsigned i, unsigned n) {
+  const float4 x = load_four<HOW>(row, i, n);
+  return float4{entry_own<HOW>(i, 0, n) ? x.x : 0.f, entry_own<HOW>(i, 1, n) ? x.y : 0.f, entry_own<HOW>(i, 2, n) ? x.z : 0.f,
+                entry_own<HOW>(i, 3, n) ? x.w : 0.f};
 }
 
 // Which head, and which of its column blocks, a workgroup of a walk over a matrix state takes (blockIdx.x of heads * col_blocks).

@@ -102,9 +102,9 @@ __global__ void __launch_bounds__(NT)
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int il = 0; il < IPT; ++il) {
-      const int i = g * IPT + il;
-      S[c][il] = (i < dk && owns[c] && !fresh) ? st[size_t(i) * dv + j[c]] : 0.f;
+    for (int il = 0; il < IPT; ++il) {      // (what is not own takes part from zero and is left out of sums and stores)
+      const int i = g * IPT + il / 4 * 4;
+      S[c][il] = (entry_own<HOW>(i, il % 4, dk) && owns[c] && !fresh) ? st[size_t(entry_place<HOW>(i, il % 4, dk)) * dv + j[c]] : 0.f;
     }
   static_assert(U <= G, "lane n of a column keeps token n's output until the U tokens are stored together");
   const size_t col = size_t(head) * dk;
@@ -117,11 +117,11 @@ __global__ void __launch_bounds__(NT)
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int i = g * IPT + 4 * q;
-      uv[n][q] = load_four<HOW>(up, i, dk);
+      uv[n][q] = load_own<HOW>(up, i, dk);      // (what is not own is left out of both sums)
       wv[n][q] = load_four<HOW>(wp, i, dk);
       av[n][q] = load_four<HOW>(ap, i, dk);
       kv[n][q] = load_four<HOW>(kp, i, dk);
-      rv[n][q] = load_four<HOW>(rp, i, dk);
+      rv[n][q] = load_own<HOW>(rp, i, dk);
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) vv[n][c] = vp[j[c]];
@@ -192,8 +192,8 @@ __global__ void __launch_bounds__(NT)
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int il = 0; il < IPT; ++il) {
-      const int i = g * IPT + il;
-      if (i < dk && owns[c]) st[size_t(i) * dv + j[c]] = S[c][il];
+      const int i = g * IPT + il / 4 * 4;
+      if (entry_own<HOW>(i, il % 4, dk) && owns[c]) st[size_t(entry_place<HOW>(i, il % 4, dk)) * dv + j[c]] = S[c][il];
     }
 }
 
@@ -232,8 +232,6 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
   KVCM_REQUIRE(static_cast<long long>(heads) * ((dv + 3) / 4) < (1ll << 31), "delta_scan: too many heads");
   KVCM_REQUIRE(S <= 65535, "delta_scan: too many sequences for one launch (%d)", S);
   KVCM_REQUIRE(ldr >= heads * dk && ldk >= heads * dk && ldv >= heads * dv && ldo >= heads * dv, "delta_scan: row strides too small");
-  auto aligned = [](const float* p, int ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; };
-  const bool wide = dk % 4 == 0 && aligned(r, ldr) && aligned(k, ldk) && aligned(w, 0) && aligned(au, 0) && aligned(u, 0);
 #define KVCM_DELTA_AS(DKP, G, NC, U, NT, HOW)                                                                                      \
   {                                                                                                                           \
     const int col_blocks = (dv + NT / G * NC - 1) / (NT / G * NC);                                                                      \
@@ -241,11 +239,11 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
                                                                                      state, run_start, seq_start,             \
                                                                                      state_slots, heads, dk, dv, col_blocks); \
   }
-#define KVCM_DELTA(DKP, G, NC, U, NT)                                 \
-  {                                                               \
-    if (wide && dk == DKP) KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowFull) \
-    else if (wide) KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowWide)         \
-    else KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowSingle)                 \
+#define KVCM_DELTA(DKP, G, NC, U, NT)                                  \
+  {                                                                \
+    if (dk == DKP) KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowFull)          \
+    else if (dk % 4 == 0) KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowWide)   \
+    else KVCM_DELTA_AS(DKP, G, NC, U, NT, kRowPart)                    \
   }
   // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
   // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 294 (16 lanes) / 374 and 261 (16 lanes; 8 lanes of two columns).
@@ -254,7 +252,8 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
   // tokens (8 rows, 32 heads of 128 x 128: 20 us, with 8 lanes and workgroups of 32 columns 14 us).
   const bool few = static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024;
   if (max_run >= 16) {
-    if (dk <= 16) KVCM_DELTA(16, 4, 1, 4, kWave)
+    if (dk < 4) KVCM_DELTA_AS(16, 4, 1, 4, kWave, kRowSingle)
+    else if (dk <= 16) KVCM_DELTA(16, 4, 1, 4, kWave)
     else if (dk <= 32) KVCM_DELTA(32, 8, 1, 4, kWave)
     else if (dk <= 64 && few && !one_order) KVCM_DELTA(64, 16, 1, 8, kWave)
     else if (dk <= 64 && few) KVCM_DELTA(64, 8, 1, 4, kWave)
@@ -262,7 +261,8 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
     else if (dk <= 128) KVCM_DELTA(128, 16, 1, 4, kWave)
     else KVCM_DELTA(256, 16, 1, 1, kWave)
   } else {
-    if (dk <= 16) KVCM_DELTA(16, 4, 1, 1, 128)
+    if (dk < 4) KVCM_DELTA_AS(16, 4, 1, 1, 128, kRowSingle)
+    else if (dk <= 16) KVCM_DELTA(16, 4, 1, 1, 128)
     else if (dk <= 32) KVCM_DELTA(32, 8, 1, 1, 256)
     else if (dk <= 64) KVCM_DELTA(64, 8, 1, 1, 256)
     else if (dk <= 128 && one_order) KVCM_DELTA(128, 16, 1, 1, 256)

@@ -153,10 +153,11 @@ __global__ void __launch_bounds__(NT)
   float S[NC][IPT], N[IPT];
 #pragma unroll
   for (int il = 0; il < IPT; ++il) {
-    const int i = g * IPT + il;
+    const int from = g * IPT + il / 4 * 4, i = entry_place<HOW>(from, il % 4, dk);
+    const bool own = entry_own<HOW>(from, il % 4, dk) && !fresh;      // (what is not takes part from zero and is left out of sums and stores)
 #pragma unroll
-    for (int c = 0; c < NC; ++c) S[c][il] = (i < dk && owns[c] && !fresh) ? st[size_t(i) * dv + j[c]] : 0.f;
-    N[il] = (i < dk && !fresh) ? nst[i] : 0.f;
+    for (int c = 0; c < NC; ++c) S[c][il] = (own && owns[c]) ? st[size_t(i) * dv + j[c]] : 0.f;
+    N[il] = own ? nst[i] : 0.f;
   }
   static_assert(U <= G, "lane n of a column keeps token n's sums until the U tokens are stored together");
   const size_t col = size_t(head) * dk;
@@ -170,7 +171,7 @@ __global__ void __launch_bounds__(NT)
     for (int p = 0; p < Q; ++p) {
       const int i = g * IPT + 4 * p;
       kv[n][p] = load_four<HOW>(kp, i, dk);
-      qv[n][p] = load_four<HOW>(qp, i, dk);
+      qv[n][p] = load_own<HOW>(qp, i, dk);      // (what is not own is left out of the sums)
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) vv[n][c] = vp[j[c]];
@@ -238,11 +239,12 @@ __global__ void __launch_bounds__(NT)
   }
 #pragma unroll
   for (int il = 0; il < IPT; ++il) {
-    const int i = g * IPT + il;
+    const int from = g * IPT + il / 4 * 4, i = entry_place<HOW>(from, il % 4, dk);
+    if (!entry_own<HOW>(from, il % 4, dk)) continue;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
-      if (i < dk && owns[c]) st[size_t(i) * dv + j[c]] = S[c][il];
-    if (i < dk && cb == 0 && threadIdx.x < G) n_new[(size_t(s) * heads + head) * dk + i] = N[il];
+      if (owns[c]) st[size_t(i) * dv + j[c]] = S[c][il];
+    if (cb == 0 && threadIdx.x < G) n_new[(size_t(s) * heads + head) * dk + i] = N[il];
   }
 }
 
@@ -291,8 +293,6 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
   auto* maxima = one_order ? mlstm_max_kernel<true> : mlstm_max_kernel<false>;
   maxima<<<S * heads, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, heads,
                                      logs_first);
-  auto aligned = [](const float* p, int ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; };
-  const bool wide = dk % 4 == 0 && aligned(q, ldq) && aligned(k, ldk);
 #define KVCM_MLSTM_AS(DKP, G, NC, U, NT, HOW)                                                                                    \
   {                                                                                                                          \
     const int col_blocks = (dv + NT / G * NC - 1) / (NT / G * NC);                                                                     \
@@ -301,11 +301,11 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
                                                                                      seq_start, state_slots, heads, dk, dv,  \
                                                                                      col_blocks);                            \
   }
-#define KVCM_MLSTM(DKP, G, NC, U, NT)                                 \
-  {                                                               \
-    if (wide && dk == DKP) KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowFull) \
-    else if (wide) KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowWide)         \
-    else KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowSingle)                 \
+#define KVCM_MLSTM(DKP, G, NC, U, NT)                                  \
+  {                                                                \
+    if (dk == DKP) KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowFull)          \
+    else if (dk % 4 == 0) KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowWide)   \
+    else KVCM_MLSTM_AS(DKP, G, NC, U, NT, kRowPart)                    \
   }
   // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
   // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 292 (16 lanes) / 247 and 217 (16 lanes; 8 lanes of two columns).
@@ -313,7 +313,8 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
   // 64: 394 us for the one sequence).
   const bool few = static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024;
   if (max_run >= 16) {
-    if (dk <= 16) KVCM_MLSTM(16, 4, 1, 4, kWave)
+    if (dk < 4) KVCM_MLSTM_AS(16, 4, 1, 4, kWave, kRowSingle)
+    else if (dk <= 16) KVCM_MLSTM(16, 4, 1, 4, kWave)
     else if (dk <= 32) KVCM_MLSTM(32, 8, 1, 4, kWave)
     else if (dk <= 64 && few && !one_order) KVCM_MLSTM(64, 16, 1, 8, kWave)
     else if (dk <= 64 && few) KVCM_MLSTM(64, 8, 1, 8, kWave)
@@ -321,7 +322,8 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
     else if (dk <= 128) KVCM_MLSTM(128, 16, 1, 6, kWave)
     else KVCM_MLSTM(256, 16, 1, 4, kWave)
   } else {
-    if (dk <= 16) KVCM_MLSTM(16, 4, 1, 1, 128)
+    if (dk < 4) KVCM_MLSTM_AS(16, 4, 1, 1, 128, kRowSingle)
+    else if (dk <= 16) KVCM_MLSTM(16, 4, 1, 1, 128)
     else if (dk <= 32) KVCM_MLSTM(32, 8, 1, 1, 256)
     else if (dk <= 64) KVCM_MLSTM(64, 8, 1, 1, 256)
     else if (dk <= 128) KVCM_MLSTM(128, 16, 1, 1, 256)

@@ -331,6 +331,28 @@ def test_matrix_memory_in_32_bits_depends_on_its_row_alone(d, dv):
     _all_equal(_rows_of_first(run, (q, k, v, gi, gf)))
 
 
+@pytest.mark.parametrize("d", [1, 3, 6, 16, 18, 32, 62, 64, 100, 128, 130, 160, 256])
+def test_matrix_memory_rows_may_begin_at_any_float(d):
+    """The projections as columns of one product whose rows are no multiple of 16 bytes: the bits of rows of their own."""
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(d)
+    heads, dv, lengths = 2, 5, (40, 1, 17)
+    D, st = heads * d, Step([(i, 0, n) for i, n in enumerate((40, 1, 17))])
+    proj = torch.randn(st.rows, 2 * D + 2 * heads + heads * dv + 2, generator=g).to(DEV)[:, 1:]
+    at = [0, D, 2 * D, 2 * D + heads * dv, 2 * D + heads * dv + heads, 2 * D + heads * dv + 2 * heads]
+    parts = [proj[:, a:b] for a, b in zip(at, at[1:])]
+    b = torch.zeros(heads, device=DEV)
+    for max_run in (40, 1):      # (the lanes of long runs and of single tokens)
+        st.max_run = max_run
+        got = []
+        for rows in (parts, [x.contiguous() for x in parts]):
+            states = [torch.zeros(shape, device=DEV) for shape in ((3, heads, d, dv), (3, heads, d), (3, heads))]
+            coef, o = torch.empty(st.rows, 4 * heads, device=DEV), torch.empty(st.rows, heads * dv, device=DEV)
+            ops.mlstm_scan(*rows, b, b, 12.0, d ** -0.5, coef, torch.empty(3 * D, device=DEV), o, *states, st, heads, d, dv)
+            got.append([o] + states)
+        assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
 def test_matrix_memory_keeps_what_an_open_gate_wrote_long_ago():
     """A recurrence that reduces to a lookup: one early token is written with its input gate wide open while every other gate
     is shut, the forget gate keeps everything; 200 tokens later a query along that key reads its value back."""

@@ -463,6 +463,29 @@ def test_delta_rule_in_32_bits_depends_on_its_row_alone(d):
     _all_equal(_rows_of_first(run, (r, k, v, torch.sigmoid(w), torch.sigmoid(a) * u, u)))
 
 
+@pytest.mark.parametrize("d", [1, 3, 6, 16, 18, 32, 62, 64, 100, 128, 130, 160, 256])
+def test_delta_rule_rows_may_begin_at_any_float(d):
+    """The projections as columns of one product whose rows are no multiple of 16 bytes: the bits of rows of their own."""
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(d)
+    heads, lengths = 2, (40, 1, 17)
+    D, step = heads * d, Step([(i, 0, n) for i, n in enumerate(lengths)])
+    proj = torch.randn(step.rows, 3 * D + 2 + 3 * D % 2, generator=g).to(DEV)[:, 1:]
+    u = torch.nn.functional.normalize(proj[:, D:2 * D].reshape(-1, heads, d), dim=-1).reshape(-1, D).contiguous()
+    w, au = torch.rand(step.rows, D, generator=g).to(DEV), 0.5 * u
+    got = []
+    for max_run in (40, 1):      # (the lanes of long runs and of single tokens)
+        step.max_run = max_run
+        for r, k, v in ([proj[:, i * D:(i + 1) * D] for i in range(3)], [proj[:, i * D:(i + 1) * D].contiguous() for i in range(3)]):
+            state, o = torch.zeros(3, heads, d, d, device=DEV), torch.empty(step.rows, D, device=DEV)
+            got.append((ops.delta_scan(r, k, v, w, au, u, o, state, step, heads, d, d), state))
+        assert torch.equal(got[-1][0], got[-2][0]) and torch.equal(got[-1][1], got[-2][1])
+    want = plain.delta_rule(*(x.double().cpu().numpy()[:40].reshape(40, heads, d) for x in (proj[:, :D], proj[:, D:2 * D], proj[:, 2 * D:3 * D], w)),
+                            np.full((40, heads, d), 0.5))
+    for o, _ in got:      # (plain: unit keys with 1e-6 beside the sum of squares, 1e-6 of a key of length one and less of longer ones)
+        np.testing.assert_allclose(o[:40].cpu().numpy().reshape(40, heads, d), want, atol=1e-4 * max(1.0, np.abs(want).max()))
+
+
 @pytest.mark.parametrize("C,N", [(70, 16), (300, 8), (20, 4), (33, 20)])
 def test_selective_scan_in_32_bits_depends_on_its_row_alone(C, N):
     from kvcm_amd import ops
