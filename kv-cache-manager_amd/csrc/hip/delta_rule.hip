@@ -250,6 +250,8 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
   // The lanes of a column are the order of its sums.  With one_order (32-bit storage, where a row's result depends on that row
   // alone) they follow from the key size, whatever the runs: 8 lanes from 33 to 64, 405 / 211 us; 16 beyond, also for single
   // tokens (8 rows, 32 heads of 128 x 128: 20 us, with 8 lanes and workgroups of 32 columns 14 us).
+  // Beyond 128 a wave of four columns is bound by fetching the vectors, which each column needs whole: 8 x 509 tokens, 8 heads of
+  // 256 x 256 2,335 us, 1,330 us with two columns a lane (1,850 as workgroups of 16 columns that shared them through LDS).
   const bool few = static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024;
   if (max_run >= 16) {
     if (dk < 4) KVCM_DELTA_AS(16, 4, 1, 4, kWave, kRowSingle)
@@ -259,7 +261,8 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
     else if (dk <= 64 && few) KVCM_DELTA(64, 8, 1, 4, kWave)
     else if (dk <= 64) KVCM_DELTA(64, 8, 2, 4, kWave)
     else if (dk <= 128) KVCM_DELTA(128, 16, 1, 4, kWave)
-    else KVCM_DELTA(256, 16, 1, 1, kWave)
+    else if (few) KVCM_DELTA(256, 16, 1, 1, kWave)
+    else KVCM_DELTA(256, 16, 2, 1, kWave)
   } else {
     if (dk < 4) KVCM_DELTA_AS(16, 4, 1, 1, 128, kRowSingle)
     else if (dk <= 16) KVCM_DELTA(16, 4, 1, 1, 128)

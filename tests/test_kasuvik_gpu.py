@@ -447,7 +447,7 @@ def _all_equal(got):
 def test_delta_rule_in_32_bits_depends_on_its_row_alone(d):
     from kvcm_amd import ops
     g = torch.Generator().manual_seed(d)
-    heads = 24 if d == 64 else 3      # (at 64 enough heads for eight sequences to fill the chip, too few for one)
+    heads = {64: 24, 256: 5}.get(d, 3)      # (at 64 and 256 enough for eight sequences to fill the chip, too few for one)
     r, k, v, w, a = (torch.randn(8, _ONE, heads * d, generator=g).to(DEV) for _ in range(5))
     u = torch.nn.functional.normalize(k.view(8, _ONE, heads, d), dim=-1).reshape(8, _ONE, heads * d)
 
