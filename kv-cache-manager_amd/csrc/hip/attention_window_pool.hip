@@ -24,7 +24,9 @@
 // Waves per row and query head, or group of query heads; blocks are walked 64 at a time from block 0, tokens 64 at a time in
 // chunks that start at absolute multiples of 64, with a running maximum: a row's result is a fixed
 // sequence of operations on its own keys, whatever else the launch holds and whichever pages it reads.
+#include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 #include "common.h"
 #include "kvcm_hip.h"
@@ -178,16 +180,15 @@ __global__ void __launch_bounds__(256)
 
 // ------------------------------------------------------------------- pooled entries of a step
 // A row whose position is the last of a block of P makes that block's entry from the pages.  A wave looks at R rows (one of
-// them, in a run, ends a block where R <= P) and makes keys or values (blockIdx.z) of one kv head, 32 tokens' pages, then their
+// them, in a run, ends a block where R <= P) and makes keys or values (blockIdx.z) of one kv head, AHEAD tokens' pages, then their
 // values, requested before the first is added, in order.  A workgroup per row that waited for every token's value in turn took
 // 86 us for a prompt of 2,048 tokens in blocks of 64, four heads of 64; 13 us so.
-template <class T>
+template <class T, int AHEAD>
 __global__ void __launch_bounds__(kWave)
     pool_update_kernel(const T* __restrict__ kcache, const T* __restrict__ vcache, float* __restrict__ pk,
                        float* __restrict__ pv, const int* __restrict__ tables, int table_stride,
                        const int* __restrict__ row_seq, const int* __restrict__ positions, const int* __restrict__ slots,
                        int rows, int R, int nkv, int d, int dv, int B, int P, int E) {
-  constexpr int AHEAD = 32;
   const int kvh = blockIdx.y, lane = threadIdx.x, row0 = blockIdx.x * R;
   const bool keys = blockIdx.z == 0;
   const int mine = row0 + lane < rows ? row0 + lane : rows - 1;
@@ -806,14 +807,20 @@ int kvcm_pool_update(const void* kcache, const void* vcache, int dtype, float* p
   KVCM_REQUIRE(T > 0 && nkv > 0 && d > 0 && dv > 0 && B > 0, "pool_update: bad sizes");
   KVCM_REQUIRE(E == (B + P - 1) / P, "pool_update: %d entries a page do not fit pages of %d and blocks of %d", E, B, P);
   KVCM_REQUIRE(nkv <= 65535, "pool_update: too many kv heads");
-  const int R = T <= kWave ? 1 : P < kWave ? P : kWave;      // (decoding requests may all end a block in one step: a wave each)
+  // Rows a wave.  In a run at most one of them ends a block where R <= P, and few waves look at many rows; but requests that
+  // decode in step may all end one, and a wave makes its entries one after the other.  Growing with the rows, both stay below
+  // what a workgroup per row takes.  Blocks of 64, 4 kv heads of 64, us, this / a row each / 64 rows each: a prompt of 2,048
+  // 11.5 / 64 / 11.5, 8 of 2,048 17 / 475 / 17; 128 rows that all end a block 11.6 / 11.6 / 660, 512 such rows 40 / 34 / 615.
+  const int R = T < 256 ? 1 : std::min({T / 128, P, kWave});
   const dim3 grid((T + R - 1) / R, nkv, 2);      // keys, values
-  if (dtype == kF32)
-    pool_update_kernel<float><<<grid, kWave, 0, s>>>(static_cast<const float*>(kcache), static_cast<const float*>(vcache), pk,
-                                                      pv, tables, table_stride, row_seq, positions, slots, T, R, nkv, d, dv, B, P, E);
-  else if (dtype == kBF16)
-    pool_update_kernel<bf16_t><<<grid, kWave, 0, s>>>(static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache),
-                                                       pk, pv, tables, table_stride, row_seq, positions, slots, T, R, nkv, d, dv, B, P, E);
+  // (short blocks do not ask for many more tokens than they have: blocks of 8, 64 rows that end one, 7.0 us as 32 ahead, 3.7 as 8)
+  auto launch = [&](auto* kc, auto* vc) {
+    using T_ = std::remove_const_t<std::remove_pointer_t<decltype(kc)>>;
+    auto* kernel = P <= 8 ? pool_update_kernel<T_, 8> : P <= 16 ? pool_update_kernel<T_, 16> : pool_update_kernel<T_, 32>;
+    kernel<<<grid, kWave, 0, s>>>(kc, vc, pk, pv, tables, table_stride, row_seq, positions, slots, T, R, nkv, d, dv, B, P, E);
+  };
+  if (dtype == kF32) launch(static_cast<const float*>(kcache), static_cast<const float*>(vcache));
+  else if (dtype == kBF16) launch(static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache));
   else KVCM_REQUIRE(false, "pool_update: unknown dtype %d", dtype);
   return launch_status("pool_update");
 }

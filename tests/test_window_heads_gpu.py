@@ -89,3 +89,36 @@ def test_heads_together(s):
     t = rows[-1]
     vc[order[t // B], :, 0, t % B] = float("inf")
     assert torch.isinf(run(nh * d, [len(rows) - 1]).reshape(nh, dv)[:, 0]).all()
+
+
+@pytest.mark.parametrize("P", [1, 5, 8, 13, 16, 17, 40, 64])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_pooled_entries_of_many_rows(P, dtype):
+    """Rows that all end a block, runs, and rows without a slot, in numbers whose waves look at one row or several: the mean of
+    every block that ends, in ascending order, and nothing else."""
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(P)
+    nkv, d, dv, B, per = 2, 6, 70, 8, 3 * P
+    pages = -(-per // B)
+    for n, run in ((3, 1), (255, 1), (256, 1), (700, 1), (30, per)):
+        kc = torch.randn(n * pages, nkv, B, d, generator=g).to(dtype).to(DEV)
+        vc = torch.randn(n * pages, nkv, dv, B, generator=g).to(dtype).to(DEV)
+        E = -(-B // P)
+        pk, pv = torch.full((n * pages, nkv, E, d), 7.0, device=DEV), torch.full((n * pages, nkv, E, dv), 7.0, device=DEV)
+        table = torch.randperm(n * pages, generator=g).to(torch.int32).reshape(n, pages)
+        rows = [(s, p) for s in range(n) for p in (range(run) if run > 1 else [2 * P - 1])]
+        slots = [-1 if i % 5 == 3 else int(table[s, p // B]) * B + p % B for i, (s, p) in enumerate(rows)]
+        i32 = lambda x: torch.as_tensor(x, dtype=torch.int32).to(DEV)
+        ops.pool_update(kc, vc, pk, pv, table.to(DEV), pages, i32([s for s, _ in rows]), i32([p for _, p in rows]), i32(slots), nkv, d, dv, P, len(rows))
+        wk, wv = torch.full_like(pk, 7.0), torch.full_like(pv, 7.0)
+        k = kc[table.to(DEV).long()].permute(0, 2, 1, 3, 4).reshape(n, nkv, pages * B, d).float()      # by sequence and position
+        v = vc[table.to(DEV).long()].permute(0, 2, 3, 1, 4).reshape(n, nkv, dv, pages * B).float()
+        ends = [(s, p, slot // B) for (s, p), slot in zip(rows, slots) if slot >= 0 and (p + 1) % P == 0]
+        for p in sorted({p for _, p, _ in ends}):
+            s, page = (torch.tensor(x, device=DEV) for x in zip(*[(s, page) for s, q, page in ends if q == p]))
+            entry = p // P - p // B * B // P
+            ak, av = torch.zeros(len(s), nkv, d, device=DEV), torch.zeros(len(s), nkv, dv, device=DEV)
+            for t in range(p - P + 1, p + 1):
+                ak, av = ak + k[s, :, t], av + v[s, :, :, t]
+            wk[page, :, entry], wv[page, :, entry] = ak * torch.tensor(1.0 / P, device=DEV), av * torch.tensor(1.0 / P, device=DEV)
+        assert torch.equal(pk, wk) and torch.equal(pv, wv), (n, run)
