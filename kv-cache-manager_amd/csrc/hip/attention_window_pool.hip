@@ -454,7 +454,7 @@ __global__ void __launch_bounds__(kWpWaves* kWave)
 // query head above, whose dots and sums over values are a thousand vector instructions for each chunk and head and which reads
 // the keys once per head, took 19.0 us a step of 8 rows of 32 heads over 4 kv heads of 64 in a window of 512 (sixteen waves in
 // place of four: 14.5 us), this 12.2 us; 1,100 such rows at once 814 us then, 137 us now; heads of 128 over 8 kv heads in a
-// window of 1,024 with pooled blocks 29.7 us then, 24.8 us now.
+// window of 1,024 with pooled blocks 29.7 us then, 24.8 us now (at 128 the fragments leave 144 bytes of scratch a lane).
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 typedef float any_four __attribute__((ext_vector_type(4), aligned(4)));      // (pooled entries may lie at any float)
@@ -846,9 +846,12 @@ int kvcm_attention_window_pool(const void* q, int dtype, int ldq, void* out, int
   const long long blocks = static_cast<long long>(T) * nh;
   KVCM_REQUIRE(blocks < (1ll << 31), "attention_window_pool: too many rows");
   // heads together where 16-byte loads fit rows and pages and a wave's sums and fragments fit its registers (at 256 values they
-  // do not); faster at every number of rows measured, from 8 (19.0 to 12.2 us) to 1,500 (2,108 to 696 us).  The rule looks at
-  // sizes and places alone, never at the rows: a row's bits do not depend on what else the launch holds.
-  if (dtype == kBF16 && d % 8 == 0 && d <= 128 && dv % 8 == 0 && dv <= 128 && B % 8 == 0 && ldq % 8 == 0 &&
+  // do not), from two query heads a kv head on; us, a workgroup per row and head / heads together, window 512, heads of 64:
+  //   8 per kv head, 8 / 64 / 1,000 rows of 600 tokens: 17 / 10, 74 / 12, 894 / 136; of 64 tokens 7.8 / 6.9, 29 / 7, 376 / 80
+  //   2 per kv head (16 in all): 15.6 / 10.0, 40 / 23, 452 / 260; 7.7 / 6.7, 14.5 / 11.7, 192 / 151
+  //   1 per kv head (32): 17.2 / 11.8, 80 / 80, 894 / 1,005; 7.8 / 6.9, 28.5 / 41, 376 / 581: one column of sixteen does the work
+  // The rule looks at sizes and places alone, never at the rows: a row's bits do not depend on what else the launch holds.
+  if (dtype == kBF16 && nh / nkv >= 2 && d % 8 == 0 && d <= 128 && dv % 8 == 0 && dv <= 128 && B % 8 == 0 && ldq % 8 == 0 &&
       (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kcache) | reinterpret_cast<uintptr_t>(vcache)) % 16 == 0 &&
       nkv * ((nh / nkv + 15) / 16) <= 65535) {
     const dim3 grid(T, nkv * ((nh / nkv + 15) / 16));
