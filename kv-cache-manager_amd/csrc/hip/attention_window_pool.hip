@@ -463,10 +463,10 @@ typedef float any_four __attribute__((ext_vector_type(4), aligned(4)));      // 
 __device__ __forceinline__ uint32_t upper_halves(float a, float b) {
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-// what a probability's upper half leaves of it, or the least bfloat16 (nothing beside any value, but times an infinite value
-// it is not the NaN that zero would make)
+// what a probability's upper half leaves of it, or, where that is nothing of a probability above zero, the least bfloat16
+// (nothing beside the rest of it, but times an infinite value it is not the NaN that zero would make)
 __device__ __forceinline__ float below_upper(float x) {
-  return fmaxf(x - __uint_as_float(__float_as_uint(x) & 0xFFFF0000u), 1.17549435e-38f);
+  return fmaxf(x - __uint_as_float(__float_as_uint(x) & 0xFFFF0000u), fminf(x, 1.17549435e-38f));
 }
 
 // largest / sum of the four lanes that share lane % 16

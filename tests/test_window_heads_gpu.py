@@ -91,6 +91,21 @@ def test_heads_together(s):
     assert torch.isinf(run(nh * d, [len(rows) - 1]).reshape(nh, dv)[:, 0]).all()
 
 
+@pytest.mark.parametrize("nh,nkv", [(4, 1), (2, 2)])
+def test_a_probability_of_zero_takes_nothing_of_its_value(nh, nkv):
+    # one key whose score lies so far below the others' that its probability is zero in 32 bits, with a value near the largest
+    from kvcm_amd import ops
+    T, B, d = 40, 8, 64
+    kc, vc = torch.zeros(5, nkv, B, d, dtype=torch.bfloat16), torch.ones(5, nkv, d, B, dtype=torch.bfloat16)
+    kc[2, :, 3, 0], vc[2, :, :, 3] = -200.0, 1e38
+    q = torch.zeros(1, nh * d, dtype=torch.bfloat16)
+    q[0, ::d] = 1.0
+    out = torch.zeros(1, nh * d, dtype=torch.bfloat16, device=DEV)
+    i32 = lambda x: torch.as_tensor(x, dtype=torch.int32).to(DEV)
+    ops.attention_window_pool(q.to(DEV), out, kc.to(DEV), vc.to(DEV), None, None, i32(range(5)), 5, i32([0]), i32([T]), nh, nkv, d, d, 1.0, 0, 0)
+    assert (out == 1.0).all()
+
+
 @pytest.mark.parametrize("P", [1, 5, 8, 13, 16, 17, 40, 64])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_pooled_entries_of_many_rows(P, dtype):
