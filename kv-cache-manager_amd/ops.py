@@ -568,12 +568,17 @@ def skinny_splits(M, N, K):
 
 
 def _rows8_takes(M, N, K):
-    """Whether a product of at most 8 rows that nobody adds slices of runs unsplit (gemm_rows8.hip) instead of split along K
-    with a second launch that adds the slices up.  Measured (us, split and added / unsplit; 8 rows): N 2048, K 2048 8.8 / 4.1;
-    8192 x 2048 14.9 / 8.6; 2048 x 4096 10.6 / 6.9; 2048 x 5632 12.3 / 9.6; 11264 x 2048 17.7 / 12.4; 4096 x 8192 19.1 / 17.7;
-    32000 x 2048 28.6 / 27.5; beyond that each of its many short workgroups reads all rows again: 16384 x 4096 28.2 / 32.1,
-    28672 x 4096 48.9 / 52.6 (one row: 28.4 / 27.7 and 47.8 / 43.7)."""
-    return M <= FUSED_NORM_MAX_ROWS and (M <= 2 or N * K <= 66_000_000) and gemm8_supported(M, N, K)
+    """Whether a product of at most 8 rows that nobody adds slices of runs unsplit in workgroups of 8 or 16 columns
+    (gemm_rows8.hip).  What speaks for it is the second launch, which adds the slices that the other kernels split K into, and
+    short chains; against it, that each workgroup reads all rows again and lives for one pass over K, so that many columns of few k
+    are many short workgroups.  Measured (us, otherwise / so; 8 rows): N 2048, K 2048 8.8 / 4.1; 8192 x 2048 14.9 / 8.6; 2048 x 4096
+    10.6 / 6.9; 2048 x 5632 12.3 / 9.6; 11264 x 2048 17.7 / 12.4; 4096 x 8192 19.1 / 17.7; 32000 x 2048 28.8 / 28.0 (a head, which is
+    not split); 50000 x 1024 25.7 / 22.0; more weights than that 16384 x 4096 28.2 / 32.1, 28672 x 4096 48.9 / 52.6 (one row: 28.4 /
+    27.7 and 47.8 / 43.7); fewer k: 8192 x 512 even, 32000 x 512 10.1 / 13.1, 128000 x 512 33.5 / 45.0 (one row 32.1 / 35.0), 50272 x
+    768 20.2 / 21.0; with an odd multiple of 8 columns, where a workgroup has 8 and the other way is the general kernel: 8200 x
+    512 9.6 / 10.7, 16392 x 1024 21.1 / 18.0, 32008 x 1024 25.3 / 30.6, 32008 x 2048 46.9 / 33.2."""
+    return (M <= FUSED_NORM_MAX_ROWS and (M <= 2 or N * K <= 66_000_000) and (N <= 8192 or K >= (1024 if N % 16 == 0 else 2048))
+            and gemm8_supported(M, N, K))
 
 
 def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False):

@@ -338,6 +338,29 @@ def test_gemm_f32_of_short_rows_is_one_ascending_chain(ops, M, N, K):
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K", [(40, 192), (520, 1024), (8200, 512), (8208, 512), (8200, 1024), (16392, 2048), (16384, 4096), (50, 128), (64, 100)])
+def test_gemm_bf16_unsplit(ops, N, K, out_dtype):
+    # both sides of the rule for products that nobody adds slices of: unsplit, split and added, the general kernel; rows at
+    # a stride, rows and weights that are not 16-byte aligned
+    g = torch.Generator().manual_seed(N + K)
+    w = torch.randn(N + 1, K + 8, generator=g).to(torch.bfloat16).to(DEV)
+    xs = torch.randn(9, K + 24, generator=g).to(torch.bfloat16).to(DEV)
+    for M in (1, 2, 3, 8, 9):
+        scratch = torch.empty(64 * M * N, device=DEV)
+        for x, ww in ((xs[:M, :K].contiguous(), w[:N, :K].contiguous()), (xs[:M, 8:8 + K], w[1:, 8:]), (xs[:M, 1:1 + K], w[:N, :K]), (xs[:M, :K], w[:N, 3:3 + K])):
+            want = x.double() @ ww.double().t()
+            # 32-bit sums of K products in some order (a random walk, six deviations), rounded to the result's type once
+            bound = 6 * 2.0 ** -24 * K + (2.0 ** -8 * want.abs() if out_dtype == torch.bfloat16 else 2.0 ** -23 * want.abs())
+            for kw in (dict(), dict(scratch=scratch), dict(scratch=scratch, keep_partial=True)):
+                out = torch.full((M, N + 3), 7.0, dtype=out_dtype, device=DEV)[:, :N]
+                got = ops.gemm(x, ww, out, unsplit=True, tuning="off", **kw)
+                if not torch.is_tensor(got):
+                    assert kw.get("keep_partial")
+                    got = got.materialize()
+                assert ((got.double() - want).abs() <= bound).all(), (M, kw)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (5, 100, 96), (64, 64, 64), (70, 176, 200), (200, 333, 1024), (3, 50, 20)])
 def test_gemm_bf16_equals_x_wT(ops, M, N, K, out_dtype):
     rng = np.random.default_rng(M * 1000 + N)
