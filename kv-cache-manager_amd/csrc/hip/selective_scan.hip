@@ -329,28 +329,33 @@ __global__ void __launch_bounds__(256)
   z[size_t(r) * ldz + c] = zz / (1.0f + expf(-zz));
 }
 
-template <class T>
+template <class X>
 int launch_scan(const void* x, int ldx, const float* dt_lin, int lddt, const float* dt_bias, const float* bc, int ldbc,
                 int off_b, int off_c, const float* a_log, const float* dskip, const float* z, int ldz, void* out, int ldo,
                 float* state, const int* run_start, const int* seq_start, const int* state_slots, int S, int C, int N,
-                int prepared, int phase, int chunk_len, int pieces, int max_run, float* carry, float* dsum, hipStream_t s) {
+                int prepared, int phase, int chunk_len, int pieces, int max_run, int T, float* carry, float* dsum, hipStream_t s) {
   auto aligned = [](const float* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (phase == 0 && max_run == 1 && (N == 8 || N == 16) && aligned(state) && aligned(a_log)) {
     const dim3 grid((C + kWave - 1) / kWave, S);
 #define KVCM_SCAN_SINGLE(N)                                                                                                    \
-  scan_single_kernel<T, N><<<grid, kWave, 0, s>>>(static_cast<const T*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, \
-                                                  a_log, dskip, z, ldz, static_cast<T*>(out), ldo, state, run_start, seq_start, \
+  scan_single_kernel<X, N><<<grid, kWave, 0, s>>>(static_cast<const X*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, \
+                                                  a_log, dskip, z, ldz, static_cast<X*>(out), ldo, state, run_start, seq_start, \
                                                   state_slots, C, prepared)
     if (N == 8) KVCM_SCAN_SINGLE(8);
     else KVCM_SCAN_SINGLE(16);
 #undef KVCM_SCAN_SINGLE
     return launch_status("selective_scan");
   }
-  if (phase != 0 && (N == 8 || N == 16)) {
+  // Pieces: a lane a channel once its waves (64 channels, chunk_len rows) are about one a CU, states over lanes before; 32-bit
+  // exponentials take longer, and a wave all of them.  Two passes over pieces with the step sizes, us, states over lanes / a lane a channel,
+  // 16 states: bfloat16 1 x 512 rows of 1,024 channels 76 / 85, 1 x 2,048 of 1,024 106 / 101, of 4,096 319 / 130, 8 x 512 of 512 100 / 98;
+  // 32 bits 1 x 2,048 of 1,024 110 / 198, of 2,048 182 / 207, of 4,096 330 / 227, 8 x 512 of 1,024 173 / 203, of 2,048 311 / 220.
+  const long long waves = static_cast<long long>(T) * C / (kWave * 128);
+  if (phase != 0 && (N == 8 || N == 16) && waves >= (std::is_same<X, float>::value ? 640 : 256)) {
     const dim3 grid((C + 255) / 256, S, pieces);
 #define KVCM_SCAN_CHANNELS(N, OUT)                                                                                            \
-  scan_channels_kernel<T, N, OUT><<<grid, 256, 0, s>>>(static_cast<const T*>(x), ldx, dt_lin, lddt, bc, ldbc, off_b, off_c,     \
-                                                       a_log, dskip, z, ldz, static_cast<T*>(out), ldo, run_start, state_slots, \
+  scan_channels_kernel<X, N, OUT><<<grid, 256, 0, s>>>(static_cast<const X*>(x), ldx, dt_lin, lddt, bc, ldbc, off_b, off_c,     \
+                                                       a_log, dskip, z, ldz, static_cast<X*>(out), ldo, run_start, state_slots, \
                                                        C, chunk_len, carry, dsum)
     if (N == 8 && phase == 1) KVCM_SCAN_CHANNELS(8, false);
     else if (N == 8) KVCM_SCAN_CHANNELS(8, true);
@@ -360,9 +365,9 @@ int launch_scan(const void* x, int ldx, const float* dt_lin, int lddt, const flo
     return launch_status("selective_scan");
   }
 #define KVCM_SCAN(LPC, NPL)                                                                                             \
-  selective_scan_kernel<T, LPC, NPL><<<dim3((C + kWave / LPC - 1) / (kWave / LPC), S, pieces), kWave, 0, s>>>(           \
-      static_cast<const T*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, a_log, dskip, z, ldz,               \
-      static_cast<T*>(out), ldo, state, run_start, seq_start, state_slots, C, N, prepared, phase, chunk_len, carry, dsum)
+  selective_scan_kernel<X, LPC, NPL><<<dim3((C + kWave / LPC - 1) / (kWave / LPC), S, pieces), kWave, 0, s>>>(           \
+      static_cast<const X*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, a_log, dskip, z, ldz,               \
+      static_cast<X*>(out), ldo, state, run_start, seq_start, state_slots, C, N, prepared, phase, chunk_len, carry, dsum)
   if (N <= 1) KVCM_SCAN(1, 1);
   else if (N <= 2) KVCM_SCAN(2, 1);
   else if (N <= 4) KVCM_SCAN(4, 1);
@@ -400,9 +405,9 @@ extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, const floa
   auto launch = [&](int phase, int pieces, float* cr, float* ds) {
     if (dtype == kF32)
       return launch_scan<float>(x, ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, a_log, dskip, z, ldz, out, ldo, state,
-                                run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, max_run, cr, ds, s);
+                                run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, max_run, T, cr, ds, s);
     return launch_scan<bf16_t>(x, ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b, off_c, a_log, dskip, z, ldz, out, ldo, state,
-                               run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, max_run, cr, ds, s);
+                               run_start, seq_start, state_slots, S, C, N, prepared, phase, chunk_len, pieces, max_run, T, cr, ds, s);
   };
   if (chunk_len <= 0) return launch(0, 1, nullptr, nullptr);
   // long runs in pieces of chunk_len rows: every piece from zero, the states that enter the pieces, every piece again

@@ -359,10 +359,11 @@ def test_delta_rule_by_sizes_and_run_lengths(d, dv):
             row, at[i] = row + n, at[i] + n
 
 
-@pytest.mark.parametrize("C,N", [(70, 16), (300, 16), (257, 8), (64, 4)])
+@pytest.mark.parametrize("C,N", [(70, 16), (300, 16), (257, 8), (64, 4), (2300, 16), (5500, 8)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_selective_scan_in_pieces_by_state_size(C, N, dtype):
-    """Pieces whose channels are a lane's each (8 and 16 states) or spread over lanes, with runs that end anywhere in a piece."""
+    """Pieces whose channels are spread over lanes or a lane's each (8 and 16 states, enough rows and channels for that), with
+    runs that end anywhere in a piece."""
     from kvcm_amd import ops
     rng = np.random.default_rng(C + N)
     lengths = (129, 1, 640, 200)
@@ -461,6 +462,26 @@ def test_delta_rule_in_32_bits_depends_on_its_row_alone(d):
             return ops.delta_scan(*x, o, state, step, heads, d, d, one_order=True)
         return call
     _all_equal(_rows_of_first(run, (r, k, v, torch.sigmoid(w), torch.sigmoid(a) * u, u)))
+
+
+@pytest.mark.parametrize("N", [8, 16])
+def test_selective_scan_in_32_bit_pieces_alone_and_beside_others(N):
+    """Eight long runs, whose channels are a lane's each, and one of them alone, whose states lie over lanes: the same bits."""
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(N)
+    C, n = 1001, 700
+    x, z, dt = (torch.randn(8 * n, C, generator=g).to(DEV) for _ in range(3))
+    bc = torch.randn(8 * n, 2 * N, generator=g).to(DEV)
+    a_log, dsk, db = torch.rand(C, N, generator=g).to(DEV), torch.randn(C, generator=g).to(DEV), torch.randn(C, generator=g).to(DEV)
+    got = []
+    for first, seqs in ((0, 8), (5, 1)):
+        step, at = Step([(first + s, 0, n) for s in range(seqs)]), slice(first * n, (first + seqs) * n)
+        step.max_run = n
+        state, out = torch.full((8, C, N), 5.0, device=DEV), torch.empty(step.rows, C, device=DEV)
+        carry = torch.empty(ops.selective_scan_carry_floats(step.rows, seqs, C, N), device=DEV)
+        ops.selective_scan(x[at], dt[at].clone(), db, bc[at], 0, N, a_log, dsk, z[at].clone(), out, state, step, prepare=True, carry=carry)
+        got.append((out[(5 - first) * n:(6 - first) * n], state[5]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
 @pytest.mark.parametrize("d", [1, 3, 6, 16, 18, 32, 62, 64, 100, 128, 130, 160, 256])
