@@ -15,7 +15,9 @@
 //
 // 32-bit storage with head sizes 16, 32, 64 and 128, up to 16 query heads per kv head and pages of a multiple of 4 tokens
 // takes attention_f32_kernel below: the same products on the matrix cores' 32-bit instruction.
+#include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 #include "common.h"
 
@@ -122,7 +124,7 @@ __global__ void __launch_bounds__(kAttnWaves* kWave)
 // ---- 32-bit storage on the matrix cores (v_mfma_f32_16x16x4_f32) -----------------------------------------------------------
 // A workgroup owns 16 items, an item being one query head of one row: the heads of a kv head's group, of one row or of 16 /
 // group consecutive rows, so that the keys and values of the group are read once.  Its waves take the chunks of 64 keys in turn
-// (chunk c goes to wave c % WAVES) and meet in LDS at the end, in wave order.  Products are transposed as in the bfloat16
+// (chunk c is of share c % WAVES, a wave's own for each sequence) and meet in LDS at the end, in the order of the shares.  Products are transposed as in the bfloat16
 // kernels, S^T = K Q^T and O^T += V^T P^T: a lane's scores are four consecutive keys of one item, which is where the second
 // product wants their probabilities, and both caches are read in 16-byte pieces.
 // A chunk in which an item sees nothing changes nothing of it, so its result does not depend on the items beside it.
@@ -151,6 +153,8 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
   const int row = r0 + (real ? own : 0), head = kvh * group + (real ? it % group : 0);
   const int ctx = real ? ctx_lens[row] : 0;
   const int first = (window > 0 && ctx > window) ? ctx - window : 0;
+  // the tile's rows, a lane each: no load waits for another as they are looked through
+  const int seqs = row_seq[r0 + (lane < rows ? lane : 0)], ctxs = ctx_lens[r0 + (lane < rows ? lane : 0)];
   f32x4 qf[NT];
 #pragma unroll
   for (int u = 0; u < NT; ++u)
@@ -162,26 +166,30 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
 #pragma unroll
   for (int d = 0; d < NT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // consecutive rows of one sequence walk its keys together
-  for (int j = 0; j < rows;) {
-    const int seq = row_seq[r0 + j];
+  // consecutive rows of one sequence walk its keys together; a wave takes another share of the chunks with each sequence, so that
+  // sequences of few chunks are walked by as many waves
+  int share = wave, own_share = wave;                           // of the sequence at hand; of the item's
+  for (int j = 0; j < rows; share = share + 1 == WAVES ? 0 : share + 1) {
+    const int seq = __builtin_amdgcn_readlane(seqs, j);
     int end = j, most = 0, least = 0x7fffffff;                  // rows j .. end - 1 see tokens in [least, most)
-    for (; end < rows && row_seq[r0 + end] == seq; ++end) {
-      const int c = ctx_lens[r0 + end];
+    for (; end < rows && __builtin_amdgcn_readlane(seqs, end) == seq; ++end) {
+      const int c = __builtin_amdgcn_readlane(ctxs, end);
       if (c <= 0) continue;
       const int f = (window > 0 && c > window) ? c - window : 0;
       most = c > most ? c : most;
       least = f < least ? f : least;
     }
     const bool mine = real && own >= j && own < end;
+    own_share = mine ? share : own_share;
     const int* table = tables + size_t(seq) * table_stride;
     int chunk = most > 0 ? least / kWave : 0;
-    chunk += (wave - chunk % WAVES + WAVES) % WAVES;
-    for (int c0 = chunk * kWave; c0 < most; c0 += WAVES * kWave) {
-      f32x4 kf[4][NT], vf[4][NT];
-      const float *kp[4], *vp[4];
+    chunk += (share - chunk % WAVES + WAVES) % WAVES;
+    auto walk = [&](int c0, auto groups) {                      // the first G sixteens of a chunk's keys
+      constexpr int G = decltype(groups)::value;
+      f32x4 kf[G][NT], vf[G][NT];
+      const float *kp[G], *vp[G];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {                             // tokens outside [least, most) read an inner token's place
+      for (int i = 0; i < G; ++i) {                             // tokens outside [least, most) read an inner token's place
         int t = c0 + 16 * i + it;
         t = t < most ? (t > least ? t : least) : most - 1;
         kp[i] = kcache + size_t(table[t / B]) * page_stride + kvh * head_stride + size_t(t % B) * hd + 4 * g;
@@ -193,23 +201,23 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
 #pragma unroll
       for (int u = 0; u < NT; ++u)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) kf[i][u] = *reinterpret_cast<const f32x4*>(kp[i] + 16 * u);
+        for (int i = 0; i < G; ++i) kf[i][u] = *reinterpret_cast<const f32x4*>(kp[i] + 16 * u);
 #pragma unroll
       for (int d = 0; d < NT; ++d)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vf[i][d] = *reinterpret_cast<const f32x4*>(vp[i] + size_t(16 * d) * B);
-      f32x4 s[4];
+        for (int i = 0; i < G; ++i) vf[i][d] = *reinterpret_cast<const f32x4*>(vp[i] + size_t(16 * d) * B);
+      f32x4 s[G];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < G; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < NT; ++u)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][u][e], qf[u][e], s[i], 0, 0, 0);
+          for (int i = 0; i < G; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][u][e], qf[u][e], s[i], 0, 0, 0);
       float top = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < G; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int t = c0 + 16 * i + 4 * g + e;
@@ -224,7 +232,7 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
       const float alpha = some ? expf(m - m_new) : 1.f;
       float sum = 0.f, bad = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < G; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int t = c0 + 16 * i + 4 * g + e;
@@ -245,7 +253,7 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
       for (int d = 0; d < NT; ++d) o[d] *= alpha;
       if (rows == 1 || __ballot(bad != bad) == 0) {      // (zero times these values is zero, or nobody else is here)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < G; ++i)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -253,12 +261,12 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
       } else {
         // a value that is not finite counts for the rows that see it only: row by row, the others' values zero
         for (int r = j; r < end; ++r) {
-          const int c = ctx_lens[r0 + r], f = (window > 0 && c > window) ? c - window : 0;
+          const int c = __builtin_amdgcn_readlane(ctxs, r), f = (window > 0 && c > window) ? c - window : 0;
           f32x4 one[NT];
 #pragma unroll
           for (int d = 0; d < NT; ++d) one[d] = o[d];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < G; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const int t = c0 + 16 * i + 4 * g + e;
@@ -270,17 +278,21 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
           for (int d = 0; d < NT; ++d) o[d] = own == r ? one[d] : o[d];
         }
       }
+    };
+    for (int c0 = chunk * kWave; c0 < most; c0 += WAVES * kWave) {      // (absent keys add zeros: left out where they are most of a chunk)
+      if (most - c0 <= 16) walk(c0, std::integral_constant<int, 1>());
+      else walk(c0, std::integral_constant<int, 4>());
     }
     j = end;
   }
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);
   if (g == 0) {
-    part_m[wave][it] = m;
-    part_l[wave][it] = l;
+    part_m[own_share][it] = m;
+    part_l[own_share][it] = l;
   }
 #pragma unroll
-  for (int d = 0; d < NT; ++d) part_o[wave][it][4 * d + g] = o[d];
+  for (int d = 0; d < NT; ++d) part_o[own_share][it][4 * d + g] = o[d];
   __syncthreads();
   for (int t = threadIdx.x; t < rows * group * NT * 4; t += WAVES * kWave) {
     const int i = t / (NT * 4), d = t % (NT * 4), r = r0 + i / group;
@@ -314,8 +326,12 @@ template <int NT>
 void launch_attention_f32(const float* q, int q_stride, float* out, int out_stride, const float* kcache, const float* vcache,
                           const int* tables, int table_stride, const int* row_seq, const int* ctx_lens, int T, int nh, int nkv,
                           int B, float scale, int window, hipStream_t s) {
-  // Few rows (decoding): one row a workgroup, whose keys nobody shares.  Many: as many rows as fill the 16 items.
-  const int per = static_cast<long long>(T) * nkv <= 512 ? 1 : 16 / (nh / nkv);
+  // As many rows a workgroup as leave each CU one (the smallest heads' registers allow two), where the 16 items hold them.
+  // Single rows of as many sequences, us, the kernel above / a full tile walked by the same wave for each sequence, all keys of a
+  // chunk multiplied / this: 32 heads over 32 kv heads of 64, 64 rows of 16 tokens 12.6 / 71.8 / 8.9, of 600 413 / 238 / 123; 256
+  // rows of 16 34 / 154 / 28; 8 over 8 of 128, 256 rows of 16 19 / 134 / 14; 32 over 4 of 64, 8 rows of 16 9.3 / 8.0 / 5.8.
+  const long long units = static_cast<long long>(T) * nkv;
+  const int per = static_cast<int>(units <= (NT == 1 ? 512 : 256) ? 1 : std::min<long long>((units + 255) / 256, 16 / (nh / nkv)));
   const unsigned blocks = static_cast<unsigned>((T + per - 1) / per) * nkv;
   attention_f32_kernel<NT><<<blocks, f32_waves<NT>() * kWave, 0, s>>>(q, q_stride, out, out_stride, kcache, vcache, tables, table_stride,
                                                                       row_seq, ctx_lens, T, nh, nkv, per, B, scale, window);

@@ -594,6 +594,20 @@ def test_paged_attention_f32_bad_values_stay_with_their_sequence(ops, nh, nkv, h
         np.testing.assert_array_equal(_run_attention(ops, one, nh, nkv, hd, torch.float32, window=window)[0], got[r])
 
 
+@pytest.mark.parametrize("nh,nkv,hd,B,window", [(8, 8, 64, 16, 0), (16, 16, 32, 8, 0), (24, 8, 128, 16, 100), (40, 40, 16, 4, 0)])
+def test_paged_attention_f32_single_rows_of_many_sequences(ops, nh, nkv, hd, B, window):
+    # tiles whose every row is of another sequence, of less than a sixteenth of a chunk to more chunks than a workgroup has waves
+    rng = np.random.default_rng(nh + hd)
+    lens = [int(n) for n in rng.choice([1, 2, 15, 16, 17, 31, 64, 65, 80, 81, 130, 513, 580, 1100], size=40)]
+    P = _paged_problem(rng, lens, nh, nkv, hd, B, all_rows=False)
+    assert P["R"] * nkv > 256
+    got = _run_attention(ops, P, nh, nkv, hd, torch.float32, window=window)
+    np.testing.assert_allclose(got, _ref_attention(P, nh, nkv, hd, window=window), atol=2e-5, rtol=0)
+    for r in range(0, P["R"], 3):
+        one = dict(P, Q=P["Q"][r:r + 1], row_seq=P["row_seq"][r:r + 1], ctx=P["ctx"][r:r + 1], R=1)
+        np.testing.assert_array_equal(_run_attention(ops, one, nh, nkv, hd, torch.float32, window=window)[0], got[r])
+
+
 # -------------------------------------------------------------------------------- sampling
 def test_argmax_reference_vector(ops):
     # tests/test_kernels.cu:96-109
