@@ -385,10 +385,11 @@ def test_selective_scan_in_pieces_by_state_size(C, N, dtype):
         row += len(x)
 
 
-@pytest.mark.parametrize("C,N", [(64, 16), (70, 16), (33, 8)])
+@pytest.mark.parametrize("C,N", [(64, 16), (70, 16), (33, 8), (2801, 16)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_selective_scan_of_single_tokens(C, N, dtype):
-    """Decoded steps whose channels are a lane's each: from a slot with rubbish, beside a padding sequence."""
+    """Decoded steps whose channels are a lane's each (in 32 bits with 16 states from 8,192 channels in all on): from a slot with
+    rubbish, beside a padding sequence."""
     from kvcm_amd import ops
     rng = np.random.default_rng(C * N)
     grid = lambda a: torch.tensor(a).to(dtype).double().numpy()
@@ -507,7 +508,7 @@ def test_delta_rule_rows_may_begin_at_any_float(d):
         np.testing.assert_allclose(o[:40].cpu().numpy().reshape(40, heads, d), want, atol=1e-4 * max(1.0, np.abs(want).max()))
 
 
-@pytest.mark.parametrize("C,N", [(70, 16), (300, 8), (20, 4), (33, 20)])
+@pytest.mark.parametrize("C,N", [(70, 16), (300, 8), (20, 4), (33, 20), (8200, 16)])
 def test_selective_scan_in_32_bits_depends_on_its_row_alone(C, N):
     from kvcm_amd import ops
     g = torch.Generator().manual_seed(C)
