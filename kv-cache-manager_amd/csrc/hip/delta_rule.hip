@@ -247,6 +247,9 @@ int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const floa
   }
   // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
   // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 294 (16 lanes) / 374 and 261 (16 lanes; 8 lanes of two columns).
+  // The other sizes, us, workgroups that share a token's vectors through LDS / so, 64 heads of 16 x 16, 64 of 32 x 32, 8 of 48 x 48, 32 of
+  // 128 x 128: one sequence of 1,024 tokens 420 / 151, 454 / 155, 493 / 121, 1,045 / 343; 8 of 129 64 / 28, 70 / 52, 70 / 26, 563 / 311;
+  // 8 single tokens 6.5 / 3.8, 6.7 / 4.4, 7.6 / 4.2, 43 / 16.
   // The lanes of a column are the order of its sums.  With one_order (32-bit storage, where a row's result depends on that row
   // alone) they follow from the key size, whatever the runs: 8 lanes from 33 to 64, 405 / 211 us; 16 beyond, also for single
   // tokens (8 rows, 32 heads of 128 x 128: 20 us, with 8 lanes and workgroups of 32 columns 14 us).

@@ -309,6 +309,9 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
   }
   // A column over 16 lanes is the shorter chain, over 8 the fewer instructions: once waves of eight columns fill the SIMDs, those.
   // 2,048 tokens of one sequence / 8 sequences of 509, 32 heads of 64 x 64, us: 292 (16 lanes) / 247 and 217 (16 lanes; 8 lanes of two columns).
+  // The other sizes, us with the maxima, workgroups that share a token's vectors through LDS / so, 64 heads of 16 x 16, 64 of 32 x 32, 8 of
+  // 48 x 48, 32 of 128 x 128, 8 of 256 x 256: one sequence of 1,024 tokens 416 / 163, 423 / 162, 499 / 146, 587 / 287, 1,367 / 508; 8 of 129
+  // 70 / 38, 73 / 51, 75 / 33, 307 / 189, 526 / 276; 8 single tokens 10.1 / 9.5, 10.5 / 10.2, 10.7 / 10.0, 37 / 32, 36 / 33.
   // The lanes of a column are the order of its sums: with one_order they follow from the key size alone (8 from 33 to
   // 64: 394 us for the one sequence).
   const bool few = static_cast<long long>(S) * heads * ((dv + 7) / 8) < 1024;
