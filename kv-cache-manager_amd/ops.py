@@ -567,7 +567,7 @@ def skinny_splits(M, N, K):
     return lib().kvcm_gemm_skinny_splits(M, N, K)
 
 
-def _rows8_takes(M, N, K):
+def _rows8_takes(M, N, K, out_dtype, splits):
     """Whether a product of at most 8 rows that nobody adds slices of runs unsplit in workgroups of 8 or 16 columns
     (gemm_rows8.hip).  What speaks for it is the second launch, which adds the slices that the other kernels split K into, and
     short chains; against it, that each workgroup reads all rows again and lives for one pass over K, so that many columns of few k
@@ -576,7 +576,16 @@ def _rows8_takes(M, N, K):
     not split); 50000 x 1024 25.7 / 22.0; more weights than that 16384 x 4096 28.2 / 32.1, 28672 x 4096 48.9 / 52.6 (one row: 28.4 /
     27.7 and 47.8 / 43.7); fewer k: 8192 x 512 even, 32000 x 512 10.1 / 13.1, 128000 x 512 33.5 / 45.0 (one row 32.1 / 35.0), 50272 x
     768 20.2 / 21.0; with an odd multiple of 8 columns, where a workgroup has 8 and the other way is the general kernel: 8200 x
-    512 9.6 / 10.7, 16392 x 1024 21.1 / 18.0, 32008 x 1024 25.3 / 30.6, 32008 x 2048 46.9 / 33.2."""
+    512 9.6 / 10.7, 16392 x 1024 21.1 / 18.0, 32008 x 1024 25.3 / 30.6, 32008 x 2048 46.9 / 33.2.
+    Where the other way may split (``splits``), a long K is many short chains there and one here, the longer the fewer columns there are:
+    bfloat16 results, one row and 8 rows, otherwise / so: 512 x 5632 8.1 / 6.5 and 8.8 / 8.5, 512 x 7168 8.7 / 8.1 and 9.4 / 10.9, 512 x
+    14336 10.5 / 11.8 and 11.2 / 16.3; 32 x 4096 6.3 / 5.2 and 7.2 / 6.5, 32 x 7168 6.9 / 7.9 and 7.1 / 10.7; 4096 x 11008 19.9 / 20.1
+    and 20.2 / 20.5, 4096 x 14336 22.6 / 23.4 and 23.0 / 24.1; 32-bit results, which that second launch stores twice as wide,
+    512 x 8192 11.2 / 8.1 and 11.9 / 10.9, 512 x 14336 14.4 / 11.8 and 15.2 / 16.3."""
+    if splits and N % 16 == 0:
+        wide = out_dtype == torch.float32
+        if K > (4096 if N < 128 else 12288 if N >= 2048 else 6144 if not wide else 8192 if M > 4 else K):
+            return False
     return (M <= FUSED_NORM_MAX_ROWS and (M <= 2 or N * K <= 66_000_000) and (N <= 8192 or K >= (1024 if N % 16 == 0 else 2048))
             and gemm8_supported(M, N, K))
 
@@ -623,7 +632,8 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
         _call("kvcm_gemm_library_f32out", _ptr(x), _ptr(w), _ptr(out), M, N, K, x.stride(0), w.stride(0), out.stride(0),
               _ptr(ws), ws.numel(), _stream())
         return out
-    if (unsplit and not (keep_partial and scratch is not None) and _rows8_takes(M, N, K) and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+    if (unsplit and not (keep_partial and scratch is not None) and _rows8_takes(M, N, K, out.dtype, scratch is not None)
+            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
         _call("kvcm_gemm8", _ptr(x), x.stride(0), _ptr(w), w.stride(0), M, N, K, 0, 0, 0.0, _ptr(out), _DT[out.dtype],
               out.stride(0), 0, _stream())

@@ -338,7 +338,8 @@ def test_gemm_f32_of_short_rows_is_one_ascending_chain(ops, M, N, K):
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("N,K", [(40, 192), (520, 1024), (8200, 512), (8208, 512), (8200, 1024), (16392, 2048), (16384, 4096), (50, 128), (64, 100)])
+@pytest.mark.parametrize("N,K", [(40, 192), (520, 1024), (8200, 512), (8208, 512), (8200, 1024), (16392, 2048), (16384, 4096), (50, 128), (64, 100),
+                                 (512, 6144), (512, 6208), (512, 8256), (32, 4096), (32, 4160), (2048, 12352)])
 def test_gemm_bf16_unsplit(ops, N, K, out_dtype):
     # both sides of the rule for products that nobody adds slices of: unsplit, split and added, the general kernel; rows at
     # a stride, rows and weights that are not 16-byte aligned
