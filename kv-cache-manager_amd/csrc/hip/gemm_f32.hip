@@ -15,6 +15,7 @@
 //               lane multiplied while the next eight are on their way; segments meet in LDS.  Two rows, K = 2048: N = 11264
 //               (92 MB) 22 us, 4.2 TB/s; N = 2048 8 us; K = 5632, N = 2048 20 us.  As 16 x 64 tiles of plain fused
 //               multiply-adds with scalar loads these took 304 us in the mean.
+//               Up to 32 rows of very many columns: tiles of 32 rows as below.
 //   more rows   bound by the matrix cores (157 TFLOP/s).  Tiles of 64 x 64 or 64 x 32, four waves, 32 k staged in LDS while the
 //               next 32 are on their way.  573 rows, K = 2048: N = 11264 254 us (104 TFLOP/s), N = 2048 68 us; 539 us in the
 //               mean of a layer's four products as 64 x 64 tiles of plain fused multiply-adds.
@@ -32,16 +33,19 @@ __host__ __device__ __forceinline__ int segment_units(int K) {
   return (units + kSegments - 1) / kSegments;
 }
 
-// Four consecutive k of one row, zero from K on.  VEC: rows are 16-byte aligned and K is a multiple of 4, so a piece lies
-// wholly inside or outside; the load is unconditional (from k = 0 where it would be outside) and masked afterwards.  FULL: no
-// piece lies outside.
-template <bool VEC, bool FULL = false>
+// Four consecutive k of one row, zero from K on.  Rows may begin at any float: the hardware takes 16-byte loads there.  FULL: no
+// piece lies outside.  FOURS: K is a multiple of 4, so a piece lies wholly inside or outside; the load is unconditional (from
+// k = 0 where it would be outside) and masked afterwards.
+typedef float any_four __attribute__((ext_vector_type(4), aligned(4)));
+template <bool FOURS, bool FULL = false>
 __device__ __forceinline__ f32x4 load4(const float* __restrict__ row, int k, int K) {
   f32x4 v;
-  if constexpr (VEC && FULL) {
-    v = *reinterpret_cast<const f32x4*>(row + k);
-  } else if constexpr (VEC) {
-    v = *reinterpret_cast<const f32x4*>(row + (k < K ? k : 0));
+  if constexpr (FULL) {
+    const any_four x = *reinterpret_cast<const any_four*>(row + k);
+    v = f32x4{x.x, x.y, x.z, x.w};
+  } else if constexpr (FOURS) {
+    const any_four x = *reinterpret_cast<const any_four*>(row + (k < K ? k : 0));
+    v = f32x4{x.x, x.y, x.z, x.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = k < K ? v[e] : 0.f;
   } else {
@@ -55,7 +59,7 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ row, int k, int
 }
 
 // ---- up to 16 * MT rows: columns 16 blockIdx.x .. + 15, wave w segment w ---------------------------------------------------
-template <int MT, bool VEC>
+template <int MT, bool FOURS>
 __global__ void __launch_bounds__(kSegments* kWave)
     gemm_f32_rows_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
                          int ldx, int ldw, int ldy) {
@@ -80,7 +84,7 @@ __global__ void __launch_bounds__(kSegments* kWave)
   constexpr int D = MT == 1 ? 4 : MT == 2 ? 2 : 1;
   f32x4 b[2][D][2], a[2][D][2][MT];
   auto fetch = [&](f32x4 (&bb)[D][2], f32x4 (&aa)[D][2][MT], int u) {
-    if (VEC && u + D <= hi && (u + D) * kUnit <= K) {
+    if (u + D <= hi && (u + D) * kUnit <= K) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
 #pragma unroll
@@ -96,9 +100,15 @@ __global__ void __launch_bounds__(kSegments* kWave)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int k = u + d < hi ? (u + d) * kUnit + 16 * h + 4 * g : K;      // (beyond the segment: zeros)
-          bb[d][h] = load4<VEC>(w, k, K);
+          if (!FOURS && u + d < hi && (u + d + 1) * kUnit <= K) {               // (single loads in the unit with the row's end only)
+            bb[d][h] = load4<true, true>(w, k, K);
 #pragma unroll
-          for (int i = 0; i < MT; ++i) aa[d][h][i] = load4<VEC>(x[i], k, K);
+            for (int i = 0; i < MT; ++i) aa[d][h][i] = load4<true, true>(x[i], k, K);
+            continue;
+          }
+          bb[d][h] = load4<FOURS>(w, k, K);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) aa[d][h][i] = load4<FOURS>(x[i], k, K);
         }
     }
   };
@@ -144,7 +154,7 @@ __global__ void __launch_bounds__(kSegments* kWave)
 // meets no bank twice.
 // ASCENDING: one chain over all of K instead, k after k: a piece's four elements then go to four pieces as they are staged, so
 // that lane group g's piece holds k = 4 m + g for m = 0..3.
-template <int TM, int TN, bool VEC, bool ASCENDING>
+template <int TM, int TN, bool FOURS, bool ASCENDING>
 __global__ void __launch_bounds__(256, 2)
     gemm_f32_tiles_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
                           int ldx, int ldw, int ldy) {
@@ -167,16 +177,16 @@ __global__ void __launch_bounds__(256, 2)
   for (int e = 0; e < 4; ++e) spread[e] = 4 * (srow * 8 + (((sc & 4) + e) ^ (srow & 7))) + (sc & 3);
   f32x4 px[TM], pw[TN];
   auto fetch = [&](int k0) {
-    if (VEC && k0 + BK <= K) {
+    if (k0 + BK <= K) {
 #pragma unroll
       for (int p = 0; p < TM; ++p) px[p] = load4<true, true>(xr[p], k0 + kc, K);
 #pragma unroll
       for (int p = 0; p < TN; ++p) pw[p] = load4<true, true>(wr[p], k0 + kc, K);
     } else {
 #pragma unroll
-      for (int p = 0; p < TM; ++p) px[p] = load4<VEC>(xr[p], k0 + kc, K);
+      for (int p = 0; p < TM; ++p) px[p] = load4<FOURS>(xr[p], k0 + kc, K);
 #pragma unroll
-      for (int p = 0; p < TN; ++p) pw[p] = load4<VEC>(wr[p], k0 + kc, K);
+      for (int p = 0; p < TN; ++p) pw[p] = load4<FOURS>(wr[p], k0 + kc, K);
     }
   };
   auto put = [&](f32x4* rows, int p, f32x4 v) {
@@ -256,13 +266,13 @@ __global__ void __launch_bounds__(256, 2)
 // K up to 256 (models of small width, low-rank factors): these launches are bound by their latency, so they are not cut.
 constexpr int kShortK = 256;
 
-template <int TM, int TN, bool VEC, bool ASCENDING>
+template <int TM, int TN, bool FOURS, bool ASCENDING>
 void launch_tiles(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t s) {
   const dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM));
-  gemm_f32_tiles_kernel<TM, TN, VEC, ASCENDING><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+  gemm_f32_tiles_kernel<TM, TN, FOURS, ASCENDING><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
 }
 
-template <bool VEC>
+template <bool FOURS>
 void launch_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t s) {
   // Measured at K = 2048 (us; rows kernel / tiles of 64 x 32 / of 64 x 64).  The rows kernel takes 22 for up to 256 workgroups
   // and about 0.09 for each beyond; the tiles take 41 / 50 as long as a CU has one or two, and 0.084 / 0.165 each beyond.  So
@@ -276,19 +286,33 @@ void launch_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int
   // L2 into a wave's registers these took 33, 33, 34, 60 and 228 us, as plain fused multiply-adds from LDS 29, 29, 30, 33 and 81.
   const long long few = (long long)((M + 63) / 64) * ((N + 31) / 32), large = (long long)((M + 63) / 64) * ((N + 63) / 64);
   if (K <= kShortK) {
-    if (large >= 256) launch_tiles<2, 2, VEC, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
-    else launch_tiles<1, 1, VEC, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    if (large >= 256) launch_tiles<2, 2, FOURS, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    else launch_tiles<1, 1, FOURS, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    return;
+  }
+  // Up to 32 rows of many columns: tiles of 32 rows, the rows kernel's blocks being short there (a wave has one segment of K).
+  // One row / 16 rows, us, rows kernel / 32 x 32 / 32 x 64: K = 512, N = 8192 9.0 / 9.7 / 10.6 and 11.7 / 10.6 / 10.9, N = 20000 21.8 /
+  // 13.1 / 14.4 and 27 / 13.5 / 14.7, N = 32000 32 / 15.9 / 14.8 and 41 / 16.5 / 15.4, N = 128000 111 / 49 / 45 and 151 / 52 / 48 (77 and
+  // 96 as plain fused multiply-adds); K = 1000, N = 20000 20.7 / 23.0 / 25.6 and 23.6 / 23.7 / 26.1, N = 32000 31 / 28 / 25.6 and 35 /
+  // 29 / 26.6; K = 2048, N = 32000 50 / 52 / 46 and 67 / 53 / 48.  A long stream for one row is the rows kernel's: K = 4096, N = 32000,
+  // 1 / 8 / 16 / 32 rows, rows kernel (64 x 32 tiles at 32) / 32 x 64: 101 / 116 / 140 / 169 and 120 / 111 / 111 / 114.
+  if (M <= 32 && (N + 63) / 64 >= 480 && (M > 4 || K <= 2048)) {
+    launch_tiles<1, 2, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    return;
+  }
+  if (M <= 32 && (N + 31) / 32 >= 500 && K <= 768) {
+    launch_tiles<1, 1, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
     return;
   }
   if (M <= 16 || few < (M <= 32 ? 600 : 228)) {
     const dim3 grid((N + 15) / 16, M <= 64 ? 1 : (M + 63) / 64);
-    if (M <= 16) gemm_f32_rows_kernel<1, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
-    else if (M <= 32) gemm_f32_rows_kernel<2, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
-    else gemm_f32_rows_kernel<4, VEC><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    if (M <= 16) gemm_f32_rows_kernel<1, FOURS><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    else if (M <= 32) gemm_f32_rows_kernel<2, FOURS><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    else gemm_f32_rows_kernel<4, FOURS><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
   } else if (large >= 704) {
-    launch_tiles<2, 2, VEC, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    launch_tiles<2, 2, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   } else {
-    launch_tiles<2, 1, VEC, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+    launch_tiles<2, 1, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   }
 }
 
@@ -301,9 +325,7 @@ extern "C" int kvcm_gemm_f32(const float* X, const float* W, float* Y, int M, in
   if (M == 0 || N == 0) return 0;
   KVCM_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   KVCM_REQUIRE(ldx >= K && ldw >= K && ldy >= N, "gemm_f32: leading dimensions too small");
-  const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(W) % 16 == 0;
-  if (vec) launch_gemm_f32<true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
+  if (K % 4 == 0) launch_gemm_f32<true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   else launch_gemm_f32<false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   return launch_status("gemm_f32");
 }

@@ -299,10 +299,10 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(ops):
         assert torch.equal(part, full[lo:hi]), "a row's sum changed with the rows beside it"
 
 
-@pytest.mark.parametrize("N,K", [(64, 16), (130, 20), (300, 333), (2560, 2048), (520, 5632)])
+@pytest.mark.parametrize("N,K", [(64, 16), (130, 20), (300, 333), (2560, 2048), (520, 5632), (16001, 300), (30700, 260), (30661, 257)])
 def test_gemm_f32_kernels_agree_bit_for_bit(ops, N, K):
-    # up to 16, 32 and 64 rows, tiles of 64 x 32 and of 64 x 64 (where those fill the chip): one sequence of operations for an element;
-    # in rows whose 16-byte pieces are aligned, and from an odd column on (single loads)
+    # up to 16, 32 and 64 rows, tiles of 64 x 32 and of 64 x 64 (where those fill the chip), of 32 x 32 and 32 x 64 for few rows of many
+    # columns: one sequence of operations for an element; in rows whose 16-byte pieces are aligned, and in rows of an odd stride
     rng = np.random.default_rng(N + K)
     M = 1700
     x = _t(rng.normal(size=(M, K + 1)).astype(np.float32), torch.float32)
