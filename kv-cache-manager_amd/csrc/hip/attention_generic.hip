@@ -279,10 +279,9 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
         }
       }
     };
-    for (int c0 = chunk * kWave; c0 < most; c0 += WAVES * kWave) {      // (absent keys add zeros: left out where they are most of a chunk)
-      if (most - c0 <= 16) walk(c0, std::integral_constant<int, 1>());
-      else walk(c0, std::integral_constant<int, 4>());
-    }
+    int c0 = chunk * kWave;
+    for (; c0 + 16 < most; c0 += WAVES * kWave) walk(c0, std::integral_constant<int, 4>());
+    if (c0 < most) walk(c0, std::integral_constant<int, 1>());      // (absent keys add zeros: left out where they are most of the last chunk)
     j = end;
   }
   l += __shfl_xor(l, 16, kWave);
