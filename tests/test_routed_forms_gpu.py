@@ -1,0 +1,89 @@
+"""The routed experts' products on the matrix cores at the edges of their tiles, against 64 bits: grouped by expert (steps of many
+rows)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _case(T, E, top, K, F, H, kind, seed, chosen=None):
+    gen = torch.Generator().manual_seed(seed)
+    bf = lambda *s, scale: (torch.randn(*s, generator=gen) * scale).bfloat16()
+    h, up, down = bf(T, K, scale=1.0), bf(E, F, K, scale=K ** -0.5), bf(E, H, F, scale=F ** -0.5)
+    gate = bf(E, F, K, scale=K ** -0.5) if kind == "silu" else None
+    if chosen is None:
+        chosen = torch.stack([torch.randperm(E, generator=gen)[:top] for _ in range(T)])
+    return h, gate, up, down, chosen.to(torch.int32), torch.rand(T, top, generator=gen) + 0.1, torch.randn(T, H, generator=gen)
+
+
+def _want(case, kind, weigh_input, add):
+    """-> (the result in 64 bits, how far rounding an activation to bfloat16 may move it: half a unit of 2^-8 each, and as much
+    again where the sum before it falls on the other side of a tie; with it the 32-bit sums' own error, which is smaller)."""
+    h, gate, up, down, chosen, weight, base = (t.double() if t is not None and t.dtype != torch.int32 else t for t in case)
+    want = base.clone() if add else torch.zeros_like(base)
+    bound = torch.zeros_like(base)
+    for t in range(h.shape[0]):
+        for s, e in enumerate(chosen[t].tolist()):
+            if not 0 <= e < up.shape[0]:
+                continue
+            g, x = weight[t, s], h[t]
+            inner, outer = (g, 1.0) if weigh_input else (1.0, g)
+            u = inner * (up[e] @ x)
+            if kind == "silu":
+                z = inner * (gate[e] @ x)
+                a = z * torch.sigmoid(z) * u
+            else:
+                a = 0.5 * u * (1.0 + torch.erf(u / 2 ** 0.5)) if kind == "gelu" else torch.relu(u) ** 2
+            want[t] += outer * (down[e] @ a)
+            bound[t] += outer * (down[e].abs() @ a.abs()) * 2.0 ** -8
+    return want, bound + 1e-5
+
+
+def _run(form, case, kind, weigh_input, add):
+    from kvcm_amd import ops
+    from kvcm_amd.parts.routed_parts import interleave_gate_up
+    h, gate, up, down, chosen, weight, base = (t.to(DEV) if t is not None else None for t in case)
+    T, K = h.shape
+    E, F, _ = up.shape
+    H, top = down.shape[1], chosen.shape[1]
+    if kind == "silu":
+        up = interleave_gate_up(gate, up)
+    wide = torch.full((T, K + 24), float("nan"), dtype=torch.bfloat16, device=DEV)      # rows apart: what lies between is not read
+    wide[:, :K] = h
+    act = torch.empty(T * top, F, dtype=torch.bfloat16, device=DEV)
+    out = torch.full((T, H), float("nan"), device=DEV)
+    how = dict(gated=kind == "silu", add=base if add else None, weigh_input=weigh_input, **({} if kind == "silu" else {"activation": kind}))
+    if form == "grouped":
+        order = torch.empty(T * top, dtype=torch.int32, device=DEV)
+        tiles = torch.empty(ops.moe_grouped_tiles(T * top, E), dtype=torch.int32, device=DEV)
+        y = torch.full((T * top, H), float("nan"), device=DEV)
+        ops.moe_grouped(wide[:, :K], up, down, chosen, weight, order, tiles, act, y, out, **how)
+    else:
+        ops.moe_rows(wide[:, :K], up, down, chosen, weight, act, out, **how)
+    return out.cpu().double()
+
+
+def _check(form, case, kind, weigh_input, add):
+    want, bound = _want(case, kind, weigh_input, add)
+    got = _run(form, case, kind, weigh_input, add)
+    assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
+    # a row that is not finite stays alone
+    bad = [case[0].clone(), *case[1:]]
+    bad[0][case[0].shape[0] // 2] = float("nan")
+    again = _run(form, bad, kind, weigh_input, add)
+    keep = torch.arange(want.shape[0]) != want.shape[0] // 2
+    assert torch.equal(again[keep], got[keep])
+
+
+# one expert with 127 to 129 of the pairs (a tile's edge), K below, at and past 64 and 128, columns that end inside a tile
+GROUPED = [(128, 3, 1, 64, 64, 128, "relu2", True), (129, 2, 1, 72, 48, 130, "silu", True), (127, 2, 2, 8, 40, 33, "gelu", False),
+           (300, 5, 2, 136, 144, 260, "silu", False), (70, 9, 3, 200, 136, 128, "relu2", False)]
+
+
+@pytest.mark.parametrize("weigh_input", [False, True])
+@pytest.mark.parametrize("shape", GROUPED)
+def test_grouped_tiles(shape, weigh_input):
+    T, E, top, K, F, H, kind, one = shape
+    chosen = torch.zeros(T, top, dtype=torch.long) if one else None
+    _check("grouped", _case(T, E, top, K, F, H, kind, T + K, chosen), kind, weigh_input, not weigh_input)
