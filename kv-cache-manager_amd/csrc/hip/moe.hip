@@ -26,6 +26,14 @@
 
 namespace kvcm {
 
+// moe_few.hip: the two products of up to 64 pairs on the matrix cores, an expert's weights read once for all its rows
+bool moe_few_up_takes(int dtype, const void* h, int ldh, int T, int K, int F, int top);
+bool moe_few_down_takes(int dtype, const void* act, int T, int F, int H, int top, int E);
+void launch_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
+                       const float* in_weight, hipStream_t s);
+void launch_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T,
+                         int F, int H, int top, int E, hipStream_t s);
+
 constexpr int kMoeMaxTop = 16;
 constexpr int kMoeMaxExperts = 1024;      // a row's logits are kept in LDS while its experts are picked
 
@@ -278,6 +286,10 @@ int kvcm_moe_up(const void* h, int dtype, int ldh, const void* w_up, const int* 
   KVCM_REQUIRE(K * sizeof(float) <= 64 * 1024, "moe_up: rows of %d values do not fit the local memory", K);
   KVCM_REQUIRE(reinterpret_cast<uintptr_t>(w_up) % 16 == 0, "moe_up: weights must be 16-byte aligned");
   KVCM_REQUIRE(dtype == kF32 || dtype == kBF16, "moe_up: unknown dtype %d", dtype);
+  if (moe_few_up_takes(dtype, h, ldh, T, K, F, top)) {
+    launch_moe_few_up(h, ldh, w_up, chosen, act, T, K, F, top, E, kind, in_weight, s);
+    return launch_status("moe_up");
+  }
   const int cw = moe_cols_per_wave(static_cast<long long>(T) * top, F);
   const dim3 grid(T * top, (F + 4 * cw - 1) / (4 * cw));
   const size_t lds = K * sizeof(float);
@@ -300,6 +312,10 @@ int kvcm_moe_down(const void* act, int dtype, const void* w_down, const int* cho
   KVCM_REQUIRE(reinterpret_cast<uintptr_t>(w_down) % 16 == 0, "moe_down: weights must be 16-byte aligned");
   KVCM_REQUIRE((H + 3) / 4 <= 65535, "moe_down: too many columns");
   KVCM_REQUIRE(dtype == kF32 || dtype == kBF16, "moe_down: unknown dtype %d", dtype);
+  if (moe_few_down_takes(dtype, act, T, F, H, top, E)) {
+    launch_moe_few_down(act, w_down, chosen, weight, add, out, T, F, H, top, E, s);
+    return launch_status("moe_down");
+  }
   const int cw = moe_cols_per_wave(T, H);
   const dim3 grid(T, (H + 4 * cw - 1) / (4 * cw));
 #define KVCM_MOE_DOWN(TT, CW)                                                                                                \

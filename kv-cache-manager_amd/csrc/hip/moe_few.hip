@@ -1,0 +1,265 @@
+// The routed feed-forward's two products for steps of a few rows (bfloat16, up to 64 (row, slot) pairs) on the matrix cores,
+// expert by expert: an expert's weights are read once for all the rows that chose it, where the row-by-row kernels of moe.hip
+// read them once per row.  Eight rows with two of eight experts each read 7 experts instead of 16.
+//
+// What bounds these launches is how many weight bytes are on their way, so the work is cut as in the products of up to 8 rows
+// (gemm_rows8.hip): many workgroups, every lane with all the weight pieces of a trip requested at once, two trips on their way.
+// Which rows share an expert is found by every wave from the pairs' experts, one a lane: the lanes that hold the same number
+// are a ballot, so nothing is sorted beforehand and no list goes through memory.
+//
+//   up     A workgroup belongs to one pair and 32 rows of its expert's matrix (gated: 16 gate and 16 up rows, the results 16
+//          activations).  It works if its pair is the first with that expert, for every pair with it, sixteen at a time; the
+//          others leave at once.  Four waves divide K; their sums meet in LDS in wave order.
+//   down   A workgroup owns 8 output columns of every row, so that the sum over a row's slots stays inside it (in slot order, no
+//          scratch, no further launch).  Its eight waves take the experts in turn; an instruction serves two halves of K (operand
+//          rows and columns 0..7 the first half, 8..15 the second, only the two diagonal blocks mean anything).
+//
+// Measured over weights that go round several copies, row by row / here, us: 8 rows, 8 experts of which a row uses 2, width
+// 2,048, 1,408 columns an expert: up 31.3 / 19.7 (92 MB, 4.7 TB/s), down 17.3 / 12.6; 15 rows 51.9 / 20.1 and 28.9 / 14.0; 4 rows 18.4 /
+// 13.3 and 11.3 / 9.3; width 4,096, 3,584 columns, 8 rows: 135 / 85 and 69 / 48.  At one and two rows, which seldom share an expert,
+// the row-by-row kernels are as fast or faster (7.5 / 8.2 and 6.4 / 8.7; 11.7 / 12.7 and 7.6 / 8.0), hence the lower limit; many
+// experts of few columns are many short turns of the down kernel's waves (64 experts, 704 columns, 48 pairs: 27.4 / 28.5), hence
+// its limit on experts.
+#include "common.h"
+#include "kvcm_hip.h"
+
+namespace kvcm {
+
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+
+namespace {
+
+constexpr int kUnit = 64;      // k of a unit: 4 lanes x 16, one 128-byte line of a row
+
+union Frag {
+  uint4 u;
+  bf16x8 v;
+};
+
+// the n-th (from 0) set bit of pairs, or the first one where there are fewer
+__device__ __forceinline__ int nth_pair(unsigned long long pairs, int n, int most) {
+  int p = __ffsll(pairs) - 1;
+#pragma unroll 4
+  for (int i = 0; i < most && pairs; ++i, pairs &= pairs - 1) p = i == n ? __ffsll(pairs) - 1 : p;
+  return p;
+}
+
+// GATED: rows of the matrix are 2F, sixteen gate rows, sixteen up rows, ...; else F, and KIND 0 square(relu), 2 gelu
+constexpr int kUpWaves = 4, kUpTrip = 2;      // waves that divide K, units of a trip
+
+template <int KIND>
+__global__ void __launch_bounds__(kUpWaves * kWave, 3)
+    moe_few_up_kernel(const uint16_t* __restrict__ h, int ldh, const uint16_t* __restrict__ w_up, const int* __restrict__ chosen,
+                      uint16_t* __restrict__ act, int n, int K, int F, int top, int E, const float* __restrict__ in_weight) {
+  constexpr bool GATED = KIND == 1;
+  __shared__ f32x4 red[kUpWaves][2][kWave];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int mine = blockIdx.y;
+  const int ch = lane < n ? chosen[lane] : -1;
+  const int e = __builtin_amdgcn_readlane(ch, mine);
+  if (e < 0 || e >= E) return;
+  unsigned long long pairs = __ballot(ch == e);
+  if (__ffsll(pairs) - 1 != mine) return;
+  const int r = lane % 16, kq = lane / 16;
+  const int rows = GATED ? 2 * F : F;
+  const uint16_t* wrow = w_up + (size_t(e) * rows + size_t(blockIdx.x) * 32 + r) * K + kq * 16;
+  const size_t next = size_t(16) * K;
+  const int units = K / kUnit, u_lo = units * wave / kUpWaves, u_hi = units * (wave + 1) / kUpWaves;
+  struct Trip {
+    Frag w[2][kUpTrip][2], x[kUpTrip][2];
+  };
+  for (; pairs;) {      // (more than sixteen pairs of one expert: the weights again, from a cache)
+    const int count = __popcll(pairs) < 16 ? __popcll(pairs) : 16;
+    const uint16_t* xrow = h + size_t(nth_pair(pairs, r, 16) / top) * ldh + kq * 16;
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    auto request = [&](int u0, Trip& t) {      // past the slice: its last unit again, not multiplied
+#pragma unroll
+      for (int d = 0; d < kUpTrip; ++d) {
+        const size_t off = size_t(u0 + d < u_hi ? u0 + d : (u_hi > 0 ? u_hi - 1 : 0)) * kUnit;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          t.w[0][d][q].u = *reinterpret_cast<const uint4*>(wrow + off + q * 8);
+          t.w[1][d][q].u = *reinterpret_cast<const uint4*>(wrow + next + off + q * 8);
+          t.x[d][q].u = *reinterpret_cast<const uint4*>(xrow + off + q * 8);
+        }
+      }
+    };
+    auto multiply = [&](int u0, const Trip& t) {
+#pragma unroll
+      for (int d = 0; d < kUpTrip; ++d) {
+        if (u0 + d >= u_hi) break;      // uniform over the wave
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t.x[d][q].v, t.w[0][d][q].v, acc[0], 0, 0, 0);
+          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t.x[d][q].v, t.w[1][d][q].v, acc[1], 0, 0, 0);
+        }
+      }
+    };
+    if (u_lo < u_hi) {
+      Trip ta, tb;
+      request(u_lo, ta);
+      request(u_lo + kUpTrip, tb);
+      for (int u = u_lo; u < u_hi; u += 2 * kUpTrip) {
+        multiply(u, ta);
+        if (u + 2 * kUpTrip < u_hi) request(u + 2 * kUpTrip, ta);
+        multiply(u + kUpTrip, tb);
+        if (u + 3 * kUpTrip < u_hi) request(u + 3 * kUpTrip, tb);
+      }
+    }
+    red[wave][0][lane] = acc[0];
+    red[wave][1][lane] = acc[1];
+    __syncthreads();
+    // thread -> (pair m of this group, column c of a tile); results: column lane % 16, rows 4 (lane / 16) + i
+    const int m = threadIdx.x / 16, c = threadIdx.x % 16;
+    if (m < count) {
+      const int pair = nth_pair(pairs, m, 16);
+      const float g = in_weight ? in_weight[pair] : 1.f;
+      float z[2] = {0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kUpWaves; ++w)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) z[t] += red[w][t][m / 4 * 16 + c][m % 4];
+      if constexpr (GATED) {
+        act[size_t(pair) * F + size_t(blockIdx.x) * 16 + c] = float_to_bf16_bits(silu<bf16_t>(g * z[0]) * (g * z[1]));
+      } else {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const float y = g * z[t], p = fmaxf(y, 0.f);
+          act[size_t(pair) * F + size_t(blockIdx.x) * 32 + t * 16 + c] = float_to_bf16_bits(KIND == 2 ? gelu_exact<bf16_t>(y) : p * p);
+        }
+      }
+    }
+    for (int i = 0; i < count; ++i) pairs &= pairs - 1;
+    if (pairs) __syncthreads();      // the sums are read before the next group's are written
+  }
+}
+
+constexpr int kDownWaves = 8, kDownTrip = 4, kMostPairs = 64;
+
+__global__ void __launch_bounds__(kDownWaves * kWave, 2)
+    moe_few_down_kernel(const uint16_t* __restrict__ act, const uint16_t* __restrict__ w_down, const int* __restrict__ chosen,
+                        const float* __restrict__ weight, const float* __restrict__ add, float* __restrict__ out, int T, int F,
+                        int H, int top, int E) {
+  __shared__ float z[kMostPairs][8];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int n = T * top, n0 = blockIdx.x * 8;
+  const int em = threadIdx.x / 8, en = threadIdx.x % 8;      // the last step's (row, column)
+  const float start = add && em < T ? add[size_t(em) * H + n0 + en] : 0.f;
+  const int ch = lane < n ? chosen[lane] : -1;
+  unsigned long long left = __ballot(ch >= 0 && ch < E);
+  const int r = lane % 16, kq = lane / 16, half = r / 8, c = r % 8;
+  const int units = F / kUnit, n_main = units / 2, n_max = units - n_main;      // the second half may have a unit more
+  const int u_lo = half * n_main, cnt = half ? n_max : n_main;
+  struct Trip {
+    Frag w[kDownTrip][2], x[kDownTrip][2];
+  };
+  for (int i = 0; left; ++i) {      // the experts in the order of their first pair, each wave every eighth
+    const int e = __builtin_amdgcn_readlane(ch, __ffsll(left) - 1);
+    unsigned long long pairs = __ballot(ch == e);
+    left &= ~pairs;
+    if (i % kDownWaves != wave) continue;
+    const uint16_t* wrow = w_down + (size_t(e) * H + n0 + c) * F + kq * 16;
+    while (pairs) {      // (more than eight pairs of one expert: the weights again, from a cache)
+      const uint16_t* xrow = act + size_t(nth_pair(pairs, c, 8)) * F + kq * 16;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      auto request = [&](int j0, Trip& t) {      // past this half's slice: its last unit again (or the row's first), not multiplied
+#pragma unroll
+        for (int d = 0; d < kDownTrip; ++d) {
+          const int j = j0 + d < cnt ? j0 + d : (cnt > 0 ? cnt - 1 : 0);
+          const size_t off = size_t(u_lo + j < units ? u_lo + j : 0) * kUnit;
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            t.w[d][q].u = *reinterpret_cast<const uint4*>(wrow + off + q * 8);
+            t.x[d][q].u = *reinterpret_cast<const uint4*>(xrow + off + q * 8);
+          }
+        }
+      };
+      auto multiply = [&](int j0, const Trip& t) {
+#pragma unroll
+        for (int d = 0; d < kDownTrip; ++d) {
+          const int j = j0 + d;
+          if (j >= n_max) break;      // uniform over the wave
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            Frag x = t.x[d][q], w = t.w[d][q];
+            if (j >= n_main && j >= cnt) {      // this half has run out: it adds nothing
+              x.u = uint4{0u, 0u, 0u, 0u};
+              w.u = uint4{0u, 0u, 0u, 0u};
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, w.v, acc, 0, 0, 0);
+          }
+        }
+      };
+      if (n_max > 0) {
+        Trip ta, tb;
+        request(0, ta);
+        request(kDownTrip, tb);
+        for (int j = 0; j < n_max; j += 2 * kDownTrip) {
+          multiply(j, ta);
+          if (j + 2 * kDownTrip < n_max) request(j + 2 * kDownTrip, ta);
+          multiply(j + kDownTrip, tb);
+          if (j + 3 * kDownTrip < n_max) request(j + 3 * kDownTrip, tb);
+        }
+      }
+      // results: column lane % 16, rows 4 (lane / 16) + i.  Pairs 0..7 of columns 0..7 over the first half are in lanes with column < 8
+      // of the first two lane groups, the second half's in lanes with column >= 8 of the last two: 40 lanes apart
+      const int count = __popcll(pairs) < 8 ? __popcll(pairs) : 8;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float far = __shfl(acc[q], (lane + 40) % kWave, kWave);
+        const int m = 4 * kq + q;
+        if (lane < 32 && r < 8 && m < count) z[nth_pair(pairs, m, 8)][c] = acc[q] + far;
+      }
+      for (int k = 0; k < count; ++k) pairs &= pairs - 1;
+    }
+  }
+  __syncthreads();
+  if (em >= T) return;
+  float sum = 0.f;
+  for (int s = 0; s < top; ++s) {
+    const int pair = em * top + s, e = chosen[pair];
+    if (e < 0 || e >= E) continue;
+    sum = fmaf(weight ? weight[pair] : 1.f, z[pair][en], sum);
+  }
+  out[size_t(em) * H + n0 + en] = add ? start + sum : sum;
+}
+
+}  // namespace
+
+constexpr int kFewRows = 3, kDownExperts = 32;      // from as many rows, up to as many experts: see the figures above
+
+bool moe_few_up_takes(int dtype, const void* h, int ldh, int T, int K, int F, int top) {
+  return dtype == kBF16 && T >= kFewRows && static_cast<long long>(T) * top <= kMostPairs && K % kUnit == 0 && F % 32 == 0 && ldh % 8 == 0 &&
+         reinterpret_cast<uintptr_t>(h) % 16 == 0;
+}
+
+bool moe_few_down_takes(int dtype, const void* act, int T, int F, int H, int top, int E) {
+  return dtype == kBF16 && T >= kFewRows && E <= kDownExperts && static_cast<long long>(T) * top <= kMostPairs && T <= kWave && F % kUnit == 0 && H % 8 == 0 &&
+         reinterpret_cast<uintptr_t>(act) % 16 == 0;
+}
+
+// (for the parts: do both products of T rows come here, whatever their strides?)
+extern "C" int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E) {
+  return moe_few_up_takes(kBF16, nullptr, 0, T, K, F, top) && moe_few_down_takes(kBF16, nullptr, T, F, H, top, E);
+}
+
+void launch_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
+                       const float* in_weight, hipStream_t s) {
+  const dim3 grid((kind == 1 ? 2 * F : F) / 32, T * top);
+#define KVCM_FEW_UP(KIND)                                                                                                       \
+  moe_few_up_kernel<KIND><<<grid, kUpWaves * kWave, 0, s>>>(static_cast<const uint16_t*>(h), ldh, static_cast<const uint16_t*>(w_up), chosen, \
+                                               static_cast<uint16_t*>(act), T * top, K, F, top, E, in_weight)
+  if (kind == 1) KVCM_FEW_UP(1);
+  else if (kind == 2) KVCM_FEW_UP(2);
+  else KVCM_FEW_UP(0);
+#undef KVCM_FEW_UP
+}
+
+void launch_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T,
+                         int F, int H, int top, int E, hipStream_t s) {
+  moe_few_down_kernel<<<H / 8, kDownWaves * kWave, 0, s>>>(static_cast<const uint16_t*>(act), static_cast<const uint16_t*>(w_down), chosen,
+                                                           weight, add, out, T, F, H, top, E);
+}
+
+}  // namespace kvcm

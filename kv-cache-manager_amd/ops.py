@@ -114,6 +114,7 @@ def _declare(lib):
     fn("kvcm_moe_table_route", vp, vp, i, i, i, vp, vp, i, vp)
     fn("kvcm_moe_up", vp, i, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
     fn("kvcm_moe_down", vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, vp)
+    fn("kvcm_moe_few_takes", i, i, i, i, i, i)
     fn("kvcm_moe_grouped_supported", i, i, i)
     fn("kvcm_moe_grouped_max_tiles", i, i)
     fn("kvcm_moe_grouped", vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, vp)
@@ -1744,6 +1745,13 @@ def moe_rows(h, w_up, w_down, chosen, weight, act, out, gated=False, add=None, a
           _expert_kind(gated, activation), _ptr(weight) if weigh_input else 0, _stream())
     _call("kvcm_moe_down", _ptr(act), _DT[act.dtype], _ptr(w_down), _ptr(chosen), 0 if weigh_input else _ptr(weight), _ptr(add), _ptr(out), T, F, H, top, E, _stream())
     return out
+
+
+def moe_few_takes(h, F, H, top, E):
+    """Does ``moe_rows`` run rows h [T, K] on the matrix cores, an expert's weights read once for all the rows that chose it?
+    (A few rows, up to 64 (row, slot) pairs.)"""
+    return (h.dtype == torch.bfloat16 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0
+            and bool(lib().kvcm_moe_few_takes(h.shape[0], h.shape[1], int(F), int(H), int(top), int(E))))
 
 
 def moe_grouped_supported(K, F, E, dtype):

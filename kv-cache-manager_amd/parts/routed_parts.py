@@ -186,7 +186,10 @@ class RoutedExperts(JoinableEnds, FeedForward):
         how = dict(gated=self.gated, add=add, weigh_input=p.get("weigh") == "input", **({} if self.gated else {"activation": self.activation}))
         act = step.ws("routed_act", (T, top * F)).view(T * top, F)
         out = step.ws("routed_out", (T, H), torch.float32)
-        if T >= self.GROUPED_MIN_ROWS and ops.moe_grouped_supported(H, F, E, act.dtype) and h.stride(0) % 8 == 0:
+        # up to 64 pairs moe_rows reads an expert once for all its rows too, without grouping (us a layer of 8 experts, two a row, 1,408 columns
+        # of 2,048: 16 rows 47 grouped, 31 so; 32 rows 47 and 39; width 4,096, 3,584 columns: 183 and 144, 183 and 173)
+        few = ops.moe_few_takes(h, F, H, top, E)
+        if T >= self.GROUPED_MIN_ROWS and not few and ops.moe_grouped_supported(H, F, E, act.dtype) and h.stride(0) % 8 == 0:
             # many rows: the pairs grouped by expert, tiles on the matrix cores, every expert's weights read once per tile
             order = step.ws("routed_order", (T, top), torch.int32)
             tiles = step.flat("routed_tiles", ops.moe_grouped_tiles(max(T, step.limits.max_tokens if step.limits else T) * top, E), torch.int32)

@@ -1,5 +1,5 @@
 """The routed experts' products on the matrix cores at the edges of their tiles, against 64 bits: grouped by expert (steps of many
-rows)."""
+rows) and expert by expert without grouping (a few rows)."""
 import pytest
 import torch
 
@@ -87,3 +87,25 @@ def test_grouped_tiles(shape, weigh_input):
     T, E, top, K, F, H, kind, one = shape
     chosen = torch.zeros(T, top, dtype=torch.long) if one else None
     _check("grouped", _case(T, E, top, K, F, H, kind, T + K, chosen), kind, weigh_input, not weigh_input)
+
+
+# (rows, experts, experts a row, K, F, H): one unit of 64 for eight or four waves, odd units, more than 8 and 16 pairs of one expert
+# ("one"), an expert named twice by a row, and numbers that name none
+FEW = [(3, 8, 2, 64, 64, 8, "silu", None), (15, 8, 2, 448, 192, 136, "relu2", None), (20, 3, 3, 128, 128, 64, "gelu", None),
+       (32, 4, 2, 320, 64, 72, "silu", "one"), (9, 40, 7, 192, 96, 24, "relu2", None), (10, 6, 2, 128, 320, 16, "silu", "odd"),
+       (17, 5, 1, 64, 448, 40, "gelu", "one"), (64, 8, 1, 576, 64, 8, "silu", None)]
+
+
+@pytest.mark.parametrize("weigh_input", [False, True])
+@pytest.mark.parametrize("shape", FEW)
+def test_few_rows(shape, weigh_input):
+    T, E, top, K, F, H, kind, how = shape
+    chosen = None
+    if how == "one":
+        chosen = torch.full((T, top), E - 1)
+        chosen[:, 0] = torch.arange(T) % 7 // 6 * (E - 2)      # six rows of seven choose expert 0
+    elif how == "odd":
+        chosen = torch.stack([torch.arange(T) % E, torch.arange(T) % 3], 1)
+        chosen[2] = 4
+        chosen[5, 0], chosen[7] = -1, E
+    _check("few", _case(T, E, top, K, F, H, kind, T + K, chosen), kind, weigh_input, not weigh_input)
