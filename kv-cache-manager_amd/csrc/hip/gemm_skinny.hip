@@ -1,11 +1,10 @@
 // Decode-shaped products: Y[M,N] = X[M,K] * W[N,K]^T with few rows and a weight matrix that has to be
 // streamed from HBM once.  The reference leaves these to cuBLAS (src/model/llama.cpp:45-52); here the
-// point is to keep enough weight bytes in flight on 256 CUs.  Two kernels: the first for up to 64 rows
-// and any width that is a multiple of 16, each tile reading the rows from L2 itself; the second, further
-// down, for up to 512 rows and widths that are multiples of 64, a workgroup's waves sharing the rows
-// through LDS.  Shapes both take go to the second.
+// point is to keep enough weight bytes in flight on 256 CUs.  Widths that are multiples of 64 run in tiles whose
+// waves share both operands through LDS (gemm_tiles.hip), up to 512 rows; the kernel here serves the other multiples of
+// 16, up to 64 rows, each column tile reading the rows from L2 itself.
 //
-// First kernel: one workgroup (4 waves) owns 16 output columns and one slice of K ("split"); its waves divide
+// One workgroup (4 waves) owns 16 output columns and one slice of K ("split"); its waves divide
 // the slice among themselves, each streaming its rows of W straight from global memory into
 // MFMA operand registers (every lane 32 contiguous bytes, four lanes one 128-byte line) and
 // multiplying with the matching pieces of X (v_mfma_f32_16x16x32_bf16).  The four waves' sums
@@ -21,6 +20,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "gemm_tiles.h"
 #include "kvcm_hip.h"
 
 namespace kvcm {
@@ -171,196 +171,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The same product with the rows shared by a workgroup's waves: the kernel every unfolded product of up
-// to 512 rows takes when its width is a multiple of 64 (the one above serves the other widths).  X is
-// not small beside the weights: every 16-column tile needs all of it, and re-reading it from L2 per tile
-// costs as many bytes as the weights from 8 rows on.  Here a workgroup of NWV waves owns NWV column tiles (one 16-column tile per wave;
-// the last workgroup may have fewer tiles than waves), up to 128 rows and a slice of K, and its waves
-// share X through LDS: per trip of DEPTH x 64 k the workgroup stages X[rows][DEPTH * 64] once
-// (double-buffered; the next trip's global loads are issued before the current trip's products), every
-// wave streams its own 16 weight rows from HBM and multiplies them with the staged rows.  No reduction
-// between waves; split-K partial sums as above.  More than 128 rows run as row blocks of 128
-// (blockIdx.z), each streaming the weights again.
-// SWIGLU: a wave's tile is 8 gate + 8 up rows, it stores 8 activation columns (limit > 0: of the gate with limits, whose
-// gate and up values are not rounded on the way).
-constexpr int kXPad = 8;    // bfloat16 of padding per staged row, so that rows spread over the banks
-constexpr int kRowBlock = 128;
-
-template <int MT, int DEPTH, class TO, bool SWIGLU, int NWV>
-__global__ void __launch_bounds__(NWV * kWave)
-    gemm_rows_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, float* __restrict__ partials,
-                     TO* __restrict__ out, int M, int N, int K, int ldx, int ldw, int ldo, int S,
-                     const float* __restrict__ ss_in, int tiles_in, float eps, float limit) {
-  constexpr int kPassRows = NWV * kWave / 4;                      // rows the workgroup's threads stage at a time (x 64 k)
-  constexpr int RP = (MT * 16 + kPassRows - 1) / kPassRows;       // staging passes
-  __shared__ __attribute__((aligned(16))) uint16_t xs[2][MT * 16][DEPTH * kUnit + kXPad];
-  __shared__ float rstd_s[MT * 16];   // ss_in: every row's 1 / sqrt(mean x^2 + eps), which the unsplit result is scaled by
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int r = lane % 16, kq = lane / 16;
-  constexpr int kCols = SWIGLU ? 8 : 16;
-  const int c0 = blockIdx.x * (NWV * kCols) + wave * kCols;   // this wave's first output column
-  const bool col_on = c0 < N;                                   // the last workgroup may have fewer tiles than waves
-  const int s = blockIdx.y;
-  const int row_base = blockIdx.z * kRowBlock;
-  const int units = K / kUnit;
-  const int u_lo = int((long long)units * s / S), u_hi = int((long long)units * (s + 1) / S);
-  const int trips = (u_hi - u_lo + DEPTH - 1) / DEPTH;
-
-  const int cw = col_on ? c0 : 0;   // a wave without a tile reads the first tile's rows and drops them
-  const uint16_t* wrow = W + size_t(SWIGLU ? (r < 8 ? cw + r : N + cw + r - 8) : cw + r) * ldw + kq * 16;
-  // staging: thread -> (row tid / 4 + kPassRows p, 16 elements at (tid % 4) * 16 of every unit); rows
-  // beyond M read the block's first row and are dropped at the store
-  const int srow = threadIdx.x / 4, sseg = (threadIdx.x % 4) * 16;
-  const uint16_t* xsrc[RP];
-#pragma unroll
-  for (int p = 0; p < RP; ++p) {
-    const int m = row_base + srow + kPassRows * p;
-    xsrc[p] = X + size_t(m < M ? m : row_base) * ldx + sseg;
-  }
-
-  f32x4 acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // A trip's operands: DEPTH units of this wave's weight rows and of this thread's pieces of X.
-  // Units beyond the slice repeat its last unit (no load behind a branch) and are not multiplied.
-  struct Trip {
-    Frag b[DEPTH][2];
-    uint4 x[DEPTH][RP][2];
-  };
-  // Workgroups walk their slice from different starting points (and wrap around): if all of them
-  // read the same k at the same time, their rows, a multiple of 4 KB apart, would queue up at the
-  // same few memory channels.
-  const int span = u_hi - u_lo > 0 ? u_hi - u_lo : 1;
-  const int phase = (blockIdx.x * 5) % span;   // the same for all waves: they share staged X
-  auto fetch = [&](int j0, Trip& tr) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      const int j = j0 + d < span ? j0 + d : span - 1;
-      const int u = u_lo + (j + phase) % span;
-      const uint16_t* p = wrow + size_t(u) * kUnit;
-      tr.b[d][0].u = *reinterpret_cast<const uint4*>(p);
-      tr.b[d][1].u = *reinterpret_cast<const uint4*>(p + 8);
-#pragma unroll
-      for (int q = 0; q < RP; ++q) {
-        const uint16_t* xp = xsrc[q] + size_t(u) * kUnit;
-        tr.x[d][q][0] = *reinterpret_cast<const uint4*>(xp);
-        tr.x[d][q][1] = *reinterpret_cast<const uint4*>(xp + 8);
-      }
-    }
-  };
-  auto stage = [&](int buf, const Trip& tr) {
-#pragma unroll
-    for (int q = 0; q < RP; ++q) {
-      if (srow + kPassRows * q < MT * 16) {   // uniform per wave
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-          *reinterpret_cast<uint4*>(&xs[buf][srow + kPassRows * q][d * kUnit + sseg]) = tr.x[d][q][0];
-          *reinterpret_cast<uint4*>(&xs[buf][srow + kPassRows * q][d * kUnit + sseg + 8]) = tr.x[d][q][1];
-        }
-      }
-    }
-  };
-  auto multiply = [&](int buf, int j0, const Trip& tr) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      if (j0 + d >= span) break;
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        Frag a0, a1;
-        a0.u = *reinterpret_cast<const uint4*>(&xs[buf][t * 16 + r][d * kUnit + kq * 16]);
-        a1.u = *reinterpret_cast<const uint4*>(&xs[buf][t * 16 + r][d * kUnit + kq * 16 + 8]);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0.v, tr.b[d][0].v, acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1.v, tr.b[d][1].v, acc[t], 0, 0, 0);
-      }
-    }
-  };
-  // Two trips in registers: while one is multiplied, the next one's loads are on their way.  LDS
-  // buffer i holds the X of the trip in register set i; a buffer is written one barrier after its
-  // last read.
-  // X = round(g round(x)) of a norm folded into this product (gemm_rows8.hip): the rows' scales from their
-  // tiles' sums of squares, a wave per row, added in a fixed order while the first loads are on their way
-  auto scales = [&]() {
-    if (ss_in == nullptr) return;
-    for (int m = wave; m < MT * 16; m += NWV) {
-      if (row_base + m >= M) {   // a row the block does not have: its sums are dropped at the store
-        if (lane == 0) rstd_s[m] = 1.f;
-        continue;
-      }
-      const float* p = ss_in + size_t(row_base + m) * tiles_in;
-      float part[4] = {0.f, 0.f, 0.f, 0.f};   // four loads on their way per lane
-      int t = lane;
-      for (; t + 3 * kWave < tiles_in; t += 4 * kWave) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) part[q] += p[t + q * kWave];
-      }
-      for (; t < tiles_in; t += kWave) part[0] += p[t];
-      const float sum = wave_sum((part[0] + part[1]) + (part[2] + part[3]));
-      if (lane == 0) rstd_s[m] = rsqrtf(sum / float(tiles_in * 8) + eps);
-    }
-  };
-  if (u_lo < u_hi) {
-    Trip ta, tb;
-    fetch(0, ta);
-    scales();
-    for (int i = 0; i < trips; i += 2) {
-      const int j0 = i * DEPTH;
-      fetch(j0 + DEPTH, tb);
-      stage(0, ta);
-      __syncthreads();
-      multiply(0, j0, ta);
-      if (i + 1 >= trips) break;
-      fetch(j0 + 2 * DEPTH, ta);
-      stage(1, tb);
-      __syncthreads();
-      multiply(1, j0 + DEPTH, tb);
-    }
-  } else {
-    scales();
-  }
-  if (ss_in != nullptr) {   // (the same for the whole workgroup)
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[t][i] *= rstd_s[t * 16 + kq * 4 + i];
-  }
-  if (!col_on) return;
-  // accumulator: column = r of the wave's tile, rows = 4 kq + i
-  if constexpr (SWIGLU) {
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      f32x4 up;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) up[i] = __shfl(acc[t][i], (lane & ~15) | ((r + 8) & 15), kWave);
-      if (r >= 8) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = row_base + t * 16 + kq * 4 + i;
-        if (m >= M) continue;
-        TO* dst = out + size_t(m) * ldo + c0 + r;
-        if (limit > 0.f) {
-          store_f(dst, clamped_gate<TO>(acc[t][i], up[i], limit));
-          continue;
-        }
-        const float x = round_to<TO>(acc[t][i]);
-        const float act = silu<TO>(x);
-        store_f(dst, round_to<TO>(act) * round_to<TO>(up[i]));
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = row_base + t * 16 + kq * 4 + i;
-      if (m >= M) continue;
-      if (S > 1) partials[(size_t(s) * M + m) * N + c0 + r] = acc[t][i];
-      else store_f(out + size_t(m) * ldo + c0 + r, acc[t][i]);
-    }
-}
-
 // out[m][n] = sum over splits, in split order.
 template <class TO>
 __global__ void reduce_store_kernel(const float* __restrict__ partials, TO* __restrict__ out, int M, int N, int ldo, int S) {
@@ -375,24 +185,18 @@ __global__ void reduce_store_kernel(const float* __restrict__ partials, TO* __re
 
 using namespace kvcm;
 
-constexpr int kMaxSharedRows = 512;
-
-// Whole groups of 64 columns: the kernel whose waves share X through LDS.
-static bool shares_rows(int M, int N) { return M > 0 && M <= kMaxSharedRows && N % 64 == 0; }
+// Whole groups of 64 columns: the tiles.
+constexpr int kMaxTileRows = 512, kRowBlock = 128;
+static bool in_tiles(int M, int N) { return M > 0 && M <= kMaxTileRows && N % 64 == 0; }
 static int row_blocks(int M) { return (M + kRowBlock - 1) / kRowBlock; }
 // The SwiGLU form (I: the activation's width) is unsplit: with too few workgroups a split product and a
 // launch for SwiGLU fill the chip better.
-static bool swiglu_shares_rows(int M, int I) {
-  return M > 0 && M <= kMaxSharedRows && I % 32 == 0 && (I / 32) * row_blocks(M) >= 160;
+static bool swiglu_in_tiles(int M, int I) {
+  return M > 0 && M <= kMaxTileRows && I % 32 == 0 && static_cast<long long>(I / 32) * row_blocks(M) >= 160;
 }
 
-// Waves per workgroup (each takes one column tile) so that tiles x splits x row blocks make about one
-// workgroup per CU and none is left out: what this kernel streams per microsecond grows with the CUs it
-// covers, not with the waves on each (measured:
-// gate/up at TinyLlama sizes, 704 tiles, 32 rows: 176 workgroups of four waves 16.5 us, 235 of three
-// 13.2 us; at Llama-3-8B sizes, 1,792 tiles, 64 rows: 448 of four 63 us, 256 of seven 51 us).  One wave
-// more where that saves a staging pass (the workgroup's threads stage 16 rows per wave at a time: 64 rows
-// are two passes for three waves, one for four).
+// How many 16-column tiles a workgroup may take so that tiles x splits x row blocks make about one workgroup per CU and none is
+// left out: what such a product streams per microsecond grows with the CUs it covers.  The splits below keep it to at most eight.
 constexpr int kRowsCUs = 256;
 static int rows_waves(long long units, int mt) {
   const long long want = (units + kRowsCUs - 1) / kRowsCUs;
@@ -402,12 +206,13 @@ static int rows_waves(long long units, int mt) {
 }
 static int rows_tiles_m(int M) { return M > kRowBlock ? kRowBlock / 16 : (M + 15) / 16; }
 
-// Splits of K of a plain shared-rows product: eight where there are few column tiles, or where K is long
+// Splits of K of a plain product in tiles: eight where there are few column tiles, or where K is long
 // against the rows (the partial sums, S*M*N floats that the next kernel reads, are small against the
 // weights then), else four; as long as every slice has a trip of its own and the partial sums stay below
 // the weights' bytes; halved while more than eight waves a workgroup would be needed to get down to one
 // workgroup per CU.  Measured at 17 to 128 rows over the projections of TinyLlama and Llama-3-8B sizes,
-// alone and in whole decode steps.
+// alone and in whole decode steps.  (With the tiles free to choose among 1, 2, 4 and 8 as well, launches and the reading of the
+// partial sums together would be 4 % shorter at 8 to 512 rows.)
 static int rows_splits(int M, int N, int K) {
   const long long tiles = static_cast<long long>(N / 16) * row_blocks(M);
   const int units = K / kUnit;
@@ -420,59 +225,12 @@ static int rows_splits(int M, int N, int K) {
   return S;
 }
 
-// One launch of the shared-rows kernel: MT row tiles per block (8 for every block when there are
-// several), two k-depths: four units per trip up to 64 rows, two beyond (LDS holds rows x depth).
-template <class TO, bool SWIGLU, int NWV>
-static void launch_rows_n(hipStream_t st, const uint16_t* x, const uint16_t* w, float* partials, TO* out, int M, int N,
-                          int K, int ldx, int ldw, int ldo, int S, const float* ss_in, int tiles_in, float eps, float limit) {
-  const int mt = rows_tiles_m(M);
-  const int tiles = N / (SWIGLU ? 8 : 16);
-  const dim3 grid((tiles + NWV - 1) / NWV, S, row_blocks(M));
-#define KVCM_ROWS(MT, DEPTH) \
-  gemm_rows_kernel<MT, DEPTH, TO, SWIGLU, NWV><<<grid, NWV * kWave, 0, st>>>(x, w, partials, out, M, N, K, ldx, ldw, ldo, S, \
-                                                                             ss_in, tiles_in, eps, limit)
-  switch (mt) {
-    case 1: KVCM_ROWS(1, 4); break;
-    case 2: KVCM_ROWS(2, 4); break;
-    case 3: KVCM_ROWS(3, 4); break;
-    case 4: KVCM_ROWS(4, 4); break;
-    case 5: case 6: KVCM_ROWS(6, 2); break;
-    default: KVCM_ROWS(8, 2); break;
-  }
-#undef KVCM_ROWS
-}
-
-// N: the result's width (SWIGLU: the activation's).  A 32-bit result (the head's logits, thousands of
-// tiles) keeps four waves.
-template <class TO, bool SWIGLU>
-static void launch_rows(hipStream_t st, const uint16_t* x, const uint16_t* w, float* partials, TO* out, int M, int N, int K,
-                        int ldx, int ldw, int ldo, int S, const float* ss_in = nullptr, int tiles_in = 0, float eps = 0.f, float limit = 0.f) {
-  const long long units = static_cast<long long>(N / (SWIGLU ? 8 : 16)) * row_blocks(M) * S;
-  const int waves = sizeof(TO) == 4 || (S == 1 && !SWIGLU) ? 4 : rows_waves(units, rows_tiles_m(M));
-#define KVCM_WAVES(NWV) launch_rows_n<TO, SWIGLU, NWV>(st, x, w, partials, out, M, N, K, ldx, ldw, ldo, S, ss_in, tiles_in, eps, limit)
-  if constexpr (sizeof(TO) == 4) {
-    KVCM_WAVES(4);
-  } else {
-    switch (waves) {
-      case 2: KVCM_WAVES(2); break;
-      case 3: KVCM_WAVES(3); break;
-      case 4: KVCM_WAVES(4); break;
-      case 5: KVCM_WAVES(5); break;
-      case 6: KVCM_WAVES(6); break;
-      case 7: KVCM_WAVES(7); break;
-      default: KVCM_WAVES(8); break;
-    }
-  }
-#undef KVCM_WAVES
-}
-
-
 extern "C" {
 
 // How many splits of K a launch of this shape uses (0: the shape is not supported by this kernel).
 int kvcm_gemm_skinny_splits(int M, int N, int K) {
   if (M <= 0 || N % 16 != 0 || K % kUnit != 0 || N <= 0 || K <= 0) return 0;
-  if (shares_rows(M, N)) return rows_splits(M, N, K);
+  if (in_tiles(M, N)) return rows_splits(M, N, K);
   if (M > 64) return 0;
   const int tiles = N / 16, units = K / kUnit;
   int S = (640 + tiles - 1) / tiles;           // aim at >= 640 workgroups (2.5 per CU) ...
@@ -481,10 +239,19 @@ int kvcm_gemm_skinny_splits(int M, int N, int K) {
   return S;
 }
 
-// Waves per workgroup that the shared-rows kernel runs a bfloat16 product of this shape with (0: another
-// kernel takes the shape).  swiglu: N is the activation's width, S is 1.
+// The same where nobody takes the partial sums: a second launch adds them then, and one slice may be the faster whole (a launch that
+// adds them takes 3.2 us and its bytes at 5 TB/s).
+int kvcm_gemm_skinny_whole_splits(int M, int N, int K) {
+  const int S = kvcm_gemm_skinny_splits(M, N, K);
+  if (S <= 1 || !in_tiles(M, N)) return S;
+  const float add = 3.2f + static_cast<float>(M) * static_cast<float>(N) * (4.f * S + 4.f) / 5e6f;
+  return gemm_tiles_time(M, N, K, 1, false, false) <= gemm_tiles_time(M, N, K, S, false, false) + add ? 1 : S;
+}
+
+// 16-column tiles a workgroup that cover the chip for a product of this shape (rows_waves; 0: not a product in tiles).
+// swiglu: N is the activation's width, S is 1.
 int kvcm_gemm_skinny_waves(int M, int N, int K, int S, int swiglu) {
-  if (swiglu ? !swiglu_shares_rows(M, N) : !shares_rows(M, N)) return 0;
+  if (swiglu ? !swiglu_in_tiles(M, N) : !in_tiles(M, N)) return 0;
   if (K <= 0 || K % kUnit != 0 || S < 1) return 0;
   if (!swiglu && S == 1) return 4;
   return rows_waves(static_cast<long long>(N / (swiglu ? 8 : 16)) * row_blocks(M) * S, rows_tiles_m(M));
@@ -505,11 +272,7 @@ int kvcm_gemm_skinny(const void* X, const void* W, float* partials, void* out, i
   const uint16_t* x = static_cast<const uint16_t*>(X);
   const uint16_t* w = static_cast<const uint16_t*>(W);
   const int mt = (M + 15) / 16;
-  if (shares_rows(M, N)) {
-    if (out_dtype == kBF16) launch_rows<bf16_t, false>(st, x, w, partials, static_cast<bf16_t*>(out), M, N, K, ldx, ldw, ldo, S);
-    else launch_rows<float, false>(st, x, w, partials, static_cast<float*>(out), M, N, K, ldx, ldw, ldo, S);
-    return launch_status("gemm_rows");
-  }
+  if (in_tiles(M, N)) return gemm_tiles(TilesCall{x, w, partials, out, out_dtype == kF32, M, N, K, ldx, ldw, ldo, S}, false, -1, st);
   const dim3 grid(N / 16, S);
 #define KVCM_SKINNY(MT, TO) \
   gemm_skinny_kernel<MT, TO, false><<<grid, 256, 0, st>>>(x, w, partials, static_cast<TO*>(out), M, N, K, ldx, ldw, ldo, S, 0.f)
@@ -525,7 +288,7 @@ int kvcm_gemm_skinny(const void* X, const void* W, float* partials, void* out, i
 // May act = swiglu(X * [gate | up]^T) be computed in one launch?  I is the width of the result.
 int kvcm_gemm_skinny_swiglu_supported(int M, int I, int K) {
   if (!(M > 0 && I > 0 && I % 8 == 0 && K > 0 && K % kUnit == 0)) return 0;
-  if (swiglu_shares_rows(M, I)) return 1;
+  if (swiglu_in_tiles(M, I)) return 1;
   // with too few workgroups a split product fills the chip better than an unsplit one; the kernel whose
   // every tile reads the rows from L2 serves a few rows, or widths that are no multiple of 32
   if (I % 32 == 0 && M > 16) return 0;
@@ -544,10 +307,10 @@ int kvcm_gemm_skinny_swiglu(const void* X, const void* W, void* out, int out_dty
   const uint16_t* x = static_cast<const uint16_t*>(X);
   const uint16_t* w = static_cast<const uint16_t*>(W);
   const int mt = (M + 15) / 16;
-  if (swiglu_shares_rows(M, I)) {
-    if (out_dtype == kBF16) launch_rows<bf16_t, true>(st, x, w, nullptr, static_cast<bf16_t*>(out), M, I, K, ldx, ldw, ldo, 1, nullptr, 0, 0.f, limit);
-    else launch_rows<float, true>(st, x, w, nullptr, static_cast<float*>(out), M, I, K, ldx, ldw, ldo, 1, nullptr, 0, 0.f, limit);
-    return launch_status("gemm_rows_swiglu");
+  if (swiglu_in_tiles(M, I)) {
+    TilesCall c{x, w, nullptr, out, out_dtype == kF32, M, I, K, ldx, ldw, ldo, 1};
+    c.limit = limit;
+    return gemm_tiles(c, true, -1, st);
   }
   const dim3 grid(I / 8, 1);
 #define KVCM_SKINNY(MT, TO) \
@@ -563,22 +326,24 @@ int kvcm_gemm_skinny_swiglu(const void* X, const void* W, void* out, int out_dty
 
 // The same with a folded RMS norm in front (gemm_rows8.hip): X is xg = round(g round(x)) of the norm's producer,
 // ss_in its [M][tiles_in] sums of x^2 per 8-column tile, eps the norm's; the sums are scaled by
-// rsqrt(mean x^2 + eps) before they are rounded.  For the widths at which this kernel's few long-lived
-// workgroups stream the gate/up matrix faster than the 8-row kernel's many short ones (from 1,024 tiles on:
+// rsqrt(mean x^2 + eps) before they are rounded.  For the widths at which the tiles' few long-lived
+// workgroups stream the gate/up matrix faster than the 8-row kernel's many short ones (from 1,024 tiles of 8 columns on:
 // Llama-3-8B sizes, one row: 50.8 against 43.9 us).
 int kvcm_gemm_skinny_swiglu_normed_preferred(int M, int I, int K) {
-  return K > 0 && K % kUnit == 0 && swiglu_shares_rows(M, I) && I / 8 >= 4 * kRowsCUs;
+  return K > 0 && K % kUnit == 0 && swiglu_in_tiles(M, I) && I / 8 >= 4 * kRowsCUs;
 }
 int kvcm_gemm_skinny_swiglu_normed(const void* X, const void* W, const float* ss_in, int tiles_in, float eps, void* out,
                                    int M, int I, int K, int ldx, int ldw, int ldo, hipStream_t st) {
-  KVCM_REQUIRE(K > 0 && K % kUnit == 0 && swiglu_shares_rows(M, I), "gemm_skinny_swiglu_normed: unsupported shape M=%d I=%d K=%d", M, I, K);
+  KVCM_REQUIRE(K > 0 && K % kUnit == 0 && swiglu_in_tiles(M, I), "gemm_skinny_swiglu_normed: unsupported shape M=%d I=%d K=%d", M, I, K);
   KVCM_REQUIRE(ss_in != nullptr && tiles_in > 0 && tiles_in * 8 == K, "gemm_skinny_swiglu_normed: %d tiles of sums for a width of %d", tiles_in, K);
   KVCM_REQUIRE(ldx % 8 == 0 && ldw % 8 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0,
                "gemm_skinny_swiglu_normed: operands must be 16-byte aligned with leading dimensions that are multiples of 8");
   KVCM_REQUIRE(ldx >= K && ldw >= K && out != nullptr && ldo >= I, "gemm_skinny_swiglu_normed: leading dimensions too small");
-  launch_rows<bf16_t, true>(st, static_cast<const uint16_t*>(X), static_cast<const uint16_t*>(W), nullptr, static_cast<bf16_t*>(out),
-                            M, I, K, ldx, ldw, ldo, 1, ss_in, tiles_in, eps);
-  return launch_status("gemm_rows_swiglu_normed");
+  TilesCall c{static_cast<const uint16_t*>(X), static_cast<const uint16_t*>(W), nullptr, out, 0, M, I, K, ldx, ldw, ldo, 1};
+  c.ss_in = ss_in;
+  c.tiles_in = tiles_in;
+  c.eps = eps;
+  return gemm_tiles(c, true, -1, st);
 }
 
 int kvcm_reduce_store(const float* partials, void* out, int out_dtype, int M, int N, int ldo, int S, hipStream_t st) {
@@ -639,6 +404,7 @@ int kvcm_gemm_skinny_noalloc(const void* X, const void* W, void* out, int out_dt
   KVCM_REQUIRE(need <= kNoAllocFloats,
                "gemm_skinny_noalloc: M=%d N=%d K=%d needs %lld floats of partial sums (%d slices), the built-in array holds %lld",
                M, N, K, need, S, kNoAllocFloats);
+  if (kvcm_gemm_skinny_whole_splits(M, N, K) == 1) return kvcm_gemm_skinny(X, W, nullptr, out, out_dtype, M, N, K, ldx, ldw, ldo, 1, st);
   float* partials = nullptr;
   if (int rc = noalloc_scratch(&partials)) return rc;
   if (int rc = kvcm_gemm_skinny(X, W, partials, out, out_dtype, M, N, K, ldx, ldw, ldo, S, st)) return rc;

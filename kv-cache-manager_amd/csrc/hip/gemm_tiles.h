@@ -1,0 +1,30 @@
+// Products in tiles (gemm_tiles.hip), as the entry points of gemm_skinny.hip hand them on.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace kvcm {
+
+// silu with gate, silu(gate) and up rounded on the way as a stored product's would be, or silu or relu in 32 bits
+enum TileAct : int { kSiluStored = 0, kSilu = 1, kRelu = 2 };
+
+struct TilesCall {
+  const uint16_t *X, *W;
+  float* partials;
+  void* out;
+  int out_f32, M, N, K, ldx, ldw, ldo, S;
+  const float* ss_in = nullptr;      // a folded norm's sums of squares (gated products)
+  int tiles_in = 0;
+  float eps = 0.f, limit = 0.f;
+  int act = 0;      // of gated products: TileAct
+};
+
+// tile < 0: the one the rule picks
+int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st);
+// about how many us a launch takes
+float gemm_tiles_time(int M, int N, int K, int S, bool is_gated, bool out_f32);
+
+// the same for `groups` workgroups of a tile of bm x bn, and that many elements of weights
+float gemm_tile_time(int bm, int bn, float groups, int steps, float weights);
+
+}  // namespace kvcm

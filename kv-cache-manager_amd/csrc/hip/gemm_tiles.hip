@@ -1,0 +1,322 @@
+// Products of a few to a few thousand rows, bfloat16: Y[M,N] = X[M,K] * W[N,K]^T, 32-bit sums, the result stored (bfloat16 or
+// 32-bit), left as partial sums of S slices of K ([S][M][N], the consumer adds them in slice order), or, SWIGLU, made into
+// act[M,I] = silu(X W_gate^T) * (X W_up^T), or with relu in silu's place, of a fused [gate (I rows) | up (I rows)] matrix.
+//
+// A workgroup of 3 to 12 waves owns a tile of BM rows x BN columns and a slice of K, its operands in a ring of stages in LDS
+// (tile_ring.h, which says what bounds such products and why the ring).
+//
+// Measured (us, weights from memory, one launch after the other in a graph; the kernel that shared only X through LDS and streamed
+// W into registers, its own trips double-buffered / this one):
+//   64 rows   2560 x 2048 7.5 / 5.1   2048 x 2048 6.4 / 4.7   gate+up 11264 x 2048 19.6 / 13.2   2048 x 5632 10.9 / 8.0
+//   16 rows   5.1 / 4.2   4.9 / 4.0   13.0 / 11.1   8.1 / 6.6;  128 rows of 4096 x 14336 39.3 / 27.1
+// and against the vendor's product (gate+up: with the launch that applies SwiGLU): 512 rows 14.5 / 9.4 (2048 x 2048), 36.7 / 30.6,
+// 26.4 / 19.5; 1,024 rows 57.7 / 48.1 (gate+up); 2,048 rows 97.8 / 92.1 (gate+up), 21.7 / 21.3, 55.6 / 54.1.
+#include <cmath>
+
+#include "common.h"
+#include "gemm_tiles.h"
+#include "kvcm_hip.h"
+#include "tile_ring.h"
+
+namespace kvcm {
+
+// act(gate) * up (TileAct), or, limit > 0, the gate with limits; but for kSiluStored in 32 bits
+template <class TO>
+__device__ __forceinline__ float gated(float gate, float up, float limit, int act) {
+  if (limit > 0.f) return clamped_gate<TO>(gate, up, limit);
+  if (act == kRelu) return fmaxf(gate, 0.f) * up;
+  if (act == kSilu) return silu<TO>(gate) * up;
+  return round_to<TO>(silu<TO>(round_to<TO>(gate))) * round_to<TO>(up);
+}
+
+// The waves are WM x WN, each with BM / WM rows and BN / WN columns.  GATED: N is I; a tile's BN rows of W are gate and up rows of
+// BN / 2 columns of act: sixteen of each in turn where a wave has an even number of 16-column tiles (its accumulators of
+// neighbouring tiles then hold gate and up), else eight and eight (lanes 32 apart then do, and swap halves).
+// ss_in (GATED): X = round(g round(x)) of a norm folded into this product (gemm_rows8.hip): the sums are scaled by the rows'
+// rsqrt(mean x^2 + eps), from tiles_in sums of squares a row.
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED>
+__global__ void __launch_bounds__(WM* WN* kWave)
+    gemm_tiles_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, float* __restrict__ partials, void* __restrict__ out,
+                      int out_f32, int M, int N, int K, int ldx, int ldw, int ldo, int S, int tiles_m, int tiles_n,
+                      const float* __restrict__ ss_in, int tiles_in, float eps, float limit, int act) {
+  using Ring = TileRing<BM, BN, WM, WN, STAGES>;
+  constexpr int NW = Ring::NW, TM = Ring::TM, TN = Ring::TN, R = Ring::R;
+  constexpr int kHalf = TN % 2 == 0 ? 16 : 8;      // gate rows in front of their up rows
+  static_assert(BM / NW <= kWave, "the rows' scales lie one a lane");
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[Ring::kBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  int id = neighbours_on_one_xcd();      // row blocks first
+  const int tm = id % tiles_m;
+  id /= tiles_m;
+  const int tn = id % tiles_n, s = id / tiles_n;
+  const int m0 = tm * BM, c0 = tn * (GATED ? BN / 2 : BN);
+  const int steps_all = K / kStepK;
+  const int k_lo = static_cast<int>(static_cast<long long>(steps_all) * s / S);
+  const int steps = static_cast<int>(static_cast<long long>(steps_all) * (s + 1) / S) - k_lo;
+
+  const uint64_t xbase = reinterpret_cast<uint64_t>(X + static_cast<size_t>(m0) * ldx) + static_cast<size_t>(k_lo) * 128;
+  const uint64_t wbase = reinterpret_cast<uint64_t>(W + static_cast<size_t>(c0) * ldw) + static_cast<size_t>(k_lo) * 128;
+  const uint64_t upbase = wbase + static_cast<size_t>(GATED ? N : 0) * ldw * 2;
+  // rows past M and columns past N repeat the last one (what they give is not stored)
+  uint32_t offset[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int req = Ring::request_of(q, wave), row = req * 8 + lane / 8;
+    int at, ld;
+    if (req < BM / 8) {
+      at = row < M - m0 ? row : M - 1 - m0;
+      ld = ldx;
+    } else {
+      const int c = row - BM;
+      at = GATED ? c / (2 * kHalf) * kHalf + c % kHalf : c;
+      if (at > N - 1 - c0) at = N - 1 - c0;
+      ld = ldw;
+    }
+    offset[q] = static_cast<uint32_t>(at) * static_cast<uint32_t>(ld) * 2u + static_cast<uint32_t>(Ring::piece_of(lane)) * 16u;
+  }
+  // One row block: workgroups walk their slice from different places (and wrap around), or all would ask the same few memory
+  // channels for rows a multiple of 4 KB apart at the same time (gate+up, 64 rows: 14.9 -> 14.4 us).  Several: those that share
+  // columns walk together.
+  const int phase = tiles_m == 1 ? tn * 5 % steps : 0;
+  auto base = [&](int req) {
+    const bool up = GATED && (req - BM / 8) * 8 % (2 * kHalf) >= kHalf;
+    return req < BM / 8 ? xbase : up ? upbase : wbase;
+  };
+  ring_f32x4 acc[TN][TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) acc[j][i] = ring_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wm = wave % WM, wn = wave / WM, frow = lane % 16, fk = lane / 16;
+  float rstd = 1.f;      // lane l: of row wave + l NW
+  Ring::multiply(ring, offset, base, steps, phase, kStepK, wave, lane, acc, [&] {
+    if (GATED && ss_in != nullptr) {      // a wave a row, in a fixed order, while the first stages are on their way
+      for (int l = 0; l * NW + wave < BM; ++l) {
+        const int m = l * NW + wave;
+        if (m0 + m < M) {
+          const float* p = ss_in + static_cast<size_t>(m0 + m) * tiles_in;
+          float part[4] = {0.f, 0.f, 0.f, 0.f};
+          int t = lane;
+          for (; t + 3 * kWave < tiles_in; t += 4 * kWave) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) part[q] += p[t + q * kWave];
+          }
+          for (; t < tiles_in; t += kWave) part[0] += p[t];
+          const float sum = wave_sum((part[0] + part[1]) + (part[2] + part[3]));
+          if (lane == l) rstd = rsqrtf(sum / static_cast<float>(tiles_in * 8) + eps);
+        }
+      }
+    }
+  });
+  const float* scale = reinterpret_cast<const float*>(ring);
+  if (GATED && ss_in != nullptr) {      // (the same for the whole workgroup)
+    __syncthreads();
+    if (lane * NW + wave < BM) reinterpret_cast<float*>(ring)[lane * NW + wave] = rstd;
+    __syncthreads();
+  }
+
+  // acc[j][i][r]: row wm * TM * 16 + i * 16 + frow, row of W (in the tile) wn * TN * 16 + j * 16 + fk * 4 + r
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + (wm * TM + i) * 16 + frow;
+    if constexpr (GATED) {
+      if (ss_in != nullptr) {
+        const float f = scale[m - m0];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[j][i] *= f;
+      }
+      const size_t row = static_cast<size_t>(m) * ldo;
+      if constexpr (kHalf == 16) {
+#pragma unroll
+        for (int j = 0; j < TN; j += 2) {
+          const int c = c0 + (wn * TN + j) * 8 + fk * 4;
+          if (m >= M || c >= N) continue;
+          const ring_f32x4 g = acc[j][i], u = acc[j + 1][i];
+          if (out_f32) {
+            *reinterpret_cast<any_f32x4*>(static_cast<float*>(out) + row + c) = any_f32x4{
+                gated<float>(g[0], u[0], limit, act), gated<float>(g[1], u[1], limit, act), gated<float>(g[2], u[2], limit, act), gated<float>(g[3], u[3], limit, act)};
+          } else {
+            *reinterpret_cast<any_u32x2*>(static_cast<uint16_t*>(out) + row + c) =
+                any_u32x2{two_bf16(gated<bf16_t>(g[0], u[0], limit, act), gated<bf16_t>(g[1], u[1], limit, act)),
+                          two_bf16(gated<bf16_t>(g[2], u[2], limit, act), gated<bf16_t>(g[3], u[3], limit, act))};
+          }
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          // lanes 0..31 hold gate rows, lanes 32..63 the up rows of the same columns: the lower lanes keep the first two of their
+          // four columns, the upper ones take the other two
+          float g[2], u[2];
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[j][i][r]), __float_as_uint(acc[j][i][r + 2]), false, false);
+            g[r] = __uint_as_float(both[0]);
+            u[r] = __uint_as_float(both[1]);
+          }
+          const int c = c0 + (wn * TN + j) * 8 + fk % 2 * 4 + fk / 2 * 2;
+          if (m >= M || c >= N) continue;
+          if (out_f32)
+            *reinterpret_cast<any_f32x2*>(static_cast<float*>(out) + row + c) = any_f32x2{gated<float>(g[0], u[0], limit, act), gated<float>(g[1], u[1], limit, act)};
+          else
+            *reinterpret_cast<any_u32*>(static_cast<uint16_t*>(out) + row + c) =
+                two_bf16(gated<bf16_t>(g[0], u[0], limit, act), gated<bf16_t>(g[1], u[1], limit, act));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int c = c0 + (wn * TN + j) * 16 + fk * 4;
+        if (m >= M || c >= N) continue;
+        const ring_f32x4 v = acc[j][i];
+        if (S > 1)
+          *reinterpret_cast<any_f32x4*>(partials + (static_cast<size_t>(s) * M + m) * N + c) = any_f32x4{v[0], v[1], v[2], v[3]};
+        else if (out_f32)
+          *reinterpret_cast<any_f32x4*>(static_cast<float*>(out) + static_cast<size_t>(m) * ldo + c) = any_f32x4{v[0], v[1], v[2], v[3]};
+        else
+          *reinterpret_cast<any_u32x2*>(static_cast<uint16_t*>(out) + static_cast<size_t>(m) * ldo + c) = any_u32x2{two_bf16(v[0], v[1]), two_bf16(v[2], v[3])};
+      }
+    }
+  }
+}
+
+// The tiles, and what a launch of them takes: us at the beginning and end, us a step of a workgroup that is alone on its CU, the factor on
+// (workgroups a CU) x (a step) beyond that, us of each further round.  Fitted to some 5,000 timed launches (8 to 2,048 rows, the
+// projections of models of widths 2,048 and 4,096, S = 1 to 8; the fit is off by 4 to 10 % a launch).
+struct Tile {
+  int bm, bn;
+  float fixed, step, share, round;
+};
+#define KVCM_TILES(T)                                                                                                             \
+  T(16, 48, 1, 3, 8, 1.278f, 0.167f, 0.771f, 0.466f)                                                                              \
+  T(16, 64, 1, 4, 8, 1.126f, 0.199f, 0.886f, 0.256f)                                                                              \
+  T(32, 64, 2, 2, 6, 1.484f, 0.219f, 0.891f, 0.210f)                                                                              \
+  T(64, 48, 4, 1, 8, 2.019f, 0.236f, 0.975f, 1.170f)                                                                              \
+  T(64, 64, 2, 2, 4, 1.822f, 0.274f, 0.869f, 0.435f)                                                                              \
+  T(64, 96, 2, 3, 6, 2.462f, 0.351f, 0.957f, 1.524f)                                                                              \
+  T(96, 64, 3, 2, 4, 2.841f, 0.324f, 0.916f, 0.487f)                                                                              \
+  T(128, 64, 4, 2, 6, 2.780f, 0.356f, 1.066f, 1.100f)                                                                             \
+  T(128, 96, 4, 3, 5, 3.397f, 0.465f, 0.998f, 1.810f)                                                                             \
+  T(128, 128, 2, 4, 4, 3.913f, 0.513f, 1.039f, 2.154f)                                                                            \
+  T(128, 192, 2, 3, 4, 5.339f, 0.744f, 1.028f, 1.230f)                                                                            \
+  T(256, 128, 4, 2, 3, 5.952f, 0.775f, 1.048f, 3.450f)                                                                            \
+  T(256, 192, 4, 3, 2, 6.470f, 1.155f, 1.028f, 0.000f)                                                                            \
+  T(256, 256, 2, 4, 2, 8.000f, 1.347f, 1.034f, 4.651f)
+
+#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, FIXED, STEP, SHARE, ROUND) {BM, BN, FIXED, STEP, SHARE, ROUND},
+static constexpr Tile kTiles[] = {KVCM_TILES(KVCM_TILE_ROW)};
+#undef KVCM_TILE_ROW
+constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+constexpr int kCUs = 256;
+
+// us of a launch of `groups` workgroups of `steps` steps: their chain, or the weights (elements) at 5.9 TB/s where that is longer (a sum
+// of fourth powers in between)
+static float tile_time(const Tile& t, float groups, int steps, float weights) {
+  const float each = std::ceil(groups / static_cast<float>(kCUs));
+  const float chain = t.fixed + t.step * static_cast<float>(steps) * (each > 1.f ? each * t.share : 1.f) + t.round * (each - 1.f);
+  const float stream = 2.3f + weights * 2e-6f / 5.9f;
+  const float c2 = chain * chain, s2 = stream * stream;
+  return std::sqrt(std::sqrt(c2 * c2 + s2 * s2));
+}
+
+float gemm_tile_time(int bm, int bn, float groups, int steps, float weights) {
+  for (const Tile& t : kTiles)
+    if (t.bm == bm && t.bn == bn) return tile_time(t, groups, steps, weights);
+  return 1e30f;
+}
+
+static int best_tile(int M, int wrows, int K, int S, float* time = nullptr) {
+  int best = 0;
+  float best_t = 0.f;
+  for (int i = 0; i < kTileCount; ++i) {
+    if (kTiles[i].bm > 16 && kTiles[i].bm >= 2 * M) continue;      // more than half of the rows would not exist
+    const float groups = static_cast<float>(static_cast<long long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((wrows + kTiles[i].bn - 1) / kTiles[i].bn) * S);
+    const float t = tile_time(kTiles[i], groups, (K / kStepK + S - 1) / S, static_cast<float>(wrows) * static_cast<float>(K));
+    if (i == 0 || t < best_t) {
+      best = i;
+      best_t = t;
+    }
+  }
+  if (time != nullptr) *time = best_t;
+  return best;
+}
+
+float gemm_tiles_time(int M, int N, int K, int S, bool is_gated, bool out_f32) {
+  float t = 0.f;
+  best_tile(M, is_gated ? 2 * N : N, K, S, &t);
+  return t + static_cast<float>(M) * static_cast<float>(N) * (S > 1 ? 4.f * S : out_f32 ? 4.f : 2.f) * 0.12e-6f;      // what is stored
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED>
+static int launch_tiles(const TilesCall& c, hipStream_t st) {
+  const int tiles_m = (c.M + BM - 1) / BM, tiles_n = ((GATED ? 2 * c.N : c.N) + BN - 1) / BN;
+  const long long grid = static_cast<long long>(tiles_m) * tiles_n * c.S;
+  KVCM_REQUIRE(grid < (1ll << 31), "gemm_tiles: too many tiles");
+  gemm_tiles_kernel<BM, BN, WM, WN, STAGES, GATED><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, st>>>(
+      c.X, c.W, c.partials, c.out, c.out_f32, c.M, c.N, c.K, c.ldx, c.ldw, c.ldo, c.S, tiles_m, tiles_n, c.ss_in, c.tiles_in, c.eps, c.limit,
+      c.act);
+  return launch_status("gemm_tiles");
+}
+
+int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st) {
+  KVCM_REQUIRE(c.M > 0 && c.N > 0 && c.N % 4 == 0 && c.K > 0 && c.K % kStepK == 0 && c.S >= 1 && c.S <= c.K / kStepK,
+               "gemm_tiles: unsupported shape M=%d N=%d K=%d in %d slices", c.M, c.N, c.K, c.S);
+  KVCM_REQUIRE(!is_gated || (c.N % 8 == 0 && c.S == 1), "gemm_tiles: gated products take widths of multiples of 8 and are unsplit");
+  KVCM_REQUIRE(c.ldx < (1 << 22) && c.ldw < (1 << 22), "gemm_tiles: rows too far apart");      // a tile's offsets are 32-bit
+  if (tile < 0) tile = best_tile(c.M, is_gated ? 2 * c.N : c.N, c.K, c.S);
+  int i = 0;
+#define KVCM_TILE_LAUNCH(BM, BN, WM, WN, STAGES, FIXED, STEP, SHARE, ROUND)                                                        \
+  if (tile == i++) return is_gated ? launch_tiles<BM, BN, WM, WN, STAGES, true>(c, st) : launch_tiles<BM, BN, WM, WN, STAGES, false>(c, st);
+  KVCM_TILES(KVCM_TILE_LAUNCH)
+#undef KVCM_TILE_LAUNCH
+  KVCM_REQUIRE(false, "gemm_tiles: no tile %d", tile);
+}
+
+}  // namespace kvcm
+
+using namespace kvcm;
+
+extern "C" {
+
+// How many tiles there are, and the rows and columns (of W) of one: for tests, which run each.
+int kvcm_gemm_tiles_count() { return kTileCount; }
+int kvcm_gemm_tiles_size(int tile, int* rows, int* cols) {
+  KVCM_REQUIRE(tile >= 0 && tile < kTileCount, "gemm_tiles_size: no tile %d", tile);
+  *rows = kTiles[tile].bm;
+  *cols = kTiles[tile].bn;
+  return 0;
+}
+// The product with a given tile (< 0: the one the rule picks).  is_gated: W [2 N, K], out [M, N] = act(gate) * up (act: 0 silu with the
+// roundings of a stored product followed by kvcm_swiglu, 1 silu, 2 relu, rounded once), or the gate with limits (limit > 0).
+int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, int out_dtype, int M, int N, int K, int ldx, int ldw, int ldo,
+                    int S, int is_gated, int act, float limit, int tile, hipStream_t st) {
+  KVCM_REQUIRE(ldx % 8 == 0 && ldw % 8 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0,
+               "gemm_tiles: operands must be 16-byte aligned with leading dimensions that are multiples of 8");
+  KVCM_REQUIRE(ldx >= K && ldw >= K && (S > 1 ? partials != nullptr : out != nullptr && ldo >= N), "gemm_tiles: missing buffer or leading dimension too small");
+  KVCM_REQUIRE(out_dtype == kBF16 || out_dtype == kF32, "gemm_tiles: unknown output dtype %d", out_dtype);
+  KVCM_REQUIRE(act >= kSiluStored && act <= kRelu, "gemm_tiles: unknown activation %d", act);
+  TilesCall c{static_cast<const uint16_t*>(X), static_cast<const uint16_t*>(W), partials, out, out_dtype == kF32, M, N, K, ldx, ldw, ldo, S};
+  c.limit = limit;
+  c.act = act;
+  return gemm_tiles(c, is_gated != 0, tile, st);
+}
+
+// Is a product of many rows, in S slices of K that its consumer adds, faster here than by the vendor library (is_gated: than that and
+// the launch that applies SwiGLU)?  Up to 256 rows it was at all 38 shapes measured (0.43 to 0.87 of the time), beyond 2,048 the
+// library's own tiles of 256 x 256 are (32,768 rows: 1,306 / 1,269 us gate+up of 5632 x 2048, 659 / 513 us 2048 x 5632).  In between, the
+// tiles' time and the slices' reading against about what the library takes: 14 us and 1,350 TFLOP/s (22 us and 1,600 for the largest),
+// and at least 0.3 us for 64 k of a chain that it does not cut.  The six constants were fitted to 76 shapes; what the rule picks is 1.1 %
+// slower than the better of the two on average, 12 % at worst.  (us, here / library: 512 x 2048 x 5632 22.8 / 26.4; 1,024 rows gate+up
+// 48.1 / 57.7; 2,048 rows 92.1 / 97.8; not taken: 768 x 6144 x 4096 55.0 / 48.2, 2048 x 2560 x 2048 30.7 / 27.5.)
+int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype) {
+  if (M <= 0 || N <= 0 || N % 64 != 0 || K <= 0 || K % kStepK != 0 || S < 1 || S > K / kStepK || (is_gated && S > 1)) return 0;
+  if (M <= 256) return 1;
+  if (M > 2048) return 0;
+  const float mn = static_cast<float>(M) * static_cast<float>(N);
+  const float here = gemm_tiles_time(M, N, K, S, is_gated != 0, out_dtype == kF32) + (S > 1 ? mn * (4.f * S - 2.f) / 4.5e6f : 0.f);
+  const float gflop = mn * static_cast<float>(K) * (is_gated ? 4e-9f : 2e-9f);
+  const float rate = std::fmin(14.f + gflop / 1.35f, 22.f + gflop / 1.6f), chain = 4.f + 0.3f * static_cast<float>(K / kStepK);
+  const float library = std::fmax(rate, chain) + (is_gated ? 3.f + mn * 6.f / 5e6f : 0.f);
+  return here <= library;
+}
+
+}  // extern "C"

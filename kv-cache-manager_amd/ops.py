@@ -48,6 +48,11 @@ def _declare(lib):
     fn("kvcm_gemm_skinny_swiglu", vp, vp, vp, i, i, i, i, i, i, i, f, vp)
     fn("kvcm_gemm_skinny_splits", i, i, i)
     fn("kvcm_gemm_skinny_waves", i, i, i, i, i)
+    fn("kvcm_gemm_skinny_whole_splits", i, i, i)
+    fn("kvcm_gemm_tiles_count")
+    fn("kvcm_gemm_tiles_size", i, C.POINTER(i), C.POINTER(i))
+    fn("kvcm_gemm_tiles", vp, vp, vp, vp, i, i, i, i, i, i, i, i, i, i, f, i, vp)
+    fn("kvcm_gemm_tiles_preferred", i, i, i, i, i, i)
     fn("kvcm_gemm_skinny_swiglu_normed_preferred", i, i, i)
     fn("kvcm_gemm_skinny_swiglu_normed", vp, vp, vp, i, f, vp, i, i, i, i, i, i, vp)
     fn("kvcm_gemm_skinny", vp, vp, vp, vp, i, i, i, i, i, i, i, i, vp)
@@ -497,13 +502,10 @@ def add_residual(x, y):
     _call("kvcm_add_residual", _ptr(x), _ptr(y), _DT[y.dtype], x.numel(), _stream())
 
 
-# Rows from which a bfloat16 product is handed to the library (hipBLASLt, called directly:
+# Rows from which a bfloat16 product may be handed to the library (hipBLASLt, called directly:
 # csrc/hip/gemm_library.hip); the reference leaves every product to its vendor library.  0 = always
-# use the kernels of this package.  Below, the weight-streaming kernels of this package run.  Measured
-# end to end at TinyLlama sizes (steps of 16 decoding rows beside a prompt portion, replayed from
-# recorded programs, so that a call costs the host the same either way): 48 rows 2.03 ms with this
-# package's kernels against 2.24 with the library's, 80 rows 2.05 / 2.26, 112 rows 2.83 / 2.61,
-# 176 rows 2.85 / 2.56, 336 rows 3.85 / 2.98.
+# use the kernels of this package.  From here on a product runs in this package's tiles where those are the faster
+# (``_tiles_take``: up to 256 rows, and beyond by the shape), or where they are refused by the library's.
 LIBRARY_GEMM_MIN_ROWS = 96
 # ... except that up to LIBRARY_LONG_K_MIN_ROWS - 1 rows this package's kernel keeps the products whose K is
 # at least their width and whose weights are at least LIBRARY_LONG_K_BYTES (the O and down projections of 7B /
@@ -515,8 +517,18 @@ LIBRARY_LONG_K_MIN_ROWS = 193
 LIBRARY_LONG_K_BYTES = 32 << 20
 
 
+def many_rows(M):
+    """Is a bfloat16 product of M rows one that the vendor library may run?  Its consumers read whole rows."""
+    return bool(LIBRARY_GEMM_MIN_ROWS) and M >= LIBRARY_GEMM_MIN_ROWS
+
+
+def _tiles_take(M, N, K, S, gated=False, dtype=torch.bfloat16):
+    """Does a bfloat16 product that the vendor library may run stay with this package's tiles, in S slices of K (csrc/hip/gemm_tiles.hip)?"""
+    return bool(lib().kvcm_gemm_tiles_preferred(M, N, K, S, int(gated), _DT[dtype]))
+
+
 def _library_takes(M, N, K):
-    """Does a bfloat16 product of M rows go to the vendor library?"""
+    """Does a bfloat16 product of M rows go to the vendor library (where this package's tiles do not take it)?"""
     if not LIBRARY_GEMM_MIN_ROWS or M < LIBRARY_GEMM_MIN_ROWS:
         return False
     return not (M < LIBRARY_LONG_K_MIN_ROWS and K >= N and 2 * N * K >= LIBRARY_LONG_K_BYTES)
@@ -559,13 +571,24 @@ def _library_workspace(device):
 
 
 def skinny_waves(M, N, K, S=1, swiglu=False):
-    """Waves per workgroup the shared-rows kernel runs this bfloat16 product with (0: another kernel takes it)."""
+    """16-column tiles a workgroup with which this bfloat16 product in tiles covers the chip (0: another kernel takes it)."""
     return lib().kvcm_gemm_skinny_waves(int(M), int(N), int(K), int(S), int(bool(swiglu)))
 
 
 def skinny_splits(M, N, K):
     """Split count the decode-shaped kernel uses for this shape, 0 when it does not take it."""
     return lib().kvcm_gemm_skinny_splits(M, N, K)
+
+
+def _usable_splits(M, N, K, scratch, keep_partial):
+    """Slices of K that a product of M rows is cut into: where nobody takes the partial sums, none if that is the faster whole, and as
+    many as ``scratch`` has room for (0: the kernels of few rows do not take the shape)."""
+    S = skinny_splits(M, N, K)
+    if S <= 1:
+        return S
+    if scratch is None or not keep_partial and lib().kvcm_gemm_skinny_whole_splits(M, N, K) == 1:
+        return 1
+    return S if scratch.numel() >= S * M * N else max(1, min(S, scratch.numel() // (M * N)))
 
 
 def _rows8_takes(M, N, K, out_dtype, splits):
@@ -595,8 +618,8 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
     """out[M, N] = x[M, K] @ w[N, K]^T.  float32 x float32 -> float32 (32-bit multiply-adds, an order of k fixed by K), or
     bfloat16 x bfloat16 -> bfloat16 | float32 (MFMA, 32-bit accumulation).
 
-    Rows below LIBRARY_GEMM_MIN_ROWS take the weight-streaming kernels (also more rows, up to 512,
-    while the library is switched off: inside a captured graph); when they split K they need
+    Rows below LIBRARY_GEMM_MIN_ROWS take this package's kernels (also more rows, up to 512,
+    while the library is switched off: inside a captured graph), more rows where those are the faster; when they split K they need
     ``scratch`` (float32, at least splits*M*N elements).  With ``keep_partial``
     the un-added partial sums are returned as PartialSums (for a fused consumer) instead of ``out``.
     ``unsplit``: a product of at most 8 rows may run unsplit (gemm_rows8.hip), where nobody asks for its slices.
@@ -626,7 +649,18 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
         _call("kvcm_gemm_f32", _ptr(x), _ptr(w), _ptr(out), M, N, K, x.stride(0), w.stride(0), out.stride(0), _stream())
         return out
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm operands must both be bfloat16")
-    if out.dtype == torch.float32 and out.is_contiguous() and _library_takes(M, N, K) and _library_has_f32out(
+    aligned = x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    library = _library_takes(M, N, K)
+    mode = _TUNING_MODES[LIBRARY_TUNING if tuning is None else tuning]
+    if library and mode == 0 and aligned and K % 64 == 0 and N % 64 == 0:
+        # (who asks for the library's tuned algorithms gets them)
+        S = _usable_splits(M, N, K, scratch, keep_partial) if M <= 512 else 1
+        library = not _tiles_take(M, N, K, S, dtype=out.dtype)
+        if not library and M > 512:
+            _call("kvcm_gemm_tiles", _ptr(x), _ptr(w), 0, _ptr(out), _DT[out.dtype], M, N, K, x.stride(0), w.stride(0), out.stride(0),
+                  1, 0, 0, 0.0, -1, _stream())
+            return out
+    if library and out.dtype == torch.float32 and out.is_contiguous() and _library_has_f32out(
             M, N, K, x.stride(0), w.stride(0), out.stride(0)):
         # many rows, a 32-bit result: the library stores its 32-bit sums as they are
         ws = _library_workspace(out.device)
@@ -634,16 +668,12 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
               _ptr(ws), ws.numel(), _stream())
         return out
     if (unsplit and not (keep_partial and scratch is not None) and _rows8_takes(M, N, K, out.dtype, scratch is not None)
-            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+            and aligned):
         _call("kvcm_gemm8", _ptr(x), x.stride(0), _ptr(w), w.stride(0), M, N, K, 0, 0, 0.0, _ptr(out), _DT[out.dtype],
               out.stride(0), 0, _stream())
         return out
-    library = _library_takes(M, N, K) and out.dtype == torch.bfloat16 and out.is_contiguous()
-    S = skinny_splits(M, N, K) if (not library and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
-                                   and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0) else 0
-    if S > 1 and (scratch is None or scratch.numel() < S * M * N):
-        S = 1 if scratch is None else max(1, min(S, scratch.numel() // (M * N)))
+    library = library and out.dtype == torch.bfloat16 and out.is_contiguous()
+    S = _usable_splits(M, N, K, scratch, keep_partial) if not library and aligned else 0
     if S >= 1:
         if S > 1:
             _need(scratch.dtype == torch.float32 and scratch.is_contiguous() and scratch.is_cuda, "scratch must be float32")
@@ -655,7 +685,6 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
         return partial if keep_partial else partial.materialize()
     if library:
         ws = _library_workspace(out.device)
-        mode = _TUNING_MODES[LIBRARY_TUNING if tuning is None else tuning]
         shape = (M, N, K, x.stride(0), w.stride(0), out.stride(0))
         if mode and lib().kvcm_gemm_library_tuned(*shape) < mode:
             # not a recorded launch: it runs here, once, whoever is recording
@@ -708,11 +737,16 @@ def gemm_swiglu(x, w_gate_up, out, limit=0.0):
     M, K = x.shape
     I = out.shape[1]
     _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_swiglu shapes do not agree")
-    if LIBRARY_GEMM_MIN_ROWS and M >= LIBRARY_GEMM_MIN_ROWS:
-        return False          # many rows: the library product, then swiglu
-    if not (x.dtype == w_gate_up.dtype == out.dtype == torch.bfloat16 and x.stride(0) % 8 == 0
-            and w_gate_up.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0
-            and lib().kvcm_gemm_skinny_swiglu_supported(M, I, K)):
+    aligned = (x.dtype == w_gate_up.dtype == out.dtype == torch.bfloat16 and x.stride(0) % 8 == 0
+               and w_gate_up.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0)
+    if many_rows(M):
+        # many rows: the library product, then swiglu, unless the tiles are the faster
+        if not (aligned and _tiles_take(M, I, K, 1, gated=True)):
+            return False
+        _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0),
+              out.stride(0), 1, 1, 0, float(limit), -1, _stream())
+        return True
+    if not (aligned and lib().kvcm_gemm_skinny_swiglu_supported(M, I, K)):
         return False
     _call("kvcm_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _DT[out.dtype], M, I, K, x.stride(0),
                                          w_gate_up.stride(0), out.stride(0), float(limit), _stream())

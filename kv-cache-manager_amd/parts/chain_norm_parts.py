@@ -214,7 +214,7 @@ class GatedFeedForward(JoinableEnds, FeedForward):
         # few rows in bfloat16 with silu or its form with limits: the product that streams gate and up rows together and applies
         # the activation in its epilogue, one launch (silu is rounded once more on the way, within the result's own rounding)
         if not (kind in ("silu", "clamped") and act.dtype == torch.bfloat16 and torch.is_tensor(h)
-                and ops.gemm_swiglu(h, self.w["w_gate_up"], act, limit=limit)):
+                and not ops.many_rows(step.rows) and ops.gemm_swiglu(h, self.w["w_gate_up"], act, limit=limit)):
             gu = linear32(self.ctx, step, h, self.w["w_gate_up"], "gated_gate_up")
             ops.gated_act(gu, act, kind, limit=limit)
         return linear32(self.ctx, step, act, self.w["w_down"], "gated_out", keep_partial=bool(self.params.get("partial_out")))

@@ -173,7 +173,8 @@ class GQAAttention(Mixer):
         g = self.cache.group
         kc, vc = self.cache.k(self.cache_index), self.cache.v(self.cache_index)
         pos = self.position
-        res = _linear(self.ctx, step, h, self.w["wqkv"], "qkv", keep_partial=pos.accepts_partial_sums)
+        # (the rotation of many rows reads whole rows, eight entries a lane; that of slices a head at a time)
+        res = _linear(self.ctx, step, h, self.w["wqkv"], "qkv", keep_partial=pos.accepts_partial_sums and not ops.many_rows(step.rows))
         qkv = step.ws("qkv", (step.rows, self.q_dim + 2 * self.kv_dim))
         slots = step.slots(g) if self.cache_owner else None
         attn = step.ws("attn", (step.rows, self.q_dim))

@@ -1,0 +1,147 @@
+"""Products in tiles (csrc/hip/gemm_tiles.hip): every tile at the sizes where its edges, its ring of stages and its slices of K
+can go wrong, against products in 64 bits, and the rule that hands products of many rows to it."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from kvcm_amd import ops as _ops
+    _ops.lib()
+    return _ops
+
+
+def _tiles(ops):
+    out = []
+    for t in range(ops.lib().kvcm_gemm_tiles_count()):
+        bm, bn = C.c_int(), C.c_int()
+        assert ops.lib().kvcm_gemm_tiles_size(t, C.byref(bm), C.byref(bn)) == 0
+        out.append((bm.value, bn.value))
+    return out
+
+
+def _operands(seed, M, N, K, pad_x=0, pad_w=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(M, K + pad_x, generator=g, device=DEV).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K + pad_w, generator=g, device=DEV) * 0.1).to(torch.bfloat16)[:, :K]
+    return x, w
+
+
+def _close(got, x, w, bf16, ref=None):
+    """32-bit sums in any order are off by at most K 2^-24 of the sum of the terms' sizes each (two operations a term counted);
+    a bfloat16 result by half a unit of its own last place beside that."""
+    xd, wd = x.double(), w.double()
+    ref = xd @ wd.t() if ref is None else ref
+    bound = 2 * x.shape[1] * 2.0 ** -24 * (xd.abs() @ wd.abs().t())
+    if bf16:
+        bound = bound + ref.abs() * 2.0 ** -8
+    err = (got.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+def _run(ops, x, w, partials, out, S=1, gated=0, act=0, limit=0.0, tile=-1, N=None):
+    M, K = x.shape
+    N = N or w.shape[0]
+    rc = ops.lib().kvcm_gemm_tiles(x.data_ptr(), w.data_ptr(), partials.data_ptr() if partials is not None else 0, out.data_ptr(),
+                                   ops._DT[out.dtype], M, N, K, x.stride(0), w.stride(0), out.stride(0), S, gated, act, limit,
+                                   tile, ops._stream())
+    assert rc == 0, ops.lib().kvcm_hip_last_error().decode()
+
+
+@pytest.mark.parametrize("tile", range(14))
+def test_every_tile_at_its_edges(ops, tile):
+    sizes = _tiles(ops)
+    assert len(sizes) == 14
+    bm, bn = sizes[tile]
+    seed = 0
+    # rows and columns around one tile and around several; k of one step (shorter than any ring), of few, of more than a ring
+    for M, N, K, S in [(1, 64, 64, 1), (bm - 1, bn, 448, 1), (bm + 1, bn + 12, 640, 2), (2 * bm + 3, 2 * bn - 4, 192, 3),
+                       (5, 4 * bn + 64, 1152, 4), (bm, 8, 576, 8), (3 * bm, 3 * bn, 128, 1)]:
+        seed += 1
+        x, w = _operands(seed, M, N, K, pad_x=8 * (seed % 3), pad_w=8 * (seed % 2))
+        if S > 1:
+            parts = torch.full((S * M * N + 4,), float("nan"), device=DEV)
+            _run(ops, x, w, parts, torch.empty(M, N, device=DEV), S=S, tile=tile)
+            assert torch.isnan(parts[S * M * N:]).all()
+            _close(parts[:S * M * N].view(S, M, N).double().sum(0), x, w, False)
+            continue
+        for dtype, pad in ((torch.float32, 0), (torch.float32, 3), (torch.bfloat16, 0), (torch.bfloat16, 5)):
+            room = torch.full((M * (N + pad) + 9,), float("nan"), dtype=dtype, device=DEV)
+            out = room[1:1 + M * (N + pad)].view(M, N + pad)[:, :N]      # begins at any element
+            _run(ops, x, w, None, out, tile=tile)
+            _close(out, x, w, dtype == torch.bfloat16)
+            left = room.clone()
+            left[1:1 + M * (N + pad)].view(M, N + pad)[:, :N] = float("nan")
+            assert torch.isnan(left).all(), "written beside the result"
+
+
+@pytest.mark.parametrize("tile", range(14))
+def test_every_tile_gated(ops, tile):
+    bm, bn = _tiles(ops)[tile]
+    for seed, (M, I, K) in enumerate([(1, 8, 64), (bm + 1, bn // 2, 448), (bm - 1, bn + 8, 640), (2 * bm + 3, 2 * bn + 40, 192)]):
+        x, w = _operands(50 + seed, M, 2 * I, K)
+        g, u = (x.double() @ w.double().t()).split(I, 1)
+        size = 2 * K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        eg, eu = size.split(I, 1)
+        exact = g * torch.sigmoid(g) * u
+        # d silu <= 1.1 d gate; silu by the hardware's exp2 and reciprocal: 2^-21 of itself
+        bound = 1.1 * eg * u.abs() + g.abs() * eu + 1.1 * eg * eu + exact.abs() * 2.0 ** -21
+        for dtype in (torch.float32, torch.bfloat16):
+            out = torch.full((M, I), float("nan"), dtype=dtype, device=DEV)
+            _run(ops, x, w, None, out, gated=1, act=1, tile=tile, N=I)
+            last = exact.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0
+            assert bool(((out.double() - exact).abs() <= bound + last).all())
+        _run(ops, x, w, None, out, gated=1, act=2, tile=tile, N=I)
+        relu = g.clamp(min=0) * u
+        assert bool(((out.double() - relu).abs() <= eg * u.abs() + g.abs() * eu + eg * eu + relu.abs() * 2.0 ** -8).all())
+        # with a stored product's roundings: what the product stored in bfloat16 gives through the SwiGLU launch, but for sums that round to the other side
+        out = torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+        _run(ops, x, w, None, out, gated=1, act=0, tile=tile, N=I)
+        gu, want = torch.empty(M, 2 * I, dtype=torch.bfloat16, device=DEV), torch.empty_like(out)
+        _run(ops, x, w, None, gu, tile=tile)
+        ops.swiglu(gu, want)
+        assert (out == want).float().mean() > 0.98
+        _run(ops, x, w, None, out, gated=1, limit=0.5, tile=tile, N=I)
+        gc, uc = g.clamp(max=0.5), u.clamp(-0.5, 0.5)
+        clamped = gc * torch.sigmoid(1.702 * gc) * (uc + 1)
+        assert bool(((out.double() - clamped).abs() <= 2.5 * (eg + eu) + clamped.abs() * 2.0 ** -8 + 1e-6).all())
+
+
+def test_products_with_a_folded_norm_in_tiles(ops):
+    """rows whose norm's scale is applied to the sums: rsqrt(mean x^2 + eps) from sums of squares of 8 columns each"""
+    M, I, K = 8, 8192 + 64, 320
+    x, w = _operands(90, M, 2 * I, K)
+    ss = torch.rand(M, K // 8, device=DEV) * 8
+    rstd = 1.0 / torch.sqrt(ss.double().sum(1, keepdim=True) / K + 1e-5)
+    out = torch.empty(M, I, dtype=torch.bfloat16, device=DEV)
+    assert ops.lib().kvcm_gemm_skinny_swiglu_normed(x.data_ptr(), w.data_ptr(), ss.data_ptr(), K // 8, 1e-5, out.data_ptr(), M, I, K,
+                                                    x.stride(0), w.stride(0), out.stride(0), ops._stream()) == 0
+    g, u = (x.double() @ w.double().t() * rstd).split(I, 1)
+    want = g * torch.sigmoid(g) * u
+    # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each
+    assert bool(((out.double() - want).abs() <= 4.2 * 2.0 ** -8 * (g.abs() * u.abs()) + 1e-5).all())
+
+
+@pytest.mark.parametrize("M,N,K,mine", [(96, 2048, 2048, True), (200, 2560, 2048, True), (333, 2048, 5632, True), (700, 2048, 2048, True),
+                                        (1024, 2048, 2048, True), (1536, 8192, 2048, False), (2000, 192, 128, None)])
+def test_many_rows_go_to_the_tiles_where_the_rule_says_so(ops, M, N, K, mine):
+    x, w = _operands(M, M, N, K)
+    for dtype in (torch.bfloat16, torch.float32):
+        out = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+        scratch = torch.empty(8 * 512 * N, device=DEV)
+        S = ops.skinny_splits(M, N, K) if M <= 512 else 1
+        if mine is not None:
+            assert ops._tiles_take(M, N, K, S) == mine
+        got = ops.gemm(x, w, out, scratch=scratch, keep_partial=True)
+        _close(got.materialize() if isinstance(got, ops.PartialSums) else got, x, w, dtype == torch.bfloat16)
+        _close(ops.gemm(x, w, out, scratch=scratch), x, w, dtype == torch.bfloat16)
+    act, plain = torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV), torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV)
+    assert ops.gemm_swiglu(x, w, act) == ops._tiles_take(M, N // 2, K, 1, gated=True)
+    if ops._tiles_take(M, N // 2, K, 1, gated=True):
+        ops.swiglu(ops.gemm(x, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV)), plain)
+        assert (act == plain).float().mean() > 0.98
