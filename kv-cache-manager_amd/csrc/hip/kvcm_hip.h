@@ -279,10 +279,11 @@ int kvcm_moe_down(const void* act, int dtype, const void* w_down, const int* cho
 int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E);
 // (moe_grouped.hip) the routed feed-forward for many rows: pairs grouped by expert, tiles on the matrix cores
 int kvcm_moe_grouped_supported(int K, int F, int E);
-int kvcm_moe_grouped_max_tiles(int n, int E);
+int kvcm_moe_grouped_lists(int n, int E);
+int kvcm_moe_grouped_tile_count();
 int kvcm_moe_grouped(const void* h, int ldh, const void* w_up, const void* w_down, const int* chosen, const float* weight,
-                     int* order, int* tiles, void* act, float* y, const float* add, float* out, int T, int K, int F, int H,
-                     int top, int E, int kind, int weigh_input, hipStream_t s);
+                     int* order, int* lists, void* act, float* y, const float* add, float* out, int T, int K, int F, int H,
+                     int top, int E, int kind, int weigh_input, int tile_up, int tile_down, hipStream_t s);
 
 // ---- recorded steps ---------------------------------------------------------------------------
 // A step program is the list of launches of one step, recorded once for a step shape and replayed

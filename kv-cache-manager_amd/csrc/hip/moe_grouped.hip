@@ -1,60 +1,43 @@
 // The routed feed-forward for steps with many rows (bfloat16): the (row, slot) pairs are grouped by their expert and
 // every expert's group is multiplied with that expert's matrices in tiles on the matrix cores, so that an expert's
-// weights are read once per tile of 128 pairs and not once per pair.
+// weights are read once per tile of pairs and not once per pair.
 //
-//   moe_group      pairs p = row * top + slot, grouped by chosen[p]: order[] lists the pairs expert by expert, tiles[]
-//                  lists (expert, first place in order, pairs) for every stretch of up to 128 pairs of one expert, with
-//                  the number of tiles in front.  One workgroup; places inside a group are handed out by an atomic
-//                  counter in LDS, so the order inside a group may differ from run to run, which changes no result: a
-//                  pair's row of a tile is computed from that row alone.
+//   moe_group      pairs p = row * top + slot, grouped by chosen[p]: order[] lists the pairs expert by expert; two lists, for the
+//                  tiles of UP and of DOWN (which may be of different heights), hold (expert, its first place in order, its
+//                  pairs, its first tile) for every tile, the tiles of an expert one after the other.  One workgroup; places inside
+//                  a group are handed out by an atomic counter in LDS, so the order inside a group may differ from run to
+//                  run, which changes no result: a pair's row of a tile is computed from that row alone.
 //   moe_grouped    UP:   act[place, :] = square(relu(W_up[e] h[row of the pair])), or gelu of it (bfloat16, in grouped order)
 //                  GATED UP: act[place, :] = silu(W_gate[e] h) * (W_up[e] h); the two matrices of an expert are stored as
 //                        one of 2F rows, interleaved sixteen at a time (gate 0..15, up 0..15, gate 16..31, ...), so that a
-//                        lane's neighbouring 16 x 16 tiles hold the gate and the up value of one column
+//                        lane's neighbouring accumulators hold the gate and the up values of the same columns
 //                  DOWN: y[pair, :]   = weight[pair] * W_down[e] act[place, :]               (32-bit, by pair)
 //                  The pairs' weights may act on the other side instead: UP then reads weight * h (the factor is applied to
 //                  its 32-bit sums) and DOWN weighs nothing.
-//                  Tile 128 pairs x 128 columns per workgroup of four waves (64 x 64 each: 4 x 4 matrix instructions of
-//                  16 x 16 x 32), K advanced 64 at a time through two halves of LDS: while one is multiplied the other fills.
+//                  A tile of BM pairs x BN rows of the expert's matrix per workgroup, its operands in a ring of stages in LDS
+//                  (tile_ring.h).
 //   moe_combine    out[row, :] = (add[row, :] +) sum over the row's slots, in slot order, of y[row * top + slot, :]
+//
+// What bounds the products is what bounds those of gemm_tiles.hip; the tile is picked by the same constants.  All five launches, us,
+// against 128 x 128 pairs and rows with two stages throughout: 8 experts of which a row uses 2, width 2,048, 1,408 columns an expert: 80
+// rows 64.6 -> 44.2, 300 69.9 -> 52.0, 1,024 86.1 -> 84.2, 2,048 134 -> 113, 4,072 230 -> 208; width 4,096, 3,584 columns, 2,048 rows 487 -> 468.
 #include "common.h"
+#include "gemm_tiles.h"
 #include "kvcm_hip.h"
+#include "tile_ring.h"
 
 namespace kvcm {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+constexpr int kLeastHigh = 64;      // pairs of the lowest tile
 
-constexpr int kGM = 128, kGN = 128, kGK = 64;
+__host__ __device__ __forceinline__ int most_tiles(int n, int E) { return n / kLeastHigh + E; }
 
-union Frag {
-  uint4 u;
-  bf16x8 v;
-};
-
-// 64 k of both operands' 128 rows.  A row's eight 16-byte pieces are permuted by the row (piece p lies at place p ^ (row % 8)),
-// so that eight rows of a fragment read meet no bank twice without any padding, which requests straight into LDS have no room for.
-struct Stage {
-  uint16_t a[kGM * kGK], b[kGN * kGK];
-};
-
-// 16 bytes a lane from memory straight into LDS: lane l's go to `to` + 16 l (the same `to` for the whole wave)
-__device__ __forceinline__ void bring16(const uint16_t* from, uint16_t* to) {
-  __builtin_amdgcn_global_load_lds(reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(from)),
-                                   reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(to)), 16, 0, 0);
-}
-
-// this wave's requests into LDS have arrived, and so have everybody else's of the workgroup
-__device__ __forceinline__ void arrived_barrier() {
-  __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0)
-  __syncthreads();
-}
-
+// lists: the numbers of tiles of UP and DOWN, two unused, then the two lists of `most` entries
 __global__ void __launch_bounds__(1024)
-    moe_group_kernel(const int* __restrict__ chosen, int n, int E, int* __restrict__ order, int* __restrict__ tiles, int max_tiles) {
-  extern __shared__ int sh[];      // count / cursor [E], base [E]
-  int* cnt = sh;
-  int* base = sh + E;
+    moe_group_kernel(const int* __restrict__ chosen, int n, int E, int* __restrict__ order, int* __restrict__ lists, int high_up, int high_down) {
+  extern __shared__ int sh[];      // per expert: pairs (later a cursor), first place, first tile of UP, of DOWN
+  int *cnt = sh, *first = sh + E, *up = sh + 2 * E, *down = sh + 3 * E;
+  const int most = most_tiles(n, E);
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
   for (int p = threadIdx.x; p < n; p += blockDim.x) {
@@ -63,198 +46,127 @@ __global__ void __launch_bounds__(1024)
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int at = 0, nt = 0;
+    int at = 0, nu = 0, nd = 0;
     for (int e = 0; e < E; ++e) {
-      base[e] = at;
-      for (int r = 0; r < cnt[e] && nt < max_tiles; r += kGM) {
-        tiles[1 + 3 * nt] = e;
-        tiles[2 + 3 * nt] = at + r;
-        tiles[3 + 3 * nt] = cnt[e] - r < kGM ? cnt[e] - r : kGM;
-        ++nt;
-      }
+      first[e] = at;
+      up[e] = nu;
+      down[e] = nd;
       at += cnt[e];
-      cnt[e] = 0;
+      nu += (cnt[e] + high_up - 1) / high_up;
+      nd += (cnt[e] + high_down - 1) / high_down;
     }
-    tiles[0] = nt;
+    lists[0] = nu;
+    lists[1] = nd;
+  }
+  __syncthreads();
+  int4* entry = reinterpret_cast<int4*>(lists + 4);
+  for (int e = threadIdx.x; e < E; e += blockDim.x) {
+    for (int r = 0, i = up[e]; r < cnt[e]; r += high_up, ++i) entry[i] = int4{e, first[e], cnt[e], up[e]};
+    for (int r = 0, i = down[e]; r < cnt[e]; r += high_down, ++i) entry[most + i] = int4{e, first[e], cnt[e], down[e]};
+    cnt[e] = 0;      // (no other thread reads it before the barrier)
   }
   __syncthreads();
   for (int p = threadIdx.x; p < n; p += blockDim.x) {
     const int e = chosen[p];
-    if (e >= 0 && e < E) order[base[e] + atomicAdd(&cnt[e], 1)] = p;
+    if (e >= 0 && e < E) order[first[e] + atomicAdd(&cnt[e], 1)] = p;
   }
 }
 
 enum : int { kDown = 0, kUp = 1, kUpGated = 2, kUpGelu = 3 };
 
-// A wave's requests for 64 k of 32 rows of each operand.  A piece past K is read from the row's start and left out of the products.
-__device__ __forceinline__ void grouped_request(const uint16_t* const (&arow)[4], const uint16_t* const (&brow)[4], int k0, int piece, int K,
-                                                int wave, Stage* to) {
-  const int off = k0 + piece < K ? k0 + piece : 0;      // K is a multiple of 8: a piece lies inside or outside
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    bring16(arow[q] + off, &to->a[(wave * 32 + q * 8) * kGK]);
-    bring16(brow[q] + off, &to->b[(wave * 32 + q * 8) * kGK]);
-  }
-}
-
-// The wave's 64 x 64 results += 64 k (not WHOLE: the first `left` of them)
-template <bool WHOLE>
-__device__ __forceinline__ void grouped_multiply(int wm, int wn, int lane, const Stage* from, int left, f32x4 (&acc)[4][4]) {
-  const int frow = lane % 16, fk = lane / 16;
-#pragma unroll
-  for (int ks = 0; ks < kGK / 32; ++ks) {
-    const int at = ((ks * 4 + fk) ^ (frow % 8)) * 8;      // (rows 16 apart have the same permutation)
-    const bool in = WHOLE || ks * 32 + fk * 8 < left;
-    Frag a[4], b[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[i].u = *reinterpret_cast<const uint4*>(&from->a[(wm * 64 + i * 16 + frow) * kGK + at]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b[j].u = *reinterpret_cast<const uint4*>(&from->b[(wn * 64 + j * 16 + frow) * kGK + at]);
-    if constexpr (!WHOLE) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[i].u = in ? a[i].u : uint4{0u, 0u, 0u, 0u};
-        b[i].u = in ? b[i].u : uint4{0u, 0u, 0u, 0u};
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i].v, b[j].v, acc[i][j], 0, 0, 0);
-  }
-}
-
-// One step: the next 64 k are asked for, then these are multiplied.  The two halves are told apart for the compiler (else it
-// makes the first fragment read wait for the requests just made).
-__device__ __forceinline__ void grouped_step(const uint16_t* const (&arow)[4], const uint16_t* const (&brow)[4], bool more, int k0, int piece,
-                                             int K, int wave, int lane, const Stage* __restrict__ from, Stage* __restrict__ to,
-                                             f32x4 (&acc)[4][4]) {
-  if (more) grouped_request(arow, brow, k0, piece, K, wave, to);
-  grouped_multiply<true>(wave / 2, wave % 2, lane, from, kGK, acc);
-}
-
 // N: rows of an expert's matrix (2F for the gated form); the output has N columns (F for the gated form)
-template <int MODE>
-__global__ void __launch_bounds__(256, 2)
+template <int BM, int BN, int WM, int WN, int STAGES, int MODE>
+__global__ void __launch_bounds__(WM* WN* kWave)
     moe_grouped_kernel(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ W, const int* __restrict__ order,
-                       const int* __restrict__ tiles, int top, void* __restrict__ out, const float* __restrict__ weight, int N,
-                       int K, int col_blocks) {
-  __shared__ __attribute__((aligned(16))) Stage staged[2];      // the results pass through it too
-  __shared__ int pair_of[kGM];
-  // The chip hands consecutive workgroups to its eight XCDs in turn, each with an L2 of its own.  Workgroup L goes to
-  // XCD L % 8; it takes a column block that is congruent to its XCD and walks the tiles in order, so that the tiles of
-  // one expert (neighbours in the list) meet the same blocks of that expert's matrix in the same L2.
-  const int col_slots = (col_blocks + 7) / 8;
-  const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
-  const int tile = turn / col_slots, col_block = (turn % col_slots) * 8 + xcd;
-  if (col_block >= col_blocks || tile >= tiles[0]) return;
-  const int e = tiles[1 + 3 * tile], p0 = tiles[2 + 3 * tile], rows = tiles[3 + 3 * tile];
-  const int n0 = col_block * kGN;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
-  if (tid < kGM) pair_of[tid] = order[p0 + (tid < rows ? tid : 0)];
-  __syncthreads();
-  // A wave brings 32 rows of each operand, 8 rows a request: lane l asks for row l / 8, and for the 16-byte piece of the
-  // row's 64 k that belongs at place l % 8 of the permuted row.  Rows past the tile and columns past N repeat others of
-  // their kind (what they give is not stored).
-  const int piece = ((lane % 8) ^ (lane / 8)) * 8;
-  const uint16_t* arow[4];
-  const uint16_t* brow[4];
+                       const int* __restrict__ count, const int4* __restrict__ list, int top, void* __restrict__ out,
+                       const float* __restrict__ weight, int N, int K, int col_blocks) {
+  using Ring = TileRing<BM, BN, WM, WN, STAGES>;
+  constexpr int TM = Ring::TM, TN = Ring::TN, R = Ring::R;
+  static_assert(MODE != kUpGated || TN % 2 == 0, "gate and up accumulators in one wave");
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[Ring::kBytes];
+  // Each XCD takes a contiguous stretch of the tiles there are, one expert after the other, an expert's tiles of one column block
+  // side by side: neighbours read the same rows of the expert's matrix.
+  const int total = count[0] * col_blocks, per = total / 8, more = total % 8, xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
+  if (turn >= per + (xcd < more ? 1 : 0)) return;
+  const int id = xcd * per + (xcd < more ? xcd : more) + turn;
+  const int4 x = list[id / col_blocks];      // some tile of the expert
+  const int e = x.x, tiles = (x.z + BM - 1) / BM, local = id - x.w * col_blocks;
+  const int r0 = local % tiles * BM, p0 = x.y + r0, rows = x.z - r0 < BM ? x.z - r0 : BM;
+  const int n0 = local / tiles * BN;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int wm = wave % WM, wn = wave / WM, frow = lane % 16, fk = lane / 16;
+  const uint64_t abase = reinterpret_cast<uint64_t>(A + (MODE == kDown ? static_cast<size_t>(p0) * lda : 0));
+  const uint64_t wbase = reinterpret_cast<uint64_t>(W + (static_cast<size_t>(e) * N + n0) * K);
+  // rows past the tile and columns past N repeat the last one (what they give is not stored)
+  uint32_t offset[R];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = wave * 32 + q * 8 + lane / 8;
-    const long long src = MODE != kDown ? pair_of[r] / top : p0 + (r < rows ? r : 0);
-    arow[q] = A + src * lda;
-    const int c = n0 + r;
-    brow[q] = W + (static_cast<long long>(e) * N + (c < N ? c : N - 1)) * K;
+  for (int q = 0; q < R; ++q) {
+    const int req = Ring::request_of(q, wave), row = req * 8 + lane / 8;
+    const int r = row < rows ? row : rows - 1, c = row - BM < N - n0 ? row - BM : N - 1 - n0;
+    const uint32_t from = MODE != kDown ? static_cast<uint32_t>(order[p0 + (req < BM / 8 ? r : 0)]) / static_cast<uint32_t>(top) : static_cast<uint32_t>(r);
+    offset[q] = (req < BM / 8 ? from * static_cast<uint32_t>(lda) : static_cast<uint32_t>(c) * static_cast<uint32_t>(K)) * 2u +
+                static_cast<uint32_t>(Ring::piece_of(lane)) * 16u;
   }
-  f32x4 acc[4][4];
+  int pair[TM];      // of this lane's rows
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int wm = wave / 2, wn = wave % 2;
-  // One barrier a step: past it every wave's requests for this step are in LDS and nobody reads the other half any more.
-  const int steps = (K + kGK - 1) / kGK, whole_steps = K / kGK;
-  grouped_request(arow, brow, 0, piece, K, wave, &staged[0]);
-  for (int t = 0; t < whole_steps; ++t) {
-    arrived_barrier();
-    grouped_step(arow, brow, t + 1 < steps, (t + 1) * kGK, piece, K, wave, lane, &staged[t & 1], &staged[(t + 1) & 1], acc);
+  for (int i = 0; i < TM; ++i) {
+    const int m = (wm * TM + i) * 16 + frow;
+    pair[i] = order[p0 + (m < rows ? m : rows - 1)];
   }
-  if (whole_steps < steps) {
-    arrived_barrier();
-    grouped_multiply<false>(wm, wn, lane, &staged[whole_steps & 1], K - whole_steps * kGK, acc);
-  }
-  __syncthreads();
-  // accumulator layout: a lane holds column lane % 16 and rows 4 * (lane / 16) + r of each 16 x 16 tile
-  if constexpr (MODE == kDown) {
-    // 32-bit results by pair: stored from the accumulators a wave's store would write 64-byte pieces of four rows.  Each
-    // wave passes its 64 x 64 results through LDS instead, 32 rows at a time, and writes whole 256-byte stretches of
-    // a row, 16 bytes a lane.
-    constexpr int kPitch = 68;      // floats
-    static_assert(4 * 32 * kPitch * sizeof(float) <= sizeof(staged), "the results of half a tile must fit the operands' space");
-    float* mine = reinterpret_cast<float*>(&staged[0]) + wave * 32 * kPitch;
+  ring_f32x4 acc[TN][TM];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
+  for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int ii = 0; ii < 2; ++ii)
+    for (int i = 0; i < TM; ++i) acc[j][i] = ring_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (K + kStepK - 1) / kStepK;
+  Ring::multiply(ring, offset, [&](int req) { return req < BM / 8 ? abase : wbase; }, steps, 0, K - (steps - 1) * kStepK, wave, lane, acc, [] {},
+                 wm * TM * 16 < rows);
+  // acc[j][i][r]: pair wm * TM * 16 + i * 16 + frow of the tile, row wn * TN * 16 + j * 16 + fk * 4 + r of the matrix (from n0 on)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+  for (int i = 0; i < TM; ++i) {
+    const int m = (wm * TM + i) * 16 + frow;
+    if (m >= rows) continue;
+    const float g = weight ? weight[pair[i]] : 1.f;
+    if constexpr (MODE == kDown) {
+      float* dst = static_cast<float*>(out) + static_cast<size_t>(pair[i]) * N;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int c = n0 + (wn * TN + j) * 16 + fk * 4;
+        const ring_f32x4 v = acc[j][i] * g;
+        if (c + 3 < N) {
+          *reinterpret_cast<any_f32x4*>(dst + c) = any_f32x4{v[0], v[1], v[2], v[3]};
+        } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            mine[(ii * 16 + (lane / 16) * 4 + r) * kPitch + j * 16 + lane % 16] = acc[half * 2 + ii][j][r];
-      __syncthreads();
-#pragma unroll
-      for (int it = 0; it < 8; ++it) {
-        const int idx = it * kWave + lane, rl = idx / 16, c4 = (idx % 16) * 4;
-        const int m = wm * 64 + half * 32 + rl;
-        const int c = n0 + wn * 64 + c4;
-        if (m >= rows || c >= N) continue;
-        const int pair = pair_of[m];
-        const float g = weight ? weight[pair] : 1.f;
-        const float4 v = *reinterpret_cast<const float4*>(mine + rl * kPitch + c4);
-        float* dst = static_cast<float*>(out) + static_cast<long long>(pair) * N + c;
-        if (c + 3 < N && N % 4 == 0) {
-          *reinterpret_cast<float4*>(dst) = float4{g * v.x, g * v.y, g * v.z, g * v.w};
-        } else {
-          const float e4[4] = {v.x, v.y, v.z, v.w};
-          for (int q = 0; q < 4 && c + q < N; ++q) dst[q] = g * e4[q];
+            if (c + r < N) dst[c + r] = v[r];
         }
       }
-      __syncthreads();
-    }
-    return;
-  }
-  // activations, in grouped order: a wave's 64 rows of them (32 columns where two accumulators make one, else 64) pass through
-  // LDS as well and are written in whole 64- or 128-byte stretches of a row, 16 bytes a lane
-  constexpr int kWide = MODE == kUpGated ? 32 : 64, kPitch = kWide + 8;
-  static_assert(4 * 64 * kPitch * sizeof(uint16_t) <= sizeof(staged), "the activations of a tile must fit the operands' space");
-  uint16_t* mine = reinterpret_cast<uint16_t*>(&staged[0]) + wave * 64 * kPitch;
+    } else if constexpr (MODE == kUpGated) {
+      uint16_t* dst = static_cast<uint16_t*>(out) + static_cast<size_t>(p0 + m) * (N / 2);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+      for (int j = 0; j < TN; j += 2) {      // (the columns are a multiple of 16: a piece lies inside or outside)
+        const int c = n0 / 2 + (wn * TN + j) * 8 + fk * 4;
+        if (c >= N / 2) continue;
+        float a[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int ml = i * 16 + (lane / 16) * 4 + r;
-      const float g = weight ? weight[pair_of[wm * 64 + ml]] : 1.f;      // a factor on what the expert reads
-      if constexpr (MODE == kUpGated) {
+        for (int r = 0; r < 4; ++r) a[r] = silu<bf16_t>(g * acc[j][i][r]) * (g * acc[j + 1][i][r]);
+        *reinterpret_cast<uint2*>(dst + c) = uint2{two_bf16(a[0], a[1]), two_bf16(a[2], a[3])};
+      }
+    } else {
+      uint16_t* dst = static_cast<uint16_t*>(out) + static_cast<size_t>(p0 + m) * N;
 #pragma unroll
-        for (int j = 0; j < 4; j += 2)      // tile j: sixteen gate columns, tile j + 1: the same sixteen up columns
-          mine[ml * kPitch + j * 8 + lane % 16] = float_to_bf16_bits(silu<bf16_t>(g * acc[i][j][r]) * (g * acc[i][j + 1][r]));
-      } else {
+      for (int j = 0; j < TN; ++j) {      // (the columns are a multiple of 8)
+        const int c = n0 + (wn * TN + j) * 16 + fk * 4;
+        if (c >= N) continue;
+        float a[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float v = g * acc[i][j][r], z = fmaxf(v, 0.f);
-          mine[ml * kPitch + j * 16 + lane % 16] = float_to_bf16_bits(MODE == kUpGelu ? gelu_exact<bf16_t>(v) : z * z);
+        for (int r = 0; r < 4; ++r) {
+          const float v = g * acc[j][i][r], z = fmaxf(v, 0.f);
+          a[r] = MODE == kUpGelu ? gelu_exact<bf16_t>(v) : z * z;
         }
+        *reinterpret_cast<uint2*>(dst + c) = uint2{two_bf16(a[0], a[1]), two_bf16(a[2], a[3])};
       }
     }
-  __syncthreads();
-  const int cols = MODE == kUpGated ? N / 2 : N, c0 = (MODE == kUpGated ? n0 / 2 : n0) + wn * kWide;
-#pragma unroll
-  for (int it = 0; it < kWide / 8; ++it) {      // (the columns are a multiple of 8: a piece lies inside or outside)
-    const int idx = it * kWave + lane, ml = idx / (kWide / 8), c8 = (idx % (kWide / 8)) * 8, c = c0 + c8;
-    if (wm * 64 + ml >= rows || c >= cols) continue;
-    *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + static_cast<long long>(p0 + wm * 64 + ml) * cols + c) =
-        *reinterpret_cast<const uint4*>(mine + ml * kPitch + c8);
   }
 }
 
@@ -271,6 +183,68 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<Vec*>(out + row * H + c) = add ? *reinterpret_cast<const Vec*>(add + row * H + c) + acc : acc;
 }
 
+// Tiles: those of gemm_tiles.hip of an even number of accumulators a wave, with the same constants of a launch's time.
+#define KVCM_GROUPED_TILES(T)      \
+  T(64, 64, 2, 2, 4)               \
+  T(128, 64, 4, 2, 6)              \
+  T(128, 128, 2, 4, 4)             \
+  T(128, 192, 2, 3, 4)             \
+  T(256, 128, 4, 2, 3)             \
+  T(256, 192, 4, 3, 2)             \
+  T(256, 256, 2, 4, 2)
+
+struct High {
+  int bm, bn;
+};
+#define KVCM_HIGH(BM, BN, WM, WN, STAGES) {BM, BN},
+static constexpr High kHighs[] = {KVCM_GROUPED_TILES(KVCM_HIGH)};
+#undef KVCM_HIGH
+constexpr int kHighCount = sizeof(kHighs) / sizeof(kHighs[0]);
+
+// The tile for n pairs over E experts, N rows of K each: groups of pairs end in a tile that is half empty on average.
+static int best_grouped(int n, int E, int N, int K) {
+  const float used = n < E ? static_cast<float>(n) : static_cast<float>(E);
+  int best = 0;
+  float best_t = 0.f;
+  for (int i = 0; i < kHighCount; ++i) {
+    const float groups = (static_cast<float>(n) / static_cast<float>(kHighs[i].bm) + 0.5f * used) * static_cast<float>((N + kHighs[i].bn - 1) / kHighs[i].bn);
+    const float t = gemm_tile_time(kHighs[i].bm, kHighs[i].bn, groups, (K + kStepK - 1) / kStepK, used * static_cast<float>(N) * static_cast<float>(K));
+    if (i == 0 || t < best_t) {
+      best = i;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
+struct GroupedCall {
+  const void* A;
+  int lda;
+  const void* W;
+  const int *order, *count;
+  const int4* list;
+  int top;
+  void* out;
+  const float* weight;
+  int N, K, n, E;
+};
+
+template <int MODE>
+static int launch_grouped(int tile, const GroupedCall& c, hipStream_t s) {
+  const int col_blocks = (c.N + kHighs[tile].bn - 1) / kHighs[tile].bn;
+  const long long grid = (static_cast<long long>(c.n / kHighs[tile].bm + c.E) * col_blocks + 7) / 8 * 8;
+  KVCM_REQUIRE(grid < (1ll << 31), "moe_grouped: too many tiles");
+  int i = 0;
+#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES)                                                                                    \
+  if (tile == i++)                                                                                                                     \
+    moe_grouped_kernel<BM, BN, WM, WN, STAGES, MODE><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, s>>>(                          \
+        static_cast<const uint16_t*>(c.A), c.lda, static_cast<const uint16_t*>(c.W), c.order, c.count, c.list, c.top, c.out, c.weight, \
+        c.N, c.K, col_blocks);
+  KVCM_GROUPED_TILES(KVCM_GROUPED_LAUNCH)
+#undef KVCM_GROUPED_LAUNCH
+  return launch_status("moe_grouped");
+}
+
 }  // namespace kvcm
 
 using namespace kvcm;
@@ -280,44 +254,41 @@ extern "C" {
 // Does the grouped form take these sizes?  (bfloat16; rows of 16-byte pieces)
 int kvcm_moe_grouped_supported(int K, int F, int E) { return K > 0 && F > 0 && K % 8 == 0 && F % 8 == 0 && E > 0 && E <= 4096; }
 
-// Tiles a step of n pairs over E experts can have at most.
-int kvcm_moe_grouped_max_tiles(int n, int E) { return (n + kGM - 1) / kGM + E; }
+// int32 values of work memory that a step of n pairs over E experts needs for its lists of tiles (16-byte aligned)
+int kvcm_moe_grouped_lists(int n, int E) { return 4 + 8 * most_tiles(n, E); }
+int kvcm_moe_grouped_tile_count() { return kHighCount; }
 
 // h [T, K] bfloat16; w_up [E, F, K], w_down [E, H, F] bfloat16; chosen [T * top], weight [T * top]; work memory:
-// order [T * top] and tiles [3 * max_tiles + 1] (int32), act [T * top, F] (bfloat16), y [T * top, H] (32-bit); out [T, H] 32-bit.
+// order [T * top] and lists [kvcm_moe_grouped_lists] (int32), act [T * top, F] (bfloat16), y [T * top, H] (32-bit); out [T, H] 32-bit.
 // kind 0: act = square(relu(up)); 2: gelu(up); 1, gated: w_up [E, 2F, K] (gate and up rows interleaved sixteen at a time), act =
 // silu(gate) * up.  weigh_input: the weights are factors on what the experts read, not on what they give.  add [T, H] 32-bit
-// or null: out = add + the experts' sum.
+// or null: out = add + the experts' sum.  tile_up, tile_down: which tiles (< 0: those the rule picks).
 int kvcm_moe_grouped(const void* h, int ldh, const void* w_up, const void* w_down, const int* chosen, const float* weight,
-                     int* order, int* tiles, void* act, float* y, const float* add, float* out, int T, int K, int F, int H,
-                     int top, int E, int kind, int weigh_input, hipStream_t s) {
+                     int* order, int* lists, void* act, float* y, const float* add, float* out, int T, int K, int F, int H,
+                     int top, int E, int kind, int weigh_input, int tile_up, int tile_down, hipStream_t s) {
   if (T == 0) return 0;
   KVCM_REQUIRE(T > 0 && top > 0 && H > 0 && ldh >= K, "moe_grouped: bad sizes");
   KVCM_REQUIRE(kvcm_moe_grouped_supported(K, F, E), "moe_grouped: sizes K=%d F=%d experts=%d are not supported", K, F, E);
   KVCM_REQUIRE(static_cast<long long>(T) * top < (1ll << 30), "moe_grouped: too many rows");
+  KVCM_REQUIRE(static_cast<long long>(T) * ldh < (1ll << 31) && K < (1 << 22) && F < (1 << 22), "moe_grouped: more than 4 GB of rows");
   KVCM_REQUIRE(ldh % 8 == 0 && reinterpret_cast<uintptr_t>(h) % 16 == 0 && reinterpret_cast<uintptr_t>(w_up) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(w_down) % 16 == 0 && reinterpret_cast<uintptr_t>(act) % 16 == 0,
+                   reinterpret_cast<uintptr_t>(w_down) % 16 == 0 && reinterpret_cast<uintptr_t>(act) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(lists) % 16 == 0,
                "moe_grouped: operands must be 16-byte aligned");
-  const int n = T * top, max_tiles = kvcm_moe_grouped_max_tiles(n, E);
   KVCM_REQUIRE(kind >= 0 && kind <= 2, "moe_grouped: unknown kind of experts %d (0 relu2, 1 silu gated, 2 gelu)", kind);
   KVCM_REQUIRE(kind != 1 || F % 16 == 0, "moe_grouped: gated experts of %d columns are not supported (a multiple of 16)", F);
-  const int up_rows = kind == 1 ? 2 * F : F;
-  const float *up_weight = weigh_input ? weight : nullptr, *down_weight = weigh_input ? nullptr : weight;
-  const int up_blocks = (up_rows + kGN - 1) / kGN, down_blocks = (H + kGN - 1) / kGN;
-  const long long up_grid = static_cast<long long>(max_tiles) * ((up_blocks + 7) / 8) * 8;
-  const long long down_grid = static_cast<long long>(max_tiles) * ((down_blocks + 7) / 8) * 8;
-  KVCM_REQUIRE(up_grid < (1ll << 31) && down_grid < (1ll << 31), "moe_grouped: too many tiles");
-  moe_group_kernel<<<1, 1024, 2 * E * sizeof(int), s>>>(chosen, n, E, order, tiles, max_tiles);
-#define KVCM_GROUPED_UP(MODE)                                                                                              \
-  moe_grouped_kernel<MODE><<<static_cast<unsigned>(up_grid), 256, 0, s>>>(static_cast<const uint16_t*>(h), ldh,            \
-                                                                          static_cast<const uint16_t*>(w_up), order, tiles, \
-                                                                          top, act, up_weight, up_rows, K, up_blocks)
-  if (kind == 1) KVCM_GROUPED_UP(kUpGated);
-  else if (kind == 2) KVCM_GROUPED_UP(kUpGelu);
-  else KVCM_GROUPED_UP(kUp);
-#undef KVCM_GROUPED_UP
-  moe_grouped_kernel<kDown><<<static_cast<unsigned>(down_grid), 256, 0, s>>>(
-      static_cast<const uint16_t*>(act), F, static_cast<const uint16_t*>(w_down), order, tiles, top, y, down_weight, H, F, down_blocks);
+  KVCM_REQUIRE(tile_up < kHighCount && tile_down < kHighCount, "moe_grouped: no such tile");
+  const int n = T * top, up_rows = kind == 1 ? 2 * F : F;
+  if (tile_up < 0) tile_up = best_grouped(n, E, up_rows, K);
+  if (tile_down < 0) tile_down = best_grouped(n, E, H, F);
+  moe_group_kernel<<<1, 1024, 4 * E * sizeof(int), s>>>(chosen, n, E, order, lists, kHighs[tile_up].bm, kHighs[tile_down].bm);
+  const int4* list = reinterpret_cast<const int4*>(lists + 4);
+  const GroupedCall up{h, ldh, w_up, order, lists, list, top, act, weigh_input ? weight : nullptr, up_rows, K, n, E};
+  int rc = kind == 1 ? launch_grouped<kUpGated>(tile_up, up, s) : kind == 2 ? launch_grouped<kUpGelu>(tile_up, up, s) : launch_grouped<kUp>(tile_up, up, s);
+  if (rc) return rc;
+  const GroupedCall down{act, F, w_down, order, lists + 1, list + most_tiles(n, E), top, y, weigh_input ? nullptr : weight, H, F, n, E};
+  rc = launch_grouped<kDown>(tile_down, down, s);
+  if (rc) return rc;
   // four columns a thread where rows are whole 16-byte pieces (2,048 rows of 2,048 columns, two experts each: 20 us a column at a
   // time with a long division for its row, 15 us so)
   const bool four = H % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 && reinterpret_cast<uintptr_t>(add) % 16 == 0 &&

@@ -121,8 +121,9 @@ def _declare(lib):
     fn("kvcm_moe_down", vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, vp)
     fn("kvcm_moe_few_takes", i, i, i, i, i, i)
     fn("kvcm_moe_grouped_supported", i, i, i)
-    fn("kvcm_moe_grouped_max_tiles", i, i)
-    fn("kvcm_moe_grouped", vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, vp)
+    fn("kvcm_moe_grouped_lists", i, i)
+    fn("kvcm_moe_grouped_tile_count")
+    fn("kvcm_moe_grouped", vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, i, i, vp)
     fn("kvcm_pool_update", vp, vp, i, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, i, vp)
     fn("kvcm_attention_window_pool", vp, i, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, f, i, i, i, i, f, i, i, vp, i, f, vp)
     fn("kvcm_attention_window_pool_tiles_supported", i, i, i)
@@ -1794,14 +1795,15 @@ def moe_grouped_supported(K, F, E, dtype):
 
 
 def moe_grouped_tiles(pairs, E):
-    """int32 values of work memory that ``moe_grouped`` needs for its list of tiles."""
-    return 3 * lib().kvcm_moe_grouped_max_tiles(int(pairs), int(E)) + 1
+    """int32 values of work memory that ``moe_grouped`` needs for its lists of tiles."""
+    return lib().kvcm_moe_grouped_lists(int(pairs), int(E))
 
 
-def moe_grouped(h, w_up, w_down, chosen, weight, order, tiles, act, y, out, gated=False, add=None, activation="relu2", weigh_input=False):
+def moe_grouped(h, w_up, w_down, chosen, weight, order, tiles, act, y, out, gated=False, add=None, activation="relu2", weigh_input=False,
+                tile_up=-1, tile_down=-1):
     """As ``moe_rows``, for steps with many rows (bfloat16): the (row, slot) pairs grouped by expert and multiplied in tiles
     on the matrix cores.  Work memory: order int32 [T * top], tiles int32 [moe_grouped_tiles], act [T * top, F],
-    y float32 [T * top, H]."""
+    y float32 [T * top, H].  ``tile_up``, ``tile_down``: the products' tiles by number (< 0: chosen by the sizes)."""
     T, K = h.shape
     E, F, _ = _expert_shapes(w_up, w_down, gated)
     H, top = w_down.shape[1], chosen.shape[1]
@@ -1819,7 +1821,8 @@ def moe_grouped(h, w_up, w_down, chosen, weight, order, tiles, act, y, out, gate
     _i32(order, "order", T * top)
     _i32(tiles, "tiles", moe_grouped_tiles(T * top, E))
     _call("kvcm_moe_grouped", _ptr(h), h.stride(0), _ptr(w_up), _ptr(w_down), _ptr(chosen), _ptr(weight), _ptr(order), _ptr(tiles),
-          _ptr(act), _ptr(y), _ptr(add), _ptr(out), T, K, F, H, top, E, _expert_kind(gated, activation), 1 if weigh_input else 0, _stream())
+          _ptr(act), _ptr(y), _ptr(add), _ptr(out), T, K, F, H, top, E, _expert_kind(gated, activation), 1 if weigh_input else 0,
+          int(tile_up), int(tile_down), _stream())
     return out
 
 

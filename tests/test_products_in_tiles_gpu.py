@@ -1,6 +1,7 @@
 """Products in tiles (csrc/hip/gemm_tiles.hip): every tile at the sizes where its edges, its ring of stages and its slices of K
 can go wrong, against products in 64 bits, and the rule that hands products of many rows to it."""
 import ctypes as C
+import functools
 
 import pytest
 import torch
@@ -145,3 +146,14 @@ def test_many_rows_go_to_the_tiles_where_the_rule_says_so(ops, M, N, K, mine):
     if ops._tiles_take(M, N // 2, K, 1, gated=True):
         ops.swiglu(ops.gemm(x, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV)), plain)
         assert (act == plain).float().mean() > 0.98
+
+
+@pytest.mark.parametrize("tile", range(7))
+def test_routed_experts_in_every_tile(ops, tile, monkeypatch):
+    """groups that end inside a tile, in several tiles of an expert, K that ends inside a step, columns that end inside a tile"""
+    import test_routed_forms_gpu as forms
+    assert ops.lib().kvcm_moe_grouped_tile_count() == 7
+    monkeypatch.setattr(ops, "moe_grouped", functools.partial(ops.moe_grouped, tile_up=tile, tile_down=(tile + 3) % 7))
+    for T, E, top, K, F, H, kind, one in forms.GROUPED + [(700, 3, 2, 320, 208, 516, "silu", False)]:
+        chosen = torch.zeros(T, top, dtype=torch.long) if one else None
+        forms._check("grouped", forms._case(T, E, top, K, F, H, kind, T + K, chosen), kind, tile % 2 == 0, tile % 2 == 1)
