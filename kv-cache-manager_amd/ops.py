@@ -711,6 +711,39 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
     return out
 
 
+# act(gate) * up in a product's epilogue (gemm_tiles.h: TileAct), without roundings before the end
+_TILE_ACTS = {"silu": 1, "clamped": 1, "relu": 2}
+
+
+def _gated_tiles_take(M, I, K):
+    """Where gate and up rows in unsplit tiles are no slower than a product cut along K and a launch for the activation (us, as two / so):
+    8 rows 5632 x 2048 14.9 / 11.4, 2816 x 2048 10.3 / 8.3 (9.5 in the kernel of few rows), 2816 x 4096 17.7 / 15.0, 1408 x 2048 7.6 / 7.5, 1024 x
+    2048 6.1 / 7.2, 2048 x 4096 13.7 / 14.4; one row 2816 x 2048 8.7 / 8.8 (8.2), 5632 x 2048 13.0 / 11.3; 16 to 64 rows 512 x 2048 8.9 / 7.2,
+    1024 x 4096 12.2 to 13.7 / 12.2 to 12.7, 2048 x 4096 13.5 to 14.8 / 13.7 to 15.5, 5632 x 4096 21.8 to 26.3 / 20.0 to 23.9."""
+    blocks = I // 32 * -(-M // 128)
+    return blocks >= 160 or (M >= 2 and blocks >= 80) or (M > 8 and K <= 2048 and I >= 512)
+
+
+def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0):
+    """out[M, I] = act(x[M, K] @ w_gate^T) * (x @ w_up^T), w_gate_up [2 I, K] the gate rows and the up rows, in one launch and in 32
+    bits up to the result ("silu", "relu", or "clamped": ``gated_act``'s with ``limit``), or False where two launches (a product with
+    a 32-bit result, ``gated_act``) are the faster or this has no kernel."""
+    if activation not in _TILE_ACTS or x.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16:
+        return False
+    _dev(x, w_gate_up, out)
+    for t, n in ((x, "x"), (w_gate_up, "w_gate_up"), (out, "out")):
+        _rows2d(t, n)
+    M, K = x.shape
+    I = out.shape[1]
+    _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_gated shapes do not agree")
+    if (I % 32 or K % 64 or x.stride(0) % 8 or w_gate_up.stride(0) % 8 or x.data_ptr() % 16 or w_gate_up.data_ptr() % 16
+            or not (_tiles_take(M, I, K, 1, gated=True) if many_rows(M) else _gated_tiles_take(M, I, K))):
+        return False
+    _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0), out.stride(0), 1,
+          1, _TILE_ACTS[activation], float(limit) if activation == "clamped" else 0.0, -1, _stream())
+    return True
+
+
 def gemm_swiglu(x, w_gate_up, out, limit=0.0):
     """out[M, I] = swiglu(x[M, K] @ w_gate_up[2 I, K]^T), or with ``limit`` > 0 its form with limits (``gated_act``'s "clamped"), in one launch, or False when this shape
     has no fused kernel (then the caller runs the product and ``swiglu`` one after the other:

@@ -167,7 +167,7 @@ class ScaledTokenEmbedding(Embedding):
 @FEED_FORWARDS.register("gated_mlp")
 class GatedFeedForward(JoinableEnds, FeedForward):
     """down(act(gate(h)) * up(h)), gate and up as one fused projection whose 32-bit sums go straight into the
-    activation (steps of few rows in bfloat16 with silu or "clamped" and without biases: in the product's own epilogue).
+    activation (in bfloat16 with silu, relu or "clamped" and without biases: in the product's own epilogue).
     params: intermediate_size, activation ("relu" | "silu" | "gelu_tanh" | "gelu", or "clamped" with ``limit``: g * sigmoid(1.702 g) *
     (u + 1) with g = min(gate, limit) and u = up held within +-limit); gate, up, down: the
     checkpoint names after the prefix (defaults "gate", "up", "down"); bias: all three projections have one (the tensor's
@@ -211,10 +211,13 @@ class GatedFeedForward(JoinableEnds, FeedForward):
         act = step.ws("gated_act", (step.rows, I))
         kind = self.params.get("activation", "silu")
         limit = self.params.get("limit", 0.0) if kind == "clamped" else 0.0
-        # few rows in bfloat16 with silu or its form with limits: the product that streams gate and up rows together and applies
-        # the activation in its epilogue, one launch (silu is rounded once more on the way, within the result's own rounding)
-        if not (kind in ("silu", "clamped") and act.dtype == torch.bfloat16 and torch.is_tensor(h)
-                and not ops.many_rows(step.rows) and ops.gemm_swiglu(h, self.w["w_gate_up"], act, limit=limit)):
+        # bfloat16 with silu, relu or silu's form with limits: the product of gate and up rows together, the activation in its
+        # epilogue, one launch; the kernel of few rows, for what that does not take, rounds silu once more on the way, within the
+        # result's own rounding
+        one = act.dtype == torch.bfloat16 and torch.is_tensor(h) and (
+            ops.gemm_gated(h, self.w["w_gate_up"], act, kind, limit)
+            or kind in ("silu", "clamped") and not ops.many_rows(step.rows) and ops.gemm_swiglu(h, self.w["w_gate_up"], act, limit=limit))
+        if not one:
             gu = linear32(self.ctx, step, h, self.w["w_gate_up"], "gated_gate_up")
             ops.gated_act(gu, act, kind, limit=limit)
         return linear32(self.ctx, step, act, self.w["w_down"], "gated_out", keep_partial=bool(self.params.get("partial_out")))

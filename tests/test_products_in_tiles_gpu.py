@@ -157,3 +157,22 @@ def test_routed_experts_in_every_tile(ops, tile, monkeypatch):
     for T, E, top, K, F, H, kind, one in forms.GROUPED + [(700, 3, 2, 320, 208, 516, "silu", False)]:
         chosen = torch.zeros(T, top, dtype=torch.long) if one else None
         forms._check("grouped", forms._case(T, E, top, K, F, H, kind, T + K, chosen), kind, tile % 2 == 0, tile % 2 == 1)
+
+
+@pytest.mark.parametrize("M,I,K,one", [(1, 2816, 2048, False), (2, 2560, 2048, True), (8, 2048, 2048, False), (9, 512, 2048, True), (95, 512, 2112, False),
+                                       (300, 1408, 2048, True), (1, 5120, 64, True), (40, 2816, 8, False)])
+def test_gated_products_without_roundings_before_the_end(ops, M, I, K, one):
+    """the rule, and each activation as ``gated_act`` of the product's 32-bit result gives it"""
+    x, w = _operands(M + I, M, 2 * I, K)
+    gu = (x.double() @ w.double().t()).float()
+    for activation, limit in (("relu", 0.0), ("silu", 0.0), ("clamped", 1.5)):
+        got = torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert ops.gemm_gated(x, w, got, activation, limit) == one
+        if one:
+            want = torch.empty_like(got)
+            ops.gated_act(gu, want, activation, limit=limit)
+            # both round once; 32-bit sums of K terms may fall on the other side of a tie
+            scale = gu[:, :I].abs() * gu[:, I:].abs() + gu.abs().amax() * 2.0 ** -8
+            assert (got == want).float().mean() > 0.98
+            assert bool(((got.float() - want.float()).abs() <= 2.0 ** -7 * (scale + want.float().abs())).all())
+    assert ops.gemm_gated(x, w, got, "gelu") is False and ops.gemm_gated(x.float(), w.float(), got.float(), "relu") is False
