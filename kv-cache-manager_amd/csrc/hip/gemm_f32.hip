@@ -11,15 +11,18 @@
 // By sizes:
 //   K <= 256    one chain over all of K in ascending order (the instruction takes its four k in ascending order, checked bit
 //               for bit); the segments above are for longer sums.  Tiles of 32 x 32 or 64 x 64.
+//   up to 8 rows of up to 2,048 columns, one or two rows of many: workgroups of 8 columns (gemm_f32_rows8_kernel).
 //   few rows    bound by reading W once.  A workgroup owns 16 columns, its waves one segment each, eight 16-byte loads of W a
 //               lane multiplied while the next eight are on their way; segments meet in LDS.  Two rows, K = 2048: N = 11264
 //               (92 MB) 22 us, 4.2 TB/s; N = 2048 8 us; K = 5632, N = 2048 20 us.  As 16 x 64 tiles of plain fused
 //               multiply-adds with scalar loads these took 304 us in the mean.
 //               Up to 32 rows of very many columns: tiles of 32 rows as below.
-//   more rows   bound by the matrix cores (157 TFLOP/s).  Tiles of 64 x 64 or 64 x 32, four waves, 32 k staged in LDS while the
-//               next 32 are on their way.  573 rows, K = 2048: N = 11264 254 us (104 TFLOP/s), N = 2048 68 us; 539 us in the
-//               mean of a layer's four products as 64 x 64 tiles of plain fused multiply-adds.
+//   more rows   bound by the matrix cores (157 TFLOP/s).  Tiles of 64 x 64 or 64 x 32, four waves, 32 k a step, three further steps on
+//               their way (gemm_f32_ring_kernel).  573 rows, K = 2048: N = 11264 225 us (118 TFLOP/s), N = 2048 54; K = 5632, N =
+//               2048 141; staged through registers, one step on its way, 247, 66 and 173.  Rows that are not whole 16-byte pieces
+//               are staged so still.
 #include "common.h"
+#include "tile_ring.h"
 
 namespace kvcm {
 
@@ -56,6 +59,84 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ row, int k, int
     }
   }
   return v;
+}
+
+// ---- up to 8 rows: columns 8 blockIdx.x .. + 7, wave w segments w and w + 4 ------------------------------------------------
+// The instruction's 16 x 16 results as two blocks of 8 x 8 on the diagonal: operand rows and columns 0..7 are X's rows and W's columns
+// over one segment, 8..15 the same over the other (the two blocks beside the diagonal mean nothing).  Every lane then loads W
+// of its own where the kernel below has 16 columns a workgroup, so that N / 8 workgroups of four waves cover the chip where N / 16 of eight
+// leave half of it idle.  Per element the same chain.
+template <bool FOURS>
+__global__ void __launch_bounds__(kSegments / 2 * kWave)
+    gemm_f32_rows8_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
+                          int ldx, int ldw, int ldy) {
+  __shared__ float sums[kSegments][8][8];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int r = lane & 15, g = lane >> 4, half = r >> 3, r8 = r & 7;
+  const int n0 = blockIdx.x * 8;
+  const int n = n0 + r8 < N ? n0 + r8 : N - 1, m = r8 < M ? r8 : M - 1;
+  const int seg = segment_units(K), units = (K + kUnit - 1) / kUnit;
+  const int s0 = wave, s1 = wave + kSegments / 2;
+  // units of the wave's two segments (the later one is never the longer)
+  const int long_units = s0 * seg + seg < units ? seg : units - s0 * seg, short_units = s1 * seg + seg < units ? seg : units - s1 * seg;
+  const int lo = (half ? s1 : s0) * seg, mine = half ? short_units : long_units;
+  const float *w = W + size_t(n) * ldw, *x = X + size_t(m) * ldx;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int D = 4;
+  f32x4 b[2][D][2], a[2][D][2];
+  auto fetch = [&](f32x4 (&bb)[D][2], f32x4 (&aa)[D][2], int u) {
+    if (u + D <= short_units && (s1 * seg + u + D) * kUnit <= K) {
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = (lo + u + d) * kUnit + 16 * h + 4 * g;
+          bb[d][h] = load4<true, true>(w, k, K);
+          aa[d][h] = load4<true, true>(x, k, K);
+        }
+    } else {
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = u + d < mine ? (lo + u + d) * kUnit + 16 * h + 4 * g : K;      // (beyond the segment: zeros)
+          bb[d][h] = load4<FOURS>(w, k, K);
+          aa[d][h] = load4<FOURS>(x, k, K);
+        }
+    }
+  };
+  auto multiply = [&](const f32x4 (&bb)[D][2], const f32x4 (&aa)[D][2]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[d][h][q], bb[d][h][q], acc, 0, 0, 0);
+  };
+  if (long_units > 0) fetch(b[0], a[0], 0);
+  for (int u = 0; u < long_units; u += 2 * D) {
+    if (u + D < long_units) fetch(b[1], a[1], u + D);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(b[0], a[0]);
+    if (u + D >= long_units) break;
+    __builtin_amdgcn_sched_barrier(0);
+    if (u + 2 * D < long_units) fetch(b[0], a[0], u + 2 * D);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(b[1], a[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (g / 2 == half) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sums[half ? s1 : s0][4 * (g & 1) + e][r8] = acc[e];
+  }
+  __syncthreads();
+  const int segments = (units + seg - 1) / seg;
+  if (threadIdx.x < 64) {
+    const int row = threadIdx.x / 8, c = threadIdx.x % 8;
+    float total = sums[0][row][c];
+    for (int i = 1; i < segments; ++i) total += sums[i][row][c];
+    if (row < M && n0 + c < N) Y[size_t(row) * ldy + n0 + c] = total;
+  }
 }
 
 // ---- up to 16 * MT rows: columns 16 blockIdx.x .. + 15, wave w segment w ---------------------------------------------------
@@ -263,12 +344,121 @@ __global__ void __launch_bounds__(256, 2)
     }
 }
 
+// The same tiles with operands by 16-byte requests straight into a ring of stages in LDS (tile_ring.h): where rows are whole 16-byte
+// pieces and K whole units.  A step has 1,024 cycles of matrix instructions a wave; staged through registers the stores, the
+// wait for them and the barrier came on top, here only the barrier.  Per element the same sequence.
+template <int TM, int TN, int STAGES>
+__global__ void __launch_bounds__(256, 2)
+    gemm_f32_ring_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
+                         int ldx, int ldw, int ldy, int tiles_m) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, R = (BM + BN) / 32;      // requests of eight rows a wave
+  constexpr int kStage = (BM + BN) * 128;
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[STAGES * kStage];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int r = lane & 15, g = lane >> 4;
+  const int id = neighbours_on_one_xcd();
+  const int m0 = id % tiles_m * BM, n0 = id / tiles_m * BN;
+  const int wm = (wave >> 1) * 16 * TM, wn = (wave & 1) * 16 * TN;
+  const int seg = segment_units(K), steps = K / kUnit;
+  const uint64_t xbase = reinterpret_cast<uint64_t>(X + size_t(m0) * ldx), wbase = reinterpret_cast<uint64_t>(W + size_t(n0) * ldw);
+  uint32_t offset[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int req = q * 4 + wave, row = req * 8 + lane / 8;
+    const int at = req < BM / 8 ? (row < M - m0 ? row : M - 1 - m0) : (row - BM < N - n0 ? row - BM : N - 1 - n0);
+    offset[q] = static_cast<uint32_t>(at) * static_cast<uint32_t>(req < BM / 8 ? ldx : ldw) * 4u + static_cast<uint32_t>((lane % 8) ^ (lane / 8)) * 16u;
+  }
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>(reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(ring)))));
+  auto request = [&](int t, int stage) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int req = q * 4 + wave;
+      ring_bring16(offset[q], (req < BM / 8 ? xbase : wbase) + static_cast<uint64_t>(t) * 128, lds0 + stage * kStage + req * 1024);
+    }
+  };
+  f32x4 acc[TM][TN], total[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int left = seg;      // units left in the segment
+  auto step = [&](int stage) {
+    const f32x4 *xs = reinterpret_cast<const f32x4*>(ring + stage * kStage), *ws = xs + BM * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4 a[TM], w[TN];
+      const int c = (4 * h + g) ^ (r & 7);      // (rows 16 apart have the same place in a row)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = xs[(wm + 16 * i + r) * 8 + c];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) w[j] = ws[(wn + 16 * j + r) * 8 + c];
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][m], w[j][m], acc[i][j], 0, 0, 0);
+    }
+    if (--left == 0) {      // a segment ends
+      left = seg;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < steps) request(t, t);
+  int stage = 0, fill = STAGES - 1;
+  for (int t = 0; t < steps; ++t) {
+    if (t + STAGES - 1 < steps) {
+      ring_arrived<(STAGES - 2) * R>();
+      request(t + STAGES - 1, fill);      // into the stage that everybody has read by now
+    } else {
+      ring_arrived<0>();
+    }
+    step(stage);
+    fill = fill + 1 == STAGES ? 0 : fill + 1;
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if (left != seg) total[i][j] += acc[i][j];      // the last segment, where it is shorter
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm + 16 * i + 4 * g + e, n = n0 + wn + 16 * j + r;
+        if (m < M && n < N) Y[size_t(m) * ldy + n] = total[i][j][e];
+      }
+    }
+}
+
 // K up to 256 (models of small width, low-rank factors): these launches are bound by their latency, so they are not cut.
 constexpr int kShortK = 256;
 
+// Rows of whole 16-byte pieces, whole units.
+inline bool through_ring(const float* X, const float* W, int K, int ldx, int ldw) {
+  return K % kUnit == 0 && ldx % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0 &&
+         ldx < (1 << 22) && ldw < (1 << 22);
+}
+
 template <int TM, int TN, bool FOURS, bool ASCENDING>
 void launch_tiles(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t s) {
-  const dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + 32 * TM - 1) / (32 * TM));
+  const int tiles_n = (N + 32 * TN - 1) / (32 * TN), tiles_m = (M + 32 * TM - 1) / (32 * TM);
+  if constexpr (!ASCENDING) {
+    const long long groups = static_cast<long long>(tiles_m) * tiles_n;
+    if (through_ring(X, W, K, ldx, ldw) && groups < (1ll << 31)) {
+      gemm_f32_ring_kernel<TM, TN, 4><<<static_cast<unsigned>(groups), 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy, tiles_m);
+      return;
+    }
+  }
+  const dim3 grid(tiles_n, tiles_m);
   gemm_f32_tiles_kernel<TM, TN, FOURS, ASCENDING><<<grid, 256, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
 }
 
@@ -285,6 +475,10 @@ void launch_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int
   // 300 x 2048 7.7 / 8.6, 128 x 8192 9.4 / 9.0, 1000 x 2048 16.6 / 13.7, 4000 x 2048 56 / 47 (90 TFLOP/s).  With operands straight from
   // L2 into a wave's registers these took 33, 33, 34, 60 and 228 us, as plain fused multiply-adds from LDS 29, 29, 30, 33 and 81.
   const long long few = (long long)((M + 63) / 64) * ((N + 31) / 32), large = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  // Through the ring (us, 64 x 32 / 64 x 64, K = 2048): 300 rows, N = 11264 125 / 136, 573 rows 225 / 239, 640 rows 240 / 239, 1000 rows 379 /
+  // 372, 2048 rows 808 / 732; 1600 rows, N = 2048 124 / 135, N = 2560 147 / 137: what the fullest CU has to do, a smaller tile 0.53 of
+  // a larger one; but not larger tiles that are alone on their CUs (300 rows, N = 2048: 39 / 43).
+  const bool larger = through_ring(X, W, K, ldx, ldw) ? large > 256 && 0.53f * static_cast<float>((few + 255) / 256) >= static_cast<float>((large + 255) / 256) : large >= 704;
   if (K <= kShortK) {
     if (large >= 256) launch_tiles<2, 2, FOURS, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
     else launch_tiles<1, 1, FOURS, true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
@@ -304,12 +498,21 @@ void launch_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int
     launch_tiles<1, 1, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
     return;
   }
+  // Up to 8 rows in blocks of 8 columns while those are at most one a CU, one or two rows also from two a CU on; us, 16 columns a workgroup /
+  // 8: one row 2048 x 2048 8.3 / 6.2, 2048 x 5632 20.8 / 14.1, 512 x 512 4.7 / 3.8, 11264 x 2048 23.0 / 21.5, 6144 x 4096 28.4 / 22.1, 28672 x 4096 95 / 86;
+  // 8 rows 2048 x 2048 9.1 / 7.3, 2048 x 5632 23.5 / 17.5.  In between, and for more rows of many columns, which each block of columns
+  // reads again, no: 2560 x 2048 8.2 / 8.4, 8 rows 8192 x 2048 19.2 / 20.9, 28672 x 4096 112 / 120; nor very long K: 4096 x 14336 46.8 / 47.3.
+  const int eights = (N + 7) / 8;
+  if (M <= 8 && (eights <= 256 || (M <= 2 && eights >= 512 && K <= 8192))) {
+    gemm_f32_rows8_kernel<FOURS><<<eights, kSegments / 2 * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
+    return;
+  }
   if (M <= 16 || few < (M <= 32 ? 600 : 228)) {
     const dim3 grid((N + 15) / 16, M <= 64 ? 1 : (M + 63) / 64);
     if (M <= 16) gemm_f32_rows_kernel<1, FOURS><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
     else if (M <= 32) gemm_f32_rows_kernel<2, FOURS><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
     else gemm_f32_rows_kernel<4, FOURS><<<grid, kSegments * kWave, 0, s>>>(X, W, Y, M, N, K, ldx, ldw, ldy);
-  } else if (large >= 704) {
+  } else if (larger) {
     launch_tiles<2, 2, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   } else {
     launch_tiles<2, 1, FOURS, false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
