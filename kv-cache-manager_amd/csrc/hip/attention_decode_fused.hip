@@ -278,8 +278,7 @@ __global__ void __launch_bounds__(WAVES* kWave, HD == 64 ? 8 / WAVES : 1)
           mx = fmaxf(mx, s[g][4 * t + i]);
         }
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float alpha = exp2f(m_run - m_new);
     m_run = m_new;
@@ -343,8 +342,7 @@ __global__ void __launch_bounds__(WAVES* kWave, HD == 64 ? 8 / WAVES : 1)
   }
 
   // ---- the waves' results, merged in wave order: out = sum_w e_w o_w / sum_w e_w l_w, e_w = 2^(m_w - m)
-  l_run += __shfl_xor(l_run, 16, kWave);
-  l_run += __shfl_xor(l_run, 32, kWave);
+  l_run = rows_sum(l_run);
   if (kq == 0) { w_max[wave][n16] = m_run; w_sum[wave][n16] = l_run; }
 #pragma unroll
   for (int d = 0; d < DT; ++d)

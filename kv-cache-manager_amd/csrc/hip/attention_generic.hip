@@ -225,8 +225,7 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
           s[i][e] = sees ? s[i][e] : -INFINITY;
           top = fmaxf(top, s[i][e]);
         }
-      top = fmaxf(top, __shfl_xor(top, 16, kWave));
-      top = fmaxf(top, __shfl_xor(top, 32, kWave));
+      top = rows_max(top);
       const float m_new = fmaxf(m, top);
       const bool some = m_new > -INFINITY;                      // the item has seen a key with a finite score
       const float alpha = some ? expf(m - m_new) : 1.f;
@@ -284,8 +283,7 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
     if (c0 < most) walk(c0, std::integral_constant<int, 1>());      // (absent keys add zeros: left out where they are most of the last chunk)
     j = end;
   }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
+  l = rows_sum(l);
   if (g == 0) {
     part_m[own_share][it] = m;
     part_l[own_share][it] = l;

@@ -76,16 +76,6 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   r.v = __builtin_convertvector(float2_t{a, b}, bf16x2_t);   // one v_cvt_pk_bf16_f32
   return r.u;
 }
-// all-reduce over the four lanes that share lane % 16 (lanes l, l^16, l^32, l^48)
-__device__ __forceinline__ float quad_rows_max(float v) {
-  // v_permlane16_swap / v_permlane32_swap with both operands the same register leave one half of
-  // each lane pair in the first result and the other half in the second
-  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 // Two waves per SIMD at least: with that bound the compiler keeps the accumulators of the matrix
 // instructions in ordinary registers (no copies to and from the accumulation registers around the softmax).
 // At head_dim 64 the kernel fits three (two tiles a wave: 168 registers) or four (one tile); the bound
@@ -294,7 +284,7 @@ __global__ void __launch_bounds__(kPfGroupThreads * KH, HD == 64 ? (RT == 1 ? 4 
 #pragma unroll
             for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[rt][j][i]);
         }
-        mx = quad_rows_max(mx);
+        mx = rows_max(mx);
         // m is finite once the row has seen a key; a row that starts before this segment's first
         // key has seen none of it yet (m_new = -FLT_MAX): its probabilities are zero
         const float m_new = fmaxf(m[rt], mx);

@@ -469,16 +469,6 @@ __device__ __forceinline__ float below_upper(float x) {
   return fmaxf(x - __uint_as_float(__float_as_uint(x) & 0xFFFF0000u), fminf(x, 1.17549435e-38f));
 }
 
-// largest / sum of the four lanes that share lane % 16
-__device__ __forceinline__ float quads_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  return fmaxf(v, __shfl_xor(v, 32, kWave));
-}
-__device__ __forceinline__ float quads_sum(float v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
-}
-
 // DP: key size padded to a multiple of 32; DVT: tiles of 16 value columns
 template <int DP, int DVT, int WAVES>
 __global__ void __launch_bounds__(WAVES* kWave)
@@ -542,7 +532,7 @@ __global__ void __launch_bounds__(WAVES* kWave)
       sv[j] = key >= lo && key < hi ? sv[j] : -INFINITY;
       mx = fmaxf(mx, sv[j]);
     }
-    const float m_new = fmaxf(m, quads_max(mx));
+    const float m_new = fmaxf(m, rows_max(mx));
     const float alpha = expf(m - m_new);
     m = m_new;
     l *= alpha;
@@ -689,7 +679,7 @@ __global__ void __launch_bounds__(WAVES* kWave)
         for (int j = 8 * g; j < 8 * g + 8; ++j) sv[j] = below_upper(sv[j]);
       }
   }
-  l = quads_sum(l);
+  l = rows_sum(l);
 #pragma unroll
   for (int vt = 0; vt < DVT; ++vt) *reinterpret_cast<f32x4*>(&parts[wave][col][vt * 16 + 4 * quad]) = o[vt];
   if (quad == 0) {

@@ -37,14 +37,6 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return uint32_t(float_to_bf16_bits(a)) | (uint32_t(float_to_bf16_bits(b)) << 16);
 }
 
-// largest of the four lanes that share lane % 16
-__device__ __forceinline__ float quad_max(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 // tanh of a score: an odd polynomial up to 5/8 (x + x^3 p(x^2), p fitted to 4e-9 of the result), (1 - e) / (1 + e) with
 // e = 2^(-2 |x| log2 e) by the hardware's exp2 and reciprocal beyond.  As exact as tanhf, which is some thirty instructions of a
 // score's fifty: over [-12, 12] at most 1.6e-7 of the result off (tanhf 1.7e-7), 2.7e-8 on average up to 5/8 and 4e-8 beyond (the same).
@@ -271,7 +263,7 @@ __global__ void __launch_bounds__(256, DP <= 64 && DVT <= 4 ? 4 : DVT <= 8 ? 2 :
     float mx = kMasked;
 #pragma unroll
     for (int j = 0; j < 16; ++j) mx = fmaxf(mx, sv[j]);
-    const float m_new = fmaxf(m, quad_max(mx));
+    const float m_new = fmaxf(m, rows_max(mx));
     const float alpha = __builtin_amdgcn_exp2f(m - m_new);
     m = m_new;
 #pragma unroll

@@ -145,20 +145,32 @@ __device__ __forceinline__ void head_and_columns(int heads, int col_blocks, int&
   }
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+// Sum and maximum of a lane's value and its partners' in the other rows of 16 lanes (l, l ^ 16, l ^ 32, l ^ 48), by the instructions that
+// swap rows of 16 and halves of 32 lanes: with both operands the same register they leave a lane's value and its partner's side
+// by side.  (A shuffle goes through LDS, some 100 cycles each.)
+__device__ __forceinline__ float halves_sum(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(both[0]) + __uint_as_float(both[1]);
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+__device__ __forceinline__ float halves_max(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
 }
+__device__ __forceinline__ float row_pairs_sum(float v) {
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+__device__ __forceinline__ float row_pairs_max(float v) {
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+__device__ __forceinline__ float rows_sum(float v) { return halves_sum(row_pairs_sum(v)); }
+__device__ __forceinline__ float rows_max(float v) { return halves_max(row_pairs_max(v)); }
 
 // Sum over aligned groups of G lanes (a power of two); every lane of a group gets the result.  Up to 16 lanes the
 // partners come by data-parallel-primitive moves inside a row of 16 (a few cycles each: lane ^ 1, lane ^ 2, then the
-// mirrored half and the mirrored row, whose lanes hold the other half's sum already); beyond that by shuffles.
+// mirrored half and the mirrored row, whose lanes hold the other half's sum already); beyond that by swaps
+// of rows and halves.
 template <int CTRL>
 __device__ __forceinline__ float dpp_take(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
@@ -169,8 +181,8 @@ __device__ __forceinline__ float group_sum(float v) {
   if constexpr (G >= 4) v += dpp_take<0x4E>(v);       // quad_perm [2, 3, 0, 1]
   if constexpr (G >= 8) v += dpp_take<0x141>(v);      // row_half_mirror
   if constexpr (G >= 16) v += dpp_take<0x140>(v);     // row_mirror
-  if constexpr (G >= 32) v += __shfl_xor(v, 16, kWave);
-  if constexpr (G >= 64) v += __shfl_xor(v, 32, kWave);
+  if constexpr (G >= 32) v = row_pairs_sum(v);
+  if constexpr (G >= 64) v = halves_sum(v);
   return v;
 }
 
@@ -180,29 +192,26 @@ __device__ __forceinline__ float group_max(float v) {      // as group_sum, the 
   if constexpr (G >= 4) v = fmaxf(v, dpp_take<0x4E>(v));
   if constexpr (G >= 8) v = fmaxf(v, dpp_take<0x141>(v));
   if constexpr (G >= 16) v = fmaxf(v, dpp_take<0x140>(v));
-  if constexpr (G >= 32) v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  if constexpr (G >= 64) v = fmaxf(v, __shfl_xor(v, 32, kWave));
+  if constexpr (G >= 32) v = row_pairs_max(v);
+  if constexpr (G >= 64) v = halves_max(v);
   return v;
 }
 
-// Sum over a block of THREADS threads (a multiple of 64); every thread gets the result.  The
-// order of additions depends on THREADS only.
+__device__ __forceinline__ float wave_sum(float v) { return group_sum<kWave>(v); }
+__device__ __forceinline__ float wave_max(float v) { return group_max<kWave>(v); }
+
+// Sum over a block of THREADS threads (a multiple of 64); every thread gets the result and adds the waves' sums itself, in wave order
+// (a second barrier keeps the next sum out of scratch until everybody has).  The order of additions depends on THREADS only.
 template <int THREADS>
-__device__ __forceinline__ float block_sum(float v, float* scratch /* THREADS/64 + 1 floats */) {
+__device__ __forceinline__ float block_sum(float v, float* scratch /* THREADS / 64 floats */) {
   v = wave_sum(v);
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  if (lane == 0) scratch[wave] = v;
+  if (threadIdx.x % kWave == 0) scratch[threadIdx.x / kWave] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
+  float s = scratch[0];
 #pragma unroll
-    for (int w = 0; w < THREADS / kWave; ++w) s += scratch[w];
-    scratch[THREADS / kWave] = s;
-  }
+  for (int w = 1; w < THREADS / kWave; ++w) s += scratch[w];
   __syncthreads();
-  const float r = scratch[THREADS / kWave];
-  __syncthreads();
-  return r;
+  return s;
 }
 
 // ---- host side ------------------------------------------------------------------------------

@@ -24,9 +24,9 @@
 // asks for all its weight bytes of a trip at once (32 contiguous bytes per row and unit, four lanes
 // one 128-byte line), two trips in flight.  The waves' sums meet in LDS in a fixed order.
 //
-// More rows than 8 go through the shared-rows product with norms of their own (gemm_skinny.hip): every
+// More rows than 8 go through products in tiles with norms of their own (gemm_tiles.hip): every
 // workgroup here reads all of X, M x K per 8 or 16 output columns, from L2, which at 8 rows is as many
-// bytes as the weights themselves (a 16-row variant of this kernel lost to the shared-rows path at every
+// bytes as the weights themselves (a 16-row variant of this kernel lost to such products at every
 // size measured: TinyLlama sizes batch 16 1.26 -> 1.17 ms, Llama-3-8B sizes 4.82 -> 4.05 ms).
 #include "common.h"
 #include "kvcm_hip.h"
@@ -228,10 +228,7 @@ __global__ void __launch_bounds__(NW * kWave) gemm8_kernel(const Gemm8Args a) {
       a.resid[size_t(m) * a.N + col] = xn;
       a.xg[size_t(m) * a.N + col] = float_to_bf16_bits(g_in * round_to<bf16_t>(xn));
     }
-    float sq = xn * xn;
-    sq += __shfl_xor(sq, 1, kWave);
-    sq += __shfl_xor(sq, 2, kWave);
-    sq += __shfl_xor(sq, 4, kWave);
+    const float sq = group_sum<8>(xn * xn);
     if (live && n == 0) a.ss_out[size_t(m) * (a.N / kCols) + blockIdx.x] = sq;
   }
 }
