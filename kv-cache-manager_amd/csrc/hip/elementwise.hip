@@ -44,6 +44,29 @@ __global__ void embed_kernel(const int* __restrict__ ids, const TW* __restrict__
   for (int i = threadIdx.x; i < H; i += blockDim.x) dst[i] = load_f(src + i);
 }
 
+// The same for rows of whole 16-byte pieces: eight (four) entries a thread, so that a row of 2,048 costs one trip to memory where one
+// entry a thread and trip cost eight (one row: 5.1 -> 2.1 us).
+template <class TW>
+__global__ void __launch_bounds__(256) embed_pieces_kernel(const int* __restrict__ ids, const TW* __restrict__ table, float* __restrict__ x, int H, int V) {
+  constexpr int kPiece = 16 / sizeof(TW);
+  const int t = blockIdx.y, i = (blockIdx.x * 256 + threadIdx.x) * kPiece;
+  if (i >= H) return;
+  const int id = ids[t];
+  const bool known = id >= 0 && id < V;      // the host refuses others; never read outside the table
+  union {
+    uint4 u;
+    TW e[kPiece];
+  } piece;
+  piece.u = *reinterpret_cast<const uint4*>(table + size_t(known ? id : 0) * H + i);
+  float* dst = x + size_t(t) * H + i;
+#pragma unroll
+  for (int q = 0; q < kPiece; q += 4) {
+    float4 v{load_f(&piece.e[q]), load_f(&piece.e[q + 1]), load_f(&piece.e[q + 2]), load_f(&piece.e[q + 3])};
+    if (!known) v = float4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<float4*>(dst + q) = v;
+  }
+}
+
 // -------------------------------------------------------------------------------- RMS norm
 // v = x[src] (+ add[src]); optionally x[src] = v; out[r] = w * round(v * inv)  with
 // inv = 1/sqrt(mean(v^2) + eps).  src = rows ? rows[r] : r.  The added term is a tensor, or the
@@ -564,6 +587,14 @@ int kvcm_act_rows(const float* in, int ld, int splits, long long split_stride, v
 int kvcm_embed(const int* ids, const void* table, int table_dtype, float* x, int T, int H, int V, hipStream_t s) {
   if (T == 0) return 0;
   KVCM_REQUIRE(T > 0 && H > 0 && V > 0, "embed: bad sizes T=%d H=%d V=%d", T, H, V);
+  const int piece = table_dtype == kBF16 ? 8 : 4;
+  if ((table_dtype == kF32 || table_dtype == kBF16) && V > 0 && H % piece == 0 && T <= 65535 && reinterpret_cast<uintptr_t>(table) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+    const dim3 grid((H / piece + 255) / 256, T);
+    if (table_dtype == kF32) embed_pieces_kernel<float><<<grid, 256, 0, s>>>(ids, static_cast<const float*>(table), x, H, V);
+    else embed_pieces_kernel<bf16_t><<<grid, 256, 0, s>>>(ids, static_cast<const bf16_t*>(table), x, H, V);
+    return launch_status("embed");
+  }
   if (table_dtype == kF32) embed_kernel<float><<<T, 256, 0, s>>>(ids, static_cast<const float*>(table), x, H, V);
   else if (table_dtype == kBF16) embed_kernel<bf16_t><<<T, 256, 0, s>>>(ids, static_cast<const bf16_t*>(table), x, H, V);
   else KVCM_REQUIRE(false, "embed: unknown table dtype %d", table_dtype);
