@@ -33,7 +33,7 @@ def kasuvik_spec(cfg: KasuvikConfig) -> ModelSpec:
         parts_ = {"norm_mixer": _norm(cfg, p + "norm1"), "mixer": mixer, "norm_mixer_out": _norm(cfg, p + "norm1b")}
         if layer.ff:
             parts_.update({"norm_ffn": _norm(cfg, p + "norm2"),
-                           "ffn": PartSpec("gated_mlp", {"intermediate_size": layer.ff, "activation": "relu"}, p + "mlp."),
+                           "ffn": PartSpec("gated_mlp", {"intermediate_size": layer.ff, "activation": "relu", "partial_out": True}, p + "mlp."),
                            "norm_ffn_out": _norm(cfg, p + "norm2b")})
         layers.append(LayerSpec(name=f"l{i}", block="sandwich_residual", parts=parts_))
     return ModelSpec(

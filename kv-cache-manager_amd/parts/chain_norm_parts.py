@@ -26,10 +26,10 @@ def pad_rows(t, multiple=16):
 
 def linear32(ctx, step, x, w, name, keep_partial=False):
     """x @ w^T as 32-bit rows for a consumer that computes in 32-bit: the product's 32-bit sums as they are, from this
-    package's kernels for few rows and from the vendor library's for many (``ops.gemm`` decides, as for every product);
+    package's kernels or, for many rows, from the vendor library's where that is the faster (``ops.gemm`` decides, as for every product);
     no path rounds the sums, so what enters a recurrence is as exact at one row as at thousands.  Products of up to 8 rows
-    run unsplit (gemm_rows8.hip), those of more rows split along K with a second launch that adds the slices up (unsplit the
-    shared-rows kernel was slower by more than that launch costs).  ``keep_partial``: the product may come
+    run unsplit (gemm_rows8.hip), those of more rows split along K with a second launch that adds the slices up where that is faster
+    than one slice.  ``keep_partial``: the product may come
     back as ops.PartialSums for a consumer that adds the slices itself.  The chained norm does: rows up to 8,192 wide
     stay in registers through all its stages, and the slices are added as they are loaded (5 us a launch at width 2048;
     the form that reads a row once per stage took 27 us with slices, more than the launch it saved).  Mixers' output

@@ -129,7 +129,7 @@ def test_products_with_a_folded_norm_in_tiles(ops):
 
 
 @pytest.mark.parametrize("M,N,K,mine", [(96, 2048, 2048, True), (200, 2560, 2048, True), (333, 2048, 5632, True), (700, 2048, 2048, True),
-                                        (1024, 2048, 2048, True), (1536, 8192, 2048, False), (2000, 192, 128, None)])
+                                        (1024, 2048, 2048, True), (1536, 8192, 2048, False), (2000, 192, 128, None), (768, 2048, 5632, None), (1000, 192, 8192, None)])
 def test_many_rows_go_to_the_tiles_where_the_rule_says_so(ops, M, N, K, mine):
     x, w = _operands(M, M, N, K)
     for dtype in (torch.bfloat16, torch.float32):
