@@ -211,13 +211,15 @@ static int rows_tiles_m(int M) { return M > kRowBlock ? kRowBlock / 16 : (M + 15
 // weights then), else four; as long as every slice has a trip of its own and the partial sums stay below
 // the weights' bytes; halved while more than eight waves a workgroup would be needed to get down to one
 // workgroup per CU.  Measured at 17 to 128 rows over the projections of TinyLlama and Llama-3-8B sizes,
-// alone and in whole decode steps.  (With the tiles free to choose among 1, 2, 4 and 8 as well, launches and the reading of the
+// alone and in whole decode steps.  Up to 16 rows the norm that follows is a workgroup a row, each reading all slices of its row: four
+// of 128 column tiles too (Kasuvik and Fisesun, eight requests, 34.61 -> 34.09 and 30.69 -> 30.30 ms a pass; at 64 rows of TinyLlama
+// sizes four were slower, 150.8 -> 152.0).  (With the tiles free to choose among 1, 2, 4 and 8 as well, launches and the reading of the
 // partial sums together would be 4 % shorter at 8 to 512 rows.)
 static int rows_splits(int M, int N, int K) {
   const long long tiles = static_cast<long long>(N / 16) * row_blocks(M);
   const int units = K / kUnit;
   if (tiles >= 4 * kRowsCUs) return 1;
-  int S = tiles <= 128 || (M > 48 && K >= 112 * M) ? 8 : 4;
+  int S = tiles <= (M <= 16 ? 64 : 128) || (M > 48 && K >= 112 * M) ? 8 : 4;
   const int trip = M <= 64 ? 4 : 2;   // units per trip (the launch's choice below)
   const int cap = units / trip < K / (2 * M) ? units / trip : K / (2 * M);
   while (S > 1 && S > cap) S >>= 1;

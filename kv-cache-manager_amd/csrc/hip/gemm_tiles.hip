@@ -2,7 +2,7 @@
 // 32-bit), left as partial sums of S slices of K ([S][M][N], the consumer adds them in slice order), or, SWIGLU, made into
 // act[M,I] = silu(X W_gate^T) * (X W_up^T), or with relu in silu's place, of a fused [gate (I rows) | up (I rows)] matrix.
 //
-// A workgroup of 3 to 12 waves owns a tile of BM rows x BN columns and a slice of K, its operands in a ring of stages in LDS
+// A workgroup of 2 to 12 waves owns a tile of BM rows x BN columns and a slice of K, its operands in a ring of stages in LDS
 // (tile_ring.h, which says what bounds such products and why the ring).
 //
 // Measured (us, weights from memory, one launch after the other in a graph; the kernel that shared only X through LDS and streamed
@@ -187,9 +187,12 @@ struct Tile {
   float fixed, step, share, round;
 };
 #define KVCM_TILES(T)                                                                                                             \
+  T(16, 32, 1, 2, 8, 1.305f, 0.144f, 0.725f, 0.000f)                                                                              \
   T(16, 48, 1, 3, 8, 1.278f, 0.167f, 0.771f, 0.466f)                                                                              \
   T(16, 64, 1, 4, 8, 1.126f, 0.199f, 0.886f, 0.256f)                                                                              \
+  T(32, 32, 2, 2, 8, 1.517f, 0.163f, 0.801f, 0.197f)                                                                              \
   T(32, 64, 2, 2, 6, 1.484f, 0.219f, 0.891f, 0.210f)                                                                              \
+  T(64, 32, 2, 2, 6, 1.770f, 0.196f, 0.899f, 0.000f)                                                                              \
   T(64, 48, 4, 1, 8, 2.019f, 0.236f, 0.975f, 1.170f)                                                                              \
   T(64, 64, 2, 2, 4, 1.822f, 0.274f, 0.869f, 0.435f)                                                                              \
   T(64, 96, 2, 3, 6, 2.462f, 0.351f, 0.957f, 1.524f)                                                                              \

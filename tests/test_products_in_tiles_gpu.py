@@ -54,10 +54,10 @@ def _run(ops, x, w, partials, out, S=1, gated=0, act=0, limit=0.0, tile=-1, N=No
     assert rc == 0, ops.lib().kvcm_hip_last_error().decode()
 
 
-@pytest.mark.parametrize("tile", range(14))
+@pytest.mark.parametrize("tile", range(17))
 def test_every_tile_at_its_edges(ops, tile):
     sizes = _tiles(ops)
-    assert len(sizes) == 14
+    assert len(sizes) == 17
     bm, bn = sizes[tile]
     seed = 0
     # rows and columns around one tile and around several; k of one step (shorter than any ring), of few, of more than a ring
@@ -81,7 +81,7 @@ def test_every_tile_at_its_edges(ops, tile):
             assert torch.isnan(left).all(), "written beside the result"
 
 
-@pytest.mark.parametrize("tile", range(14))
+@pytest.mark.parametrize("tile", range(17))
 def test_every_tile_gated(ops, tile):
     bm, bn = _tiles(ops)[tile]
     for seed, (M, I, K) in enumerate([(1, 8, 64), (bm + 1, bn // 2, 448), (bm - 1, bn + 8, 640), (2 * bm + 3, 2 * bn + 40, 192)]):
