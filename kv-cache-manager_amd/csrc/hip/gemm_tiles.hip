@@ -304,7 +304,7 @@ int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, in
 }
 
 // Is a product of many rows, in S slices of K that its consumer adds, faster here than by the vendor library (is_gated: than that and
-// the launch that applies SwiGLU)?  Up to 256 rows it was at all 38 shapes measured (0.43 to 0.87 of the time), beyond 2,048 the
+// the launch that applies SwiGLU)?  Up to 256 rows it was at 39 of 41 shapes measured (0.43 to 0.87 of the time, two 1.01), beyond 2,048 the
 // library's own tiles of 256 x 256 are (32,768 rows: 1,306 / 1,269 us gate+up of 5632 x 2048, 659 / 513 us 2048 x 5632).  In between, the
 // tiles' time and the slices' reading against about what the library takes: 14 us and 1,350 TFLOP/s (22 us and 1,600 for the largest),
 // and at least 0.3 us for 64 k of a chain that it does not cut.  The six constants were fitted to 76 shapes; what the rule picks is 1.1 %
