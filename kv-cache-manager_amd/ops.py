@@ -581,6 +581,11 @@ def skinny_splits(M, N, K):
     return lib().kvcm_gemm_skinny_splits(M, N, K)
 
 
+def _in_pieces(*operands):
+    """Do the operands' rows begin at 16-byte pieces, not so far apart that a tile's offsets pass 32 bits?  (Others take the general kernel.)"""
+    return all(t.stride(0) % 8 == 0 and t.stride(0) < 1 << 22 and t.data_ptr() % 16 == 0 for t in operands)
+
+
 def _usable_splits(M, N, K, scratch, keep_partial):
     """Slices of K that a product of M rows is cut into: where nobody takes the partial sums, none if that is the faster whole, and as
     many as ``scratch`` has room for (0: the kernels of few rows do not take the shape)."""
@@ -650,7 +655,7 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
         _call("kvcm_gemm_f32", _ptr(x), _ptr(w), _ptr(out), M, N, K, x.stride(0), w.stride(0), out.stride(0), _stream())
         return out
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm operands must both be bfloat16")
-    aligned = x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    aligned = _in_pieces(x, w)
     library = _library_takes(M, N, K)
     mode = _TUNING_MODES[LIBRARY_TUNING if tuning is None else tuning]
     if library and mode == 0 and aligned and K % 64 == 0 and N % 64 == 0:
@@ -736,7 +741,7 @@ def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0):
     M, K = x.shape
     I = out.shape[1]
     _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_gated shapes do not agree")
-    if (I % 32 or K % 64 or x.stride(0) % 8 or w_gate_up.stride(0) % 8 or x.data_ptr() % 16 or w_gate_up.data_ptr() % 16
+    if (I % 32 or K % 64 or not _in_pieces(x, w_gate_up)
             or not (_tiles_take(M, I, K, 1, gated=True) if many_rows(M) else _gated_tiles_take(M, I, K))):
         return False
     _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0), out.stride(0), 1,
@@ -771,8 +776,7 @@ def gemm_swiglu(x, w_gate_up, out, limit=0.0):
     M, K = x.shape
     I = out.shape[1]
     _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_swiglu shapes do not agree")
-    aligned = (x.dtype == w_gate_up.dtype == out.dtype == torch.bfloat16 and x.stride(0) % 8 == 0
-               and w_gate_up.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0)
+    aligned = x.dtype == w_gate_up.dtype == out.dtype == torch.bfloat16 and _in_pieces(x, w_gate_up)
     if many_rows(M):
         # many rows: the library product, then swiglu, unless the tiles are the faster
         if not (aligned and _tiles_take(M, I, K, 1, gated=True)):
