@@ -282,14 +282,14 @@ int kvcm_moe_up(const void* h, int dtype, int ldh, const void* w_up, const int* 
   KVCM_REQUIRE(T > 0 && K > 0 && F > 0 && top > 0 && E > 0 && ldh >= K, "moe_up: bad sizes");
   KVCM_REQUIRE(kind >= 0 && kind <= 2, "moe_up: unknown kind of experts %d (0 relu2, 1 silu gated, 2 gelu)", kind);
   KVCM_REQUIRE(kind != 1 || F % 16 == 0, "moe_up: gated experts of %d columns are not supported (a multiple of 16)", F);
-  KVCM_REQUIRE(static_cast<long long>(T) * top < (1ll << 31) && (F + 3) / 4 <= 65535, "moe_up: too many rows or columns");
-  KVCM_REQUIRE(K * sizeof(float) <= 64 * 1024, "moe_up: rows of %d values do not fit the local memory", K);
   KVCM_REQUIRE(reinterpret_cast<uintptr_t>(w_up) % 16 == 0, "moe_up: weights must be 16-byte aligned");
   KVCM_REQUIRE(dtype == kF32 || dtype == kBF16, "moe_up: unknown dtype %d", dtype);
-  if (moe_few_up_takes(dtype, h, ldh, T, K, F, top)) {
+  if (moe_few_up_takes(dtype, h, ldh, T, K, F, top)) {      // (keeps no row in LDS: any width)
     launch_moe_few_up(h, ldh, w_up, chosen, act, T, K, F, top, E, kind, in_weight, s);
     return launch_status("moe_up");
   }
+  KVCM_REQUIRE(static_cast<long long>(T) * top < (1ll << 31) && (F + 3) / 4 <= 65535, "moe_up: too many rows or columns");
+  KVCM_REQUIRE(K * sizeof(float) <= 64 * 1024, "moe_up: rows of %d values do not fit the local memory", K);
   const int cw = moe_cols_per_wave(static_cast<long long>(T) * top, F);
   const dim3 grid(T * top, (F + 4 * cw - 1) / (4 * cw));
   const size_t lds = K * sizeof(float);
@@ -307,15 +307,15 @@ int kvcm_moe_down(const void* act, int dtype, const void* w_down, const int* cho
                   float* out, int T, int F, int H, int top, int E, hipStream_t s) {
   if (T == 0) return 0;
   KVCM_REQUIRE(T > 0 && H > 0 && F > 0 && top > 0 && E > 0, "moe_down: bad sizes");
-  const size_t lds = static_cast<size_t>(top) * ((F + 3) & ~3) * sizeof(float);
-  KVCM_REQUIRE(lds <= 64 * 1024, "moe_down: %d activations of %d values do not fit the local memory", top, F);
   KVCM_REQUIRE(reinterpret_cast<uintptr_t>(w_down) % 16 == 0, "moe_down: weights must be 16-byte aligned");
-  KVCM_REQUIRE((H + 3) / 4 <= 65535, "moe_down: too many columns");
   KVCM_REQUIRE(dtype == kF32 || dtype == kBF16, "moe_down: unknown dtype %d", dtype);
-  if (moe_few_down_takes(dtype, act, T, F, H, top, E)) {
+  if (moe_few_down_takes(dtype, act, T, F, H, top, E)) {      // (keeps no activations in LDS: any width)
     launch_moe_few_down(act, w_down, chosen, weight, add, out, T, F, H, top, E, s);
     return launch_status("moe_down");
   }
+  const size_t lds = static_cast<size_t>(top) * ((F + 3) & ~3) * sizeof(float);
+  KVCM_REQUIRE(lds <= 64 * 1024, "moe_down: %d activations of %d values do not fit the local memory", top, F);
+  KVCM_REQUIRE((H + 3) / 4 <= 65535, "moe_down: too many columns");
   const int cw = moe_cols_per_wave(T, H);
   const dim3 grid(T, (H + 4 * cw - 1) / (4 * cw));
 #define KVCM_MOE_DOWN(TT, CW)                                                                                                \

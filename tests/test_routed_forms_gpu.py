@@ -93,7 +93,9 @@ def test_grouped_tiles(shape, weigh_input):
 # ("one"), an expert named twice by a row, and numbers that name none
 FEW = [(3, 8, 2, 64, 64, 8, "silu", None), (15, 8, 2, 448, 192, 136, "relu2", None), (20, 3, 3, 128, 128, 64, "gelu", None),
        (32, 4, 2, 320, 64, 72, "silu", "one"), (9, 40, 7, 192, 96, 24, "relu2", None), (10, 6, 2, 128, 320, 16, "silu", "odd"),
-       (17, 5, 1, 64, 448, 40, "gelu", "one"), (64, 8, 1, 576, 64, 8, "silu", None)]
+       (17, 5, 1, 64, 448, 40, "gelu", "one"), (64, 8, 1, 576, 64, 8, "silu", None),
+       # activations of a row, and rows, that a workgroup's LDS would not hold
+       (16, 3, 2, 64, 8256, 8, "silu", None), (16, 2, 1, 16448, 64, 8, "relu2", None)]
 
 
 @pytest.mark.parametrize("weigh_input", [False, True])
@@ -109,3 +111,29 @@ def test_few_rows(shape, weigh_input):
         chosen[2] = 4
         chosen[5, 0], chosen[7] = -1, E
     _check("few", _case(T, E, top, K, F, H, kind, T + K, chosen), kind, weigh_input, not weigh_input)
+
+
+@pytest.mark.parametrize("T,top,H,F", [(16, 2, 64, 8256), (32, 2, 64, 8256), (20, 1, 16448, 64)])
+def test_layers_wider_than_a_workgroups_local_memory(T, top, H, F):
+    """the layer takes rows and activations of any width from 16 rows on, by whichever kernels"""
+    from kvcm_amd import ops
+    from kvcm_amd.parts.base import BuildContext
+    from kvcm_amd.parts.routed_parts import RoutedExperts
+    E = 3
+    h, _, up, down, chosen, _, _ = case = _case(T, E, top, H, F, H, "relu2", T + F)
+    part = RoutedExperts({"experts": E, "top": top, "ff": F, "routing": "table", "vocab_size": T}, "",
+                         BuildContext(torch.bfloat16, torch.device(DEV), H, 16, ops))
+    part.bind({"table": chosen.to(DEV), "w_up": up.view(E * F, H).to(DEV), "w_down": down.view(E * H, F).to(DEV)})
+
+    class Step:
+        rows, limits, tune_products, tokens = T, None, None, torch.arange(T, dtype=torch.int32, device=DEV)
+
+        def ws(self, name, shape, dtype=torch.bfloat16):
+            return torch.empty(shape, dtype=dtype, device=DEV)
+
+        def flat(self, name, numel, dtype=torch.float32):
+            return torch.empty(numel, dtype=dtype, device=DEV)
+
+    got = part.forward(Step(), h.to(DEV)).cpu().double()
+    want, bound = _want((*case[:5], torch.full((T, top), 1.0 / top), case[6]), "relu2", False, False)
+    assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
