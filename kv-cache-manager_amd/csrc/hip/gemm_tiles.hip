@@ -34,7 +34,8 @@ __device__ __forceinline__ float gated(float gate, float up, float limit, int ac
 // neighbouring tiles then hold gate and up), else eight and eight (lanes 32 apart then do, and swap halves).
 // ss_in (GATED): X = round(g round(x)) of a norm folded into this product (gemm_rows8.hip): the sums are scaled by the rows'
 // rsqrt(mean x^2 + eps), from tiles_in sums of squares a row.
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED>
+// Offset: of an operand's pieces from its tile's beginning, in bytes; uint64_t for rows that are far apart.
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, class Offset>
 __global__ void __launch_bounds__(WM* WN* kWave)
     gemm_tiles_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, float* __restrict__ partials, void* __restrict__ out,
                       int out_f32, int M, int N, int K, int ldx, int ldw, int ldo, int S, int tiles_m, int tiles_n,
@@ -58,7 +59,7 @@ __global__ void __launch_bounds__(WM* WN* kWave)
   const uint64_t wbase = reinterpret_cast<uint64_t>(W + static_cast<size_t>(c0) * ldw) + static_cast<size_t>(k_lo) * 128;
   const uint64_t upbase = wbase + static_cast<size_t>(GATED ? N : 0) * ldw * 2;
   // rows past M and columns past N repeat the last one (what they give is not stored)
-  uint32_t offset[R];
+  Offset offset[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int req = Ring::request_of(q, wave), row = req * 8 + lane / 8;
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(WM* WN* kWave)
       if (at > N - 1 - c0) at = N - 1 - c0;
       ld = ldw;
     }
-    offset[q] = static_cast<uint32_t>(at) * static_cast<uint32_t>(ld) * 2u + static_cast<uint32_t>(Ring::piece_of(lane)) * 16u;
+    offset[q] = static_cast<Offset>(at) * static_cast<Offset>(ld) * 2u + static_cast<Offset>(Ring::piece_of(lane)) * 16u;
   }
   // One row block: workgroups walk their slice from different places (and wrap around), or all would ask the same few memory
   // channels for rows a multiple of 4 KB apart at the same time (gate+up, 64 rows: 14.9 -> 14.4 us).  Several: those that share
@@ -249,12 +250,12 @@ float gemm_tiles_time(int M, int N, int K, int S, bool is_gated, bool out_f32) {
   return t + static_cast<float>(M) * static_cast<float>(N) * (S > 1 ? 4.f * S : out_f32 ? 4.f : 2.f) * 0.12e-6f;      // what is stored
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED>
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, class Offset = uint32_t>
 static int launch_tiles(const TilesCall& c, hipStream_t st) {
   const int tiles_m = (c.M + BM - 1) / BM, tiles_n = ((GATED ? 2 * c.N : c.N) + BN - 1) / BN;
   const long long grid = static_cast<long long>(tiles_m) * tiles_n * c.S;
   KVCM_REQUIRE(grid < (1ll << 31), "gemm_tiles: too many tiles");
-  gemm_tiles_kernel<BM, BN, WM, WN, STAGES, GATED><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, st>>>(
+  gemm_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, Offset><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, st>>>(
       c.X, c.W, c.partials, c.out, c.out_f32, c.M, c.N, c.K, c.ldx, c.ldw, c.ldo, c.S, tiles_m, tiles_n, c.ss_in, c.tiles_in, c.eps, c.limit,
       c.act);
   return launch_status("gemm_tiles");
@@ -264,7 +265,9 @@ int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st) {
   KVCM_REQUIRE(c.M > 0 && c.N > 0 && c.N % 4 == 0 && c.K > 0 && c.K % kStepK == 0 && c.S >= 1 && c.S <= c.K / kStepK,
                "gemm_tiles: unsupported shape M=%d N=%d K=%d in %d slices", c.M, c.N, c.K, c.S);
   KVCM_REQUIRE(!is_gated || (c.N % 8 == 0 && c.S == 1), "gemm_tiles: gated products take widths of multiples of 8 and are unsplit");
-  KVCM_REQUIRE(c.ldx < (1 << 22) && c.ldw < (1 << 22), "gemm_tiles: rows too far apart");      // a tile's offsets are 32-bit
+  // (rows of 8 MB or that far apart: one tile for all sizes; what such a product takes is its bytes)
+  if (c.ldx >= kFarRows || c.ldw >= kFarRows)
+    return is_gated ? launch_tiles<64, 64, 2, 2, 4, true, uint64_t>(c, st) : launch_tiles<64, 64, 2, 2, 4, false, uint64_t>(c, st);
   if (tile < 0) tile = best_tile(c.M, is_gated ? 2 * c.N : c.N, c.K, c.S);
   int i = 0;
 #define KVCM_TILE_LAUNCH(BM, BN, WM, WN, STAGES, FIXED, STEP, SHARE, ROUND)                                                        \

@@ -47,6 +47,14 @@ __device__ __forceinline__ void ring_bring16(uint32_t offset, uint64_t base, uin
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base) : "memory", "m0");
 }
 
+// The same where offsets do not fit 32 bits: every lane has an address of its own.
+__device__ __forceinline__ void ring_bring16(uint64_t offset, uint64_t base, uint32_t to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(base + offset) : "memory", "m0");
+}
+
+// Rows this many elements apart or more need offsets of 64 bits: a tile has up to 256 of them.
+constexpr int kFarRows = 1 << 22;
+
 // Workgroups go to the eight XCDs in turn: each XCD takes a contiguous stretch of the numbers, so that neighbours, which read the
 // same rows of W, meet in one L2.
 __device__ __forceinline__ int neighbours_on_one_xcd() {
@@ -69,12 +77,12 @@ struct TileRing {
   // Lane l of a request brings, of row l / 8, the piece (of eight elements) that belongs at place l % 8.
   static __device__ __forceinline__ int piece_of(int lane) { return (lane % 8) ^ (lane / 8); }
 
-  // acc += X W^T over `steps` steps of k.  offset[q]: bytes from base(request) to the lane's piece at the first k; base: the same
-  // for the whole wave; the steps are walked from step `phase` on and wrap around.  left < 64 (with phase 0): the last step has that many
+  // acc += X W^T over `steps` steps of k.  offset[q] (uint32_t, or uint64_t for far rows): bytes from base(request) to the lane's piece
+  // at the first k; base: the same for the whole wave; the steps are walked from step `phase` on and wrap around.  left < 64 (with phase 0): the last step has that many
   // k (a multiple of 8), the lanes whose pieces lie beyond bring the row's first piece of the step, which is not multiplied.
   // between: done once while the first stages are on their way.  works: this wave has rows (else it only brings operands).
-  template <class Base, class Between>
-  static __device__ __forceinline__ void multiply(unsigned char* ring, const uint32_t (&offset)[R], Base base, int steps, int phase, int left,
+  template <class Offset, class Base, class Between>
+  static __device__ __forceinline__ void multiply(unsigned char* ring, const Offset (&offset)[R], Base base, int steps, int phase, int left,
                                                   int wave, int lane, ring_f32x4 (&acc)[TN][TM], Between between, bool works = true) {
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
         reinterpret_cast<uintptr_t>(reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(ring)))));

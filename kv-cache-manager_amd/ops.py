@@ -582,8 +582,13 @@ def skinny_splits(M, N, K):
 
 
 def _in_pieces(*operands):
-    """Do the operands' rows begin at 16-byte pieces, not so far apart that a tile's offsets pass 32 bits?  (Others take the general kernel.)"""
-    return all(t.stride(0) % 8 == 0 and t.stride(0) < 1 << 22 and t.data_ptr() % 16 == 0 for t in operands)
+    """Do the operands' rows begin at 16-byte pieces?  (Others take the general kernel.)"""
+    return all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in operands)
+
+
+def _near(*operands):
+    """Are the operands' rows near enough for a tile's 32-bit offsets (csrc/hip/tile_ring.h)?  The form for others is no rival of the vendor library's."""
+    return all(t.stride(0) < 1 << 22 for t in operands)
 
 
 def _usable_splits(M, N, K, scratch, keep_partial):
@@ -658,7 +663,7 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
     aligned = _in_pieces(x, w)
     library = _library_takes(M, N, K)
     mode = _TUNING_MODES[LIBRARY_TUNING if tuning is None else tuning]
-    if library and mode == 0 and aligned and K % 64 == 0 and N % 64 == 0:
+    if library and mode == 0 and aligned and _near(x, w) and K % 64 == 0 and N % 64 == 0:
         # (who asks for the library's tuned algorithms gets them)
         S = _usable_splits(M, N, K, scratch, keep_partial) if M <= 512 else 1
         library = not _tiles_take(M, N, K, S, dtype=out.dtype)
@@ -741,7 +746,7 @@ def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0):
     M, K = x.shape
     I = out.shape[1]
     _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_gated shapes do not agree")
-    if (I % 32 or K % 64 or not _in_pieces(x, w_gate_up)
+    if (I % 32 or K % 64 or not _in_pieces(x, w_gate_up) or not _near(x, w_gate_up)
             or not (_tiles_take(M, I, K, 1, gated=True) if many_rows(M) else _gated_tiles_take(M, I, K))):
         return False
     _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0), out.stride(0), 1,
@@ -779,7 +784,7 @@ def gemm_swiglu(x, w_gate_up, out, limit=0.0):
     aligned = x.dtype == w_gate_up.dtype == out.dtype == torch.bfloat16 and _in_pieces(x, w_gate_up)
     if many_rows(M):
         # many rows: the library product, then swiglu, unless the tiles are the faster
-        if not (aligned and _tiles_take(M, I, K, 1, gated=True)):
+        if not (aligned and _near(x, w_gate_up) and _tiles_take(M, I, K, 1, gated=True)):
             return False
         _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0),
               out.stride(0), 1, 1, 0, float(limit), -1, _stream())

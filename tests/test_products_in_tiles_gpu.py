@@ -128,6 +128,50 @@ def test_products_with_a_folded_norm_in_tiles(ops):
     assert bool(((out.double() - want).abs() <= 4.2 * 2.0 ** -8 * (g.abs() * u.abs()) + 1e-5).all())
 
 
+def _apart(t, ld):
+    """the same rows, ld elements apart"""
+    room = torch.empty((t.shape[0] - 1) * ld + t.shape[1], dtype=t.dtype, device=t.device)
+    out = room.as_strided(t.shape, (ld, 1))
+    out.copy_(t)
+    return out
+
+
+# ld: the first that a tile's 32-bit offsets are not meant for; rows so far apart that offsets inside a tile pass 32 bits
+@pytest.mark.parametrize("M,N,K,ld", [(5, 64, 128, 1 << 22), (40, 128, 256, 1 << 22), (40, 64, 640, 1 << 26), (200, 64, 128, 1 << 22)])
+def test_rows_far_apart(ops, M, N, K, ld):
+    lib, x, w = ops.lib(), *_operands(M + N, M, N, K)
+    for far_x, far_w in ((_apart(x, ld), w), (x, _apart(w, ld)), (_apart(x, ld), _apart(w, ld))):
+        ends = (far_x.data_ptr(), far_w.data_ptr()), (M, N, K, far_x.stride(0), far_w.stride(0), N)
+        S = min(2, K // 64)
+        parts, out = torch.empty(S, M, N, device=DEV), torch.full((M, N), float("nan"), device=DEV)
+        assert lib.kvcm_gemm_skinny(*ends[0], parts.data_ptr(), 0, ops._DT[torch.float32], *ends[1], S, ops._stream()) == 0, lib.kvcm_hip_last_error()
+        _close(parts.double().sum(0), x, w, False)
+        assert lib.kvcm_gemm_skinny(*ends[0], 0, out.data_ptr(), ops._DT[torch.float32], *ends[1], 1, ops._stream()) == 0, lib.kvcm_hip_last_error()
+        _close(out, x, w, False)
+        if M < ops.LIBRARY_GEMM_MIN_ROWS:
+            _close(ops.gemm(far_x, far_w, out.fill_(float("nan"))), x, w, False)
+
+
+@pytest.mark.parametrize("M,I,K", [(40, 5120, 64), (3, 8192, 128)])
+def test_gated_products_of_rows_far_apart(ops, M, I, K):
+    x, w = _operands(M + I, M, 2 * I, K)
+    far, out = _apart(x, 1 << 22), torch.empty(M, I, dtype=torch.bfloat16, device=DEV)
+    ss = torch.rand(M, K // 8, device=DEV) * 8
+    g, u = (x.double() @ w.double().t()).split(I, 1)
+    rstd = 1.0 / torch.sqrt(ss.double().sum(1, keepdim=True) / K + 1e-5)
+    at, to = (far.data_ptr(), w.data_ptr()), (M, I, K, far.stride(0), K, I)
+    for scale in (1.0, rstd):
+        out.fill_(float("nan"))
+        if scale is rstd:
+            rc = ops.lib().kvcm_gemm_skinny_swiglu_normed(*at, ss.data_ptr(), K // 8, 1e-5, out.data_ptr(), *to, ops._stream())
+        else:
+            rc = ops.lib().kvcm_gemm_skinny_swiglu(*at, out.data_ptr(), ops._DT[torch.bfloat16], *to, 0.0, ops._stream())
+        assert rc == 0, ops.lib().kvcm_hip_last_error()
+        want = g * scale * torch.sigmoid(g * scale) * u * scale
+        # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each
+        assert bool(((out.double() - want).abs() <= 4.2 * 2.0 ** -8 * (g * scale).abs() * (u * scale).abs() + 1e-5).all())
+
+
 @pytest.mark.parametrize("M,N,K,mine", [(96, 2048, 2048, True), (200, 2560, 2048, True), (333, 2048, 5632, True), (700, 2048, 2048, True),
                                         (1024, 2048, 2048, True), (1536, 8192, 2048, False), (2000, 192, 128, None), (768, 2048, 5632, None), (1000, 192, 8192, None)])
 def test_many_rows_go_to_the_tiles_where_the_rule_says_so(ops, M, N, K, mine):

@@ -112,3 +112,17 @@ def test_products_beyond_the_built_in_array_are_refused(ops, clib):
     # shapes the kernel does not take at all are refused the same way
     rc, _ = _noalloc(clib, *_operands(6, 4, 40, 64), torch.bfloat16)
     assert rc != 0 and "unsupported shape" in clib.kvcm_hip_last_error().decode()
+
+
+def test_rows_far_apart(ops, clib):
+    """rows 2^22 elements apart, on one side and on both, split and unsplit"""
+    for M, N, K in ((40, 128, 512), (17, 64, 64)):
+        x, w = _operands(M, M, N, K)
+        rc, want = _noalloc(clib, x, w, torch.float32)
+        assert rc == 0, clib.kvcm_hip_last_error().decode()
+        far = [torch.empty((t.shape[0] - 1 << 22) + K, dtype=t.dtype, device=DEV).as_strided(t.shape, (1 << 22, 1)).copy_(t) for t in (x, w)]
+        for a, b in ((far[0], w), (x, far[1]), far):
+            rc, got = _noalloc(clib, a, b, torch.float32)
+            assert rc == 0, clib.kvcm_hip_last_error().decode()
+            # 32-bit sums of the same terms in another order
+            assert bool(((got - want).abs() <= 2 * K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())).all())
