@@ -74,8 +74,9 @@ __global__ void __launch_bounds__(1024)
 
 enum : int { kDown = 0, kUp = 1, kUpGated = 2, kUpGelu = 3 };
 
-// N: rows of an expert's matrix (2F for the gated form); the output has N columns (F for the gated form)
-template <int BM, int BN, int WM, int WN, int STAGES, int MODE>
+// N: rows of an expert's matrix (2F for the gated form); the output has N columns (F for the gated form).  Offset: of an operand's
+// pieces from its beginning, in bytes; uint64_t for rows that lie beyond 4 GB or far apart.
+template <int BM, int BN, int WM, int WN, int STAGES, int MODE, class Offset>
 __global__ void __launch_bounds__(WM* WN* kWave)
     moe_grouped_kernel(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ W, const int* __restrict__ order,
                        const int* __restrict__ count, const int4* __restrict__ list, int top, void* __restrict__ out,
@@ -98,14 +99,14 @@ __global__ void __launch_bounds__(WM* WN* kWave)
   const uint64_t abase = reinterpret_cast<uint64_t>(A + (MODE == kDown ? static_cast<size_t>(p0) * lda : 0));
   const uint64_t wbase = reinterpret_cast<uint64_t>(W + (static_cast<size_t>(e) * N + n0) * K);
   // rows past the tile and columns past N repeat the last one (what they give is not stored)
-  uint32_t offset[R];
+  Offset offset[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int req = Ring::request_of(q, wave), row = req * 8 + lane / 8;
     const int r = row < rows ? row : rows - 1, c = row - BM < N - n0 ? row - BM : N - 1 - n0;
     const uint32_t from = MODE != kDown ? static_cast<uint32_t>(order[p0 + (req < BM / 8 ? r : 0)]) / static_cast<uint32_t>(top) : static_cast<uint32_t>(r);
-    offset[q] = (req < BM / 8 ? from * static_cast<uint32_t>(lda) : static_cast<uint32_t>(c) * static_cast<uint32_t>(K)) * 2u +
-                static_cast<uint32_t>(Ring::piece_of(lane)) * 16u;
+    offset[q] = (req < BM / 8 ? static_cast<Offset>(from) * static_cast<Offset>(lda) : static_cast<Offset>(c) * static_cast<Offset>(K)) * 2u +
+                static_cast<Offset>(Ring::piece_of(lane)) * 16u;
   }
   int pair[TM];      // of this lane's rows
 #pragma unroll
@@ -200,6 +201,8 @@ struct High {
 static constexpr High kHighs[] = {KVCM_GROUPED_TILES(KVCM_HIGH)};
 #undef KVCM_HIGH
 constexpr int kHighCount = sizeof(kHighs) / sizeof(kHighs[0]);
+constexpr int kFarTile = 2;      // the one that is there with 64-bit offsets too
+static_assert(kHighs[kFarTile].bm == 128 && kHighs[kFarTile].bn == 128, "launch_grouped names it");
 
 // The tile for n pairs over E experts, N rows of K each: groups of pairs end in a tile that is half empty on average.
 static int best_grouped(int n, int E, int N, int K) {
@@ -227,6 +230,7 @@ struct GroupedCall {
   void* out;
   const float* weight;
   int N, K, n, E;
+  bool far;      // operands need offsets of 64 bits (the tile is kFarTile)
 };
 
 template <int MODE>
@@ -234,14 +238,20 @@ static int launch_grouped(int tile, const GroupedCall& c, hipStream_t s) {
   const int col_blocks = (c.N + kHighs[tile].bn - 1) / kHighs[tile].bn;
   const long long grid = (static_cast<long long>(c.n / kHighs[tile].bm + c.E) * col_blocks + 7) / 8 * 8;
   KVCM_REQUIRE(grid < (1ll << 31), "moe_grouped: too many tiles");
+#define KVCM_GROUPED(BM, BN, WM, WN, STAGES, OFFSET)                                                                                   \
+  moe_grouped_kernel<BM, BN, WM, WN, STAGES, MODE, OFFSET><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, s>>>(                    \
+      static_cast<const uint16_t*>(c.A), c.lda, static_cast<const uint16_t*>(c.W), c.order, c.count, c.list, c.top, c.out, c.weight,   \
+      c.N, c.K, col_blocks)
+  if (c.far) {
+    KVCM_GROUPED(128, 128, 2, 4, 4, uint64_t);
+    return launch_status("moe_grouped");
+  }
   int i = 0;
-#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES)                                                                                    \
-  if (tile == i++)                                                                                                                     \
-    moe_grouped_kernel<BM, BN, WM, WN, STAGES, MODE><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, s>>>(                          \
-        static_cast<const uint16_t*>(c.A), c.lda, static_cast<const uint16_t*>(c.W), c.order, c.count, c.list, c.top, c.out, c.weight, \
-        c.N, c.K, col_blocks);
+#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES) \
+  if (tile == i++) KVCM_GROUPED(BM, BN, WM, WN, STAGES, uint32_t);
   KVCM_GROUPED_TILES(KVCM_GROUPED_LAUNCH)
 #undef KVCM_GROUPED_LAUNCH
+#undef KVCM_GROUPED
   return launch_status("moe_grouped");
 }
 
@@ -270,7 +280,6 @@ int kvcm_moe_grouped(const void* h, int ldh, const void* w_up, const void* w_dow
   KVCM_REQUIRE(T > 0 && top > 0 && H > 0 && ldh >= K, "moe_grouped: bad sizes");
   KVCM_REQUIRE(kvcm_moe_grouped_supported(K, F, E), "moe_grouped: sizes K=%d F=%d experts=%d are not supported", K, F, E);
   KVCM_REQUIRE(static_cast<long long>(T) * top < (1ll << 30), "moe_grouped: too many rows");
-  KVCM_REQUIRE(static_cast<long long>(T) * ldh < (1ll << 31) && K < (1 << 22) && F < (1 << 22), "moe_grouped: more than 4 GB of rows");
   KVCM_REQUIRE(ldh % 8 == 0 && reinterpret_cast<uintptr_t>(h) % 16 == 0 && reinterpret_cast<uintptr_t>(w_up) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(w_down) % 16 == 0 && reinterpret_cast<uintptr_t>(act) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(lists) % 16 == 0,
@@ -279,14 +288,15 @@ int kvcm_moe_grouped(const void* h, int ldh, const void* w_up, const void* w_dow
   KVCM_REQUIRE(kind != 1 || F % 16 == 0, "moe_grouped: gated experts of %d columns are not supported (a multiple of 16)", F);
   KVCM_REQUIRE(tile_up < kHighCount && tile_down < kHighCount, "moe_grouped: no such tile");
   const int n = T * top, up_rows = kind == 1 ? 2 * F : F;
-  if (tile_up < 0) tile_up = best_grouped(n, E, up_rows, K);
-  if (tile_down < 0) tile_down = best_grouped(n, E, H, F);
+  const bool far_up = static_cast<long long>(T) * ldh >= (1ll << 31) || K >= kFarRows, far_down = F >= kFarRows;
+  tile_up = far_up ? kFarTile : tile_up < 0 ? best_grouped(n, E, up_rows, K) : tile_up;
+  tile_down = far_down ? kFarTile : tile_down < 0 ? best_grouped(n, E, H, F) : tile_down;
   moe_group_kernel<<<1, 1024, 4 * E * sizeof(int), s>>>(chosen, n, E, order, lists, kHighs[tile_up].bm, kHighs[tile_down].bm);
   const int4* list = reinterpret_cast<const int4*>(lists + 4);
-  const GroupedCall up{h, ldh, w_up, order, lists, list, top, act, weigh_input ? weight : nullptr, up_rows, K, n, E};
+  const GroupedCall up{h, ldh, w_up, order, lists, list, top, act, weigh_input ? weight : nullptr, up_rows, K, n, E, far_up};
   int rc = kind == 1 ? launch_grouped<kUpGated>(tile_up, up, s) : kind == 2 ? launch_grouped<kUpGelu>(tile_up, up, s) : launch_grouped<kUp>(tile_up, up, s);
   if (rc) return rc;
-  const GroupedCall down{act, F, w_down, order, lists + 1, list + most_tiles(n, E), top, y, weigh_input ? nullptr : weight, H, F, n, E};
+  const GroupedCall down{act, F, w_down, order, lists + 1, list + most_tiles(n, E), top, y, weigh_input ? nullptr : weight, H, F, n, E, far_down};
   rc = launch_grouped<kDown>(tile_down, down, s);
   if (rc) return rc;
   // four columns a thread where rows are whole 16-byte pieces (2,048 rows of 2,048 columns, two experts each: 20 us a column at a

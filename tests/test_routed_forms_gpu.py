@@ -40,7 +40,7 @@ def _want(case, kind, weigh_input, add):
     return want, bound + 1e-5
 
 
-def _run(form, case, kind, weigh_input, add):
+def _run(form, case, kind, weigh_input, add, ld=None):
     from kvcm_amd import ops
     from kvcm_amd.parts.routed_parts import interleave_gate_up
     h, gate, up, down, chosen, weight, base = (t.to(DEV) if t is not None else None for t in case)
@@ -49,7 +49,10 @@ def _run(form, case, kind, weigh_input, add):
     H, top = down.shape[1], chosen.shape[1]
     if kind == "silu":
         up = interleave_gate_up(gate, up)
-    wide = torch.full((T, K + 24), float("nan"), dtype=torch.bfloat16, device=DEV)      # rows apart: what lies between is not read
+    if ld is None:
+        wide = torch.full((T, K + 24), float("nan"), dtype=torch.bfloat16, device=DEV)      # rows apart: what lies between is not read
+    else:
+        wide = torch.empty((T - 1) * ld + K, dtype=torch.bfloat16, device=DEV).as_strided((T, K), (ld, 1))
     wide[:, :K] = h
     act = torch.empty(T * top, F, dtype=torch.bfloat16, device=DEV)
     out = torch.full((T, H), float("nan"), device=DEV)
@@ -87,6 +90,17 @@ def test_grouped_tiles(shape, weigh_input):
     T, E, top, K, F, H, kind, one = shape
     chosen = torch.zeros(T, top, dtype=torch.long) if one else None
     _check("grouped", _case(T, E, top, K, F, H, kind, T + K, chosen), kind, weigh_input, not weigh_input)
+
+
+# rows that lie beyond 4 GB, rows of the experts' matrices and of activations that are 8 MB apart
+@pytest.mark.parametrize("shape,ld", [((40, 3, 2, 72, 48, 130, "silu"), 1 << 26), ((20, 2, 1, (1 << 22) + 8, 16, 24, "gelu"), None),
+                                      ((20, 2, 1, 8, (1 << 22) + 16, 8, "relu2"), None)])
+def test_grouped_rows_far_apart(shape, ld):
+    T, E, top, K, F, H, kind = shape
+    case = _case(T, E, top, K, F, H, kind, T + E)
+    want, bound = _want(case, kind, False, True)
+    got = _run("grouped", case, kind, False, True, ld)
+    assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
 
 
 # (rows, experts, experts a row, K, F, H): one unit of 64 for eight or four waves, odd units, more than 8 and 16 pairs of one expert
