@@ -5,7 +5,9 @@
 
 namespace kvcm {
 
-// silu with gate, silu(gate) and up rounded on the way as a stored product's would be, or silu or relu in 32 bits
+// What becomes of gate and up.  kSiluStored: silu with gate, silu(gate) and up rounded on the way as a stored product's would be, by
+// the function that serves bfloat16 results.  kSilu, kRelu: in 32 bits with the exact functions, rounded once, whatever the result is
+// stored as: what kvcm_gated_act gives for the same sums, bit for bit (the gate with limits too).
 enum TileAct : int { kSiluStored = 0, kSilu = 1, kRelu = 2 };
 
 struct TilesCall {

@@ -20,12 +20,12 @@
 
 namespace kvcm {
 
-// act(gate) * up (TileAct), or, limit > 0, the gate with limits; but for kSiluStored in 32 bits
+// act(gate) * up (TileAct), or, limit > 0, the gate with limits
 template <class TO>
 __device__ __forceinline__ float gated(float gate, float up, float limit, int act) {
-  if (limit > 0.f) return clamped_gate<TO>(gate, up, limit);
+  if (limit > 0.f) return act == kSiluStored ? clamped_gate<TO>(gate, up, limit) : clamped_gate<float>(gate, up, limit);
   if (act == kRelu) return fmaxf(gate, 0.f) * up;
-  if (act == kSilu) return silu<TO>(gate) * up;
+  if (act == kSilu) return silu<float>(gate) * up;
   return round_to<TO>(silu<TO>(round_to<TO>(gate))) * round_to<TO>(up);
 }
 
@@ -292,7 +292,7 @@ int kvcm_gemm_tiles_size(int tile, int* rows, int* cols) {
   return 0;
 }
 // The product with a given tile (< 0: the one the rule picks).  is_gated: W [2 N, K], out [M, N] = act(gate) * up (act: 0 silu with the
-// roundings of a stored product followed by kvcm_swiglu, 1 silu, 2 relu, rounded once), or the gate with limits (limit > 0).
+// roundings of a stored product followed by kvcm_swiglu; 1 silu, 2 relu, exact and rounded once), or the gate with limits (limit > 0).
 int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, int out_dtype, int M, int N, int K, int ldx, int ldw, int ldo,
                     int S, int is_gated, int act, float limit, int tile, hipStream_t st) {
   KVCM_REQUIRE(ldx % 8 == 0 && ldw % 8 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0,

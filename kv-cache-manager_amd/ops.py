@@ -721,7 +721,7 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
     return out
 
 
-# act(gate) * up in a product's epilogue (gemm_tiles.h: TileAct), without roundings before the end
+# act(gate) * up in a product's epilogue (gemm_tiles.h: TileAct), without roundings before the end, as ``gated_act`` computes it
 _TILE_ACTS = {"silu": 1, "clamped": 1, "relu": 2}
 
 
@@ -787,7 +787,7 @@ def gemm_swiglu(x, w_gate_up, out, limit=0.0):
         if not (aligned and _near(x, w_gate_up) and _tiles_take(M, I, K, 1, gated=True)):
             return False
         _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0),
-              out.stride(0), 1, 1, 0, float(limit), -1, _stream())
+              out.stride(0), 1, 1, 1 if limit > 0 else 0, float(limit), -1, _stream())
         return True
     if not (aligned and lib().kvcm_gemm_skinny_swiglu_supported(M, I, K)):
         return False

@@ -220,3 +220,19 @@ def test_gated_products_without_roundings_before_the_end(ops, M, I, K, one):
             assert (got == want).float().mean() > 0.98
             assert bool(((got.float() - want.float()).abs() <= 2.0 ** -7 * (scale + want.float().abs())).all())
     assert ops.gemm_gated(x, w, got, "gelu") is False and ops.gemm_gated(x.float(), w.float(), got.float(), "relu") is False
+
+
+@pytest.mark.parametrize("M", [64, 200])
+@pytest.mark.parametrize("activation,limit", [("silu", 0.0), ("clamped", 7.0), ("relu", 0.0)])
+def test_gated_products_apply_the_exact_functions(ops, M, activation, limit):
+    """sums of one term each are exact, so the product gives what ``gated_act`` gives for them, bit for bit: the hardware's exp2 and
+    reciprocal, 2^-24 of the gate's size off, would fall on the other side of a tie here and there"""
+    I, K = 1024, 64
+    x, w = torch.zeros(M, K, device=DEV), torch.zeros(2 * I, K, device=DEV)
+    x[:, 0], x[:, 1] = torch.linspace(-60.0, 8.0, M, device=DEV), 1.0
+    w[:I, 0], w[I:, 1] = torch.linspace(0.25, 1.0, I, device=DEV), torch.linspace(-3.0, 5.0, I, device=DEV)
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    got, want = (torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    assert ops.gemm_gated(x, w, got, activation, limit)
+    ops.gated_act((x.double() @ w.double().t()).float(), want, activation, limit=limit)
+    assert torch.equal(got, want), int((got != want).sum())
