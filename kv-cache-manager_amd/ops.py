@@ -740,6 +740,8 @@ def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0):
     a 32-bit result, ``gated_act``) are the faster or this has no kernel."""
     if activation not in _TILE_ACTS or x.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16:
         return False
+    if activation == "clamped" and not limit > 0:
+        return False          # (``gated_act`` refuses it)
     _dev(x, w_gate_up, out)
     for t, n in ((x, "x"), (w_gate_up, "w_gate_up"), (out, "out")):
         _rows2d(t, n)

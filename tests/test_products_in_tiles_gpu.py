@@ -236,3 +236,11 @@ def test_gated_products_apply_the_exact_functions(ops, M, activation, limit):
     assert ops.gemm_gated(x, w, got, activation, limit)
     ops.gated_act((x.double() @ w.double().t()).float(), want, activation, limit=limit)
     assert torch.equal(got, want), int((got != want).sum())
+
+
+def test_a_gate_with_limits_needs_a_limit(ops):
+    x, w = _operands(7, 200, 1024, 64)
+    got = torch.empty(200, 512, dtype=torch.bfloat16, device=DEV)
+    assert ops.gemm_gated(x, w, got, "clamped", 1.0) and not ops.gemm_gated(x, w, got, "clamped", 0.0) and not ops.gemm_gated(x, w, got, "clamped")
+    with pytest.raises(ops.KernelError, match="positive limit"):
+        ops.gated_act(torch.zeros(200, 1024, device=DEV), got, "clamped")
