@@ -563,6 +563,11 @@ def _library_has_f32out(*shape):
     return _f32out_shapes[shape]
 
 
+def _tuning_mode(tuning):
+    """``tuning`` ("off" | "heuristic" | "all"; None: LIBRARY_TUNING) as a number."""
+    return _TUNING_MODES[LIBRARY_TUNING if tuning is None else tuning]
+
+
 def _library_workspace(device):
     """Device memory the vendor library's product may use (one buffer, kept: recorded steps hold its address)."""
     global _library_ws
@@ -662,8 +667,7 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm operands must both be bfloat16")
     aligned = _in_pieces(x, w)
     library = _library_takes(M, N, K)
-    mode = _TUNING_MODES[LIBRARY_TUNING if tuning is None else tuning]
-    if library and mode == 0 and aligned and _near(x, w) and K % 64 == 0 and N % 64 == 0:
+    if library and aligned and _near(x, w) and K % 64 == 0 and N % 64 == 0 and not _tuning_mode(tuning):
         # (who asks for the library's tuned algorithms gets them)
         S = _usable_splits(M, N, K, scratch, keep_partial) if M <= 512 else 1
         library = not _tiles_take(M, N, K, S, dtype=out.dtype)
@@ -696,6 +700,7 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
         return partial if keep_partial else partial.materialize()
     if library:
         ws = _library_workspace(out.device)
+        mode = _tuning_mode(tuning)
         shape = (M, N, K, x.stride(0), w.stride(0), out.stride(0))
         if mode and lib().kvcm_gemm_library_tuned(*shape) < mode:
             # not a recorded launch: it runs here, once, whoever is recording
@@ -734,10 +739,10 @@ def _gated_tiles_take(M, I, K):
     return blocks >= 160 or (M >= 2 and blocks >= 80) or (M > 8 and K <= 2048 and I >= 512)
 
 
-def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0):
+def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0, tuning=None):
     """out[M, I] = act(x[M, K] @ w_gate^T) * (x @ w_up^T), w_gate_up [2 I, K] the gate rows and the up rows, in one launch and in 32
     bits up to the result ("silu", "relu", or "clamped": ``gated_act``'s with ``limit``), or False where two launches (a product with
-    a 32-bit result, ``gated_act``) are the faster or this has no kernel."""
+    a 32-bit result, ``gated_act``) are the faster, this has no kernel, or ``tuning`` asks for the library's tuned product (many rows)."""
     if activation not in _TILE_ACTS or x.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16:
         return False
     if activation == "clamped" and not limit > 0:
@@ -749,17 +754,18 @@ def gemm_gated(x, w_gate_up, out, activation="silu", limit=0.0):
     I = out.shape[1]
     _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_gated shapes do not agree")
     if (I % 32 or K % 64 or not _in_pieces(x, w_gate_up) or not _near(x, w_gate_up)
-            or not (_tiles_take(M, I, K, 1, gated=True) if many_rows(M) else _gated_tiles_take(M, I, K))):
+            or not (_tiles_take(M, I, K, 1, gated=True) and not _tuning_mode(tuning) if many_rows(M) else _gated_tiles_take(M, I, K))):
         return False
     _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0), out.stride(0), 1,
           1, _TILE_ACTS[activation], float(limit) if activation == "clamped" else 0.0, -1, _stream())
     return True
 
 
-def gemm_swiglu(x, w_gate_up, out, limit=0.0):
+def gemm_swiglu(x, w_gate_up, out, limit=0.0, tuning=None):
     """out[M, I] = swiglu(x[M, K] @ w_gate_up[2 I, K]^T), or with ``limit`` > 0 its form with limits (``gated_act``'s "clamped"), in one launch, or False when this shape
     has no fused kernel (then the caller runs the product and ``swiglu`` one after the other:
-    the same values up to the order of the sums)."""
+    the same values up to the order of the sums).  Many rows with ``tuning`` (as ``gemm``'s) other than "off" have none: the library's
+    tuned product runs."""
     if isinstance(x, NormedRows):
         if limit > 0:
             return False          # (the kernels that take rows whose norm is still to be applied know silu only)
@@ -786,7 +792,7 @@ def gemm_swiglu(x, w_gate_up, out, limit=0.0):
     aligned = x.dtype == w_gate_up.dtype == out.dtype == torch.bfloat16 and _in_pieces(x, w_gate_up)
     if many_rows(M):
         # many rows: the library product, then swiglu, unless the tiles are the faster
-        if not (aligned and _near(x, w_gate_up) and _tiles_take(M, I, K, 1, gated=True)):
+        if not (aligned and _near(x, w_gate_up) and not _tuning_mode(tuning) and _tiles_take(M, I, K, 1, gated=True)):
             return False
         _call("kvcm_gemm_tiles", _ptr(x), _ptr(w_gate_up), 0, _ptr(out), _DT[out.dtype], M, I, K, x.stride(0), w_gate_up.stride(0),
               out.stride(0), 1, 1, 1 if limit > 0 else 0, float(limit), -1, _stream())

@@ -215,7 +215,7 @@ class GatedFeedForward(JoinableEnds, FeedForward):
         # epilogue, one launch; the kernel of few rows, for what that does not take, rounds silu once more on the way, within the
         # result's own rounding
         one = act.dtype == torch.bfloat16 and torch.is_tensor(h) and (
-            ops.gemm_gated(h, self.w["w_gate_up"], act, kind, limit)
+            ops.gemm_gated(h, self.w["w_gate_up"], act, kind, limit, tuning=step.tune_products)
             or kind in ("silu", "clamped") and not ops.many_rows(step.rows) and ops.gemm_swiglu(h, self.w["w_gate_up"], act, limit=limit))
         if not one:
             gu = linear32(self.ctx, step, h, self.w["w_gate_up"], "gated_gate_up")

@@ -210,9 +210,9 @@ class SwiGLU(FeedForward):
     def forward(self, step, h):
         I = self.params["intermediate_size"]
         act = step.ws("act", (step.rows, I))
-        if not self.ctx.ops.gemm_swiglu(h, self.w["w_gate_up"], act):      # few rows: one launch
+        if not self.ctx.ops.gemm_swiglu(h, self.w["w_gate_up"], act, tuning=step.tune_products):      # few rows: one launch
             h = as_tensor(h)
-            if not self.ctx.ops.gemm_swiglu(h, self.w["w_gate_up"], act):
+            if not self.ctx.ops.gemm_swiglu(h, self.w["w_gate_up"], act, tuning=step.tune_products):
                 gu = _linear(self.ctx, step, h, self.w["w_gate_up"], "gate_up")
                 self.ctx.ops.swiglu(gu, act)
         return _to_residual(self.ctx, step, act, self.w["w_down"], "ffn_out")

@@ -244,3 +244,30 @@ def test_a_gate_with_limits_needs_a_limit(ops):
     assert ops.gemm_gated(x, w, got, "clamped", 1.0) and not ops.gemm_gated(x, w, got, "clamped", 0.0) and not ops.gemm_gated(x, w, got, "clamped")
     with pytest.raises(ops.KernelError, match="positive limit"):
         ops.gated_act(torch.zeros(200, 1024, device=DEV), got, "clamped")
+
+
+def test_tuned_library_products_take_gate_and_up_too(ops, tmp_path, monkeypatch):
+    """who asks for the library's tuned algorithms gets them for the largest product of a layer as for the others"""
+    x, w = _operands(8, 128, 1024, 64)
+    act = torch.empty(128, 512, dtype=torch.bfloat16, device=DEV)
+    for mode in ("heuristic", "all"):
+        assert not ops.gemm_swiglu(x, w, act, tuning=mode) and not ops.gemm_gated(x, w, act, tuning=mode)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "LIBRARY_TUNING", mode)
+            assert not ops.gemm_swiglu(x, w, act) and not ops.gemm_gated(x, w, act)
+            assert ops.gemm_swiglu(x, w, act, tuning="off") and ops.gemm_gated(x, w, act, tuning="off")
+        assert ops.gemm_gated(x[:64], w, act[:64], tuning=mode)      # (few rows are never the library's)
+    assert ops.gemm_swiglu(x, w, act) and ops.gemm_gated(x, w, act)
+
+    from kvcm_amd.config.engine_config import EngineConfig
+    from kvcm_amd.config.model_config import LlamaConfig
+    from kvcm_amd.engine.engine import Engine
+    from kvcm_amd.weights.random_init import write_model_dir
+    raw = dict(vocab_size=256, hidden_size=64, intermediate_size=320, num_hidden_layers=1, num_attention_heads=4, num_key_value_heads=2, head_dim=16,
+               max_position_embeddings=256, rope_theta=10000.0, rms_norm_eps=1e-5, tie_word_embeddings=False)
+    write_model_dir(str(tmp_path), "LlamaForCausalLM", LlamaConfig.from_dict(raw), seed=0, dtype=torch.float32)
+    eng = Engine(str(tmp_path), EngineConfig(block_size=16, num_blocks=64, max_seq_len=256, max_num_seqs=2, max_batched_tokens=160, dtype="bfloat16",
+                                             tune_products="heuristic"))
+    before = len(ops.library_tuning_log)
+    eng.generate([list(range(130))], max_new_tokens=1)
+    assert (640, 64) in [entry[1:3] for entry in ops.library_tuning_log[before:]], ops.library_tuning_log[before:]
