@@ -275,8 +275,13 @@ int kvcm_moe_up(const void* h, int dtype, int ldh, const void* w_up, const int* 
                 int E, int kind, const float* in_weight, hipStream_t s);
 int kvcm_moe_down(const void* act, int dtype, const void* w_down, const int* chosen, const float* weight, const float* add,
                   float* out, int T, int F, int H, int top, int E, hipStream_t s);
-// (moe_few.hip) do the two products above take these sizes on the matrix cores, an expert's weights read once for all its rows?  (bfloat16)
-int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E);
+// (moe_few.hip) are steps of T rows best left to the two products above, which then run on the matrix cores, an expert's weights read
+// once for all its rows?  (bfloat16)  Those two kernels, whatever is the faster.
+int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E, int kind);
+int kvcm_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
+                    const float* in_weight, hipStream_t s);
+int kvcm_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T, int F,
+                      int H, int top, int E, hipStream_t s);
 // (moe_grouped.hip) the routed feed-forward for many rows: pairs grouped by expert, tiles on the matrix cores
 int kvcm_moe_grouped_supported(int K, int F, int E);
 int kvcm_moe_grouped_lists(int n, int E);

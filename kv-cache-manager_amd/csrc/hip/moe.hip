@@ -26,9 +26,10 @@
 
 namespace kvcm {
 
-// moe_few.hip: the two products of up to 64 pairs on the matrix cores, an expert's weights read once for all its rows
-bool moe_few_up_takes(int dtype, const void* h, int ldh, int T, int K, int F, int top);
-bool moe_few_down_takes(int dtype, const void* act, int T, int F, int H, int top, int E);
+// moe_few.hip: the two products of up to 64 pairs on the matrix cores, an expert's weights read once for all its rows.  takes: the
+// operands fit and, where the kernels here could run them (others), that is the faster.
+bool moe_few_up_takes(int dtype, const void* h, int ldh, int T, int K, int F, int top, int E, int kind, bool others);
+bool moe_few_down_takes(int dtype, const void* act, int T, int F, int H, int top, int E, bool others);
 void launch_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
                        const float* in_weight, hipStream_t s);
 void launch_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T,
@@ -284,7 +285,8 @@ int kvcm_moe_up(const void* h, int dtype, int ldh, const void* w_up, const int* 
   KVCM_REQUIRE(kind != 1 || F % 16 == 0, "moe_up: gated experts of %d columns are not supported (a multiple of 16)", F);
   KVCM_REQUIRE(reinterpret_cast<uintptr_t>(w_up) % 16 == 0, "moe_up: weights must be 16-byte aligned");
   KVCM_REQUIRE(dtype == kF32 || dtype == kBF16, "moe_up: unknown dtype %d", dtype);
-  if (moe_few_up_takes(dtype, h, ldh, T, K, F, top)) {      // (keeps no row in LDS: any width)
+  const bool row_fits = K * sizeof(float) <= 64 * 1024 && (F + 3) / 4 <= 65535;
+  if (moe_few_up_takes(dtype, h, ldh, T, K, F, top, E, kind, row_fits)) {      // (keeps no row in LDS: any width)
     launch_moe_few_up(h, ldh, w_up, chosen, act, T, K, F, top, E, kind, in_weight, s);
     return launch_status("moe_up");
   }
@@ -309,11 +311,11 @@ int kvcm_moe_down(const void* act, int dtype, const void* w_down, const int* cho
   KVCM_REQUIRE(T > 0 && H > 0 && F > 0 && top > 0 && E > 0, "moe_down: bad sizes");
   KVCM_REQUIRE(reinterpret_cast<uintptr_t>(w_down) % 16 == 0, "moe_down: weights must be 16-byte aligned");
   KVCM_REQUIRE(dtype == kF32 || dtype == kBF16, "moe_down: unknown dtype %d", dtype);
-  if (moe_few_down_takes(dtype, act, T, F, H, top, E)) {      // (keeps no activations in LDS: any width)
+  const size_t lds = static_cast<size_t>(top) * ((F + 3) & ~3) * sizeof(float);
+  if (moe_few_down_takes(dtype, act, T, F, H, top, E, lds <= 64 * 1024 && (H + 3) / 4 <= 65535)) {      // (keeps no activations in LDS: any width)
     launch_moe_few_down(act, w_down, chosen, weight, add, out, T, F, H, top, E, s);
     return launch_status("moe_down");
   }
-  const size_t lds = static_cast<size_t>(top) * ((F + 3) & ~3) * sizeof(float);
   KVCM_REQUIRE(lds <= 64 * 1024, "moe_down: %d activations of %d values do not fit the local memory", top, F);
   KVCM_REQUIRE((H + 3) / 4 <= 65535, "moe_down: too many columns");
   const int cw = moe_cols_per_wave(T, H);

@@ -16,10 +16,9 @@
 //
 // Measured over weights that go round several copies, row by row / here, us: 8 rows, 8 experts of which a row uses 2, width
 // 2,048, 1,408 columns an expert: up 31.3 / 19.7 (92 MB, 4.7 TB/s), down 17.3 / 12.6; 15 rows 51.9 / 20.1 and 28.9 / 14.0; 4 rows 18.4 /
-// 13.3 and 11.3 / 9.3; width 4,096, 3,584 columns, 8 rows: 135 / 85 and 69 / 48.  At one and two rows, which seldom share an expert,
-// the row-by-row kernels are as fast or faster (7.5 / 8.2 and 6.4 / 8.7; 11.7 / 12.7 and 7.6 / 8.0), hence the lower limit; many
-// experts of few columns are many short turns of the down kernel's waves (64 experts, 704 columns, 48 pairs: 27.4 / 28.5), hence
-// its limit on experts.
+// 13.3 and 11.3 / 9.3; width 4,096, 3,584 columns, 8 rows: 135 / 85 and 69 / 48.  Which sizes come here: up_gains, down_gains, below.
+#include <cmath>
+
 #include "common.h"
 #include "kvcm_hip.h"
 
@@ -227,21 +226,52 @@ __global__ void __launch_bounds__(kDownWaves * kWave, 2)
 
 }  // namespace
 
-constexpr int kFewRows = 3, kDownExperts = 32;      // from as many rows, up to as many experts: see the figures above
+constexpr int kFewRows = 3, kDownExperts = 32;
 
-bool moe_few_up_takes(int dtype, const void* h, int ldh, int T, int K, int F, int top) {
-  return dtype == kBF16 && T >= kFewRows && static_cast<long long>(T) * top <= kMostPairs && K % kUnit == 0 && F % 32 == 0 && ldh % 8 == 0 &&
+// Do the kernels take these operands?
+static bool up_fits(int dtype, const void* h, int ldh, int T, int K, int F, int top) {
+  return dtype == kBF16 && static_cast<long long>(T) * top <= kMostPairs && K % kUnit == 0 && F % 32 == 0 && ldh % 8 == 0 &&
          reinterpret_cast<uintptr_t>(h) % 16 == 0;
 }
-
-bool moe_few_down_takes(int dtype, const void* act, int T, int F, int H, int top, int E) {
-  return dtype == kBF16 && T >= kFewRows && E <= kDownExperts && static_cast<long long>(T) * top <= kMostPairs && T <= kWave && F % kUnit == 0 && H % 8 == 0 &&
-         reinterpret_cast<uintptr_t>(act) % 16 == 0;
+static bool down_fits(int dtype, const void* act, int T, int F, int H, int top) {
+  return dtype == kBF16 && static_cast<long long>(T) * top <= kMostPairs && F % kUnit == 0 && H % 8 == 0 && reinterpret_cast<uintptr_t>(act) % 16 == 0;
 }
 
-// (for the parts: do both products of T rows come here, whatever their strides?)
-extern "C" int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E) {
-  return moe_few_up_takes(kBF16, nullptr, 0, T, K, F, top) && moe_few_down_takes(kBF16, nullptr, T, F, H, top, E);
+// How many experts the pairs of T rows name on average, evenly loaded: the row-by-row kernels read T top matrices, these so many.
+static float experts_met(int T, int top, int E) {
+  return static_cast<float>(E) * (1.f - std::pow(1.f - static_cast<float>(top < E ? top : E) / static_cast<float>(E), static_cast<float>(T)));
+}
+
+// Are they the faster?  Lines through 1,745 measured sizes (3 to 15 rows; 2 to 64 experts, of which a row uses 1 to 6; width 512 to 4,096, 256 to
+// 14,336 columns an expert; other weights and choices from launch to launch).  Both launches against the row-by-row kernels': 0.87 of the
+// time on average and 1.03 at worst where the load is even, 0.77 and 1.09 where all rows name the same experts; 0.95 and 1.73, 0.75 and
+// 1.63 if all came here.  Row by row / here, us, evenly loaded:
+//   up, rows of an expert's matrices (gate and up together).  From 2,816 on (width 1,024 on) a workgroup for each 32 of them fills the chip
+//   for few pairs: 16 experts, one a row, 2,816 x 2,048: 4 rows 11.7 / 12.9, 6 rows 18.6 / 16.1.  From 1,408 on it takes more pairs, or pairs that share
+//   experts: 1,408 x 2,048, 8 experts, one a row: 8 rows 11.1 / 11.9, 11 rows 13.7 / 12.7; two a row: 5 rows 13.3 / 12.4.  From 1,024 on (width 768 on) more
+//   still: 1,024 x 1,024, 8 experts, two a row: 8 rows 8.6 / 7.7; one a row: 8 rows 5.8 / 6.0, 15 rows 7.8 / 7.5.
+//   down: an expert is a turn of a wave, however few its pairs, so that sharing decides: 1,408 columns, width 2,048, 16 experts, one a row: 8
+//   rows 10.0 / 10.3, 15 rows 16.1 / 13.7; 8 experts, two a row: 3 rows 8.8 / 9.1, 5 rows 12.4 / 10.6.  Width 1,024 is 128 workgroups: 2,048 columns, 8
+//   experts, two a row: 8 rows 13.4 / 13.4, 15 rows 20.4 / 16.1; 4 experts, one a row, 4 rows 5.7 / 7.5.
+static bool up_gains(int T, int K, int rows, int top, int E) {
+  const float n = static_cast<float>(T * top), met = experts_met(T, top, E);
+  if (T < kFewRows || K < 768 || rows < 1024) return false;
+  if (K >= 1024 && rows >= 2816) return n >= 5.f || n >= 1.6f * met;
+  if (K >= 1024 && rows >= 1408 && (n >= 10.f || (n >= 5.f && n >= 1.6f * met))) return true;
+  return n >= 16.f || (n >= 8.f && n >= 2.3f * met);
+}
+static bool down_gains(int T, int F, int H, int top, int E) {
+  const float n = static_cast<float>(T * top), met = experts_met(T, top, E);
+  if (T < kFewRows || E > kDownExperts) return false;
+  if (H >= 2048 && F >= 704) return n >= 6.f && n >= 1.6f * met;
+  return n >= 16.f && n >= 2.6f * met && ((H >= 2048 && F >= 512) || (H >= 1024 && F >= 1024));
+}
+
+bool moe_few_up_takes(int dtype, const void* h, int ldh, int T, int K, int F, int top, int E, int kind, bool others) {
+  return up_fits(dtype, h, ldh, T, K, F, top) && (!others || up_gains(T, K, kind == 1 ? 2 * F : F, top, E));
+}
+bool moe_few_down_takes(int dtype, const void* act, int T, int F, int H, int top, int E, bool others) {
+  return down_fits(dtype, act, T, F, H, top) && (!others || down_gains(T, F, H, top, E));
 }
 
 void launch_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
@@ -263,3 +293,39 @@ void launch_moe_few_down(const void* act, const void* w_down, const int* chosen,
 }
 
 }  // namespace kvcm
+
+using namespace kvcm;
+
+extern "C" {
+
+// (for the parts, whose other choice from 16 rows on is kvcm_moe_grouped) do both products of T rows come here, whatever their strides?
+// At 16 rows an expert has at most sixteen pairs, one pass over its matrices, and the down kernel's workgroups are to be about one a CU: both
+// products took 0.87 of the time of all launches of the grouped form on average (60 sizes of width 2,048, up to 32 experts; 1.04 at worst), 0.85 and 1.06 where
+// all rows name the same experts.  With more rows an expert may be several passes of one wave: evenly loaded 24 rows with two of 8
+// experts each take 36.3 us here and 39.5 grouped (1,408 columns), but 31.0 and 24.1 where all name the same two, 64 rows up to 2.7 times as long.
+// Width 4,096, 3,584 columns, 8 experts, two a row, 16 rows: 139 / 134.
+int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E, int kind) {
+  if (!up_fits(kBF16, nullptr, 0, T, K, F, top) || !down_fits(kBF16, nullptr, T, F, H, top)) return 0;
+  if (T == 16) return H > 1536 && H <= 2048 && F >= 256 && top <= 2 && E <= kDownExperts;
+  return T < 16 && up_gains(T, K, kind == 1 ? 2 * F : F, top, E) && down_gains(T, F, H, top, E);
+}
+
+// The two products by these kernels whatever is the faster (operands as kvcm_moe_up's and kvcm_moe_down's, bfloat16).
+int kvcm_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
+                    const float* in_weight, hipStream_t s) {
+  if (T == 0) return 0;
+  KVCM_REQUIRE(T > 0 && K > 0 && F > 0 && top > 0 && E > 0 && ldh >= K && kind >= 0 && kind <= 2, "moe_few_up: bad sizes");
+  KVCM_REQUIRE(up_fits(kBF16, h, ldh, T, K, F, top) && reinterpret_cast<uintptr_t>(w_up) % 16 == 0, "moe_few_up: unsupported sizes or alignment");
+  launch_moe_few_up(h, ldh, w_up, chosen, act, T, K, F, top, E, kind, in_weight, s);
+  return launch_status("moe_few_up");
+}
+int kvcm_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T, int F,
+                      int H, int top, int E, hipStream_t s) {
+  if (T == 0) return 0;
+  KVCM_REQUIRE(T > 0 && H > 0 && F > 0 && top > 0 && E > 0, "moe_few_down: bad sizes");
+  KVCM_REQUIRE(down_fits(kBF16, act, T, F, H, top) && reinterpret_cast<uintptr_t>(w_down) % 16 == 0, "moe_few_down: unsupported sizes or alignment");
+  launch_moe_few_down(act, w_down, chosen, weight, add, out, T, F, H, top, E, s);
+  return launch_status("moe_few_down");
+}
+
+}  // extern "C"

@@ -119,7 +119,9 @@ def _declare(lib):
     fn("kvcm_moe_table_route", vp, vp, i, i, i, vp, vp, i, vp)
     fn("kvcm_moe_up", vp, i, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
     fn("kvcm_moe_down", vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, vp)
-    fn("kvcm_moe_few_takes", i, i, i, i, i, i)
+    fn("kvcm_moe_few_takes", i, i, i, i, i, i, i)
+    fn("kvcm_moe_few_up", vp, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
+    fn("kvcm_moe_few_down", vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp)
     fn("kvcm_moe_grouped_supported", i, i, i)
     fn("kvcm_moe_grouped_lists", i, i)
     fn("kvcm_moe_grouped_tile_count")
@@ -1807,12 +1809,14 @@ def _expert_kind(gated, activation):
     return EXPERT_KINDS["silu_gated" if gated else activation]
 
 
-def moe_rows(h, w_up, w_down, chosen, weight, act, out, gated=False, add=None, activation="relu2", weigh_input=False):
+def moe_rows(h, w_up, w_down, chosen, weight, act, out, gated=False, add=None, activation="relu2", weigh_input=False, few=False):
     """out[T, H] (float32) = sum over a row's chosen experts e of weight * W_down[e] square(relu(W_up[e] h)), a row at a
     time, reading only the chosen experts.  h [T, K]; w_up [E, F, K]; w_down [E, H, F]; act: work memory [T * top, F].
     ``gated``: w_up is ``interleave_gate_up`` of the experts' gate and up matrices and the activation is
     silu(W_gate h) * (W_up h); otherwise ``activation`` may be "gelu" instead of "relu2".  ``weigh_input``: the weights are
-    factors on what the experts read, not on what they give.  ``add`` (float32 [T, H]): out = add + the sum."""
+    factors on what the experts read, not on what they give.  ``add`` (float32 [T, H]): out = add + the sum.
+    Up to 64 (row, slot) pairs in bfloat16 run on the matrix cores where that is the faster, an expert's weights read once for
+    all the rows that chose it (csrc/hip/moe_few.hip); ``few``: in any case."""
     T, K = h.shape
     E, F, _ = _expert_shapes(w_up, w_down, gated)
     H, top = w_down.shape[1], chosen.shape[1]
@@ -1826,17 +1830,23 @@ def moe_rows(h, w_up, w_down, chosen, weight, act, out, gated=False, add=None, a
     _need(out.dtype == torch.float32 and out.is_contiguous() and tuple(out.shape) == (T, H), "out must be float32 [T, H]")
     _need(chosen.dtype == torch.int32 and chosen.is_contiguous() and chosen.shape[0] >= T, "chosen must be int32 [T, top]")
     _need(weight.dtype == torch.float32 and weight.is_contiguous() and tuple(weight.shape) == tuple(chosen.shape), "weight must match chosen")
+    if few:
+        _need(h.dtype == torch.bfloat16, "moe_rows: the kernels of a few rows take bfloat16")
+        _call("kvcm_moe_few_up", _ptr(h), h.stride(0), _ptr(w_up), _ptr(chosen), _ptr(act), T, K, F, top, E,
+              _expert_kind(gated, activation), _ptr(weight) if weigh_input else 0, _stream())
+        _call("kvcm_moe_few_down", _ptr(act), _ptr(w_down), _ptr(chosen), 0 if weigh_input else _ptr(weight), _ptr(add), _ptr(out), T, F, H, top, E, _stream())
+        return out
     _call("kvcm_moe_up", _ptr(h), _DT[h.dtype], h.stride(0), _ptr(w_up), _ptr(chosen), _ptr(act), T, K, F, top, E,
           _expert_kind(gated, activation), _ptr(weight) if weigh_input else 0, _stream())
     _call("kvcm_moe_down", _ptr(act), _DT[act.dtype], _ptr(w_down), _ptr(chosen), 0 if weigh_input else _ptr(weight), _ptr(add), _ptr(out), T, F, H, top, E, _stream())
     return out
 
 
-def moe_few_takes(h, F, H, top, E):
-    """Does ``moe_rows`` run rows h [T, K] on the matrix cores, an expert's weights read once for all the rows that chose it?
-    (A few rows, up to 64 (row, slot) pairs.)"""
+def moe_few_takes(h, F, H, top, E, gated=False):
+    """Are rows h [T, K] best left to ``moe_rows``, which then runs them on the matrix cores, an expert's weights read once for all the
+    rows that chose it?  (A few rows, up to 64 (row, slot) pairs.)"""
     return (h.dtype == torch.bfloat16 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0
-            and bool(lib().kvcm_moe_few_takes(h.shape[0], h.shape[1], int(F), int(H), int(top), int(E))))
+            and bool(lib().kvcm_moe_few_takes(h.shape[0], h.shape[1], int(F), int(H), int(top), int(E), int(bool(gated)))))
 
 
 def moe_grouped_supported(K, F, E, dtype):

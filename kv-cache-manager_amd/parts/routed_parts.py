@@ -186,9 +186,8 @@ class RoutedExperts(JoinableEnds, FeedForward):
         how = dict(gated=self.gated, add=add, weigh_input=p.get("weigh") == "input", **({} if self.gated else {"activation": self.activation}))
         act = step.ws("routed_act", (T, top * F)).view(T * top, F)
         out = step.ws("routed_out", (T, H), torch.float32)
-        # up to 64 pairs moe_rows reads an expert once for all its rows too, without grouping (us a layer of 8 experts, two a row, 1,408 columns
-        # of 2,048: 16 rows 47 grouped, 31 so; 32 rows 47 and 39; width 4,096, 3,584 columns: 183 and 144, 183 and 173)
-        few = ops.moe_few_takes(h, F, H, top, E)
+        # moe_rows reads an expert once for all its rows too, without grouping, where that is the faster (csrc/hip/moe_few.hip)
+        few = ops.moe_few_takes(h, F, H, top, E, self.gated)
         if T >= self.GROUPED_MIN_ROWS and not few and ops.moe_grouped_supported(H, F, E, act.dtype) and h.stride(0) % 8 == 0:
             # many rows: the pairs grouped by expert, tiles on the matrix cores, every expert's weights read once per tile
             order = step.ws("routed_order", (T, top), torch.int32)

@@ -63,7 +63,7 @@ def _run(form, case, kind, weigh_input, add, ld=None):
         y = torch.full((T * top, H), float("nan"), device=DEV)
         ops.moe_grouped(wide[:, :K], up, down, chosen, weight, order, tiles, act, y, out, **how)
     else:
-        ops.moe_rows(wide[:, :K], up, down, chosen, weight, act, out, **how)
+        ops.moe_rows(wide[:, :K], up, down, chosen, weight, act, out, few=form == "few", **how)
     return out.cpu().double()
 
 
@@ -106,7 +106,7 @@ def test_grouped_rows_far_apart(shape, ld):
 # (rows, experts, experts a row, K, F, H): one unit of 64 for eight or four waves, odd units, more than 8 and 16 pairs of one expert
 # ("one"), an expert named twice by a row, and numbers that name none
 FEW = [(3, 8, 2, 64, 64, 8, "silu", None), (15, 8, 2, 448, 192, 136, "relu2", None), (20, 3, 3, 128, 128, 64, "gelu", None),
-       (32, 4, 2, 320, 64, 72, "silu", "one"), (9, 40, 7, 192, 96, 24, "relu2", None), (10, 6, 2, 128, 320, 16, "silu", "odd"),
+       (32, 4, 2, 320, 64, 72, "silu", "one"), (9, 40, 7, 192, 128, 24, "relu2", None), (10, 6, 2, 128, 320, 16, "silu", "odd"),
        (17, 5, 1, 64, 448, 40, "gelu", "one"), (64, 8, 1, 576, 64, 8, "silu", None),
        # activations of a row, and rows, that a workgroup's LDS would not hold
        (16, 3, 2, 64, 8256, 8, "silu", None), (16, 2, 1, 16448, 64, 8, "relu2", None)]
@@ -125,6 +125,26 @@ def test_few_rows(shape, weigh_input):
         chosen[2] = 4
         chosen[5, 0], chosen[7] = -1, E
     _check("few", _case(T, E, top, K, F, H, kind, T + K, chosen), kind, weigh_input, not weigh_input)
+
+
+# sizes at which a row-by-row kernel, one of a few rows' two, or both run (the way whose measured time is the shorter)
+@pytest.mark.parametrize("T,E,top,K,F,H,kind", [(3, 8, 2, 64, 64, 64, "silu"), (4, 16, 1, 1024, 1408, 2048, "silu"), (6, 16, 1, 1024, 1408, 2048, "silu"),
+                                                (3, 2, 1, 1024, 1408, 64, "silu"), (5, 8, 2, 1024, 704, 2048, "gelu"), (15, 8, 2, 768, 512, 1024, "relu2"),
+                                                (15, 8, 2, 1024, 1024, 1024, "relu2"), (11, 40, 2, 1024, 704, 2048, "silu"), (2, 8, 4, 1024, 1408, 2048, "silu"),
+                                                # what a row-by-row kernel's LDS would not hold
+                                                (8, 3, 2, 64, 8256, 64, "silu"), (4, 2, 1, 16448, 64, 8, "relu2")])
+def test_rows_by_the_faster_kernels(T, E, top, K, F, H, kind):
+    _check("rows", _case(T, E, top, K, F, H, kind, T + F), kind, False, True)
+
+
+@pytest.mark.parametrize("T,K,F,H,top,E,gated,few", [
+    (8, 2048, 1408, 2048, 2, 8, True, True), (16, 2048, 1408, 2048, 2, 8, True, True), (17, 2048, 1408, 2048, 2, 8, True, False),
+    (16, 2048, 1408, 2048, 1, 16, True, True), (16, 2048, 1408, 2048, 1, 33, True, False), (64, 2048, 1408, 2048, 1, 16, True, False), (16, 4096, 3584, 4096, 2, 8, True, False), (15, 4096, 3584, 4096, 2, 8, True, True),
+    (15, 512, 256, 512, 2, 8, True, False), (3, 2048, 1408, 2048, 1, 4, True, False), (2, 2048, 1408, 2048, 8, 8, True, False),
+    (8, 2048, 1408, 2048, 2, 64, True, False), (8, 1024, 704, 2048, 2, 8, True, True), (8, 1024, 704, 2048, 2, 16, False, False), (16, 2048, 1408, 2048, 5, 32, True, False)])
+def test_which_steps_a_few_rows_kernels_take(T, K, F, H, top, E, gated, few):
+    from kvcm_amd import ops
+    assert bool(ops.lib().kvcm_moe_few_takes(T, K, F, H, top, E, int(gated))) == few
 
 
 @pytest.mark.parametrize("T,top,H,F", [(16, 2, 64, 8256), (32, 2, 64, 8256), (20, 1, 16448, 64)])
