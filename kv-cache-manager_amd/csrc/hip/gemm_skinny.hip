@@ -195,33 +195,24 @@ static bool swiglu_in_tiles(int M, int I) {
   return M > 0 && M <= kMaxTileRows && I % 32 == 0 && static_cast<long long>(I / 32) * row_blocks(M) >= 160;
 }
 
-// How many 16-column tiles a workgroup may take so that tiles x splits x row blocks make about one workgroup per CU and none is
-// left out: what such a product streams per microsecond grows with the CUs it covers.  The splits below keep it to at most eight.
-constexpr int kRowsCUs = 256;
-static int rows_waves(long long units, int mt) {
-  const long long want = (units + kRowsCUs - 1) / kRowsCUs;
-  int w = want < 2 ? 2 : want > 8 ? 8 : static_cast<int>(want);
-  if (w < 8 && (mt + w) / (w + 1) < (mt + w - 1) / w) ++w;
-  return w;
-}
-static int rows_tiles_m(int M) { return M > kRowBlock ? kRowBlock / 16 : (M + 15) / 16; }
-
-// Splits of K of a plain product in tiles: eight where there are few column tiles, or where K is long
+// Splits of K of a plain product in tiles: eight where there are few columns, or where K is long
 // against the rows (the partial sums, S*M*N floats that the next kernel reads, are small against the
-// weights then), else four; as long as every slice has a trip of its own and the partial sums stay below
-// the weights' bytes; halved while more than eight waves a workgroup would be needed to get down to one
-// workgroup per CU.  Measured at 17 to 128 rows over the projections of TinyLlama and Llama-3-8B sizes,
-// alone and in whole decode steps.  Up to 16 rows the norm that follows is a workgroup a row, each reading all slices of its row: four
-// of 128 column tiles too (Kasuvik and Fisesun, eight requests, 34.61 -> 34.09 and 30.69 -> 30.30 ms a pass; at 64 rows of TinyLlama
-// sizes four were slower, 150.8 -> 152.0).  (With the tiles free to choose among 1, 2, 4 and 8 as well, launches and the reading of the
-// partial sums together would be 4 % shorter at 8 to 512 rows.)
+// weights then), else four; as long as every slice has 256 k (more than 64 rows: 128), two to four steps of the ring,
+// and the partial sums stay below the weights' bytes; none where the columns are enough for the chip, and halved where the slices
+// would be more than eight 16-column tiles a CU.  Measured at 17 to 128 rows over the projections of TinyLlama and Llama-3-8B sizes,
+// alone and in whole decode steps, with the kernel that streamed W into registers, and kept for its successor: the tile is chosen for
+// these slices (gemm_tiles.hip).  (With the tiles free to choose among 1, 2, 4 and 8 as well, launches and the reading of the
+// partial sums together would be 4 % shorter at 8 to 512 rows.)  Up to 16 rows the norm that follows is a workgroup a row, each reading
+// all slices of its row: four of 128 column tiles too (Kasuvik and Fisesun, eight requests, 34.61 -> 34.09 and 30.69 -> 30.30 ms a pass;
+// at 64 rows of TinyLlama sizes four were slower, 150.8 -> 152.0).
+constexpr int kRowsCUs = 256;
 static int rows_splits(int M, int N, int K) {
   const long long tiles = static_cast<long long>(N / 16) * row_blocks(M);
   const int units = K / kUnit;
   if (tiles >= 4 * kRowsCUs) return 1;
   int S = tiles <= (M <= 16 ? 64 : 128) || (M > 48 && K >= 112 * M) ? 8 : 4;
-  const int trip = M <= 64 ? 4 : 2;   // units per trip (the launch's choice below)
-  const int cap = units / trip < K / (2 * M) ? units / trip : K / (2 * M);
+  const int least = M <= 64 ? 4 : 2;   // units of a slice
+  const int cap = units / least < K / (2 * M) ? units / least : K / (2 * M);
   while (S > 1 && S > cap) S >>= 1;
   while (S > 1 && tiles * S > 8 * kRowsCUs) S >>= 1;
   return S;
@@ -248,15 +239,6 @@ int kvcm_gemm_skinny_whole_splits(int M, int N, int K) {
   if (S <= 1 || !in_tiles(M, N)) return S;
   const float add = 3.2f + static_cast<float>(M) * static_cast<float>(N) * (4.f * S + 4.f) / 5e6f;
   return gemm_tiles_time(M, N, K, 1, false, false) <= gemm_tiles_time(M, N, K, S, false, false) + add ? 1 : S;
-}
-
-// 16-column tiles a workgroup that cover the chip for a product of this shape (rows_waves; 0: not a product in tiles).
-// swiglu: N is the activation's width, S is 1.
-int kvcm_gemm_skinny_waves(int M, int N, int K, int S, int swiglu) {
-  if (swiglu ? !swiglu_in_tiles(M, N) : !in_tiles(M, N)) return 0;
-  if (K <= 0 || K % kUnit != 0 || S < 1) return 0;
-  if (!swiglu && S == 1) return 4;
-  return rows_waves(static_cast<long long>(N / (swiglu ? 8 : 16)) * row_blocks(M) * S, rows_tiles_m(M));
 }
 
 // S == 1: the result is stored to `out` (bfloat16 or float32).  S > 1: partial sums are written to

@@ -283,13 +283,17 @@ using namespace kvcm;
 
 extern "C" {
 
-// How many tiles there are, and the rows and columns (of W) of one: for tests, which run each.
+// How many tiles there are, the rows and columns (of W) of one, and the one the rule picks: for tests, which run each.
 int kvcm_gemm_tiles_count() { return kTileCount; }
 int kvcm_gemm_tiles_size(int tile, int* rows, int* cols) {
   KVCM_REQUIRE(tile >= 0 && tile < kTileCount, "gemm_tiles_size: no tile %d", tile);
   *rows = kTiles[tile].bm;
   *cols = kTiles[tile].bn;
   return 0;
+}
+int kvcm_gemm_tiles_pick(int M, int N, int K, int S, int is_gated) {
+  KVCM_REQUIRE(M > 0 && N > 0 && K > 0 && S >= 1, "gemm_tiles_pick: bad sizes");
+  return best_tile(M, is_gated ? 2 * N : N, K, S);
 }
 // The product with a given tile (< 0: the one the rule picks).  is_gated: W [2 N, K], out [M, N] = act(gate) * up (act: 0 silu with the
 // roundings of a stored product followed by kvcm_swiglu; 1 silu, 2 relu, exact and rounded once), or the gate with limits (limit > 0).

@@ -26,12 +26,10 @@ int kvcm_gemm_skinny(const void* X, const void* W, float* partials, void* out, i
 int kvcm_reduce_store(const float* partials, void* out, int out_dtype, int M, int N, int ldo, int S, hipStream_t stream);
 // The same where nobody takes the partial sums (one slice may then be faster than several and a launch that adds them).
 int kvcm_gemm_skinny_whole_splits(int M, int N, int K);
-// 16-column tiles a workgroup with which column tiles x splits x row blocks come to about one workgroup per CU (0: not a
-// product in tiles): what the split count is kept to.
-int kvcm_gemm_skinny_waves(int M, int N, int K, int S, int swiglu);
 // Products in tiles (gemm_tiles.hip), any number of rows: N a multiple of 4 (gated: 8), K of 64.
 int kvcm_gemm_tiles_count();
 int kvcm_gemm_tiles_size(int tile, int* rows, int* cols);
+int kvcm_gemm_tiles_pick(int M, int N, int K, int S, int is_gated);
 int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, int out_dtype, int M, int N, int K, int ldx, int ldw, int ldo,
                     int S, int is_gated, int act, float limit, int tile, hipStream_t stream);
 int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype);

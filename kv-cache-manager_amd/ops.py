@@ -47,10 +47,10 @@ def _declare(lib):
     fn("kvcm_gemm_skinny_swiglu_supported", i, i, i)
     fn("kvcm_gemm_skinny_swiglu", vp, vp, vp, i, i, i, i, i, i, i, f, vp)
     fn("kvcm_gemm_skinny_splits", i, i, i)
-    fn("kvcm_gemm_skinny_waves", i, i, i, i, i)
     fn("kvcm_gemm_skinny_whole_splits", i, i, i)
     fn("kvcm_gemm_tiles_count")
     fn("kvcm_gemm_tiles_size", i, C.POINTER(i), C.POINTER(i))
+    fn("kvcm_gemm_tiles_pick", i, i, i, i, i)
     fn("kvcm_gemm_tiles", vp, vp, vp, vp, i, i, i, i, i, i, i, i, i, i, f, i, vp)
     fn("kvcm_gemm_tiles_preferred", i, i, i, i, i, i)
     fn("kvcm_gemm_skinny_swiglu_normed_preferred", i, i, i)
@@ -576,11 +576,6 @@ def _library_workspace(device):
     if _library_ws is None:
         _library_ws = torch.empty(lib().kvcm_gemm_library_workspace_bytes(), dtype=torch.uint8, device=device)
     return _library_ws
-
-
-def skinny_waves(M, N, K, S=1, swiglu=False):
-    """16-column tiles a workgroup with which this bfloat16 product in tiles covers the chip (0: another kernel takes it)."""
-    return lib().kvcm_gemm_skinny_waves(int(M), int(N), int(K), int(S), int(bool(swiglu)))
 
 
 def skinny_splits(M, N, K):

@@ -683,8 +683,8 @@ def test_gemm_skinny_with_and_without_splits(ops, M, N, K):
 @pytest.mark.parametrize("M", [65, 96, 100, 128, 129, 300, 512])
 @pytest.mark.parametrize("N,K", [(2048, 2048), (2560, 512), (192, 320)])
 def test_gemm_shared_rows_beyond_64_rows(ops, M, N, K):
-    """The weight-streaming kernel for up to 512 rows (row blocks of 128), which the engine uses
-    where the library product may not run: inside captured graphs."""
+    """Products of up to 512 rows by this package's kernels, which the engine uses where the library product may not run: inside
+    captured graphs."""
     rng = np.random.default_rng(M + N)
     x = _bf16_grid(rng.normal(size=(M, K)))
     w = _bf16_grid(rng.normal(size=(N, K)) * 0.05)
@@ -714,35 +714,33 @@ def test_gemm_shared_rows_beyond_64_rows(ops, M, N, K):
         ops.LIBRARY_GEMM_MIN_ROWS = keep
 
 
-def test_gemm_shared_rows_with_every_number_of_waves(ops):
-    """The shared-rows kernel sizes its workgroups (two to eight waves, one column tile each) so that tiles x
-    splits come to about one workgroup per CU: every number of waves, plain and with the SwiGLU epilogue, with a
-    last workgroup that has fewer tiles than waves, against the 64-bit product."""
+def test_products_in_the_tiles_that_the_rule_picks(ops):
+    """Shapes for which the rule picks eleven of the tiles, plain (split along K) and with the SwiGLU epilogue, columns that end inside a
+    tile among them, against the 64-bit product."""
     keep, ops.LIBRARY_GEMM_MIN_ROWS = ops.LIBRARY_GEMM_MIN_ROWS, 0
-    seen, seen_act = set(), set()
+    pick = ops.lib().kvcm_gemm_tiles_pick
+    seen = set()
     try:
-        for M, N, K in [(24, 1024, 2048), (32, 2560, 2048), (64, 2560, 2048), (64, 2560, 8192), (40, 6144, 1024),
+        for M, N, K in [(8, 2048, 2048), (24, 1024, 2048), (32, 2560, 2048), (64, 2560, 2048), (64, 2560, 8192), (40, 6144, 1024),
                         (100, 7168, 1024), (33, 8192, 1024), (96, 2048, 2048)]:
             rng = np.random.default_rng(M + N + K)
             x = _bf16_grid(rng.normal(size=(M, K)))
             w = _bf16_grid(rng.normal(size=(N, K)) * 0.05)
             ref = plain.linear(x, w)
             S = ops.skinny_splits(M, N, K)
-            waves = ops.skinny_waves(M, N, K, S)
-            assert S > 1 and 2 <= waves <= 8 and (N // 16 + waves - 1) // waves * S <= 256 + 64, (M, N, K, S, waves)
-            seen.add(waves)
+            assert S > 1
+            seen.add(pick(M, N, K, S, 0))
             scratch = torch.zeros(S * M * N, dtype=torch.float32, device=DEV)
             out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
-            ops.gemm(_t(x, torch.bfloat16), _t(w, torch.bfloat16), out, scratch=scratch)
-            np.testing.assert_allclose(_np(out), ref, rtol=2 ** -7, atol=1e-3, err_msg=f"{M}x{N}x{K}: {waves} waves, {S} splits")
-        for M, I, K in [(32, 5120, 256), (64, 5632, 256), (24, 5632, 256), (48, 10240, 128), (96, 11008, 128),
-                        (17, 14336, 128), (128, 14336, 128), (20, 16384, 128)]:
+            got = ops.gemm(_t(x, torch.bfloat16), _t(w, torch.bfloat16), out, scratch=scratch, keep_partial=True)
+            assert isinstance(got, ops.PartialSums) and got.splits == S
+            np.testing.assert_allclose(_np(got.materialize()), ref, rtol=2 ** -7, atol=1e-3, err_msg=f"{M}x{N}x{K}: {S} splits")
+        for M, I, K in [(8, 5632, 2048), (32, 5120, 256), (64, 5632, 256), (24, 5632, 256), (48, 10240, 128), (96, 11008, 128),
+                        (17, 14336, 128), (128, 14336, 128), (20, 16384, 128), (512, 5632, 256)]:
             rng = np.random.default_rng(M + I + K)
             x = _bf16_grid(rng.normal(size=(M, K)))
             w = _bf16_grid(rng.normal(size=(2 * I, K)) * 0.2)
-            waves = ops.skinny_waves(M, I, K, 1, swiglu=True)
-            assert 2 <= waves <= 8
-            seen_act.add(waves)
+            seen.add(pick(M, I, K, 1, 1))
             xt, wt = _t(x, torch.bfloat16), _t(w, torch.bfloat16)
             act = torch.full((M, I), 7.0, dtype=torch.bfloat16, device=DEV)
             assert ops.gemm_swiglu(xt, wt, act)
@@ -754,16 +752,17 @@ def test_gemm_shared_rows_with_every_number_of_waves(ops):
             # the two launches walk K from different starting points: a sum may round to the neighbouring bfloat16
             # (2^-7 relative), in the gate, in the up value, or in both, and SiLU below zero multiplies a step of
             # its argument by up to four
-            assert np.mean(a == b) > 0.98, f"{M}x{I}x{K}: {waves} waves"
-            np.testing.assert_allclose(a, b, rtol=2 ** -5, atol=2e-3, err_msg=f"{M}x{I}x{K}: {waves} waves")
+            assert np.mean(a == b) > 0.98, f"{M}x{I}x{K}"
+            np.testing.assert_allclose(a, b, rtol=2 ** -5, atol=2e-3, err_msg=f"{M}x{I}x{K}")
     finally:
         ops.LIBRARY_GEMM_MIN_ROWS = keep
-    assert seen == {2, 3, 4, 5, 6, 7, 8} and seen_act >= {3, 4, 5, 6, 7, 8}, (seen, seen_act)
+    assert len(seen) == 11, seen
 
 
 def test_long_k_products_of_wide_models_stay_with_this_packages_kernel_up_to_192_rows(ops):
-    """From 96 rows on a bfloat16 product is the vendor library's, except those whose K is at least their width and
-    whose weights are 32 MB or more, up to 192 rows: the shared-rows kernel takes them, split, and the result is right."""
+    """Where the tiles are not asked (tuned library algorithms, rows that they do not take) a bfloat16 product of 96 rows and more is the
+    vendor library's, except those whose K is at least their width and whose weights are 32 MB or more, up to 192 rows: this
+    package's kernel takes them, split, and the result is right."""
     assert ops._library_takes(128, 2048, 5632) and ops._library_takes(96, 6144, 4096)          # 23 MB; wider than K
     assert not ops._library_takes(128, 4096, 4096) and not ops._library_takes(192, 4096, 14336)
     assert ops._library_takes(193, 4096, 4096) and not ops._library_takes(95, 2048, 2048)
@@ -783,8 +782,8 @@ def test_long_k_products_of_wide_models_stay_with_this_packages_kernel_up_to_192
 @pytest.mark.parametrize("mode", ["off", "heuristic", "all"])
 @pytest.mark.parametrize("M,N,K", [(96, 192, 320), (200, 2560, 512), (333, 328, 136)])
 def test_library_product_with_each_choice_of_algorithm(ops, mode, M, N, K):
-    """Many-row products go to the vendor library; which of its algorithms runs is its heuristic's first
-    choice, or the fastest of the timed candidates whose result agrees with that one's.  Whatever was
+    """Many-row products that the tiles do not take, or for which tuned algorithms are asked, go to the vendor library; which
+    of its algorithms runs is its heuristic's first choice (here at 333 rows), or the fastest of the timed candidates whose result agrees with that one's.  Whatever was
     chosen, the product is x w^T, the choice is made once per shape, and a view with a row stride works."""
     rng = np.random.default_rng(M + N + K)
     x = _bf16_grid(rng.normal(size=(M, K)))
