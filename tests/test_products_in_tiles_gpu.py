@@ -107,6 +107,8 @@ def test_every_tile_gated(ops, tile):
         _run(ops, x, w, None, gu, tile=tile)
         ops.swiglu(gu, want)
         assert (out == want).float().mean() > 0.98
+        # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each
+        assert bool(((out.double() - exact).abs() <= 1.1 * bound + 4.2 * 2.0 ** -8 * g.abs() * u.abs()).all())
         _run(ops, x, w, None, out, gated=1, limit=0.5, tile=tile, N=I)
         gc, uc = g.clamp(max=0.5), u.clamp(-0.5, 0.5)
         clamped = gc * torch.sigmoid(1.702 * gc) * (uc + 1)
@@ -190,6 +192,9 @@ def test_many_rows_go_to_the_tiles_where_the_rule_says_so(ops, M, N, K, mine):
     if ops._tiles_take(M, N // 2, K, 1, gated=True):
         ops.swiglu(ops.gemm(x, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV)), plain)
         assert (act == plain).float().mean() > 0.98
+        # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each
+        g, u = (x.double() @ w.double().t()).split(N // 2, 1)
+        assert bool(((act.double() - g * torch.sigmoid(g) * u).abs() <= 4.2 * 2.0 ** -8 * g.abs() * u.abs() + 1e-4).all())
 
 
 @pytest.mark.parametrize("tile", range(7))

@@ -64,13 +64,14 @@ def _noalloc(clib, x, w, out_dtype):
     return rc, out
 
 
-# (M, N, K) pairs: a first call and a smaller second one.  The first of each pair splits K (the
-# column tiles alone do not fill the chip); both forms of the kernel: the one whose waves share the
-# rows through LDS (widths that are multiples of 64), and the one whose every tile reads them itself.
+# (M, N, K) pairs: a first call and a smaller second one.  Both kernels: products in tiles (widths that are multiples of
+# 64) and the one whose every 16 columns read the rows themselves.  The last two pairs go through the built-in array in both calls; of
+# the others, which split K where a consumer adds the slices, only the second's first call: one slice is the faster whole.
 _PAIRS = [
     ((8, 2048, 2048), (3, 512, 1024)),
     ((64, 2048, 5632), (24, 1024, 512)),
     ((16, 2560, 2048), (1, 2560, 2048)),
+    ((64, 2048, 5632), (33, 512, 8192)),
     ((8, 2064, 2048), (3, 528, 1024)),
 ]
 
@@ -78,7 +79,7 @@ _PAIRS = [
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("first,second", _PAIRS)
 def test_two_calls_in_a_row_equal_the_ordinary_split_product(ops, clib, first, second, out_dtype):
-    splits = []
+    splits, whole = [], [ops.lib().kvcm_gemm_skinny_whole_splits(*shape) for shape in (first, second)]
     for seed, (M, N, K) in enumerate((first, second)):
         x, w = _operands(seed, M, N, K)
         want, S = _existing(ops, x, w, out_dtype)
@@ -93,7 +94,9 @@ def test_two_calls_in_a_row_equal_the_ordinary_split_product(ops, clib, first, s
         ref = x.float().cpu().numpy().astype(np.float64) @ w.float().cpu().numpy().astype(np.float64).T
         tol = 2e-2 * np.abs(ref).max() if out_dtype == torch.bfloat16 else 1e-4 * np.abs(ref).max()
         np.testing.assert_allclose(got.float().cpu().numpy(), ref, atol=tol, rtol=0)
-    assert splits[0] > 1, "the first call of a pair is meant to go through the built-in array"
+    assert splits[0] > 1
+    if (first, second) in _PAIRS[-2:]:
+        assert min(whole) > 1, "both calls are meant to go through the built-in array"
 
 
 def test_products_beyond_the_built_in_array_are_refused(ops, clib):
