@@ -9,8 +9,8 @@
 // W into registers, its own trips double-buffered / this one):
 //   64 rows   2560 x 2048 7.5 / 5.1   2048 x 2048 6.4 / 4.7   gate+up 11264 x 2048 19.6 / 13.2   2048 x 5632 10.9 / 8.0
 //   16 rows   5.1 / 4.2   4.9 / 4.0   13.0 / 11.1   8.1 / 6.6;  128 rows of 4096 x 14336 39.3 / 27.1
-// and against the vendor's product (gate+up: with the launch that applies SwiGLU): 512 rows 14.5 / 9.4 (2048 x 2048), 36.7 / 30.6,
-// 26.4 / 19.5; 1,024 rows 57.7 / 48.1 (gate+up); 2,048 rows 97.8 / 92.1 (gate+up), 21.7 / 21.3, 55.6 / 54.1.
+// and against the vendor's product (gate+up: with the launch that applies SwiGLU): 512 rows 35.1 / 32.9 (gate+up), 29.9 / 26.1 (2048 x 5632,
+// with the norm that adds the slices); 1,024 rows 56.7 / 49.9 (gate+up); where the line lies: kvcm_gemm_tiles_preferred, below.
 #include <cmath>
 
 #include "common.h"
@@ -244,10 +244,14 @@ static int best_tile(int M, int wrows, int K, int S, float* time = nullptr) {
   return best;
 }
 
+static float stored_time(int M, int N, int S, bool out_f32) {
+  return static_cast<float>(M) * static_cast<float>(N) * (S > 1 ? 4.f * S : out_f32 ? 4.f : 2.f) * 0.12e-6f;
+}
+
 float gemm_tiles_time(int M, int N, int K, int S, bool is_gated, bool out_f32) {
   float t = 0.f;
   best_tile(M, is_gated ? 2 * N : N, K, S, &t);
-  return t + static_cast<float>(M) * static_cast<float>(N) * (S > 1 ? 4.f * S : out_f32 ? 4.f : 2.f) * 0.12e-6f;      // what is stored
+  return t + stored_time(M, N, S, out_f32);
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, class Offset = uint32_t>
@@ -311,22 +315,33 @@ int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, in
 }
 
 // Is a product of many rows, in S slices of K that its consumer adds, faster here than by the vendor library (is_gated: than that and
-// the launch that applies SwiGLU)?  Up to 256 rows it was at 39 of 41 shapes measured (0.43 to 0.87 of the time, two 1.01), beyond 2,048 the
-// library's own tiles of 256 x 256 are (32,768 rows: 1,306 / 1,269 us gate+up of 5632 x 2048, 659 / 513 us 2048 x 5632).  In between, the
-// tiles' time and the slices' reading against about what the library takes: 14 us and 1,350 TFLOP/s (22 us and 1,600 for the largest),
-// and at least 0.3 us for 64 k of a chain that it does not cut.  The six constants were fitted to 76 shapes; what the rule picks is 1.1 %
-// slower than the better of the two on average, 12 % at worst.  (us, here / library: 512 x 2048 x 5632 22.8 / 26.4; 1,024 rows gate+up
-// 48.1 / 57.7; 2,048 rows 92.1 / 97.8; not taken: 768 x 6144 x 4096 55.0 / 48.2, 2048 x 2560 x 2048 30.7 / 27.5.)
+// the launch that applies the activation)?  Beyond 2,048 rows the library's own tiles of 256 x 256 are (32,768 rows: 1,306 / 1,269 us gate+up
+// of 5632 x 2048, 659 / 513 us 2048 x 5632).  Up to there the tiles' time against about what the library takes.  Here: the launch as the tile was
+// picked, with what that model leaves out, the rows of X that every column of tiles reads again (10 TB/s), and the slices' reading (4.5 TB/s,
+// and 55 KB a us of one row's through the CU that norms it).  There: 8.3 us, or 1.6 us, 0.21 us for 64 k of a chain and 1,520 TFLOP/s, or, where
+// few results let it cut K, 8.3 us and 0.029 us for 64 k of 131,072 results; and 4 us and 6 bytes a result for the second launch.
+// Up to 256 rows the library is often far above that, so that it has to be 1.3 times as fast.
+// The constants were fitted to 2,177 plain products (64 to 32,000 columns, K 256 to 14,336; 1,032 of them with the norm that adds the slices
+// too) and 1,937 gated ones (64 to 14,336 columns), 96 to 2,048 rows.  What the rule picks takes 0.80, 0.75 and 0.73 of the library's time on average and
+// is 1.9, 1.0 and 0.7 % slower than the better of the two; slower than the library by more than 8 % are 17, 11 and 37 of them, the worst where
+// few columns of long K are cut by it and not here: 256 x 1024 x 4096 13.4 / 10.1 us, gated 2048 x 128 x 4096 21.9 / 16.3.  (us, here / library:
+// 512 x 2048 x 5632 with the norm 26.1 / 29.9, 1024 x 1024 x 512 5.0 / 8.9; 1,024 rows gate+up of 5632 x 2048 49.9 / 56.7; not taken: 640 x 64 x 14336 29.5 / 13.3, 2048 x 256 x 5632 28.9 / 17.4,
+// 1024 x 8192 x 2048 36.9 / 34.3.)
 int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype) {
   if (M <= 0 || N <= 0 || N % 64 != 0 || K <= 0 || K % kStepK != 0 || S < 1 || S > K / kStepK || (is_gated && S > 1)) return 0;
-  if (M <= 256) return 1;
   if (M > 2048) return 0;
-  const float mn = static_cast<float>(M) * static_cast<float>(N);
-  const float here = gemm_tiles_time(M, N, K, S, is_gated != 0, out_dtype == kF32) + (S > 1 ? mn * (4.f * S - 2.f) / 4.5e6f : 0.f);
-  const float gflop = mn * static_cast<float>(K) * (is_gated ? 4e-9f : 2e-9f);
-  const float rate = std::fmin(14.f + gflop / 1.35f, 22.f + gflop / 1.6f), chain = 4.f + 0.3f * static_cast<float>(K / kStepK);
-  const float library = std::fmax(rate, chain) + (is_gated ? 3.f + mn * 6.f / 5e6f : 0.f);
-  return here <= library;
+  const float m = static_cast<float>(M), n = static_cast<float>(N), k = static_cast<float>(K), steps = static_cast<float>(K / kStepK);
+  const int wrows = is_gated ? 2 * N : N;
+  float t = 0.f;
+  const Tile& tile = kTiles[best_tile(M, wrows, K, S, &t)];
+  const float again = 2.3f + m * k * 2e-7f * static_cast<float>((wrows + tile.bn - 1) / tile.bn);
+  const float t2 = t * t, again2 = again * again;
+  const float here = std::sqrt(std::sqrt(t2 * t2 + again2 * again2)) + stored_time(M, N, S, out_dtype == kF32) +
+                     (S > 1 ? m * n * (4.f * S - 2.f) / 4.5e6f + n * 4.f * S / 55e3f : 0.f);
+  const float results = m * static_cast<float>(wrows);
+  const float whole = 1.6f + 0.21f * steps + results * k * 2e-9f / 1.52f, cut = 8.3f + 0.029f * steps * results / 131072.f;
+  const float library = std::fmax(8.3f, std::fmin(whole, cut)) + (is_gated ? 4.f + m * n * 6.f / 5e6f : 0.f);
+  return here <= (M <= 256 ? 1.3f : 1.f) * library;
 }
 
 }  // extern "C"

@@ -174,8 +174,8 @@ def test_gated_products_of_rows_far_apart(ops, M, I, K):
         assert bool(((out.double() - want).abs() <= 4.2 * 2.0 ** -8 * (g * scale).abs() * (u * scale).abs() + 1e-5).all())
 
 
-@pytest.mark.parametrize("M,N,K,mine", [(96, 2048, 2048, True), (200, 2560, 2048, True), (333, 2048, 5632, True), (700, 2048, 2048, True),
-                                        (1024, 2048, 2048, True), (1536, 8192, 2048, False), (2000, 192, 128, None), (768, 2048, 5632, None), (1000, 192, 8192, None)])
+@pytest.mark.parametrize("M,N,K,mine", [(96, 2048, 2048, True), (200, 2560, 2048, True), (333, 2048, 5632, True), (700, 2048, 2048, False),
+                                        (700, 512, 1024, True), (1024, 1536, 512, True), (640, 64, 14336, False), (2000, 256, 5632, False), (1536, 8192, 2048, False), (2000, 192, 128, None), (768, 2048, 5632, None), (1000, 192, 8192, None)])
 def test_many_rows_go_to_the_tiles_where_the_rule_says_so(ops, M, N, K, mine):
     x, w = _operands(M, M, N, K)
     for dtype in (torch.bfloat16, torch.float32):
