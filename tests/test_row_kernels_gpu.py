@@ -7,7 +7,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H", [4, 8, 12, 2048, 2056, 4104])
+@pytest.mark.parametrize("H", [4, 8, 12, 256, 260, 264, 2048, 2056, 4104])      # (pieces beyond 256)
 def test_embedding_by_pieces_gathers_rows(H, dtype):
     from kvcm_amd import ops
     V = 37
