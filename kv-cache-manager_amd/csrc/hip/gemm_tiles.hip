@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(WM* WN* kWave)
     offset[q] = static_cast<Offset>(at) * static_cast<Offset>(ld) * 2u + static_cast<Offset>(Ring::piece_of(lane)) * 16u;
   }
   // One row block: workgroups walk their slice from different places (and wrap around), or all would ask the same few memory
-  // channels for rows a multiple of 4 KB apart at the same time (gate+up, 64 rows: 14.9 -> 14.4 us).  Several: those that share
+  // channels for rows a multiple of 4 KB apart at the same time.  Several: those that share
   // columns walk together.
   const int phase = tiles_m == 1 ? tn * 5 % steps : 0;
   auto base = [&](int req) {
@@ -324,7 +324,8 @@ int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, in
 // The constants were fitted to 2,177 plain products (64 to 32,000 columns, K 256 to 14,336; 1,032 of them with the norm that adds the slices
 // too) and 1,937 gated ones (64 to 14,336 columns), 96 to 2,048 rows.  What the rule picks takes 0.80, 0.75 and 0.73 of the library's time on average and
 // is 1.9, 1.0 and 0.7 % slower than the better of the two; slower than the library by more than 8 % are 17, 11 and 37 of them, the worst where
-// few columns of long K are cut by it and not here: 256 x 1024 x 4096 13.4 / 10.1 us, gated 2048 x 128 x 4096 21.9 / 16.3.  (us, here / library:
+// few columns of long K are cut by it and not here: 256 x 1024 x 4096 13.4 / 10.1 us, gated 2048 x 128 x 4096 21.9 / 16.3.  At 3,142 further ones, of
+// row counts between those: 0.83 and 0.76, 2.7 and 1.3 %, 14 and 19.  (us, here / library:
 // 512 x 2048 x 5632 with the norm 26.1 / 29.9, 1024 x 1024 x 512 5.0 / 8.9; 1,024 rows gate+up of 5632 x 2048 49.9 / 56.7; not taken: 640 x 64 x 14336 29.5 / 13.3, 2048 x 256 x 5632 28.9 / 17.4,
 // 1024 x 8192 x 2048 36.9 / 34.3.)
 int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype) {

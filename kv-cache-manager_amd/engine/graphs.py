@@ -27,9 +27,9 @@ import torch
 from .runner import StepContext
 
 # Decode-shaped steps of more rows replay their program without a graph, and with the library's
-# products, which a graph may not hold: measured at TinyLlama sizes, graph with this package's products
-# against program with the library's: 96 rows 1.94 / 2.14 ms, 128 rows 2.15 / 2.20, 192 rows 2.87 / 2.62,
-# 256 rows 3.21 / 2.88 (beyond 128 rows this package's kernel streams the weights once per 128 rows).
+# products where those are the faster, which a graph may not hold.  The line was drawn where graphs had a kernel that read the
+# weights once per 128 rows; at TinyLlama sizes, graph / program: 96 rows 1.55 / 1.56 ms, 128 rows 1.58 / 1.60, 192 rows 1.81 /
+# 1.84, 256 rows 2.01 / 2.07 (a capture takes some 8 ms per batch bucket and context class).
 GRAPH_ROWS = 128
 
 

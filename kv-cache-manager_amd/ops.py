@@ -508,14 +508,12 @@ def add_residual(x, y):
 # Rows from which a bfloat16 product may be handed to the library (hipBLASLt, called directly:
 # csrc/hip/gemm_library.hip); the reference leaves every product to its vendor library.  0 = always
 # use the kernels of this package.  From here on a product runs in this package's tiles where those are the faster
-# (``_tiles_take``: up to 256 rows, and beyond by the shape), or where they are refused by the library's.
+# (``_tiles_take``), or else by the library's.
 LIBRARY_GEMM_MIN_ROWS = 96
-# ... except that up to LIBRARY_LONG_K_MIN_ROWS - 1 rows this package's kernel keeps the products whose K is
+# ... except that up to LIBRARY_LONG_K_MIN_ROWS - 1 rows this package's kernels keep the products whose K is
 # at least their width and whose weights are at least LIBRARY_LONG_K_BYTES (the O and down projections of 7B /
-# 8B sizes): the library's first choice is slow there.  Measured at Llama-3-8B sizes, library against this
-# package's kernel: down 74.9 / 44.3 us at 128 rows, 102 / 69 at 192, 61.5 / 72.5 at 256; O 23.1 / 19.3 at 128,
-# 31.9 / 26.6 at 192, 21.9 / 28.6 at 256; a prompt step of 128 rows 7.15 -> 6.38 ms.  TinyLlama's down projection
-# (23 MB) is the library's at every row count from 96 on (12.9 / 16.4 us at 128 rows).
+# 8B sizes), tuned or not: the library's first choice is slow there.  Measured at Llama-3-8B sizes, library / this
+# package's tiles (the kernel before them): down at 128 rows 74.9 / 33.0 us (44.3), 192 rows 102 / 43.0 (69); O 23.1 / 16.7 (19.3), 31.9 / 21.1 (26.6).
 LIBRARY_LONG_K_MIN_ROWS = 193
 LIBRARY_LONG_K_BYTES = 32 << 20
 
