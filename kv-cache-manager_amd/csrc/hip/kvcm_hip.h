@@ -84,6 +84,16 @@ int kvcm_gemm8(const void* X, int ldx, const void* W, int ldw, int M, int N, int
                float eps, void* out, int out_dtype, int ldo, int swiglu, hipStream_t stream);
 int kvcm_gemm8_residual_norm(const void* X, int ldx, const void* W, int ldw, int M, int N, int K, float* resid,
                              const void* g, int g_dtype, void* xg, float* ss_out, hipStream_t stream);
+// The attention half of a decoding layer of at most 8 rows in one launch (decode_front.hip): QKV product, rotation, page write,
+// attention, output product, residual addition and the next norm's preparation, handed on through two buffers in turn.
+int kvcm_decode_front_supported(int M, int H, int nh, int nkv, int hd, int B);
+int kvcm_decode_front_parts(int max_context);
+long long kvcm_decode_front_words(int M, int nh, int nkv, int hd, int parts);
+int kvcm_decode_front_empty(uint32_t* words, long long n, hipStream_t stream);
+int kvcm_decode_front(const void* X, int ldx, const void* Wqkv, int ldqkv, const float* ss_in, int tiles_in, float eps, const void* Wo, int ldo,
+                      int M, int H, const float* cos_sin, const int* slots, void* kcache, void* vcache, const int* tables, int table_stride,
+                      int seqs, const int* row_seq, const int* ctx_lens, int nh, int nkv, int hd, int B, float scale, float* resid, const void* g,
+                      int g_dtype, void* xg, float* ss_out, uint32_t* now, uint32_t* next, long long words, int parts, hipStream_t stream);
 // The vendor library's product (hipBLASLt), bfloat16 operands and result, 32-bit accumulation, for
 // the many-row products of prompt steps, where the reference calls cuBLAS (src/model/llama.cpp:45-52).
 // `workspace` is device memory the caller owns (at least kvcm_gemm_library_workspace_bytes()).

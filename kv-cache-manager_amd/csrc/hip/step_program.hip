@@ -87,6 +87,8 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_gemm_library_f32out),
     KVCM_ENTRY(kvcm_gemm8),
     KVCM_ENTRY(kvcm_gemm8_residual_norm),
+    KVCM_ENTRY(kvcm_decode_front_empty),
+    KVCM_ENTRY(kvcm_decode_front),
     KVCM_ENTRY(kvcm_attention_generic),
     KVCM_ENTRY(kvcm_attention_decode),
     KVCM_ENTRY(kvcm_attention_decode_fused),

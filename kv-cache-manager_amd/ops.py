@@ -46,6 +46,13 @@ def _declare(lib):
     fn("kvcm_attention_decode_fused_info", i, i, i, vp)
     fn("kvcm_gemm_skinny_swiglu_supported", i, i, i)
     fn("kvcm_gemm_skinny_swiglu", vp, vp, vp, i, i, i, i, i, i, i, f, vp)
+    fn("kvcm_decode_front_supported", i, i, i, i, i, i)
+    fn("kvcm_decode_front_parts", i)
+    lib.kvcm_decode_front_words.restype = C.c_longlong
+    lib.kvcm_decode_front_words.argtypes = [i] * 5
+    fn("kvcm_decode_front_empty", vp, C.c_longlong, vp)
+    fn("kvcm_decode_front", vp, i, vp, i, vp, i, f, vp, i, i, i, vp, vp, vp, vp, vp, i, i, vp, vp, i, i, i, i, f, vp, vp, i, vp, vp, vp, vp,
+       C.c_longlong, i, vp)
     fn("kvcm_gemm_skinny_splits", i, i, i)
     fn("kvcm_gemm_skinny_whole_splits", i, i, i)
     fn("kvcm_gemm_tiles_count")
@@ -368,6 +375,78 @@ class PendingProduct:
         return self.run(False)
 
 
+class PendingAttention(PendingProduct):
+    """An attention half of a layer that has not run yet: QKV product, rotation, page write, attention and output product, of at most
+    8 rows of different sequences.  ``gemm_residual_norm`` runs all of it in one launch (csrc/hip/decode_front.hip) where that takes
+    the operands; ``run`` the ordinary way: ``attend()`` leaves the attention's rows in ``x``, then the output product.
+    h: the normed rows or NormedRows; handover: (a function that gives the launch its two buffers) see ``decode_front_buffers``."""
+
+    def __init__(self, attend, h, wqkv, x, w, out, scratch, cache, tables, table_stride, row_seq, ctx_lens, slots, cos_sin, heads, scale, parts, handover):
+        super().__init__(x, w, out, scratch)
+        self.attend, self.h, self.wqkv, self.cache, self.tables, self.table_stride = attend, h, wqkv, cache, tables, table_stride
+        self.row_seq, self.ctx_lens, self.slots, self.cos_sin, self.heads, self.scale = row_seq, ctx_lens, slots, cos_sin, heads, scale
+        self.parts, self.handover = parts, handover
+
+    def run(self, keep_partial=False):
+        self.attend()
+        return super().run(keep_partial)
+
+    def takes(self, x, xg, ss):
+        h = self.h.xg if isinstance(self.h, NormedRows) else self.h
+        return (_in_pieces(h, self.wqkv, self.w) and h.data_ptr() != xg.data_ptr() and x.shape == (h.shape[0], self.w.shape[0])
+                and not (isinstance(self.h, NormedRows) and self.h.ss.data_ptr() == ss.data_ptr()))
+
+    def run_with_norm(self, x, weight, eps, xg, ss, out):
+        normed = isinstance(self.h, NormedRows)
+        h = self.h.xg if normed else self.h
+        nh, nkv, hd = self.heads
+        kc, vc = self.cache
+        M, H = x.shape
+        _dev(h, self.wqkv, self.w, x, weight, xg, ss, kc, vc)
+        for t, n in ((h, "h"), (self.wqkv, "wqkv"), (self.w, "wo")):
+            _rows2d(t, n)
+            _need(t.dtype == torch.bfloat16, "decode_front needs bfloat16 operands")
+        _need(self.wqkv.shape == ((nh + 2 * nkv) * hd, H) and self.w.shape == (H, nh * hd) and h.shape == (M, H), "decode_front: projections of other shapes")
+        _need(x.dtype == torch.float32 and x.is_contiguous(), "the residual stream must be contiguous float32 [M, H]")
+        _need(weight.numel() == H and weight.is_contiguous(), "norm weight must have H entries")
+        _need(xg.dtype == torch.bfloat16 and xg.is_contiguous() and xg.shape[0] >= M and xg.shape[1] == H, "xg must be bfloat16 [>= M, H]")
+        _need(ss.dtype == torch.float32 and ss.is_contiguous() and ss.shape[0] >= M and ss.shape[1] == H // 8, "ss must be float32 [>= M, H / 8]")
+        B = kc.shape[2]
+        _need(kc.dtype == vc.dtype == torch.bfloat16 and kc.is_contiguous() and vc.is_contiguous() and tuple(kc.shape[1:]) == (nkv, B, hd)
+              and tuple(vc.shape[1:]) == (nkv, hd, B), "caches must be bfloat16 [pages, nkv, block_size, hd] and [pages, nkv, hd, block_size]")
+        for t, n in ((self.slots, "slots"), (self.row_seq, "row_seq"), (self.ctx_lens, "ctx_lens")):
+            _i32(t, n, M)
+        _i32(self.tables, "tables", self.table_stride)
+        if self.cos_sin is not None:
+            _need(self.cos_sin.dtype == torch.float32 and self.cos_sin.is_contiguous() and self.cos_sin.numel() >= M * hd, "cos_sin must be float32 [rows, head_dim/2, 2]")
+        now, after = self.handover()
+        _call("kvcm_decode_front", _ptr(h), h.stride(0), _ptr(self.wqkv), self.wqkv.stride(0), _ptr(self.h.ss) if normed else 0,
+              self.h.ss.shape[1] if normed else 0, self.h.eps if normed else 0.0, _ptr(self.w), self.w.stride(0), M, H, _ptr(self.cos_sin),
+              _ptr(self.slots), _ptr(kc), _ptr(vc), _ptr(self.tables), self.table_stride, self.tables.numel() // self.table_stride,
+              _ptr(self.row_seq), _ptr(self.ctx_lens), nh, nkv, hd, B, float(self.scale), _ptr(x), _ptr(weight), _DT[weight.dtype], _ptr(xg),
+              _ptr(ss), _ptr(now), _ptr(after), now.numel(), self.parts, _stream())
+        return NormedRows(xg[:M], ss[:M], eps, x, weight, out)
+
+
+def decode_front_parts(M, H, nh, nkv, hd, block_size, max_context):
+    """Workgroups per row and KV head of the launch above for contexts of up to max_context tokens, 0 where it does not take the shape."""
+    return lib().kvcm_decode_front_parts(max_context) if lib().kvcm_decode_front_supported(M, H, nh, nkv, hd, block_size) else 0
+
+
+def decode_front_buffers(step, M, nh, nkv, hd, parts):
+    """The two hand-over buffers of a step's next such launch: the one it reads, which is empty, and the one it empties for the launch
+    after it.  They change places from launch to launch; the first of a step is emptied here."""
+    words = lib().kvcm_decode_front_words(M, nh, nkv, hd, parts)
+    both = step.flat("decode_front", 2 * words, torch.int32)[:2 * words].view(2, words)
+    key = ("decode_front", words, nh, nkv, hd, parts)
+    n = step.shared.get(key, 0)
+    step.shared[key] = n + 1
+    if n == 0 or step.shared.get("decode_front_last") != key:      # (layers of other sizes share the buffer)
+        _call("kvcm_decode_front_empty", _ptr(both[n % 2]), words, _stream())
+    step.shared["decode_front_last"] = key
+    return both[n % 2], both[1 - n % 2]
+
+
 class NormedRows:
     """The rows a product after an RMS norm multiplies, with the norm's scale still to be applied:
     ``xg`` = round(g * round(x)) [rows, H] and ``ss`` [rows, H / 8] sums of x^2 per 8-column tile, left
@@ -389,6 +468,10 @@ def gemm_residual_norm(product, x, weight, eps, xg, ss, out):
     half of the folded norm.  product: PendingProduct of at most 8 bfloat16 rows; x: the 32-bit residual
     stream [rows, H]; xg [>= rows, H] bfloat16 and ss [>= rows, H / 8] float32 receive the result; out:
     where ``materialize`` would put ordinary normed rows."""
+    if isinstance(product, PendingAttention):
+        if product.takes(x, xg, ss):
+            return product.run_with_norm(x, weight, eps, xg, ss, out)
+        product.attend()
     a, w = product.x, product.w
     M, K = a.shape
     H = w.shape[0]

@@ -313,6 +313,9 @@ class PositionEncoding(Part):
 class Mixer(Part):
     # True: ``h`` may be a Deferred (ops.NormedRows) that the mixer's first product consumes as it is.
     accepts_normed_rows = False
+    # True: ``forward`` takes ``defer=True``, passed by a block whose norm behind the mixer folds and runs next, before anything else
+    # touches what the mixer reads or writes: the mixer may then return an ops.PendingProduct none of whose launches has run yet.
+    defers = False
 
     def forward(self, step, h):
         """h: normed hidden states [rows, H] in the compute dtype -> the mixer's output [rows, H]."""

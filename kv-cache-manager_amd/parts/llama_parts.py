@@ -132,6 +132,7 @@ class GQAAttention(Mixer):
 
     capturable = True
     accepts_normed_rows = True
+    defers = True
 
     def sub_parts(self):
         return (self.position,)
@@ -168,7 +169,32 @@ class GQAAttention(Mixer):
         # the two projections, and q.k and p.v over every (row, key) pair of every query head
         return super().flops(rows) + 4.0 * attended * self.hd * self.nh
 
-    def forward(self, step, h):
+    def forward(self, step, h, defer=False):
+        wo = self.w["wo"]
+        parts = self._one_launch_parts(step, h) if defer else 0
+        if not parts:
+            return _to_residual(self.ctx, step, self._attention(step, h), wo, "mixer_out")
+        ops, g = self.ctx.ops, self.cache.group
+        table = self.position.rotation_table(step, self.hd) if self.position.rotates else None
+        return ops.PendingAttention(
+            lambda: self._attention(step, h), h, self.w["wqkv"], step.ws("attn", (step.rows, self.q_dim)), wo,
+            step.ws("mixer_out", (step.rows, wo.shape[0])), step.scratch("mixer_out", step.rows, wo.shape[0], wo.shape[1]),
+            (self.cache.k(self.cache_index), self.cache.v(self.cache_index)), step.tables(g), step.table_stride(g), step.row_seq, step.ctx_lens,
+            step.slots(g), table, (self.nh, self.nkv, self.hd), self.scale, parts,
+            lambda: ops.decode_front_buffers(step, step.rows, self.nh, self.nkv, self.hd, parts))
+
+    def _one_launch_parts(self, step, h):
+        """How the step's attention half is cut where it can be one launch with the norm that follows (ops.PendingAttention), else 0."""
+        ops = self.ctx.ops
+        if not (step.fold_norms and step.max_run == 1 and step.attention_mode == "auto" and self.window == 0 and self.cache_owner
+                and h.dtype == torch.bfloat16 and step.rows <= min(ops.FUSED_NORM_MAX_ROWS, step.fold_rows)):
+            return 0
+        if self.position.rotates and self.position.rotation_table(step, self.hd) is None:
+            return 0
+        return ops.decode_front_parts(step.rows, self.ctx.hidden_size, self.nh, self.nkv, self.hd, self.ctx.block_size, step.max_context_bound)
+
+    def _attention(self, step, h):
+        """The attention's rows, in the work buffer ``attn``."""
         ops = self.ctx.ops
         g = self.cache.group
         kc, vc = self.cache.k(self.cache_index), self.cache.v(self.cache_index)
@@ -183,7 +209,7 @@ class GQAAttention(Mixer):
         table = pos.rotation_table(step, self.hd) if pos.rotates else None
         if (table is not None or not pos.rotates) and paged_attention.attend_from_projection(
                 step, ops, res, attn, kc, vc, g, self.nh, self.nkv, self.hd, self.scale, self.window, table, slots):
-            return _to_residual(self.ctx, step, attn, self.w["wo"], "mixer_out")
+            return attn
         extra = {"source": res} if hasattr(res, "materialize") else {}
         stored = pos.apply(step, qkv, self.nh, self.nkv, self.hd,
                            cache=(kc, vc) if self.cache_owner else None, slots=slots, **extra)
@@ -191,7 +217,7 @@ class GQAAttention(Mixer):
             ops.rope_cache(qkv, self.nh, self.nkv, self.hd, slots=slots, kcache=kc, vcache=vc,
                            block_size=self.ctx.block_size, rows=step.rows)
         paged_attention.attend(step, ops, qkv, attn, kc, vc, g, self.nh, self.nkv, self.hd, self.scale, self.window)
-        return _to_residual(self.ctx, step, attn, self.w["wo"], "mixer_out")
+        return attn
 
 
 @FEED_FORWARDS.register("swiglu")
@@ -286,6 +312,8 @@ class PreNormResidual(Block):
         fold1 = {"defer": True} if (n1.defers and mixer.accepts_normed_rows) else {}
         fold2 = {"defer": True} if (n2.defers and ffn.accepts_normed_rows) else {}
         h = n1.forward(x, buf, add=pending if n1.accepts_partial_sums else as_tensor(pending), **fold1)
-        a = mixer.forward(step, buf if h is None else h)
+        # a mixer may leave all of its launches to the norm behind it (Mixer.defers), which runs at once
+        late = {"defer": True} if (n2.defers and n2.accepts_partial_sums and mixer.defers and fold2) else {}
+        a = mixer.forward(step, buf if h is None else h, **late)
         h = n2.forward(x, buf, add=a if n2.accepts_partial_sums else as_tensor(a), **fold2)
         return ffn.forward(step, buf if h is None else h)
