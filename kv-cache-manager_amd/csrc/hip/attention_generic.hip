@@ -135,12 +135,14 @@ using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 template <int NT>      // head size / 16
 constexpr int f32_waves() { return NT <= 4 ? 8 : 4; }      // (a wave's share of the output lies in LDS: 1 KB a tile, 32 KB in all)
 
-template <int NT>
+// STORES: q are rows of the projection [q | k | v], every row of a sequence of its own; its key and value go to their slot first, q and k
+// rotated by cos_sin [T][hd / 2] (null: not), with the operations of the rotation's own kernel: a launch and 4 to 5 us a layer less.
+template <int NT, bool STORES>
 __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
     attention_f32_kernel(const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
-                         const float* __restrict__ kcache, const float* __restrict__ vcache, const int* __restrict__ tables,
+                         const float* kcache, const float* vcache, const int* __restrict__ tables,
                          int table_stride, const int* __restrict__ row_seq, const int* __restrict__ ctx_lens, int T, int nh, int nkv,
-                         int rows_per_tile, int B, float scale, int window) {
+                         int rows_per_tile, int B, float scale, int window, const float2* __restrict__ cos_sin, const int* __restrict__ slots) {
   constexpr int WAVES = f32_waves<NT>(), hd = 16 * NT;
   __shared__ f32x4 part_o[WAVES][16][NT * 4];
   __shared__ float part_m[WAVES][16], part_l[WAVES][16];
@@ -157,8 +159,59 @@ __global__ void __launch_bounds__(f32_waves<NT>() * kWave)
   const int seqs = row_seq[r0 + (lane < rows ? lane : 0)], ctxs = ctx_lens[r0 + (lane < rows ? lane : 0)];
   f32x4 qf[NT];
 #pragma unroll
-  for (int u = 0; u < NT; ++u)
-    qf[u] = *reinterpret_cast<const f32x4*>(q + size_t(row) * q_stride + size_t(head) * hd + 16 * u + 4 * g) * scale;
+  for (int u = 0; u < NT; ++u) qf[u] = *reinterpret_cast<const f32x4*>(q + size_t(row) * q_stride + size_t(head) * hd + 16 * u + 4 * g);
+  if constexpr (STORES) {
+    constexpr int half = hd / 2;
+    if (cos_sin) {
+      const float2* angle = cos_sin + size_t(row) * half;
+      if constexpr (NT == 1) {      // dims 4 g + e: the partner's lane is 32 away
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float2 t = angle[4 * (g & 1) + e];
+          const float there = __shfl_xor(qf[0][e], 32, kWave);
+          float a = g < 2 ? qf[0][e] : there, b = g < 2 ? there : qf[0][e];
+          rotate_pair(a, b, t.x, t.y);
+          qf[0][e] = g < 2 ? a : b;
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < NT / 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float2 t = angle[16 * u + 4 * g + e];
+            float a = qf[u][e], b = qf[u + NT / 2][e];
+            rotate_pair(a, b, t.x, t.y);
+            qf[u][e] = a;
+            qf[u + NT / 2][e] = b;
+          }
+      }
+    }
+    for (int i = threadIdx.x; i < rows * hd; i += WAVES * kWave) {      // pairs of k, then pairs of v, of every row
+      const int t = r0 + i / hd, j = i % half, slot = slots[t];
+      const bool is_v = i % hd >= half;
+      if (slot < 0) continue;
+      const float* src = q + size_t(t) * q_stride + size_t(nh + (is_v ? nkv : 0) + kvh) * hd + j;
+      float a = src[0], b = src[half];
+      const size_t page = slot / B;
+      const int off = slot % B;
+      if (is_v) {
+        float* to = const_cast<float*>(vcache) + (page * nkv + kvh) * size_t(hd) * B + off;
+        to[size_t(j) * B] = a;
+        to[size_t(j + half) * B] = b;
+      } else {
+        if (cos_sin) {
+          const float2 c = cos_sin[size_t(t) * half + j];
+          rotate_pair(a, b, c.x, c.y);
+        }
+        float* to = const_cast<float*>(kcache) + ((page * nkv + kvh) * B + off) * hd + j;
+        to[0] = a;
+        to[half] = b;
+      }
+    }
+    __syncthreads();      // stored before any wave of this workgroup, which alone reads them, loads them
+  }
+#pragma unroll
+  for (int u = 0; u < NT; ++u) qf[u] = qf[u] * scale;
 
   const size_t head_stride = size_t(B) * hd, page_stride = head_stride * nkv;
   float m = -INFINITY, l = 0.f;
@@ -322,7 +375,7 @@ bool attention_f32_takes(int nh, int nkv, int hd, int B) {
 template <int NT>
 void launch_attention_f32(const float* q, int q_stride, float* out, int out_stride, const float* kcache, const float* vcache,
                           const int* tables, int table_stride, const int* row_seq, const int* ctx_lens, int T, int nh, int nkv,
-                          int B, float scale, int window, hipStream_t s) {
+                          int B, float scale, int window, const float2* cos_sin, const int* slots, hipStream_t s) {
   // As many rows a workgroup as leave each CU one (the smallest heads' registers allow two), where the 16 items hold them.
   // Single rows of as many sequences, us, the kernel above / a full tile walked by the same wave for each sequence, all keys of a
   // chunk multiplied / this: 32 heads over 32 kv heads of 64, 64 rows of 16 tokens 12.6 / 71.8 / 8.9, of 600 413 / 238 / 123; 256
@@ -330,8 +383,9 @@ void launch_attention_f32(const float* q, int q_stride, float* out, int out_stri
   const long long units = static_cast<long long>(T) * nkv;
   const int per = static_cast<int>(units <= (NT == 1 ? 512 : 256) ? 1 : std::min<long long>((units + 255) / 256, 16 / (nh / nkv)));
   const unsigned blocks = static_cast<unsigned>((T + per - 1) / per) * nkv;
-  attention_f32_kernel<NT><<<blocks, f32_waves<NT>() * kWave, 0, s>>>(q, q_stride, out, out_stride, kcache, vcache, tables, table_stride,
-                                                                      row_seq, ctx_lens, T, nh, nkv, per, B, scale, window);
+  auto* kernel = slots ? attention_f32_kernel<NT, true> : attention_f32_kernel<NT, false>;
+  kernel<<<blocks, f32_waves<NT>() * kWave, 0, s>>>(q, q_stride, out, out_stride, kcache, vcache, tables, table_stride, row_seq, ctx_lens, T, nh, nkv,
+                                                    per, B, scale, window, cos_sin, slots);
 }
 
 }  // namespace kvcm
@@ -373,7 +427,7 @@ extern "C" int kvcm_attention_generic(const void* q, int dtype, int q_stride, vo
     auto* launch = hd == 16 ? launch_attention_f32<1> : hd == 32 ? launch_attention_f32<2> : hd == 64 ? launch_attention_f32<4>
                                                                                               : launch_attention_f32<8>;
     launch(static_cast<const float*>(q), q_stride, static_cast<float*>(out), out_stride, static_cast<const float*>(kcache),
-           static_cast<const float*>(vcache), tables, table_stride, row_seq, ctx_lens, T, nh, nkv, B, scale, window, s);
+           static_cast<const float*>(vcache), tables, table_stride, row_seq, ctx_lens, T, nh, nkv, B, scale, window, nullptr, nullptr, s);
     return launch_status("attention_f32");
   }
   if (dtype == kF32)
@@ -388,4 +442,29 @@ extern "C" int kvcm_attention_generic(const void* q, int dtype, int q_stride, vo
         ctx_lens, items, nh, nkv, hd, B, scale, window);
   else KVCM_REQUIRE(false, "attention: unknown dtype %d", dtype);
   return launch_status("attention_generic");
+}
+
+// 1 when kvcm_attention_f32_decode takes the shape, else 0.
+extern "C" int kvcm_attention_f32_decode_supported(int nh, int nkv, int hd, int B) {
+  return nkv > 0 && nh > 0 && nh % nkv == 0 && B > 0 && attention_f32_takes(nh, nkv, hd, B);
+}
+
+// 32-bit rows of T different sequences, from the projection's rows [q | k | v] to the attention's: q and k rotated by cos_sin [T][hd / 2]
+// (null: not), keys and values stored to slots [T] (negative: not stored).  The bits of kvcm_rope_cache and kvcm_attention_generic; the
+// rows themselves stay as they are.
+extern "C" int kvcm_attention_f32_decode(const float* qkv, int qkv_stride, float* out, int out_stride, const float* cos_sin, const int* slots,
+                                         float* kcache, float* vcache, const int* tables, int table_stride, const int* row_seq, const int* ctx_lens,
+                                         int T, int nh, int nkv, int hd, int B, float scale, int window, hipStream_t s) {
+  if (T == 0) return 0;
+  KVCM_REQUIRE(kvcm_attention_f32_decode_supported(nh, nkv, hd, B), "attention_f32_decode: unsupported shape heads=%d kv_heads=%d head_dim=%d page=%d", nh, nkv, hd, B);
+  KVCM_REQUIRE(T > 0 && static_cast<long long>(T) * nkv < (1ll << 31), "attention_f32_decode: bad row count %d", T);
+  KVCM_REQUIRE(qkv && out && slots && kcache && vcache && tables && row_seq && ctx_lens, "attention_f32_decode: null operand");
+  KVCM_REQUIRE(qkv_stride >= (nh + 2 * nkv) * hd && out_stride >= nh * hd && window >= 0, "attention_f32_decode: row strides too small or a negative window");
+  const auto piece = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  KVCM_REQUIRE(piece(qkv) && qkv_stride % 4 == 0 && piece(kcache) && piece(vcache) && reinterpret_cast<uintptr_t>(cos_sin) % 8 == 0,
+               "attention_f32_decode: operands must be 16-byte aligned");
+  auto* launch = hd == 16 ? launch_attention_f32<1> : hd == 32 ? launch_attention_f32<2> : hd == 64 ? launch_attention_f32<4> : launch_attention_f32<8>;
+  launch(qkv, qkv_stride, out, out_stride, kcache, vcache, tables, table_stride, row_seq, ctx_lens, T, nh, nkv, B, scale, window,
+         reinterpret_cast<const float2*>(cos_sin), slots, s);
+  return launch_status("attention_f32_decode");
 }

@@ -200,6 +200,13 @@ __device__ __forceinline__ float group_max(float v) {      // as group_sum, the 
 __device__ __forceinline__ float wave_sum(float v) { return group_sum<kWave>(v); }
 __device__ __forceinline__ float wave_max(float v) { return group_max<kWave>(v); }
 
+// ss plus the squares of a thread's next four entries; the first four begin the sum.  Written out, so that every kernel that norms a row
+// rounds alike (left to the compiler, which pair of the first products is fused is its choice).
+__device__ __forceinline__ float add_squares(float ss, bool first, float a, float b, float c, float d) {
+  ss = first ? __fmaf_rn(a, a, __fmul_rn(b, b)) : __fmaf_rn(b, b, __fmaf_rn(a, a, ss));
+  return __fmaf_rn(d, d, __fmaf_rn(c, c, ss));
+}
+
 // Sum over a block of THREADS threads (a multiple of 64); every thread gets the result and adds the waves' sums itself, in wave order
 // (a second barrier keeps the next sum out of scratch until everybody has).  The order of additions depends on THREADS only.
 template <int THREADS>

@@ -212,9 +212,7 @@ __global__ void __launch_bounds__(kNormThreads)
   }
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < VPT; ++k)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += v[k][e] * v[k][e];
+  for (int k = 0; k < VPT; ++k) ss = add_squares(ss, k == 0, v[k][0], v[k][1], v[k][2], v[k][3]);
   ss = block_sum<kNormThreads>(ss, scratch);
   const float inv = 1.0f / sqrtf(ss / float(H) + eps);
   TO* o = out + size_t(r) * H;

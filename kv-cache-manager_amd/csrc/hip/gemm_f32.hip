@@ -22,59 +22,28 @@
 //               2048 141; staged through registers, one step on its way, 247, 66 and 173.  Rows that are not whole 16-byte pieces
 //               are staged so still.
 #include "common.h"
+#include "gemm_f32_order.h"
+#include "kvcm_hip.h"
 #include "tile_ring.h"
 
 namespace kvcm {
-
-using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
-
-constexpr int kUnit = 32, kSegments = 8;      // k of a unit; most segments
-
-// Units of 32 k per segment: up to 8 segments of equal length.
-__host__ __device__ __forceinline__ int segment_units(int K) {
-  const int units = (K + kUnit - 1) / kUnit;
-  return (units + kSegments - 1) / kSegments;
-}
-
-// Four consecutive k of one row, zero from K on.  Rows may begin at any float: the hardware takes 16-byte loads there.  FULL: no
-// piece lies outside.  FOURS: K is a multiple of 4, so a piece lies wholly inside or outside; the load is unconditional (from
-// k = 0 where it would be outside) and masked afterwards.
-typedef float any_four __attribute__((ext_vector_type(4), aligned(4)));
-template <bool FOURS, bool FULL = false>
-__device__ __forceinline__ f32x4 load4(const float* __restrict__ row, int k, int K) {
-  f32x4 v;
-  if constexpr (FULL) {
-    const any_four x = *reinterpret_cast<const any_four*>(row + k);
-    v = f32x4{x.x, x.y, x.z, x.w};
-  } else if constexpr (FOURS) {
-    const any_four x = *reinterpret_cast<const any_four*>(row + (k < K ? k : 0));
-    v = f32x4{x.x, x.y, x.z, x.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = k < K ? v[e] : 0.f;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float x = row[k + e < K ? k + e : 0];
-      v[e] = k + e < K ? x : 0.f;
-    }
-  }
-  return v;
-}
 
 // ---- up to 8 rows: columns 8 blockIdx.x .. + 7, wave w segments w and w + 4 ------------------------------------------------
 // The instruction's 16 x 16 results as two blocks of 8 x 8 on the diagonal: operand rows and columns 0..7 are X's rows and W's columns
 // over one segment, 8..15 the same over the other (the two blocks beside the diagonal mean nothing).  Every lane then loads W
 // of its own where the kernel below has 16 columns a workgroup, so that N / 8 workgroups of four waves cover the chip where N / 16 of eight
 // leave half of it idle.  Per element the same chain.
-template <bool FOURS>
+// GATED: W is N gate rows and N up rows; a workgroup has four columns of silu(gate) * up, as the SwiGLU kernel computes it from the same
+// sums, whose launch it saves: 2048 x 5632, us, 1 row 24.0 -> 22.5, 8 rows 28.1 -> 27.3; 1024 x 2816 10.0 -> 8.6, 12.9 -> 10.1.
+template <bool FOURS, bool GATED = false>
 __global__ void __launch_bounds__(kSegments / 2 * kWave)
     gemm_f32_rows8_kernel(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
                           int ldx, int ldw, int ldy) {
   __shared__ float sums[kSegments][8][8];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int r = lane & 15, g = lane >> 4, half = r >> 3, r8 = r & 7;
-  const int n0 = blockIdx.x * 8;
-  const int n = n0 + r8 < N ? n0 + r8 : N - 1, m = r8 < M ? r8 : M - 1;
+  const int n0 = blockIdx.x * (GATED ? 4 : 8);
+  const int at = n0 + (GATED ? r8 % 4 : r8), n = (at < N ? at : N - 1) + (GATED && r8 >= 4 ? N : 0), m = r8 < M ? r8 : M - 1;
   const int seg = segment_units(K), units = (K + kUnit - 1) / kUnit;
   const int s0 = wave, s1 = wave + kSegments / 2;
   // units of the wave's two segments (the later one is never the longer)
@@ -131,11 +100,18 @@ __global__ void __launch_bounds__(kSegments / 2 * kWave)
   }
   __syncthreads();
   const int segments = (units + seg - 1) / seg;
-  if (threadIdx.x < 64) {
+  auto total = [&](int row, int c) {
+    float t = sums[0][row][c];
+    for (int i = 1; i < segments; ++i) t += sums[i][row][c];
+    return t;
+  };
+  if constexpr (GATED) {
+    const int row = threadIdx.x / 4, c = threadIdx.x % 4;
+    if (row < M && n0 + c < N) Y[size_t(row) * ldy + n0 + c] = silu<float>(total(row, c)) * total(row, c + 4);
+  } else if (threadIdx.x < 64) {
     const int row = threadIdx.x / 8, c = threadIdx.x % 8;
-    float total = sums[0][row][c];
-    for (int i = 1; i < segments; ++i) total += sums[i][row][c];
-    if (row < M && n0 + c < N) Y[size_t(row) * ldy + n0 + c] = total;
+    const float t = total(row, c);
+    if (row < M && n0 + c < N) Y[size_t(row) * ldy + n0 + c] = t;
   }
 }
 
@@ -439,9 +415,6 @@ __global__ void __launch_bounds__(256, 2)
     }
 }
 
-// K up to 256 (models of small width, low-rank factors): these launches are bound by their latency, so they are not cut.
-constexpr int kShortK = 256;
-
 // Rows of whole 16-byte pieces, whole units.
 inline bool through_ring(const float* X, const float* W, int K, int ldx, int ldw) {
   return K % kUnit == 0 && ldx % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0 &&
@@ -531,4 +504,19 @@ extern "C" int kvcm_gemm_f32(const float* X, const float* W, float* Y, int M, in
   if (K % 4 == 0) launch_gemm_f32<true>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   else launch_gemm_f32<false>(X, W, Y, M, N, K, ldx, ldw, ldy, s);
   return launch_status("gemm_f32");
+}
+
+// Is gate and up in one launch with SwiGLU (kvcm_gemm_f32_swiglu), I columns of K > 256, the faster?  In blocks of 8 columns up to 8 rows
+// are no slower than otherwise by more than SwiGLU's launch while the matrix is small (8 rows of 2048 x 8192: 35.8 / 36.0 us; above
+// it 8 rows of 4096 x 28672 8 us slower), and not where the other way are tiles of very many columns, or K is very long.
+extern "C" int kvcm_gemm_f32_swiglu_preferred(int M, int I, int K) {
+  return M >= 1 && M <= 8 && I > 0 && K > kvcm::kShortK && K <= 8192 && K % 4 == 0 && I < 240 * 64 && (M <= 2 || 2ll * I * K <= 60000000);
+}
+
+// Y[M, I] = silu(X Wg^T) * (X Wu^T), W = [Wg; Wu]: the bits of kvcm_gemm_f32 and kvcm_swiglu.
+extern "C" int kvcm_gemm_f32_swiglu(const float* X, const float* W, float* Y, int M, int I, int K, int ldx, int ldw, int ldy, hipStream_t s) {
+  KVCM_REQUIRE(kvcm_gemm_f32_swiglu_preferred(M, I, K), "gemm_f32_swiglu: unsupported shape M=%d I=%d K=%d", M, I, K);
+  KVCM_REQUIRE(X && W && Y && ldx >= K && ldw >= K && ldy >= I, "gemm_f32_swiglu: missing operand or leading dimensions too small");
+  gemm_f32_rows8_kernel<true, true><<<(I + 3) / 4, kSegments / 2 * kWave, 0, s>>>(X, W, Y, M, I, K, ldx, ldw, ldy);
+  return launch_status("gemm_f32_swiglu");
 }

@@ -84,6 +84,12 @@ int kvcm_gemm8(const void* X, int ldx, const void* W, int ldw, int M, int N, int
                float eps, void* out, int out_dtype, int ldo, int swiglu, hipStream_t stream);
 int kvcm_gemm8_residual_norm(const void* X, int ldx, const void* W, int ldw, int M, int N, int K, float* resid,
                              const void* g, int g_dtype, void* xg, float* ss_out, hipStream_t stream);
+// 32-bit products of few rows with the norm in front, SwiGLU or the residual addition behind (gemm_f32_few.hip); of wider rows with SwiGLU.
+int kvcm_gemm_f32_swiglu_preferred(int M, int I, int K);
+int kvcm_gemm_f32_swiglu(const float* X, const float* W, float* Y, int M, int I, int K, int ldx, int ldw, int ldy, hipStream_t stream);
+int kvcm_gemm_f32_few_supported(int M, int K);
+int kvcm_gemm_f32_few(const float* X, const float* g, float eps, const float* W, float* Y, int M, int N, int K, int ldx, int ldw, int ldy,
+                      int behind, hipStream_t stream);
 // The attention half of a decoding layer of at most 8 rows in one launch (decode_front.hip): QKV product, rotation, page write,
 // attention, output product, residual addition and the next norm's preparation, handed on through two buffers in turn.
 int kvcm_decode_front_supported(int M, int H, int nh, int nkv, int hd, int B);
@@ -121,6 +127,11 @@ int kvcm_attention_generic(const void* q, int dtype, int q_stride, void* out, in
                            const void* vcache, const int* tables, int table_stride, const int* row_seq,
                            const int* ctx_lens, int T, int nh, int nkv, int hd, int B, float scale, int window,
                            hipStream_t s);
+// 32-bit single-token rows: rotation, page write and attention in one launch.
+int kvcm_attention_f32_decode_supported(int nh, int nkv, int hd, int B);
+int kvcm_attention_f32_decode(const float* qkv, int qkv_stride, float* out, int out_stride, const float* cos_sin, const int* slots,
+                              float* kcache, float* vcache, const int* tables, int table_stride, const int* row_seq, const int* ctx_lens,
+                              int T, int nh, int nkv, int hd, int B, float scale, int window, hipStream_t s);
 int kvcm_attention_decode(const void* q, int q_stride, void* out, int out_stride, const void* kcache, const void* vcache,
                           const int* tables, int table_stride, const int* row_seq, const int* ctx_lens, int T, int nh,
                           int nkv, int hd, int B, float scale, int max_context, float* scratch, long long scratch_floats,

@@ -82,6 +82,8 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_gemm_skinny_swiglu_normed),
     KVCM_ENTRY(kvcm_gemm_tiles),
     KVCM_ENTRY(kvcm_gemm_f32),
+    KVCM_ENTRY(kvcm_gemm_f32_few),
+    KVCM_ENTRY(kvcm_gemm_f32_swiglu),
     KVCM_ENTRY(kvcm_gemm_bf16),
     KVCM_ENTRY(kvcm_gemm_library),
     KVCM_ENTRY(kvcm_gemm_library_f32out),
@@ -90,6 +92,7 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_decode_front_empty),
     KVCM_ENTRY(kvcm_decode_front),
     KVCM_ENTRY(kvcm_attention_generic),
+    KVCM_ENTRY(kvcm_attention_f32_decode),
     KVCM_ENTRY(kvcm_attention_decode),
     KVCM_ENTRY(kvcm_attention_decode_fused),
     KVCM_ENTRY(kvcm_attention_prefill),

@@ -46,6 +46,12 @@ def _declare(lib):
     fn("kvcm_attention_decode_fused_info", i, i, i, vp)
     fn("kvcm_gemm_skinny_swiglu_supported", i, i, i)
     fn("kvcm_gemm_skinny_swiglu", vp, vp, vp, i, i, i, i, i, i, i, f, vp)
+    fn("kvcm_gemm_f32_few_supported", i, i)
+    fn("kvcm_gemm_f32_swiglu_preferred", i, i, i)
+    fn("kvcm_gemm_f32_swiglu", vp, vp, vp, i, i, i, i, i, i, vp)
+    fn("kvcm_gemm_f32_few", vp, vp, f, vp, vp, i, i, i, i, i, i, i, vp)
+    fn("kvcm_attention_f32_decode_supported", i, i, i, i)
+    fn("kvcm_attention_f32_decode", vp, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, i, i, i, i, i, f, i, vp)
     fn("kvcm_decode_front_supported", i, i, i, i, i, i)
     fn("kvcm_decode_front_parts", i)
     lib.kvcm_decode_front_words.restype = C.c_longlong
@@ -463,6 +469,55 @@ class NormedRows:
         return self.out
 
 
+class RowsToNorm:
+    """32-bit rows whose RMS norm has not run: the residual stream ``x`` [rows, H] (any addition done) and the norm's ``weight`` and
+    ``eps``.  ``gemm`` and ``gemm_swiglu`` take it in x's place and norm the rows themselves where they are few (csrc/hip/gemm_f32_few.hip),
+    with the bits of the norm's own launch; ``materialize`` runs that into ``out``."""
+
+    def __init__(self, x, weight, eps, out):
+        self.x, self.weight, self.eps, self.out = x, weight, float(eps), out
+        self.shape, self.dtype = x.shape, x.dtype
+
+    def materialize(self):
+        rmsnorm(self.x, self.weight, self.out, self.eps)
+        return self.out
+
+
+def f32_few_takes(M, K):
+    """Do 32-bit products of M rows of K entries take the norm before them and the addition to the residual stream, or SwiGLU, behind
+    them (``RowsToNorm``, ``gemm_residual``, ``gemm_swiglu``)?"""
+    return bool(lib().kvcm_gemm_f32_few_supported(M, K))
+
+
+def can_norm_rows(x, weight, out):
+    """May the 32-bit rows ``x`` be handed on as RowsToNorm (their products norm them with the bits of ``rmsnorm``'s kernel for such rows)?"""
+    M, H = x.shape
+    return (x.dtype == weight.dtype == out.dtype == torch.float32 and x.stride() == (H, 1) and weight.is_contiguous()
+            and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) and out.shape[0] == M and f32_few_takes(M, H))
+
+
+_BEHIND_PLAIN, _BEHIND_ADD, _BEHIND_SWIGLU = 0, 1, 2
+
+
+def _gemm_f32_few(x, w, out, N, behind):
+    normed = isinstance(x, RowsToNorm)
+    a = x.x if normed else x
+    M, K = a.shape
+    _dev(a, w, out)
+    for t, n in ((a, "x"), (w, "w"), (out, "out")):
+        _rows2d(t, n)
+        _need(t.dtype == torch.float32, "a float32 gemm needs float32 operands")
+    _need(w.shape == (N * (2 if behind == _BEHIND_SWIGLU else 1), K) and out.shape == (M, N), f"gemm shapes do not agree: {tuple(a.shape)} {tuple(w.shape)} {tuple(out.shape)}")
+    _call("kvcm_gemm_f32_few", _ptr(a), _ptr(x.weight) if normed else 0, x.eps if normed else 0.0, _ptr(w), _ptr(out), M, N, K, a.stride(0),
+          w.stride(0), out.stride(0), behind, _stream())
+
+
+def gemm_residual(product, x):
+    """x += product, of few 32-bit rows (PendingProduct): the addition in the product's epilogue, with the bits of ``add_residual``."""
+    _need(x.dtype == torch.float32 and x.is_contiguous(), "the residual stream must be contiguous float32 [M, H]")
+    _gemm_f32_few(product.x, product.w, x, product.w.shape[0], _BEHIND_ADD)
+
+
 def gemm_residual_norm(product, x, weight, eps, xg, ss, out):
     """x += round(product); returns NormedRows for the norm (weight, eps) that follows: the producer
     half of the folded norm.  product: PendingProduct of at most 8 bfloat16 rows; x: the 32-bit residual
@@ -732,6 +787,9 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
             _gemm8(x, w, out, N, False)
             return out
         x = x.materialize()
+    if isinstance(x, RowsToNorm):
+        _gemm_f32_few(x, w, out, w.shape[0], _BEHIND_PLAIN)
+        return out
     _dev(x, w, out)
     for t, n in ((x, "x"), (w, "w"), (out, "out")):
         _rows2d(t, n)
@@ -861,6 +919,22 @@ def gemm_swiglu(x, w_gate_up, out, limit=0.0, tuning=None):
         else:
             _gemm8(x, w_gate_up, out, I, True)
         return True
+    if isinstance(x, RowsToNorm) or x.dtype == torch.float32:
+        M, K = x.shape
+        I = out.shape[1]
+        if limit > 0 or w_gate_up.dtype != torch.float32 or out.dtype != torch.float32:
+            return False
+        if isinstance(x, RowsToNorm) or f32_few_takes(M, K):
+            _gemm_f32_few(x, w_gate_up, out, I, _BEHIND_SWIGLU)
+            return True
+        if not lib().kvcm_gemm_f32_swiglu_preferred(M, I, K):
+            return False
+        _dev(x, w_gate_up, out)
+        for t, n in ((x, "x"), (w_gate_up, "w_gate_up"), (out, "out")):
+            _rows2d(t, n)
+        _need(w_gate_up.shape == (2 * I, K) and out.shape[0] == M, "gemm_swiglu shapes do not agree")
+        _call("kvcm_gemm_f32_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), M, I, K, x.stride(0), w_gate_up.stride(0), out.stride(0), _stream())
+        return True
     _dev(x, w_gate_up, out)
     for t, n in ((x, "x"), (w_gate_up, "w_gate_up"), (out, "out")):
         _rows2d(t, n)
@@ -908,6 +982,30 @@ def attention(q, out, kcache, vcache, tables, table_stride, row_seq, ctx_lens, n
     _call("kvcm_attention_generic", _ptr(q), _DT[q.dtype], q.stride(0), _ptr(out), out.stride(0), _ptr(kcache),
                                         _ptr(vcache), _ptr(tables), table_stride, _ptr(row_seq), _ptr(ctx_lens), T, nh,
                                         nkv, hd, kcache.shape[2], float(scale), int(window), _stream())
+
+
+def attention_f32_decode_supported(nh, nkv, hd, block_size):
+    return bool(lib().kvcm_attention_f32_decode_supported(nh, nkv, hd, block_size))
+
+
+def attention_f32_decode(qkv, out, kcache, vcache, tables, table_stride, row_seq, ctx_lens, nh, nkv, hd, scale, slots, cos_sin=None, window=0,
+                         rows=None):
+    """32-bit rows of different sequences, from the projection's rows to the attention's: ``rope_cache`` and ``attention`` in one
+    launch, with their bits (``qkv`` itself is left as it is)."""
+    _dev(qkv, out, kcache, vcache, tables, row_seq, ctx_lens, slots, cos_sin)
+    _rows2d(qkv, "qkv")
+    _rows2d(out, "out")
+    T = qkv.shape[0] if rows is None else rows
+    _need(qkv.dtype == out.dtype == kcache.dtype == vcache.dtype == torch.float32, "attention_f32_decode operands must be float32")
+    _need(qkv.shape[1] >= (nh + 2 * nkv) * hd, "qkv rows are too short for the head layout")
+    _check_caches(kcache, vcache, nkv, hd)
+    for t, n in ((row_seq, "row_seq"), (ctx_lens, "ctx_lens"), (slots, "slots")):
+        _i32(t, n, T)
+    _i32(tables, "tables")
+    if cos_sin is not None:
+        _need(cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.numel() >= T * hd, "cos_sin must be float32 [rows, head_dim/2, 2]")
+    _call("kvcm_attention_f32_decode", _ptr(qkv), qkv.stride(0), _ptr(out), out.stride(0), _ptr(cos_sin), _ptr(slots), _ptr(kcache), _ptr(vcache),
+          _ptr(tables), table_stride, _ptr(row_seq), _ptr(ctx_lens), T, nh, nkv, hd, kcache.shape[2], float(scale), int(window), _stream())
 
 
 def attention_decode_supported(nh, nkv, hd, dtype, block_size=16):

@@ -324,6 +324,7 @@ class Mixer(Part):
 
 class FeedForward(Part):
     accepts_normed_rows = False      # as Mixer.accepts_normed_rows
+    defers = False                   # as Mixer.defers
 
     def forward(self, step, h):
         raise NotImplementedError

@@ -22,15 +22,18 @@ def _linear(ctx, step, x, w, name, keep_partial=False, dtype=None):
                         tuning=step.tune_products, unsplit=True)
 
 
-def _to_residual(ctx, step, x, w, name):
+def _to_residual(ctx, step, x, w, name, defer=False):
     """A part's last product, whose result goes to the residual stream.  For decode steps of a few
     rows it is handed on unrun (ops.PendingProduct): the norm that follows runs it with the addition
-    and its own preparation in the epilogue.  Otherwise it runs here, split sums left un-added."""
+    and its own preparation in the epilogue.  Otherwise it runs here, split sums left un-added.  ``defer``: the
+    caller takes it unrun in 32 bits too."""
     ops = ctx.ops
     if (step.fold_norms and x.dtype == torch.bfloat16 and x.shape[0] <= min(ops.FUSED_NORM_MAX_ROWS, step.fold_rows)
             and ops.gemm8_supported(x.shape[0], w.shape[0], w.shape[1])):
         out = step.ws(name, (x.shape[0], w.shape[0]))
         return ops.PendingProduct(x, w, out, step.scratch(name, x.shape[0], w.shape[0], w.shape[1]))
+    if defer and step.fold_norms and x.dtype == torch.float32 and ops.f32_few_takes(x.shape[0], w.shape[1]):
+        return ops.PendingProduct(x, w, step.ws(name, (x.shape[0], w.shape[0])))
     return _linear(ctx, step, x, w, name, keep_partial=True)
 
 
@@ -58,6 +61,10 @@ class RMSNorm(Norm):
 
     def forward(self, x, out, add=None, rows=None, defer=False):
         ops = self.ctx.ops
+        if defer and rows is None and (add is None or isinstance(add, ops.PendingProduct)) and ops.can_norm_rows(x, self.w["weight"], out):
+            if add is not None:
+                ops.gemm_residual(add, x)
+            return ops.RowsToNorm(x, self.w["weight"], self.params["eps"], out)
         if isinstance(add, ops.PendingProduct):
             if (defer and rows is None and self._folded is not None and add.x.shape[0] == x.shape[0] <= ops.FUSED_NORM_MAX_ROWS
                     and add.dtype == torch.bfloat16):
@@ -173,7 +180,7 @@ class GQAAttention(Mixer):
         wo = self.w["wo"]
         parts = self._one_launch_parts(step, h) if defer else 0
         if not parts:
-            return _to_residual(self.ctx, step, self._attention(step, h), wo, "mixer_out")
+            return _to_residual(self.ctx, step, self._attention(step, h), wo, "mixer_out", defer)
         ops, g = self.ctx.ops, self.cache.group
         table = self.position.rotation_table(step, self.hd) if self.position.rotates else None
         return ops.PendingAttention(
@@ -210,6 +217,12 @@ class GQAAttention(Mixer):
         if (table is not None or not pos.rotates) and paged_attention.attend_from_projection(
                 step, ops, res, attn, kc, vc, g, self.nh, self.nkv, self.hd, self.scale, self.window, table, slots):
             return attn
+        # 32-bit rows of different sequences: rotation, page write and attention in one launch, the same bits
+        if (slots is not None and step.max_run == 1 and qkv.dtype == torch.float32 and (table is not None or not pos.rotates)
+                and ops.attention_f32_decode_supported(self.nh, self.nkv, self.hd, self.ctx.block_size)):
+            ops.attention_f32_decode(res, attn, kc, vc, step.tables(g), step.table_stride(g), step.row_seq, step.ctx_lens, self.nh, self.nkv, self.hd,
+                                     self.scale, slots, cos_sin=table, window=self.window, rows=step.rows)
+            return attn
         extra = {"source": res} if hasattr(res, "materialize") else {}
         stored = pos.apply(step, qkv, self.nh, self.nkv, self.hd,
                            cache=(kc, vc) if self.cache_owner else None, slots=slots, **extra)
@@ -227,13 +240,14 @@ class SwiGLU(FeedForward):
 
     capturable = True
     accepts_normed_rows = True
+    defers = True
 
     def param_specs(self):
         H, I, pre = self.ctx.hidden_size, self.params["intermediate_size"], self.prefix
         return [ParamSpec("w_gate_up", ((pre + "gate_proj.weight", (I, H)), (pre + "up_proj.weight", (I, H)))),
                 ParamSpec("w_down", ((pre + "down_proj.weight", (H, I)),))]
 
-    def forward(self, step, h):
+    def forward(self, step, h, defer=False):
         I = self.params["intermediate_size"]
         act = step.ws("act", (step.rows, I))
         if not self.ctx.ops.gemm_swiglu(h, self.w["w_gate_up"], act, tuning=step.tune_products):      # few rows: one launch
@@ -241,7 +255,7 @@ class SwiGLU(FeedForward):
             if not self.ctx.ops.gemm_swiglu(h, self.w["w_gate_up"], act, tuning=step.tune_products):
                 gu = _linear(self.ctx, step, h, self.w["w_gate_up"], "gate_up")
                 self.ctx.ops.swiglu(gu, act)
-        return _to_residual(self.ctx, step, act, self.w["w_down"], "ffn_out")
+        return _to_residual(self.ctx, step, act, self.w["w_down"], "ffn_out", defer)
 
 
 @EMBEDDINGS.register("token_embedding")
@@ -309,11 +323,11 @@ class PreNormResidual(Block):
         n1, n2 = self.parts["norm_mixer"], self.parts["norm_ffn"]
         mixer, ffn = self.parts["mixer"], self.parts["ffn"]
         # a norm may leave its scale to the product that follows (Norm.defers) where that part takes it
-        fold1 = {"defer": True} if (n1.defers and mixer.accepts_normed_rows) else {}
-        fold2 = {"defer": True} if (n2.defers and ffn.accepts_normed_rows) else {}
+        fold1 = {"defer": True} if (step.fold_norms and n1.defers and mixer.accepts_normed_rows) else {}
+        fold2 = {"defer": True} if (step.fold_norms and n2.defers and ffn.accepts_normed_rows) else {}
         h = n1.forward(x, buf, add=pending if n1.accepts_partial_sums else as_tensor(pending), **fold1)
         # a mixer may leave all of its launches to the norm behind it (Mixer.defers), which runs at once
         late = {"defer": True} if (n2.defers and n2.accepts_partial_sums and mixer.defers and fold2) else {}
         a = mixer.forward(step, buf if h is None else h, **late)
         h = n2.forward(x, buf, add=a if n2.accepts_partial_sums else as_tensor(a), **fold2)
-        return ffn.forward(step, buf if h is None else h)
+        return ffn.forward(step, buf if h is None else h, **({"defer": True} if fold2 and ffn.defers else {}))
