@@ -87,7 +87,8 @@ class RecordedSteps:
         s = self.sampler
         self._h = self.lib.kvcm_engine_new(
             self.core.handle, fns, self.runner._pinned.data_ptr(), self.runner.meta_dev.data_ptr(), self.runner.meta_dev.numel(),
-            s.out.data_ptr(), s._host.data_ptr(), s.max_rows, self.core.num_groups, engine.config.block_size,
+            0, s._host.data_ptr(), s.max_rows,      # (recorded steps sample into pinned host memory)
+            self.core.num_groups, engine.config.block_size,
             lim.max_context_len, lim.max_tokens, lim.max_seqs, lim.max_logit_rows, GRAPH_ROWS if use_graphs else 0,
             self.stream.cuda_stream)
         if not self._h:
@@ -156,10 +157,11 @@ class RecordedSteps:
                 with ops.recording(program):
                     logits = runner.model.forward(step)
                     t, seeds, ids, idx = step.sampling_params()
-                    ops.sample(logits, self.sampler.out[:shape.logit_rows], t, seeds, ids, idx)
+                    ops.sample(logits, self.sampler._host[:shape.logit_rows], t, seeds, ids, idx)
             finally:
                 ops.LIBRARY_GEMM_MIN_ROWS = keep
-            sampled = self.sampler.download(sampling)
+            self.stream.synchronize()
+            sampled = self.sampler._host[:sampling].numpy().copy()
             if self.lib.kvcm_engine_register(self._h, program.release(), int(self.wants_graph)) != 0:
                 raise ops.KernelError(self.lib.kvcm_hip_last_error().decode())
             self.recorded_shapes[shape] = "graph" if self.wants_graph else "program"

@@ -1247,8 +1247,10 @@ def fill_index(out, key, modulus):
 
 
 def sample(logits, out, temperature=None, seeds=None, request_ids=None, token_index=None):
-    """out[r] = argmax of row r, or a Gumbel-max draw where temperature[r] > 0."""
-    _dev(logits, out, temperature, seeds, request_ids, token_index)
+    """out[r] = argmax of row r, or a Gumbel-max draw where temperature[r] > 0.  ``out`` may be pinned host memory: the ids are there once
+    the stream has been waited for."""
+    _dev(logits, temperature, seeds, request_ids, token_index)
+    _need(out.is_cuda or out.is_pinned(), "kernel operands must live on the GPU (the sampled ids: or in pinned host memory)")
     _rows2d(logits, "logits")
     R, V = logits.shape
     _need(logits.dtype == torch.float32, "logits must be float32")
