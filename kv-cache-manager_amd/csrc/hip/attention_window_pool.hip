@@ -183,6 +183,30 @@ __global__ void __launch_bounds__(256)
 // them, in a run, ends a block where R <= P) and makes keys or values (blockIdx.z) of one kv head, AHEAD tokens' pages, then their
 // values, requested before the first is added, in order.  A workgroup per row that waited for every token's value in turn took
 // 86 us for a prompt of 2,048 tokens in blocks of 64, four heads of 64; 13 us so.
+// A wave makes the mean key (or value) of the block that ends at position p, whose token lies in `slot`.
+template <class T, int AHEAD>
+__device__ __forceinline__ void pool_entry(const T* kcache, const T* vcache, float* pk, float* pv, const int* table, bool keys, int p, int slot, int kvh,
+                                           int lane, int nkv, int d, int dv, int B, int P, int E) {
+  const int first = p - P + 1, entry = p / P - (p / B * B) / P;
+  const size_t at = (size_t(slot / B) * nkv + kvh) * E + entry;
+  const float inv = 1.0f / float(P);
+  for (int i = lane; i < (keys ? d : dv); i += kWave) {
+    float acc = 0.f;
+    for (int t0 = first; t0 <= p; t0 += AHEAD) {
+      float x[AHEAD];
+#pragma unroll
+      for (int a = 0; a < AHEAD; ++a) {
+        const int t = t0 + a <= p ? t0 + a : p;
+        const size_t page = size_t(table[t / B]) * nkv + kvh;
+        x[a] = load_f(keys ? kcache + (page * B + t % B) * d + i : vcache + (page * dv + i) * B + t % B);
+      }
+#pragma unroll
+      for (int a = 0; a < AHEAD; ++a) acc = t0 + a <= p ? acc + x[a] : acc;
+    }
+    (keys ? pk[at * d + i] : pv[at * dv + i]) = acc * inv;
+  }
+}
+
 template <class T, int AHEAD>
 __global__ void __launch_bounds__(kWave)
     pool_update_kernel(const T* __restrict__ kcache, const T* __restrict__ vcache, float* __restrict__ pk,
@@ -195,26 +219,9 @@ __global__ void __launch_bounds__(kWave)
   const bool ends = lane < R && row0 + lane < rows && slots[mine] >= 0 && (positions[mine] + 1) % P == 0;
   for (unsigned long long left = __ballot(ends); left != 0; left &= left - 1) {
     const int row = row0 + __builtin_ctzll(left);
-    const int p = positions[row], slot = slots[row], first = p - P + 1;
+    const int p = positions[row], slot = slots[row];
     const int* table = tables + size_t(row_seq[row]) * table_stride;
-    const int entry = p / P - (p / B * B) / P;
-    const size_t at = (size_t(slot / B) * nkv + kvh) * E + entry;
-    const float inv = 1.0f / float(P);
-    for (int i = lane; i < (keys ? d : dv); i += kWave) {
-      float acc = 0.f;
-      for (int t0 = first; t0 <= p; t0 += AHEAD) {
-        float x[AHEAD];
-#pragma unroll
-        for (int a = 0; a < AHEAD; ++a) {
-          const int t = t0 + a <= p ? t0 + a : p;
-          const size_t page = size_t(table[t / B]) * nkv + kvh;
-          x[a] = load_f(keys ? kcache + (page * B + t % B) * d + i : vcache + (page * dv + i) * B + t % B);
-        }
-#pragma unroll
-        for (int a = 0; a < AHEAD; ++a) acc = t0 + a <= p ? acc + x[a] : acc;
-      }
-      (keys ? pk[at * d + i] : pv[at * dv + i]) = acc * inv;
-    }
+    pool_entry<T, AHEAD>(kcache, vcache, pk, pv, table, keys, p, slot, kvh, lane, nkv, d, dv, B, P, E);
   }
 }
 
@@ -454,7 +461,7 @@ __global__ void __launch_bounds__(kWpWaves* kWave)
 // query head above, whose dots and sums over values are a thousand vector instructions for each chunk and head and which reads
 // the keys once per head, took 19.0 us a step of 8 rows of 32 heads over 4 kv heads of 64 in a window of 512 (sixteen waves in
 // place of four: 14.5 us), this 12.2 us; 1,100 such rows at once 814 us then, 137 us now; heads of 128 over 8 kv heads in a
-// window of 1,024 with pooled blocks 29.7 us then, 24.8 us now (at 128 the fragments leave 144 bytes of scratch a lane).
+// window of 1,024 with pooled blocks 29.7 us then, 24.8 us now.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 typedef float any_four __attribute__((ext_vector_type(4), aligned(4)));      // (pooled entries may lie at any float)
@@ -469,18 +476,43 @@ __device__ __forceinline__ float below_upper(float x) {
   return fmaxf(x - __uint_as_float(__float_as_uint(x) & 0xFFFF0000u), fminf(x, 1.17549435e-38f));
 }
 
-// DP: key size padded to a multiple of 32; DVT: tiles of 16 value columns
-template <int DP, int DVT, int WAVES>
+// What steps in which every sequence runs one row do between the projection and the attention: the workgroup of a row and a kv head, which
+// alone needs and stores them, takes its channels from the projection's row [q | k | v] and gives them, with the operations of the kernels
+// above and of short_conv.hip in their order: the convolution (its state moved on), the rotation, the page's new key and value, and at last the
+// pooled entry where one is due.  Bound by the trips to memory one after the other; the first keys and values and what the front
+// needs are on their way together.  Four launches as one, 8 rows of 32 heads over 4 kv heads of 64, window 512, blocks of 64, 4 taps: in a row
+// of such launches 540 tokens 16.7 -> 15.6 us, 60 tokens 14.0 -> 11.4; between a decoder's other launches 22.8 -> 16.9.  Heads of 128, whose first
+// keys and values the registers do not hold beside it, lose (8 rows, 30.1 -> 31.2), and so do norms over all heads in its place (13.4 -> 13.8).
+struct WpFront {
+  const float* src; int ld;
+  const float* conv_w; const float* conv_bias; float* conv_state; const int* state_slots; int taps;
+  const float2* cos_sin; int rot, halves;
+  const int* slots;
+};
+
+// what an entry of the front needs from memory besides its convolution's state
+constexpr int kFrontTaps = 8;
+struct FrontEntry {
+  float x, bias, w[kFrontTaps];
+  float2 turn;
+};
+
+// DP: key size padded to a multiple of 32; DVT: tiles of 16 value columns.  FRONT: q comes from `fr` (a workgroup per row and kv head: at most
+// 16 query heads each); no cap, kept tokens, chunk, sink, slope or gate.
+template <int DP, int DVT, int WAVES, bool FRONT>
 __global__ void __launch_bounds__(WAVES* kWave)
     attention_window_pool_heads_kernel(const uint16_t* __restrict__ q, int ldq, uint16_t* __restrict__ out, int ldo,
-                                       const uint16_t* __restrict__ kcache, const uint16_t* __restrict__ vcache,
-                                       const float* __restrict__ pk, const float* __restrict__ pv,
+                                       const uint16_t* kcache, const uint16_t* vcache,
+                                       const float* pk, const float* pv,
                                        const int* __restrict__ tables, int table_stride, const int* __restrict__ row_seq,
                                        const int* __restrict__ ctx_lens, const float* __restrict__ head_scale,
                                        const float* __restrict__ dist_slope, const float* __restrict__ gate, int ldg,
                                        int nh, int nkv, int d, int dv, int B, float scale, int window, int P, int E, int keep_first,
-                                       float softcap, int chunk, int sink, const float* __restrict__ sink_logit, int gate_heads, float out_scale) {
+                                       float softcap, int chunk, int sink, const float* __restrict__ sink_logit, int gate_heads, float out_scale,
+                                       const WpFront fr) {
+  if constexpr (FRONT) softcap = 0.f, keep_first = chunk = sink = 0, out_scale = 1.0f;
   constexpr int KS = DP / 32, DVP = DVT * 16, PITCH = DVP + 4;
+  constexpr bool kAhead = FRONT;      // the first chunk's keys and values asked for before the front
   __shared__ __attribute__((aligned(16))) float parts[WAVES][16][PITCH];      // a wave's sums, head by head
   __shared__ float maxima[WAVES][16], sums[WAVES][16], weights[WAVES][16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -491,21 +523,34 @@ __global__ void __launch_bounds__(WAVES* kWave)
   const int my_head = head0 + (col < heads ? col : 0);
   const int ctx = ctx_lens[row], seq = row_seq[row];
   uint16_t* orow = out + size_t(row) * ldo + size_t(head0) * dv;
+  // the front's entries: q of the heads, k, v.  The first of a thread is on its way before the context, the pages and the state's place are known.
+  const int nq = nh * d, nk = nkv * d, mine = heads * d, entries = mine + d + dv;
+  const float* r = FRONT ? fr.src + size_t(row) * fr.ld : nullptr;
+  const int new_slot = FRONT ? fr.slots[row] : -1;
+  const auto channel = [&](int e) { return e < mine ? head0 * d + e : e < mine + d ? nq + kvh * d + (e - mine) : nq + nk + kvh * dv + (e - mine - d); };
+  const auto turned_with = [&](int i) { return !fr.halves ? i ^ 1 : i >= fr.rot / 2 ? i - fr.rot / 2 : i + fr.rot / 2; };
+  const auto gather = [&](int e, FrontEntry& en) {
+    const int ch = channel(e);
+    en.x = r[ch];
+    en.bias = fr.conv_bias ? fr.conv_bias[ch] : 0.f;
+#pragma unroll
+    for (int j = 0; j < kFrontTaps; ++j) en.w[j] = fr.conv_w[size_t(ch) * fr.taps + (j < fr.taps ? j : 0)];
+    if (e < mine + d) {
+      const int i = e % d, j = i < fr.rot ? turned_with(i) : i;
+      if (i < fr.rot) en.turn = fr.cos_sin[size_t(row) * (fr.rot / 2) + (fr.halves ? (i < j ? i : j) : i / 2)];
+    }
+  };
+  FrontEntry early_entry;
+  if constexpr (FRONT) {
+    if (tid < entries) gather(tid, early_entry);
+  }
   if (ctx <= 0) {
     for (int i = tid; i < heads * dv; i += WAVES * kWave) orow[i] = 0;
     return;
   }
   const int* table = tables + size_t(seq) * table_stride;
-  const uint16_t* my_q = q + size_t(row) * ldq + size_t(my_head) * d;
-  bf16x8 qf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int k = ks * 32 + quad * 8;
-    const uint4 v = *reinterpret_cast<const uint4*>(my_q + (k < d ? k : 0));
-    qf[ks] = __builtin_bit_cast(bf16x8, k < d ? v : uint4{0u, 0u, 0u, 0u});
-  }
   const float f = head_scale ? scale * head_scale[my_head] : scale;
-  const float slope = dist_slope ? dist_slope[my_head] : 0.f;
+  const float slope = !FRONT && dist_slope ? dist_slope[my_head] : 0.f;
   const float inv_cap = softcap > 0.f ? 1.0f / softcap : 0.f;
 
   const int first = chunk > 0 ? (ctx - 1) / chunk * chunk : (window > 0 && ctx > window) ? ctx - window : 0;
@@ -514,6 +559,122 @@ __global__ void __launch_bounds__(WAVES* kWave)
   const int kept = keep_first < first ? keep_first : first;
   const int head_chunks = block_chunks + (kept + kWave - 1) / kWave;
   const int first_chunk = first / kWave, chunks = head_chunks + ((ctx - 1) / kWave - first_chunk + 1);
+
+  // the chunk's tokens (place j of a lane below): the kept first tokens before the window, or the window; [lo, hi) is what it sees
+  const auto stretch = [&](int c, int& c0, int& lo, int& hi) {
+    const bool early = c < head_chunks;
+    c0 = early ? (c - block_chunks) * kWave : (first_chunk + (c - head_chunks)) * kWave;
+    lo = early ? 0 : first;
+    hi = early ? kept : ctx;
+  };
+  uint4 kreg[2][2][KS], vreg[2][DVT];
+  // A lane looks up the page of the token at its place, clamped into the stretch (pages that the window has passed may have been given back).
+  const auto ask = [&](int c) {
+    int c0, lo, hi;
+    stretch(c, c0, lo, hi);
+    const int at = c0 + lane < lo ? lo : c0 + lane < hi ? c0 + lane : hi - 1;
+    const int page_no = at / B, slot = at - page_no * B, page = table[page_no];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int from = 32 * g + 8 * (col / 4) + 4 * t + col % 4;
+        const uint16_t* src = kcache + ((size_t(__shfl(page, from, kWave)) * nkv + kvh) * B + __shfl(slot, from, kWave)) * d;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int k = ks * 32 + quad * 8;
+          kreg[g][t][ks] = *reinterpret_cast<const uint4*>(src + (k < d ? k : 0));
+        }
+      }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int from = 32 * g + 8 * quad;
+      const uint16_t* src = vcache + (size_t(__shfl(page, from, kWave)) * nkv + kvh) * dv * B + __shfl(slot, from, kWave) / 8 * 8;
+#pragma unroll
+      for (int vt = 0; vt < DVT; ++vt) {
+        const int dim = vt * 16 + col;
+        vreg[g][vt] = *reinterpret_cast<const uint4*>(src + size_t(dim < dv ? dim : dv - 1) * B);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);      // (all of them on their way before the first is waited for)
+  };
+
+  // the front's values, where the waves' sums come later: 32-bit, then as stored (q of the heads, k, v)
+  constexpr int kMostFront = 16 * DP + DP + DVP;
+  float* const xs = &parts[0][0][0];
+  uint16_t* const stored = reinterpret_cast<uint16_t*>(xs + kMostFront);
+  static_assert(sizeof(parts) >= size_t(kMostFront) * (sizeof(float) + sizeof(uint16_t)), "the front's values lie where the sums come");
+  int c = wave;
+  if constexpr (FRONT) {
+    const int C = nq + nk + nkv * dv, state_slot = fr.state_slots ? fr.state_slots[seq] : -1;
+    if (kAhead && c >= block_chunks && c < chunks) ask(c);
+    const auto convolved = [&](int e, const FrontEntry& en) {
+      float* st = state_slot >= 0 ? fr.conv_state + size_t(state_slot) * (fr.taps - 1) * C + channel(e) : nullptr;
+      float seen[kFrontTaps];
+#pragma unroll
+      for (int j = 0; j < kFrontTaps; ++j) {
+        seen[j] = 0.f;
+        if (j < fr.taps - 1 && st && ctx - fr.taps + j >= 0) seen[j] = st[size_t(j) * C];
+      }
+      float y = 0.f;
+#pragma unroll
+      for (int j = 0; j < kFrontTaps; ++j)
+        if (j < fr.taps) {
+          if (j == fr.taps - 1) seen[j] = en.x + en.bias;
+          y = fmaf(en.w[j], seen[j], y);
+        }
+      if (st) {
+#pragma unroll
+        for (int j = 1; j < kFrontTaps; ++j)
+          if (j < fr.taps) st[size_t(j - 1) * C] = seen[j];
+      }
+      return y;
+    };
+    if (tid < entries) xs[tid] = convolved(tid, early_entry);
+    for (int e = tid + WAVES * kWave; e < entries; e += WAVES * kWave) {
+      FrontEntry en;
+      gather(e, en);
+      xs[e] = convolved(e, en);
+    }
+    __syncthreads();
+    const size_t new_page = size_t(new_slot < 0 ? 0 : new_slot / B) * nkv + kvh;
+    uint16_t* kp = const_cast<uint16_t*>(kcache) + (new_page * B + (new_slot < 0 ? 0 : new_slot % B)) * d;
+    uint16_t* vp = const_cast<uint16_t*>(vcache) + new_page * dv * B + (new_slot < 0 ? 0 : new_slot % B);
+    const auto finish = [&](int e, const FrontEntry& en) {
+      float x = xs[e];
+      if (e < mine + d) {
+        const int i = e % d;
+        if (i < fr.rot) {
+          const int j = turned_with(i);
+          const float y = xs[e - i + j];
+          x = i > j ? __fmaf_rn(x, en.turn.x, __fmul_rn(y, en.turn.y)) : __fmaf_rn(x, en.turn.x, -__fmul_rn(y, en.turn.y));
+        }
+      }
+      const uint16_t bits = float_to_bf16_bits(x);
+      stored[e] = bits;
+      if (new_slot >= 0 && e >= mine) {
+        if (e < mine + d) kp[e - mine] = bits;
+        else vp[size_t(e - mine - d) * B] = bits;
+      }
+    };
+    if (tid < entries) finish(tid, early_entry);
+    for (int e = tid + WAVES * kWave; e < entries; e += WAVES * kWave) {
+      FrontEntry en;
+      gather(e, en);
+      finish(e, en);
+    }
+    __syncthreads();
+  }
+  const uint16_t* my_q = q + size_t(row) * ldq + size_t(my_head) * d;
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int k = ks * 32 + quad * 8;
+    uint4 v;
+    if constexpr (FRONT) v = *reinterpret_cast<const uint4*>(stored + (my_head - head0) * d + (k < d ? k : 0));
+    else v = *reinterpret_cast<const uint4*>(my_q + (k < d ? k : 0));
+    qf[ks] = __builtin_bit_cast(bf16x8, k < d ? v : uint4{0u, 0u, 0u, 0u});
+  }
 
   float m = -INFINITY, l = 0.f;      // the head's largest score; this lane's part of its sum
   f32x4 o[DVT];                      // O^T: column = head, rows = dims 16 vt + 4 quad + i
@@ -528,7 +689,7 @@ __global__ void __launch_bounds__(WAVES* kWave)
       const int key = key_of(j);
       sv[j] *= f;
       if (softcap > 0.f) sv[j] = softcap * tanhf(sv[j] * inv_cap);
-      if (dist_slope && tokens) sv[j] = fmaf(-slope, float(ctx - 1 - key), sv[j]);
+      if (!FRONT && dist_slope && tokens) sv[j] = fmaf(-slope, float(ctx - 1 - key), sv[j]);
       sv[j] = key >= lo && key < hi ? sv[j] : -INFINITY;
       mx = fmaxf(mx, sv[j]);
     }
@@ -548,8 +709,8 @@ __global__ void __launch_bounds__(WAVES* kWave)
       for (int i = 0; i < 4; ++i) o[vt][i] *= alpha;
   };
 
-  for (int c = wave; c < chunks; c += WAVES) {
-    if (c < block_chunks) {      // pooled: score 4 t + i is block c0 + 16 t + 4 quad + i
+  if (c < block_chunks) {      // (the chunk asked for ahead is not kept through this: it is another wave's)
+    do {      // pooled: score 4 t + i is block c0 + 16 t + 4 quad + i
       const int c0 = c * kWave;
       const int b = c0 + lane < blocks ? c0 + lane : blocks - 1, page_no = (b * P + P - 1) / B;
       const int page = table[page_no], entry = b - page_no * B / P;
@@ -566,7 +727,8 @@ __global__ void __launch_bounds__(WAVES* kWave)
           for (int n = 0; n < DP / 16; ++n) {
             const int k = 16 * n + 4 * quad;
             x[n] = *reinterpret_cast<const any_four*>(src + (k < d ? k : 0));
-            y[n] = *reinterpret_cast<const uint2*>(my_q + (k < d ? k : 0));
+            if constexpr (FRONT) y[n] = *reinterpret_cast<const uint2*>(stored + (my_head - head0) * d + (k < d ? k : 0));
+            else y[n] = *reinterpret_cast<const uint2*>(my_q + (k < d ? k : 0));
           }
 #pragma unroll
           for (int n = 0; n < DP / 16; ++n) {
@@ -601,40 +763,43 @@ __global__ void __launch_bounds__(WAVES* kWave)
           }
         }
       }
-      continue;
-    }
-    // tokens: score 8 g + 4 t + i is token c0 + 32 g + 8 quad + 4 t + i.  The chunk sees the stretch [lo, hi): the kept first
-    // tokens before the window, or the window.  A lane looks up the page of the token at its place, clamped into the stretch
-    // (pages that the window has passed may have been given back).
-    const bool early = c < head_chunks;
-    const int c0 = early ? (c - block_chunks) * kWave : (first_chunk + (c - head_chunks)) * kWave;
-    const int lo = early ? 0 : first, hi = early ? kept : ctx;
-    const int at = c0 + lane < lo ? lo : c0 + lane < hi ? c0 + lane : hi - 1;
-    const int page_no = at / B, slot = at - page_no * B, page = table[page_no];
-    uint4 kreg[2][2][KS], vreg[2][DVT];
+      c += WAVES;
+    } while (c < block_chunks);
+    if (kAhead && c < chunks) ask(c);
+  }
+  while (c < chunks) {
+    // tokens: score 8 g + 4 t + i is token c0 + 32 g + 8 quad + 4 t + i
+    int c0, lo, hi;
+    stretch(c, c0, lo, hi);
+    if (!kAhead) ask(c);
+    if (FRONT && new_slot >= 0 && c == chunks - 1) {      // the newest token: its key and value as they were just made
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+      for (int g = 0; g < 2; ++g)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int from = 32 * g + 8 * (col / 4) + 4 * t + col % 4;
-        const uint16_t* src = kcache + ((size_t(__shfl(page, from, kWave)) * nkv + kvh) * B + __shfl(slot, from, kWave)) * d;
+        for (int t = 0; t < 2; ++t)
+          if (c0 + 32 * g + 8 * (col / 4) + 4 * t + col % 4 == ctx - 1) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const int k = ks * 32 + quad * 8;
-          kreg[g][t][ks] = *reinterpret_cast<const uint4*>(src + (k < d ? k : 0));
+            for (int ks = 0; ks < KS; ++ks) {
+              const int k = ks * 32 + quad * 8;
+              kreg[g][t][ks] = *reinterpret_cast<const uint4*>(stored + heads * d + (k < d ? k : 0));
+            }
+          }
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int j = ctx - 1 - (c0 + 32 * g + 8 * quad);
+        if (j >= 0 && j < 8) {
+#pragma unroll
+          for (int vt = 0; vt < DVT; ++vt) {
+            const int dim = vt * 16 + col;
+            const uint32_t bits = stored[heads * d + d + (dim < dv ? dim : dv - 1)];
+            const auto with = [&](uint32_t w, int n) {      // word n of the piece: tokens 2 n and 2 n + 1
+              return j == 2 * n ? (w & 0xFFFF0000u) | bits : j == 2 * n + 1 ? (w & 0xFFFFu) | bits << 16 : w;
+            };
+            vreg[g][vt] = uint4{with(vreg[g][vt].x, 0), with(vreg[g][vt].y, 1), with(vreg[g][vt].z, 2), with(vreg[g][vt].w, 3)};
+          }
         }
       }
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const int from = 32 * g + 8 * quad;
-      const uint16_t* src = vcache + (size_t(__shfl(page, from, kWave)) * nkv + kvh) * dv * B + __shfl(slot, from, kWave) / 8 * 8;
-#pragma unroll
-      for (int vt = 0; vt < DVT; ++vt) {
-        const int dim = vt * 16 + col;
-        vreg[g][vt] = *reinterpret_cast<const uint4*>(src + size_t(dim < dv ? dim : dv - 1) * B);
-      }
     }
-    __builtin_amdgcn_sched_barrier(0);      // (all of them on their way before the first is waited for)
     if (d < DP) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
@@ -678,8 +843,11 @@ __global__ void __launch_bounds__(WAVES* kWave)
 #pragma unroll
         for (int j = 8 * g; j < 8 * g + 8; ++j) sv[j] = below_upper(sv[j]);
       }
+    c += WAVES;
+    if (kAhead && c < chunks) ask(c);
   }
   l = rows_sum(l);
+  if constexpr (FRONT) __syncthreads();      // (the sums come where the front's values were)
 #pragma unroll
   for (int vt = 0; vt < DVT; ++vt) *reinterpret_cast<f32x4*>(&parts[wave][col][vt * 16 + 4 * quad]) = o[vt];
   if (quad == 0) {
@@ -709,8 +877,13 @@ __global__ void __launch_bounds__(WAVES* kWave)
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) acc = fmaf(parts[w][h][e], weights[w][h], acc);
     float res = acc / sums[0][h] * out_scale;
-    if (gate) res *= 1.0f / (1.0f + expf(-gate[size_t(row) * ldg + (gate_heads ? head0 + h : (head0 + h) * dv + e)]));
+    if (!FRONT && gate) res *= 1.0f / (1.0f + expf(-gate[size_t(row) * ldg + (gate_heads ? head0 + h : (head0 + h) * dv + e)]));
     orow[i] = float_to_bf16_bits(res);
+  }
+  if constexpr (FRONT) {      // the block that this token ends lies in the window: its entry is for later steps
+    if (P > 0 && new_slot >= 0 && ctx % P == 0 && wave < 2)
+      pool_entry<bf16_t, 8>(reinterpret_cast<const bf16_t*>(kcache), reinterpret_cast<const bf16_t*>(vcache), const_cast<float*>(pk), const_cast<float*>(pv), table,
+                             wave == 0, ctx - 1, new_slot, kvh, lane, nkv, d, dv, B, P, E);
   }
 }
 
@@ -846,10 +1019,10 @@ int kvcm_attention_window_pool(const void* q, int dtype, int ldq, void* out, int
       nkv * ((nh / nkv + 15) / 16) <= 65535) {
     const dim3 grid(T, nkv * ((nh / nkv + 15) / 16));
 #define KVCM_WINDOW_POOL_HEADS(DP, DVT, WAVES)                                                                                 \
-  attention_window_pool_heads_kernel<DP, DVT, WAVES><<<grid, (WAVES) * kWave, 0, s>>>(                                         \
+  attention_window_pool_heads_kernel<DP, DVT, WAVES, false><<<grid, (WAVES) * kWave, 0, s>>>(                                         \
       static_cast<const uint16_t*>(q), ldq, static_cast<uint16_t*>(out), ldo, static_cast<const uint16_t*>(kcache),            \
       static_cast<const uint16_t*>(vcache), pk, pv, tables, table_stride, row_seq, ctx_lens, head_scale, dist_slope, gate, ldg, \
-      nh, nkv, d, dv, B, scale, window, P, E, keep_first, softcap, chunk, sink, sink_logit, gate_heads, out_scale)
+      nh, nkv, d, dv, B, scale, window, P, E, keep_first, softcap, chunk, sink, sink_logit, gate_heads, out_scale, WpFront{})
     if (d <= 64 && dv <= 64) KVCM_WINDOW_POOL_HEADS(64, 4, 12);
     else KVCM_WINDOW_POOL_HEADS(128, 8, 7);      // (what 64 KB of local memory hold)
 #undef KVCM_WINDOW_POOL_HEADS
@@ -868,6 +1041,41 @@ int kvcm_attention_window_pool(const void* q, int dtype, int ldq, void* out, int
         ldg, nh, nkv, d, dv, B, scale, window, P, E, keep_first, softcap, chunk, sink, sink_logit, gate_heads, out_scale);
   else KVCM_REQUIRE(false, "attention_window_pool: unknown dtype %d", dtype);
   return launch_status("attention_window_pool");
+}
+
+// 1 when kvcm_attention_window_pool_rows takes the head shape and pages.
+int kvcm_attention_window_pool_rows_supported(int nh, int nkv, int d, int dv, int B) {
+  return nkv > 0 && nh % nkv == 0 && nh / nkv >= 2 && nh / nkv <= 16 && d > 0 && dv > 0 && d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 64 && B > 0 &&
+         B % 8 == 0 && nkv <= 65535;
+}
+
+// bfloat16 rows of T different sequences, one each, from the projection's 32-bit rows [q | k | v] to the attention's: convolution (conv_w [C][taps],
+// bias before it, conv_state [slots][taps - 1][C] moved on), rotation (as kvcm_rotate_store), keys and values to slots [T] (negative: not
+// stored), the attention, and the pooled entries that end with these rows.  The rows' positions are ctx_lens - 1.  The results are those of the
+// launches one by one, bit for bit.
+int kvcm_attention_window_pool_rows(const float* src, int ld, const float* conv_w, const float* conv_bias, float* conv_state, const int* state_slots,
+                                    int taps, const float* cos_sin, int rot, int halves, const int* slots, void* out, int ldo, void* kcache, void* vcache,
+                                    float* pk, float* pv, const int* tables, int table_stride, const int* row_seq, const int* ctx_lens,
+                                    const float* head_scale, int T, int nh, int nkv, int d, int dv, int B, float scale, int window, int P, hipStream_t s) {
+  if (T == 0) return 0;
+  KVCM_REQUIRE(T > 0 && kvcm_attention_window_pool_rows_supported(nh, nkv, d, dv, B),
+               "attention_window_pool_rows: unsupported shape T=%d heads=%d kv_heads=%d d=%d dv=%d page=%d", T, nh, nkv, d, dv, B);
+  const int C = (nh + nkv) * d + nkv * dv;
+  KVCM_REQUIRE(src && conv_w && out && kcache && vcache && slots && tables && row_seq && ctx_lens, "attention_window_pool_rows: null operand");
+  KVCM_REQUIRE(ld >= C && ldo >= nh * dv, "attention_window_pool_rows: row strides too small");
+  KVCM_REQUIRE(taps >= 1 && taps <= kFrontTaps && (taps == 1 || (conv_state && state_slots)),
+               "attention_window_pool_rows: %d taps are not supported (1 to %d are), or the state is missing", taps, kFrontTaps);
+  KVCM_REQUIRE(rot % 2 == 0 && rot >= 0 && rot <= d && (rot == 0 || cos_sin), "attention_window_pool_rows: bad rotation of %d dims", rot);
+  KVCM_REQUIRE(window >= 0 && P >= 0 && (P == 0 || (pk && pv)), "attention_window_pool_rows: bad window or blocks");
+  KVCM_REQUIRE((reinterpret_cast<uintptr_t>(kcache) | reinterpret_cast<uintptr_t>(vcache)) % 16 == 0 && reinterpret_cast<uintptr_t>(cos_sin) % 8 == 0,
+               "attention_window_pool_rows: pages must be 16-byte aligned");
+  const int E = P > 0 ? (B + P - 1) / P : 0;
+  const WpFront fr{src, ld, conv_w, conv_bias, taps > 1 ? conv_state : nullptr, taps > 1 ? state_slots : nullptr, taps,
+                   reinterpret_cast<const float2*>(cos_sin), rot, halves, slots};
+  attention_window_pool_heads_kernel<64, 4, 12, true><<<dim3(T, nkv), 12 * kWave, 0, s>>>(
+      nullptr, 0, static_cast<uint16_t*>(out), ldo, static_cast<const uint16_t*>(kcache), static_cast<const uint16_t*>(vcache), pk, pv, tables,
+      table_stride, row_seq, ctx_lens, head_scale, nullptr, nullptr, 0, nh, nkv, d, dv, B, scale, window, P, E, 0, 0.f, 0, 0, nullptr, 0, 1.0f, fr);
+  return launch_status("attention_window_pool_rows");
 }
 
 }  // extern "C"

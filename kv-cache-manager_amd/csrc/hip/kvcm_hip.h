@@ -214,6 +214,11 @@ int kvcm_norm_rotate_store(const float* src, int ld, const float* wq, const floa
                            float mix, float* v_keep, int ldvk, const float* cos_sin, int rot, int halves, const int* slots,
                            void* q_out, int dtype, int ldq, void* kcache, void* vcache, int T, int nh, int nkv, int d, int dv, int B,
                            hipStream_t s);
+int kvcm_attention_window_pool_rows_supported(int nh, int nkv, int d, int dv, int B);
+int kvcm_attention_window_pool_rows(const float* src, int ld, const float* conv_w, const float* conv_bias, float* conv_state, const int* state_slots,
+                                    int taps, const float* cos_sin, int rot, int halves, const int* slots, void* out, int ldo, void* kcache, void* vcache,
+                                    float* pk, float* pv, const int* tables, int table_stride, const int* row_seq, const int* ctx_lens,
+                                    const float* head_scale, int T, int nh, int nkv, int d, int dv, int B, float scale, int window, int P, hipStream_t s);
 // (attention_window_pool_tiles.hip) the same attention for runs of consecutive positions, on the matrix cores (bfloat16)
 int kvcm_attention_window_pool_tiles_supported(int d, int dv, int B);
 int kvcm_attention_window_pool_tiles(const void* q, int ldq, void* out, int ldo, const void* kcache, const void* vcache,

@@ -123,6 +123,7 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_moe_grouped),
     KVCM_ENTRY(kvcm_pool_update),
     KVCM_ENTRY(kvcm_attention_window_pool),
+    KVCM_ENTRY(kvcm_attention_window_pool_rows),
     KVCM_ENTRY(kvcm_attention_window_pool_tiles),
     KVCM_ENTRY(kvcm_selective_scan),
     KVCM_ENTRY(kvcm_scan_prepare),

@@ -141,6 +141,8 @@ def _declare(lib):
     fn("kvcm_moe_grouped", vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, i, i, vp)
     fn("kvcm_pool_update", vp, vp, i, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, i, vp)
     fn("kvcm_attention_window_pool", vp, i, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, f, i, i, i, i, f, i, i, vp, i, f, vp)
+    fn("kvcm_attention_window_pool_rows_supported", i, i, i, i, i)
+    fn("kvcm_attention_window_pool_rows", vp, i, vp, vp, vp, vp, i, vp, i, i, vp, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp)
     fn("kvcm_attention_window_pool_tiles_supported", i, i, i)
     fn("kvcm_attention_window_pool_tiles", vp, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, f, i, i, i, i, f, i, i, vp, i, f, vp)
     fn("kvcm_selective_scan", vp, i, i, vp, i, vp, vp, i, i, i, vp, vp, vp, i, vp, i, vp, vp, vp, vp, i, i, i, i, i, i, vp, C.c_longlong, i, vp)
@@ -1564,6 +1566,42 @@ def attention_window_pool(q, out, kcache, vcache, pk, pv, tables, table_stride, 
           _ptr(pk), _ptr(pv), _ptr(tables), table_stride, _ptr(row_seq), _ptr(ctx_lens), _ptr(head_scale), _ptr(dist_slope), _ptr(gate),
           gate.stride(0) if gate is not None else 0, T, nh, nkv, d, dv,
           B, float(scale), int(window), int(P), E, int(keep_first), float(softcap or 0.0), int(chunk), sink, _ptr(sink_logit), 1 if gate_heads else 0, float(out_scale), _stream())
+
+
+def attention_window_pool_rows_supported(nh, nkv, d, dv, dtype, block_size):
+    return dtype == torch.bfloat16 and bool(lib().kvcm_attention_window_pool_rows_supported(nh, nkv, d, dv, block_size))
+
+
+def attention_window_pool_rows(qkv, out, kcache, vcache, pk, pv, step, tables, table_stride, slots, nh, nkv, d, dv, scale, window, P, conv, conv_state,
+                               conv_bias=None, head_scale=None, cos_sin=None, rot=0, halves=False):
+    """A step in which every sequence runs one row (bfloat16), from the projection's 32-bit rows [q | k | v] to the attention's in one launch:
+    ``short_conv`` (``conv`` [C, taps], ``conv_bias`` before it, ``conv_state`` moved on), ``rotate_store``, ``pool_update`` and
+    ``attention_window_pool``, with their results.  ``qkv`` itself is left as it is."""
+    T, C = step.rows, (nh + nkv) * d + nkv * dv
+    _need(step.max_run == 1, "attention_window_pool_rows: every sequence runs one row")
+    _dev(qkv, out, kcache, vcache, tables, step.row_seq, step.ctx_lens, slots)
+    _f32rows(qkv, "qkv", C)
+    _rows2d(out, "out")
+    _need(out.dtype == kcache.dtype == vcache.dtype == torch.bfloat16, "attention_window_pool_rows takes bfloat16 pages and output")
+    _need(out.shape[1] >= nh * dv and out.shape[0] >= T and qkv.shape[0] >= T, "attention_window_pool_rows: shapes do not agree")
+    B, _ = _check_pool(kcache, vcache, pk, pv, nkv, d, dv, P)
+    _f32(head_scale, "head_scale", nh)
+    _f32(conv_bias, "conv_bias", C)
+    _f32(conv, "conv")
+    taps = conv.shape[1]
+    _need(conv.shape[0] == C, "the convolution's weight must be float32 [channels, taps]")
+    _need(taps == 1 or (conv_state is not None and conv_state.dtype == torch.float32 and conv_state.is_contiguous() and conv_state.is_cuda
+                        and conv_state.dim() == 3 and tuple(conv_state.shape[1:]) == (taps - 1, C)), "state must be float32 [slots, taps-1, C]")
+    for t, name in ((step.row_seq, "row_seq"), (step.ctx_lens, "ctx_lens"), (slots, "slots")):
+        _i32(t, name, T)
+    _i32(tables, "tables")
+    if rot:
+        _need(cos_sin is not None and cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.numel() >= T * rot,
+              "cos_sin must be float32 [rows, rot/2, 2]")
+    _call("kvcm_attention_window_pool_rows", _ptr(qkv), qkv.stride(0), _ptr(conv), _ptr(conv_bias), _ptr(conv_state) if taps > 1 else 0,
+          _ptr(step.state_slots) if taps > 1 else 0, taps, _ptr(cos_sin), rot, 1 if halves else 0, _ptr(slots), _ptr(out), out.stride(0), _ptr(kcache),
+          _ptr(vcache), _ptr(pk), _ptr(pv), _ptr(tables), table_stride, _ptr(step.row_seq), _ptr(step.ctx_lens), _ptr(head_scale), T, nh, nkv, d, dv, B,
+          float(scale), int(window), int(P), _stream())
 
 
 def attention_window_pool_tiles_supported(d, dv, dtype, block_size):

@@ -85,6 +85,9 @@ class ConvWindowPoolAttention(Mixer):
     def flops(self, rows, attended=0):
         return super().flops(rows) + 2.0 * attended * (self.d + self.dv) * self.nh
 
+    def conv_state(self):
+        return self.caches["conv"][0].slots(self.caches["conv"][1]) if self.params["conv"] > 1 else None
+
     def forward(self, step, h):
         ops, p, w = self.ctx.ops, self.params, self.w
         g = self.cache.group
@@ -93,20 +96,28 @@ class ConvWindowPoolAttention(Mixer):
         pk, pv = (self.cache.pooled_k(self.cache_index), self.cache.pooled_v(self.cache_index)) if pool else (None, None)
         T, K = step.rows, p["conv"]
         proj = linear32(self.ctx, step, h, w["w_qkv"], "cwp_proj")
+        slots = step.slots(g) if self.cache_owner else None
+        attn = step.ws("cwp_attn", (T, self.nh * self.dv))
+        if (step.max_run == 1 and slots is not None
+                and ops.attention_window_pool_rows_supported(self.nh, self.nkv, self.d, self.dv, attn.dtype, kc.shape[2])):
+            # every sequence runs one row: all between the two products is one launch, a workgroup per row and KV head
+            ops.attention_window_pool_rows(proj, attn, kc, vc, pk, pv, step, step.tables(g), step.table_stride(g), slots, self.nh, self.nkv,
+                                           self.d, self.dv, p["scale"], p["window"], pool, w["conv"], self.conv_state(),
+                                           conv_bias=w["bias"], head_scale=w["temp"], cos_sin=self.position.pairs_table(step),
+                                           rot=self.position.params["dims"])
+            return linear32(self.ctx, step, attn, w["w_o"], "cwp_out")
         mixed = step.ws("cwp_conv", (T, self.channels), torch.float32)
-        conv_state = self.caches["conv"][0].slots(self.caches["conv"][1]) if K > 1 else None
+        conv_state = self.conv_state()
         single = step.max_run == 1      # every sequence runs one row: the convolution leaves the new state itself
         ops.short_conv(proj, w["conv"], mixed, step, conv_state, bias_in=w["bias"], update_state=single)
         if not single:
             ops.short_conv_state(proj, conv_state, step, K, bias_in=w["bias"])
         q = step.ws("cwp_q", (T, self.nh * self.d))
-        slots = step.slots(g) if self.cache_owner else None
         ops.rotate_store(mixed, q, self.nh, self.nkv, self.d, self.dv, cos_sin=self.position.pairs_table(step),
                          rot=self.position.params["dims"], slots=slots, kcache=kc, vcache=vc, rows=T)
         if pool and self.cache_owner:
             ops.pool_update(kc, vc, pk, pv, step.tables(g), step.table_stride(g), step.row_seq, step.positions, slots,
                             self.nkv, self.d, self.dv, pool, T)
-        attn = step.ws("cwp_attn", (T, self.nh * self.dv))
         if step.max_run > 1 and ops.attention_window_pool_tiles_supported(self.d, self.dv, attn.dtype, kc.shape[2]):
             # runs of consecutive positions: 64 rows of a run share every staged key, on the matrix cores
             ops.attention_window_pool_tiles(q, attn, kc, vc, pk, pv, step.tables(g), step.table_stride(g), step.run_start,
