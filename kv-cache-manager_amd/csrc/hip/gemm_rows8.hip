@@ -28,6 +28,9 @@
 // workgroup here reads all of X, M x K per 8 or 16 output columns, from L2, which at 8 rows is as many
 // bytes as the weights themselves (a 16-row variant of this kernel lost to such products at every
 // size measured: TinyLlama sizes batch 16 1.26 -> 1.17 ms, Llama-3-8B sizes 4.82 -> 4.05 ms).
+#include <type_traits>
+#include <utility>
+
 #include "common.h"
 #include "kvcm_hip.h"
 
@@ -55,7 +58,10 @@ struct Gemm8Args {
   const float* ss_in; int tiles_in; float inv_width, eps;   // SCALED
   void* out; int ldo;                                       // kStore, kSwiglu
   float* resid; const void* g; int g_f32; uint16_t* xg; float* ss_out;   // kResidualNorm (width N)
+  int out_f32;                                              // kStore of Either
 };
+
+struct Either {};      // a result's type that the arguments name
 
 // One trip: UT units of this lane's weight rows (RG groups) and of its batch row.
 template <int RG, int UT>
@@ -64,16 +70,16 @@ struct Trip {
   Frag x[UT][2];
 };
 
+// Workgroup `block` of a product; red: NW * RG * kWave, rstd_s: 8 (SCALED), in LDS.
 template <int NW, int RG, int UT, bool SCALED, int EPI, class TO>
-__global__ void __launch_bounds__(NW * kWave) gemm8_kernel(const Gemm8Args a) {
+__device__ __forceinline__ void gemm8_block(const Gemm8Args& a, int block, f32x4* red_, float* rstd_s) {
   static_assert(NW == 4 || NW == 8, "four or eight waves share a tile's K");
   constexpr int kSlots = 2 * NW, kRowsPerWave = 8 / NW;
-  __shared__ f32x4 red[NW][RG][kWave];
-  __shared__ float rstd_s[8];
+  f32x4(*red)[RG][kWave] = reinterpret_cast<f32x4(*)[RG][kWave]>(red_);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int r = lane % 16, kq = lane / 16;
   const int half = r / 8, c = r % 8;
-  const int n0 = blockIdx.x * (kCols * RG);   // kSwiglu: N is the width of the result, RG == 2 means gate and up
+  const int n0 = block * (kCols * RG);   // kSwiglu: N is the width of the result, RG == 2 means gate and up
   const int units = a.K / kUnit;
   // this lane's slice of K: slot = 2 * wave + half of 2 * NW
   const int slot = 2 * wave + half;
@@ -210,7 +216,15 @@ __global__ void __launch_bounds__(NW * kWave) gemm8_kernel(const Gemm8Args a) {
   if constexpr (EPI == kStore) {
     if (live) {
 #pragma unroll
-      for (int g = 0; g < RG; ++g) store_f(static_cast<TO*>(a.out) + size_t(m) * a.ldo + n0 + g * kCols + n, v[g]);
+      for (int g = 0; g < RG; ++g) {
+        const size_t at = size_t(m) * a.ldo + n0 + g * kCols + n;
+        if constexpr (std::is_same_v<TO, Either>) {
+          if (a.out_f32) static_cast<float*>(a.out)[at] = v[g];
+          else store_f(static_cast<bf16_t*>(a.out) + at, v[g]);
+        } else {
+          store_f(static_cast<TO*>(a.out) + at, v[g]);
+        }
+      }
     }
   } else if constexpr (EPI == kSwiglu) {
     static_assert(EPI != kSwiglu || RG == 2, "gate and up are the two row groups");
@@ -229,8 +243,51 @@ __global__ void __launch_bounds__(NW * kWave) gemm8_kernel(const Gemm8Args a) {
       a.xg[size_t(m) * a.N + col] = float_to_bf16_bits(g_in * round_to<bf16_t>(xn));
     }
     const float sq = group_sum<8>(xn * xn);
-    if (live && n == 0) a.ss_out[size_t(m) * (a.N / kCols) + blockIdx.x] = sq;
+    if (live && n == 0) a.ss_out[size_t(m) * (a.N / kCols) + block] = sq;
   }
+}
+
+template <int NW, int RG, int UT, bool SCALED, int EPI, class TO>
+__global__ void __launch_bounds__(NW * kWave) gemm8_kernel(const Gemm8Args a) {
+  __shared__ f32x4 red[NW * RG * kWave];
+  __shared__ float rstd_s[8];
+  gemm8_block<NW, RG, UT, SCALED, EPI, TO>(a, blockIdx.x, red, rstd_s);
+}
+
+// Two products that do not wait for one another: the workgroups of both in one launch.  A launch of few rows is mostly its start, its first
+// loads and its end, and most of these products leave CUs without a workgroup.  8 rows, us, one after the other / together:
+// 2560 x 2048 and 8192 x 2048 14.5 / 12.3; 2048 x 2048 and 2048 x 4096 11.6 / 9.1; 128 x 4096 and 32 x 4096 12.0 / 6.9; 4096 x 4096 and 4096 x 8192
+// 28.3 / 24.0; 256 x 8192 and 32 x 8192 21.1 / 11.6; one row alike.
+// Form of a product: bit 0: two row groups, bit 1: the longer trips, chosen as for a launch of its own, so that the sums are the same.
+struct Gemm8Pair {
+  Gemm8Args first, second;
+  int blocks, form_first, form_second;
+};
+template <bool LONG>      // false: none has the longer trips, whose registers halve the workgroups of a CU
+__global__ void __launch_bounds__(4 * kWave) gemm8_pair_kernel(const Gemm8Pair p) {
+  __shared__ f32x4 red[4 * 2 * kWave];
+  const bool second = int(blockIdx.x) >= p.blocks;
+  const Gemm8Args& a = second ? p.second : p.first;
+  const int block = second ? blockIdx.x - p.blocks : blockIdx.x;
+  const int form = second ? p.form_second : p.form_first;
+  if (form == 0) gemm8_block<4, 1, 4, false, kStore, Either>(a, block, red, nullptr);
+  else if (form == 1) gemm8_block<4, 2, 2, false, kStore, Either>(a, block, red, nullptr);
+  if constexpr (LONG) {
+    if (form == 2) gemm8_block<4, 1, 6, false, kStore, Either>(a, block, red, nullptr);
+    else if (form == 3) gemm8_block<4, 2, 3, false, kStore, Either>(a, block, red, nullptr);
+  }
+}
+
+// Whether a product of N columns has two row groups a workgroup: once a single one would give more than about four workgroups per CU
+// (measured in whole decode steps: the head and the QKV product of a 7B model), and also where that leaves no CU
+// with more columns than it has with one (TinyLlama's QKV product: 320 tiles are two workgroups on 64 of the
+// 256 CUs either way, and 160 workgroups of two groups start and end faster: batch 8 1.027 -> 1.008 ms; at 768
+// tiles, a width of 4,096 with 8 KV heads, two groups give some CUs four tiles instead of three and are slower)
+bool two_groups(int N) {
+  constexpr int kCUs = 256;
+  const int tiles = N / kCols;
+  const bool two_fit = tiles > kCUs && 2 * ((tiles / 2 + kCUs - 1) / kCUs) <= (tiles + kCUs - 1) / kCUs;
+  return N % (2 * kCols) == 0 && (tiles > 1024 || two_fit);
 }
 
 bool operands_ok(const Gemm8Args& a) {
@@ -277,15 +334,7 @@ int kvcm_gemm8(const void* X, int ldx, const void* W, int ldw, int M, int N, int
     else { if (scaled) KVCM_G8(2, 2, true, kSwiglu, float); else KVCM_G8(2, 2, false, kSwiglu, float); }
     return launch_status("gemm8_swiglu");
   }
-  // two row groups per workgroup once a single one would give more than about four workgroups per CU
-  // (measured in whole decode steps: the head and the QKV product of a 7B model), and also where that leaves no CU
-  // with more columns than it has with one (TinyLlama's QKV product: 320 tiles are two workgroups on 64 of the
-  // 256 CUs either way, and 160 workgroups of two groups start and end faster: batch 8 1.027 -> 1.008 ms; at 768
-  // tiles, a width of 4,096 with 8 KV heads, two groups give some CUs four tiles instead of three and are slower)
-  constexpr int kCUs = 256;
-  const int tiles = N / kCols;
-  const bool two_fit = tiles > kCUs && 2 * ((tiles / 2 + kCUs - 1) / kCUs) <= (tiles + kCUs - 1) / kCUs;
-  if (N % (2 * kCols) == 0 && (tiles > 1024 || two_fit)) {
+  if (two_groups(N)) {
     const dim3 grid(N / (2 * kCols));
     if (out_dtype == kBF16) { if (scaled) KVCM_G8(2, 2, true, kStore, bf16_t); else KVCM_G8(2, 2, false, kStore, bf16_t); }
     else { if (scaled) KVCM_G8(2, 2, true, kStore, float); else KVCM_G8(2, 2, false, kStore, float); }
@@ -295,6 +344,33 @@ int kvcm_gemm8(const void* X, int ldx, const void* W, int ldw, int M, int N, int
     else { if (scaled) KVCM_G8(1, 4, true, kStore, float); else KVCM_G8(1, 4, false, kStore, float); }
   }
   return launch_status("gemm8");
+}
+
+// Y1 = X1 * W1^T and Y2 = X2 * W2^T, M rows each, in one launch: the results of two calls of kvcm_gemm8.
+int kvcm_gemm8_pair(const void* X1, int ldx1, const void* W1, int ldw1, int N1, int K1, void* out1, int dtype1, int ldo1, const void* X2, int ldx2,
+                    const void* W2, int ldw2, int N2, int K2, void* out2, int dtype2, int ldo2, int M, hipStream_t st) {
+  auto args = [&](const void* X, int ldx, const void* W, int ldw, int N, int K, void* out, int dtype, int ldo) {
+    Gemm8Args a{};
+    a.X = static_cast<const uint16_t*>(X); a.ldx = ldx; a.W = static_cast<const uint16_t*>(W); a.ldw = ldw;
+    a.M = M; a.N = N; a.K = K; a.out = out; a.ldo = ldo; a.out_f32 = dtype == kF32;
+    return a;
+  };
+  Gemm8Pair p{args(X1, ldx1, W1, ldw1, N1, K1, out1, dtype1, ldo1), args(X2, ldx2, W2, ldw2, N2, K2, out2, dtype2, ldo2), 0, 0, 0};
+  for (const Gemm8Args* a : {&p.first, &p.second}) {
+    KVCM_REQUIRE(kvcm_gemm8_supported(M, a->N, a->K), "gemm8_pair: unsupported shape M=%d N=%d K=%d", M, a->N, a->K);
+    KVCM_REQUIRE(a->out != nullptr && a->ldo >= a->N, "gemm8_pair: missing output or leading dimension below N");
+    KVCM_REQUIRE(operands_ok(*a), "gemm8_pair: operands must be 16-byte aligned with leading dimensions that are multiples of 8 and at least K");
+  }
+  KVCM_REQUIRE((dtype1 == kBF16 || dtype1 == kF32) && (dtype2 == kBF16 || dtype2 == kF32), "gemm8_pair: unknown output dtype %d or %d", dtype1, dtype2);
+  if (p.first.K < p.second.K) std::swap(p.first, p.second);      // the longer workgroups start first
+  auto form = [](const Gemm8Args& a) { return (two_groups(a.N) ? 1 : 0) | (a.K / kUnit > 8 * 2 * (two_groups(a.N) ? 2 : 4) ? 2 : 0); };
+  auto blocks = [](const Gemm8Args& a) { return a.N / (two_groups(a.N) ? 2 * kCols : kCols); };
+  p.form_first = form(p.first);
+  p.form_second = form(p.second);
+  p.blocks = blocks(p.first);
+  auto* kernel = p.form_first >= 2 || p.form_second >= 2 ? gemm8_pair_kernel<true> : gemm8_pair_kernel<false>;
+  kernel<<<p.blocks + blocks(p.second), 4 * kWave, 0, st>>>(p);
+  return launch_status("gemm8_pair");
 }
 
 // resid[M, N] += round(X * W^T); xg[M, N] = round(g * round(resid)); ss_out[M][N / 8] = sums of resid^2

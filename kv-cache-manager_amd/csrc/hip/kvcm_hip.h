@@ -82,6 +82,8 @@ int kvcm_gemm_bf16(const void* X, const void* W, void* Y, int out_dtype, int M, 
 int kvcm_gemm8_supported(int M, int N, int K);
 int kvcm_gemm8(const void* X, int ldx, const void* W, int ldw, int M, int N, int K, const float* ss_in, int tiles_in,
                float eps, void* out, int out_dtype, int ldo, int swiglu, hipStream_t stream);
+int kvcm_gemm8_pair(const void* X1, int ldx1, const void* W1, int ldw1, int N1, int K1, void* out1, int dtype1, int ldo1, const void* X2, int ldx2,
+                    const void* W2, int ldw2, int N2, int K2, void* out2, int dtype2, int ldo2, int M, hipStream_t stream);
 int kvcm_gemm8_residual_norm(const void* X, int ldx, const void* W, int ldw, int M, int N, int K, float* resid,
                              const void* g, int g_dtype, void* xg, float* ss_out, hipStream_t stream);
 // 32-bit products of few rows with the norm in front, SwiGLU or the residual addition behind (gemm_f32_few.hip); of wider rows with SwiGLU.

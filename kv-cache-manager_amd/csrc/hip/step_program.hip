@@ -88,6 +88,7 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_gemm_library),
     KVCM_ENTRY(kvcm_gemm_library_f32out),
     KVCM_ENTRY(kvcm_gemm8),
+    KVCM_ENTRY(kvcm_gemm8_pair),
     KVCM_ENTRY(kvcm_gemm8_residual_norm),
     KVCM_ENTRY(kvcm_decode_front_empty),
     KVCM_ENTRY(kvcm_decode_front),

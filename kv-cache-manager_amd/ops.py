@@ -106,6 +106,7 @@ def _declare(lib):
     fn("kvcm_fill_index", vp, C.c_longlong, C.c_uint64, i, vp)
     fn("kvcm_gemm8_supported", i, i, i)
     fn("kvcm_gemm8", vp, i, vp, i, i, i, i, vp, i, f, vp, i, i, i, vp)
+    fn("kvcm_gemm8_pair", vp, i, vp, i, i, i, vp, i, i, vp, i, vp, i, i, i, vp, i, i, i, vp)
     fn("kvcm_gemm8_residual_norm", vp, i, vp, i, i, i, i, vp, vp, i, vp, vp, vp)
     fn("kvcm_embed_scaled", vp, vp, i, vp, i, i, i, f, vp, vp, i, vp)
     fn("kvcm_gated_act", vp, i, vp, vp, i, vp, i, i, i, i, i, f, vp)
@@ -862,6 +863,28 @@ def gemm(x, w, out, scratch=None, keep_partial=False, tuning=None, unsplit=False
     _call("kvcm_gemm_bf16", _ptr(x), _ptr(w), _ptr(out), _DT[out.dtype], M, N, K, x.stride(0), w.stride(0),
                                 out.stride(0), _stream())
     return out
+
+
+def gemm_pair(x1, w1, out1, x2, w2, out2, split1=True, split2=True):
+    """out1 = x1 @ w1^T and out2 = x2 @ w2^T, which do not wait for one another, in one launch with the results of ``gemm(..., unsplit=True)``: -> True.
+    False: nothing was done (a product is none that ``gemm`` runs unsplit in gemm_rows8.hip).  ``split1``, ``split2``: ``gemm`` would have scratch
+    for slices."""
+    for x, w, out, split in ((x1, w1, out1, split1), (x2, w2, out2, split2)):
+        if isinstance(x, (NormedRows, RowsToNorm)) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+            return False
+        _dev(x, w, out)
+        for t, n in ((x, "x"), (w, "w"), (out, "out")):
+            _rows2d(t, n)
+        (M, K), N = x.shape, w.shape[0]
+        _need(w.shape[1] == K and out.shape == (M, N), f"gemm shapes do not agree: {tuple(x.shape)} {tuple(w.shape)} {tuple(out.shape)}")
+        if _library_takes(M, N, K) or not _rows8_takes(M, N, K, out.dtype, split) or not _in_pieces(x, w):
+            return False
+    if x1.shape[0] != x2.shape[0]:
+        return False
+    args = [a for x, w, out in ((x1, w1, out1), (x2, w2, out2))
+            for a in (_ptr(x), x.stride(0), _ptr(w), w.stride(0), w.shape[0], w.shape[1], _ptr(out), _DT[out.dtype], out.stride(0))]
+    _call("kvcm_gemm8_pair", *args, x1.shape[0], _stream())
+    return True
 
 
 # act(gate) * up in a product's epilogue (gemm_tiles.h: TileAct), without roundings before the end, as ``gated_act`` computes it

@@ -7,7 +7,8 @@ import torch
 
 from ..registry import MIXERS, POSITIONS
 from .base import KVCacheNeed, Mixer, ParamSpec, PartSpec, PositionEncoding, StateNeed
-from .chain_norm_parts import BranchPair, f32_params, linear32
+from .chain_norm_parts import BranchPair, f32_params
+from .llama_parts import run_stages, side_by_side
 
 
 @POSITIONS.register("rotary_pairs")
@@ -88,14 +89,20 @@ class ConvWindowPoolAttention(Mixer):
     def conv_state(self):
         return self.caches["conv"][0].slots(self.caches["conv"][1]) if self.params["conv"] > 1 else None
 
+    buffers = "cwp"
+
     def forward(self, step, h):
+        return run_stages(self.ctx, step, self.stages(step, h))
+
+    def stages(self, step, h):
+        """``forward``, with the products handed out (side_by_side)."""
         ops, p, w = self.ctx.ops, self.params, self.w
         g = self.cache.group
         kc, vc = self.cache.k(self.cache_index), self.cache.v(self.cache_index)
         pool = p["pool"] if p["window"] > 0 else 0
         pk, pv = (self.cache.pooled_k(self.cache_index), self.cache.pooled_v(self.cache_index)) if pool else (None, None)
         T, K = step.rows, p["conv"]
-        proj = linear32(self.ctx, step, h, w["w_qkv"], "cwp_proj")
+        proj = yield h, w["w_qkv"], "cwp_proj", torch.float32
         slots = step.slots(g) if self.cache_owner else None
         attn = step.ws("cwp_attn", (T, self.nh * self.dv))
         if (step.max_run == 1 and slots is not None
@@ -105,7 +112,7 @@ class ConvWindowPoolAttention(Mixer):
                                            self.d, self.dv, p["scale"], p["window"], pool, w["conv"], self.conv_state(),
                                            conv_bias=w["bias"], head_scale=w["temp"], cos_sin=self.position.pairs_table(step),
                                            rot=self.position.params["dims"])
-            return linear32(self.ctx, step, attn, w["w_o"], "cwp_out")
+            return (yield attn, w["w_o"], "cwp_out", torch.float32)
         mixed = step.ws("cwp_conv", (T, self.channels), torch.float32)
         conv_state = self.conv_state()
         single = step.max_run == 1      # every sequence runs one row: the convolution leaves the new state itself
@@ -123,10 +130,10 @@ class ConvWindowPoolAttention(Mixer):
             ops.attention_window_pool_tiles(q, attn, kc, vc, pk, pv, step.tables(g), step.table_stride(g), step.run_start,
                                             step.seq_start, step.seqs, step.max_run, self.nh, self.nkv, self.d, self.dv,
                                             p["scale"], p["window"], pool, head_scale=w["temp"])
-            return linear32(self.ctx, step, attn, w["w_o"], "cwp_out")
+            return (yield attn, w["w_o"], "cwp_out", torch.float32)
         ops.attention_window_pool(q, attn, kc, vc, pk, pv, step.tables(g), step.table_stride(g), step.row_seq, step.ctx_lens,
                                   self.nh, self.nkv, self.d, self.dv, p["scale"], p["window"], pool, head_scale=w["temp"], rows=T)
-        return linear32(self.ctx, step, attn, w["w_o"], "cwp_out")
+        return (yield attn, w["w_o"], "cwp_out", torch.float32)
 
 
 @MIXERS.register("parallel_mixers")
@@ -157,6 +164,10 @@ class ParallelMixers(Mixer):
         super().bind(f32_params(tensors))
 
     def forward(self, step, h):
-        a = self.left.forward(step, h)
-        b = self.right.forward(step, h)
+        left, right = self.left, self.right
+        if getattr(left, "buffers", None) and getattr(right, "buffers", None) and left.buffers != right.buffers:
+            a, b = side_by_side(self.ctx, step, left.stages(step, h), right.stages(step, h))
+        else:
+            a = left.forward(step, h)
+            b = right.forward(step, h)
         return BranchPair(a, self.w["w_left"], b, self.w["w_right"], self.params.get("combine", 0.5))

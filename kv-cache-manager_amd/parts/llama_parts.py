@@ -22,6 +22,54 @@ def _linear(ctx, step, x, w, name, keep_partial=False, dtype=None):
                         tuning=step.tune_products, unsplit=True)
 
 
+def linear_pair(ctx, step, first, second):
+    """Two products that do not wait for one another, each (x, w, name, dtype) of ``_linear``: in one launch where they are of few rows."""
+    ops = ctx.ops
+    if step.rows <= ops.FUSED_NORM_MAX_ROWS:
+        outs = [step.ws(name, (x.shape[0], w.shape[0]), dtype) for x, w, name, dtype in (first, second)]
+        splits = [step.scratch(name, x.shape[0], *w.shape) is not None for x, w, name, _ in (first, second)]
+        if ops.gemm_pair(*first[:2], outs[0], *second[:2], outs[1], *splits):
+            return outs
+    return [_linear(ctx, step, x, w, name, dtype=dtype) for x, w, name, dtype in (first, second)]
+
+
+# A mixer that has ``stages(step, h)`` runs as a generator: it yields its larger products, (x, w, name, dtype) of ``_linear``, takes their results
+# and returns its output, so that two mixers on one input can run in step.  ``buffers``: what its work buffers' names begin with; in step
+# only with a mixer of other names.
+def run_stages(ctx, step, stages):
+    try:
+        product = next(stages)
+        while True:
+            x, w, name, dtype = product
+            product = stages.send(_linear(ctx, step, x, w, name, dtype=dtype))
+    except StopIteration as end:
+        return end.value
+
+
+def side_by_side(ctx, step, left, right):
+    """Two mixers' stages in step: the first products of both together, then what follows each, and so on.  -> both outputs."""
+    both, asked, outputs = [left, right], [None, None], [None, None]
+
+    def go(i, result):
+        try:
+            asked[i] = both[i].send(result)
+        except StopIteration as end:
+            asked[i], outputs[i] = None, end.value
+
+    go(0, None)
+    go(1, None)
+    while asked[0] is not None or asked[1] is not None:
+        if asked[0] is not None and asked[1] is not None:
+            results = linear_pair(ctx, step, *asked)
+        else:
+            results = [q and _linear(ctx, step, *q[:3], dtype=q[3]) for q in asked]
+        waits = [q is not None for q in asked]
+        for i in (0, 1):
+            if waits[i]:
+                go(i, results[i])
+    return outputs
+
+
 def _to_residual(ctx, step, x, w, name, defer=False):
     """A part's last product, whose result goes to the residual stream.  For decode steps of a few
     rows it is handed on unrun (ops.PendingProduct): the norm that follows runs it with the addition

@@ -10,7 +10,7 @@ from ..registry import MIXERS
 from .base import Mixer, ParamSpec, StateNeed
 from .chain_norm_parts import f32_params, linear32
 from .ends import EndsMixer
-from .llama_parts import _linear
+from .llama_parts import linear_pair, run_stages
 
 _SMALL = ("conv", "conv_bias", "dt_bias", "a_log", "d_skip", "a_bias", "w0", "w2", "norm")
 
@@ -58,10 +58,16 @@ class SelectiveScanMixer(_StatefulMixer):
         p = self.params
         return super().flops(rows) + rows * p["inner"] * (6.0 * p["state"] + 2.0 * p["conv"])
 
+    buffers = "scan"
+
     def forward(self, step, h):
+        return run_stages(self.ctx, step, self.stages(step, h))
+
+    def stages(self, step, h):
+        """``forward``, with the products handed out (side_by_side)."""
         ops, p, w = self.ctx.ops, self.params, self.w
         C, N, R, K = p["inner"], p["state"], p["dt_rank"], p["conv"]
-        xz = linear32(self.ctx, step, h, w["w_in"], "scan_xz")
+        xz = yield h, w["w_in"], "scan_xz", torch.float32
         conv_state = self.state("conv") if K > 1 else None
         x = step.ws("scan_x", (step.rows, C))
         single = step.max_run == 1      # every sequence runs one row: the convolution leaves the new state itself
@@ -69,8 +75,7 @@ class SelectiveScanMixer(_StatefulMixer):
         if not single:
             ops.short_conv_state(xz, conv_state, step, K)
         # the step size's low-rank input feeds a product (compute dtype); B and C enter the recurrence (32-bit)
-        low = _linear(self.ctx, step, x, w["w_x"][:R], "scan_dt_low")
-        bc = linear32(self.ctx, step, x, w["w_x"][R:], "scan_bc")
+        low, bc = linear_pair(self.ctx, step, (x, w["w_x"][:R], "scan_dt_low", None), (x, w["w_x"][R:], "scan_bc", torch.float32))
         dt = linear32(self.ctx, step, low, w["w_dt"], "scan_dt")
         y = step.ws("scan_y", (step.rows, C))
         # runs of some length: step sizes and gates made ahead; long runs: walked in pieces, all pieces at once.  Two passes pay
@@ -83,7 +88,7 @@ class SelectiveScanMixer(_StatefulMixer):
             carry = step.flat("scan_carry", ops.selective_scan_carry_floats(max(step.rows, step.limits.max_tokens), step.limits.max_seqs, C, N))
         ops.selective_scan(x, dt, w["dt_bias"], bc, 0, N, w["a_log"], w["d_skip"], xz[:, C:], y, self.state("scan"), step,
                            prepare=step.max_run >= 16, carry=carry)
-        return linear32(self.ctx, step, y, w["w_o"], "scan_out")
+        return (yield y, w["w_o"], "scan_out", torch.float32)
 
 
 @MIXERS.register("general_delta")
