@@ -304,6 +304,12 @@ int kvcm_moe_down(const void* act, int dtype, const void* w_down, const int* cho
 // (moe_few.hip) are steps of T rows best left to the two products above, which then run on the matrix cores, an expert's weights read
 // once for all its rows?  (bfloat16)  Those two kernels, whatever is the faster.
 int kvcm_moe_few_takes(int T, int K, int F, int H, int top, int E, int kind);
+int kvcm_moe_few_beside_supported(int T, int K, int F, int H, int top, int E, int Fs);
+int kvcm_moe_few_beside_takes(int T, int K, int F, int H, int top, int E, int Fs);
+int kvcm_moe_few_beside_up(const void* h, int ldh, const void* w_up, int* chosen, float* weight, const int* tokens, const int* table, int vocab, int ld_table,
+                           const void* w_shared_up, void* act_shared, int Fs, void* act, int T, int K, int F, int H, int top, int E, int weigh_input, hipStream_t s);
+int kvcm_moe_few_beside_down(const void* act, const void* w_down, const int* chosen, const float* weight, const void* act_shared, const void* w_shared_down, int Fs,
+                             float* out, int T, int K, int F, int H, int top, int E, hipStream_t s);
 int kvcm_moe_few_up(const void* h, int ldh, const void* w_up, const int* chosen, void* act, int T, int K, int F, int top, int E, int kind,
                     const float* in_weight, hipStream_t s);
 int kvcm_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T, int F,

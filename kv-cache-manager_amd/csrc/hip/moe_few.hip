@@ -14,6 +14,9 @@
 //          scratch, no further launch).  Its eight waves take the experts in turn; an instruction serves two halves of K (operand
 //          rows and columns 0..7 the first half, 8..15 the second, only the two diagonal blocks mean anything).
 //
+// A shared feed-forward that runs for every row, and a route by a table, may run in the same two launches (MoeBeside): what they cost otherwise
+// is mostly the start and the end of launches that leave CUs idle.
+//
 // Measured over weights that go round several copies, row by row / here, us: 8 rows, 8 experts of which a row uses 2, width
 // 2,048, 1,408 columns an expert: up 31.3 / 19.7 (92 MB, 4.7 TB/s), down 17.3 / 12.6; 15 rows 51.9 / 20.1 and 28.9 / 14.0; 4 rows 18.4 /
 // 13.3 and 11.3 / 9.3; width 4,096, 3,584 columns, 8 rows: 135 / 85 and 69 / 48.  Which sizes come here: up_gains, down_gains, below.
@@ -47,30 +50,65 @@ __device__ __forceinline__ int nth_pair(unsigned long long pairs, int n, int mos
 // GATED: rows of the matrix are 2F, sixteen gate rows, sixteen up rows, ...; else F, and KIND 0 square(relu), 2 gelu
 constexpr int kUpWaves = 4, kUpTrip = 2;      // waves that divide K, units of a trip
 
-template <int KIND>
+// What runs beside the experts in their launches: a feed-forward of silu(gate) * up for every row (F columns; w_up [gate rows | up rows], act [T, F],
+// w_down [H, F]), and the route by a table per token id (tokens null: none), which is left for the second launch.
+struct MoeBeside {
+  const uint16_t* w_up; uint16_t* act; int F;
+  const int* tokens; const int* table; int vocab, ld_table;
+  int* chosen; float* weight; float in_scale;      // in_scale: the factor on what an expert reads where no in_weight is given
+};
+
+// BESIDE: the first `beside_rows` rows of the grid are the shared feed-forward's, 16 columns a workgroup.
+template <int KIND, bool BESIDE>
 __global__ void __launch_bounds__(kUpWaves * kWave, 3)
     moe_few_up_kernel(const uint16_t* __restrict__ h, int ldh, const uint16_t* __restrict__ w_up, const int* __restrict__ chosen,
-                      uint16_t* __restrict__ act, int n, int K, int F, int top, int E, const float* __restrict__ in_weight) {
+                      uint16_t* act, int n, int K, int F, int top, int E, const float* __restrict__ in_weight, const MoeBeside by, int beside_rows) {
   constexpr bool GATED = KIND == 1;
+  static_assert(GATED || !BESIDE, "a shared feed-forward beside gated experts only");
   __shared__ f32x4 red[kUpWaves][2][kWave];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
-  const int mine = blockIdx.y;
-  const int ch = lane < n ? chosen[lane] : -1;
-  const int e = __builtin_amdgcn_readlane(ch, mine);
-  if (e < 0 || e >= E) return;
-  unsigned long long pairs = __ballot(ch == e);
-  if (__ffsll(pairs) - 1 != mine) return;
   const int r = lane % 16, kq = lane / 16;
-  const int rows = GATED ? 2 * F : F;
-  const uint16_t* wrow = w_up + (size_t(e) * rows + size_t(blockIdx.x) * 32 + r) * K + kq * 16;
-  const size_t next = size_t(16) * K;
+  const bool shared = BESIDE && int(blockIdx.y) < beside_rows;
+  const int tile = shared ? int(blockIdx.y) * gridDim.x + blockIdx.x : blockIdx.x;      // of 32 rows
+  const uint16_t* wrow;
+  size_t next;
+  unsigned long long pairs;
+  if (shared) {      // every row is a pair of its own
+    if (tile * 16 >= by.F) return;
+    wrow = by.w_up + (size_t(tile) * 16 + r) * K + kq * 16;
+    next = size_t(by.F) * K;
+    const int T = n / top;
+    pairs = T >= 64 ? ~0ull : (1ull << T) - 1;
+  } else {
+    const int mine = int(blockIdx.y) - (BESIDE ? beside_rows : 0);
+    int ch = -1;
+    if (lane < n) {
+      if (BESIDE && by.tokens) {
+        const int tok = by.tokens[lane / top];
+        ch = tok >= 0 && tok < by.vocab ? by.table[size_t(tok) * by.ld_table + lane % top] : -1;
+      } else {
+        ch = chosen[lane];
+      }
+    }
+    if (BESIDE && by.tokens && mine == 0 && tile == 0 && int(threadIdx.x) < n) {
+      by.chosen[threadIdx.x] = ch;
+      by.weight[threadIdx.x] = 1.0f / float(top);
+    }
+    const int e = __builtin_amdgcn_readlane(ch, mine);
+    if (e < 0 || e >= E) return;
+    pairs = __ballot(ch == e);
+    if (__ffsll(pairs) - 1 != mine) return;
+    wrow = w_up + (size_t(e) * (GATED ? 2 * F : F) + size_t(tile) * 32 + r) * K + kq * 16;
+    next = size_t(16) * K;
+  }
+  const int per_row = shared ? 1 : top;
   const int units = K / kUnit, u_lo = units * wave / kUpWaves, u_hi = units * (wave + 1) / kUpWaves;
   struct Trip {
     Frag w[2][kUpTrip][2], x[kUpTrip][2];
   };
   for (; pairs;) {      // (more than sixteen pairs of one expert: the weights again, from a cache)
     const int count = __popcll(pairs) < 16 ? __popcll(pairs) : 16;
-    const uint16_t* xrow = h + size_t(nth_pair(pairs, r, 16) / top) * ldh + kq * 16;
+    const uint16_t* xrow = h + size_t(nth_pair(pairs, r, 16) / per_row) * ldh + kq * 16;
     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     auto request = [&](int u0, Trip& t) {      // past the slice: its last unit again, not multiplied
 #pragma unroll
@@ -113,19 +151,21 @@ __global__ void __launch_bounds__(kUpWaves * kWave, 3)
     const int m = threadIdx.x / 16, c = threadIdx.x % 16;
     if (m < count) {
       const int pair = nth_pair(pairs, m, 16);
-      const float g = in_weight ? in_weight[pair] : 1.f;
+      const float g = shared ? 1.f : in_weight ? in_weight[pair] : BESIDE ? by.in_scale : 1.f;
       float z[2] = {0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < kUpWaves; ++w)
 #pragma unroll
         for (int t = 0; t < 2; ++t) z[t] += red[w][t][m / 4 * 16 + c][m % 4];
-      if constexpr (GATED) {
-        act[size_t(pair) * F + size_t(blockIdx.x) * 16 + c] = float_to_bf16_bits(silu<bf16_t>(g * z[0]) * (g * z[1]));
+      if (shared) {      // (with the exact functions, as the products of gate and up rows have it)
+        if constexpr (BESIDE) by.act[size_t(pair) * by.F + size_t(tile) * 16 + c] = float_to_bf16_bits(silu<float>(z[0]) * z[1]);
+      } else if constexpr (GATED) {
+        act[size_t(pair) * F + size_t(tile) * 16 + c] = float_to_bf16_bits(silu<bf16_t>(g * z[0]) * (g * z[1]));
       } else {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const float y = g * z[t], p = fmaxf(y, 0.f);
-          act[size_t(pair) * F + size_t(blockIdx.x) * 32 + t * 16 + c] = float_to_bf16_bits(KIND == 2 ? gelu_exact<bf16_t>(y) : p * p);
+          act[size_t(pair) * F + size_t(tile) * 32 + t * 16 + c] = float_to_bf16_bits(KIND == 2 ? gelu_exact<bf16_t>(y) : p * p);
         }
       }
     }
@@ -134,39 +174,40 @@ __global__ void __launch_bounds__(kUpWaves * kWave, 3)
   }
 }
 
-constexpr int kDownWaves = 8, kDownTrip = 4, kMostPairs = 64;
+constexpr int kDownWaves = 8, kBesideWaves = 4, kMostPairs = 64;
 
-__global__ void __launch_bounds__(kDownWaves * kWave, 2)
+// BESIDE: four more waves take the shared feed-forward's second product, a quarter of its columns each, which is added to the experts' sum in wave
+// order.  (As one more turn of the experts' waves it waits for theirs: 19.5 us, as much as two launches.)
+template <bool BESIDE>
+__global__ void __launch_bounds__((kDownWaves + (BESIDE ? kBesideWaves : 0)) * kWave, BESIDE ? 3 : 2)
     moe_few_down_kernel(const uint16_t* __restrict__ act, const uint16_t* __restrict__ w_down, const int* __restrict__ chosen,
                         const float* __restrict__ weight, const float* __restrict__ add, float* __restrict__ out, int T, int F,
-                        int H, int top, int E) {
+                        int H, int top, int E, const uint16_t* __restrict__ by_act, const uint16_t* __restrict__ by_down, int by_F) {
   __shared__ float z[kMostPairs][8];
+  __shared__ float by_z[BESIDE ? kBesideWaves : 1][BESIDE ? kMostPairs : 1][8];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int n = T * top, n0 = blockIdx.x * 8;
   const int em = threadIdx.x / 8, en = threadIdx.x % 8;      // the last step's (row, column)
-  const float start = add && em < T ? add[size_t(em) * H + n0 + en] : 0.f;
+  const float start = !BESIDE && add && em < T ? add[size_t(em) * H + n0 + en] : 0.f;
   const int ch = lane < n ? chosen[lane] : -1;
   unsigned long long left = __ballot(ch >= 0 && ch < E);
   const int r = lane % 16, kq = lane / 16, half = r / 8, c = r % 8;
-  const int units = F / kUnit, n_main = units / 2, n_max = units - n_main;      // the second half may have a unit more
-  const int u_lo = half * n_main, cnt = half ? n_max : n_main;
+  constexpr int kDownTrip = BESIDE ? 3 : 4;      // (twelve waves have fewer registers each)
   struct Trip {
     Frag w[kDownTrip][2], x[kDownTrip][2];
   };
-  for (int i = 0; left; ++i) {      // the experts in the order of their first pair, each wave every eighth
-    const int e = __builtin_amdgcn_readlane(ch, __ffsll(left) - 1);
-    unsigned long long pairs = __ballot(ch == e);
-    left &= ~pairs;
-    if (i % kDownWaves != wave) continue;
-    const uint16_t* wrow = w_down + (size_t(e) * H + n0 + c) * F + kq * 16;
+  // `units` of K from u0 on: eight columns' rows of a matrix (wrow: this lane's) with the rows of `pairs` (xs, `width` apart), to zs
+  auto turn = [&](const uint16_t* wrow, const uint16_t* xs, int width, int u0, int units, unsigned long long pairs, float(*zs)[8]) {
+    const int n_main = units / 2, n_max = units - n_main;      // the second half may have a unit more
+    const int u_lo = half * n_main, cnt = half ? n_max : n_main;
     while (pairs) {      // (more than eight pairs of one expert: the weights again, from a cache)
-      const uint16_t* xrow = act + size_t(nth_pair(pairs, c, 8)) * F + kq * 16;
+      const uint16_t* xrow = xs + size_t(nth_pair(pairs, c, 8)) * width + kq * 16;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
       auto request = [&](int j0, Trip& t) {      // past this half's slice: its last unit again (or the row's first), not multiplied
 #pragma unroll
         for (int d = 0; d < kDownTrip; ++d) {
           const int j = j0 + d < cnt ? j0 + d : (cnt > 0 ? cnt - 1 : 0);
-          const size_t off = size_t(u_lo + j < units ? u_lo + j : 0) * kUnit;
+          const size_t off = size_t(u0 + (u_lo + j < units ? u_lo + j : 0)) * kUnit;
 #pragma unroll
           for (int q = 0; q < 2; ++q) {
             t.w[d][q].u = *reinterpret_cast<const uint4*>(wrow + off + q * 8);
@@ -208,10 +249,20 @@ __global__ void __launch_bounds__(kDownWaves * kWave, 2)
       for (int q = 0; q < 4; ++q) {
         const float far = __shfl(acc[q], (lane + 40) % kWave, kWave);
         const int m = 4 * kq + q;
-        if (lane < 32 && r < 8 && m < count) z[nth_pair(pairs, m, 8)][c] = acc[q] + far;
+        if (lane < 32 && r < 8 && m < count) zs[nth_pair(pairs, m, 8)][c] = acc[q] + far;
       }
       for (int k = 0; k < count; ++k) pairs &= pairs - 1;
     }
+  };
+  for (int i = 0; left; ++i) {      // the experts in the order of their first pair, each wave every eighth
+    const int e = __builtin_amdgcn_readlane(ch, __ffsll(left) - 1);
+    const unsigned long long pairs = __ballot(ch == e);
+    left &= ~pairs;
+    if (i % kDownWaves == wave) turn(w_down + (size_t(e) * H + n0 + c) * F + kq * 16, act, F, 0, F / kUnit, pairs, z);
+  }
+  if (BESIDE && wave >= kDownWaves) {
+    const int q = wave - kDownWaves, units = by_F / kUnit, u0 = units * q / kBesideWaves, u1 = units * (q + 1) / kBesideWaves;
+    turn(by_down + size_t(n0 + c) * by_F + kq * 16, by_act, by_F, u0, u1 - u0, T >= 64 ? ~0ull : (1ull << T) - 1, by_z[q]);
   }
   __syncthreads();
   if (em >= T) return;
@@ -221,7 +272,14 @@ __global__ void __launch_bounds__(kDownWaves * kWave, 2)
     if (e < 0 || e >= E) continue;
     sum = fmaf(weight ? weight[pair] : 1.f, z[pair][en], sum);
   }
-  out[size_t(em) * H + n0 + en] = add ? start + sum : sum;
+  if constexpr (BESIDE) {
+    float shared = by_z[0][em][en];
+#pragma unroll
+    for (int w = 1; w < kBesideWaves; ++w) shared += by_z[w][em][en];
+    out[size_t(em) * H + n0 + en] = shared + sum;
+  } else {
+    out[size_t(em) * H + n0 + en] = add ? start + sum : sum;
+  }
 }
 
 }  // namespace
@@ -278,8 +336,8 @@ void launch_moe_few_up(const void* h, int ldh, const void* w_up, const int* chos
                        const float* in_weight, hipStream_t s) {
   const dim3 grid((kind == 1 ? 2 * F : F) / 32, T * top);
 #define KVCM_FEW_UP(KIND)                                                                                                       \
-  moe_few_up_kernel<KIND><<<grid, kUpWaves * kWave, 0, s>>>(static_cast<const uint16_t*>(h), ldh, static_cast<const uint16_t*>(w_up), chosen, \
-                                               static_cast<uint16_t*>(act), T * top, K, F, top, E, in_weight)
+  moe_few_up_kernel<KIND, false><<<grid, kUpWaves * kWave, 0, s>>>(static_cast<const uint16_t*>(h), ldh, static_cast<const uint16_t*>(w_up), chosen, \
+                                               static_cast<uint16_t*>(act), T * top, K, F, top, E, in_weight, MoeBeside{}, 0)
   if (kind == 1) KVCM_FEW_UP(1);
   else if (kind == 2) KVCM_FEW_UP(2);
   else KVCM_FEW_UP(0);
@@ -288,8 +346,8 @@ void launch_moe_few_up(const void* h, int ldh, const void* w_up, const int* chos
 
 void launch_moe_few_down(const void* act, const void* w_down, const int* chosen, const float* weight, const float* add, float* out, int T,
                          int F, int H, int top, int E, hipStream_t s) {
-  moe_few_down_kernel<<<H / 8, kDownWaves * kWave, 0, s>>>(static_cast<const uint16_t*>(act), static_cast<const uint16_t*>(w_down), chosen,
-                                                           weight, add, out, T, F, H, top, E);
+  moe_few_down_kernel<false><<<H / 8, kDownWaves * kWave, 0, s>>>(static_cast<const uint16_t*>(act), static_cast<const uint16_t*>(w_down), chosen,
+                                                           weight, add, out, T, F, H, top, E, nullptr, nullptr, 0);
 }
 
 }  // namespace kvcm
@@ -326,6 +384,49 @@ int kvcm_moe_few_down(const void* act, const void* w_down, const int* chosen, co
   KVCM_REQUIRE(down_fits(kBF16, act, T, F, H, top) && reinterpret_cast<uintptr_t>(w_down) % 16 == 0, "moe_few_down: unsupported sizes or alignment");
   launch_moe_few_down(act, w_down, chosen, weight, add, out, T, F, H, top, E, s);
   return launch_status("moe_few_down");
+}
+
+// The two products with a shared feed-forward of Fs columns beside gated experts (silu, no biases): silu(gate) * up of w_shared_up [2 Fs, K] (gate rows, up
+// rows) to act_shared [T, Fs], and out = act_shared w_shared_down^T + the experts' sum.  tokens (null: chosen and weight are read): the route
+// by a table per token id as kvcm_moe_table_route leaves it in chosen and weight.  weigh_input: the weights are factors on what an expert reads.
+int kvcm_moe_few_beside_supported(int T, int K, int F, int H, int top, int E, int Fs) {
+  return T > 0 && E > 0 && top > 0 && Fs > 0 && Fs % kUnit == 0 && F / 16 > 0 && up_fits(kBF16, nullptr, 0, T, K, F, top) && down_fits(kBF16, nullptr, T, F, H, top);
+}
+// Are they the faster?  Up to 8 rows: two launches of 0.52 to 1.00 of the time of the four (five) one after the other, also where those are the row-by-row
+// kernels (us; width 2,048, 1,408 columns an expert, two of 8, shared 2,816: one row 25.2 / 20.9, 4 rows 43.4 / 32.3, 8 rows 51.8 / 45.0; 704, four of 16, shared 704: 8
+// rows 51.1 / 41.4; width 1,024, 704, shared 1,408: 8 rows 28.8 / 21.9; width 4,096, 3,584, shared 7,168: 1 row 80.0 / 74.0, 8 rows 150.4 / 147.3, shared 11,264: 120.1 /
+// 120.3).  Up to 16 rows while the shared matrices are small: sixteen of the experts' pairs are one pass, but the products of gate and up rows that the
+// shared ones take otherwise read them at a better rate (2,816: 12 rows 47.2 / 43.8, 16 rows 52.9 / 50.1; 5,632: 57.2 / 58.0; 4,096 x 7,168: 182.5 / 189.6).
+int kvcm_moe_few_beside_takes(int T, int K, int F, int H, int top, int E, int Fs) {
+  const long long shared = 2ll * Fs * K;
+  return kvcm_moe_few_beside_supported(T, K, F, H, top, E, Fs) && E <= kDownExperts && ((T <= 8 && shared <= 100000000) || (T <= 16 && shared <= 16000000));
+}
+int kvcm_moe_few_beside_up(const void* h, int ldh, const void* w_up, int* chosen, float* weight, const int* tokens, const int* table, int vocab, int ld_table,
+                           const void* w_shared_up, void* act_shared, int Fs, void* act, int T, int K, int F, int H, int top, int E, int weigh_input, hipStream_t s) {
+  if (T == 0) return 0;
+  KVCM_REQUIRE(kvcm_moe_few_beside_supported(T, K, F, H, top, E, Fs) && ldh >= K && ldh % 8 == 0, "moe_few_beside_up: unsupported sizes");
+  KVCM_REQUIRE(h && w_up && chosen && weight && w_shared_up && act_shared && act && (!tokens || (table && vocab > 0 && ld_table >= top)), "moe_few_beside_up: null operand");
+  KVCM_REQUIRE((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(w_up) | reinterpret_cast<uintptr_t>(w_shared_up)) % 16 == 0,
+               "moe_few_beside_up: operands must be 16-byte aligned");
+  const int tiles = 2 * F / 32, beside = (Fs / 16 + tiles - 1) / tiles;
+  KVCM_REQUIRE(beside + T * top <= 65535, "moe_few_beside_up: the shared feed-forward is too wide");
+  const MoeBeside by{static_cast<const uint16_t*>(w_shared_up), static_cast<uint16_t*>(act_shared), Fs, tokens, table, vocab, ld_table, chosen, weight,
+                     tokens && weigh_input ? 1.0f / float(top) : 1.0f};
+  moe_few_up_kernel<1, true><<<dim3(tiles, beside + T * top), kUpWaves * kWave, 0, s>>>(
+      static_cast<const uint16_t*>(h), ldh, static_cast<const uint16_t*>(w_up), chosen, static_cast<uint16_t*>(act), T * top, K, F, top, E,
+      !tokens && weigh_input ? weight : nullptr, by, beside);
+  return launch_status("moe_few_beside_up");
+}
+int kvcm_moe_few_beside_down(const void* act, const void* w_down, const int* chosen, const float* weight, const void* act_shared, const void* w_shared_down, int Fs,
+                             float* out, int T, int K, int F, int H, int top, int E, hipStream_t s) {
+  if (T == 0) return 0;
+  KVCM_REQUIRE(kvcm_moe_few_beside_supported(T, K, F, H, top, E, Fs), "moe_few_beside_down: unsupported sizes");
+  KVCM_REQUIRE(act && w_down && chosen && act_shared && w_shared_down && out, "moe_few_beside_down: null operand");
+  KVCM_REQUIRE((reinterpret_cast<uintptr_t>(act) | reinterpret_cast<uintptr_t>(w_down) | reinterpret_cast<uintptr_t>(act_shared) | reinterpret_cast<uintptr_t>(w_shared_down)) % 16 == 0,
+               "moe_few_beside_down: operands must be 16-byte aligned");
+  moe_few_down_kernel<true><<<H / 8, (kDownWaves + kBesideWaves) * kWave, 0, s>>>(static_cast<const uint16_t*>(act), static_cast<const uint16_t*>(w_down), chosen, weight, nullptr, out, T, F, H,
+                                                                top, E, static_cast<const uint16_t*>(act_shared), static_cast<const uint16_t*>(w_shared_down), Fs);
+  return launch_status("moe_few_beside_down");
 }
 
 }  // extern "C"

@@ -120,6 +120,8 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_moe_up),
     KVCM_ENTRY(kvcm_moe_down),
     KVCM_ENTRY(kvcm_moe_few_up),
+    KVCM_ENTRY(kvcm_moe_few_beside_up),
+    KVCM_ENTRY(kvcm_moe_few_beside_down),
     KVCM_ENTRY(kvcm_moe_few_down),
     KVCM_ENTRY(kvcm_moe_grouped),
     KVCM_ENTRY(kvcm_pool_update),

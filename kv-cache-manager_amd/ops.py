@@ -134,6 +134,9 @@ def _declare(lib):
     fn("kvcm_moe_up", vp, i, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
     fn("kvcm_moe_down", vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, vp)
     fn("kvcm_moe_few_takes", i, i, i, i, i, i, i)
+    fn("kvcm_moe_few_beside_takes", i, i, i, i, i, i, i)
+    fn("kvcm_moe_few_beside_up", vp, i, vp, vp, vp, vp, vp, i, i, vp, vp, i, vp, i, i, i, i, i, i, i, vp)
+    fn("kvcm_moe_few_beside_down", vp, vp, vp, vp, vp, vp, i, vp, i, i, i, i, i, i, vp)
     fn("kvcm_moe_few_up", vp, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
     fn("kvcm_moe_few_down", vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp)
     fn("kvcm_moe_grouped_supported", i, i, i)
@@ -2084,6 +2087,42 @@ def moe_few_takes(h, F, H, top, E, gated=False):
     rows that chose it?  (A few rows, up to 64 (row, slot) pairs.)"""
     return (h.dtype == torch.bfloat16 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0
             and bool(lib().kvcm_moe_few_takes(h.shape[0], h.shape[1], int(F), int(H), int(top), int(E), int(bool(gated)))))
+
+
+def moe_few_beside_takes(h, F, H, top, E, w_shared_up):
+    """Are rows h beside a shared feed-forward of these gate and up rows [2 Fs, K] best left to ``moe_few_beside``?"""
+    return (h.dtype == w_shared_up.dtype == torch.bfloat16 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and w_shared_up.shape[0] % 2 == 0
+            and bool(lib().kvcm_moe_few_beside_takes(h.shape[0], h.shape[1], int(F), int(H), int(top), int(E), w_shared_up.shape[0] // 2)))
+
+
+def moe_few_beside(h, w_up, w_down, chosen, weight, act, w_shared_up, w_shared_down, act_shared, out, weigh_input=False, tokens=None, table=None):
+    """``moe_rows`` (gated, a few rows) and a shared feed-forward silu(gate) * up, down (w_shared_up [2 Fs, K]: gate rows, up rows; w_shared_down [H, Fs]; act_shared:
+    work memory [T, Fs]) in two launches: out = the shared one's + the experts' sum.  With ``tokens`` and ``table`` the first also routes
+    (``moe_table_route``), and leaves ``chosen`` and ``weight``."""
+    T, K = h.shape
+    E, F, _ = _expert_shapes(w_up, w_down, True)
+    H, top, Fs = w_down.shape[1], chosen.shape[1], w_shared_up.shape[0] // 2
+    _rows2d(h, "h")
+    _dev(h, w_up, w_down, chosen, weight, act, w_shared_up, w_shared_down, act_shared, out)
+    _need(all(t.dtype == torch.bfloat16 for t in (h, w_up, w_down, act, w_shared_up, w_shared_down, act_shared)), "moe_few_beside takes bfloat16")
+    _need(w_up.is_contiguous() and w_down.is_contiguous() and w_up.shape[2] == K and tuple(w_down.shape) == (E, H, F),
+          "moe_few_beside: expert weights must be [E, 2F, K] and [E, H, F]")
+    _need(w_shared_up.is_contiguous() and w_shared_down.is_contiguous() and tuple(w_shared_up.shape) == (2 * Fs, K) and tuple(w_shared_down.shape) == (H, Fs),
+          "moe_few_beside: the shared feed-forward's weights must be [2 Fs, K] and [H, Fs]")
+    _need(act.is_contiguous() and act.shape[0] >= T * top and act.shape[1] == F and act_shared.is_contiguous() and tuple(act_shared.shape) == (T, Fs),
+          "act must be [T * top, F], act_shared [T, Fs]")
+    _need(out.dtype == torch.float32 and out.is_contiguous() and tuple(out.shape) == (T, H), "out must be float32 [T, H]")
+    _need(chosen.dtype == torch.int32 and chosen.is_contiguous() and chosen.shape[0] >= T, "chosen must be int32 [T, top]")
+    _need(weight.dtype == torch.float32 and weight.is_contiguous() and tuple(weight.shape) == tuple(chosen.shape), "weight must match chosen")
+    if tokens is not None:
+        _i32(tokens, "tokens", T)
+        _need(table.dtype == torch.int32 and table.is_cuda and table.dim() == 2 and table.stride(1) == 1 and table.shape[1] >= top, "table must be int32 [vocabulary, top]")
+    _call("kvcm_moe_few_beside_up", _ptr(h), h.stride(0), _ptr(w_up), _ptr(chosen), _ptr(weight), _ptr(tokens), _ptr(table) if tokens is not None else 0,
+          table.shape[0] if tokens is not None else 0, table.stride(0) if tokens is not None else 0, _ptr(w_shared_up), _ptr(act_shared), Fs, _ptr(act), T, K, F, H,
+          top, E, 1 if weigh_input else 0, _stream())
+    _call("kvcm_moe_few_beside_down", _ptr(act), _ptr(w_down), _ptr(chosen), 0 if weigh_input else _ptr(weight), _ptr(act_shared), _ptr(w_shared_down), Fs, _ptr(out),
+          T, K, F, H, top, E, _stream())
+    return out
 
 
 def moe_grouped_supported(K, F, E, dtype):

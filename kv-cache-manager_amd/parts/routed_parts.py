@@ -6,7 +6,7 @@ import torch
 
 from ..registry import FEED_FORWARDS
 from .base import FeedForward, JoinableEnds, ParamSpec
-from .chain_norm_parts import linear32, pad_rows
+from .chain_norm_parts import GatedFeedForward, linear32, pad_rows
 
 
 def interleave_gate_up(gate, up):
@@ -168,21 +168,36 @@ class RoutedExperts(JoinableEnds, FeedForward):
                                     (experts, 1.0)], self.out_bias())
         return self._experts(step, h)
 
+    def _beside(self, h, F, H, top, E):
+        """Does the shared feed-forward run in the experts' launches (ops.moe_few_beside)?"""
+        sh = self.shared
+        return (self.gated and isinstance(sh, GatedFeedForward) and not self.by_ends and not sh.params.get("bias") and not sh.params.get("joined")
+                and sh.params.get("activation", "silu") == "silu" and torch.is_tensor(h) and h.dtype == torch.bfloat16
+                and self.ctx.ops.moe_few_beside_takes(h, F, H, top, E, sh.w["w_gate_up"]))
+
     def _experts(self, step, h, logits=None):
         """The experts' weighted sum, 32-bit [T, H]; ``logits``: the router's, where somebody else made them."""
         ops, p, w = self.ctx.ops, self.params, self.w
         E, top, F, T = p["experts"], p["top"], self.F, step.rows
         chosen = step.ws("routed_chosen", (T, top), torch.int32)
         weight = step.ws("routed_weight", (T, top), torch.float32)
+        H = self.ctx.hidden_size
+        beside = self._beside(h, F, H, top, E)
         if self.routing == "table":
-            ops.moe_table_route(step.tokens, w["table"], top, chosen, weight, rows=T)
+            if not beside:
+                ops.moe_table_route(step.tokens, w["table"], top, chosen, weight, rows=T)
         else:
             if logits is None:
                 logits = linear32(self.ctx, step, h, w["w_router"], "routed_logits", keep_partial=True)      # the route adds the slices
             ops.moe_route(logits, E, top, chosen, weight, rows=T, over_chosen=self.routing == "softmax_chosen", sigmoid=self.routing == "sigmoid",
                           factor=p.get("route_factor", 1.0))
+        if beside:      # a few rows: the shared feed-forward (and a table's route) in the experts' two launches
+            sh = self.shared
+            by_table = dict(tokens=step.tokens, table=w["table"]) if self.routing == "table" else {}
+            return ops.moe_few_beside(h, w["w_up"], w["w_down"], chosen, weight, step.ws("routed_act", (T, top * F)).view(T * top, F), sh.w["w_gate_up"],
+                                      sh.w["w_down"], step.ws("gated_act", (T, sh.params["intermediate_size"])), step.ws("routed_out", (T, H), torch.float32),
+                                      weigh_input=p.get("weigh") == "input", **by_table)
         add = self.shared.forward(step, h) if self.shared is not None and not self.by_ends else None      # 32-bit [T, H]: the experts' sum starts from it
-        H = self.ctx.hidden_size
         how = dict(gated=self.gated, add=add, weigh_input=p.get("weigh") == "input", **({} if self.gated else {"activation": self.activation}))
         act = step.ws("routed_act", (T, top * F)).view(T * top, F)
         out = step.ws("routed_out", (T, H), torch.float32)
