@@ -10,6 +10,8 @@
 // nothing else: one workgroup per row runs all of them, so a layer boundary costs one launch instead
 // of up to four, and the branches' outputs are read once.  Sums of squares are added in a tree whose
 // shape depends on the row length only; a row's result does not depend on the other rows.
+#include <type_traits>
+
 #include "common.h"
 #include "kvcm_hip.h"
 
@@ -91,51 +93,105 @@ __global__ void __launch_bounds__(kChainThreads)
 // The same chain for rows whose length is a multiple of 4 and at most 1024 * G (G groups of four values a thread):
 // the branches' and the stream's values of a row are read once, 16 bytes a load, and stay in registers through all
 // stages, so the row costs one trip to memory instead of one per stage.  A branch that is still the slices of a split
-// product is added up as it is read, slice after slice.  Which of the two kernels runs depends on the row length only,
-// never on the batch.
-template <class TO, int G>
+// product (SLICES) is added up slice after slice.  Which of the two kernels runs depends on the row length only,
+// never on the batch.  Of few rows the launch is its waits: everything it reads, the weights of all stages included, is asked for before the first
+// wait (up to rows of 4,096, which leave the registers for it; a trip of slices at a time), and a stage is one barrier.  us, one
+// branch / one of 4 slices / two / two of 4, before (weights read stage by stage, slices of a remainder one by one) -> now: width 2,048, 8 rows 4.4 / 5.1 / 4.9 / 6.2 ->
+// 3.5 / 3.9 / 4.0 / 4.8, 2,048 rows 12.4 / 24.1 / 16.7 / 36.3 -> 9.8 / 20.1 / 14.1 / 33.6; 4,096, 8 rows 5.8 / 7.3 / 6.6 / 9.5 -> 4.0 / 4.3 / 4.6 / 5.5; 8,192, 8 rows 9.0 /
+// 11.9 / 10.1 / 16.1 -> 4.9 / 5.8 / 6.0 / 8.0.
+typedef float chain_four __attribute__((ext_vector_type(4), aligned(4)));      // (weights may lie at any float)
+
+// The sums of one value (b: of two) over the workgroup, as block_sum has them; `scratch` is this stage's own.
+template <bool TWO>
+__device__ __forceinline__ void chain_sums(float& a, float& b, float (*scratch)[kChainThreads / kWave]) {
+  a = wave_sum(a);
+  if constexpr (TWO) b = wave_sum(b);
+  if (threadIdx.x % kWave == 0) {
+    scratch[0][threadIdx.x / kWave] = a;
+    if constexpr (TWO) scratch[1][threadIdx.x / kWave] = b;
+  }
+  __syncthreads();
+  a = scratch[0][0];
+  if constexpr (TWO) b = scratch[1][0];
+#pragma unroll
+  for (int w = 1; w < kChainThreads / kWave; ++w) {
+    a += scratch[0][w];
+    if constexpr (TWO) b += scratch[1][w];
+  }
+}
+
+template <class TO, int G, bool PAIR, bool SLICES>
 __global__ void __launch_bounds__(kChainThreads)
     rmsnorm_chain_rows_kernel(float* __restrict__ x, const float* __restrict__ a, int a_splits, const float* __restrict__ b,
                               int b_splits, size_t split_stride,
                               const float* __restrict__ wa, const float* __restrict__ wb, float combine,
                               const float* __restrict__ w_post, const int* __restrict__ rows,
                               const float* __restrict__ w_pre, TO* __restrict__ out, int H, float eps, int write_back) {
-  __shared__ float scratch[kChainThreads / kWave + 1];
+  __shared__ float scratch[4][kChainThreads / kWave];
+  constexpr int TRIP = !SLICES ? 1 : G <= 2 ? 8 : G <= 4 ? 4 : 2;
+  constexpr bool EARLY = G <= 4;
   const int r = blockIdx.x;
   const int src = rows ? rows[r] : r;
   float* xr = x + size_t(src) * H;
+  const float* ar = a ? a + size_t(src) * H : xr;      // (what is not there is read from the row itself, and not used)
+  const float* br = PAIR ? b + size_t(src) * H : nullptr;
   const float inv_h = 1.0f / float(H);
-  float xv[G][4], av[G][4], bv[G][4];
+  chain_four xv[G], av[G], bv[G], ta[TRIP][G], tb[PAIR ? TRIP : 1][G], va[G], vb[G], vpost[G], vpre[G];
   bool in[G];
+  int at[G];
+  // slices s0 .. s0 + TRIP - 1 of a branch (past its last: that one again, not added)
+  const auto ask = [&](const float* p, int splits, int s0, chain_four (*t)[G]) {
+#pragma unroll
+    for (int j = 0; j < TRIP; ++j)
+#pragma unroll
+      for (int g = 0; g < G; ++g) t[j][g] = *reinterpret_cast<const chain_four*>(p + size_t(s0 + j < splits ? s0 + j : splits - 1) * split_stride + at[g]);
+  };
+  const auto add_up = [&](const float* p, int splits, chain_four (*t)[G], chain_four* v) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) v[g] = t[0][g];
+    if constexpr (SLICES) {
+      for (int s0 = 0;;) {
+#pragma unroll
+        for (int j = 0; j < TRIP; ++j)
+          if (s0 + j > 0 && s0 + j < splits) {      // (the same for all lanes)
+#pragma unroll
+            for (int g = 0; g < G; ++g) v[g] += t[j][g];
+          }
+        s0 += TRIP;
+        if (s0 >= splits) break;
+        ask(p, splits, s0, t);
+      }
+    }
+  };
+  const auto weights = [&](const float* w, chain_four* v) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) v[g] = *reinterpret_cast<const chain_four*>(w + at[g]);
+  };
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     const int i = (g * kChainThreads + threadIdx.x) * 4;
     in[g] = i < H;
-    const int ic = in[g] ? i : 0;
-    const float4 vx = *reinterpret_cast<const float4*>(xr + ic);
-    xv[g][0] = vx.x; xv[g][1] = vx.y; xv[g][2] = vx.z; xv[g][3] = vx.w;
-    if (a) {
-      const float* p = a + size_t(src) * H + ic;
-      float4 va = *reinterpret_cast<const float4*>(p);
-#pragma unroll 4
-      for (int sl = 1; sl < a_splits; ++sl) {
-        const float4 t = *reinterpret_cast<const float4*>(p + size_t(sl) * split_stride);
-        va.x += t.x; va.y += t.y; va.z += t.z; va.w += t.w;
-      }
-      av[g][0] = va.x; av[g][1] = va.y; av[g][2] = va.z; av[g][3] = va.w;
-    }
-    if (b) {
-      const float* p = b + size_t(src) * H + ic;
-      float4 vb = *reinterpret_cast<const float4*>(p);
-#pragma unroll 4
-      for (int sl = 1; sl < b_splits; ++sl) {
-        const float4 t = *reinterpret_cast<const float4*>(p + size_t(sl) * split_stride);
-        vb.x += t.x; vb.y += t.y; vb.z += t.z; vb.w += t.w;
-      }
-      bv[g][0] = vb.x; bv[g][1] = vb.y; bv[g][2] = vb.z; bv[g][3] = vb.w;
-    }
+    at[g] = in[g] ? i : 0;
+    xv[g] = *reinterpret_cast<const chain_four*>(xr + at[g]);
   }
-  if (b) {
+  ask(ar, a ? a_splits : 1, 0, ta);
+  if constexpr (PAIR) ask(br, b_splits, 0, tb);
+  if constexpr (EARLY) {
+    if constexpr (PAIR) {
+      weights(wa, va);
+      weights(wb, vb);
+    }
+    weights(a ? w_post : xr, vpost);
+    weights(w_pre ? w_pre : xr, vpre);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  add_up(ar, a ? a_splits : 1, ta, av);
+  if constexpr (PAIR) {
+    add_up(br, b_splits, tb, bv);
+    if constexpr (!EARLY) {
+      weights(wa, va);
+      weights(wb, vb);
+    }
     float sa = 0.f, sb = 0.f;
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -145,52 +201,50 @@ __global__ void __launch_bounds__(kChainThreads)
           sa = fmaf(av[g][e], av[g][e], sa);
           sb = fmaf(bv[g][e], bv[g][e], sb);
         }
-    sa = block_sum<kChainThreads>(sa, scratch);
-    sb = block_sum<kChainThreads>(sb, scratch);
+    chain_sums<true>(sa, sb, scratch);
     const float inv_a = 1.0f / sqrtf(sa * inv_h + eps), inv_b = 1.0f / sqrtf(sb * inv_h + eps);
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int i = in[g] ? (g * kChainThreads + threadIdx.x) * 4 : 0;
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) av[g][e] = combine * (av[g][e] * inv_a * wa[i + e] + bv[g][e] * inv_b * wb[i + e]);
-    }
+      for (int e = 0; e < 4; ++e) av[g][e] = combine * __fmaf_rn(__fmul_rn(av[g][e], inv_a), va[g][e], __fmul_rn(__fmul_rn(bv[g][e], inv_b), vb[g][e]));
   }
+  float unused = 0.f;
   if (a) {
+    if constexpr (!EARLY) weights(w_post, vpost);
     float sm = 0.f;
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (in[g]) sm = fmaf(av[g][e], av[g][e], sm);
-    sm = block_sum<kChainThreads>(sm, scratch);
+    chain_sums<false>(sm, unused, scratch + 2);
     const float inv_m = 1.0f / sqrtf(sm * inv_h + eps);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      const int i = in[g] ? (g * kChainThreads + threadIdx.x) * 4 : 0;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) xv[g][e] += av[g][e] * inv_m * w_post[i + e];
-      if (in[g] && write_back) *reinterpret_cast<float4*>(xr + i) = float4{xv[g][0], xv[g][1], xv[g][2], xv[g][3]};
+      for (int e = 0; e < 4; ++e) xv[g][e] = __fmaf_rn(__fmul_rn(av[g][e], inv_m), vpost[g][e], xv[g][e]);
+      if (in[g] && write_back) *reinterpret_cast<float4*>(xr + at[g]) = float4{xv[g][0], xv[g][1], xv[g][2], xv[g][3]};
     }
   }
   if (!out) return;
   float inv_x = 1.f;
   if (w_pre) {
+    if constexpr (!EARLY) weights(w_pre, vpre);
     float sx = 0.f;
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (in[g]) sx = fmaf(xv[g][e], xv[g][e], sx);
-    sx = block_sum<kChainThreads>(sx, scratch);
+    chain_sums<false>(sx, unused, scratch + 3);
     inv_x = 1.0f / sqrtf(sx * inv_h + eps);
   }
   TO* o = out + size_t(r) * H;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     if (!in[g]) continue;
-    const int i = (g * kChainThreads + threadIdx.x) * 4;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) store_f(o + i + e, w_pre ? xv[g][e] * inv_x * w_pre[i + e] : xv[g][e]);
+    for (int e = 0; e < 4; ++e) store_f(o + at[g] + e, w_pre ? xv[g][e] * inv_x * vpre[g][e] : xv[g][e]);
   }
 }
 
@@ -243,14 +297,22 @@ int kvcm_rmsnorm_chain(float* x, const float* a, int a_splits, const float* b, i
   const bool f32 = !out || out_dtype == kF32;
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (H % 4 == 0 && H <= 8192 && aligned(x) && aligned(a) && aligned(b)) {      // slices lie split_stride = T * H floats apart
-#define KVCM_CHAIN_ROWS(TO, G)                                                                                     \
-  rmsnorm_chain_rows_kernel<TO, G><<<R, kChainThreads, 0, s>>>(x, a, a_splits, b, b_splits,                         \
-                                                               static_cast<size_t>(split_stride), wa, wb, combine, \
-                                                               w_post, rows, w_pre, static_cast<TO*>(out), H, eps, wb_flag)
-    if (H <= 2048) { if (f32) KVCM_CHAIN_ROWS(float, 2); else KVCM_CHAIN_ROWS(bf16_t, 2); }
-    else if (H <= 4096) { if (f32) KVCM_CHAIN_ROWS(float, 4); else KVCM_CHAIN_ROWS(bf16_t, 4); }
-    else { if (f32) KVCM_CHAIN_ROWS(float, 8); else KVCM_CHAIN_ROWS(bf16_t, 8); }
-#undef KVCM_CHAIN_ROWS
+    auto launch = [&](auto g, auto to) {
+      using TO = decltype(to);
+      constexpr int G = decltype(g)::value;
+      const bool slices = a_splits > 1 || (b && b_splits > 1);
+      auto* kernel = b ? (slices ? rmsnorm_chain_rows_kernel<TO, G, true, true> : rmsnorm_chain_rows_kernel<TO, G, true, false>)
+                       : (slices ? rmsnorm_chain_rows_kernel<TO, G, false, true> : rmsnorm_chain_rows_kernel<TO, G, false, false>);
+      kernel<<<R, kChainThreads, 0, s>>>(x, a, a_splits, b, b_splits, static_cast<size_t>(split_stride), wa, wb, combine, w_post, rows, w_pre,
+                                         static_cast<TO*>(out), H, eps, wb_flag);
+    };
+    auto typed = [&](auto to) {
+      if (H <= 2048) launch(std::integral_constant<int, 2>{}, to);
+      else if (H <= 4096) launch(std::integral_constant<int, 4>{}, to);
+      else launch(std::integral_constant<int, 8>{}, to);
+    };
+    if (f32) typed(float{});
+    else typed(bf16_t{});
     return launch_status("rmsnorm_chain");
   }
   if (f32)

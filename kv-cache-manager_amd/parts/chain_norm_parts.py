@@ -31,7 +31,7 @@ def linear32(ctx, step, x, w, name, keep_partial=False):
     run unsplit (gemm_rows8.hip), those of more rows split along K with a second launch that adds the slices up where that is faster
     than one slice.  ``keep_partial``: the product may come
     back as ops.PartialSums for a consumer that adds the slices itself.  The chained norm does: rows up to 8,192 wide
-    stay in registers through all its stages, and the slices are added as they are loaded (5 us a launch at width 2048;
+    stay in registers through all its stages, and the slices are added as they are loaded (4 us a launch at width 2048;
     the form that reads a row once per stage took 27 us with slices, more than the launch it saved).  Mixers' output
     projections use it; a feed-forward's does not where another part (a routed feed-forward's sum) starts from it."""
     return _linear(ctx, step, x, w, name, keep_partial=keep_partial, dtype=torch.float32)
