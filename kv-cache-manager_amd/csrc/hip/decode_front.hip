@@ -10,13 +10,19 @@
 // work, and hand results on through memory, past the caches, in words that are their own flags: a buffer is full of kEmpty before
 // the launch, a word that is something else is there.  No counter, no fence, no order between words is needed, and a hand-over
 // costs 0.8 to 1 us.  Measured (us a layer: three launches / this one, eight layers of distinct weights in a graph, contexts of 600 and
-// 1,900 tokens): TinyLlama sizes 1 row 18.8 / 11.3 and 19.5 / 11.8, 8 rows 20.4 / 13.4 and 22.0 / 16.6; width 4096, 8 KV heads of 128, 1
-// row 34.1 / 28.3 and 34.3 / 28.6, with 32 KV heads 45.0 / 40.1 and 46.6 / 43.0; nothing measured was slower by more than 1 % (32 KV heads of
-// 64, 8 rows: 1,024 workgroups of attention, 41.8 / 42.4).
+// 1,900 tokens): TinyLlama sizes 1 row 18.7 / 11.7 and 26.4 / 12.0, 8 rows 20.1 / 13.7 and 30.1 / 17.1; width 4096, 8 KV heads of 128, 1
+// row 37.7 / 28.9 and 53.1 / 29.0, 8 rows 46.2 / 33.1 and 62.8 / 41.6; 32 KV heads of 128, 1 row of 600 49.2 / 41.0.
 //
-// Nobody waits for a workgroup of a higher number: [QKV tiles | attention, a row's and KV head's parts in ascending order | output tiles].
-// Workgroups are started in the order of their numbers on each XCD, so the lowest unfinished one is always running or next,
-// whatever else runs on the chip and however few CUs there are; every wait is bounded all the same (kPolls, some 0.2 s; results are then NaN).
+// Nobody waits for a workgroup of a higher number: [QKV tiles | attention, a row's and KV head's parts in ascending order | output tiles],
+// and workgroups are started in the order of their numbers on each XCD, so a launch that has the chip to itself always gets on.  Two at a time (engines with a
+// stream each, or two processes) may not: a waiting workgroup keeps its place, and what waits in one launch can fill an XCD on which the other
+// still has products to start, while the other does the same elsewhere.  So every wait has an end, after which the workgroup makes what it
+// waits for itself: an attention workgroup the QKV tiles of its heads, an output tile all QKV tiles and all of the attention, in order, and
+// then its own part again.  It is the same code on the same operands, which the launch leaves as they are, so whoever else makes a word
+// too, and however late, stores the same bits; nothing depends on who runs beside whom.  This costs 0.3 to 0.4 us a layer (in the code's
+// shape, no wait more).  Several streams of such layers at once, us a layer of each, three launches / this one: TinyLlama sizes, 8 rows of 600, two
+// streams 26.3 / 20.0, three 29.6 / 25.5, four 33.6 / 33.4 (up to 44); width 4096, 8 KV heads, 8 rows of 1,900 84.4 / 67.3, 107.5 / 128 (up to 375 where
+// output tiles gave up), 137.5 / 133.
 //
 // Attention: a wave takes windows of 64 tokens (both products on the matrix cores, transposed, as in attention_decode_fused.hip), one
 // each: `parts` workgroups of eight waves share a row's KV head, window 8 w + part belonging to wave w.  The last part adds the
@@ -58,8 +64,12 @@ constexpr int kUnit = 64, kCols = 8, kGroups = 2, kTrip = 4, kSlots = 2 * kWaves
 constexpr int kWindow = 64;                 // tokens of a wave
 constexpr int kMaxParts = 4;
 constexpr float kNone = -1.0e30f;           // "no score": finite, so that differences stay finite
+constexpr float kLate = 3.40282347e38f;     // a wave's largest score where q, the key or the value did not come
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;    // no 32-bit float rounded to bfloat16 has these bits; other words that would have them are stored as another NaN
-constexpr int kPolls = 1 << 18;
+// Looks at what is not there before a workgroup makes it itself.  A look takes some 0.8 us: an attention workgroup waits 50 us (its 12 to 40
+// tiles then take it about 100), an output tile, which would have all of the launch to make, a millisecond at each of its waits.
+constexpr int kNearPolls = 64, kFarPolls = 1024;
+constexpr int kOwnPolls = 1 << 18;          // ... at what the workgroup has stored itself: there at the first or second look
 
 struct FrontArgs {
   const uint16_t *X, *Wqkv, *Wo;
@@ -68,7 +78,7 @@ struct FrontArgs {
   const float2* cos_sin; const int *slots, *tables, *row_seq, *ctx_lens;
   uint16_t *kcache, *vcache;
   uint32_t *now, *next;      // handed over in this launch: q, k, v [M][width] as floats, attention [M][nh hd / 2] as pairs, parts; emptied for the next
-  int ldx, ldqkv, ldo, tiles_in, M, H, g_f32, table_stride, nh, nkv, B, seqs, parts, n_qkv, n_att;
+  int ldx, ldqkv, ldo, tiles_in, M, H, g_f32, table_stride, nh, nkv, B, seqs, parts, n_qkv, n_att, near_polls, far_polls;
   uint32_t per_page;
   float inv_width, eps, scale;
 };
@@ -102,10 +112,17 @@ struct Slice {
 };
 struct WTrip { Frag w[kTrip][kGroups][2]; };
 struct XTrip { Frag x[kTrip][2]; };
+// What fragments hold before they are loaded is nothing (else the registers of one part of the work are kept for the next: 210 in place of 163)
+template <class T>
+__device__ __forceinline__ void nothing(T& t) {
+  Frag* f = reinterpret_cast<Frag*>(&t);
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / sizeof(Frag); ++i) asm volatile("" : "=v"(f[i].u.x), "=v"(f[i].u.y), "=v"(f[i].u.z), "=v"(f[i].u.w));
+}
 
 template <int HD, int GROUP>
 union Lds {
-  struct { f32x4 red[kWaves][kGroups][kWave]; float rstd[8]; } p;
+  struct { f32x4 red[kWaves][kGroups][kWave]; float rstd[8]; int late[kWaves]; } p;
   struct {
     uint16_t q[GROUP][HD], k_new[HD], v_new[HD];
     float red[kWaves][GROUP][HD + 4];
@@ -113,10 +130,11 @@ union Lds {
   } a;
 };
 
-// A tile of 16 columns of the QKV product (first) or of the output product.
+// A tile of 16 columns of the QKV product (first) or of the output product.  True: what it waits for did not come, and it has
+// stored nothing.  `made`: the workgroup has made all of that itself.
 template <int HD, int GROUP>
-__device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, bool first, int tile) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+__device__ __forceinline__ bool products(const FrontArgs& a, Lds<HD, GROUP>& L, int tid, bool first, int tile, bool made) {
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const int M = a.M, H = a.H, qw = a.nh * HD, width = qw + 2 * a.nkv * HD;
   const int n0 = tile * (kCols * kGroups);
   const int r = lane % 16, kq = lane / 16, half = r / 8, c = r % 8;
@@ -159,7 +177,7 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
     }
   };
   // the first 128 threads' element of the result
-  const int eg = threadIdx.x / kWave, em = lane / 8, en = lane % 8;
+  const int eg = tid / kWave, em = lane / 8, en = lane % 8;
   const int col = n0 + (eg < kGroups ? eg : 0) * kCols + en;
   const bool live = eg < kGroups && em < M;
   float resid_in = 0.f, g_in = 0.f;
@@ -187,6 +205,8 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
     }
     WTrip wa;
     XTrip xa;
+    nothing(wa);
+    nothing(xa);
     fetch_w(0, wa);
     fetch_x(0, xa);
     if (live) leave(a.next + size_t(em) * width + col, kEmpty);
@@ -208,18 +228,21 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
       resid_in = a.resid[size_t(em < M ? em : 0) * H + col];
       g_in = a.g_f32 ? static_cast<const float*>(a.g)[col] : load_f(static_cast<const bf16_t*>(a.g) + col);
     }
+    int polls = made ? kOwnPolls : a.far_polls;
+    bool late = false;
     if (wave == 0) {      // QKV's weights first
-      const uint32_t* word = a.now + size_t(tile) * a.n_qkv / (gridDim.x - a.n_qkv - a.n_att) * (kCols * kGroups);
-      for (int poll = 0; poll < kPolls && take(word) == kEmpty; ++poll) __builtin_amdgcn_s_sleep(4);
+      const uint32_t* word = a.now + size_t(tile) * a.n_qkv / (H / (kCols * kGroups)) * (kCols * kGroups);
+      for (int poll = 0; poll < polls && take(word) == kEmpty; ++poll) __builtin_amdgcn_s_sleep(4);
     }
     __syncthreads();
     WTrip wa;
+    nothing(wa);
     fetch_w(0, wa);
     const uint32_t* xrow = a.now + size_t(M) * width + (size_t(c < M ? c : 0) * qw + kq * 16) / 2;
     const bool cached = M > 2;
     if (cached) {
       if (wave == 0) {
-        for (int poll = 0; poll < kPolls; ++poll) {
+        for (int poll = 0; poll < polls; ++poll) {
           bool none = false;
           for (int i = lane; i < M * a.nkv; i += kWave) none |= take(a.now + size_t(M) * width + size_t(i) * (GROUP * HD / 2)) == kEmpty;
           if (!__any(none)) break;
@@ -246,7 +269,7 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
         }
         if (!__any(none)) return;
       }
-      for (int poll = 0; poll < kPolls; ++poll) {
+      auto look = [&] {
         none = false;
 #pragma unroll
         for (int d = 0; d < kTrip; ++d) {
@@ -261,11 +284,17 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
 #pragma unroll
           for (int e = 0; e < 4; ++e) none |= empty_half(t.x[d][e / 2].d[e % 2]);
         }
-        if (!__any(none)) break;
+        return __any(none);
+      };
+      bool empty = look();
+      for (int poll = 0; empty && poll < polls; ++poll) {
         __builtin_amdgcn_s_sleep(1);
+        empty = look();
       }
+      if (empty) late = true, polls = 0;
     };
     XTrip xa;
+    nothing(xa);
     await(0, xa);
     multiply(0, wa, xa);
     for (int j0 = kTrip; j0 < s.most; j0 += kTrip) {
@@ -273,17 +302,30 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
       await(j0, xa);
       multiply(j0, wa, xa);
     }
+    if (lane == 0) L.p.late[wave] = late;
+    if (late) {      // (all of the results are then NaN, in both waves that add them up: they look at the flags only where they meet one)
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) acc[g] = f32x4{NAN, NAN, NAN, NAN};
+    }
   }
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) L.p.red[wave][g][lane] = acc[g];
   __syncthreads();
-  if (eg >= kGroups) return;
   float v = 0.f;
+  if (eg < kGroups) {
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    v += L.p.red[w][eg][(em / 4) * 16 + en][em % 4];
-    v += L.p.red[w][eg][(2 + em / 4) * 16 + en + 8][em % 4];
+    for (int w = 0; w < kWaves; ++w) {
+      v += L.p.red[w][eg][(em / 4) * 16 + en][em % 4];
+      v += L.p.red[w][eg][(2 + em / 4) * 16 + en + 8][em % 4];
+    }
   }
+  if (!first && !made && (eg >= kGroups || __any(v != v))) {
+    int late = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) late |= L.p.late[w];
+    if (__builtin_amdgcn_readfirstlane(late)) return true;
+  }
+  if (eg >= kGroups) return false;
   if (first) {
     if (a.ss_in) v *= L.p.rstd[em];
     if (live) leave(a.now + size_t(em) * width + col, __float_as_uint(round_to<bf16_t>(v)));
@@ -297,14 +339,16 @@ __device__ __forceinline__ void products(const FrontArgs& a, Lds<HD, GROUP>& L, 
     const float sq = group_sum<8>(xn * xn);
     if (live && en == 0) a.ss_out[size_t(em) * (H / kCols) + tile * kGroups + eg] = sq;
   }
+  return false;
 }
 
-// Part `id` of (row, KV head, part): the row's query heads of that KV head over the part's windows.
+// Part `id` of (row, KV head, part): the row's query heads of that KV head over the part's windows.  True: q, the key or the value did not
+// come, and no word is stored.  `made`: the workgroup has made them itself.
 template <int HD, int GROUP>
-__device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, int id) {
+__device__ __forceinline__ bool attend(const FrontArgs& a, Lds<HD, GROUP>& L, int tid, int id, bool made) {
   constexpr int KSTEPS = HD / 32, DT = HD / 16, HALF = HD / 2;
   constexpr int kPartWords = GROUP * (HD + 2);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const int part = id % a.parts, kvh = id / a.parts % a.nkv, row = id / a.parts / a.nkv;
   const bool merges = part == a.parts - 1;
   const int qw = a.nh * HD, width = qw + 2 * a.nkv * HD, B = a.B;
@@ -314,28 +358,31 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
   const int entry = min(page_of(t_first + lane), a.table_stride - 1);
   int page = a.tables[size_t(row < a.seqs ? row : 0) * a.table_stride + entry];
   const int ctx_all = a.ctx_lens[row], slot = a.slots[row], seq = a.row_seq[row];
-  const int ih = threadIdx.x / HALF, ij = threadIdx.x % HALF;
+  const int ih = tid / HALF, ij = tid % HALF;
   static_assert((GROUP + 2) * HALF <= 2 * kThreads, "two pairs a thread");
   float2 rot = float2{1.0f, 0.0f};
   if (a.cos_sin) rot = a.cos_sin[size_t(row) * HALF + ij];
   const size_t a_at = size_t(a.M) * width, p_at = a_at + size_t(a.M) * qw / 2 + size_t(row * a.nkv + kvh) * (a.parts - 1) * kPartWords;
   const size_t out = a_at + (size_t(row) * qw + size_t(kvh) * GROUP * HD) / 2;
   if (merges) {
-    for (int i = threadIdx.x; i < GROUP * HALF; i += kThreads) leave(a.next + out + i, kEmpty);
+    for (int i = tid; i < GROUP * HALF; i += kThreads) leave(a.next + out + i, kEmpty);
   } else {
-    for (int i = threadIdx.x; i < kPartWords; i += kThreads) leave(a.next + p_at + size_t(part) * kPartWords + i, kEmpty);
+    for (int i = tid; i < kPartWords; i += kThreads) leave(a.next + p_at + size_t(part) * kPartWords + i, kEmpty);
   }
   if (ctx_all <= 0) {
     if (merges)
-      for (int i = threadIdx.x; i < GROUP * HALF; i += kThreads) leave(a.now + out + i, 0u);
-    return;
+      for (int i = tid; i < GROUP * HALF; i += kThreads) leave(a.now + out + i, 0u);
+    return false;
   }
   const int ctx = slot >= 0 ? ctx_all - 1 : ctx_all;      // tokens whose keys are in their pages
-  if (!merges && part * kWindow >= ctx) return;
+  if (!merges && part * kWindow >= ctx) return false;
   // (a row's sequence is nearly always the row itself: its page numbers are asked for before that is known)
   if (seq != row) page = a.tables[size_t(seq) * a.table_stride + entry];
+  asm volatile("" : "+v"(page));      // here, once (a wave without tokens would wait for it, and all behind it, where its register is next used)
   const int n16 = lane % 16, kq = lane / 16;
   Frag kf[2][2][KSTEPS], vf[2][DT];
+  nothing(kf);
+  nothing(vf);
   const bool works = t_first < ctx;
   if (works) {
     const int t0 = t_first + lane, over = t0 - (ctx - 1);
@@ -358,19 +405,25 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
     }
   }
   const uint32_t* qrow = a.now + size_t(row) * width;
+  const int polls = made ? kOwnPolls : a.near_polls;
+  bool late = false;
   auto await_pair = [&](int col, float& va, float& vb) {
-    uint32_t wa = kEmpty, wb = kEmpty;
-    for (int poll = 0; poll < kPolls; ++poll) {
+    // (the first look apart: in front of a loop the compiler waits for all that is on its way, here the keys and values)
+    uint32_t wa = take(qrow + col), wb = take(qrow + col + HALF);
+    for (int poll = 0; __any(wa == kEmpty || wb == kEmpty); ++poll) {
+      if (poll >= polls) {
+        late = true;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
       wa = take(qrow + col);
       wb = take(qrow + col + HALF);
-      if (!__any(wa == kEmpty || wb == kEmpty)) break;
-      __builtin_amdgcn_s_sleep(1);
     }
     va = __uint_as_float(wa);
     vb = __uint_as_float(wb);
   };
   // q: a pair (j, j + HD / 2) of a head a thread
-  if (threadIdx.x < GROUP * HALF) {
+  if (tid < GROUP * HALF) {
     float va, vb;
     await_pair((kvh * GROUP + ih) * HD + ij, va, vb);
     if (a.cos_sin) rotate_pair(va, vb, rot.x, rot.y);
@@ -378,24 +431,23 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
     L.a.q[ih][ij + HALF] = float_to_bf16_bits(vb);
   }
   // the last threads (other waves where there are enough): the new key and value
-  if (merges && slot >= 0 && threadIdx.x >= kThreads - 2 * HALF) {
-    const bool is_v = threadIdx.x >= kThreads - HALF;
+  if (merges && slot >= 0 && tid >= kThreads - 2 * HALF) {
+    const bool is_v = tid >= kThreads - HALF;
     float va, vb;
     await_pair((a.nh + (is_v ? a.nkv : 0) + kvh) * HD + ij, va, vb);
     if (!is_v && a.cos_sin) rotate_pair(va, vb, rot.x, rot.y);
     const uint16_t ab = float_to_bf16_bits(va), bb = float_to_bf16_bits(vb);
     const size_t pg = slot / B;
     const int off = slot % B;
-    if (!is_v) {
-      L.a.k_new[ij] = ab;
-      L.a.k_new[ij + HALF] = bb;
-      uint16_t* kr = a.kcache + ((pg * a.nkv + kvh) * B + off) * HD;
+    uint16_t* kr = a.kcache + ((pg * a.nkv + kvh) * B + off) * HD;
+    uint16_t* vr = a.vcache + (pg * a.nkv + kvh) * size_t(HD) * B + off;
+    uint16_t* fresh = is_v ? L.a.v_new : L.a.k_new;
+    fresh[ij] = ab;
+    fresh[ij + HALF] = bb;
+    if (!late && !is_v) {
       kr[ij] = ab;
       kr[ij + HALF] = bb;
-    } else {
-      L.a.v_new[ij] = ab;
-      L.a.v_new[ij + HALF] = bb;
-      uint16_t* vr = a.vcache + (pg * a.nkv + kvh) * size_t(HD) * B + off;
+    } else if (!late) {
       vr[size_t(ij) * B] = ab;
       vr[size_t(ij + HALF) * B] = bb;
     }
@@ -458,6 +510,7 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
     }
     l_run = rows_sum(l_run);
   }
+  if (__any(late)) m_run = kLate;
   if (kq == 0) { L.a.top[wave][n16] = m_run; L.a.sum[wave][n16] = l_run; }
   if (n16 < GROUP) {
 #pragma unroll
@@ -465,11 +518,17 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
   }
   __syncthreads();
   // a pair of dims of a head a thread: this workgroup's waves, the other parts, the newest token
-  const int g = threadIdx.x / HALF, d = 2 * (threadIdx.x % HALF);
-  if (g >= GROUP) return;
+  const int g = tid / HALF, d = 2 * (tid % HALF);
+  static_assert(kThreads / HALF <= 16, "every thread has a column of top");
   float m = L.a.top[0][g];
+  bool in_vain = m == kLate;
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) m = fmaxf(m, L.a.top[w][g]);
+  for (int w = 1; w < kWaves; ++w) {
+    in_vain |= L.a.top[w][g] == kLate;
+    m = fmaxf(m, L.a.top[w][g]);
+  }
+  if (__any(in_vain) && !made) return true;
+  if (g >= GROUP) return false;
   float n0 = 0.f, n1 = 0.f, den = 0.f;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) {
@@ -487,24 +546,30 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
       leave(dst + HD, filled(m));
       leave(dst + HD + 1, filled(den));
     }
-    return;
+    return false;
   }
   const int others = min(a.parts - 1, (ctx + kWindow - 1) / kWindow);
   if (others > 0) {
     uint64_t v[kMaxParts - 1], ml[kMaxParts - 1];
-    for (int poll = 0; poll < kPolls; ++poll) {
-      bool none = false;
+    const int looks = made ? kOwnPolls : a.far_polls;
+    auto look = [&] {
 #pragma unroll
       for (int p = 0; p < kMaxParts - 1; ++p) {
         const uint32_t* src = a.now + p_at + size_t(p < others ? p : 0) * kPartWords + g * (HD + 2);
         v[p] = take_two(src + d);
         ml[p] = take_two(src + HD);
       }
+      bool none = false;
 #pragma unroll
       for (int p = 0; p < kMaxParts - 1; ++p) none |= empty_half(v[p]) || empty_half(ml[p]);
-      if (!__any(none)) break;
+      return __any(none);
+    };
+    bool empty = look();
+    for (int poll = 0; empty && poll < looks; ++poll) {
       __builtin_amdgcn_s_sleep(1);
+      empty = look();
     }
+    if (empty) return false;      // (left to the output tiles: these words stay empty)
 #pragma unroll
     for (int p = 0; p < kMaxParts - 1; ++p)
       if (p < others) {
@@ -526,19 +591,57 @@ __device__ __forceinline__ void attend(const FrontArgs& a, Lds<HD, GROUP>& L, in
     den = den * ea + eb;
   }
   uint32_t word = pack2(n0 / den, n1 / den);
-  leave(a.now + out + threadIdx.x, word == kEmpty ? 0x7FFF7FFFu : word);
+  leave(a.now + out + tid, word == kEmpty ? 0x7FFF7FFFu : word);
+  return false;
+}
+
+// Tells the compiler that pointers lead to device memory (it knows so of a kernel's own arguments only).
+template <class... P>
+__device__ __forceinline__ void in_memory(P*&... p) {
+  ((p = (P*)(__attribute__((address_space(1))) P*)p), ...);
 }
 
 template <int HD, int GROUP>
-__global__ void __launch_bounds__(kThreads, 2) decode_front_kernel(const FrontArgs a) {
+__global__ void __launch_bounds__(kThreads, 2) decode_front_kernel(const FrontArgs) {
   __shared__ Lds<HD, GROUP> L;
-  // all arguments at once: asked for where they are used they are three trips one behind the other (0.2 to 0.4 us)
-  asm volatile("" ::"s"(a.X), "s"(a.Wqkv), "s"(a.Wo), "s"(a.ss_in), "s"(a.resid), "s"(a.g), "s"(a.xg), "s"(a.ss_out), "s"(a.cos_sin), "s"(a.slots));
-  asm volatile("" ::"s"(a.tables), "s"(a.row_seq), "s"(a.ctx_lens), "s"(a.kcache), "s"(a.vcache), "s"(a.now), "s"(a.next), "s"(a.ldx), "s"(a.ldqkv), "s"(a.ldo), "s"(a.tiles_in), "s"(a.M), "s"(a.H));
-  asm volatile("" ::"s"(a.table_stride), "s"(a.nh), "s"(a.nkv), "s"(a.B), "s"(a.seqs), "s"(a.parts), "s"(a.n_qkv), "s"(a.n_att), "s"(a.per_page), "s"(a.inv_width), "s"(a.eps), "s"(a.scale), "s"(a.g_f32));
-  const int id = blockIdx.x;
-  if (id >= a.n_qkv && id < a.n_qkv + a.n_att) attend<HD, GROUP>(a, L, id - a.n_qkv);
-  else products<HD, GROUP>(a, L, id < a.n_qkv, id < a.n_qkv ? id : id - a.n_qkv - a.n_att);
+  typedef __attribute__((address_space(4))) const FrontArgs KernelArgs;
+  const int own = blockIdx.x;
+  int id = own, next = -1;      // -1: nothing of what it waits for
+  for (;;) {
+    // The arguments and the thread's number anew for each part (nothing made of them is kept through the loop, which is for workgroups
+    // that waited in vain: 256 registers and spills otherwise).  All arguments at once: asked for where they are used they are three
+    // trips one behind the other (0.2 to 0.4 us)
+    auto* given = (KernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    unsigned thread = threadIdx.x;
+    asm volatile("" : "+s"(given), "+v"(thread));
+    const int tid = thread % kThreads;
+    FrontArgs a = *(const FrontArgs*)given;
+    in_memory(a.X, a.Wqkv, a.Wo, a.ss_in, a.resid, a.g, a.xg, a.ss_out, a.cos_sin, a.slots, a.tables, a.row_seq, a.ctx_lens, a.kcache, a.vcache, a.now, a.next);
+    asm volatile("" ::"s"(a.X), "s"(a.Wqkv), "s"(a.Wo), "s"(a.ss_in), "s"(a.resid), "s"(a.g), "s"(a.xg), "s"(a.ss_out), "s"(a.cos_sin), "s"(a.slots));
+    asm volatile("" ::"s"(a.tables), "s"(a.row_seq), "s"(a.ctx_lens), "s"(a.kcache), "s"(a.vcache), "s"(a.now), "s"(a.next), "s"(a.ldx), "s"(a.ldqkv), "s"(a.ldo), "s"(a.tiles_in), "s"(a.M), "s"(a.H));
+    asm volatile("" ::"s"(a.table_stride), "s"(a.nh), "s"(a.nkv), "s"(a.B), "s"(a.seqs), "s"(a.parts), "s"(a.n_qkv), "s"(a.n_att), "s"(a.per_page), "s"(a.inv_width), "s"(a.eps), "s"(a.scale), "s"(a.g_f32));
+    const int n_in = a.n_qkv + a.n_att;
+    bool late;
+    if (id >= a.n_qkv && id < n_in) late = attend<HD, GROUP>(a, L, tid, id - a.n_qkv, next >= 0);
+    else late = products<HD, GROUP>(a, L, tid, id < a.n_qkv, id < a.n_qkv ? id : id - n_in, next >= 0);
+    if (id == own) {
+      if (!__builtin_amdgcn_readfirstlane(late)) return;
+      next = 0;
+    }
+    __syncthreads();      // (the next part writes the LDS that this one reads)
+    // an attention workgroup: the tiles of its q heads, key and value; an output tile: all QKV tiles and the attention; then its own part again
+    const bool attends = own < n_in;
+    constexpr int kHeadTiles = HD / (kCols * kGroups);
+    if (next >= (attends ? (GROUP + 2) * kHeadTiles : n_in)) {
+      id = own;
+    } else if (!attends) {
+      id = next;
+    } else {
+      const int kvh = (own - a.n_qkv) / a.parts % a.nkv, h = next / kHeadTiles;
+      id = (h < GROUP ? kvh * GROUP + h : a.nh + (h - GROUP) * a.nkv + kvh) * kHeadTiles + next % kHeadTiles;
+    }
+    ++next;
+  }
 }
 
 }  // namespace
@@ -598,11 +701,12 @@ int kvcm_decode_front_empty(uint32_t* words, long long n, hipStream_t st) {
 // resid[M, H] += round(attention(X Wqkv^T) Wo^T), xg = round(g round(resid)), ss_out[M][H / 8] its sums of squares per 8 columns.
 // X: normed rows, or with ss_in [M][tiles_in] what a producer of the folded norm left (kvcm_gemm8).  cos_sin, slots, tables, row_seq,
 // ctx_lens as kvcm_attention_decode_fused takes them, tables of `seqs` sequences; no context exceeds 512 * parts tokens.  now: empty
-// (kvcm_decode_front_empty, or the launch before had it as next); both of `words` words.
-int kvcm_decode_front(const void* X, int ldx, const void* Wqkv, int ldqkv, const float* ss_in, int tiles_in, float eps, const void* Wo, int ldo,
+// (kvcm_decode_front_empty, or the launch before had it as next); both of `words` words.  kvcm_decode_front_waiting: polls: looks at what is not there before a workgroup
+// makes it itself (negative: as measured).
+int kvcm_decode_front_waiting(const void* X, int ldx, const void* Wqkv, int ldqkv, const float* ss_in, int tiles_in, float eps, const void* Wo, int ldo,
                       int M, int H, const float* cos_sin, const int* slots, void* kcache, void* vcache, const int* tables, int table_stride,
                       int seqs, const int* row_seq, const int* ctx_lens, int nh, int nkv, int hd, int B, float scale, float* resid, const void* g,
-                      int g_dtype, void* xg, float* ss_out, uint32_t* now, uint32_t* next, long long words, int parts, hipStream_t st) {
+                      int g_dtype, void* xg, float* ss_out, uint32_t* now, uint32_t* next, long long words, int parts, int polls, hipStream_t st) {
   KVCM_REQUIRE(kvcm_decode_front_supported(M, H, nh, nkv, hd, B), "decode_front: unsupported shape M=%d H=%d heads=%d kv_heads=%d head_dim=%d page=%d", M, H, nh,
                nkv, hd, B);
   KVCM_REQUIRE(parts >= 1 && parts <= kMaxParts, "decode_front: %d parts", parts);
@@ -626,12 +730,19 @@ int kvcm_decode_front(const void* X, int ldx, const void* Wqkv, int ldqkv, const
   a.kcache = static_cast<uint16_t*>(kcache); a.vcache = static_cast<uint16_t*>(vcache); a.table_stride = table_stride; a.seqs = seqs;
   a.nh = nh; a.nkv = nkv; a.B = B; a.scale = scale; a.per_page = static_cast<uint32_t>(((1ull << 32) + B - 1) / B);
   a.resid = resid; a.g = g; a.g_f32 = g_dtype == kF32; a.xg = static_cast<uint16_t*>(xg); a.ss_out = ss_out;
-  a.now = now; a.next = next; a.parts = parts;
+  a.now = now; a.next = next; a.parts = parts; a.near_polls = polls < 0 ? kNearPolls : polls; a.far_polls = polls < 0 ? kFarPolls : polls;
   a.n_qkv = width / (kCols * kGroups); a.n_att = M * nkv * parts;
   const int grid = a.n_qkv + a.n_att + H / (kCols * kGroups);
   const int rc = hd == 64 ? launch_front<64>(nh / nkv, grid, st, a) : launch_front<128>(nh / nkv, grid, st, a);
   KVCM_REQUIRE(rc == 0, "decode_front: no kernel for group size %d", nh / nkv);
   return launch_status("decode_front");
+}
+int kvcm_decode_front(const void* X, int ldx, const void* Wqkv, int ldqkv, const float* ss_in, int tiles_in, float eps, const void* Wo, int ldo,
+                      int M, int H, const float* cos_sin, const int* slots, void* kcache, void* vcache, const int* tables, int table_stride,
+                      int seqs, const int* row_seq, const int* ctx_lens, int nh, int nkv, int hd, int B, float scale, float* resid, const void* g,
+                      int g_dtype, void* xg, float* ss_out, uint32_t* now, uint32_t* next, long long words, int parts, hipStream_t st) {
+  return kvcm_decode_front_waiting(X, ldx, Wqkv, ldqkv, ss_in, tiles_in, eps, Wo, ldo, M, H, cos_sin, slots, kcache, vcache, tables, table_stride, seqs, row_seq,
+                                   ctx_lens, nh, nkv, hd, B, scale, resid, g, g_dtype, xg, ss_out, now, next, words, parts, -1, st);
 }
 
 }  // extern "C"

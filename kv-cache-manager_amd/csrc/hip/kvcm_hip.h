@@ -102,6 +102,11 @@ int kvcm_decode_front(const void* X, int ldx, const void* Wqkv, int ldqkv, const
                       int M, int H, const float* cos_sin, const int* slots, void* kcache, void* vcache, const int* tables, int table_stride,
                       int seqs, const int* row_seq, const int* ctx_lens, int nh, int nkv, int hd, int B, float scale, float* resid, const void* g,
                       int g_dtype, void* xg, float* ss_out, uint32_t* now, uint32_t* next, long long words, int parts, hipStream_t stream);
+// kvcm_decode_front with the looks a workgroup waits before it makes what it waits for (negative: as measured).
+int kvcm_decode_front_waiting(const void* X, int ldx, const void* Wqkv, int ldqkv, const float* ss_in, int tiles_in, float eps, const void* Wo, int ldo,
+                      int M, int H, const float* cos_sin, const int* slots, void* kcache, void* vcache, const int* tables, int table_stride,
+                      int seqs, const int* row_seq, const int* ctx_lens, int nh, int nkv, int hd, int B, float scale, float* resid, const void* g,
+                      int g_dtype, void* xg, float* ss_out, uint32_t* now, uint32_t* next, long long words, int parts, int polls, hipStream_t stream);
 // The vendor library's product (hipBLASLt), bfloat16 operands and result, 32-bit accumulation, for
 // the many-row products of prompt steps, where the reference calls cuBLAS (src/model/llama.cpp:45-52).
 // `workspace` is device memory the caller owns (at least kvcm_gemm_library_workspace_bytes()).

@@ -92,6 +92,7 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_gemm8_residual_norm),
     KVCM_ENTRY(kvcm_decode_front_empty),
     KVCM_ENTRY(kvcm_decode_front),
+    KVCM_ENTRY(kvcm_decode_front_waiting),
     KVCM_ENTRY(kvcm_attention_generic),
     KVCM_ENTRY(kvcm_attention_f32_decode),
     KVCM_ENTRY(kvcm_attention_decode),

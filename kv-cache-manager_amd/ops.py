@@ -57,8 +57,9 @@ def _declare(lib):
     lib.kvcm_decode_front_words.restype = C.c_longlong
     lib.kvcm_decode_front_words.argtypes = [i] * 5
     fn("kvcm_decode_front_empty", vp, C.c_longlong, vp)
-    fn("kvcm_decode_front", vp, i, vp, i, vp, i, f, vp, i, i, i, vp, vp, vp, vp, vp, i, i, vp, vp, i, i, i, i, f, vp, vp, i, vp, vp, vp, vp,
-       C.c_longlong, i, vp)
+    front = (vp, i, vp, i, vp, i, f, vp, i, i, i, vp, vp, vp, vp, vp, i, i, vp, vp, i, i, i, i, f, vp, vp, i, vp, vp, vp, vp, C.c_longlong, i)
+    fn("kvcm_decode_front", *front, vp)
+    fn("kvcm_decode_front_waiting", *front, i, vp)
     fn("kvcm_gemm_skinny_splits", i, i, i)
     fn("kvcm_gemm_skinny_whole_splits", i, i, i)
     fn("kvcm_gemm_tiles_count")
@@ -393,6 +394,8 @@ class PendingAttention(PendingProduct):
     the operands; ``run`` the ordinary way: ``attend()`` leaves the attention's rows in ``x``, then the output product.
     h: the normed rows or NormedRows; handover: (a function that gives the launch its two buffers) see ``decode_front_buffers``."""
 
+    polls = -1      # looks at what is not there before a workgroup of the launch makes it itself (-1: as measured)
+
     def __init__(self, attend, h, wqkv, x, w, out, scratch, cache, tables, table_stride, row_seq, ctx_lens, slots, cos_sin, heads, scale, parts, handover):
         super().__init__(x, w, out, scratch)
         self.attend, self.h, self.wqkv, self.cache, self.tables, self.table_stride = attend, h, wqkv, cache, tables, table_stride
@@ -432,11 +435,12 @@ class PendingAttention(PendingProduct):
         if self.cos_sin is not None:
             _need(self.cos_sin.dtype == torch.float32 and self.cos_sin.is_contiguous() and self.cos_sin.numel() >= M * hd, "cos_sin must be float32 [rows, head_dim/2, 2]")
         now, after = self.handover()
-        _call("kvcm_decode_front", _ptr(h), h.stride(0), _ptr(self.wqkv), self.wqkv.stride(0), _ptr(self.h.ss) if normed else 0,
+        waits = () if self.polls < 0 else (self.polls,)
+        _call("kvcm_decode_front_waiting" if waits else "kvcm_decode_front", _ptr(h), h.stride(0), _ptr(self.wqkv), self.wqkv.stride(0), _ptr(self.h.ss) if normed else 0,
               self.h.ss.shape[1] if normed else 0, self.h.eps if normed else 0.0, _ptr(self.w), self.w.stride(0), M, H, _ptr(self.cos_sin),
               _ptr(self.slots), _ptr(kc), _ptr(vc), _ptr(self.tables), self.table_stride, self.tables.numel() // self.table_stride,
               _ptr(self.row_seq), _ptr(self.ctx_lens), nh, nkv, hd, B, float(self.scale), _ptr(x), _ptr(weight), _DT[weight.dtype], _ptr(xg),
-              _ptr(ss), _ptr(now), _ptr(after), now.numel(), self.parts, _stream())
+              _ptr(ss), _ptr(now), _ptr(after), now.numel(), self.parts, *waits, _stream())
         return NormedRows(xg[:M], ss[:M], eps, x, weight, out)
 
 
