@@ -683,6 +683,16 @@ int kvcm_decode_front_parts(int max_context) {
   return max_context <= 0 || fit > kMaxParts ? 0 : fit;
 }
 
+// The parts for rows that the launch takes, and faster than three launches do; else 0.  It is not for heads of 64 with more than 192 (row, KV head)
+// pairs in more than one part each, where its attention, a workgroup a CU, is the longer (us, three launches / this one; 32 KV heads: 6 rows of 600, 1,200
+// and 1,900 tokens 24.7 / 23.7, 31.2 / 30.6, 38.0 / 37.7; 8 rows 26.6 / 27.0, 34.4 / 36.0, 42.7 / 44.6, of 100 tokens 20.9 / 20.4; heads of 128, 8 rows
+// 61.3 / 57.5, 74.1 / 71.5, 89.9 / 87.7).
+int kvcm_decode_front_takes(int M, int H, int nh, int nkv, int hd, int B, int max_context) {
+  if (!kvcm_decode_front_supported(M, H, nh, nkv, hd, B)) return 0;
+  const int parts = kvcm_decode_front_parts(max_context);
+  return hd == 64 && M * nkv > 192 && parts > 1 ? 0 : parts;
+}
+
 // 32-bit words of one of the two hand-over buffers (a multiple of four).
 long long kvcm_decode_front_words(int M, int nh, int nkv, int hd, int parts) {
   const long long n = static_cast<long long>(M) * ((nh + 2 * nkv) * hd + nh * hd / 2 + nh * (parts - 1) * (hd + 2));

@@ -96,6 +96,7 @@ int kvcm_gemm_f32_few(const float* X, const float* g, float eps, const float* W,
 // attention, output product, residual addition and the next norm's preparation, handed on through two buffers in turn.
 int kvcm_decode_front_supported(int M, int H, int nh, int nkv, int hd, int B);
 int kvcm_decode_front_parts(int max_context);
+int kvcm_decode_front_takes(int M, int H, int nh, int nkv, int hd, int B, int max_context);
 long long kvcm_decode_front_words(int M, int nh, int nkv, int hd, int parts);
 int kvcm_decode_front_empty(uint32_t* words, long long n, hipStream_t stream);
 int kvcm_decode_front(const void* X, int ldx, const void* Wqkv, int ldqkv, const float* ss_in, int tiles_in, float eps, const void* Wo, int ldo,

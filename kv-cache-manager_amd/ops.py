@@ -53,7 +53,7 @@ def _declare(lib):
     fn("kvcm_attention_f32_decode_supported", i, i, i, i)
     fn("kvcm_attention_f32_decode", vp, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, i, i, i, i, i, f, i, vp)
     fn("kvcm_decode_front_supported", i, i, i, i, i, i)
-    fn("kvcm_decode_front_parts", i)
+    fn("kvcm_decode_front_takes", i, i, i, i, i, i, i)
     lib.kvcm_decode_front_words.restype = C.c_longlong
     lib.kvcm_decode_front_words.argtypes = [i] * 5
     fn("kvcm_decode_front_empty", vp, C.c_longlong, vp)
@@ -445,8 +445,9 @@ class PendingAttention(PendingProduct):
 
 
 def decode_front_parts(M, H, nh, nkv, hd, block_size, max_context):
-    """Workgroups per row and KV head of the launch above for contexts of up to max_context tokens, 0 where it does not take the shape."""
-    return lib().kvcm_decode_front_parts(max_context) if lib().kvcm_decode_front_supported(M, H, nh, nkv, hd, block_size) else 0
+    """Workgroups per row and KV head of the launch above for contexts of up to max_context tokens, 0 where it does not take the shape or is
+    not the faster."""
+    return lib().kvcm_decode_front_takes(M, H, nh, nkv, hd, block_size, max_context)
 
 
 def decode_front_buffers(step, M, nh, nkv, hd, parts):

@@ -51,3 +51,11 @@ def test_two_streams_at_once(ops):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_many_short_heads_keep_three_launches(ops):
+    """Heads of 64 with more than 192 pairs of a row and a KV head, in more than one part each: the one launch was up to 5 % slower."""
+    parts = ops.decode_front_parts
+    assert parts(8, 2048, 32, 32, 64, 16, 513) == 0 and parts(7, 2048, 32, 32, 64, 16, 2048) == 0
+    assert parts(8, 2048, 32, 32, 64, 16, 512) == 1 and parts(6, 2048, 32, 32, 64, 16, 2048) == 4
+    assert parts(8, 4096, 32, 32, 128, 16, 2048) == 4 and parts(8, 2048, 32, 16, 64, 16, 2048) == 4
