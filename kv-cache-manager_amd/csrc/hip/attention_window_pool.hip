@@ -506,6 +506,8 @@ __device__ __forceinline__ float below_upper(float x) {
 // needs are on their way together.  Four launches as one, 8 rows of 32 heads over 4 kv heads of 64, window 512, blocks of 64, 4 taps: in a row
 // of such launches 540 tokens 16.7 -> 15.6 us, 60 tokens 14.0 -> 11.4; between a decoder's other launches 22.8 -> 16.9.  Heads of 128, whose first
 // keys and values the registers do not hold beside it, lose (8 rows, 30.1 -> 31.2), and so do norms over all heads in its place (13.4 -> 13.8).
+// With the front the kernel has 168 registers, 14 of which are spilled (60 bytes a lane), without it 138 and none: a workgroup fills its CU, which is
+// why more workgroups than CUs run the launches one by one (kvcm_attention_window_pool_rows_takes).
 struct WpFront {
   const float* src; int ld;
   const float* conv_w; const float* conv_bias; float* conv_state; const int* state_slots; int taps;
@@ -1070,6 +1072,16 @@ int kvcm_attention_window_pool(const void* q, int dtype, int ldq, void* out, int
 int kvcm_attention_window_pool_rows_supported(int nh, int nkv, int d, int dv, int B) {
   return nkv > 0 && nh % nkv == 0 && nh / nkv >= 2 && nh / nkv <= 16 && d > 0 && dv > 0 && d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 64 && B > 0 &&
          B % 8 == 0 && nkv <= 65535;
+}
+
+// ... and T rows of them faster than the four launches do: while every workgroup has a CU to itself.  Its registers leave no room for a second one beside
+// it, and where a second turn follows, a workgroup that ends with a pooled entry (a wave that walks the block's tokens) holds everything up.  us, four
+// launches / one, blocks of 64, window 512: 32 heads over 4 of 64, 16 / 32 / 64 rows of 540 tokens 18.3 / 16.6, 23.1 / 17.0, 26.0 / 19.6, some of them
+// at the end of a block (60 to 75 tokens) 23.7 / 20.2, 27.8 / 20.4, 29.8 / 21.1; 80, 128, 256, 512 rows 34.1 / 32.6, 37.4 / 36.8, 72.3 / 82.4, 125.3 / 153.5 and 34.8 / 39.3, 38.9 /
+// 39.9, 56.1 / 76.8, 84.2 / 149.4; 16 heads over 8, 32 rows 24.6 / 17.7, 48 rows 32.0 / 29.9 and 33.4 / 37.4, 128 rows 61.0 / 70.0.
+int kvcm_attention_window_pool_rows_takes(int T, int nh, int nkv, int d, int dv, int B) {
+  constexpr int kCUs = 256;
+  return kvcm_attention_window_pool_rows_supported(nh, nkv, d, dv, B) && T > 0 && T <= kCUs / nkv;
 }
 
 // bfloat16 rows of T different sequences, one each, from the projection's 32-bit rows [q | k | v] to the attention's: convolution (conv_w [C][taps],

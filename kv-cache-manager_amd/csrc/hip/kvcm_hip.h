@@ -223,6 +223,7 @@ int kvcm_norm_rotate_store(const float* src, int ld, const float* wq, const floa
                            void* q_out, int dtype, int ldq, void* kcache, void* vcache, int T, int nh, int nkv, int d, int dv, int B,
                            hipStream_t s);
 int kvcm_attention_window_pool_rows_supported(int nh, int nkv, int d, int dv, int B);
+int kvcm_attention_window_pool_rows_takes(int T, int nh, int nkv, int d, int dv, int B);
 int kvcm_attention_window_pool_rows(const float* src, int ld, const float* conv_w, const float* conv_bias, float* conv_state, const int* state_slots,
                                     int taps, const float* cos_sin, int rot, int halves, const int* slots, void* out, int ldo, void* kcache, void* vcache,
                                     float* pk, float* pv, const int* tables, int table_stride, const int* row_seq, const int* ctx_lens,

@@ -147,6 +147,7 @@ def _declare(lib):
     fn("kvcm_pool_update", vp, vp, i, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, i, vp)
     fn("kvcm_attention_window_pool", vp, i, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, f, i, i, i, i, f, i, i, vp, i, f, vp)
     fn("kvcm_attention_window_pool_rows_supported", i, i, i, i, i)
+    fn("kvcm_attention_window_pool_rows_takes", i, i, i, i, i, i)
     fn("kvcm_attention_window_pool_rows", vp, i, vp, vp, vp, vp, i, vp, i, i, vp, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, f, i, i, vp)
     fn("kvcm_attention_window_pool_tiles_supported", i, i, i)
     fn("kvcm_attention_window_pool_tiles", vp, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, f, i, i, i, i, f, i, i, vp, i, f, vp)
@@ -1601,6 +1602,11 @@ def attention_window_pool(q, out, kcache, vcache, pk, pv, tables, table_stride, 
 
 def attention_window_pool_rows_supported(nh, nkv, d, dv, dtype, block_size):
     return dtype == torch.bfloat16 and bool(lib().kvcm_attention_window_pool_rows_supported(nh, nkv, d, dv, block_size))
+
+
+def attention_window_pool_rows_takes(T, nh, nkv, d, dv, dtype, block_size):
+    """Does ``attention_window_pool_rows`` take T rows of these heads, and faster than the launches one by one?"""
+    return dtype == torch.bfloat16 and bool(lib().kvcm_attention_window_pool_rows_takes(T, nh, nkv, d, dv, block_size))
 
 
 def attention_window_pool_rows(qkv, out, kcache, vcache, pk, pv, step, tables, table_stride, slots, nh, nkv, d, dv, scale, window, P, conv, conv_state,

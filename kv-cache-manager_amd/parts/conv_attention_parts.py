@@ -106,8 +106,8 @@ class ConvWindowPoolAttention(Mixer):
         slots = step.slots(g) if self.cache_owner else None
         attn = step.ws("cwp_attn", (T, self.nh * self.dv))
         if (step.max_run == 1 and slots is not None
-                and ops.attention_window_pool_rows_supported(self.nh, self.nkv, self.d, self.dv, attn.dtype, kc.shape[2])):
-            # every sequence runs one row: all between the two products is one launch, a workgroup per row and KV head
+                and ops.attention_window_pool_rows_takes(T, self.nh, self.nkv, self.d, self.dv, attn.dtype, kc.shape[2])):
+            # every sequence runs one row, of not too many: all between the two products is one launch, a workgroup per row and KV head
             ops.attention_window_pool_rows(proj, attn, kc, vc, pk, pv, step, step.tables(g), step.table_stride(g), slots, self.nh, self.nkv,
                                            self.d, self.dv, p["scale"], p["window"], pool, w["conv"], self.conv_state(),
                                            conv_bias=w["bias"], head_scale=w["temp"], cos_sin=self.position.pairs_table(step),

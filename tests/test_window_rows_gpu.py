@@ -89,3 +89,13 @@ def test_what_it_refuses():
     for nh, nkv, d, dv, B in ((4, 4, 64, 64, 16), (34, 2, 64, 64, 16), (8, 2, 68, 64, 16), (8, 2, 72, 64, 16), (8, 2, 64, 72, 16), (8, 2, 64, 64, 12)):
         assert not sup(nh, nkv, d, dv, torch.bfloat16, B)
     assert not sup(8, 2, 64, 64, torch.float32, 16)
+
+
+def test_it_is_left_alone_where_workgroups_outnumber_the_chip():
+    """256 workgroups have a CU each; more rows ran up to 1.8 times as long as in the launches one by one."""
+    from kvcm_amd import ops
+    takes = ops.attention_window_pool_rows_takes
+    for nkv, most in ((4, 64), (8, 32), (3, 85), (1, 256)):
+        assert takes(most, 4 * nkv, nkv, 64, 64, torch.bfloat16, 16) and not takes(most + 1, 4 * nkv, nkv, 64, 64, torch.bfloat16, 16)
+    assert not takes(0, 8, 2, 64, 64, torch.bfloat16, 16) and not takes(1, 8, 512, 64, 64, torch.bfloat16, 16)
+    assert not takes(8, 8, 2, 64, 64, torch.float32, 16) and not takes(8, 8, 2, 72, 64, torch.bfloat16, 16)
