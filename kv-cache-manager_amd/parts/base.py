@@ -203,6 +203,14 @@ def as_tensor(value):
     return value.materialize() if hasattr(value, "materialize") else value
 
 
+def said_with(part, name, method):
+    """Does what ``part`` says by ``name`` hold for the ``method`` it runs: is it said by the class that defines the method, or by one derived
+    from it?  A part that replaces a method of its base's has not said what the base says about its own, and runs the ordinary way."""
+    places = [vars(part)] + [vars(c) for c in type(part).__mro__]
+    first = [next((i for i, place in enumerate(places) if n in place), len(places)) for n in (name, method)]
+    return first[0] < len(places) and first[0] <= first[1]
+
+
 class Part:
     """Base of every part.  Subclasses read ``params``, declare tensors in ``param_specs`` and get
     them (already on the device, in the precision their role asks for) through ``bind``."""
@@ -315,6 +323,7 @@ class Mixer(Part):
     accepts_normed_rows = False
     # True: ``forward`` takes ``defer=True``, passed by a block whose norm behind the mixer folds and runs next, before anything else
     # touches what the mixer reads or writes: the mixer may then return an ops.PendingProduct none of whose launches has run yet.
+    # (A subclass with a ``forward`` of its own says it anew.)
     defers = False
 
     def forward(self, step, h):

@@ -6,7 +6,7 @@ Every size, constant and tensor name is a parameter.
 import torch
 
 from ..registry import MIXERS, POSITIONS
-from .base import KVCacheNeed, Mixer, ParamSpec, PartSpec, PositionEncoding, StateNeed
+from .base import KVCacheNeed, Mixer, ParamSpec, PartSpec, PositionEncoding, StateNeed, said_with
 from .chain_norm_parts import BranchPair, f32_params
 from .llama_parts import run_stages, side_by_side
 
@@ -165,7 +165,8 @@ class ParallelMixers(Mixer):
 
     def forward(self, step, h):
         left, right = self.left, self.right
-        if getattr(left, "buffers", None) and getattr(right, "buffers", None) and left.buffers != right.buffers:
+        in_step = [m for m in (left, right) if getattr(m, "buffers", None) and said_with(m, "stages", "forward")]
+        if len(in_step) == 2 and left.buffers != right.buffers:
             a, b = side_by_side(self.ctx, step, left.stages(step, h), right.stages(step, h))
         else:
             a = left.forward(step, h)

@@ -10,7 +10,7 @@ import torch
 
 from ..registry import BLOCKS, EMBEDDINGS, FEED_FORWARDS, HEADS, MIXERS, NORMS, POSITIONS
 from . import paged_attention
-from .base import (Block, Embedding, FeedForward, Head, KVCacheNeed, Mixer, Norm, ParamSpec, PositionEncoding, as_tensor)
+from .base import (Block, Embedding, FeedForward, Head, KVCacheNeed, Mixer, Norm, ParamSpec, PositionEncoding, as_tensor, said_with)
 
 
 def _linear(ctx, step, x, w, name, keep_partial=False, dtype=None):
@@ -270,7 +270,8 @@ class GQAAttention(Mixer):
                 step, ops, res, attn, kc, vc, g, self.nh, self.nkv, self.hd, self.scale, self.window, table, slots):
             return attn
         # 32-bit rows of different sequences: rotation, page write and attention in one launch, the same bits
-        if (slots is not None and step.max_run == 1 and qkv.dtype == torch.float32 and (table is not None or not pos.rotates)
+        if (slots is not None and step.max_run == 1 and qkv.dtype == torch.float32
+                and (table is not None and said_with(pos, "rotation_table", "apply") or not pos.rotates)
                 and ops.attention_f32_decode_supported(self.nh, self.nkv, self.hd, self.ctx.block_size)):
             ops.attention_f32_decode(res, attn, kc, vc, step.tables(g), step.table_stride(g), step.row_seq, step.ctx_lens, self.nh, self.nkv, self.hd,
                                      self.scale, slots, cos_sin=table, window=self.window, rows=step.rows)
@@ -379,7 +380,7 @@ class PreNormResidual(Block):
         fold2 = {"defer": True} if (step.fold_norms and n2.defers and ffn.accepts_normed_rows) else {}
         h = n1.forward(x, buf, add=pending if n1.accepts_partial_sums else as_tensor(pending), **fold1)
         # a mixer may leave all of its launches to the norm behind it (Mixer.defers), which runs at once
-        late = {"defer": True} if (n2.defers and n2.accepts_partial_sums and mixer.defers and fold2) else {}
+        late = {"defer": True} if (n2.defers and n2.accepts_partial_sums and mixer.defers and fold2 and said_with(mixer, "defers", "forward")) else {}
         a = mixer.forward(step, buf if h is None else h, **late)
         h = n2.forward(x, buf, add=a if n2.accepts_partial_sums else as_tensor(a), **fold2)
-        return ffn.forward(step, buf if h is None else h, **({"defer": True} if fold2 and ffn.defers else {}))
+        return ffn.forward(step, buf if h is None else h, **({"defer": True} if fold2 and ffn.defers and said_with(ffn, "defers", "forward") else {}))

@@ -171,7 +171,7 @@ class RoutedExperts(JoinableEnds, FeedForward):
     def _beside(self, h, F, H, top, E):
         """Does the shared feed-forward run in the experts' launches (ops.moe_few_beside)?"""
         sh = self.shared
-        return (self.gated and isinstance(sh, GatedFeedForward) and not self.by_ends and not sh.params.get("bias") and not sh.params.get("joined")
+        return (self.gated and isinstance(sh, GatedFeedForward) and getattr(sh.forward, "__func__", None) is GatedFeedForward.forward and not self.by_ends and not sh.params.get("bias") and not sh.params.get("joined")
                 and sh.params.get("activation", "silu") == "silu" and torch.is_tensor(h) and h.dtype == torch.bfloat16
                 and self.ctx.ops.moe_few_beside_takes(h, F, H, top, E, sh.w["w_gate_up"]))
 
