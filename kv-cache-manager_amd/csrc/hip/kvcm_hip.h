@@ -351,12 +351,12 @@ int kvcm_program_run(void* program, hipStream_t stream);
 // reached through the addresses of nine of its C functions: kvcm_sched_schedule_summary,
 // kvcm_build_batch_from_plan_shaped, kvcm_sched_update_sampled, kvcm_last_error, kvcm_sched_add,
 // kvcm_sched_idle, kvcm_sched_collect_finished, kvcm_finished_get, kvcm_finished_clear), the pinned and the
-// device metadata buffers of the model's step function, the sampler's device and pinned id buffers, the
+// device metadata buffers of the model's step function, the sampler's pinned id buffer, the
 // engine's limits and a stream of its own.  A step runs here from schedule to update when its canonical
 // shape has a recorded program (kvcm_program_*); the first step of a shape is recorded by whoever holds the
 // model's parts (they decide the launches), and handed over with kvcm_engine_register.
 void* kvcm_engine_new(void* core, const uint64_t* host_functions, int32_t* meta_host, int32_t* meta_dev, long long meta_ints,
-                      int32_t* sampled_dev, int32_t* sampled_host, int max_sampled, int num_groups, int block_size,
+                      int32_t* sampled_host, int max_sampled, int num_groups, int block_size,
                       int max_context, int max_tokens, int max_seqs, int max_logit_rows, int graph_rows, hipStream_t stream);
 void kvcm_engine_delete(void* engine);
 int kvcm_engine_add(void* engine, long long id, const int32_t* tokens, int n, int max_new_tokens, float temperature,

@@ -87,7 +87,6 @@ struct Engine {
   int32_t* meta_host = nullptr;   // pinned
   int32_t* meta_dev = nullptr;
   long long meta_ints = 0;
-  int32_t* sampled_dev = nullptr;
   int32_t* sampled_host = nullptr;   // pinned
   int max_sampled = 0;
   int block_size = 16, max_context = 0, max_tokens = 0, max_seqs = 0, max_logit_rows = 0;
@@ -147,10 +146,10 @@ extern "C" {
 
 // host_functions: addresses of kvcm_sched_schedule_summary, kvcm_build_batch_from_plan_shaped,
 // kvcm_sched_update_sampled, kvcm_last_error, kvcm_sched_add, kvcm_sched_idle, kvcm_sched_collect_finished,
-// kvcm_finished_get and kvcm_finished_clear of the host core library, in this order.  meta_host, sampled_host: pinned.  sampled_dev: where
-// the programs leave the sampled ids; null: they write sampled_host themselves.
+// kvcm_finished_get and kvcm_finished_clear of the host core library, in this order.  meta_host, sampled_host: pinned; the
+// recorded programs write the sampled ids to sampled_host themselves.
 void* kvcm_engine_new(void* core, const uint64_t* host_functions, int32_t* meta_host, int32_t* meta_dev, long long meta_ints,
-                      int32_t* sampled_dev, int32_t* sampled_host, int max_sampled, int num_groups, int block_size,
+                      int32_t* sampled_host, int max_sampled, int num_groups, int block_size,
                       int max_context, int max_tokens, int max_seqs, int max_logit_rows, int graph_rows, hipStream_t stream) {
   if (!core || !host_functions || !meta_host || !meta_dev || !sampled_host || !stream) {
     kvcm::set_error("engine_new: null argument (the engine needs a stream of its own, not the default one)");
@@ -173,7 +172,7 @@ void* kvcm_engine_new(void* core, const uint64_t* host_functions, int32_t* meta_
       return nullptr;
     }
   e->meta_host = meta_host; e->meta_dev = meta_dev; e->meta_ints = meta_ints;
-  e->sampled_dev = sampled_dev; e->sampled_host = sampled_host; e->max_sampled = max_sampled;
+  e->sampled_host = sampled_host; e->max_sampled = max_sampled;
   e->block_size = block_size; e->max_context = max_context; e->max_tokens = max_tokens; e->max_seqs = max_seqs;
   e->max_logit_rows = max_logit_rows < max_sampled ? max_logit_rows : max_sampled;
   e->graph_rows = graph_rows;
@@ -256,7 +255,7 @@ int kvcm_engine_register(void* engine, void* program, int as_graph) {
   return 0;
 }
 
-// Runs the planned step from its recorded program: build, upload, launches, download, update.
+// Runs the planned step from its recorded program: build, upload, launches, update.
 // info[0..4]: rows, sequences, sampled ids, 1 if a graph was replayed, microseconds the host spent
 // from the scheduler's call to the last launch (before it waits for the GPU).  Returns 1 when the step
 // ran, 0 when its shape has no program (nothing was done: the caller runs and records it),
@@ -292,10 +291,6 @@ int kvcm_engine_run(void* engine, double now, int defer_update, int64_t* info) {
     ++e->steps_as_graph;
   } else {
     if (int rc = kvcm_program_run(rec.program, e->stream)) return rc;
-  }
-  if (sampling > 0 && e->sampled_dev) {
-    err = hipMemcpyAsync(e->sampled_host, e->sampled_dev, size_t(sampling) * 4, hipMemcpyDeviceToHost, e->stream);
-    KVCM_REQUIRE(err == hipSuccess, "engine_run: download: %s", hipGetErrorString(err));
   }
   const double issued = std::chrono::duration<double>(std::chrono::steady_clock::now() - e->t_plan).count();
   err = hipStreamSynchronize(e->stream);

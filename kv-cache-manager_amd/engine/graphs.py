@@ -87,7 +87,7 @@ class RecordedSteps:
         s = self.sampler
         self._h = self.lib.kvcm_engine_new(
             self.core.handle, fns, self.runner._pinned.data_ptr(), self.runner.meta_dev.data_ptr(), self.runner.meta_dev.numel(),
-            0, s._host.data_ptr(), s.max_rows,      # (recorded steps sample into pinned host memory)
+            s._host.data_ptr(), s.max_rows,      # (recorded steps sample into pinned host memory)
             self.core.num_groups, engine.config.block_size,
             lim.max_context_len, lim.max_tokens, lim.max_seqs, lim.max_logit_rows, GRAPH_ROWS if use_graphs else 0,
             self.stream.cuda_stream)

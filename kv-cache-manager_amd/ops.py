@@ -173,7 +173,7 @@ def _declare(lib):
     fn("kvcm_program_size", vp)
     fn("kvcm_program_run", vp, vp)
     lib.kvcm_engine_new.restype = vp
-    lib.kvcm_engine_new.argtypes = [vp, C.POINTER(C.c_uint64), vp, vp, C.c_longlong, vp, vp, i, i, i, i, i, i, i, i, vp]
+    lib.kvcm_engine_new.argtypes = [vp, C.POINTER(C.c_uint64), vp, vp, C.c_longlong, vp, i, i, i, i, i, i, i, i, vp]
     lib.kvcm_engine_delete.restype = None
     lib.kvcm_engine_delete.argtypes = [vp]
     fn("kvcm_engine_plan", vp, C.c_double, C.POINTER(C.c_int64))
