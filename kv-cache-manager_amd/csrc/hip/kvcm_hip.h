@@ -372,7 +372,7 @@ void kvcm_engine_finished_clear(void* engine);
 int kvcm_engine_plan(void* engine, double now, int64_t* out);
 int kvcm_engine_last_plan(void* engine, int64_t* out);      // the same report again, the scheduler not run
 int kvcm_engine_run(void* engine, double now, int defer_update, int64_t* info);
-int kvcm_engine_register(void* engine, void* program, int as_graph);
+int kvcm_engine_register(void* engine, void* program, int as_graph, long long step_ints);
 void kvcm_engine_stats(void* engine, int64_t* out);
 
 #ifdef __cplusplus

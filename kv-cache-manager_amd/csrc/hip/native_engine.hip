@@ -94,7 +94,6 @@ struct Engine {
   hipStream_t stream = nullptr;
   std::map<decltype(Shape().key()), std::unique_ptr<Recorded>> recorded;
   std::vector<int32_t> desc;
-  int num_groups = 0;
   int64_t summary[10] = {};
   int64_t last_plan[20] = {};   // what kvcm_engine_plan last reported
   int last_plan_entries = 0;
@@ -178,7 +177,6 @@ void* kvcm_engine_new(void* core, const uint64_t* host_functions, int32_t* meta_
   e->graph_rows = graph_rows;
   e->stream = stream;
   e->desc.assign(20 + 4 * num_groups, 0);
-  e->num_groups = num_groups;
   return e.release();
 }
 
@@ -225,21 +223,20 @@ int kvcm_engine_last_plan(void* engine, int64_t* out) {
 }
 
 // Hands a recorded program for the current plan's shape to the engine (which owns it from now on).
-// as_graph: capture it into a HIP graph (only launches of this library's kernels may be in it).
-int kvcm_engine_register(void* engine, void* program, int as_graph) {
+// as_graph: capture it into a HIP graph (only launches of this library's kernels may be in it).  step_ints: what the
+// step's metadata holds, which is the same for every step of the shape.
+int kvcm_engine_register(void* engine, void* program, int as_graph, long long step_ints) {
   auto* e = static_cast<Engine*>(engine);
   KVCM_REQUIRE(e->planned && program != nullptr, "engine_register: no planned step of a canonical shape");
+  KVCM_REQUIRE(step_ints > 0 && step_ints <= e->meta_ints, "engine_register: metadata of %lld ints, the buffers hold %lld", step_ints, e->meta_ints);
   auto rec = std::make_unique<Recorded>();
   rec->program = program;
   if (as_graph) {
     hipError_t err = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal);
     KVCM_REQUIRE(err == hipSuccess, "engine_register: begin capture: %s", hipGetErrorString(err));
-    // room for the shape's metadata, with its gaps: tokens, positions, contexts, slots, tables, sampling parameters
-    const Shape& sh = e->shape;
-    long long ints = 8ll * sh.rows + 8ll * sh.seqs + 8ll * sh.logit_rows + static_cast<long long>(e->num_groups) * (sh.rows + static_cast<long long>(sh.seqs) * sh.table_stride) + 256;
-    ints = (ints < e->meta_ints ? ints : e->meta_ints) / 4 * 4;
+    const long long ints = (step_ints + 3) / 4 * 4;
     const bool pieces = reinterpret_cast<uintptr_t>(e->meta_host) % 16 == 0 && reinterpret_cast<uintptr_t>(e->meta_dev) % 16 == 0;
-    if (pieces && ints <= kUploadInts) {
+    if (pieces && ints <= e->meta_ints && ints <= kUploadInts) {
       rec->uploads = ints;
       upload_kernel<<<static_cast<int>((ints / 4 + 255) / 256), 256, 0, e->stream>>>(reinterpret_cast<const int4*>(e->meta_host), reinterpret_cast<int4*>(e->meta_dev),
                                                                                     static_cast<int>(ints / 4));
@@ -281,7 +278,8 @@ int kvcm_engine_run(void* engine, double now, int defer_update, int64_t* info) {
   const int sampling = int(e->summary[3]);
   KVCM_REQUIRE(sampling <= e->max_sampled, "engine_run: %d sampling rows exceed the sampler's %d", sampling, e->max_sampled);
   hipError_t err = hipSuccess;
-  if (total > rec.uploads) {
+  KVCM_REQUIRE(rec.uploads == 0 || total <= rec.uploads, "engine_run: metadata of %d ints, the recorded graph fetches %lld", total, rec.uploads);
+  if (rec.uploads == 0) {
     err = hipMemcpyAsync(e->meta_dev, e->meta_host, size_t(total) * 4, hipMemcpyHostToDevice, e->stream);
     KVCM_REQUIRE(err == hipSuccess, "engine_run: upload: %s", hipGetErrorString(err));
   }

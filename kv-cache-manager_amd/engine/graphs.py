@@ -162,7 +162,7 @@ class RecordedSteps:
                 ops.LIBRARY_GEMM_MIN_ROWS = keep
             self.stream.synchronize()
             sampled = self.sampler._host[:sampling].numpy().copy()
-            if self.lib.kvcm_engine_register(self._h, program.release(), int(self.wants_graph)) != 0:
+            if self.lib.kvcm_engine_register(self._h, program.release(), int(self.wants_graph), layout.total) != 0:
                 raise ops.KernelError(self.lib.kvcm_hip_last_error().decode())
             self.recorded_shapes[shape] = "graph" if self.wants_graph else "program"
         return layout, sampled

@@ -24,3 +24,21 @@ def test_graphs_fetch_their_metadata(tmp_path, rows, longest):
         if graphs:
             assert eng.decode_graphs.graph_shapes(), "no graph was captured"
     assert out[0] == out[1]
+
+
+def test_a_graph_that_fetches_less_than_a_step_holds_is_an_error(tmp_path):
+    """The graph fetches what the step it was recorded from holds, not a guess at it: a step that holds more is not run."""
+    from kvcm_amd import Engine, EngineConfig, ops
+    d = str(tmp_path / "m")
+    H.make_model_dir(d, H.TINY_D, H.WEIGHT_SEED["D"], torch.bfloat16, sharpen=H.SHARPEN["D"])
+    eng = Engine(d, EngineConfig(dtype="bfloat16", block_size=8, num_blocks=64, max_seq_len=64, max_num_seqs=4, max_batched_tokens=64))
+    build = eng.core.build_batch_from_plan
+
+    def short(*args, **kw):
+        layout = build(*args, **kw)
+        layout.total -= 4
+        return layout
+
+    eng.core.build_batch_from_plan = short
+    with pytest.raises(ops.KernelError, match="metadata of"):
+        eng.generate([[1, 2, 3]], 6)
