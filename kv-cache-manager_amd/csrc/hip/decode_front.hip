@@ -10,8 +10,8 @@
 // work, and hand results on through memory, past the caches, in words that are their own flags: a buffer is full of kEmpty before
 // the launch, a word that is something else is there.  No counter, no fence, no order between words is needed, and a hand-over
 // costs 0.8 to 1 us.  Measured (us a layer: three launches / this one, eight layers of distinct weights in a graph, contexts of 600 and
-// 1,900 tokens): TinyLlama sizes 1 row 18.7 / 11.7 and 26.4 / 12.0, 8 rows 20.1 / 13.7 and 30.1 / 17.1; width 4096, 8 KV heads of 128, 1
-// row 37.7 / 28.9 and 53.1 / 29.0, 8 rows 46.2 / 33.1 and 62.8 / 41.6; 32 KV heads of 128, 1 row of 600 49.2 / 41.0.
+// 1,900 tokens): TinyLlama sizes 1 row 18.5 / 11.7 and 18.9 / 12.0, 8 rows 20.1 / 13.7 and 21.6 / 16.8; width 4096, 8 KV heads of 128, 1
+// row 33.9 / 29.0 and 34.3 / 29.0, 8 rows 42.1 / 33.1 and 49.5 / 41.8; 32 KV heads of 128, 1 row of 600 45.3 / 41.2.
 //
 // Nobody waits for a workgroup of a higher number: [QKV tiles | attention, a row's and KV head's parts in ascending order | output tiles],
 // and workgroups are started in the order of their numbers on each XCD, so a launch that has the chip to itself always gets on.  Two at a time (engines with a
@@ -21,8 +21,9 @@
 // then its own part again.  It is the same code on the same operands, which the launch leaves as they are, so whoever else makes a word
 // too, and however late, stores the same bits; nothing depends on who runs beside whom.  This costs 0.3 to 0.4 us a layer (in the code's
 // shape, no wait more).  Several streams of such layers at once, us a layer of each, three launches / this one: TinyLlama sizes, 8 rows of 600, two
-// streams 26.3 / 20.0, three 29.6 / 25.5, four 33.6 / 33.4 (up to 44); width 4096, 8 KV heads, 8 rows of 1,900 84.4 / 67.3, 107.5 / 128 (up to 375 where
-// output tiles gave up), 137.5 / 133.
+// streams 26.0 / 20.0, three 29.5 / 25.5, four 33.4 / 33.4 to 44; width 4096, 8 KV heads, 8 rows of 1,900, whose 256 output tiles are all the places
+// there are, 80.5 / 68, 120 / 128 to 375, 155 / 133 to 324: three or more engines of that size share a GPU better without (giving up takes an
+// output tile some 2 ms, as it makes everything).
 //
 // Attention: a wave takes windows of 64 tokens (both products on the matrix cores, transposed, as in attention_decode_fused.hip), one
 // each: `parts` workgroups of eight waves share a row's KV head, window 8 w + part belonging to wave w.  The last part adds the
@@ -91,7 +92,8 @@ __device__ __forceinline__ uint32_t filled(float v) {
   const uint32_t w = __float_as_uint(v);
   return w == kEmpty ? 0x7FC00000u : w;
 }
-// 2^(s - top), nothing for what is masked
+// 2^(s - top), nothing for what is masked.  (The hardware's exp2: exact to an ulp, but a share below 2^-126 is zero where exp2f's is 2^-149 at the least.  Values
+// are at most 2^128, so what is lost matters where one's value is 2^117 times the result's; exp2f costs 0.3 us a layer at width 2,048, 2 at 4,096.)
 __device__ __forceinline__ float share(float s, float top) { return s > 0.5f * kNone ? __builtin_amdgcn_exp2f(s - top) : 0.f; }
 __device__ __forceinline__ bool empty_half(uint64_t v) { return uint32_t(v) == kEmpty || uint32_t(v >> 32) == kEmpty; }
 
@@ -684,9 +686,9 @@ int kvcm_decode_front_parts(int max_context) {
 }
 
 // The parts for rows that the launch takes, and faster than three launches do; else 0.  It is not for heads of 64 with more than 192 (row, KV head)
-// pairs in more than one part each, where its attention, a workgroup a CU, is the longer (us, three launches / this one; 32 KV heads: 6 rows of 600, 1,200
-// and 1,900 tokens 24.7 / 23.7, 31.2 / 30.6, 38.0 / 37.7; 8 rows 26.6 / 27.0, 34.4 / 36.0, 42.7 / 44.6, of 100 tokens 20.9 / 20.4; heads of 128, 8 rows
-// 61.3 / 57.5, 74.1 / 71.5, 89.9 / 87.7).
+// pairs in more than one part each, where its attention, a workgroup a CU, is the longer (us, three launches / this one; 32 KV heads, contexts of 100, 600, 1,000, 1,200 and
+// 1,900 tokens: 6 rows 20.5 / 21.8, 24.4 / 23.5, 29.8 / 26.8, 38.5 / 33.9, 46.4 / 37.5; 8 rows 21.1 / 23.5, 26.9 / 27.3, 32.4 / 32.6, 34.4 / 39.8, 42.7 / 44.7; heads of
+// 128, 8 rows 51.6 / 48.5, 61.8 / 57.9, 70.0 / 66.4, 74.4 / 73.6, 90.5 / 88.4).
 int kvcm_decode_front_takes(int M, int H, int nh, int nkv, int hd, int B, int max_context) {
   if (!kvcm_decode_front_supported(M, H, nh, nkv, hd, B)) return 0;
   const int parts = kvcm_decode_front_parts(max_context);

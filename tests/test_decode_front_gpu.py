@@ -92,7 +92,8 @@ def _layers(ops, H, nh, nkv, hd, B, lens, layers, seed, rotate=True, stored=None
 def test_attention_half_in_one_launch(ops, H, nh, nkv, hd, B, lens):
     """Every edge of a window, of a part and of a page, a row's first token, padding rows, rows in another order than their sequences,
     K slices of unequal length, three layers through the two buffers in turn.  What differs is the order of 32-bit sums, that
-    is single bfloat16 roundings: of q, k and v, of the attention's rows, of the product (2^-9 of their size each, most of them equal)."""
+    is single bfloat16 roundings: of q, k and v, of the attention's rows, of the product (at most a unit of the last place, 2^-7 of
+    their size, most of them equal).  Entry by entry: test_decode_front_exact_gpu.py."""
     run, x0, slots = _layers(ops, H, nh, nkv, hd, B, lens, 3, seed=H + nh + len(lens), scaled_first=len(lens) % 2 == 0)
     want, got = run(False), run(True)
     live = np.array([s >= 0 for s in slots])
