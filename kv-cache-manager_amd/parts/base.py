@@ -287,7 +287,8 @@ class Norm(Part):
     accepts_partial_sums = False
     # True: ``forward`` takes ``defer=True`` and may then return, instead of ``out``, a Deferred whose
     # scale is still to be applied by the product that consumes it (ops.NormedRows); the arrangement
-    # asks for it only when the consuming part ``accepts_normed_rows``.
+    # asks for it only when the consuming part ``accepts_normed_rows``.  ``defer="rows"``, for parts that
+    # say ``accepts_rows_to_norm``: or 32-bit rows that the product norms itself (ops.RowsToNorm).
     defers = False
 
     def forward(self, x, out, add=None, rows=None):
@@ -321,6 +322,8 @@ class PositionEncoding(Part):
 class Mixer(Part):
     # True: ``h`` may be a Deferred (ops.NormedRows) that the mixer's first product consumes as it is.
     accepts_normed_rows = False
+    # True: ``h`` may also be an ops.RowsToNorm.  (A subclass with a ``forward`` of its own says it anew.)
+    accepts_rows_to_norm = False
     # True: ``forward`` takes ``defer=True``, passed by a block whose norm behind the mixer folds and runs next, before anything else
     # touches what the mixer reads or writes: the mixer may then return an ops.PendingProduct none of whose launches has run yet.
     # (A subclass with a ``forward`` of its own says it anew.)
@@ -333,6 +336,7 @@ class Mixer(Part):
 
 class FeedForward(Part):
     accepts_normed_rows = False      # as Mixer.accepts_normed_rows
+    accepts_rows_to_norm = False     # as Mixer.accepts_rows_to_norm
     defers = False                   # as Mixer.defers
 
     def forward(self, step, h):

@@ -113,7 +113,7 @@ class RMSNorm(Norm):
 
     def forward(self, x, out, add=None, rows=None, defer=False):
         ops = self.ctx.ops
-        if defer and rows is None and (add is None or isinstance(add, ops.PendingProduct)) and ops.can_norm_rows(x, self.w["weight"], out):
+        if defer == "rows" and rows is None and (add is None or isinstance(add, ops.PendingProduct)) and ops.can_norm_rows(x, self.w["weight"], out):
             if add is not None:
                 ops.gemm_residual(add, x)
             return ops.RowsToNorm(x, self.w["weight"], self.params["eps"], out)
@@ -190,7 +190,7 @@ class GQAAttention(Mixer):
     params: num_heads, num_kv_heads, head_dim, scale, window (0 = all keys), position (PartSpec)."""
 
     capturable = True
-    accepts_normed_rows = True
+    accepts_normed_rows = accepts_rows_to_norm = True
     defers = True
 
     def sub_parts(self):
@@ -292,7 +292,7 @@ class SwiGLU(FeedForward):
     (src/model/llama.cpp:119-122, src/cuda/kernels.cu:72-82).  params: intermediate_size."""
 
     capturable = True
-    accepts_normed_rows = True
+    accepts_normed_rows = accepts_rows_to_norm = True
     defers = True
 
     def param_specs(self):
@@ -376,8 +376,8 @@ class PreNormResidual(Block):
         n1, n2 = self.parts["norm_mixer"], self.parts["norm_ffn"]
         mixer, ffn = self.parts["mixer"], self.parts["ffn"]
         # a norm may leave its scale to the product that follows (Norm.defers) where that part takes it
-        fold1 = {"defer": True} if (step.fold_norms and n1.defers and mixer.accepts_normed_rows) else {}
-        fold2 = {"defer": True} if (step.fold_norms and n2.defers and ffn.accepts_normed_rows) else {}
+        fold1, fold2 = ({"defer": "rows" if part.accepts_rows_to_norm and said_with(part, "accepts_rows_to_norm", "forward") else True}
+                        if (step.fold_norms and norm.defers and part.accepts_normed_rows) else {} for norm, part in ((n1, mixer), (n2, ffn)))
         h = n1.forward(x, buf, add=pending if n1.accepts_partial_sums else as_tensor(pending), **fold1)
         # a mixer may leave all of its launches to the norm behind it (Mixer.defers), which runs at once
         late = {"defer": True} if (n2.defers and n2.accepts_partial_sums and mixer.defers and fold2 and said_with(mixer, "defers", "forward")) else {}

@@ -9,7 +9,7 @@ from kvcm_amd.parts import llama_parts
 from kvcm_amd.parts.base import Mixer, Norm, said_with
 from kvcm_amd.parts.chain_norm_parts import GatedFeedForward
 from kvcm_amd.parts.conv_attention_parts import ConvWindowPoolAttention, ParallelMixers
-from kvcm_amd.parts.llama_parts import GQAAttention, PreNormResidual, Rotary, SwiGLU
+from kvcm_amd.parts.llama_parts import GQAAttention, PreNormResidual, RMSNorm, Rotary, SwiGLU
 from kvcm_amd.parts.recurrent_parts import SelectiveScanMixer
 from kvcm_amd.parts.routed_parts import RoutedExperts
 
@@ -56,6 +56,41 @@ def test_a_block_runs_mixers_and_feed_forwards_with_a_forward_of_their_own():
         assert torch.equal(block.forward(STEP, x, None), torch.full((2, 4), float(result)))
     block = _bare(PreNormResidual, parts=dict(norm_mixer=_Fold(), norm_ffn=_Fold(), mixer=_bare(Double), ffn=_bare(SwiGLU, forward=lambda step, h: h)))
     assert torch.equal(block.forward(STEP, x, None), torch.full((2, 4), 3.0))
+
+
+def test_a_forward_of_its_own_gets_normed_rows_and_not_rows_to_norm():
+    """32-bit rows that a product norms itself go to the package's own forwards only, or to those that say they take them."""
+    class RowsToNorm:
+        def __init__(self, x, weight, eps, out):
+            self.x = x
+
+    ops = SimpleNamespace(PendingProduct=type("PendingProduct", (), {}), RowsToNorm=RowsToNorm, can_norm_rows=lambda x, weight, out: True,
+                          rmsnorm=lambda x, weight, out, eps, add=None, rows=None: out.copy_(x if add is None else x.add_(add)))
+    norm = _bare(RMSNorm, ctx=SimpleNamespace(ops=ops), params=dict(eps=0.0), w=dict(weight=None), _folded=None)
+
+    class Double(GQAAttention):
+        def forward(self, step, h):
+            return 2 * h
+
+    class Triple(SwiGLU):
+        def forward(self, step, h):
+            return 3 * h
+
+    class Takes(Triple):
+        accepts_rows_to_norm = True
+
+        def forward(self, step, h):
+            return 5 * h.x
+
+    run = lambda mixer, ffn: _bare(PreNormResidual, parts=dict(norm_mixer=norm, norm_ffn=norm, mixer=mixer, ffn=ffn)).forward(STEP, torch.ones(2, 4), None)
+    assert torch.equal(run(_bare(Double), _bare(Triple)), torch.full((2, 4), 9.0))
+    assert torch.equal(run(_bare(GQAAttention, forward=lambda step, h: 2 * h), _bare(SwiGLU, forward=lambda step, h: 3 * h)), torch.full((2, 4), 9.0))
+    norm_two = _bare(RMSNorm, **{**vars(norm), "w": dict(weight=1)})
+    got = _bare(PreNormResidual, parts=dict(norm_mixer=norm, norm_ffn=norm_two, mixer=_bare(Double, forward=lambda step, h: None), ffn=_bare(Takes))).forward(
+        STEP, torch.ones(2, 4), None)
+    assert torch.equal(got, torch.full((2, 4), 5.0))
+    out = torch.zeros(2, 4)
+    assert norm.forward(torch.ones(2, 4), out, defer=True) is out and isinstance(norm.forward(torch.ones(2, 4), out, defer="rows"), RowsToNorm)
 
 
 @pytest.mark.parametrize("side", ("left", "right"))
