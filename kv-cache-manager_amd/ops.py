@@ -427,9 +427,9 @@ class PendingAttention(PendingProduct):
         _need(weight.numel() == H and weight.is_contiguous(), "norm weight must have H entries")
         _need(xg.dtype == torch.bfloat16 and xg.is_contiguous() and xg.shape[0] >= M and xg.shape[1] == H, "xg must be bfloat16 [>= M, H]")
         _need(ss.dtype == torch.float32 and ss.is_contiguous() and ss.shape[0] >= M and ss.shape[1] == H // 8, "ss must be float32 [>= M, H / 8]")
+        _need(kc.dtype == vc.dtype == torch.bfloat16, "decode_front needs bfloat16 caches")
+        _check_caches(kc, vc, nkv, hd, packed_offsets=True)
         B = kc.shape[2]
-        _need(kc.dtype == vc.dtype == torch.bfloat16 and kc.is_contiguous() and vc.is_contiguous() and tuple(kc.shape[1:]) == (nkv, B, hd)
-              and tuple(vc.shape[1:]) == (nkv, hd, B), "caches must be bfloat16 [pages, nkv, block_size, hd] and [pages, nkv, hd, block_size]")
         for t, n in ((self.slots, "slots"), (self.row_seq, "row_seq"), (self.ctx_lens, "ctx_lens")):
             _i32(t, n, M)
         _i32(self.tables, "tables", self.table_stride)
