@@ -206,9 +206,12 @@ def as_tensor(value):
 def said_with(part, name, method):
     """Does what ``part`` says by ``name`` hold for the ``method`` it runs: is it said by the class that defines the method, or by one derived
     from it?  A part that replaces a method of its base's has not said what the base says about its own, and runs the ordinary way."""
-    places = [vars(part)] + [vars(c) for c in type(part).__mro__]
-    first = [next((i for i, place in enumerate(places) if n in place), len(places)) for n in (name, method)]
-    return first[0] < len(places) and first[0] <= first[1]
+    for place in (vars(part), *map(vars, type(part).__mro__)):
+        if name in place:
+            return True
+        if method in place:
+            return False
+    return False
 
 
 class Part:
