@@ -28,7 +28,7 @@ from .runner import StepContext
 
 # Decode-shaped steps of more rows replay their program without a graph, and with the library's
 # products where those are the faster, which a graph may not hold.  The line was drawn where graphs had a kernel that read the
-# weights once per 128 rows; at TinyLlama sizes, graph / program: 96 rows 1.55 / 1.56 ms, 128 rows 1.58 / 1.60, 192 rows 1.81 /
+# weights once per 128 rows; at TinyLlama sizes and contexts around 100, graph / program: 96 rows 1.55 / 1.56 ms, 128 rows 1.58 / 1.60, 192 rows 1.81 /
 # 1.84, 256 rows 2.01 / 2.07 (a capture takes some 8 ms per batch bucket and context class).
 GRAPH_ROWS = 128
 
