@@ -395,13 +395,12 @@ class PendingAttention(PendingProduct):
     the operands; ``run`` the ordinary way: ``attend()`` leaves the attention's rows in ``x``, then the output product.
     h: the normed rows or NormedRows; handover: (a function that gives the launch its two buffers) see ``decode_front_buffers``."""
 
-    polls = -1      # looks at what is not there before a workgroup of the launch makes it itself (-1: as measured)
-
     def __init__(self, attend, h, wqkv, x, w, out, scratch, cache, tables, table_stride, row_seq, ctx_lens, slots, cos_sin, heads, scale, parts, handover):
         super().__init__(x, w, out, scratch)
         self.attend, self.h, self.wqkv, self.cache, self.tables, self.table_stride = attend, h, wqkv, cache, tables, table_stride
         self.row_seq, self.ctx_lens, self.slots, self.cos_sin, self.heads, self.scale = row_seq, ctx_lens, slots, cos_sin, heads, scale
         self.parts, self.handover = parts, handover
+        self.polls = -1      # looks at what is not there before a workgroup of the launch makes it itself (-1: as measured)
 
     def run(self, keep_partial=False):
         self.attend()

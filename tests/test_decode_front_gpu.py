@@ -45,7 +45,7 @@ def _layers(ops, H, nh, nkv, hd, B, lens, layers, seed, rotate=True, stored=None
     normed = torch.empty(M, H, dtype=bf, device=DEV)
     ops.rmsnorm(x0, g[0], normed, 1e-5)
 
-    def run(one_launch):
+    def run(one_launch, polls=-1):
         x = x0.clone()
         kc, vc = _t(P["Kc"], bf), _vt(P["Vc"], bf)
         pairs = [(torch.zeros(8, H, dtype=bf, device=DEV), torch.zeros(8, H // 8, device=DEV)) for _ in range(2)]
@@ -65,6 +65,7 @@ def _layers(ops, H, nh, nkv, hd, B, lens, layers, seed, rotate=True, stored=None
 
             product = ops.PendingAttention(attend, h, wqkv[i], attn, wo[i], out, None, (kc, vc), tables, P["max_blocks"], row_seq, ctx_t, slots_t, table,
                                            (nh, nkv, hd), 1 / math.sqrt(hd), parts, lambda: ops.decode_front_buffers(step, M, nh, nkv, hd, parts))
+            product.polls = polls
             if not one_launch:
                 attend()
                 product = ops.PendingProduct(attn, wo[i], out)

@@ -19,15 +19,14 @@ pytestmark = pytest.mark.gpu
     (256, 7, 1, 128, 32, [1, 640, 33]),
     (512, 8, 1, 128, 16, [1100, 20]),                                # the most query heads of 128: every wave rotates q, the last two k and v too
 ])
-def test_made_by_who_waits(ops, monkeypatch, H, nh, nkv, hd, B, lens):
+def test_made_by_who_waits(ops, H, nh, nkv, hd, B, lens):
     """No wait at all: attention workgroups that come before q make it, output tiles make everything.  Every bit of the stream, of what the norm
     leaves and of the pages is as without."""
     run, _, _ = _layers(ops, H, nh, nkv, hd, B, lens, 3, seed=H + hd + len(lens), scaled_first=len(lens) % 2 == 0)
     want = run(True)
     assert all(np.isfinite(a).all() for a in want)
     for polls in (0, 1):
-        monkeypatch.setattr(ops.PendingAttention, "polls", polls)
-        assert all(np.array_equal(a, b) for a, b in zip(run(True), want)), polls
+        assert all(np.array_equal(a, b) for a, b in zip(run(True, polls), want)), polls
 
 
 def test_two_streams_at_once(ops):
