@@ -2,21 +2,21 @@
 // 32-bit), left as partial sums of S slices of K ([S][M][N], the consumer adds them in slice order), or, SWIGLU, made into
 // act[M,I] = silu(X W_gate^T) * (X W_up^T), or with relu in silu's place, of a fused [gate (I rows) | up (I rows)] matrix.
 //
-// A workgroup of 2 to 12 waves owns a tile of BM rows x BN columns and a slice of K, its operands in a ring of stages in LDS
-// (tile_ring.h, which says what bounds such products and why the ring).
+// A workgroup of 2 to 6 waves owns a tile of BM rows x BN columns and a slice of K, its operands in a ring of stages in LDS
+// (tile_ring.h, which says what bounds such products and why the ring); from 96 rows on four waves that read ahead (tile_pipe.h).
 //
 // Measured (us, weights from memory, one launch after the other in a graph; the kernel that shared only X through LDS and streamed
 // W into registers, its own trips double-buffered / this one):
 //   64 rows   2560 x 2048 7.5 / 5.1   2048 x 2048 6.4 / 4.7   gate+up 11264 x 2048 19.6 / 13.2   2048 x 5632 10.9 / 8.0
 //   16 rows   5.1 / 4.2   4.9 / 4.0   13.0 / 11.1   8.1 / 6.6;  128 rows of 4096 x 14336 39.3 / 27.1
-// and against the vendor's product (gate+up: with the launch that applies SwiGLU): 512 rows 35.1 / 32.9 (gate+up), 29.9 / 26.1 (2048 x 5632,
-// with the norm that adds the slices); 1,024 rows 56.7 / 49.9 (gate+up); where the line lies: kvcm_gemm_tiles_preferred, below.
+// and against the vendor's product: kvcm_gemm_tiles_preferred, below.
 #include <cmath>
+#include <utility>
 
 #include "common.h"
 #include "gemm_tiles.h"
 #include "kvcm_hip.h"
-#include "tile_ring.h"
+#include "tile_pipe.h"
 
 namespace kvcm {
 
@@ -180,33 +180,174 @@ __global__ void __launch_bounds__(WM* WN* kWave)
   }
 }
 
+template <int... I, class F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// The same product in large tiles (tile_pipe.h), 32-bit offsets.  GATED: gate and up rows lie sixteen (an odd number of 16-column tiles a wave: eight) of each
+// in turn, as above.
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED>
+__global__ void __launch_bounds__(WM* WN* kWave)
+    gemm_pipe_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, float* __restrict__ partials, void* __restrict__ out,
+                     int out_f32, int M, int N, int K, int ldx, int ldw, int ldo, int S, int tiles_m, int tiles_n, float limit, int act) {
+  using Pipe = TilePipe<BM, BN, WM, WN, STAGES>;
+  constexpr int TM = Pipe::TM, TN = Pipe::TN, R = Pipe::R;
+  constexpr bool kEights = GATED && TN % 2 != 0;
+  constexpr int kBlocks = GATED ? TN / 2 : TN;      // of 16 columns of the result (kEights: not used)
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[Pipe::kBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  int id = neighbours_on_one_xcd(), tm, tn;
+  const int s = id / (tiles_m * tiles_n);
+  id -= s * tiles_m * tiles_n;
+  tile_of<BM>(id, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, c0 = tn * (GATED ? BN / 2 : BN);
+  const int steps_all = K / kStepK;
+  const int k_lo = static_cast<int>(static_cast<long long>(steps_all) * s / S);
+  const int steps = static_cast<int>(static_cast<long long>(steps_all) * (s + 1) / S) - k_lo;
+  const uint64_t xbase = reinterpret_cast<uint64_t>(X + static_cast<size_t>(m0) * ldx) + static_cast<size_t>(k_lo) * 128;
+  const uint64_t wbase = reinterpret_cast<uint64_t>(W + static_cast<size_t>(c0) * ldw) + static_cast<size_t>(k_lo) * 128;
+  const uint64_t upbase = wbase + static_cast<size_t>(GATED ? N : 0) * ldw * 2;
+  constexpr int kHalf = kEights ? 8 : 16;
+  // rows past M and columns past N repeat the last one (what they give is not stored)
+  uint32_t offset[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int req = Pipe::request_of(q, wave), row = req * 8 + lane / 8;
+    int at, ld;
+    if (req < BM / 8) {
+      at = row < M - m0 ? row : M - 1 - m0;
+      ld = ldx;
+    } else {
+      const int r = row - BM, part = r / (TN * 16), block = r / 16 % TN, a = r % 16;
+      if constexpr (kEights) at = r / 16 * 8 + a % 8;
+      else if constexpr (GATED) at = part * (TN * 8) + paired_row(block / 2, a, kBlocks);
+      else at = part * (TN * 16) + paired_row(block, a, kBlocks);
+      if (at > N - 1 - c0) at = N - 1 - c0;
+      ld = ldw;
+    }
+    offset[q] = static_cast<uint32_t>(at) * static_cast<uint32_t>(ld) * 2u + static_cast<uint32_t>(Pipe::piece_of(lane)) * 16u;
+  }
+  // one row block: as above
+  const int phase = tiles_m == 1 ? tn * 5 % steps : 0;
+  auto base = [&](int req) {
+    const bool up = GATED && (req - BM / 8) * 8 % (2 * kHalf) >= kHalf;
+    return req < BM / 8 ? xbase : up ? upbase : wbase;
+  };
+  ring_f32x4 acc[TN][TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) acc[j][i] = ring_f32x4{0.f, 0.f, 0.f, 0.f};
+  Pipe::multiply(ring, offset, base, steps, phase, kStepK, wave, lane, acc, [] {});
+  const int wm = wave % WM, wn = wave / WM, frow = lane % 16, fk = lane / 16;
+  // A row of the result; acc's indexes have to be constants, and what the gated forms compute is too long for the compiler to unroll on
+  // request: hence a function of a constant, and the activation chosen outside.
+  auto store_row = [&](auto i_, auto gated_by) __attribute__((always_inline)) {
+    constexpr int i = decltype(i_)::value;
+    const int m = m0 + (wm * TM + i) * 16 + frow;
+    if (m >= M) return;
+    const size_t row = static_cast<size_t>(m) * ldo;
+    if constexpr (kEights) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {      // (as above)
+        float g[2], u[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[j][i][r]), __float_as_uint(acc[j][i][r + 2]), false, false);
+          g[r] = __uint_as_float(both[0]);
+          u[r] = __uint_as_float(both[1]);
+        }
+        const int c = c0 + (wn * TN + j) * 8 + fk % 2 * 4 + fk / 2 * 2;
+        if (c >= N) continue;
+        if (out_f32) *reinterpret_cast<any_f32x2*>(static_cast<float*>(out) + row + c) = any_f32x2{gated_by(0.f, g[0], u[0]), gated_by(0.f, g[1], u[1])};
+        else *reinterpret_cast<any_u32*>(static_cast<uint16_t*>(out) + row + c) = two_bf16(gated_by(bf16_t{}, g[0], u[0]), gated_by(bf16_t{}, g[1], u[1]));
+      }
+    } else {
+      auto four_of = [&](int b, auto type) {      // four columns of the result
+        if constexpr (GATED) {
+          const ring_f32x4 g = acc[2 * b % TN][i], u = acc[(2 * b + 1) % TN][i];
+          return ring_f32x4{gated_by(type, g[0], u[0]), gated_by(type, g[1], u[1]), gated_by(type, g[2], u[2]), gated_by(type, g[3], u[3])};
+        } else {
+          return acc[b % TN][i];
+        }
+      };
+      if ((!GATED && S > 1) || out_f32) {
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) {
+          const int c = c0 + wn * kBlocks * 16 + paired_row(b, fk * 4, kBlocks);
+          if (c >= N) continue;
+          const ring_f32x4 v = four_of(b, 0.f);
+          float* to = !GATED && S > 1 ? partials + (static_cast<size_t>(s) * M + m) * N + c : static_cast<float*>(out) + row + c;
+          *reinterpret_cast<any_f32x4*>(to) = any_f32x4{v[0], v[1], v[2], v[3]};
+        }
+      } else {
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) {
+          const bool paired = b / 2 * 2 + 1 < kBlocks;
+          if (paired && b % 2 != 0) continue;      // (stored with the block before)
+          const int c = c0 + wn * kBlocks * 16 + paired_row(b, fk * 4, kBlocks);
+          if (c >= N) continue;
+          uint16_t* to = static_cast<uint16_t*>(out) + row + c;
+          const ring_f32x4 v = four_of(b, bf16_t{});
+          const any_u32x2 four{two_bf16(v[0], v[1]), two_bf16(v[2], v[3])};
+          if (paired && c + 4 < N) {
+            const ring_f32x4 next = four_of(b + 1, bf16_t{});
+            *reinterpret_cast<any_u32x4*>(to) = any_u32x4{four[0], four[1], two_bf16(next[0], next[1]), two_bf16(next[2], next[3])};
+          } else {
+            *reinterpret_cast<any_u32x2*>(to) = four;
+          }
+        }
+      }
+    }
+  };
+  auto store = [&](auto gated_by) __attribute__((always_inline)) {
+    each_of(std::make_integer_sequence<int, TM>{}, [&](auto i) __attribute__((always_inline)) { store_row(i, gated_by); });
+  };
+  if constexpr (!GATED) {
+    store([](auto, float g, float) { return g; });
+  } else if (limit > 0.f) {
+    store([&](auto type, float g, float u) { return act == kSiluStored ? clamped_gate<decltype(type)>(g, u, limit) : clamped_gate<float>(g, u, limit); });
+  } else if (act == kRelu) {
+    store([](auto, float g, float u) { return fmaxf(g, 0.f) * u; });
+  } else if (act == kSilu) {
+    store([](auto, float g, float u) { return silu<float>(g) * u; });
+  } else {
+    store([](auto type, float g, float u) { return gated<decltype(type)>(g, u, 0.f, kSiluStored); });
+  }
+}
+
 // The tiles, and what a launch of them takes: us at the beginning and end, us a step of a workgroup that is alone on its CU, the factor on
 // (workgroups a CU) x (a step) beyond that, us of each further round.  Fitted to some 5,000 timed launches (8 to 2,048 rows, the
-// projections of models of widths 2,048 and 4,096, S = 1 to 8; the fit is off by 4 to 10 % a launch).
+// projections of models of widths 2,048 and 4,096, S = 1 to 8; the fit is off by 4 to 10 % a launch), the tiles of tile_pipe.h, from 96
+// rows on, to 7,500 further ones (96 to 4,096 rows, 64 to 16,384 columns, K 256 to 14,336, S = 1, 2, 4; off by 8 to 15 % a launch; what the rule picks
+// is 1.0 % slower than the best tile on average, 29 % at worst: 96 x 4096 x 14336 in two slices).  Below that the ring of tile_ring.h is the faster: 64 x 64
+// of 64 rows of 2048 x 2048 in eight slices 5.2 us, 5.7 with fragments read ahead.
+// (columns, after the sizes and waves: the stages, and whether the tile is tile_pipe.h's)
 struct Tile {
   int bm, bn;
   float fixed, step, share, round;
 };
 #define KVCM_TILES(T)                                                                                                             \
-  T(16, 32, 1, 2, 8, 1.305f, 0.144f, 0.725f, 0.000f)                                                                              \
-  T(16, 48, 1, 3, 8, 1.278f, 0.167f, 0.771f, 0.466f)                                                                              \
-  T(16, 64, 1, 4, 8, 1.126f, 0.199f, 0.886f, 0.256f)                                                                              \
-  T(32, 32, 2, 2, 8, 1.517f, 0.163f, 0.801f, 0.197f)                                                                              \
-  T(32, 64, 2, 2, 6, 1.484f, 0.219f, 0.891f, 0.210f)                                                                              \
-  T(64, 32, 2, 2, 6, 1.770f, 0.196f, 0.899f, 0.000f)                                                                              \
-  T(64, 48, 4, 1, 8, 2.019f, 0.236f, 0.975f, 1.170f)                                                                              \
-  T(64, 64, 2, 2, 4, 1.822f, 0.274f, 0.869f, 0.435f)                                                                              \
-  T(64, 96, 2, 3, 6, 2.462f, 0.351f, 0.957f, 1.524f)                                                                              \
-  T(96, 64, 3, 2, 4, 2.841f, 0.324f, 0.916f, 0.487f)                                                                              \
-  T(128, 64, 4, 2, 6, 2.780f, 0.356f, 1.066f, 1.100f)                                                                             \
-  T(128, 96, 4, 3, 5, 3.397f, 0.465f, 0.998f, 1.810f)                                                                             \
-  T(128, 128, 2, 4, 4, 3.913f, 0.513f, 1.039f, 2.154f)                                                                            \
-  T(128, 192, 2, 3, 4, 5.339f, 0.744f, 1.028f, 1.230f)                                                                            \
-  T(256, 128, 4, 2, 3, 5.952f, 0.775f, 1.048f, 3.450f)                                                                            \
-  T(256, 192, 4, 3, 2, 6.470f, 1.155f, 1.028f, 0.000f)                                                                            \
-  T(256, 256, 2, 4, 2, 8.000f, 1.347f, 1.034f, 4.651f)
+  T(16, 32, 1, 2, 8, false, 1.305f, 0.144f, 0.725f, 0.000f)                                                                       \
+  T(16, 48, 1, 3, 8, false, 1.278f, 0.167f, 0.771f, 0.466f)                                                                       \
+  T(16, 64, 1, 4, 8, false, 1.126f, 0.199f, 0.886f, 0.256f)                                                                       \
+  T(32, 32, 2, 2, 8, false, 1.517f, 0.163f, 0.801f, 0.197f)                                                                       \
+  T(32, 64, 2, 2, 6, false, 1.484f, 0.219f, 0.891f, 0.210f)                                                                       \
+  T(64, 48, 4, 1, 8, false, 2.019f, 0.236f, 0.975f, 1.170f)                                                                       \
+  T(64, 64, 2, 2, 4, false, 1.822f, 0.274f, 0.869f, 0.435f)                                                                       \
+  T(64, 96, 2, 3, 6, false, 2.462f, 0.351f, 0.957f, 1.524f)                                                                       \
+  T(96, 64, 2, 2, 4, true, 3.147f, 0.242f, 1.040f, 0.523f)                                                                        \
+  T(96, 96, 2, 2, 4, true, 3.426f, 0.308f, 1.007f, 3.111f)                                                                        \
+  T(96, 128, 2, 2, 4, true, 3.607f, 0.349f, 1.084f, 3.262f)                                                                       \
+  T(128, 128, 2, 2, 4, true, 4.093f, 0.430f, 1.025f, 3.974f)                                                                      \
+  T(192, 128, 2, 2, 3, true, 5.115f, 0.537f, 1.001f, 4.856f)                                                                      \
+  T(192, 192, 2, 2, 3, true, 6.493f, 0.662f, 1.037f, 6.782f)                                                                      \
+  T(256, 128, 2, 2, 3, true, 6.230f, 0.612f, 1.059f, 6.453f)                                                                      \
+  T(256, 192, 2, 2, 2, true, 6.172f, 0.944f, 1.065f, 7.188f)                                                                      \
+  T(256, 256, 2, 2, 2, true, 8.118f, 1.175f, 1.013f, 8.000f)
 
-#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, FIXED, STEP, SHARE, ROUND) {BM, BN, FIXED, STEP, SHARE, ROUND},
+#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, FIXED, STEP, SHARE, ROUND},
 static constexpr Tile kTiles[] = {KVCM_TILES(KVCM_TILE_ROW)};
 #undef KVCM_TILE_ROW
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
@@ -254,6 +395,17 @@ float gemm_tiles_time(int M, int N, int K, int S, bool is_gated, bool out_f32) {
   return t + stored_time(M, N, S, out_f32);
 }
 
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED>
+static int launch_pipe(const TilesCall& c, hipStream_t st) {
+  const int tiles_m = (c.M + BM - 1) / BM, tiles_n = ((GATED ? 2 * c.N : c.N) + BN - 1) / BN;
+  const long long grid = static_cast<long long>(tiles_m) * tiles_n * c.S;
+  KVCM_REQUIRE(grid < (1ll << 31), "gemm_tiles: too many tiles");
+  KVCM_REQUIRE(c.ss_in == nullptr, "gemm_tiles: large tiles take no folded norm");
+  gemm_pipe_kernel<BM, BN, WM, WN, STAGES, GATED><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, st>>>(
+      c.X, c.W, c.partials, c.out, c.out_f32, c.M, c.N, c.K, c.ldx, c.ldw, c.ldo, c.S, tiles_m, tiles_n, c.limit, c.act);
+  return launch_status("gemm_tiles");
+}
+
 template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, class Offset = uint32_t>
 static int launch_tiles(const TilesCall& c, hipStream_t st) {
   const int tiles_m = (c.M + BM - 1) / BM, tiles_n = ((GATED ? 2 * c.N : c.N) + BN - 1) / BN;
@@ -265,6 +417,12 @@ static int launch_tiles(const TilesCall& c, hipStream_t st) {
   return launch_status("gemm_tiles");
 }
 
+template <int BM, int BN, int WM, int WN, int STAGES, bool PIPE, bool GATED>
+static int launch(const TilesCall& c, hipStream_t st) {
+  if constexpr (PIPE) return launch_pipe<BM, BN, WM, WN, STAGES, GATED>(c, st);
+  else return launch_tiles<BM, BN, WM, WN, STAGES, GATED>(c, st);
+}
+
 int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st) {
   KVCM_REQUIRE(c.M > 0 && c.N > 0 && c.N % 4 == 0 && c.K > 0 && c.K % kStepK == 0 && c.S >= 1 && c.S <= c.K / kStepK,
                "gemm_tiles: unsupported shape M=%d N=%d K=%d in %d slices", c.M, c.N, c.K, c.S);
@@ -274,8 +432,8 @@ int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st) {
     return is_gated ? launch_tiles<64, 64, 2, 2, 4, true, uint64_t>(c, st) : launch_tiles<64, 64, 2, 2, 4, false, uint64_t>(c, st);
   if (tile < 0) tile = best_tile(c.M, is_gated ? 2 * c.N : c.N, c.K, c.S);
   int i = 0;
-#define KVCM_TILE_LAUNCH(BM, BN, WM, WN, STAGES, FIXED, STEP, SHARE, ROUND)                                                        \
-  if (tile == i++) return is_gated ? launch_tiles<BM, BN, WM, WN, STAGES, true>(c, st) : launch_tiles<BM, BN, WM, WN, STAGES, false>(c, st);
+#define KVCM_TILE_LAUNCH(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) \
+  if (tile == i++) return is_gated ? launch<BM, BN, WM, WN, STAGES, PIPE, true>(c, st) : launch<BM, BN, WM, WN, STAGES, PIPE, false>(c, st);
   KVCM_TILES(KVCM_TILE_LAUNCH)
 #undef KVCM_TILE_LAUNCH
   KVCM_REQUIRE(false, "gemm_tiles: no tile %d", tile);
@@ -315,34 +473,36 @@ int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, in
 }
 
 // Is a product of many rows, in S slices of K that its consumer adds, faster here than by the vendor library (is_gated: than that and
-// the launch that applies the activation)?  Beyond 2,048 rows the library's own tiles of 256 x 256 are (32,768 rows: 1,306 / 1,269 us gate+up
-// of 5632 x 2048, 659 / 513 us 2048 x 5632).  Up to there the tiles' time against about what the library takes.  Here: the launch as the tile was
-// picked, with what that model leaves out, the rows of X that every column of tiles reads again (10 TB/s), and the slices' reading (4.5 TB/s,
-// and 55 KB a us of one row's through the CU that norms it).  There: 8.3 us, or 1.6 us, 0.21 us for 64 k of a chain and 1,520 TFLOP/s, or, where
-// few results let it cut K, 8.3 us and 0.029 us for 64 k of 131,072 results; and 4 us and 6 bytes a result for the second launch.
-// Up to 256 rows the library is often far above that, so that it has to be 1.3 times as fast.
-// The constants were fitted to 2,177 plain products (64 to 32,000 columns, K 256 to 14,336; 1,032 of them with the norm that adds the slices
-// too) and 1,937 gated ones (64 to 14,336 columns), 96 to 2,048 rows.  What the rule picks takes 0.80, 0.75 and 0.73 of the library's time on average and
-// is 1.9, 1.0 and 0.7 % slower than the better of the two; slower than the library by more than 8 % are 17, 11 and 37 of them, the worst where
-// few columns of long K are cut by it and not here: 256 x 1024 x 4096 13.4 / 10.1 us, gated 2048 x 128 x 4096 21.9 / 16.3.  At 3,142 further ones, of
-// row counts between those: 0.83 and 0.76, 2.7 and 1.3 %, 14 and 19.  (us, here / library:
-// 512 x 2048 x 5632 with the norm 26.1 / 29.9, 1024 x 1024 x 512 5.0 / 8.9; 1,024 rows gate+up of 5632 x 2048 49.9 / 56.7; not taken: 640 x 64 x 14336 29.5 / 13.3, 2048 x 256 x 5632 28.9 / 17.4,
-// 1024 x 8192 x 2048 36.9 / 34.3.)
+// the launch that applies the activation)?  Beyond 2,048 rows a plain product is the library's, whose tiles of 256 x 256 are 5 to 15 %
+// faster once every CU has several (32,768 rows: 2048 x 5632 565 / 505 us, 2560 x 2048 266 / 240), a gated one is not: it saves the second launch and
+// the product's trip to memory (32,768 rows of gate and up, 5632 x 2048: 1,118 / 1,276 us; 8,192 rows 309 / 394; 9,608 rows, 14336 x 4096 1,696 / 1,783).  Up to there the
+// tiles' time against about what the library takes.  Here: the launch as the tile was
+// picked, with what that model leaves out, the rows of X that every column of tiles reads again (7 TB/s), and the slices' reading (4.5 TB/s,
+// and 55 KB a us of one row's through the CU that norms it).  There: 5.5 us, or 1.8 us, 0.26 us for 64 k of a chain and 1,300 to 1,700 TFLOP/s (the more the
+// more results there are) and 1.15 us a million results, or, where
+// few results let it cut K, 6.7 us and 0.043 us for 64 k of 131,072 results, and the same a result; and 7.2 us and 6 bytes a result for the second launch.
+// Up to 256 rows the library is often far above that, so that it has to be 1.45 times as fast.
+// The constants were fitted to 230 plain products (64 to 16,384 columns, K 256 to 14,336, 96 to 2,048 rows) and 257 gated ones (64 to 14,336
+// columns, 96 to 33,000 rows).  What the rule picks takes 0.87 and 0.79 of the library's time on average and
+// is 2.0 and 1.0 % slower than the better of the two; slower than the library by more than 8 % are 9 and 4 of them: 1040 x 8192 x 2048 43.9 / 35.4,
+// 384 x 2048 x 5632 32.8 / 26.0.  (us, here / library: 2048 x 2560 x 2048 22.8 / 25.2, 2048 x 2048 x 5632 51.8 / 54.0, 1040 x 2048 x 2048 13.6 / 20.0; 2,048 and 1,024 rows gate+up of
+// 5632 x 2048 88.9 / 92.7 and 45.3 / 55.2; not taken: 640 x 64 x 14336 33 / 13.3, 2048 x 256 x 5632 22 / 17.4, 2048 x 8192 x 2048 53 / 49.7.)
 int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype) {
   if (M <= 0 || N <= 0 || N % 64 != 0 || K <= 0 || K % kStepK != 0 || S < 1 || S > K / kStepK || (is_gated && S > 1)) return 0;
-  if (M > 2048) return 0;
+  if (M > 2048 && !is_gated) return 0;
   const float m = static_cast<float>(M), n = static_cast<float>(N), k = static_cast<float>(K), steps = static_cast<float>(K / kStepK);
   const int wrows = is_gated ? 2 * N : N;
   float t = 0.f;
   const Tile& tile = kTiles[best_tile(M, wrows, K, S, &t)];
-  const float again = 2.3f + m * k * 2e-7f * static_cast<float>((wrows + tile.bn - 1) / tile.bn);
+  const float again = 2.3f + m * k * 2.81e-7f * static_cast<float>((wrows + tile.bn - 1) / tile.bn);
   const float t2 = t * t, again2 = again * again;
   const float here = std::sqrt(std::sqrt(t2 * t2 + again2 * again2)) + stored_time(M, N, S, out_dtype == kF32) +
                      (S > 1 ? m * n * (4.f * S - 2.f) / 4.5e6f + n * 4.f * S / 55e3f : 0.f);
-  const float results = m * static_cast<float>(wrows);
-  const float whole = 1.6f + 0.21f * steps + results * k * 2e-9f / 1.52f, cut = 8.3f + 0.029f * steps * results / 131072.f;
-  const float library = std::fmax(8.3f, std::fmin(whole, cut)) + (is_gated ? 4.f + m * n * 6.f / 5e6f : 0.f);
-  return here <= (M <= 256 ? 1.3f : 1.f) * library;
+  const float results = m * static_cast<float>(wrows), rounds = results / (256.f * 256.f * 256.f);
+  const float rate = 1.304f + 0.412f * rounds / (rounds + 17.6f), stored = results * 1.15e-6f;      // (PFLOP/s; us)
+  const float whole = 1.8f + 0.26f * steps + results * k * 2e-9f / rate, cut = 6.7f + 0.043f * steps * results / 131072.f;
+  const float library = std::fmax(5.51f, std::fmin(whole, cut) + stored) + (is_gated ? 7.18f + m * n * 6.f / 7.93e6f : 0.f);
+  return here <= (M <= 256 ? 1.45f : 1.f) * library;
 }
 
 }  // extern "C"

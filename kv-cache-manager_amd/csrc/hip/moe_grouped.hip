@@ -24,7 +24,7 @@
 #include "common.h"
 #include "gemm_tiles.h"
 #include "kvcm_hip.h"
-#include "tile_ring.h"
+#include "tile_pipe.h"
 
 namespace kvcm {
 
@@ -76,12 +76,12 @@ enum : int { kDown = 0, kUp = 1, kUpGated = 2, kUpGelu = 3 };
 
 // N: rows of an expert's matrix (2F for the gated form); the output has N columns (F for the gated form).  Offset: of an operand's
 // pieces from its beginning, in bytes; uint64_t for rows that lie beyond 4 GB or far apart.
-template <int BM, int BN, int WM, int WN, int STAGES, int MODE, class Offset>
+template <int BM, int BN, int WM, int WN, int STAGES, bool PIPE, int MODE, class Offset>
 __global__ void __launch_bounds__(WM* WN* kWave)
     moe_grouped_kernel(const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ W, const int* __restrict__ order,
                        const int* __restrict__ count, const int4* __restrict__ list, int top, void* __restrict__ out,
                        const float* __restrict__ weight, int N, int K, int col_blocks) {
-  using Ring = TileRing<BM, BN, WM, WN, STAGES>;
+  using Ring = std::conditional_t<PIPE, TilePipe<BM, BN, WM, WN, STAGES>, TileRing<BM, BN, WM, WN, STAGES>>;
   constexpr int TM = Ring::TM, TN = Ring::TN, R = Ring::R;
   static_assert(MODE != kUpGated || TN % 2 == 0, "gate and up accumulators in one wave");
   __shared__ __attribute__((aligned(1024))) unsigned char ring[Ring::kBytes];
@@ -186,18 +186,18 @@ __global__ void __launch_bounds__(256)
 
 // Tiles: those of gemm_tiles.hip of an even number of accumulators a wave, with the same constants of a launch's time.
 #define KVCM_GROUPED_TILES(T)      \
-  T(64, 64, 2, 2, 4)               \
-  T(128, 64, 4, 2, 6)              \
-  T(128, 128, 2, 4, 4)             \
-  T(128, 192, 2, 3, 4)             \
-  T(256, 128, 4, 2, 3)             \
-  T(256, 192, 4, 3, 2)             \
-  T(256, 256, 2, 4, 2)
+  T(64, 64, 2, 2, 4, false)        \
+  T(96, 64, 2, 2, 4, true)         \
+  T(128, 128, 2, 2, 4, true)       \
+  T(192, 128, 2, 2, 3, true)       \
+  T(256, 128, 2, 2, 3, true)       \
+  T(256, 192, 2, 2, 2, true)       \
+  T(256, 256, 2, 2, 2, true)
 
 struct High {
   int bm, bn;
 };
-#define KVCM_HIGH(BM, BN, WM, WN, STAGES) {BM, BN},
+#define KVCM_HIGH(BM, BN, WM, WN, STAGES, PIPE) {BM, BN},
 static constexpr High kHighs[] = {KVCM_GROUPED_TILES(KVCM_HIGH)};
 #undef KVCM_HIGH
 constexpr int kHighCount = sizeof(kHighs) / sizeof(kHighs[0]);
@@ -238,17 +238,17 @@ static int launch_grouped(int tile, const GroupedCall& c, hipStream_t s) {
   const int col_blocks = (c.N + kHighs[tile].bn - 1) / kHighs[tile].bn;
   const long long grid = (static_cast<long long>(c.n / kHighs[tile].bm + c.E) * col_blocks + 7) / 8 * 8;
   KVCM_REQUIRE(grid < (1ll << 31), "moe_grouped: too many tiles");
-#define KVCM_GROUPED(BM, BN, WM, WN, STAGES, OFFSET)                                                                                   \
-  moe_grouped_kernel<BM, BN, WM, WN, STAGES, MODE, OFFSET><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, s>>>(                    \
+#define KVCM_GROUPED(BM, BN, WM, WN, STAGES, PIPE, OFFSET)                                                                                   \
+  moe_grouped_kernel<BM, BN, WM, WN, STAGES, PIPE, MODE, OFFSET><<<static_cast<unsigned>(grid), WM * WN * kWave, 0, s>>>(                    \
       static_cast<const uint16_t*>(c.A), c.lda, static_cast<const uint16_t*>(c.W), c.order, c.count, c.list, c.top, c.out, c.weight,   \
       c.N, c.K, col_blocks)
   if (c.far) {
-    KVCM_GROUPED(128, 128, 2, 4, 4, uint64_t);
+    KVCM_GROUPED(128, 128, 2, 4, 4, false, uint64_t);
     return launch_status("moe_grouped");
   }
   int i = 0;
-#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES) \
-  if (tile == i++) KVCM_GROUPED(BM, BN, WM, WN, STAGES, uint32_t);
+#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES, PIPE) \
+  if (tile == i++) KVCM_GROUPED(BM, BN, WM, WN, STAGES, PIPE, uint32_t);
   KVCM_GROUPED_TILES(KVCM_GROUPED_LAUNCH)
 #undef KVCM_GROUPED_LAUNCH
 #undef KVCM_GROUPED

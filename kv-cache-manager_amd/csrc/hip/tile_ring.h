@@ -32,6 +32,7 @@ constexpr int kStepK = 64;      // k of a stage: 128 bytes a row
 typedef float any_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float any_f32x2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t any_u32x2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t any_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t any_u32 __attribute__((aligned(2)));
 
 __device__ __forceinline__ uint32_t two_bf16(float a, float b) { return uint32_t(float_to_bf16_bits(a)) | uint32_t(float_to_bf16_bits(b)) << 16; }

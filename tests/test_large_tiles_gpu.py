@@ -1,0 +1,42 @@
+"""Large tiles (csrc/hip/tile_pipe.h): several groups of row blocks, columns that end inside a lane's eight, and the rule beyond 2,048 rows."""
+import pytest
+import torch
+
+import test_products_in_tiles_gpu as tiles
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ops = tiles.ops
+
+
+@pytest.mark.parametrize("tile", range(8, 17))
+def test_groups_of_row_blocks(ops, tile):
+    """more row blocks than a group of neighbours has (four or eight), the last group not whole; slices and gate and up too"""
+    bm, bn = tiles._tiles(ops)[tile]
+    M, N, K = 9 * bm + 5, 2 * bn + 20, 320
+    x, w = tiles._operands(tile, M, N, K)
+    for dtype in (torch.float32, torch.bfloat16):
+        out = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+        tiles._run(ops, x, w, None, out, tile=tile)
+        tiles._close(out, x, w, dtype == torch.bfloat16)
+    parts = torch.full((2, M, N), float("nan"), device=DEV)
+    tiles._run(ops, x, w, parts, out, S=2, tile=tile)
+    tiles._close(parts.double().sum(0), x, w, False)
+    I = bn + 8
+    x, w = tiles._operands(tile + 50, M, 2 * I, K)
+    act, gu, want = (torch.full((M, n), float("nan"), dtype=torch.bfloat16, device=DEV) for n in (I, 2 * I, I))
+    tiles._run(ops, x, w, None, act, gated=1, act=0, tile=tile, N=I)
+    tiles._run(ops, x, w, None, gu, tile=tile)
+    ops.swiglu(gu, want)
+    # the same roundings of sums that both tiles add in the same order
+    assert torch.equal(act, want)
+
+
+@pytest.mark.parametrize("M,I,K,fused", [(2049, 5632, 2048, True), (9608, 1408, 512, True)])
+def test_gated_products_of_many_rows(ops, M, I, K, fused):
+    x, w = tiles._operands(M, M, 2 * I, K)
+    act = torch.empty(M, I, dtype=torch.bfloat16, device=DEV)
+    assert ops.gemm_swiglu(x, w, act) == fused and not ops._tiles_take(M, 2048, K, 1)
+    g, u = (x.double() @ w.double().t()).split(I, 1)
+    # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each
+    assert bool(((act.double() - g * torch.sigmoid(g) * u).abs() <= 4.2 * 2.0 ** -8 * g.abs() * u.abs() + 1e-4).all())
