@@ -299,6 +299,12 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
                     float* n_new, float* o, int ldo, float* s_state, float* n_state, float* m_state, const int* run_start,
                     const int* seq_start, const int* state_slots, int S, int heads, int dk, int dv, int T, int max_run, int one_order,
                     hipStream_t s);
+// (mlstm_chunks.hip) the same in matrix form, for long runs
+long long kvcm_mlstm_carry_floats(int rows, int S, int heads, int dk, int dv, int piece);
+int kvcm_mlstm_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* ig, int ldi, const float* fg,
+                      int ldf, const float* i_bias, const float* f_bias, float cap, float q_scale, float* coef, float* o, int ldo, float* s_state,
+                      float* n_state, float* m_state, const int* run_start, const int* seq_start, const int* state_slots, int S, int heads,
+                      int dk, int dv, int T, int max_run, int piece, float* carry, long long carry_floats, hipStream_t s);
 // (moe.hip) a routed feed-forward: the choice of experts, and the experts' two products a row at a time
 int kvcm_moe_route(const float* logits, int ld, int splits, long long split_stride, int E, int top, int mode, float factor, int* chosen,
                    float* weight, int T, hipStream_t s);

@@ -20,6 +20,7 @@
 // state that another one of the same launch writes.
 #include "common.h"
 #include "kvcm_hip.h"
+#include "mlstm.h"
 
 namespace kvcm {
 
@@ -112,6 +113,81 @@ __global__ void __launch_bounds__(kWave)
     if (in) coef[size_t(t0 + lane) * heads + head] = float4{expf(lf + before - after), expf(li - after), expf(-after), 0.f};
   }
   if (lane == 0) *mst = m;
+}
+
+// The same for long runs, whose scan is a chain of tiles of 64 rows (0.85 us each): kMaxWaves waves take a stretch of the run each, put its steps
+// together first (m -> max(m + a, b), as the scan's), and scan it from the maximum that enters it.  2,048 rows of 32 heads: 27 us with one
+// wave, 9 us so.
+constexpr int kMaxWaves = 8;
+__global__ void __launch_bounds__(kMaxWaves* kWave)
+    mlstm_max_stretches_kernel(float4* __restrict__ coef, float* __restrict__ m_state, const int* __restrict__ run_start,
+                               const int* __restrict__ seq_start, const int* __restrict__ state_slots, int heads) {
+  __shared__ float whole_a[kMaxWaves], whole_b[kMaxWaves];
+  const int s = blockIdx.x / heads, head = blockIdx.x % heads, lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int r0 = run_start[s], r1 = run_start[s + 1];
+  const int slot = state_slots[s];
+  if (r1 <= r0) return;
+  if (slot < 0) {
+    for (int row = r0 + static_cast<int>(threadIdx.x); row < r1; row += kMaxWaves * kWave) coef[size_t(row) * heads + head] = float4{0.f, 0.f, 0.f, 0.f};
+    return;
+  }
+  float* mst = m_state + size_t(slot) * heads + head;
+  float m = seq_start[s] == 0 ? 0.f : *mst;
+  const int tiles = (r1 - r0 + kWave - 1) / kWave, per = (tiles + kMaxWaves - 1) / kMaxWaves;
+  const int first = wave * per, last = first + per < tiles ? first + per : tiles;
+  auto request = [&](int tile) {
+    const int row = r0 + tile * kWave + lane;
+    return coef[size_t(row < r1 ? row : r1 - 1) * heads + head];
+  };
+  // a, b: the steps up to this lane's token together (beyond the run: m stays)
+  auto scanned = [&](int tile, const float4& c, float& a, float& b) {
+    const bool in = r0 + tile * kWave + lane < r1;
+    b = in ? c.x : -INFINITY;
+    a = in ? c.y : 0.f;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const float pa = __shfl_up(a, d, kWave), pb = __shfl_up(b, d, kWave);
+      if (lane >= d) {
+        b = fmaxf(pb + a, b);
+        a += pa;
+      }
+    }
+  };
+  float all_a = 0.f, all_b = -INFINITY;
+  if (first < last && wave + 1 < kMaxWaves) {
+    float4 next = request(first);
+    for (int t = first; t < last; ++t) {
+      const float4 c = next;
+      if (t + 1 < last) next = request(t + 1);
+      float a, b;
+      scanned(t, c, a, b);
+      a = lane_of(a, kWave - 1);
+      b = lane_of(b, kWave - 1);
+      all_b = fmaxf(all_b + a, b);
+      all_a += a;
+    }
+  }
+  if (lane == 0) {
+    whole_a[wave] = all_a;
+    whole_b[wave] = all_b;
+  }
+  __syncthreads();      // (everybody has read the slot's m)
+  for (int w = 0; w < wave; ++w) m = fmaxf(m + whole_a[w], whole_b[w]);
+  if (first >= last) return;
+  float4 next = request(first);
+  for (int t = first; t < last; ++t) {
+    const float4 c = next;
+    if (t + 1 < last) next = request(t + 1);
+    const int row = r0 + t * kWave + lane;
+    float a, b;
+    scanned(t, c, a, b);
+    const float after = fmaxf(m + a, b);
+    float before = __shfl_up(after, 1, kWave);
+    before = lane == 0 ? m : before;
+    m = __shfl(after, kWave - 1, kWave);
+    if (row < r1) coef[size_t(row) * heads + head] = float4{expf(c.y + before - after), expf(c.x - after), expf(-after), 0.f};
+  }
+  if (last == tiles && lane == 0) *mst = m;
 }
 
 // A wave owns 64 / G * NC value columns of one head of one sequence (NC a lane); U tokens' vectors are in registers or on their way.  Runs of a
@@ -259,6 +335,22 @@ __global__ void __launch_bounds__(256)
   n_state[size_t(slot) * per_seq + idx % per_seq] = n_new[idx];
 }
 
+void mlstm_factors(const float* ig, int ldi, const float* fg, int ldf, const float* i_bias, const float* f_bias, float cap, float4* coef,
+                   float* m_state, const int* run_start, const int* seq_start, const int* state_slots, int S, int heads, int T, int max_run,
+                   int one_order, hipStream_t s) {
+  const int logs_first = max_run >= 16 ? 1 : 0;      // long runs: the gates' logarithms of all T rows first, in parallel
+  if (logs_first) {
+    const long long n = static_cast<long long>(T) * heads;
+    mlstm_gate_logs_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, coef, n, heads);
+    if (!one_order && max_run > 2 * kWave) {
+      mlstm_max_stretches_kernel<<<S * heads, kMaxWaves * kWave, 0, s>>>(coef, m_state, run_start, seq_start, state_slots, heads);
+      return;
+    }
+  }
+  auto* maxima = one_order ? mlstm_max_kernel<true> : mlstm_max_kernel<false>;
+  maxima<<<S * heads, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, coef, m_state, run_start, seq_start, state_slots, heads, logs_first);
+}
+
 }  // namespace kvcm
 
 using namespace kvcm;
@@ -284,15 +376,8 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
                "mlstm_scan: row strides too small");
   KVCM_REQUIRE(coef && n_new && reinterpret_cast<uintptr_t>(coef) % 16 == 0, "mlstm_scan: the scratch must be there, 16-byte aligned");
   float4* cf = reinterpret_cast<float4*>(coef);
-  const int logs_first = max_run >= 16 ? 1 : 0;      // long runs: the gates' logarithms of all T rows first, in parallel
-  if (logs_first) {
-    KVCM_REQUIRE(T > 0, "mlstm_scan: the row count is needed for runs of %d", max_run);
-    const long long n = static_cast<long long>(T) * heads;
-    mlstm_gate_logs_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, n, heads);
-  }
-  auto* maxima = one_order ? mlstm_max_kernel<true> : mlstm_max_kernel<false>;
-  maxima<<<S * heads, kWave, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, heads,
-                                     logs_first);
+  KVCM_REQUIRE(max_run < 16 || T > 0, "mlstm_scan: the row count is needed for runs of %d", max_run);
+  mlstm_factors(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, S, heads, T, max_run, one_order, s);
 #define KVCM_MLSTM_AS(DKP, G, NC, U, NT, HOW)                                                                                    \
   {                                                                                                                          \
     const int col_blocks = (dv + NT / G * NC - 1) / (NT / G * NC);                                                                     \

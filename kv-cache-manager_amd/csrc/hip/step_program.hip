@@ -116,6 +116,7 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_head_gate),
     KVCM_ENTRY(kvcm_rms_groups),
     KVCM_ENTRY(kvcm_mlstm_scan),
+    KVCM_ENTRY(kvcm_mlstm_chunks),
     KVCM_ENTRY(kvcm_moe_route),
     KVCM_ENTRY(kvcm_moe_table_route),
     KVCM_ENTRY(kvcm_moe_up),

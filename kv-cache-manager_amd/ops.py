@@ -130,6 +130,9 @@ def _declare(lib):
     fn("kvcm_gemm_heads", vp, i, i, vp, vp, i, i, vp, i, i, i, i, i, vp)
     fn("kvcm_act_rows", vp, i, i, C.c_longlong, vp, i, i, i, i, i, vp)
     fn("kvcm_mlstm_scan", vp, i, vp, i, vp, i, vp, i, vp, i, vp, vp, f, f, vp, vp, vp, i, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, vp)
+    fn("kvcm_mlstm_chunks", vp, i, vp, i, vp, i, vp, i, vp, i, vp, vp, f, f, vp, vp, i, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, vp, C.c_longlong, vp)
+    lib.kvcm_mlstm_carry_floats.restype = C.c_longlong
+    lib.kvcm_mlstm_carry_floats.argtypes = [i] * 6
     fn("kvcm_moe_route", vp, i, i, C.c_longlong, i, i, i, f, vp, vp, i, vp)
     fn("kvcm_moe_table_route", vp, vp, i, i, i, vp, vp, i, vp)
     fn("kvcm_moe_up", vp, i, i, vp, vp, vp, i, i, i, i, i, i, vp, vp)
@@ -1986,11 +1989,27 @@ def act_rows(x, out, activation):
     return out
 
 
-def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, coef, n_new, o, s_state, n_state, m_state, step, heads, dk, dv, one_order=False):
+MLSTM_PIECE = 128            # rows of a piece of ``mlstm_scan``'s matrix form
+MLSTM_MIN_RUN = 256          # rows of a step's longest run from which that form is worth it (us, 32 heads of 64 x 64, walk / so: 192 rows 38.0 / 40.2, 256 rows 44.9 / 42.3)
+
+
+def mlstm_in_chunks(step, dk, one_order=False):
+    """Does ``mlstm_scan``, given scratch for the pieces, take this step's runs in matrix form (csrc/hip/mlstm_chunks.hip)?"""
+    return not one_order and dk <= 128 and step.max_run >= MLSTM_MIN_RUN and step.seqs * -(-int(step.max_run) // MLSTM_PIECE) <= 65535
+
+
+def mlstm_carry_floats(rows, seqs, heads, dk, dv):
+    """32-bit values of scratch that ``mlstm_scan`` needs to take a step of this shape in matrix form."""
+    return int(lib().kvcm_mlstm_carry_floats(rows, seqs, heads, dk, dv, MLSTM_PIECE))
+
+
+def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, coef, n_new, o, s_state, n_state, m_state, step, heads, dk, dv, one_order=False,
+               carry=None):
     """The matrix memory with exponential gates over the step's runs (csrc/hip/mlstm.hip).  q, k [T, heads*dk], v [T, heads*dv],
     gate_in, gate_keep [T, heads] (projections without biases): 32-bit rows; coef: float32 scratch of 4 T heads values;
     n_new: float32 scratch of seqs heads dk values; states [slots, heads, dk, dv], [slots, heads, dk], [slots, heads].
-    ``one_order``: a row's maximum and sums are taken in one order whatever else the step holds (32-bit storage)."""
+    ``one_order``: a row's maximum and sums are taken in one order whatever else the step holds (32-bit storage).
+    ``carry`` (float32 scratch of ``mlstm_carry_floats``): steps with long runs (``mlstm_in_chunks``) take them in matrix form."""
     T = o.shape[0]
     for t, n, c in ((q, "q", heads * dk), (k, "k", heads * dk), (v, "v", heads * dv), (o, "o", heads * dv), (gate_in, "gate_in", heads),
                     (gate_keep, "gate_keep", heads)):
@@ -2002,6 +2021,13 @@ def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, co
     _f32(n_new, "n_new", step.seqs * heads * dk)
     for t, n, shape in ((s_state, "s_state", (heads, dk, dv)), (n_state, "n_state", (heads, dk)), (m_state, "m_state", (heads,))):
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.is_cuda and tuple(t.shape[1:]) == shape, f"{n} must be float32 [slots, {shape}]")
+    if carry is not None and mlstm_in_chunks(step, dk, one_order):
+        _f32(carry, "carry")
+        _call("kvcm_mlstm_chunks", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_in), gate_in.stride(0),
+              _ptr(gate_keep), gate_keep.stride(0), _ptr(in_bias), _ptr(keep_bias), float(cap), float(q_scale), _ptr(coef), _ptr(o),
+              o.stride(0), _ptr(s_state), _ptr(n_state), _ptr(m_state), _ptr(step.run_start), _ptr(step.seq_start),
+              _ptr(step.state_slots), step.seqs, heads, dk, dv, T, int(step.max_run), MLSTM_PIECE, _ptr(carry), carry.numel(), _stream())
+        return o
     _call("kvcm_mlstm_scan", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_in), gate_in.stride(0),
           _ptr(gate_keep), gate_keep.stride(0), _ptr(in_bias), _ptr(keep_bias), float(cap), float(q_scale), _ptr(coef), _ptr(n_new), _ptr(o),
           o.stride(0), _ptr(s_state), _ptr(n_state), _ptr(m_state), _ptr(step.run_start), _ptr(step.seq_start),

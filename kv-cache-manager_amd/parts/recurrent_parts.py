@@ -178,6 +178,14 @@ class MatrixMemoryMixer(_StatefulMixer):
                 "normalizer": StateNeed((p["heads"], p["dim"]), torch.float32),
                 "maximum": StateNeed((p["heads"],), torch.float32)}
 
+    def carry(self, step, one_order):
+        """Scratch for steps whose long runs go in matrix form, sized for the engine's largest step."""
+        ops, p, lim = self.ctx.ops, self.params, step.limits
+        if not ops.mlstm_in_chunks(step, p["dim"], one_order):
+            return None
+        rows, seqs = max(step.rows, lim.max_tokens if lim else 0), max(step.seqs, lim.max_seqs if lim else 0)
+        return step.flat("memory_carry", ops.mlstm_carry_floats(rows, seqs, p["heads"], p["dim"], p["vdim"]))
+
     def flops(self, rows, attended=0):
         p = self.params
         return super().flops(rows) + rows * p["heads"] * (4.0 * p["dim"] * p["vdim"] + 4.0 * p["dim"])
@@ -196,7 +204,7 @@ class MatrixMemoryMixer(_StatefulMixer):
         gated = step.ws("memory_gated", (T, heads * dv))
         ops.mlstm_scan(q, k, v, gi, gf, w["in_bias"], w["keep_bias"], p["gate_cap"], float(d) ** -0.5, coef, n_new, o,
                        self.state("memory"), self.state("normalizer"), self.state("maximum"), step, heads, d, dv,
-                       one_order=gated.dtype == torch.float32)
+                       one_order=gated.dtype == torch.float32, carry=self.carry(step, gated.dtype == torch.float32))
         ops.head_norm_gate(o, g, w["norm"], gated, heads, dv, p["eps"])
         return linear32(self.ctx, step, gated, w["w_o"], "memory_out", keep_partial=True)      # the stream's next norm adds the slices
 

@@ -1,0 +1,70 @@
+"""The matrix memory in matrix form (csrc/hip/mlstm_chunks.hip) against the plain recurrence: chunks of 64 rows and pieces of 128 that end
+anywhere, runs that begin in the middle of a sequence, keys and values that end inside a tile, rows that begin at any float, dead slots."""
+import numpy as np
+import pytest
+import torch
+
+import plain_furapel as plain
+from test_kasuvik_gpu import Step
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("d,dv,shift", [(64, 64, 0), (64, 130, 0), (16, 6, 1), (100, 20, 0), (128, 72, 0), (20, 33, 1), (65, 4, 0)])
+def test_long_runs_against_the_plain_recurrence(d, dv, shift):
+    from kvcm_amd import ops
+    rng = np.random.default_rng(d + dv)
+    heads, cap, parts = 2, 12.0, ((256, 1, 129, 64), (63, 321, 128, 7), (257, 192, 1, 385))
+    seqs = len(parts[0])
+    total = [sum(x[i] for x in parts) for i in range(seqs)]
+    # positive keys and queries: the divisor n . q has no cancellation; then sums of up to 256 products and 64 rows in up to three pieces stay
+    # within 3e-5 of 32-bit rounding (twice 256 steps of 2^-24)
+    data = [[np.abs(rng.normal(size=(n, heads, d))), np.abs(rng.normal(size=(n, heads, d))), rng.normal(size=(n, heads, dv)),
+             rng.normal(size=(n, heads)) * 4, rng.normal(size=(n, heads)) * 4 + 2] for n in total]
+    bi, bf = rng.normal(size=heads), rng.normal(size=heads)
+    want = []
+    for q, k, v, gi, gf in data:
+        o = np.zeros((q.shape[0], heads, dv))
+        for a in range(heads):
+            o[:, a], _ = plain.matrix_memory(q[:, a] * d ** -0.5, k[:, a], v[:, a], plain.soft_cap(gi[:, a] + bi[a], cap),
+                                             plain.log_sigmoid(plain.soft_cap(gf[:, a] + bf[a], cap)))
+        want.append(o.reshape(-1, heads * dv))
+
+    def dev(x):
+        return torch.tensor(np.asarray(x), dtype=torch.float32, device=DEV)
+
+    # (a dead slot beside them: its rows are zero, and it has no state)
+    S = torch.full((seqs, heads, d, dv), 9.0, device=DEV)
+    N, M = torch.full((seqs, heads, d), -3.0, device=DEV), torch.full((seqs, heads), 50.0, device=DEV)
+    cols = np.cumsum([0, heads * d, heads * d, heads * dv, heads])
+    at = [0] * seqs
+    for part in parts:
+        st = Step([(i, at[i], n) for i, n in enumerate(part)] + [(0, 5, 140)])
+        st.max_run = max(part)
+        slots = st.state_slots.clone()
+        slots[-1] = -1
+        st.state_slots = slots
+        rows = np.concatenate([np.concatenate([x[at[i]:at[i] + n].reshape(n, -1) for x in data[i]], 1) for i, n in enumerate(part)]
+                              + [rng.normal(size=(140, cols[-1] + heads))], 0)
+        packed = torch.full((rows.shape[0], rows.shape[1] + 2 + shift), float("nan"), device=DEV)[:, shift:]
+        packed[:, :rows.shape[1]] = dev(rows)
+        x = [packed[:, lo:] for lo in cols]
+        assert ops.mlstm_in_chunks(st, d) and not ops.mlstm_in_chunks(st, d, True)
+        carry = torch.full((ops.mlstm_carry_floats(st.rows, st.seqs, heads, d, dv),), float("nan"), device=DEV)
+        coef, o = torch.empty(st.rows, 4 * heads, device=DEV), torch.full((st.rows, heads * dv), float("nan"), device=DEV)
+        ops.mlstm_scan(*x, dev(bi), dev(bf), cap, d ** -0.5, coef, torch.empty(st.seqs * heads * d, device=DEV), o, S, N, M, st, heads, d, dv,
+                       carry=carry)
+        row = 0
+        for i, n in enumerate(part):
+            ref = want[i][at[i]:at[i] + n]
+            np.testing.assert_allclose(o[row:row + n].cpu().numpy(), ref, atol=3e-5 * max(1.0, np.abs(ref).max()), err_msg=f"sequence {i} from {at[i]}")
+            row, at[i] = row + n, at[i] + n
+        assert not bool(o[row:].any())
+
+
+def test_the_line_between_the_forms():
+    from kvcm_amd import ops
+    short, long = Step([(0, 0, 255), (1, 0, 3)]), Step([(0, 0, 256), (1, 0, 3)])
+    short.max_run, long.max_run = 255, 256
+    assert not ops.mlstm_in_chunks(short, 64) and ops.mlstm_in_chunks(long, 128) and not ops.mlstm_in_chunks(long, 129)
