@@ -236,9 +236,9 @@ int kvcm_attention_window_pool_tiles(const void* q, int ldq, void* out, int ldo,
                                      const float* gate, int ldg, int S, int max_run, int nh, int nkv, int d, int dv, int B, float scale, int window, int P,
                                      int E, int keep_first, float softcap, int chunk, int sink, const float* sink_logit, int gate_heads, float out_scale, hipStream_t s);
 // (selective_scan.hip, delta_rule.hip) recurrences with a 32-bit state per sequence
-int kvcm_selective_scan(const void* x, int dtype, int ldx, const float* dt_lin, int lddt, const float* dt_bias,
+int kvcm_selective_scan(const void* x, int dtype, int ldx, float* dt_lin, int lddt, const float* dt_bias,
                         const float* bc, int ldbc, int off_b, int off_c, const float* a_log, const float* dskip,
-                        const float* z, int ldz, void* out, int ldo, float* state, const int* run_start,
+                        float* z, int ldz, void* out, int ldo, float* state, const int* run_start,
                         const int* seq_start, const int* state_slots, int S, int C, int N, int prepared, int chunk_len,
                         int max_run, float* carry, long long carry_floats, int T, hipStream_t s);
 int kvcm_scan_prepare(float* dt, int lddt, const float* dt_bias, float* z, int ldz, int T, int C, hipStream_t s);

@@ -30,6 +30,19 @@ template <class T> __device__ __forceinline__ float decay_exp(float v);
 template <> __device__ __forceinline__ float decay_exp<float>(float v) { return expf(v); }
 template <> __device__ __forceinline__ float decay_exp<bf16_t>(float v) { return __builtin_amdgcn_exp2f(1.44269504088896341f * v); }
 
+// log(1 + exp(v)) = max(v, 0) + log1p(exp(-|v|)): exp2 of -|v| log2(e) times what that product's rounding lost, and the logarithm of the
+// rounded 1 + e with what its rounding lost.  A dozen instructions with three of a quarter's rate, where log1pf(expf(v)) is some
+// hundred (21 of a pass's 62 us at 2,048 x 4,096).  Largest error against 64 bits, log1pf(expf(v)) / so: 1.4e-6 / 2.6e-7 over
+// [-30, -15), 8.5e-7 / 2.3e-7 to -5, 3.4e-7 / 2.2e-7 to -1, 2.1e-7 / 1.7e-7 to 0, 1.5e-7 / 1.1e-7 beyond.
+__device__ __forceinline__ float softplus(float v) {
+  const float m = fabsf(v), a = m > 200.f ? 200.f : m;      // (what is no number stays none)
+  const float p = a * 1.44269504088896341f;
+  const float lost = fmaf(a, 1.925962991e-8f, fmaf(a, 1.44269504088896341f, -p));
+  const float e0 = __builtin_amdgcn_exp2f(-p), e = fmaf(e0 * lost, -0.69314718055994531f, e0);
+  const float w = 1.f + e, c = e - (w - 1.f);
+  return fmaxf(v, 0.f) + fmaf(__builtin_amdgcn_logf(w), 0.69314718055994531f, c * __builtin_amdgcn_rcpf(w));      // (logf: to base 2)
+}
+
 constexpr int kScanAhead = 4;      // tokens whose inputs are on their way while the ones before are computed
 
 template <class T, int LPC, int NPL>
@@ -101,7 +114,7 @@ __global__ void __launch_bounds__(kWave)
       const int r = first + u;
       if (r < r1) {
         const float v = dtv[from][u] + db;
-        const float dt = prepared ? dtv[from][u] : (v > 20.f ? v : log1pf(expf(v)));
+        const float dt = prepared ? dtv[from][u] : softplus(v);
         const float dx = dt * xv[from][u];
         dt_total += dt;
         float y = 0.f;
@@ -142,8 +155,10 @@ __global__ void __launch_bounds__(kWave)
 // Pieces of long runs with 8 or 16 states a channel: a lane owns a channel with all its states, so that a token costs a lane one
 // exponential and three multiply-adds a state and no sum crosses lanes (with the states over lanes every lane also fetched the
 // channel's step size, input and gate, and a wave's sums took a sixth of its instructions).  B and C, the same for all channels,
-// are staged through LDS 64 tokens at a time and read by all lanes at once.  Bound by the exponentials, a quarter of the rate of
-// other instructions.  2,048 tokens, 4,096 channels, 16 states: 146 us a phase in the mean -> 40 us (the first) and 52 us.
+// are staged through LDS 64 tokens at a time and read by all lanes at once.  Bound by a wave's own chain while there are few waves, then by
+// the exponentials, a quarter of the rate of other instructions.  4,096 channels, 16 states, both passes and what is between: 512 / 1,024 / 2,048
+// tokens 98 / 170 / 136 us in pieces of 128 tokens behind a launch that made step sizes and gates; 48 / 71 / 112 us in pieces of 32 to 64
+// without it, and the last, with the step size's formula above, 94 us (41, 8 and 45).
 template <class T> __device__ __forceinline__ float scaled_rate(float a) { return a; }
 template <> __device__ __forceinline__ float scaled_rate<bf16_t>(float a) { return 1.44269504088896341f * a; }      // for exp2
 template <class T> __device__ __forceinline__ float scaled_exp(float v) { return expf(v); }
@@ -189,7 +204,7 @@ __global__ void __launch_bounds__(kWave)
   const float lin = dt_lin[size_t(r) * lddt + c], xx = load_f(x + size_t(r) * ldx + c), zz = z[size_t(r) * ldz + c];
   const float v = lin + (dt_bias ? dt_bias[c] : 0.f), skip = dskip[c];
   const float *b = bc + size_t(r) * ldbc + off_b, *cc = bc + size_t(r) * ldbc + off_c;
-  const float dt = prepared ? lin : (v > 20.f ? v : log1pf(expf(v))), dx = dt * xx;
+  const float dt = prepared ? lin : softplus(v), dx = dt * xx;
   float ys[N];
 #pragma unroll
   for (int n = 0; n < N / 4; ++n) {
@@ -206,13 +221,15 @@ __global__ void __launch_bounds__(kWave)
   store_f(out + size_t(r) * ldo + c, fmaf(skip, xx, states_sum(ys)) * (prepared ? zz : zz / (1.0f + expf(-zz))));
 }
 
+// The first pass makes the step sizes as it walks and leaves them in place for the second, which makes the gates (a launch of
+// their own read and wrote both, 134 MB of 32-bit rows and 37 us at 2,048 x 4,096).
 template <class T, int N, bool OUT>
 __global__ void __launch_bounds__(256)
-    scan_channels_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ dt, int lddt, const float* __restrict__ bc,
-                         int ldbc, int off_b, int off_c, const float* __restrict__ a_log, const float* __restrict__ dskip,
-                         const float* __restrict__ z, int ldz, T* __restrict__ out, int ldo, const int* __restrict__ run_start,
-                         const int* __restrict__ state_slots, int C, int chunk_len, float* __restrict__ carry,
-                         float* __restrict__ dsum) {
+    scan_channels_kernel(const T* __restrict__ x, int ldx, float* __restrict__ dt, int lddt, const float* __restrict__ dt_bias,
+                         const float* __restrict__ bc, int ldbc, int off_b, int off_c, const float* __restrict__ a_log,
+                         const float* __restrict__ dskip, const float* __restrict__ z, int ldz, T* __restrict__ out, int ldo,
+                         const int* __restrict__ run_start, const int* __restrict__ state_slots, int C, int chunk_len,
+                         float* __restrict__ carry, float* __restrict__ dsum) {
   constexpr int U = 4, W = OUT ? 2 * N : N;
   constexpr bool kOneOrder = std::is_same<T, float>::value;      // (32-bit results do not depend on how the states are dealt out)
   __shared__ __attribute__((aligned(16))) float tile[kScanTile][W];
@@ -236,7 +253,7 @@ __global__ void __launch_bounds__(256)
     A[n] = scaled_rate<T>(-expf(a_log[size_t(c) * N + n]));
     S[n] = OUT ? at[n] : 0.f;
   }
-  const float skip = OUT ? dskip[c] : 0.f;
+  const float skip = OUT ? dskip[c] : 0.f, db = !OUT && dt_bias ? dt_bias[c] : 0.f;
   float dt_total = 0.f;
   float dtv[2][U], xv[2][U], zv[2][U];
   auto request = [&](int first, int into) {
@@ -253,7 +270,12 @@ __global__ void __launch_bounds__(256)
     for (int u = 0; u < U; ++u) {
       const int r = first + u;
       if (r >= r1) break;
-      const float step = dtv[from][u], dx = step * xv[from][u];
+      float step = dtv[from][u];
+      if (!OUT) {
+        step = softplus(step + db);
+        if (owns) dt[size_t(r) * lddt + c] = step;
+      }
+      const float dx = step * xv[from][u];
       const float* bt = tile[r - t0];
       dt_total += step;
       float y = 0.f, ys[N];
@@ -264,18 +286,21 @@ __global__ void __launch_bounds__(256)
         else if (OUT) y = fmaf(S[n], bt[N + n], y);
       }
       if (OUT && kOneOrder) y = states_sum(ys);
-      if (OUT && owns) store_f(out + size_t(r) * ldo + c, fmaf(skip, xv[from][u], y) * zv[from][u]);
+      if (OUT && owns) {
+        const float zz = zv[from][u];
+        store_f(out + size_t(r) * ldo + c, fmaf(skip, xv[from][u], y) * (zz / (1.0f + expf(-zz))));
+      }
     }
   };
   request(r0, 0);
   for (int t0 = r0; t0 < r1; t0 += kScanTile) {
     if (t0 > r0) __syncthreads();
-    for (int e = threadIdx.x; e < kScanTile * W; e += 256) {
-      const int t = e / W, n = e % W, r = t0 + t < r1 ? t0 + t : r1 - 1;
-      tile[t][n] = bc[size_t(r) * ldbc + (n < N ? off_b + n : off_c + n - N)];
+    const int end = r1 < t0 + kScanTile ? r1 : t0 + kScanTile;
+    for (int e = threadIdx.x; e < (end - t0) * W; e += 256) {
+      const int t = e / W, n = e % W;
+      tile[t][n] = bc[size_t(t0 + t) * ldbc + (n < N ? off_b + n : off_c + n - N)];
     }
     __syncthreads();
-    const int end = r1 < t0 + kScanTile ? r1 : t0 + kScanTile;
     for (int r = t0; r < end; r += 2 * U) {      // (a tile is a multiple of 2 U tokens)
       request(r + U, 1);
       walk(r, 0, t0);
@@ -308,11 +333,21 @@ __global__ void __launch_bounds__(256)
   float S = seq_start[s] == 0 ? 0.f : *st;
   const size_t first = size_t(r0 / chunk_len + s);
   const int pieces = (len + chunk_len - 1) / chunk_len;
-  for (int j = 0; j < pieces; ++j) {
-    float* at = carry + (first + j) * C * N + e;
-    const float end = *at;
-    *at = S;
-    S = fmaf(expf(A * dsum[(first + j) * C + c]), S, end);
+  constexpr int kAhead = 16;      // pieces requested together
+  for (int j0 = 0; j0 < pieces; j0 += kAhead) {
+    float end[kAhead], steps[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const size_t at = first + (j0 + i < pieces ? j0 + i : pieces - 1);
+      end[i] = carry[at * C * N + e];
+      steps[i] = dsum[at * C + c];
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (j0 + i >= pieces) break;
+      carry[(first + j0 + i) * C * N + e] = S;
+      S = fmaf(expf(A * steps[i]), S, end[i]);
+    }
   }
   *st = S;
 }
@@ -324,13 +359,27 @@ __global__ void __launch_bounds__(256)
   const int r = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
   if (c >= C) return;
   const float v = dt[size_t(r) * lddt + c] + (dt_bias ? dt_bias[c] : 0.f);
-  dt[size_t(r) * lddt + c] = v > 20.f ? v : log1pf(expf(v));
+  dt[size_t(r) * lddt + c] = softplus(v);
   const float zz = z[size_t(r) * ldz + c];
   z[size_t(r) * ldz + c] = zz / (1.0f + expf(-zz));
 }
 
+// Pieces: a lane a channel or states over lanes.  bfloat16, both passes with what is between, pieces of 32 rows, us, states over lanes / a
+// lane a channel, 16 states (before the step size's formula above): 256 rows of 1,024 channels 32 / 40, of 2,048 38 / 41, of 4,096 60 / 42; 512 of 1,024 42 / 43, of 2,048 64 / 44;
+// 1,024 of 4,096 183 / 71.  32-bit exponentials take longer, and a wave all of them (pieces of 128): 1 x 2,048 of 1,024 110 / 198, of 2,048
+// 182 / 207, of 4,096 330 / 227, 8 x 512 of 1,024 173 / 203, of 2,048 311 / 220.
+bool scan_by_channels(bool f32, int T, int C, int N) {
+  return (N == 8 || N == 16) && static_cast<long long>(T) * C >= (f32 ? 640ll * kWave * 128 : 1ll << 19);
+}
+
+int prepare_scan(float* dt, int lddt, const float* dt_bias, float* z, int ldz, int T, int C, hipStream_t s) {
+  KVCM_REQUIRE(T <= 65535, "scan_prepare: too many rows for one launch (%d)", T);
+  scan_prepare_kernel<<<dim3((C + 255) / 256, T), 256, 0, s>>>(dt, lddt, dt_bias, z, ldz, C);
+  return launch_status("scan_prepare");
+}
+
 template <class X>
-int launch_scan(const void* x, int ldx, const float* dt_lin, int lddt, const float* dt_bias, const float* bc, int ldbc,
+int launch_scan(const void* x, int ldx, float* dt_lin, int lddt, const float* dt_bias, const float* bc, int ldbc,
                 int off_b, int off_c, const float* a_log, const float* dskip, const float* z, int ldz, void* out, int ldo,
                 float* state, const int* run_start, const int* seq_start, const int* state_slots, int S, int C, int N,
                 int prepared, int phase, int chunk_len, int pieces, int max_run, int T, float* carry, float* dsum, hipStream_t s) {
@@ -349,17 +398,12 @@ int launch_scan(const void* x, int ldx, const float* dt_lin, int lddt, const flo
 #undef KVCM_SCAN_SINGLE
     return launch_status("selective_scan");
   }
-  // Pieces: a lane a channel once its waves (64 channels, chunk_len rows) are about one a CU, states over lanes before; 32-bit
-  // exponentials take longer, and a wave all of them.  Two passes over pieces with the step sizes, us, states over lanes / a lane a channel,
-  // 16 states: bfloat16 1 x 512 rows of 1,024 channels 76 / 85, 1 x 2,048 of 1,024 106 / 101, of 4,096 319 / 130, 8 x 512 of 512 100 / 98;
-  // 32 bits 1 x 2,048 of 1,024 110 / 198, of 2,048 182 / 207, of 4,096 330 / 227, 8 x 512 of 1,024 173 / 203, of 2,048 311 / 220.
-  const long long waves = static_cast<long long>(T) * C / (kWave * 128);
-  if (phase != 0 && (N == 8 || N == 16) && waves >= (std::is_same<X, float>::value ? 640 : 256)) {
+  if (phase != 0 && scan_by_channels(std::is_same<X, float>::value, T, C, N)) {
     const dim3 grid((C + 255) / 256, S, pieces);
 #define KVCM_SCAN_CHANNELS(N, OUT)                                                                                            \
-  scan_channels_kernel<X, N, OUT><<<grid, 256, 0, s>>>(static_cast<const X*>(x), ldx, dt_lin, lddt, bc, ldbc, off_b, off_c,     \
-                                                       a_log, dskip, z, ldz, static_cast<X*>(out), ldo, run_start, state_slots, \
-                                                       C, chunk_len, carry, dsum)
+  scan_channels_kernel<X, N, OUT><<<grid, 256, 0, s>>>(static_cast<const X*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b,   \
+                                                       off_c, a_log, dskip, z, ldz, static_cast<X*>(out), ldo, run_start,       \
+                                                       state_slots, C, chunk_len, carry, dsum)
     if (N == 8 && phase == 1) KVCM_SCAN_CHANNELS(8, false);
     else if (N == 8) KVCM_SCAN_CHANNELS(8, true);
     else if (phase == 1) KVCM_SCAN_CHANNELS(16, false);
@@ -392,10 +436,11 @@ using namespace kvcm;
 // (B at off_b, C at off_c, N each), z [T, ldz], a_log [C, N], dt_bias, dskip [C], state [slots, C, N]: 32-bit.
 // prepared: dt_lin holds the step sizes and z the gates already (kvcm_scan_prepare).
 // chunk_len > 0: runs (of up to max_run rows, T rows in all) are walked in pieces of chunk_len rows, all pieces at once, with
-// carry (at least (T / chunk_len + S + 1) * C * (N + 1) floats) between the phases; 0: every run in one walk.
-extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, const float* dt_lin, int lddt, const float* dt_bias,
+// carry (at least (T / chunk_len + S + 1) * C * (N + 1) floats) between the phases; dt_lin (and z) hold step sizes (and gates)
+// afterwards; 0: every run in one walk.
+extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, float* dt_lin, int lddt, const float* dt_bias,
                                    const float* bc, int ldbc, int off_b, int off_c, const float* a_log, const float* dskip,
-                                   const float* z, int ldz, void* out, int ldo, float* state, const int* run_start,
+                                   float* z, int ldz, void* out, int ldo, float* state, const int* run_start,
                                    const int* seq_start, const int* state_slots, int S, int C, int N, int prepared,
                                    int chunk_len, int max_run, float* carry, long long carry_floats, int T, hipStream_t s) {
   if (S == 0) return 0;
@@ -414,25 +459,26 @@ extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, const floa
   };
   if (chunk_len <= 0) return launch(0, 1, nullptr, nullptr);
   // long runs in pieces of chunk_len rows: every piece from zero, the states that enter the pieces, every piece again
-  KVCM_REQUIRE(prepared, "selective_scan: runs are cut into pieces only with the step sizes made ahead");
+  KVCM_REQUIRE(!prepared, "selective_scan: runs that are cut into pieces take their step sizes as they are projected");
   const int pieces = (max_run + chunk_len - 1) / chunk_len;
   const long long slots = static_cast<long long>(T) / chunk_len + S + 1;      // piece j of sequence s: run_start / chunk_len + s + j
   KVCM_REQUIRE(pieces >= 1 && pieces <= 65535 && carry != nullptr && carry_floats >= slots * C * (N + 1),
                "selective_scan: the scratch for %lld pieces is too small", slots);
   float* dsum = carry + slots * C * N;
+  if (!scan_by_channels(dtype == kF32, T, C, N)) {
+    if (int rc = prepare_scan(dt_lin, lddt, dt_bias, z, ldz, T, C, s)) return rc;
+    prepared = 1;
+  }
   if (int rc = launch(1, pieces, carry, dsum)) return rc;
   scan_carry_kernel<<<dim3((C * N + 255) / 256, S), 256, 0, s>>>(carry, dsum, a_log, state, run_start, seq_start, state_slots, C, N,
                                                                  chunk_len);
   if (int rc = launch_status("scan_carry")) return rc;
   return launch(2, pieces, carry, dsum);
-  KVCM_REQUIRE(false, "selective_scan: unknown dtype %d", dtype);
 }
 
 // dt [T, C] <- softplus(dt + dt_bias), z [T, C] <- silu(z), in place; kvcm_selective_scan then runs with prepared = 1.
 extern "C" int kvcm_scan_prepare(float* dt, int lddt, const float* dt_bias, float* z, int ldz, int T, int C, hipStream_t s) {
   if (T == 0) return 0;
   KVCM_REQUIRE(T > 0 && C > 0 && lddt >= C && ldz >= C, "scan_prepare: bad sizes T=%d C=%d", T, C);
-  KVCM_REQUIRE(T <= 65535, "scan_prepare: too many rows for one launch (%d)", T);
-  scan_prepare_kernel<<<dim3((C + 255) / 256, T), 256, 0, s>>>(dt, lddt, dt_bias, z, ldz, C);
-  return launch_status("scan_prepare");
+  return prepare_scan(dt, lddt, dt_bias, z, ldz, T, C, s);
 }

@@ -1675,12 +1675,33 @@ def attention_window_pool_tiles(q, out, kcache, vcache, pk, pv, tables, table_st
           float(out_scale), _stream())
 
 
-SCAN_PIECE = 128      # rows of a piece when long runs are walked in pieces
+SCAN_PIECE = 128      # rows of a piece when long runs are walked in pieces, at most
 
 
-def selective_scan_carry_floats(rows, seqs, C, N, piece=SCAN_PIECE):
-    """32-bit values of scratch that ``selective_scan(..., pieces=True)`` needs for a step of this shape."""
-    return (rows // piece + seqs + 1) * C * (N + 1)
+def scan_piece(rows, C, dtype):
+    """Rows of a piece for a step of ``rows`` rows.  A piece is one wave's chain for every 64 channels, and costs its states to be
+    written and read: short ones until the chip is full (bfloat16, 16 states, us, pieces of 32 / 64 / 128: 4,096 channels 512 rows
+    48 / 70 / 122, 1,024 rows 71 / 77 / 126, 2,048 rows 117 / 112 / 134, 6,144 rows 254 / 243 / 251).  In 32-bit storage, where the
+    pieces are part of a result's order, always the longest."""
+    if dtype != torch.bfloat16 or rows * C >= 1 << 25:
+        return SCAN_PIECE
+    return 64 if rows * C >= 1 << 23 else 32
+
+
+def scan_in_pieces(step, C, N, dtype):
+    """Is a step worth two passes over pieces?  From four pieces of 128 rows on; with the hardware's exponentials (bfloat16) and 8 or 16
+    states from 128 rows, many rows of shorter runs from 64, if most rows are in runs: single tokens pay for both passes and gain
+    nothing (us, whole / in pieces, 4,096 channels: 96 rows 40 / 34, 128 rows 50 / 38, 300 rows 101 / 44, 4 x 64 39 / 42, 16 x 64
+    114 / 69, 8 x 509 439 / 169; 2,048 channels 16 x 64 65 / 47; 128 beside 7 single tokens 51 / 53, 300 beside 31 108 / 106)."""
+    if dtype == torch.bfloat16 and N in (8, 16) and step.rows >= 32 * step.seqs:
+        return step.max_run >= 128 or (step.max_run >= 64 and step.rows * C >= 1 << 21)
+    return step.max_run >= 4 * SCAN_PIECE
+
+
+def selective_scan_carry_floats(rows, seqs, C, N):
+    """32-bit values of scratch that ``selective_scan(..., carry=...)`` needs for steps of up to this shape."""
+    short = min(rows // 32, (1 << 19) // C)      # (shorter pieces are no more than that)
+    return (max(rows // SCAN_PIECE, short) + seqs + 1) * C * (N + 1)
 
 
 def selective_scan(x, dt_lin, dt_bias, bc, off_b, off_c, a_log, dskip, z, out, state, step, prepare=False, carry=None):
@@ -1688,7 +1709,7 @@ def selective_scan(x, dt_lin, dt_bias, bc, off_b, off_c, a_log, dskip, z, out, s
     dt_lin [T, C], bc rows with B at off_b and C at off_c, z rows: 32-bit; state [slots, C, N].  ``prepare``: the step
     sizes and gates of all rows are made first, in place in dt_lin and z, by a launch of their own (pays for long runs).
     ``carry`` (float32 scratch of ``selective_scan_carry_floats``; needs ``prepare``): runs are walked in pieces of
-    SCAN_PIECE rows, all pieces at once: each from zero, then the states that enter the pieces (a short walk over the
+    ``scan_piece`` rows, all pieces at once: each from zero, then the states that enter the pieces (a short walk over the
     pieces' ends), then each again from its entering state.  The sums are the token-by-token ones in another order."""
     C, N = a_log.shape
     _rows2d(x, "x")
@@ -1705,12 +1726,12 @@ def selective_scan(x, dt_lin, dt_bias, bc, off_b, off_c, a_log, dskip, z, out, s
     if carry is not None:
         _need(prepare and carry.dtype == torch.float32 and carry.is_contiguous() and carry.is_cuda
               and carry.numel() >= selective_scan_carry_floats(out.shape[0], step.seqs, C, N), "the scratch for the pieces is too small")
-    if prepare:
+    if prepare and carry is None:
         _call("kvcm_scan_prepare", _ptr(dt_lin), dt_lin.stride(0), _ptr(dt_bias), _ptr(z), z.stride(0), out.shape[0], C, _stream())
     _call("kvcm_selective_scan", _ptr(x), _DT[x.dtype], x.stride(0), _ptr(dt_lin), dt_lin.stride(0), _ptr(dt_bias), _ptr(bc),
           bc.stride(0), off_b, off_c, _ptr(a_log), _ptr(dskip), _ptr(z), z.stride(0), _ptr(out), out.stride(0), _ptr(state),
-          _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs, C, N, 1 if prepare else 0,
-          SCAN_PIECE if carry is not None else 0, step.max_run, _ptr(carry), carry.numel() if carry is not None else 0,
+          _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs, C, N, 1 if prepare and carry is None else 0,
+          scan_piece(out.shape[0], C, x.dtype) if carry is not None else 0, step.max_run, _ptr(carry), carry.numel() if carry is not None else 0,
           out.shape[0], _stream())
     return out
 

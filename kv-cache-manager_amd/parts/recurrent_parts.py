@@ -78,13 +78,9 @@ class SelectiveScanMixer(_StatefulMixer):
         low, bc = linear_pair(self.ctx, step, (x, w["w_x"][:R], "scan_dt_low", None), (x, w["w_x"][R:], "scan_bc", torch.float32))
         dt = linear32(self.ctx, step, low, w["w_dt"], "scan_dt")
         y = step.ws("scan_y", (step.rows, C))
-        # runs of some length: step sizes and gates made ahead; long runs: walked in pieces, all pieces at once.  Two passes pay
-        # from four pieces on; with the hardware's exponentials (bfloat16) and 8 or 16 states from two, if most rows are in runs: single
-        # tokens pay for both passes and gain nothing (us, whole / in pieces, 4,096 channels: 300 rows 105 / 86, 8 x 509 439 / 182, 300
-        # beside 7 single tokens 110 / 91, beside 31 122 / 131, 256 beside 15 100 / 104)
+        # runs of some length: step sizes and gates made ahead; long runs: walked in pieces, all pieces at once
         carry = None
-        runs = x.dtype == torch.bfloat16 and N in (8, 16) and step.max_run >= 2 * ops.SCAN_PIECE and step.rows >= 32 * step.seqs
-        if runs or step.max_run >= 4 * ops.SCAN_PIECE:
+        if ops.scan_in_pieces(step, C, N, x.dtype):
             carry = step.flat("scan_carry", ops.selective_scan_carry_floats(max(step.rows, step.limits.max_tokens), step.limits.max_seqs, C, N))
         ops.selective_scan(x, dt, w["dt_bias"], bc, 0, N, w["a_log"], w["d_skip"], xz[:, C:], y, self.state("scan"), step,
                            prepare=step.max_run >= 16, carry=carry)
