@@ -1,0 +1,454 @@
+// The generalized delta rule (delta_rule.hip) for long runs, in matrix form.  In a chunk of C rows that starts from S, with W_i = w_0 .. w_i per
+// key channel and the rows
+//
+//   U_i = u_i W_(i-1)    R_i = r_i W_i    K_j = k_j / W_j    A_j = (a u)_j / W_j
+//
+// u_i^T S_(i-1) is row i of Z = X S + Y, where L = lower(U A^T) without its diagonal and (I + L) [X | Y] = [U | lower(U K^T) V], and
+//
+//   o = (R - P X) S + (lower(R K^T) V - P Y)        P = lower(R A^T), with its diagonal
+//   S <- diag(W) (I - A^T X) S + diag(W) (K^T V - A^T Y)        W = W_(C-1)
+//
+// Everything but the two products with S is made for all chunks at once (delta_chunk_kernel leaves a chunk's M = diag(W) (I - A^T X), its N, its
+// Q = R - P X and what its outputs have without S); what is left of the walk is one product of [M; Q] with S a chunk (delta_pass_kernel).  All of it
+// in 32 bits on the matrix cores (v_mfma_f32_16x16x4_f32).
+//
+// The quotients: w is exp(-exp(-1/2) sigmoid(.)), so 0.545 < w <= 1, W of 64 rows is above 1e-17 and a factor W_i / W_j of a term that is used is at
+// most one and has the relative error of a few roundings.  What lies above the diagonals may be large and is left out by selection.  (What is
+// not finite in a row reaches the rows of its chunk in front of it too.)
+//
+// The walk's time is a token's chain of dependent instructions whatever the chip could do.  One sequence of 2,048 tokens, 32 heads of 64 x 64: 293 us,
+// 120 so: 80 for the chunks (matrix instructions 35 of them, vector instructions as much, in 64-bit products of the decays and the rows' scaling, and
+// 164 MB moved) and 39 for the pass (32 steps of a product, a barrier and a trip through LDS).  128 x 128: 689 / 323 us.
+// Error against 64 bits of outputs and states, the walk / so: 1.11e-7 / 1.05e-7 and 8.8e-8 / 7.9e-8; 128 x 128 1.17e-7 / 1.16e-7 and 8.9e-8 / 7.8e-8
+// (with each sum in one chain 2.4e-7 and 2.0e-7).
+// A workgroup of the first kernel is eight waves, one a CU: four matrices of C rows by the keys and four of C by C in LDS, a wave with 16 columns of
+// X or Y in registers throughout, whose accumulators are the next product's second operand as they lie (key 4 g + e of lane group g is element e).
+#include "common.h"
+#include "kvcm_hip.h"
+
+namespace kvcm {
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+
+struct DeltaChunkArgs {
+  const float *r, *k, *v, *w, *au, *u;
+  int ldr, ldk, ldv;
+  float* o;
+  int ldo;
+  float* state;
+  const int *run_start, *seq_start, *state_slots;
+  int heads, dk, dv, col_blocks;
+  float* carry;      // per (sequence, chunk of the window, head): M, N [DKP][DKP], Q [C][DKP] in tiles of 16 x 16
+  int first, window, per_group;      // chunks first .. first + window - 1 of every run; chunks a workgroup takes one after the other
+};
+
+__host__ __device__ constexpr int delta_chunk_rows(int dkp) { return dkp == 64 ? 64 : 32; }
+__host__ __device__ constexpr long long delta_chunk_floats(int dkp) { return 2ll * dkp * dkp + delta_chunk_rows(dkp) * dkp; }
+
+template <int DKP>
+__device__ __forceinline__ float* delta_chunk_place(const DeltaChunkArgs& A, int s, int p, int head) {
+  return A.carry + ((size_t(s) * A.window + (p - A.first)) * A.heads + head) * delta_chunk_floats(DKP);
+}
+
+// A sum of products a (16 x 16, a row's four values a lane) times b (16 x 16, as an accumulator lies) in four chains, so that 64 terms are added in
+// sixteen steps: in one chain the roundings of the partial sums were most of the error.
+struct Chains {
+  f32x4 v[4] = {};
+  __device__ __forceinline__ void add(float4 a, f32x4 b) {
+    v[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], v[0], 0, 0, 0);
+    v[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], v[1], 0, 0, 0);
+    v[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], v[2], 0, 0, 0);
+    v[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], v[3], 0, 0, 0);
+  }
+  // the transpose of what `add` adds
+  __device__ __forceinline__ void add_turned(float4 a, f32x4 b) {
+    v[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[0], a.x, v[0], 0, 0, 0);
+    v[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[1], a.y, v[1], 0, 0, 0);
+    v[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[2], a.z, v[2], 0, 0, 0);
+    v[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[3], a.w, v[3], 0, 0, 0);
+  }
+  __device__ __forceinline__ f32x4 sum() const { return (v[0] + v[1]) + (v[2] + v[3]); }
+};
+
+constexpr int kDeltaThreads = 512;
+
+template <int DKP>
+__global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkArgs A) {
+  constexpr int C = delta_chunk_rows(DKP), RT = C / 16, KT = DKP / 16, KP = DKP + 4, PP = C + 4, NW = kDeltaThreads / kWave;
+  constexpr int RG = kDeltaThreads / DKP, RPT = C / RG;      // row groups, rows a thread scales
+  constexpr bool kBoth = KT == NW;      // every wave has a column tile of X and one of Y; else half of the waves have either
+  static_assert(kBoth || 2 * KT == NW, "the column tiles are dealt out to eight waves");
+  __shared__ __attribute__((aligned(16))) float Us[C][KP], Rs[C][KP], Ks[C][KP], As[C][KP];
+  __shared__ __attribute__((aligned(16))) float Ps[4][C][PP];      // U A^T, U K^T, R A^T, R K^T
+  __shared__ __attribute__((aligned(16))) float Ds[RT][16][20];      // the inverses of (I + L)'s diagonal blocks
+  __shared__ double tot[RG][DKP];
+  __shared__ __attribute__((aligned(16))) float Wc[DKP];
+  const int head = blockIdx.x, groups = (A.window + A.per_group - 1) / A.per_group;
+  const int s = blockIdx.y / groups, p0 = A.first + blockIdx.y % groups * A.per_group;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, col = lane % 16, g = lane / 16;
+  const int dk = A.dk, dv = A.dv;
+  const int run0 = A.run_start[s], run1 = A.run_start[s + 1], slot = A.state_slots[s];
+  int p1 = p0 + A.per_group < A.first + A.window ? p0 + A.per_group : A.first + A.window;
+  const int all = (run1 - run0 + C - 1) / C;
+  if (p1 > all) p1 = all;
+  if (p0 >= p1) return;
+  if (slot < 0) {      // a padding sequence: its rows carry nothing
+    const int r0 = run0 + p0 * C, r1 = run0 + p1 * C < run1 ? run0 + p1 * C : run1;
+    for (int e = tid; e < (r1 - r0) * dv; e += kDeltaThreads) A.o[size_t(r0 + e / dv) * A.ldo + size_t(head) * dv + e % dv] = 0.f;
+    return;
+  }
+  const size_t D = size_t(A.heads) * dk;
+  const int c = tid % DKP, q = tid / DKP;
+  const bool own = c < dk;
+  const size_t kc = size_t(head) * dk + (own ? c : 0);
+  const bool has_y = kBoth || wave >= KT;
+  const int x0 = (wave % KT) * 16;      // this wave's columns, of X and (or) Y
+  const bool vown = x0 + col < dv;
+  const size_t vc = size_t(head) * dv + (vown ? x0 + col : 0);
+  float wr[RPT], ur[RPT], rr[RPT], kr[RPT], ar[RPT];
+  f32x4 vr[RT];
+  auto request = [&](int p) {      // (rows beyond the run's end are loaded from its last one and masked afterwards)
+    const int r0 = run0 + p * C, n = run1 - r0;
+    if (n >= C) {
+      const size_t row = r0 + q * RPT;
+      const float *wp = A.w + row * D + kc, *up = A.u + row * D + kc, *ap = A.au + row * D + kc, *rp = A.r + row * A.ldr + kc, *kp = A.k + row * A.ldk + kc;
+#pragma unroll
+      for (int m = 0; m < RPT; ++m) {
+        wr[m] = wp[m * D];
+        ur[m] = up[m * D];
+        ar[m] = ap[m * D];
+        rr[m] = rp[size_t(m) * A.ldr];
+        kr[m] = kp[size_t(m) * A.ldk];
+      }
+      const float* vp = A.v + size_t(r0 + g * 4) * A.ldv + vc;
+      if (has_y) {
+#pragma unroll
+        for (int b = 0; b < RT; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) vr[b][i] = vp[size_t(b * 16 + i) * A.ldv];
+      }
+      return;
+    }
+#pragma unroll
+    for (int m = 0; m < RPT; ++m) {
+      const int i = q * RPT + m;
+      const size_t row = r0 + (i < n ? i : n - 1);
+      wr[m] = A.w[row * D + kc];
+      ur[m] = A.u[row * D + kc];
+      ar[m] = A.au[row * D + kc];
+      rr[m] = A.r[row * A.ldr + kc];
+      kr[m] = A.k[row * A.ldk + kc];
+    }
+    if (has_y) {
+#pragma unroll
+      for (int b = 0; b < RT; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = b * 16 + g * 4 + i;
+          vr[b][i] = A.v[size_t(r0 + (j < n ? j : n - 1)) * A.ldv + vc];
+        }
+    }
+  };
+  request(p0);
+  for (int p = p0; p < p1; ++p) {
+    const int r0 = run0 + p * C, n = run1 - r0 < C ? run1 - r0 : C;
+    float* part = delta_chunk_place<DKP>(A, s, p, head);
+    // the rows' products of w, and the scaled rows
+    double cum[RPT], x = 1.0;
+#pragma unroll
+    for (int m = 0; m < RPT; ++m) {
+      x *= own && q * RPT + m < n ? double(wr[m]) : 1.0;
+      cum[m] = x;
+    }
+    tot[q][c] = x;
+    f32x4 vt[RT];
+#pragma unroll
+    for (int b = 0; b < RT; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vt[b][i] = has_y && vown && b * 16 + g * 4 + i < n ? vr[b][i] : 0.f;
+    __syncthreads();      // (the chunk before is done with everything in LDS but this)
+    double entered = 1.0;
+    for (int b = 0; b < q; ++b) entered *= tot[b][c];
+    if (q == RG - 1) Wc[c] = static_cast<float>(entered * x);
+    double before = entered;
+#pragma unroll
+    for (int m = 0; m < RPT; ++m) {
+      const int i = q * RPT + m;
+      const bool in = own && i < n;
+      const double W = entered * cum[m];
+      double inv = __builtin_amdgcn_rcpf(static_cast<float>(W));
+      inv = fma(fma(-W, inv, 1.0), inv, inv);
+      Us[i][c] = in ? static_cast<float>(ur[m] * before) : 0.f;
+      Rs[i][c] = in ? static_cast<float>(rr[m] * W) : 0.f;
+      Ks[i][c] = in ? static_cast<float>(kr[m] * inv) : 0.f;
+      As[i][c] = in ? static_cast<float>(ar[m] * inv) : 0.f;
+      before = W;
+    }
+    if (p + 1 < p1) request(p + 1);      // on its way while this chunk is multiplied
+    __syncthreads();
+    // the four products of rows with rows, the tiles up to the diagonal
+    constexpr int LT = RT * (RT + 1) / 2;
+#pragma unroll 1
+    for (int job = wave; job < 4 * LT; job += NW) {
+      const int m = job % 4, t = job / 4;
+      const int bi = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3, bj = t - bi * (bi + 1) / 2;
+      const float* left = m < 2 ? &Us[bi * 16 + col][g * 4] : &Rs[bi * 16 + col][g * 4];
+      const float* right = m % 2 == 0 ? &As[bj * 16 + col][g * 4] : &Ks[bj * 16 + col][g * 4];
+      Chains sums[2];
+#pragma unroll
+      for (int kk = 0; kk < KT; ++kk) {
+        const float4 a = *reinterpret_cast<const float4*>(left + kk * 16), b = *reinterpret_cast<const float4*>(right + kk * 16);
+        sums[kk % 2].add(a, f32x4{b.x, b.y, b.z, b.w});
+      }
+      const f32x4 acc = sums[0].sum() + sums[1].sum();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = g * 4 + i;
+        Ps[m][bi * 16 + row][bj * 16 + col] = bj < bi || col < row || (col == row && m >= 2) ? acc[i] : 0.f;
+      }
+    }
+    __syncthreads();
+    auto four = [&](int m, int bi, int bj) { return *reinterpret_cast<const float4*>(&Ps[m][bi * 16 + col][bj * 16 + g * 4]); };
+    if (wave < RT) {      // (I + L)^-1 of diagonal block `wave`, a column a lane (every sixteen lanes make the same)
+      float t[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float lrow[16];
+#pragma unroll
+        for (int j = 0; j < 16; j += 4) {
+          const float4 y = *reinterpret_cast<const float4*>(&Ps[0][wave * 16 + i][wave * 16 + j]);
+          lrow[j] = y.x; lrow[j + 1] = y.y; lrow[j + 2] = y.z; lrow[j + 3] = y.w;
+        }
+        float y = i == col ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < i; ++j) y = fmaf(-lrow[j], t[j], y);
+        t[i] = y;
+      }
+      if (g == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Ds[wave][i][col] = t[i];
+      }
+    }
+    f32x4 rhs[RT];
+    if (has_y) {      // lower(U K^T) V
+#pragma unroll
+      for (int b = 0; b < RT; ++b) {
+        Chains sums;
+#pragma unroll
+        for (int a = 0; a <= b; ++a) sums.add(four(1, b, a), vt[a]);
+        rhs[b] = sums.sum();
+      }
+    }
+    __syncthreads();
+    // z = (I + L)^-1 rhs, block by block; left negative, as the products that follow take it
+    auto solve = [&](f32x4 (&z)[RT]) {
+#pragma unroll
+      for (int b = 0; b < RT; ++b) {
+        if (b > 0) {
+          Chains sums;
+#pragma unroll
+          for (int a = 0; a < b; ++a) sums.add(four(0, b, a), z[a]);
+          z[b] += sums.sum();
+        }
+        Chains y;
+        y.add(*reinterpret_cast<const float4*>(&Ds[b][col][g * 4]), z[b]);
+        z[b] = -y.sum();
+      }
+    };
+    auto column = [&](const float (&m)[C][KP], int b, int t) {      // four rows of a key column: the first operand of a product with m^T
+      const float* at = &m[b * 16 + g * 4][t * 16 + col];
+      return float4{at[0], at[KP], at[2 * KP], at[3 * KP]};
+    };
+    // row tile t of this wave's columns of M, N or Q: 16 x 16 as the next launch's lanes take them
+    auto place = [&](float* m, int t) -> float4& { return *reinterpret_cast<float4*>(m + (t * KT + x0 / 16) * 256 + lane * 4); };
+    if (has_y) {
+      solve(rhs);
+      float* N = part + DKP * DKP;
+#pragma unroll 1
+      for (int t = 0; t < KT; ++t) {
+        Chains learnt, lost;
+#pragma unroll
+        for (int b = 0; b < RT; ++b) {
+          learnt.add(column(Ks, b, t), vt[b]);
+          lost.add(column(As, b, t), rhs[b]);
+        }
+        const f32x4 acc = learnt.sum() + lost.sum();
+        const float4 through = *reinterpret_cast<const float4*>(&Wc[t * 16 + g * 4]);
+        place(N, t) = float4{through.x * acc[0], through.y * acc[1], through.z * acc[2], through.w * acc[3]};
+      }
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        Chains learnt, lost;
+#pragma unroll
+        for (int b = 0; b <= t; ++b) {
+          learnt.add(four(3, t, b), vt[b]);
+          lost.add(four(2, t, b), rhs[b]);
+        }
+        const f32x4 acc = learnt.sum() + lost.sum();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (vown && t * 16 + g * 4 + i < n) A.o[size_t(r0 + t * 16 + g * 4 + i) * A.ldo + vc] = acc[i];
+      }
+    }
+    if (kBoth || !has_y) {
+#pragma unroll
+      for (int b = 0; b < RT; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rhs[b][i] = Us[b * 16 + g * 4 + i][x0 + col];
+      solve(rhs);
+#pragma unroll 1
+      for (int t = 0; t < KT; ++t) {
+        Chains sums;
+#pragma unroll
+        for (int b = 0; b < RT; ++b) sums.add_turned(column(As, b, t), rhs[b]);
+        const f32x4 acc = sums.sum();
+        const int key = t * 16 + col, at = x0 + g * 4;
+        const float through = Wc[key];
+        place(part, t) = float4{through * (key == at ? 1.f + acc[0] : acc[0]), through * (key == at + 1 ? 1.f + acc[1] : acc[1]),
+                                through * (key == at + 2 ? 1.f + acc[2] : acc[2]), through * (key == at + 3 ? 1.f + acc[3] : acc[3])};
+      }
+      float* Q = part + 2 * DKP * DKP;
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        Chains sums;
+#pragma unroll
+        for (int b = 0; b <= t; ++b) sums.add_turned(four(2, t, b), rhs[b]);
+        const f32x4 acc = sums.sum();
+        const float4 own = *reinterpret_cast<const float4*>(&Rs[t * 16 + col][x0 + g * 4]);
+        place(Q, t) = float4{own.x + acc[0], own.y + acc[1], own.z + acc[2], own.w + acc[3]};
+      }
+    }
+  }
+}
+
+// The states that enter a run's chunks, one after the other, and the outputs' part of them: a workgroup has 16 value columns of a head, a wave a row
+// tile of M or of Q.  The state lies in LDS, column by column, in two buffers; the chunks' matrices are on their way kAhead chunks before their use.
+template <int DKP>
+__global__ void __launch_bounds__((DKP + delta_chunk_rows(DKP)) / 16 * kWave) delta_pass_kernel(DeltaChunkArgs A) {
+  constexpr int C = delta_chunk_rows(DKP), KT = DKP / 16, SP = DKP + 4, NT = (DKP + C) / 16 * kWave, kAhead = DKP == 64 ? 4 : 2;
+  __shared__ __attribute__((aligned(16))) float Ss[2][16][SP];
+  int head, c0;
+  head_and_columns(A.heads, A.col_blocks, head, c0);      // (a head's workgroups on one XCD: they read the same M and Q)
+  c0 *= 16;
+  const int s = blockIdx.y;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, col = lane % 16, g = lane / 16;
+  const int dk = A.dk, dv = A.dv;
+  const int run0 = A.run_start[s], run1 = A.run_start[s + 1], slot = A.state_slots[s];
+  if (run1 - run0 <= A.first * C || slot < 0) return;
+  const int all = (run1 - run0 + C - 1) / C, end = A.first + A.window < all ? A.first + A.window : all;
+  float* home = A.state + (size_t(slot) * A.heads + head) * dk * dv;
+  const bool fresh = A.first == 0 && A.seq_start[s] == 0;
+  for (int e = tid; e < DKP * 16; e += NT) {
+    const int key = e / 16, cc = e % 16;
+    Ss[0][cc][key] = !fresh && key < dk && c0 + cc < dv ? home[size_t(key) * dv + c0 + cc] : 0.f;
+  }
+  const bool keeps = wave < KT;      // a row tile of M, or of Q
+  const int tile = keeps ? wave : wave - KT;
+  const bool cown = c0 + col < dv;
+  const size_t oc = size_t(head) * dv + (cown ? c0 + col : 0);
+  float4 m[kAhead][KT];
+  f32x4 add[kAhead];
+  auto request = [&](int p, int into) {
+    const float* part = delta_chunk_place<DKP>(A, s, p, head);
+    const float* rows = (keeps ? part : part + 2 * DKP * DKP) + tile * KT * 256 + lane * 4;
+#pragma unroll
+    for (int kk = 0; kk < KT; ++kk) m[into][kk] = *reinterpret_cast<const float4*>(rows + kk * 256);
+    const int r0 = run0 + p * C, n = run1 - r0;
+    if (keeps) {
+      const float4 x = *reinterpret_cast<const float4*>(part + DKP * DKP + (tile * KT + c0 / 16) * 256 + lane * 4);
+      add[into] = f32x4{x.x, x.y, x.z, x.w};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = tile * 16 + g * 4 + i;
+        add[into][i] = A.o[size_t(r0 + (row < n ? row : n - 1)) * A.ldo + oc];
+      }
+    }
+  };
+#pragma unroll
+  for (int a = 0; a < kAhead; ++a)
+    if (A.first + a < end) request(A.first + a, a);
+  int at = 0;
+  __syncthreads();
+  for (int pb = A.first; pb < end; pb += kAhead) {
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) {
+      const int p = pb + a;
+      if (p >= end) break;
+      Chains sums[2];
+#pragma unroll
+      for (int kk = 0; kk < KT; ++kk) {
+        const float4 b = *reinterpret_cast<const float4*>(&Ss[at][col][kk * 16 + g * 4]);
+        sums[kk % 2].add(m[a][kk], f32x4{b.x, b.y, b.z, b.w});
+      }
+      const f32x4 acc = add[a] + (sums[0].sum() + sums[1].sum());
+      if (p + kAhead < end) request(p + kAhead, a);
+      if (keeps) {
+        *reinterpret_cast<float4*>(&Ss[at ^ 1][col][tile * 16 + g * 4]) = float4{acc[0], acc[1], acc[2], acc[3]};
+      } else {
+        const int r0 = run0 + p * C, n = run1 - r0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (cown && tile * 16 + g * 4 + i < n) A.o[size_t(r0 + tile * 16 + g * 4 + i) * A.ldo + oc] = acc[i];
+      }
+      at ^= 1;
+      __syncthreads();
+    }
+  }
+  for (int e = tid; e < DKP * 16; e += NT) {
+    const int key = e / 16, cc = e % 16;
+    if (key < dk && c0 + cc < dv) home[size_t(key) * dv + c0 + cc] = Ss[at][cc][key];
+  }
+}
+
+template <int DKP>
+static int launch_delta_chunks(DeltaChunkArgs A, int S, int T, int max_run, long long carry_floats, hipStream_t s) {
+  constexpr int C = delta_chunk_rows(DKP);
+  const int chunks = (max_run + C - 1) / C;
+  const long long column = static_cast<long long>(S) * A.heads * delta_chunk_floats(DKP);      // one chunk of every sequence
+  const long long fit = carry_floats / column;
+  KVCM_REQUIRE(fit >= 1, "delta_chunks: the scratch is too small");
+  A.window = static_cast<int>(fit < chunks ? fit : chunks);
+  // one workgroup a CU: some chunks in a row, whose rows are asked for while the one before is multiplied, once there is more than one a CU
+  const long long most = static_cast<long long>(S) * A.window, rows = T / C + S;      // (chunks of this many rows, a part of one in every sequence)
+  const long long turns = (A.heads * (most < rows ? most : rows) + 255) / 256;
+  A.per_group = static_cast<int>(turns < 8 ? turns : 8);
+  const long long groups = static_cast<long long>(S) * ((A.window + A.per_group - 1) / A.per_group);
+  KVCM_REQUIRE(groups <= 65535, "delta_chunks: too many sequences and chunks for one launch");
+  for (A.first = 0; A.first < chunks; A.first += A.window) {
+    delta_chunk_kernel<DKP><<<dim3(A.heads, static_cast<unsigned>(groups)), kDeltaThreads, 0, s>>>(A);
+    delta_pass_kernel<DKP><<<dim3(A.heads * A.col_blocks, S), (DKP + C) / 16 * kWave, 0, s>>>(A);
+  }
+  return launch_status("delta_chunks");
+}
+
+}  // namespace kvcm
+
+using namespace kvcm;
+
+extern "C" {
+
+// floats of scratch that a step of S sequences and runs of up to max_run rows takes at once (with less, down to a chunk of every sequence, it goes in turns)
+long long kvcm_delta_carry_floats(int S, int max_run, int heads, int dk) {
+  if (S <= 0 || max_run <= 0 || heads <= 0) return 0;
+  const int dkp = dk <= 64 ? 64 : 128, rows = delta_chunk_rows(dkp);
+  return static_cast<long long>(S) * ((max_run + rows - 1) / rows) * heads * delta_chunk_floats(dkp);
+}
+
+// As kvcm_delta_scan (all operands alike), in matrix form, for key sizes up to 128, values no larger than the keys' tile (64 or 128), and w no smaller
+// than exp(-exp(-1/2)), as kvcm_delta_prepare makes it.
+int kvcm_delta_chunks(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* w, const float* au, const float* u,
+                      float* o, int ldo, float* state, const int* run_start, const int* seq_start, const int* state_slots, int S, int heads,
+                      int dk, int dv, int T, int max_run, float* carry, long long carry_floats, hipStream_t s) {
+  if (S == 0) return 0;
+  KVCM_REQUIRE(S > 0 && heads > 0 && dk > 0 && dv > 0 && T > 0 && max_run > 0, "delta_chunks: bad sizes S=%d heads=%d dk=%d dv=%d", S, heads, dk, dv);
+  KVCM_REQUIRE(dk <= 128 && dv <= (dk <= 64 ? 64 : 128), "delta_chunks: heads of %d x %d are not supported", dk, dv);
+  KVCM_REQUIRE(S <= 65535 && heads <= (1 << 20), "delta_chunks: too many sequences or heads for one launch");
+  KVCM_REQUIRE(ldr >= heads * dk && ldk >= heads * dk && ldv >= heads * dv && ldo >= heads * dv, "delta_chunks: row strides too small");
+  KVCM_REQUIRE(carry && reinterpret_cast<uintptr_t>(carry) % 16 == 0, "delta_chunks: the scratch must be there, 16-byte aligned");
+  DeltaChunkArgs A = {r, k, v, w, au, u, ldr, ldk, ldv, o, ldo, state, run_start, seq_start, state_slots, heads, dk, dv, (dv + 15) / 16, carry, 0, 0, 0};
+  if (dk <= 64) return launch_delta_chunks<64>(A, S, T, max_run, carry_floats, s);
+  return launch_delta_chunks<128>(A, S, T, max_run, carry_floats, s);
+}
+
+}  // extern "C"

@@ -15,7 +15,7 @@
 // chain of dependent instructions, so a wave has few columns, its key dimension over up to 16 lanes, and a workgroup is one
 // wave: nothing is shared and nobody waits.  The per-token vectors (r, k, w, a*u, u, v) go from L2 into the lanes that use
 // them, a few tokens ahead.  A run that starts at position 0 starts from zero without reading its slot.  Tokens are taken one
-// by one in prompts and in decoding.
+// by one in prompts and in decoding; delta_chunks.hip takes long runs in matrix form.
 #include "common.h"
 #include "kvcm_hip.h"
 

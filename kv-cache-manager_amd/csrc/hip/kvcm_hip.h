@@ -248,6 +248,11 @@ int kvcm_delta_prepare(const float* k, int ldk, const float* a_lin, int lda, con
 int kvcm_delta_scan(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* w, const float* au,
                     const float* u, float* o, int ldo, float* state, const int* run_start, const int* seq_start,
                     const int* state_slots, int S, int heads, int dk, int dv, int max_run, int one_order, hipStream_t s);
+// (delta_chunks.hip) the same in matrix form, for long runs
+long long kvcm_delta_carry_floats(int S, int max_run, int heads, int dk);
+int kvcm_delta_chunks(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* w, const float* au, const float* u,
+                      float* o, int ldo, float* state, const int* run_start, const int* seq_start, const int* state_slots, int S, int heads,
+                      int dk, int dv, int T, int max_run, float* carry, long long carry_floats, hipStream_t s);
 
 // (stream_norms.hip) a norm without statistics beside the residual additions of a layer whose mixer and feed-forward run
 // side by side; the stream packed with the embedding for a product; a factor on logits; a gate per head; small norms in place

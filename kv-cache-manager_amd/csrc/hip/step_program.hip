@@ -134,6 +134,7 @@ const Entry kEntries[] = {
     KVCM_ENTRY(kvcm_scan_prepare),
     KVCM_ENTRY(kvcm_delta_prepare),
     KVCM_ENTRY(kvcm_delta_scan),
+    KVCM_ENTRY(kvcm_delta_chunks),
     KVCM_ENTRY(kvcm_layernorm_post),
     KVCM_ENTRY(kvcm_head_norm_store),
     KVCM_ENTRY(kvcm_gemm_heads),

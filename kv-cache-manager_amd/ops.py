@@ -166,6 +166,9 @@ def _declare(lib):
     fn("kvcm_scan_prepare", vp, i, vp, vp, i, i, i, vp)
     fn("kvcm_delta_prepare", vp, i, vp, i, vp, vp, i, vp, i, vp, vp, vp, vp, i, i, i, vp)
     fn("kvcm_delta_scan", vp, i, vp, i, vp, i, vp, vp, vp, vp, i, vp, vp, vp, vp, i, i, i, i, i, i, vp)
+    fn("kvcm_delta_chunks", vp, i, vp, i, vp, i, vp, vp, vp, vp, i, vp, vp, vp, vp, i, i, i, i, i, i, vp, C.c_longlong, vp)
+    lib.kvcm_delta_carry_floats.restype = C.c_longlong
+    lib.kvcm_delta_carry_floats.argtypes = [i] * 4
     lib.kvcm_gemm_library_workspace_bytes.restype = C.c_longlong
     lib.kvcm_gemm_library_workspace_bytes.argtypes = []
     lib.kvcm_program_new.restype = vp
@@ -1754,15 +1757,43 @@ def delta_prepare(k, a_lin, a_bias, low, w2t, w0, w_out, au_out, u_out, heads, d
           _ptr(w2t), rank, _ptr(w0), _ptr(w_out), _ptr(au_out), _ptr(u_out), rows, heads, d, _stream())
 
 
-def delta_scan(r, k, v, w, au, u, o, state, step, heads, dk, dv, one_order=False):
+DELTA_CARRY = 9 << 22        # 32-bit values of scratch that ``delta_scan``'s matrix form asks for at most (1,024 chunks of a head of 128); the rest goes in turns
+
+
+def delta_in_chunks(step, heads, dk, dv, one_order=False):
+    """Does ``delta_scan``, given scratch for the chunks, take this step's runs in matrix form (csrc/hip/delta_chunks.hip)?  It is worth it
+    where the walk waits for its own chain, and while runs are of similar lengths (every sequence has the longest's scratch and a whole
+    chunk at least).  us, walk / so: 32 heads of 64 x 64, one run of 128 rows 22 / 25, 192 30 / 26, 512 72 / 36, 2,048 293 / 120, 3 of 1,024
+    314 / 187, 8 of 128 56 / 61, 8 of 509 208 / 210, one of 1,024 beside 7 single tokens 272 / 321; 32 heads of 128 x 128, one run of 128 rows
+    46 / 34, 2,048 689 / 323, 4 of 1,024 1,311 / 647, 8 of 256 608 / 349."""
+    if (one_order or not 32 < dk <= 128 or dv > (64 if dk <= 64 else 128) or 2 * step.rows < step.seqs * step.max_run
+            or int(lib().kvcm_delta_carry_floats(step.seqs, 1, heads, dk)) > DELTA_CARRY):
+        return False
+    return step.max_run >= 128 if dk > 64 else step.max_run >= 192 and step.rows * heads <= 96 * step.max_run
+
+
+def delta_carry_floats(rows, seqs, heads, dk):
+    """32-bit values of scratch that ``delta_scan`` takes for steps of up to this shape in matrix form."""
+    return min(DELTA_CARRY, int(lib().kvcm_delta_carry_floats(1, rows, heads, dk)) + int(lib().kvcm_delta_carry_floats(seqs, 1, heads, dk)))
+
+
+def delta_scan(r, k, v, w, au, u, o, state, step, heads, dk, dv, one_order=False, carry=None):
     """The delta-rule recurrence over the step's runs (csrc/hip/delta_rule.hip); state [slots, heads, dk, dv].  ``one_order``: a
-    row's sums are taken in one order whatever else the step holds (32-bit storage), not in the one that is fastest for its runs."""
+    row's sums are taken in one order whatever else the step holds (32-bit storage), not in the one that is fastest for its runs.
+    ``carry`` (float32 scratch of ``delta_carry_floats``; w from ``delta_prepare``, whose w is never under exp(-exp(-1/2))): steps with long
+    runs (``delta_in_chunks``) take them in matrix form."""
     for t, n, c in ((r, "r", heads * dk), (k, "k", heads * dk), (v, "v", heads * dv), (o, "o", heads * dv)):
         _f32rows(t, n, c)
     for t, n in ((w, "w"), (au, "au"), (u, "u")):
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.is_cuda and t.shape[1] == heads * dk, f"{n} must be contiguous float32")
     _need(state.dtype == torch.float32 and state.is_contiguous() and state.is_cuda and tuple(state.shape[1:]) == (heads, dk, dv),
           "state must be float32 [slots, heads, dk, dv]")
+    if carry is not None and delta_in_chunks(step, heads, dk, dv, one_order):
+        _f32(carry, "carry")
+        _call("kvcm_delta_chunks", _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w), _ptr(au), _ptr(u),
+              _ptr(o), o.stride(0), _ptr(state), _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs,
+              heads, dk, dv, o.shape[0], int(step.max_run), _ptr(carry), carry.numel(), _stream())
+        return o
     _call("kvcm_delta_scan", _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w), _ptr(au), _ptr(u),
           _ptr(o), o.stride(0), _ptr(state), _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs,
           heads, dk, dv, int(getattr(step, "max_run", o.shape[0])), int(one_order), _stream())

@@ -135,7 +135,11 @@ class GeneralDeltaMixer(_StatefulMixer):
         ops.delta_prepare(k, a, w["a_bias"], low, w["w2"], w["w0"], decay, au, u, heads, d, T)
         o = step.ws("delta_o", (T, D), torch.float32)
         gated = step.ws("delta_gated", (T, D))
-        ops.delta_scan(r, k, v, decay, au, u, o, self.state("delta"), step, heads, d, d, one_order=gated.dtype == torch.float32)
+        one_order, carry, lim = gated.dtype == torch.float32, None, step.limits
+        if ops.delta_in_chunks(step, heads, d, d, one_order):      # (sized for the engine's largest step)
+            carry = step.flat("delta_carry", ops.delta_carry_floats(max(T, lim.max_tokens if lim else 0), max(step.seqs, lim.max_seqs if lim else 0),
+                                                                    heads, d))
+        ops.delta_scan(r, k, v, decay, au, u, o, self.state("delta"), step, heads, d, d, one_order=one_order, carry=carry)
         ops.head_norm_gate(o, g, w["norm"], gated, heads, d, p["eps"])
         return linear32(self.ctx, step, gated, w["w_o"], "delta_out")
 

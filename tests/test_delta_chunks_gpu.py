@@ -1,0 +1,67 @@
+"""The delta rule in matrix form (csrc/hip/delta_chunks.hip) against the plain recurrence: chunks of 64 and 32 rows that end anywhere, runs that
+begin in the middle of a sequence, heads that end inside a tile, rows that begin at any float, dead slots, scratch for a part of a run."""
+import numpy as np
+import pytest
+import torch
+
+import plain_kasuvik as plain
+from test_kasuvik_gpu import Step, dev
+
+DEV = "cuda:0"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("turns", [False, True])
+@pytest.mark.parametrize("d,dv,shift", [(64, 64, 0), (64, 50, 1), (33, 64, 1), (60, 20, 0), (128, 128, 0), (100, 17, 1), (65, 128, 0)])
+def test_long_runs_against_the_plain_recurrence(d, dv, shift, turns, monkeypatch):
+    from kvcm_amd import ops
+    monkeypatch.setattr(ops, "delta_in_chunks", lambda *a: True)
+    rng = np.random.default_rng(d + dv)
+    heads, parts = 2, ((256, 1, 129, 64), (63, 321, 128, 7), (257, 192, 1, 385))
+    seqs, D = len(parts[0]), 2 * d
+    lowest = np.exp(-np.exp(-0.5))
+    data = []
+    for n in (sum(x[i] for x in parts) for i in range(seqs)):
+        q = {"r": rng.normal(size=(n, heads, d)), "k": rng.normal(size=(n, heads, d)), "v": rng.normal(size=(n, heads, dv)),
+             "w": np.where(rng.random((n, heads, d)) < 0.3, lowest, rng.uniform(lowest, 1.0, size=(n, heads, d))), "a": rng.uniform(0, 1, size=(n, heads, d))}
+        q["w"][:, 1, ::2] = lowest ** rng.uniform(0, 0.02, size=(n, heads, d))[:, 1, ::2]      # (channels that keep for long beside some that forget at once)
+        q["u"] = q["k"] / np.sqrt((q["k"] ** 2).sum(-1, keepdims=True) + 1e-6)
+        data.append(q)
+    want = [plain.delta_rule(q["r"], q["k"], q["v"], q["w"], q["a"]) for q in data]
+    S, at = torch.full((seqs, heads, d, dv), 9.0, device=DEV), [0] * seqs
+    for part in parts:
+        st = Step([(i, at[i], n) for i, n in enumerate(part)] + [(0, 5, 140)])
+        st.max_run = max(part)
+        st.state_slots[-1] = -1      # a padding sequence beside them
+        cat = lambda f, c: dev(np.concatenate([f(q)[at[i]:at[i] + n].reshape(n, -1) for i, (q, n) in enumerate(zip(data, part))] + [rng.uniform(0.6, 1, (140, c))]))
+        r, k, v = (cat(lambda q, x=x: q[x], c) for x, c in (("r", D), ("k", D), ("v", heads * dv)))
+        packed = torch.full((st.rows, 2 * D + heads * dv + 2 + shift), float("nan"), device=DEV)[:, shift:]
+        packed[:, :D], packed[:, D:2 * D], packed[:, 2 * D:2 * D + heads * dv] = r, k, v
+        w, au, u = cat(lambda q: q["w"], D), cat(lambda q: q["a"] * q["u"], D), cat(lambda q: q["u"], D)
+        one = int(ops.lib().kvcm_delta_carry_floats(st.seqs, 1, heads, d))
+        carry = torch.full((3 * one if turns else ops.delta_carry_floats(st.rows, st.seqs, heads, d),), float("nan"), device=DEV)
+        o = torch.full((st.rows, heads * dv + shift), float("nan"), device=DEV)
+        ops.delta_scan(packed, packed[:, D:], packed[:, 2 * D:], w, au, u, o, S, st, heads, d, dv, carry=carry)
+        row, got = 0, o[:, :heads * dv].double().cpu().numpy()
+        for i, n in enumerate(part):
+            ref = want[i][at[i]:at[i] + n].reshape(n, -1)
+            # as the walk's: sums of up to 128 keys a row, handed on by a state that forgets
+            np.testing.assert_allclose(got[row:row + n], ref, atol=5e-5 * max(1.0, np.abs(ref).max()), err_msg=f"sequence {i} from {at[i]}")
+            row, at[i] = row + n, at[i] + n
+        assert not got[row:].any()
+
+
+@pytest.mark.gpu
+def test_the_line_between_the_forms():
+    from kvcm_amd import ops
+    def step(*runs):
+        st = Step([(i, 0, n) for i, n in enumerate(runs)])
+        st.max_run = max(runs)
+        return st
+    assert ops.delta_in_chunks(step(192), 4, 64, 64) and not ops.delta_in_chunks(step(191), 4, 64, 64)
+    assert ops.delta_in_chunks(step(128), 4, 65, 128) and not ops.delta_in_chunks(step(127), 4, 65, 128)
+    assert ops.delta_in_chunks(step(192, 192, 192), 32, 64, 64) and not ops.delta_in_chunks(step(192, 192, 192), 33, 64, 64)
+    for heads, d, dv, takes in ((4, 128, 128, True), (4, 129, 64, False), (4, 32, 32, False), (4, 33, 64, True), (4, 64, 65, False), (1 << 17, 128, 64, False)):
+        assert ops.delta_in_chunks(step(200), heads, d, dv) == takes
+    assert not ops.delta_in_chunks(step(200), 4, 64, 64, True)
+    assert ops.delta_in_chunks(step(200, 1), 4, 64, 64) and not ops.delta_in_chunks(step(200, 1, 1), 4, 64, 64)      # (runs of similar lengths)
