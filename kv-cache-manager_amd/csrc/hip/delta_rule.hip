@@ -21,41 +21,74 @@
 
 namespace kvcm {
 
-// one wave per (row, head).  The decay's logit is a two-step projection whose second step runs here in 32-bit:
-// w_lin[c] = sum_j w2[c, j] * tanh(low[j]), low = the first step's output (rank values a row); w2 comes transposed,
-// [rank, heads*d].
-constexpr int kDeltaMaxRank = 256;
+// A wave makes R rows of a head, a workgroup of four those of four heads.  The decay's logit is a two-step projection whose second step
+// runs here in 32-bit: w_lin[c] = sum_j w2[c, j] * tanh(low[j]), low = the first step's output (rank values a row), tanh once for the
+// workgroup's heads; w2 comes transposed, [rank, heads*d], sixteen of a channel's values on their way together: one at a time a
+// step of few rows was a chain of `rank` trips to L2.  us, a wave of its own for every row and head /
+// so, rank 64, 32 heads of 64: 8 rows 5.2 / 4.2, 2,048 rows 66 / 44; of 128 7.4 / 5.6 and 115 / 77 (its bits are the same either way).
+constexpr int kDeltaMaxRank = 256, kDeltaRows = 8;
+template <int R>
 __global__ void __launch_bounds__(256)
     delta_prepare_kernel(const float* __restrict__ k, int ldk, const float* __restrict__ a_lin, int lda,
                          const float* __restrict__ a_bias, const float* __restrict__ low, int ldlow,
                          const float* __restrict__ w2t, int rank, const float* __restrict__ w0,
-                         float* __restrict__ w_out, float* __restrict__ au_out, float* __restrict__ u_out, long long items,
-                         int heads, int d) {
-  __shared__ float th[256 / kWave][kDeltaMaxRank];
+                         float* __restrict__ w_out, float* __restrict__ au_out, float* __restrict__ u_out, int heads, int d, int T) {
+  constexpr int kWaves = 256 / kWave, kAhead = 16;
+  __shared__ __attribute__((aligned(16))) float th[kDeltaMaxRank][R];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const long long item = static_cast<long long>(blockIdx.x) * (256 / kWave) + wave;
-  const bool active = item < items;
-  const int row = active ? static_cast<int>(item / heads) : 0, head = active ? static_cast<int>(item % heads) : 0;
-  if (active)
-    for (int j = lane; j < rank; j += kWave) th[wave][j] = tanhf(low[size_t(row) * ldlow + j]);
+  const int row0 = blockIdx.x * R, head = blockIdx.y * kWaves + wave;
+  auto row_of = [&](int n) { return size_t(row0 + n < T ? row0 + n : T - 1); };      // (rows beyond the last are left out of the stores)
+  if constexpr (R == 1) {
+    for (int j = threadIdx.x; j < rank; j += 256) th[j][0] = tanhf(low[row_of(0) * ldlow + j]);
+  } else {
+    for (int n = wave; n < R; n += kWaves)
+      for (int j = lane; j < rank; j += kWave) th[j][n] = tanhf(low[row_of(n) * ldlow + j]);
+  }
   __syncthreads();
-  if (!active) return;
+  if (head >= heads) return;
   const size_t col = size_t(head) * d, D = size_t(heads) * d;
-  const float* kr = k + size_t(row) * ldk + col;
-  float ss = 0.f;
-  for (int i = lane; i < d; i += kWave) ss = fmaf(kr[i], kr[i], ss);
-  ss = wave_sum(ss);
-  const float inv = 1.0f / sqrtf(ss + 1e-6f);
+  float inv[R];
+#pragma unroll
+  for (int n = 0; n < R; ++n) {
+    const float* kr = k + row_of(n) * ldk + col;
+    float ss = 0.f;
+    for (int i = lane; i < d; i += kWave) ss = fmaf(kr[i], kr[i], ss);
+    inv[n] = 1.0f / sqrtf(wave_sum(ss) + 1e-6f);
+  }
   const float rate = 0.60653065971263342f;      // exp(-1/2)
   for (int i = lane; i < d; i += kWave) {
-    const float u = kr[i] * inv;
-    const float a = 1.0f / (1.0f + expf(-(a_lin[size_t(row) * lda + col + i] + a_bias[col + i])));
-    float wl = 0.f;
-    for (int j = 0; j < rank; ++j) wl = fmaf(w2t[size_t(j) * D + col + i], th[wave][j], wl);      // neighbours read neighbours
-    const float g = 1.0f / (1.0f + expf(-(wl + w0[col + i])));
-    w_out[size_t(row) * D + col + i] = expf(-rate * g);
-    au_out[size_t(row) * D + col + i] = a * u;
-    u_out[size_t(row) * D + col + i] = u;
+    const float* w2 = w2t + col + i;      // neighbours read neighbours
+    float wl[R] = {}, kx[R], ax[R];
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      kx[n] = k[row_of(n) * ldk + col + i];
+      ax[n] = a_lin[row_of(n) * lda + col + i];
+    }
+    int j = 0;
+    for (; j + kAhead <= rank; j += kAhead) {
+      float x[kAhead];
+#pragma unroll
+      for (int m = 0; m < kAhead; ++m) x[m] = w2[size_t(j + m) * D];
+#pragma unroll
+      for (int m = 0; m < kAhead; ++m)
+#pragma unroll
+        for (int n = 0; n < R; ++n) wl[n] = fmaf(x[m], th[j + m][n], wl[n]);
+    }
+    for (; j < rank; ++j)
+#pragma unroll
+      for (int n = 0; n < R; ++n) wl[n] = fmaf(w2[size_t(j) * D], th[j][n], wl[n]);
+    const float ab = a_bias[col + i], wb = w0[col + i];
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const float u = kx[n] * inv[n];
+      const float a = 1.0f / (1.0f + expf(-(ax[n] + ab)));
+      const float g = 1.0f / (1.0f + expf(-(wl[n] + wb)));
+      if (row0 + n >= T) break;
+      const size_t at = size_t(row0 + n) * D + col + i;
+      w_out[at] = expf(-rate * g);
+      au_out[at] = a * u;
+      u_out[at] = u;
+    }
   }
 }
 
@@ -212,11 +245,14 @@ int kvcm_delta_prepare(const float* k, int ldk, const float* a_lin, int lda, con
   KVCM_REQUIRE(T > 0 && heads > 0 && d > 0, "delta_prepare: bad sizes T=%d heads=%d d=%d", T, heads, d);
   KVCM_REQUIRE(rank > 0 && rank <= kDeltaMaxRank, "delta_prepare: a rank of %d is not supported (1 to %d)", rank, kDeltaMaxRank);
   KVCM_REQUIRE(ldk >= heads * d && lda >= heads * d && ldlow >= rank, "delta_prepare: row strides too small");
-  const long long items = static_cast<long long>(T) * heads;
-  const long long blocks = (items + 3) / 4;
-  KVCM_REQUIRE(blocks < (1ll << 31), "delta_prepare: too many rows");
-  delta_prepare_kernel<<<static_cast<unsigned>(blocks), 256, 0, s>>>(k, ldk, a_lin, lda, a_bias, low, ldlow, w2t, rank, w0, w_out,
-                                                                     au_out, u_out, items, heads, d);
+  const unsigned groups = (heads + 3) / 4;
+  KVCM_REQUIRE(groups <= 65535, "delta_prepare: too many heads");
+  // (a row a wave while eight would leave CUs without work, and where w2 is read soon anyway)
+  if (static_cast<long long>(T) * groups < 256 * kDeltaRows || rank < 16)
+    delta_prepare_kernel<1><<<dim3(T, groups), 256, 0, s>>>(k, ldk, a_lin, lda, a_bias, low, ldlow, w2t, rank, w0, w_out, au_out, u_out, heads, d, T);
+  else
+    delta_prepare_kernel<kDeltaRows><<<dim3((T + kDeltaRows - 1) / kDeltaRows, groups), 256, 0, s>>>(
+        k, ldk, a_lin, lda, a_bias, low, ldlow, w2t, rank, w0, w_out, au_out, u_out, heads, d, T);
   return launch_status("delta_prepare");
 }
 
