@@ -398,7 +398,7 @@ int launch_scan(const void* x, int ldx, float* dt_lin, int lddt, const float* dt
 #undef KVCM_SCAN_SINGLE
     return launch_status("selective_scan");
   }
-  if (phase != 0 && scan_by_channels(std::is_same<X, float>::value, T, C, N)) {
+  if (phase != 0 && !prepared && scan_by_channels(std::is_same<X, float>::value, T, C, N)) {
     const dim3 grid((C + 255) / 256, S, pieces);
 #define KVCM_SCAN_CHANNELS(N, OUT)                                                                                            \
   scan_channels_kernel<X, N, OUT><<<grid, 256, 0, s>>>(static_cast<const X*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b,   \
@@ -436,8 +436,8 @@ using namespace kvcm;
 // (B at off_b, C at off_c, N each), z [T, ldz], a_log [C, N], dt_bias, dskip [C], state [slots, C, N]: 32-bit.
 // prepared: dt_lin holds the step sizes and z the gates already (kvcm_scan_prepare).
 // chunk_len > 0: runs (of up to max_run rows, T rows in all) are walked in pieces of chunk_len rows, all pieces at once, with
-// carry (at least (T / chunk_len + S + 1) * C * (N + 1) floats) between the phases; dt_lin (and z) hold step sizes (and gates)
-// afterwards; 0: every run in one walk.
+// carry (at least (T / chunk_len + S + 1) * C * (N + 1) floats) between the phases; what is not prepared is then made here, dt_lin (and
+// z, where the states lie over lanes) hold it afterwards; 0: every run in one walk.
 extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, float* dt_lin, int lddt, const float* dt_bias,
                                    const float* bc, int ldbc, int off_b, int off_c, const float* a_log, const float* dskip,
                                    float* z, int ldz, void* out, int ldo, float* state, const int* run_start,
@@ -459,13 +459,12 @@ extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, float* dt_
   };
   if (chunk_len <= 0) return launch(0, 1, nullptr, nullptr);
   // long runs in pieces of chunk_len rows: every piece from zero, the states that enter the pieces, every piece again
-  KVCM_REQUIRE(!prepared, "selective_scan: runs that are cut into pieces take their step sizes as they are projected");
   const int pieces = (max_run + chunk_len - 1) / chunk_len;
   const long long slots = static_cast<long long>(T) / chunk_len + S + 1;      // piece j of sequence s: run_start / chunk_len + s + j
   KVCM_REQUIRE(pieces >= 1 && pieces <= 65535 && carry != nullptr && carry_floats >= slots * C * (N + 1),
                "selective_scan: the scratch for %lld pieces is too small", slots);
   float* dsum = carry + slots * C * N;
-  if (!scan_by_channels(dtype == kF32, T, C, N)) {
+  if (!prepared && !scan_by_channels(dtype == kF32, T, C, N)) {
     if (int rc = prepare_scan(dt_lin, lddt, dt_bias, z, ldz, T, C, s)) return rc;
     prepared = 1;
   }
