@@ -44,6 +44,34 @@ def test_pieces_against_the_plain_recurrence(C, N, piece, monkeypatch):
         assert not bool(out[row:].any())
 
 
+@pytest.mark.gpu
+def test_step_sizes_and_gates_that_are_made_already(monkeypatch):
+    """The entry point with prepared rows and pieces: what it makes itself, within the result's own rounding."""
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(3)
+    T, C, N = 300, 1800, 16
+    x, z, dt = (torch.randn(T, C, generator=g).to(DEV) for _ in range(3))
+    bc, a_log, dsk, db = (torch.randn(*n, generator=g).to(DEV) for n in ((T, 2 * N), (C, N), (C,), (C,)))
+    step, call = Step([(0, 0, T)]), ops._call
+    step.max_run = T
+    got = []
+    for made in (False, True):
+        def entry(name, *args, made=made):
+            args = list(args)
+            if name == "kvcm_selective_scan":
+                if made:
+                    call("kvcm_scan_prepare", *args[3:6], *args[12:14], T, C, args[-1])
+                args[23] = int(made)
+            return call(name, *args)
+        monkeypatch.setattr(ops, "_call", entry)
+        out, state = torch.empty(T, C, dtype=torch.bfloat16, device=DEV), torch.zeros(1, C, N, device=DEV)
+        carry = torch.empty(ops.selective_scan_carry_floats(T, 1, C, N), device=DEV)
+        ops.selective_scan(x.bfloat16(), dt.clone(), db, bc, 0, N, a_log, dsk, z.clone(), out, state, step, prepare=True, carry=carry)
+        got.append((out.float(), state))
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=0, atol=2.0 ** -8 * float(b.abs().max()))
+
+
 def test_the_scratch_holds_the_pieces_of_every_smaller_step():
     from kvcm_amd import ops
     for C, N, seqs, most in ((4096, 16, 3, 32768), (8192, 16, 1, 5000), (64, 8, 9, 40000), (1, 8, 1, 100), (600000, 8, 1, 700)):
