@@ -326,6 +326,7 @@ __global__ void __launch_bounds__(WM* WN* kWave)
 // (columns, after the sizes and waves: the stages, and whether the tile is tile_pipe.h's)
 struct Tile {
   int bm, bn;
+  bool pipe;
   float fixed, step, share, round;
 };
 #define KVCM_TILES(T)                                                                                                             \
@@ -347,7 +348,7 @@ struct Tile {
   T(256, 192, 2, 2, 2, true, 6.172f, 0.944f, 1.065f, 7.188f)                                                                      \
   T(256, 256, 2, 2, 2, true, 8.118f, 1.175f, 1.013f, 8.000f)
 
-#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, FIXED, STEP, SHARE, ROUND},
+#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, PIPE, FIXED, STEP, SHARE, ROUND},
 static constexpr Tile kTiles[] = {KVCM_TILES(KVCM_TILE_ROW)};
 #undef KVCM_TILE_ROW
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
@@ -369,10 +370,12 @@ float gemm_tile_time(int bm, int bn, float groups, int steps, float weights) {
   return 1e30f;
 }
 
-static int best_tile(int M, int wrows, int K, int S, float* time = nullptr) {
+// folded: rows whose norm is still to be applied, which the tiles of tile_pipe.h do not take
+static int best_tile(int M, int wrows, int K, int S, float* time = nullptr, bool folded = false) {
   int best = 0;
   float best_t = 0.f;
   for (int i = 0; i < kTileCount; ++i) {
+    if (folded && kTiles[i].pipe) continue;
     if (kTiles[i].bm > 16 && kTiles[i].bm >= 2 * M) continue;      // more than half of the rows would not exist
     const float groups = static_cast<float>(static_cast<long long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((wrows + kTiles[i].bn - 1) / kTiles[i].bn) * S);
     const float t = tile_time(kTiles[i], groups, (K / kStepK + S - 1) / S, static_cast<float>(wrows) * static_cast<float>(K));
@@ -430,7 +433,7 @@ int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st) {
   // (rows of 8 MB or that far apart: one tile for all sizes; what such a product takes is its bytes)
   if (c.ldx >= kFarRows || c.ldw >= kFarRows)
     return is_gated ? launch_tiles<64, 64, 2, 2, 4, true, uint64_t>(c, st) : launch_tiles<64, 64, 2, 2, 4, false, uint64_t>(c, st);
-  if (tile < 0) tile = best_tile(c.M, is_gated ? 2 * c.N : c.N, c.K, c.S);
+  if (tile < 0) tile = best_tile(c.M, is_gated ? 2 * c.N : c.N, c.K, c.S, nullptr, c.ss_in != nullptr);
   int i = 0;
 #define KVCM_TILE_LAUNCH(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) \
   if (tile == i++) return is_gated ? launch<BM, BN, WM, WN, STAGES, PIPE, true>(c, st) : launch<BM, BN, WM, WN, STAGES, PIPE, false>(c, st);

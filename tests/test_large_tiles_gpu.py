@@ -40,3 +40,20 @@ def test_gated_products_of_many_rows(ops, M, I, K, fused):
     g, u = (x.double() @ w.double().t()).split(I, 1)
     # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each
     assert bool(((act.double() - g * torch.sigmoid(g) * u).abs() <= 4.2 * 2.0 ** -8 * g.abs() * u.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("M,I,K", [(49, 8192, 4096), (64, 14336, 4096), (128, 8224, 320), (512, 2048, 192)])
+def test_folded_norms_of_many_rows_stay_with_the_tiles_that_take_them(ops, M, I, K):
+    x, w = tiles._operands(M + I, M, 2 * I, K)
+    ss = torch.rand(M, K // 8, device=DEV) * 8
+    rstd = 1.0 / torch.sqrt(ss.double().sum(1, keepdim=True) / K + 1e-5)
+    out = torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+    rc = ops.lib().kvcm_gemm_skinny_swiglu_normed(x.data_ptr(), w.data_ptr(), ss.data_ptr(), K // 8, 1e-5, out.data_ptr(), M, I, K,
+                                                  x.stride(0), w.stride(0), out.stride(0), ops._stream())
+    assert rc == 0, ops.lib().kvcm_hip_last_error().decode()
+    g, u = (x.double() @ w.double().t() * rstd).split(I, 1)
+    # gate (d silu <= 1.1 d gate), silu(gate), up and the result are rounded to bfloat16, by at most 2^-8 of themselves each; the sums of up to
+    # 4,096 products before are off by up to 2 K roundings of 2^-24
+    eg, eu = (2 * K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) * rstd).split(I, 1)
+    bound = 1.1 * eg * u.abs() + g.abs() * eu + 1.1 * eg * eu
+    assert bool(((out.double() - g * torch.sigmoid(g) * u).abs() <= 1.1 * bound + 4.2 * 2.0 ** -8 * (g.abs() * u.abs()) + 1e-5).all())
