@@ -26,7 +26,13 @@ int gemm_tiles(const TilesCall& c, bool is_gated, int tile, hipStream_t st);
 // about how many us a launch takes
 float gemm_tiles_time(int M, int N, int K, int S, bool is_gated, bool out_f32);
 
-// the same for `groups` workgroups of a tile of bm x bn, and that many elements of weights
-float gemm_tile_time(int bm, int bn, float groups, int steps, float weights);
+// What a launch of one tile takes: us at the beginning and end, us a step of a workgroup that is alone on its CU, the factor on
+// (workgroups a CU) x (a step) beyond that, us of each further round.
+struct TileTime {
+  float fixed, step, share, round;
+};
+// us of a launch of `groups` workgroups of `steps` steps: their chain, or the weights (elements) at 5.9 TB/s, or the rows that every column of
+// tiles reads again (`again` elements, 11 TB/s; 0: left out) where those are longer (a sum of fourth powers in between)
+float tile_time(const TileTime& t, float groups, int steps, float weights, float again);
 
 }  // namespace kvcm

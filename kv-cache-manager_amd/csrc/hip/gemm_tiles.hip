@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(WM* WN* kWave)
 struct Tile {
   int bm, bn;
   bool pipe;
-  float fixed, step, share, round;
+  TileTime time;
 };
 #define KVCM_TILES(T)                                                                                                             \
   T(16, 32, 1, 2, 8, false, 1.305f, 0.144f, 0.725f, 0.000f)                                                                       \
@@ -348,26 +348,18 @@ struct Tile {
   T(256, 192, 2, 2, 2, true, 6.172f, 0.944f, 1.065f, 7.188f)                                                                      \
   T(256, 256, 2, 2, 2, true, 8.118f, 1.175f, 1.013f, 8.000f)
 
-#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, PIPE, FIXED, STEP, SHARE, ROUND},
+#define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, PIPE, {FIXED, STEP, SHARE, ROUND}},
 static constexpr Tile kTiles[] = {KVCM_TILES(KVCM_TILE_ROW)};
 #undef KVCM_TILE_ROW
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int kCUs = 256;
 
-// us of a launch of `groups` workgroups of `steps` steps: their chain, or the weights (elements) at 5.9 TB/s where that is longer (a sum
-// of fourth powers in between)
-static float tile_time(const Tile& t, float groups, int steps, float weights) {
-  const float each = std::ceil(groups / static_cast<float>(kCUs));
+float tile_time(const TileTime& t, float groups, int steps, float weights, float again) {
+  const float each = groups > static_cast<float>(kCUs) ? std::ceil(groups / static_cast<float>(kCUs)) : 1.f;
   const float chain = t.fixed + t.step * static_cast<float>(steps) * (each > 1.f ? each * t.share : 1.f) + t.round * (each - 1.f);
-  const float stream = 2.3f + weights * 2e-6f / 5.9f;
-  const float c2 = chain * chain, s2 = stream * stream;
-  return std::sqrt(std::sqrt(c2 * c2 + s2 * s2));
-}
-
-float gemm_tile_time(int bm, int bn, float groups, int steps, float weights) {
-  for (const Tile& t : kTiles)
-    if (t.bm == bm && t.bn == bn) return tile_time(t, groups, steps, weights);
-  return 1e30f;
+  const float stream = 2.3f + weights * 2e-6f / 5.9f, rows = again > 0.f ? 2.3f + again * 1.8e-7f : 0.f;
+  const float c2 = chain * chain, s2 = stream * stream, r2 = rows * rows;
+  return std::sqrt(std::sqrt(c2 * c2 + s2 * s2 + r2 * r2));
 }
 
 // folded: rows whose norm is still to be applied, which the tiles of tile_pipe.h do not take
@@ -378,7 +370,7 @@ static int best_tile(int M, int wrows, int K, int S, float* time = nullptr, bool
     if (folded && kTiles[i].pipe) continue;
     if (kTiles[i].bm > 16 && kTiles[i].bm >= 2 * M) continue;      // more than half of the rows would not exist
     const float groups = static_cast<float>(static_cast<long long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((wrows + kTiles[i].bn - 1) / kTiles[i].bn) * S);
-    const float t = tile_time(kTiles[i], groups, (K / kStepK + S - 1) / S, static_cast<float>(wrows) * static_cast<float>(K));
+    const float t = tile_time(kTiles[i].time, groups, (K / kStepK + S - 1) / S, static_cast<float>(wrows) * static_cast<float>(K), 0.f);
     if (i == 0 || t < best_t) {
       best = i;
       best_t = t;

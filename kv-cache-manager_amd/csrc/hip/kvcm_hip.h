@@ -336,6 +336,7 @@ int kvcm_moe_few_down(const void* act, const void* w_down, const int* chosen, co
 int kvcm_moe_grouped_supported(int K, int F, int E);
 int kvcm_moe_grouped_lists(int n, int E);
 int kvcm_moe_grouped_tile_count();
+int kvcm_moe_grouped_pick(int n, int E, int N, int K);
 int kvcm_moe_grouped(const void* h, int ldh, const void* w_up, const void* w_down, const int* chosen, const float* weight,
                      int* order, int* lists, void* act, float* y, const float* add, float* out, int T, int K, int F, int H,
                      int top, int E, int kind, int weigh_input, int tile_up, int tile_down, hipStream_t s);

@@ -18,9 +18,11 @@
 //                  (tile_ring.h).
 //   moe_combine    out[row, :] = (add[row, :] +) sum over the row's slots, in slot order, of y[row * top + slot, :]
 //
-// What bounds the products is what bounds those of gemm_tiles.hip; the tile is picked by the same constants.  All five launches, us,
+// What bounds the products is what bounds those of gemm_tiles.hip.  All five launches, us,
 // against 128 x 128 pairs and rows with two stages throughout: 8 experts of which a row uses 2, width 2,048, 1,408 columns an expert: 80
 // rows 64.6 -> 44.2, 300 69.9 -> 52.0, 1,024 86.1 -> 84.2, 2,048 134 -> 113, 4,072 230 -> 208; width 4,096, 3,584 columns, 2,048 rows 487 -> 468.
+#include <cmath>
+
 #include "common.h"
 #include "gemm_tiles.h"
 #include "kvcm_hip.h"
@@ -184,34 +186,50 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<Vec*>(out + row * H + c) = add ? *reinterpret_cast<const Vec*>(add + row * H + c) + acc : acc;
 }
 
-// Tiles: those of gemm_tiles.hip of an even number of accumulators a wave, with the same constants of a launch's time.
-#define KVCM_GROUPED_TILES(T)      \
-  T(64, 64, 2, 2, 4, false)        \
-  T(96, 64, 2, 2, 4, true)         \
-  T(128, 128, 2, 2, 4, true)       \
-  T(192, 128, 2, 2, 3, true)       \
-  T(256, 128, 2, 2, 3, true)       \
-  T(256, 192, 2, 2, 2, true)       \
-  T(256, 256, 2, 2, 2, true)
+// The tiles, of an even number of accumulators a wave, and what a launch of them takes (gemm_tiles.h).  The eight to twelve waves of tile_ring.h in large tiles
+// but for 192 x 128: an expert's few tiles do not make up for the longer beginning and end of the four waves of tile_pipe.h.  Fitted to 6,200 timed
+// launches of 13 tiles at 472 products (33 sizes of experts, 4 to 64 of them, 64 to 8,192 rows).  At 858 further products (65 sizes) the pick takes 0.967 of the time of these waves'
+// by the constants of gemm_tiles.hip with half a tile lost an expert, and 0.945 of what that rule took with six of tile_pipe.h's tiles instead, which were slower than these
+// by a tenth at a quarter of the products.  Up and down, us, six of tile_pipe.h / so: 5,632 columns of 2,048, 8 experts, one a row, 509 rows
+// 117 / 94; 1,408 columns gated, two a row, 4,072 rows 198 / 187, 2,048 rows 94 / 96, 1,024 rows 62 / 66; 256 columns of 512, 64 experts, eight a row, 4,072 rows 66 / 57.
+#define KVCM_GROUPED_TILES(T)                                      \
+  T(64, 64, 2, 2, 4, false, 3.293f, 0.253f, 0.752f, 0.696f)        \
+  T(128, 64, 4, 2, 6, false, 3.734f, 0.322f, 1.004f, 2.392f)       \
+  T(128, 128, 2, 4, 4, false, 4.219f, 0.517f, 1.032f, 2.958f)      \
+  T(192, 128, 2, 2, 3, true, 6.472f, 0.589f, 1.071f, 4.782f)       \
+  T(256, 128, 4, 2, 3, false, 6.426f, 0.794f, 1.037f, 4.013f)      \
+  T(256, 192, 4, 3, 2, false, 5.680f, 1.201f, 1.033f, 4.175f)      \
+  T(256, 256, 2, 4, 2, false, 7.658f, 1.491f, 0.991f, 6.674f)
 
 struct High {
   int bm, bn;
+  TileTime time;
 };
-#define KVCM_HIGH(BM, BN, WM, WN, STAGES, PIPE) {BM, BN},
+#define KVCM_HIGH(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, {FIXED, STEP, SHARE, ROUND}},
 static constexpr High kHighs[] = {KVCM_GROUPED_TILES(KVCM_HIGH)};
 #undef KVCM_HIGH
 constexpr int kHighCount = sizeof(kHighs) / sizeof(kHighs[0]);
 constexpr int kFarTile = 2;      // the one that is there with 64-bit offsets too
 static_assert(kHighs[kFarTile].bm == 128 && kHighs[kFarTile].bn == 128, "launch_grouped names it");
 
-// The tile for n pairs over E experts, N rows of K each: groups of pairs end in a tile that is half empty on average.
+// Tiles of bm pairs that n pairs over E experts make up, if each expert is as likely: the sum over j of P(an expert has more than j bm pairs)
+static float expected_tiles(int n, int E, int bm) {
+  const double mean = static_cast<double>(n) / E, sd = std::sqrt(mean);
+  const int whole = mean > 6.0 * sd ? static_cast<int>((mean - 6.0 * sd) / bm) : 0;
+  double sum = whole;
+  for (int j = whole; static_cast<double>(j) * bm < mean + 6.0 * sd + 1.0; ++j) sum += 0.5 * std::erfc((static_cast<double>(j) * bm + 0.5 - mean) / (sd * 1.41421356));
+  return static_cast<float>(E * sum);
+}
+
+// The tile for n pairs over E experts, N rows of K each.
 static int best_grouped(int n, int E, int N, int K) {
-  const float used = n < E ? static_cast<float>(n) : static_cast<float>(E);
+  const float used = n < E ? static_cast<float>(n) : static_cast<float>(E), k = static_cast<float>(K);
   int best = 0;
   float best_t = 0.f;
   for (int i = 0; i < kHighCount; ++i) {
-    const float groups = (static_cast<float>(n) / static_cast<float>(kHighs[i].bm) + 0.5f * used) * static_cast<float>((N + kHighs[i].bn - 1) / kHighs[i].bn);
-    const float t = gemm_tile_time(kHighs[i].bm, kHighs[i].bn, groups, (K + kStepK - 1) / kStepK, used * static_cast<float>(N) * static_cast<float>(K));
+    const float cols = static_cast<float>((N + kHighs[i].bn - 1) / kHighs[i].bn);
+    const float t = tile_time(kHighs[i].time, expected_tiles(n, E, kHighs[i].bm) * cols, (K + kStepK - 1) / kStepK, used * static_cast<float>(N) * k,
+                              static_cast<float>(n) * k * cols);
     if (i == 0 || t < best_t) {
       best = i;
       best_t = t;
@@ -247,7 +265,7 @@ static int launch_grouped(int tile, const GroupedCall& c, hipStream_t s) {
     return launch_status("moe_grouped");
   }
   int i = 0;
-#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES, PIPE) \
+#define KVCM_GROUPED_LAUNCH(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) \
   if (tile == i++) KVCM_GROUPED(BM, BN, WM, WN, STAGES, PIPE, uint32_t);
   KVCM_GROUPED_TILES(KVCM_GROUPED_LAUNCH)
 #undef KVCM_GROUPED_LAUNCH
@@ -267,6 +285,12 @@ int kvcm_moe_grouped_supported(int K, int F, int E) { return K > 0 && F > 0 && K
 // int32 values of work memory that a step of n pairs over E experts needs for its lists of tiles (16-byte aligned)
 int kvcm_moe_grouped_lists(int n, int E) { return 4 + 8 * most_tiles(n, E); }
 int kvcm_moe_grouped_tile_count() { return kHighCount; }
+// the tile that the rule picks for n pairs over E experts and N rows of K each, as 1,000 x its pairs + its rows: for tests
+int kvcm_moe_grouped_pick(int n, int E, int N, int K) {
+  KVCM_REQUIRE(n > 0 && E > 0 && N > 0 && K > 0, "moe_grouped_pick: bad sizes");
+  const High& tile = kHighs[best_grouped(n, E, N, K)];
+  return tile.bm * 1000 + tile.bn;
+}
 
 // h [T, K] bfloat16; w_up [E, F, K], w_down [E, H, F] bfloat16; chosen [T * top], weight [T * top]; work memory:
 // order [T * top] and lists [kvcm_moe_grouped_lists] (int32), act [T * top, F] (bfloat16), y [T * top, H] (32-bit); out [T, H] 32-bit.

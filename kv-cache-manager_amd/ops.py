@@ -146,6 +146,7 @@ def _declare(lib):
     fn("kvcm_moe_grouped_supported", i, i, i)
     fn("kvcm_moe_grouped_lists", i, i)
     fn("kvcm_moe_grouped_tile_count")
+    fn("kvcm_moe_grouped_pick", i, i, i, i)
     fn("kvcm_moe_grouped", vp, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, i, i, i, vp)
     fn("kvcm_pool_update", vp, vp, i, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, i, vp)
     fn("kvcm_attention_window_pool", vp, i, i, vp, i, vp, vp, vp, vp, vp, i, vp, vp, vp, vp, vp, i, i, i, i, i, i, i, f, i, i, i, i, f, i, i, vp, i, f, vp)
