@@ -32,7 +32,7 @@ struct TileTime {
   float fixed, step, share, round;
 };
 // us of a launch of `groups` workgroups of `steps` steps: their chain, or the weights (elements) at 5.9 TB/s, or the rows that every column of
-// tiles reads again (`again` elements, 11 TB/s; 0: left out) where those are longer (a sum of fourth powers in between)
+// tiles reads again (`again` elements, 11 TB/s) where those are longer (a sum of fourth powers in between)
 float tile_time(const TileTime& t, float groups, int steps, float weights, float again);
 
 }  // namespace kvcm

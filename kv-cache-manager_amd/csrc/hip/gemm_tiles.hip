@@ -317,47 +317,51 @@ __global__ void __launch_bounds__(WM* WN* kWave)
   }
 }
 
-// The tiles, and what a launch of them takes: us at the beginning and end, us a step of a workgroup that is alone on its CU, the factor on
-// (workgroups a CU) x (a step) beyond that, us of each further round.  Fitted to some 5,000 timed launches (8 to 2,048 rows, the
-// projections of models of widths 2,048 and 4,096, S = 1 to 8; the fit is off by 4 to 10 % a launch), the tiles of tile_pipe.h, from 96
-// rows on, to 7,500 further ones (96 to 4,096 rows, 64 to 16,384 columns, K 256 to 14,336, S = 1, 2, 4; off by 8 to 15 % a launch; what the rule picks
-// is 1.0 % slower than the best tile on average, 29 % at worst: 96 x 4096 x 14336 in two slices).  Below that the ring of tile_ring.h is the faster: 64 x 64
-// of 64 rows of 2048 x 2048 in eight slices 5.2 us, 5.7 with fragments read ahead.
+// The tiles, and what a launch of them takes (TileTime).  Fitted to 120,000 timed launches (kernel times; 1 to 33,000 rows, 64 to
+// 32,000 columns, K 256 to 14,336, S as rows_splits has it, gated or not) of these tiles and two more at 5,800 shapes, widths as models have them and random ones; with half of the
+// shapes for the fit a pick is 0.6 % slower than the fastest tile below 96 rows and 0.9 % from there on at the other half, 27 % at worst (576 x 3072 x 5120: 96 x 96, 40.6 us,
+// 128 x 64 31.9).  From 96 rows on tile_pipe.h's are mostly the faster, but not everywhere: the ring's 128 x 64, 128 x 96 and 128 x 128 stay for short chains and for tiles that just
+// fill the chip (us, the best of tile_pipe.h / so: gate and up of 512 x 2816 x 2048 24.6 / 20.2, 128 x 11264 x 2048 in two slices 17.7 / 15.6, 256 x 8192 x 2048 19.2 / 17.1,
+// 117 x 7680 x 1600 in four 14.2 / 12.0), its 64 x 32 for few columns (48 x 8192 x 2048 10.3 in 32 x 64, 9.6).
 // (columns, after the sizes and waves: the stages, and whether the tile is tile_pipe.h's)
 struct Tile {
   int bm, bn;
   bool pipe;
   TileTime time;
 };
-#define KVCM_TILES(T)                                                                                                             \
-  T(16, 32, 1, 2, 8, false, 1.305f, 0.144f, 0.725f, 0.000f)                                                                       \
-  T(16, 48, 1, 3, 8, false, 1.278f, 0.167f, 0.771f, 0.466f)                                                                       \
-  T(16, 64, 1, 4, 8, false, 1.126f, 0.199f, 0.886f, 0.256f)                                                                       \
-  T(32, 32, 2, 2, 8, false, 1.517f, 0.163f, 0.801f, 0.197f)                                                                       \
-  T(32, 64, 2, 2, 6, false, 1.484f, 0.219f, 0.891f, 0.210f)                                                                       \
-  T(64, 48, 4, 1, 8, false, 2.019f, 0.236f, 0.975f, 1.170f)                                                                       \
-  T(64, 64, 2, 2, 4, false, 1.822f, 0.274f, 0.869f, 0.435f)                                                                       \
-  T(64, 96, 2, 3, 6, false, 2.462f, 0.351f, 0.957f, 1.524f)                                                                       \
-  T(96, 64, 2, 2, 4, true, 3.147f, 0.242f, 1.040f, 0.523f)                                                                        \
-  T(96, 96, 2, 2, 4, true, 3.426f, 0.308f, 1.007f, 3.111f)                                                                        \
-  T(96, 128, 2, 2, 4, true, 3.607f, 0.349f, 1.084f, 3.262f)                                                                       \
-  T(128, 128, 2, 2, 4, true, 4.093f, 0.430f, 1.025f, 3.974f)                                                                      \
-  T(192, 128, 2, 2, 3, true, 5.115f, 0.537f, 1.001f, 4.856f)                                                                      \
-  T(192, 192, 2, 2, 3, true, 6.493f, 0.662f, 1.037f, 6.782f)                                                                      \
-  T(256, 128, 2, 2, 3, true, 6.230f, 0.612f, 1.059f, 6.453f)                                                                      \
-  T(256, 192, 2, 2, 2, true, 6.172f, 0.944f, 1.065f, 7.188f)                                                                      \
-  T(256, 256, 2, 2, 2, true, 8.118f, 1.175f, 1.013f, 8.000f)
+#define KVCM_TILES(T)                                         \
+  T(16, 32, 1, 2, 8, false, 2.786f, 0.121f, 0.654f, 0.267f)   \
+  T(16, 48, 1, 3, 8, false, 2.807f, 0.137f, 0.742f, 0.631f)   \
+  T(16, 64, 1, 4, 8, false, 2.851f, 0.169f, 0.772f, 0.596f)   \
+  T(32, 32, 2, 2, 8, false, 2.822f, 0.137f, 0.779f, 0.448f)   \
+  T(32, 64, 2, 2, 6, false, 3.181f, 0.192f, 0.768f, 0.705f)   \
+  T(64, 32, 2, 2, 6, false, 3.325f, 0.205f, 0.636f, 0.782f)   \
+  T(64, 64, 2, 2, 4, false, 3.307f, 0.257f, 0.813f, 0.702f)   \
+  T(64, 96, 2, 3, 6, false, 4.094f, 0.323f, 1.025f, 2.233f)   \
+  T(128, 96, 4, 3, 5, false, 5.016f, 0.443f, 1.016f, 2.905f)  \
+  T(96, 64, 2, 2, 4, true, 4.215f, 0.262f, 0.807f, 0.743f)    \
+  T(96, 96, 2, 2, 4, true, 4.792f, 0.337f, 0.974f, 2.752f)    \
+  T(96, 128, 2, 2, 4, true, 5.086f, 0.416f, 0.968f, 2.478f)   \
+  T(128, 128, 2, 2, 4, true, 5.719f, 0.475f, 0.956f, 3.012f)  \
+  T(192, 128, 2, 2, 3, true, 6.599f, 0.560f, 0.986f, 3.838f)  \
+  T(192, 192, 2, 2, 3, true, 7.789f, 0.727f, 1.051f, 4.891f)  \
+  T(256, 192, 2, 2, 2, true, 8.017f, 1.076f, 0.992f, 5.221f)  \
+  T(256, 256, 2, 2, 2, true, 9.432f, 1.289f, 1.014f, 6.981f)  \
+  T(128, 64, 4, 2, 6, false, 4.459f, 0.311f, 1.049f, 2.637f)  \
+  T(128, 128, 2, 4, 4, false, 5.580f, 0.519f, 0.993f, 3.535f) \
+  T(256, 128, 2, 2, 3, true, 7.905f, 0.649f, 0.998f, 5.019f)
 
 #define KVCM_TILE_ROW(BM, BN, WM, WN, STAGES, PIPE, FIXED, STEP, SHARE, ROUND) {BM, BN, PIPE, {FIXED, STEP, SHARE, ROUND}},
 static constexpr Tile kTiles[] = {KVCM_TILES(KVCM_TILE_ROW)};
 #undef KVCM_TILE_ROW
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+constexpr int kFurtherTiles = 3;      // the last ones, which have numbers of their own
 constexpr int kCUs = 256;
 
 float tile_time(const TileTime& t, float groups, int steps, float weights, float again) {
   const float each = groups > static_cast<float>(kCUs) ? std::ceil(groups / static_cast<float>(kCUs)) : 1.f;
   const float chain = t.fixed + t.step * static_cast<float>(steps) * (each > 1.f ? each * t.share : 1.f) + t.round * (each - 1.f);
-  const float stream = 2.3f + weights * 2e-6f / 5.9f, rows = again > 0.f ? 2.3f + again * 1.8e-7f : 0.f;
+  const float stream = 2.3f + weights * 2e-6f / 5.9f, rows = 2.3f + again * 1.8e-7f;
   const float c2 = chain * chain, s2 = stream * stream, r2 = rows * rows;
   return std::sqrt(std::sqrt(c2 * c2 + s2 * s2 + r2 * r2));
 }
@@ -369,8 +373,9 @@ static int best_tile(int M, int wrows, int K, int S, float* time = nullptr, bool
   for (int i = 0; i < kTileCount; ++i) {
     if (folded && kTiles[i].pipe) continue;
     if (kTiles[i].bm > 16 && kTiles[i].bm >= 2 * M) continue;      // more than half of the rows would not exist
-    const float groups = static_cast<float>(static_cast<long long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((wrows + kTiles[i].bn - 1) / kTiles[i].bn) * S);
-    const float t = tile_time(kTiles[i].time, groups, (K / kStepK + S - 1) / S, static_cast<float>(wrows) * static_cast<float>(K), 0.f);
+    const int cols = (wrows + kTiles[i].bn - 1) / kTiles[i].bn;
+    const float groups = static_cast<float>(static_cast<long long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * cols * S), k = static_cast<float>(K);
+    const float t = tile_time(kTiles[i].time, groups, (K / kStepK + S - 1) / S, static_cast<float>(wrows) * k, static_cast<float>(M) * k * static_cast<float>(cols));
     if (i == 0 || t < best_t) {
       best = i;
       best_t = t;
@@ -440,8 +445,10 @@ using namespace kvcm;
 
 extern "C" {
 
-// How many tiles there are, the rows and columns (of W) of one, and the one the rule picks: for tests, which run each.
-int kvcm_gemm_tiles_count() { return kTileCount; }
+// How many tiles there are (and how many further ones, numbered on from there), the rows and columns (of W) of one, and the one the rule picks: for
+// tests, which run each.
+int kvcm_gemm_tiles_count() { return kTileCount - kFurtherTiles; }
+int kvcm_gemm_tiles_further() { return kFurtherTiles; }
 int kvcm_gemm_tiles_size(int tile, int* rows, int* cols) {
   KVCM_REQUIRE(tile >= 0 && tile < kTileCount, "gemm_tiles_size: no tile %d", tile);
   *rows = kTiles[tile].bm;
@@ -467,37 +474,54 @@ int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, in
   return gemm_tiles(c, is_gated != 0, tile, st);
 }
 
+// What the library takes for M x wrows x K, us: the fastest of three sizes of tile, each with a constant, a step's chain for every round of 256
+// workgroups and a step's share of the chip, or tiles of 128 x 128 with K cut into up to 16 slices until they are 256; and the results' storing.
+static float library_time(int M, int wrows, int K) {
+  struct LibraryTile {
+    int size;
+    float fixed, chain, share;
+  };
+  static constexpr LibraryTile kLibrary[] = {{256, 5.87f, 0.321f, 0.929f}, {128, 7.47f, 0.115f, 0.525f}, {64, 0.68f, 1.28f, 0.182f}};
+  const float steps = static_cast<float>(K) / kStepK;
+  float best = 0.f, part = 0.f;
+  for (const LibraryTile& l : kLibrary) {
+    const float tiles = static_cast<float>((M + l.size - 1) / l.size) * static_cast<float>((wrows + l.size - 1) / l.size) / static_cast<float>(kCUs);
+    const float t = l.fixed + steps * (l.chain * std::ceil(tiles) + l.share * tiles);
+    if (best == 0.f || t < best) best = t;
+    if (l.size == 128) part = tiles;
+  }
+  const float slices = std::fmin(std::fmax(std::floor(1.f / part), 1.f), 16.f), cut = 8.22f + steps * (0.585f / slices + 1.028f * part);
+  return std::fmin(best, cut) + static_cast<float>(M) * static_cast<float>(wrows) * 0.595e-6f;
+}
+
 // Is a product of many rows, in S slices of K that its consumer adds, faster here than by the vendor library (is_gated: than that and
-// the launch that applies the activation)?  Beyond 2,048 rows a plain product is the library's, whose tiles of 256 x 256 are 5 to 15 %
+// the launch that applies the activation, 3.4 us and 6 bytes a result at 5 TB/s)?  Beyond 2,048 rows a plain product is the library's, whose tiles of 256 x 256 are 5 to 15 %
 // faster once every CU has several (32,768 rows: 2048 x 5632 565 / 505 us, 2560 x 2048 266 / 240), a gated one is not: it saves the second launch and
-// the product's trip to memory (32,768 rows of gate and up, 5632 x 2048: 1,118 / 1,276 us; 8,192 rows 309 / 394; 9,608 rows, 14336 x 4096 1,696 / 1,783).  Up to there the
-// tiles' time against about what the library takes.  Here: the launch as the tile was
-// picked, with what that model leaves out, the rows of X that every column of tiles reads again (7 TB/s), and the slices' reading (4.5 TB/s,
-// and 55 KB a us of one row's through the CU that norms it).  There: 5.5 us, or 1.8 us, 0.26 us for 64 k of a chain and 1,300 to 1,700 TFLOP/s (the more the
-// more results there are) and 1.15 us a million results, or, where
-// few results let it cut K, 6.7 us and 0.043 us for 64 k of 131,072 results, and the same a result; and 7.2 us and 6 bytes a result for the second launch.
-// Up to 256 rows the library is often far above that, so that it has to be 1.45 times as fast.
-// The constants were fitted to 230 plain products (64 to 16,384 columns, K 256 to 14,336, 96 to 2,048 rows) and 257 gated ones (64 to 14,336
-// columns, 96 to 33,000 rows).  What the rule picks takes 0.87 and 0.79 of the library's time on average and
-// is 2.0 and 1.0 % slower than the better of the two; slower than the library by more than 8 % are 9 and 4 of them: 1040 x 8192 x 2048 43.9 / 35.4,
-// 384 x 2048 x 5632 32.8 / 26.0.  (us, here / library: 2048 x 2560 x 2048 22.8 / 25.2, 2048 x 2048 x 5632 51.8 / 54.0, 1040 x 2048 x 2048 13.6 / 20.0; 2,048 and 1,024 rows gate+up of
-// 5632 x 2048 88.9 / 92.7 and 45.3 / 55.2; not taken: 640 x 64 x 14336 33 / 13.3, 2048 x 256 x 5632 22 / 17.4, 2048 x 8192 x 2048 53 / 49.7.)
+// the product's trip to memory (32,768 rows of gate and up, 5632 x 2048: 1,118 / 1,276 us; 8,192 rows 308 / 408; 9,608 rows, 14336 x 4096 1,698 / 1,779).  Up to there the
+// tile's modelled time, with the slices' reading (4.5 TB/s, and 55 KB a us of one row's through the CU that norms it), against the modelled library's, which was fitted to
+// half of 2,329 plain shapes (1,397 of widths as models have them, the others random; 64 to 32,000 columns, K 256 to 14,336, 96 to 2,048 rows).  It is off by 11 and 18 % a shape: which of
+// its kernels the library picks hangs on more than the sizes (256 x 128 x 5632 9.1 us, x 5120 17.5).  So the line lies a little on its side, and further where it is known to be better
+// than modelled and little is lost by it: 513 to 1,024 rows of fewer than 116 tiles of 128 x 128 (640 x 2048 x 2048 15.5, here 14.2; 768 rows 14.5, 14.4), and few columns of long K;
+// on the tiles' up to 256 rows of more than 16, where it is often far slower than modelled (256 x 5632 x 5632 54, here 37).
+// What the rule picks is 2.1 and 5 % slower than the better of the two, gated (1,197 shapes, 96 to 33,000 rows) 1.2 and 0.6 %.  Against the line and the tiles from before there were
+// tiles of four waves: 0.96 and 0.93 of the time, gated 0.90 and 0.80, slower by more than 5 % at 53 and 9, gated 19 and 8; with the line that came with those tiles it was 209 and 71,
+// gated 64 and 33.  At 1,420 plain shapes that the fit had not seen 0.965 and 0.95, slower by more than 5 % at 83 of 1,220 and 19 of 200; 571 gated 0.92 and 0.85, at 37 and 14.
+// (us, here / library: taken 2048 x 2560 x 2048 25.8 / 29.0, 1040 x 2048 x 2048 17.2 / 23.0, 1024 x 1024 x 512 5.9 / 9.0, 2048 x 2048 x 5632 52.2 / 52.7; 2,048 and 1,024 rows of gate and up,
+// 5632 x 2048, 90 / 92 and 49 / 57; not taken 640 x 64 x 14336 30 / 17, 1040 x 8192 x 2048 44 / 36, 2048 x 8192 x 2048 52 / 50, 384 x 2048 x 5632 whole 27 / 25, 2048 x 256 x 5632 21.7 / 20.6.)
 int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype) {
   if (M <= 0 || N <= 0 || N % 64 != 0 || K <= 0 || K % kStepK != 0 || S < 1 || S > K / kStepK || (is_gated && S > 1)) return 0;
   if (M > 2048 && !is_gated) return 0;
-  const float m = static_cast<float>(M), n = static_cast<float>(N), k = static_cast<float>(K), steps = static_cast<float>(K / kStepK);
+  const float results = static_cast<float>(M) * static_cast<float>(N);
   const int wrows = is_gated ? 2 * N : N;
-  float t = 0.f;
-  const Tile& tile = kTiles[best_tile(M, wrows, K, S, &t)];
-  const float again = 2.3f + m * k * 2.81e-7f * static_cast<float>((wrows + tile.bn - 1) / tile.bn);
-  const float t2 = t * t, again2 = again * again;
-  const float here = std::sqrt(std::sqrt(t2 * t2 + again2 * again2)) + stored_time(M, N, S, out_dtype == kF32) +
-                     (S > 1 ? m * n * (4.f * S - 2.f) / 4.5e6f + n * 4.f * S / 55e3f : 0.f);
-  const float results = m * static_cast<float>(wrows), rounds = results / (256.f * 256.f * 256.f);
-  const float rate = 1.304f + 0.412f * rounds / (rounds + 17.6f), stored = results * 1.15e-6f;      // (PFLOP/s; us)
-  const float whole = 1.8f + 0.26f * steps + results * k * 2e-9f / rate, cut = 6.7f + 0.043f * steps * results / 131072.f;
-  const float library = std::fmax(5.51f, std::fmin(whole, cut) + stored) + (is_gated ? 7.18f + m * n * 6.f / 7.93e6f : 0.f);
-  return here <= (M <= 256 ? 1.45f : 1.f) * library;
+  float here = 0.f;
+  best_tile(M, wrows, K, S, &here);
+  here += stored_time(M, N, S, out_dtype == kF32) +
+          (S > 1 ? results * (4.f * S - 2.f) / 4.5e6f + static_cast<float>(N) * 4.f * S / 55e3f : 0.f);
+  const float library = library_time(M, wrows, K);
+  if (is_gated) return here <= library + 3.4f + results * 6.f / 5e6f;
+  const long long tiles = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128);
+  const float side = M <= 256 && tiles > 16 ? 1.1f : M > 512 && M <= 1024 && tiles < 116 ? 0.78f : N <= 320 && K >= 5632 ? 0.84f : 0.98f;
+  return here <= side * library;
 }
 
 }  // extern "C"

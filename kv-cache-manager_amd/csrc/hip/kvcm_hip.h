@@ -28,6 +28,7 @@ int kvcm_reduce_store(const float* partials, void* out, int out_dtype, int M, in
 int kvcm_gemm_skinny_whole_splits(int M, int N, int K);
 // Products in tiles (gemm_tiles.hip), any number of rows: N a multiple of 4 (gated: 8), K of 64.
 int kvcm_gemm_tiles_count();
+int kvcm_gemm_tiles_further();
 int kvcm_gemm_tiles_size(int tile, int* rows, int* cols);
 int kvcm_gemm_tiles_pick(int M, int N, int K, int S, int is_gated);
 int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, int out_dtype, int M, int N, int K, int ldx, int ldw, int ldo,

@@ -63,6 +63,7 @@ def _declare(lib):
     fn("kvcm_gemm_skinny_splits", i, i, i)
     fn("kvcm_gemm_skinny_whole_splits", i, i, i)
     fn("kvcm_gemm_tiles_count")
+    fn("kvcm_gemm_tiles_further")
     fn("kvcm_gemm_tiles_size", i, C.POINTER(i), C.POINTER(i))
     fn("kvcm_gemm_tiles_pick", i, i, i, i, i)
     fn("kvcm_gemm_tiles", vp, vp, vp, vp, i, i, i, i, i, i, i, i, i, i, f, i, vp)

@@ -42,6 +42,34 @@ def test_gated_products_of_many_rows(ops, M, I, K, fused):
     assert bool(((act.double() - g * torch.sigmoid(g) * u).abs() <= 4.2 * 2.0 ** -8 * g.abs() * u.abs() + 1e-4).all())
 
 
+def test_further_tiles(ops, monkeypatch):
+    """the tiles that are numbered on from the count: each at its edges, gated, and over several groups of row blocks"""
+    import ctypes
+    first = ops.lib().kvcm_gemm_tiles_count()
+
+    def size(lib, t):
+        rows, cols = ctypes.c_int(), ctypes.c_int()
+        assert lib.kvcm_gemm_tiles_size(t, ctypes.byref(rows), ctypes.byref(cols)) == 0
+        return rows.value, cols.value
+    more = range(first, first + ops.lib().kvcm_gemm_tiles_further())
+    assert len(more) == 3
+    everything = [size(ops.lib(), t) for t in range(more.stop)]
+    assert size_is_refused(ops, more.stop)
+    for tile in more:
+        with monkeypatch.context() as m:
+            m.setattr(tiles, "_tiles", lambda ops, tile=tile: [everything[tile]] * 17)
+            run = tiles._run
+            m.setattr(tiles, "_run", lambda *a, tile=tile, **kw: run(*a, **{**kw, "tile": tile}))
+            tiles.test_every_tile_at_its_edges(ops, 0)
+            tiles.test_every_tile_gated(ops, 0)
+            test_groups_of_row_blocks(ops, 0)
+
+
+def size_is_refused(ops, tile):
+    import ctypes
+    return ops.lib().kvcm_gemm_tiles_size(tile, ctypes.byref(ctypes.c_int()), ctypes.byref(ctypes.c_int())) != 0
+
+
 @pytest.mark.parametrize("M,I,K", [(49, 8192, 4096), (64, 14336, 4096), (128, 8224, 320), (512, 2048, 192)])
 def test_folded_norms_of_many_rows_stay_with_the_tiles_that_take_them(ops, M, I, K):
     x, w = tiles._operands(M + I, M, 2 * I, K)
