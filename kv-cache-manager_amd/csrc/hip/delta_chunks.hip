@@ -1,4 +1,5 @@
-// The generalized delta rule (delta_rule.hip) for long runs, in matrix form.  In a chunk of C rows that starts from S, with W_i = w_0 .. w_i per
+// The generalized delta rule (delta_rule.hip) for long runs, in matrix form (a chunk's rank-one updates as one triangular solve and products, as published for
+// products of Householder reflections, Bischof and Van Loan's WY form, and for delta rules over sequences).  In a chunk of C rows that starts from S, with W_i = w_0 .. w_i per
 // key channel and the rows
 //
 //   U_i = u_i W_(i-1)    R_i = r_i W_i    K_j = k_j / W_j    A_j = (a u)_j / W_j
@@ -8,27 +9,36 @@
 //   o = (R - P X) S + (lower(R K^T) V - P Y)        P = lower(R A^T), with its diagonal
 //   S <- diag(W) (I - A^T X) S + diag(W) (K^T V - A^T Y)        W = W_(C-1)
 //
+// Where keys resemble each other the two sums of N = K^T V - A^T Y, of the outputs and of Y's own equations grow with the rows and nearly cancel, which the walk never
+// has: it learns v - what the state already says.  So nothing is summed that way: with a factor t_j a row, the one that brings t_j k_j closest to (a u)_j, B_j = t_j K_j - A_j
+// and D_j = v_j - t_j Y_j,
+//
+//   N = diag(W) (K^T D + B^T Y)      lower(R K^T) D + lower(R B^T) Y      row block b of Y: lower(U K^T) D + lower(U B^T) Y of the blocks before, then the block's own inverse
+//
+// whose terms are as small as what there is to learn.  lower(U K^T), lower(U B^T) and Y are made in 64 bits (v_mfma_f64_16x16x4_f64), and kept in 32; so are the decays' products.
 // Everything but the two products with S is made for all chunks at once (delta_chunk_kernel leaves a chunk's M = diag(W) (I - A^T X), its N, its
-// Q = R - P X and what its outputs have without S); what is left of the walk is one product of [M; Q] with S a chunk (delta_pass_kernel).  All of it
-// in 32 bits on the matrix cores (v_mfma_f32_16x16x4_f32).
+// Q = R - P X and what its outputs have without S); what is left of the walk is one product of [M; Q] with S a chunk (delta_pass_kernel), in 32 bits on the
+// matrix cores (v_mfma_f32_16x16x4_f32) like all the rest.
 //
 // The quotients: w is exp(-exp(-1/2) sigmoid(.)), so 0.545 < w <= 1, W of 64 rows is above 1e-17 and a factor W_i / W_j of a term that is used is at
 // most one and has the relative error of a few roundings.  What lies above the diagonals may be large and is left out by selection.  (What is
 // not finite in a row reaches the rows of its chunk in front of it too.)
 //
-// The walk's time is a token's chain of dependent instructions whatever the chip could do.  One sequence of 2,048 tokens, 32 heads of 64 x 64: 293 us,
-// 120 so: 80 for the chunks (matrix instructions 35 of them, vector instructions as much, in 64-bit products of the decays and the rows' scaling, and
-// 164 MB moved) and 39 for the pass (32 steps of a product, a barrier and a trip through LDS).  128 x 128: 689 / 323 us.
-// Error against 64 bits of outputs and states, the walk / so: 1.11e-7 / 1.05e-7 and 8.8e-8 / 7.9e-8; 128 x 128 1.17e-7 / 1.16e-7 and 8.9e-8 / 7.8e-8
-// (with each sum in one chain 2.4e-7 and 2.0e-7).
+// Errors against 64 bits as parts of the walk's: keys and values with a common mean of 0 to 5 times their spread, rates of removal around 0.05 to 0.98:
+// outputs 0.54 .. 0.86, states 0.64 .. 0.99; in 32 bits, with N and the outputs as the plain differences above, up to 4.2 times the walk's.
+// us, walk / so / with those differences: 32 heads of 64 x 64, 2,048 tokens 291 / 147 / 125, 512 72 / 42 / 37, 192 29.3 / 31.4 / 25.7, 3 of 1,024
+// 332 / 240 / 196; 32 heads of 128 x 128, 2,048 tokens 711 / 359 / 322, 4 of 1,024 1,328 / 721 / 657.
+//
 // A workgroup of the first kernel is eight waves, one a CU: four matrices of C rows by the keys and four of C by C in LDS, a wave with 16 columns of
-// X or Y in registers throughout, whose accumulators are the next product's second operand as they lie (key 4 g + e of lane group g is element e).
+// X or Y in registers throughout, whose accumulators are the next product's second operand as they lie (key 4 g + e of lane group g is element e; the ones of
+// 64 bits, 4 e + g, are turned by four swaps of lanes).
 #include "common.h"
 #include "kvcm_hip.h"
 
 namespace kvcm {
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(4 * sizeof(double)))) double f64x4;
 
 struct DeltaChunkArgs {
   const float *r, *k, *v, *w, *au, *u;
@@ -70,6 +80,45 @@ struct Chains {
   __device__ __forceinline__ f32x4 sum() const { return (v[0] + v[1]) + (v[2] + v[3]); }
 };
 
+// The same in 64 bits, in two chains (an instruction waits long for the one it adds to): an element of lane group g is row 4 e + g of the sum.
+struct Chains64 {
+  f64x4 v[2] = {};
+  __device__ __forceinline__ void add(float4 a, f32x4 b) {
+    v[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b[0], v[0], 0, 0, 0);
+    v[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b[1], v[1], 0, 0, 0);
+    v[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.z, b[2], v[0], 0, 0, 0);
+    v[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.w, b[3], v[1], 0, 0, 0);
+  }
+  __device__ __forceinline__ f64x4 sum() const { return v[0] + v[1]; }
+};
+// four registers turned over the four lane groups: element e of group g <- element g of group e
+__device__ __forceinline__ void turn(uint32_t (&x)[4]) {
+  const auto a = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false), b = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  x[0] = c[0]; x[1] = c[1]; x[2] = d[0]; x[3] = d[1];
+}
+__device__ __forceinline__ void turn(f32x4& v) {
+  uint32_t x[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = __float_as_uint(v[e]);
+  turn(x);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(x[e]);
+}
+__device__ __forceinline__ void turn(f64x4& v) {
+  uint32_t low[4], high[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint64_t bits = __builtin_bit_cast(uint64_t, static_cast<double>(v[e]));
+    low[e] = static_cast<uint32_t>(bits);
+    high[e] = static_cast<uint32_t>(bits >> 32);
+  }
+  turn(low);
+  turn(high);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __builtin_bit_cast(double, uint64_t(high[e]) << 32 | low[e]);
+}
+
 constexpr int kDeltaThreads = 512;
 
 template <int DKP>
@@ -78,9 +127,11 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
   constexpr int RG = kDeltaThreads / DKP, RPT = C / RG;      // row groups, rows a thread scales
   constexpr bool kBoth = KT == NW;      // every wave has a column tile of X and one of Y; else half of the waves have either
   static_assert(kBoth || 2 * KT == NW, "the column tiles are dealt out to eight waves");
-  __shared__ __attribute__((aligned(16))) float Us[C][KP], Rs[C][KP], Ks[C][KP], As[C][KP];
-  __shared__ __attribute__((aligned(16))) float Ps[4][C][PP];      // U A^T, U K^T, R A^T, R K^T
+  __shared__ __attribute__((aligned(16))) float Us[C][KP], Rs[C][KP], Ks[C][KP], Bs[C][KP];
+  __shared__ __attribute__((aligned(16))) float Ps[4][C][PP];      // U K^T, U B^T, R K^T, R B^T
   __shared__ __attribute__((aligned(16))) float Ds[RT][16][20];      // the inverses of (I + L)'s diagonal blocks
+  __shared__ __attribute__((aligned(16))) double Dd[RT][16][18];      // the same in 64 bits, the columns in the order 0, 4, 8, 12, 1, ..
+  __shared__ __attribute__((aligned(16))) float ts[2][C];      // the rows' t, of this chunk and the next
   __shared__ double tot[RG][DKP];
   __shared__ __attribute__((aligned(16))) float Wc[DKP];
   const int head = blockIdx.x, groups = (A.window + A.per_group - 1) / A.per_group;
@@ -152,6 +203,7 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
   request(p0);
   for (int p = p0; p < p1; ++p) {
     const int r0 = run0 + p * C, n = run1 - r0 < C ? run1 - r0 : C;
+    float* const tr = ts[(p - p0) % 2];      // (the chunk before may still read its own)
     float* part = delta_chunk_place<DKP>(A, s, p, head);
     // the rows' products of w, and the scaled rows
     double cum[RPT], x = 1.0;
@@ -161,7 +213,15 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
       cum[m] = x;
     }
     tot[q][c] = x;
-    f32x4 vt[RT];
+    if (c < kWave) {      // (this wave's channels, the first 64, are enough for t)
+#pragma unroll
+      for (int m = 0; m < RPT; ++m) {
+        const float kx = own && q * RPT + m < n ? kr[m] : 0.f;
+        const float t = wave_sum(kx * ar[m]) / wave_sum(kx * kx);
+        if (lane == 0) tr[q * RPT + m] = fabsf(t) < INFINITY ? t : 0.f;      // (any number would do; a row of zeros has none)
+      }
+    }
+    f32x4 vt[RT];      // v, later D
 #pragma unroll
     for (int b = 0; b < RT; ++b)
 #pragma unroll
@@ -181,43 +241,71 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
       Us[i][c] = in ? static_cast<float>(ur[m] * before) : 0.f;
       Rs[i][c] = in ? static_cast<float>(rr[m] * W) : 0.f;
       Ks[i][c] = in ? static_cast<float>(kr[m] * inv) : 0.f;
-      As[i][c] = in ? static_cast<float>(ar[m] * inv) : 0.f;
+      Bs[i][c] = in ? static_cast<float>((double(tr[i]) * kr[m] - ar[m]) * inv) : 0.f;
       before = W;
     }
     if (p + 1 < p1) request(p + 1);      // on its way while this chunk is multiplied
     __syncthreads();
-    // the four products of rows with rows, the tiles up to the diagonal
+    // the products of rows with rows, tile t of those up to the diagonal: with K in 64 bits
     constexpr int LT = RT * (RT + 1) / 2;
-#pragma unroll 1
-    for (int job = wave; job < 4 * LT; job += NW) {
-      const int m = job % 4, t = job / 4;
+    auto rows_product = [&](int m, int t) __attribute__((always_inline)) {
       const int bi = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3, bj = t - bi * (bi + 1) / 2;
       const float* left = m < 2 ? &Us[bi * 16 + col][g * 4] : &Rs[bi * 16 + col][g * 4];
-      const float* right = m % 2 == 0 ? &As[bj * 16 + col][g * 4] : &Ks[bj * 16 + col][g * 4];
-      Chains sums[2];
+      const float* right = m % 2 == 0 ? &Ks[bj * 16 + col][g * 4] : &Bs[bj * 16 + col][g * 4];
+      const int above = m < 2 ? 0 : 1;      // the columns of row r that are used are those below r + above
+      if (m % 2 == 0) {
+        Chains64 sums;
 #pragma unroll
-      for (int kk = 0; kk < KT; ++kk) {
-        const float4 a = *reinterpret_cast<const float4*>(left + kk * 16), b = *reinterpret_cast<const float4*>(right + kk * 16);
-        sums[kk % 2].add(a, f32x4{b.x, b.y, b.z, b.w});
-      }
-      const f32x4 acc = sums[0].sum() + sums[1].sum();
+        for (int kk = 0; kk < KT; ++kk) {
+          const float4 b = *reinterpret_cast<const float4*>(right + kk * 16);
+          sums.add(*reinterpret_cast<const float4*>(left + kk * 16), f32x4{b.x, b.y, b.z, b.w});
+        }
+        const f64x4 acc = sums.sum();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = g * 4 + i;
-        Ps[m][bi * 16 + row][bj * 16 + col] = bj < bi || col < row || (col == row && m >= 2) ? acc[i] : 0.f;
+        for (int e = 0; e < 4; ++e) {
+          const int row = 4 * e + g;
+          Ps[m][bi * 16 + row][bj * 16 + col] = bj < bi || col < row + above ? static_cast<float>(acc[e]) : 0.f;
+        }
+      } else {
+        Chains sums[2];
+#pragma unroll
+        for (int kk = 0; kk < KT; ++kk) {
+          const float4 a = *reinterpret_cast<const float4*>(left + kk * 16), b = *reinterpret_cast<const float4*>(right + kk * 16);
+          sums[kk % 2].add(a, f32x4{b.x, b.y, b.z, b.w});
+        }
+        const f32x4 acc = sums[0].sum() + sums[1].sum();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = g * 4 + i;
+          Ps[m][bi * 16 + row][bj * 16 + col] = bj < bi || col < row + above ? acc[i] : 0.f;
+        }
       }
-    }
+    };
+#pragma unroll 1
+    for (int n = 0; n * (NW / 2) + wave / 2 < LT; ++n) rows_product((wave + n) % 2, n * (NW / 2) + wave / 2);
     __syncthreads();
     auto four = [&](int m, int bi, int bj) { return *reinterpret_cast<const float4*>(&Ps[m][bi * 16 + col][bj * 16 + g * 4]); };
-    if (wave < RT) {      // (I + L)^-1 of diagonal block `wave`, a column a lane (every sixteen lanes make the same)
-      float t[16];
+    // the same of U A^T or R A^T, and of a key column of A
+    auto four_a = [&](int m, int bi, int bj) {
+      const float4 x = four(m, bi, bj), y = four(m + 1, bi, bj), t = *reinterpret_cast<const float4*>(&tr[bj * 16 + g * 4]);
+      return float4{fmaf(x.x, t.x, -y.x), fmaf(x.y, t.y, -y.y), fmaf(x.z, t.z, -y.z), fmaf(x.w, t.w, -y.w)};
+    };
+    if (wave < RT) {      // (I + L)^-1 of diagonal block `wave`: X in 32 bits, a column a lane (every sixteen lanes make the same), then X + X (1 - (1 + L) X) in 64
+      float (*const inverse)[20] = Ds[wave];
+      float t[16], rate[16];
+#pragma unroll
+      for (int j = 0; j < 16; j += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(&tr[wave * 16 + j]);
+        rate[j] = x.x; rate[j + 1] = x.y; rate[j + 2] = x.z; rate[j + 3] = x.w;
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         float lrow[16];
 #pragma unroll
-        for (int j = 0; j < 16; j += 4) {
-          const float4 y = *reinterpret_cast<const float4*>(&Ps[0][wave * 16 + i][wave * 16 + j]);
-          lrow[j] = y.x; lrow[j + 1] = y.y; lrow[j + 2] = y.z; lrow[j + 3] = y.w;
+        for (int j = 0; j < i; j += 4) {
+          const float4 x = *reinterpret_cast<const float4*>(&Ps[0][wave * 16 + i][wave * 16 + j]), y = *reinterpret_cast<const float4*>(&Ps[1][wave * 16 + i][wave * 16 + j]);
+          lrow[j] = fmaf(x.x, rate[j], -y.x); lrow[j + 1] = fmaf(x.y, rate[j + 1], -y.y);
+          lrow[j + 2] = fmaf(x.z, rate[j + 2], -y.z); lrow[j + 3] = fmaf(x.w, rate[j + 3], -y.w);
         }
         float y = i == col ? 1.f : 0.f;
 #pragma unroll
@@ -226,35 +314,32 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
       }
       if (g == 0) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) Ds[wave][i][col] = t[i];
+        for (int i = 0; i < 16; ++i) inverse[i][col] = t[i];
       }
-    }
-    f32x4 rhs[RT];
-    if (has_y) {      // lower(U K^T) V
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      // (as it lies in a product's sum, a matrix is the second operand of the next one)
+      f64x4 left, right, rest, l;
 #pragma unroll
-      for (int b = 0; b < RT; ++b) {
-        Chains sums;
-#pragma unroll
-        for (int a = 0; a <= b; ++a) sums.add(four(1, b, a), vt[a]);
-        rhs[b] = sums.sum();
+      for (int e = 0; e < 4; ++e) {
+        const int x = 4 * e + g;
+        left[e] = inverse[col][x];
+        right[e] = inverse[x][col];
+        l[e] = fma(double(Ps[0][wave * 16 + col][wave * 16 + x]), double(tr[wave * 16 + x]), -double(Ps[1][wave * 16 + col][wave * 16 + x]));
+        rest[e] = (x == col ? 1. : 0.) - right[e];
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rest = __builtin_amdgcn_mfma_f64_16x16x4f64(-l[e], right[e], rest, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) right = __builtin_amdgcn_mfma_f64_16x16x4f64(left[e], rest[e], right, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) Dd[wave][4 * e + g][col % 4 * 4 + col / 4] = right[e];
+    } else {      // those with R meanwhile
+      constexpr int others = (NW - RT) / 2;
+      const int w = wave - RT;
+#pragma unroll 1
+      for (int n = 0; n * others + w / 2 < LT; ++n) rows_product(2 + (w + n) % 2, n * others + w / 2);
     }
     __syncthreads();
-    // z = (I + L)^-1 rhs, block by block; left negative, as the products that follow take it
-    auto solve = [&](f32x4 (&z)[RT]) {
-#pragma unroll
-      for (int b = 0; b < RT; ++b) {
-        if (b > 0) {
-          Chains sums;
-#pragma unroll
-          for (int a = 0; a < b; ++a) sums.add(four(0, b, a), z[a]);
-          z[b] += sums.sum();
-        }
-        Chains y;
-        y.add(*reinterpret_cast<const float4*>(&Ds[b][col][g * 4]), z[b]);
-        z[b] = -y.sum();
-      }
-    };
     auto column = [&](const float (&m)[C][KP], int b, int t) {      // four rows of a key column: the first operand of a product with m^T
       const float* at = &m[b * 16 + g * 4][t * 16 + col];
       return float4{at[0], at[KP], at[2 * KP], at[3 * KP]};
@@ -262,45 +347,92 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
     // row tile t of this wave's columns of M, N or Q: 16 x 16 as the next launch's lanes take them
     auto place = [&](float* m, int t) -> float4& { return *reinterpret_cast<float4*>(m + (t * KT + x0 / 16) * 256 + lane * 4); };
     if (has_y) {
-      solve(rhs);
+      f32x4 y[RT];
+#pragma unroll
+      for (int b = 0; b < RT; ++b) {
+        Chains64 own;
+        own.add(four(0, b, b), vt[b]);
+        f64x4 rhs = own.sum();
+        if (b > 0) {      // (terms as small as what there is to learn: 32 bits are enough)
+          Chains learnt, left;
+#pragma unroll
+          for (int a = 0; a < b; ++a) {
+            learnt.add(four(0, b, a), vt[a]);
+            left.add(four(1, b, a), y[a]);
+          }
+          f32x4 before = learnt.sum() + left.sum();
+          turn(before);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) rhs[e] += before[e];
+        }
+        const double* inverse = &Dd[b][col][g * 4];
+        f64x4 z = {0., 0., 0., 0.}, w = {0., 0., 0., 0.};
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          z = __builtin_amdgcn_mfma_f64_16x16x4f64(inverse[e], rhs[e], z, 0, 0, 0);
+          w = __builtin_amdgcn_mfma_f64_16x16x4f64(inverse[e + 1], rhs[e + 1], w, 0, 0, 0);
+        }
+        z += w;
+        turn(z);
+        const float4 t = *reinterpret_cast<const float4*>(&tr[b * 16 + g * 4]);
+        const float te[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y[b][e] = static_cast<float>(z[e]);
+          vt[b][e] = static_cast<float>(fma(-double(te[e]), z[e], double(vt[b][e])));
+        }
+      }
       float* N = part + DKP * DKP;
 #pragma unroll 1
       for (int t = 0; t < KT; ++t) {
-        Chains learnt, lost;
+        Chains learnt, left;
 #pragma unroll
         for (int b = 0; b < RT; ++b) {
           learnt.add(column(Ks, b, t), vt[b]);
-          lost.add(column(As, b, t), rhs[b]);
+          left.add(column(Bs, b, t), y[b]);
         }
-        const f32x4 acc = learnt.sum() + lost.sum();
+        const f32x4 acc = learnt.sum() + left.sum();
         const float4 through = *reinterpret_cast<const float4*>(&Wc[t * 16 + g * 4]);
         place(N, t) = float4{through.x * acc[0], through.y * acc[1], through.z * acc[2], through.w * acc[3]};
       }
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        Chains learnt, lost;
+        Chains learnt, left;
 #pragma unroll
         for (int b = 0; b <= t; ++b) {
-          learnt.add(four(3, t, b), vt[b]);
-          lost.add(four(2, t, b), rhs[b]);
+          learnt.add(four(2, t, b), vt[b]);
+          left.add(four(3, t, b), y[b]);
         }
-        const f32x4 acc = learnt.sum() + lost.sum();
+        const f32x4 acc = learnt.sum() + left.sum();
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           if (vown && t * 16 + g * 4 + i < n) A.o[size_t(r0 + t * 16 + g * 4 + i) * A.ldo + vc] = acc[i];
       }
     }
     if (kBoth || !has_y) {
+      f32x4 x[RT];      // -X, block by block
 #pragma unroll
-      for (int b = 0; b < RT; ++b)
+      for (int b = 0; b < RT; ++b) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) rhs[b][i] = Us[b * 16 + g * 4 + i][x0 + col];
-      solve(rhs);
+        for (int i = 0; i < 4; ++i) x[b][i] = Us[b * 16 + g * 4 + i][x0 + col];
+        if (b > 0) {
+          Chains sums;
+#pragma unroll
+          for (int a = 0; a < b; ++a) sums.add(four_a(0, b, a), x[a]);
+          x[b] += sums.sum();
+        }
+        Chains y;
+        y.add(*reinterpret_cast<const float4*>(&Ds[b][col][g * 4]), x[b]);
+        x[b] = -y.sum();
+      }
 #pragma unroll 1
       for (int t = 0; t < KT; ++t) {
         Chains sums;
 #pragma unroll
-        for (int b = 0; b < RT; ++b) sums.add_turned(column(As, b, t), rhs[b]);
+        for (int b = 0; b < RT; ++b) {
+          const float4 k = column(Ks, b, t), y = column(Bs, b, t), f = *reinterpret_cast<const float4*>(&tr[b * 16 + g * 4]);
+          sums.add_turned(float4{fmaf(k.x, f.x, -y.x), fmaf(k.y, f.y, -y.y), fmaf(k.z, f.z, -y.z), fmaf(k.w, f.w, -y.w)}, x[b]);
+        }
         const f32x4 acc = sums.sum();
         const int key = t * 16 + col, at = x0 + g * 4;
         const float through = Wc[key];
@@ -312,7 +444,7 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
       for (int t = 0; t < RT; ++t) {
         Chains sums;
 #pragma unroll
-        for (int b = 0; b <= t; ++b) sums.add_turned(four(2, t, b), rhs[b]);
+        for (int b = 0; b <= t; ++b) sums.add_turned(four_a(2, t, b), x[b]);
         const f32x4 acc = sums.sum();
         const float4 own = *reinterpret_cast<const float4*>(&Rs[t * 16 + col][x0 + g * 4]);
         place(Q, t) = float4{own.x + acc[0], own.y + acc[1], own.z + acc[2], own.w + acc[3]};

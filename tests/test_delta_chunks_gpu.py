@@ -65,3 +65,38 @@ def test_the_line_between_the_forms():
         assert ops.delta_in_chunks(step(200), heads, d, dv) == takes
     assert not ops.delta_in_chunks(step(200), 4, 64, 64, True)
     assert ops.delta_in_chunks(step(200, 1), 4, 64, 64) and not ops.delta_in_chunks(step(200, 1, 1), 4, 64, 64)      # (runs of similar lengths)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 100])
+@pytest.mark.parametrize("mean", [0, 1, 2, 5])
+def test_keys_that_resemble_each_other(d, mean):
+    """Keys and values around a common row, removed at nearly the whole rate: what a chunk learns is small beside what it says, and the form's errors
+    against 64 bits are no larger than the walk's."""
+    from kvcm_amd import ops
+    heads, T = 8, 512
+    rng = np.random.default_rng(100 * d + mean)
+    f32 = lambda x: x.astype(np.float32)
+    k, v = (f32(rng.normal(size=(T, heads, d)) + mean * rng.normal(size=(1, heads, d))) for _ in range(2))
+    r, u = f32(rng.normal(size=(T, heads, d))), f32(k / np.sqrt((k.astype(np.float64) ** 2).sum(-1, keepdims=True)))
+    sigmoid = lambda x: 1 / (1 + np.exp(-x))
+    w = f32(np.exp(-np.exp(-0.5) * sigmoid(rng.normal(size=(T, heads, d)) - 2)))
+    au = f32(sigmoid(rng.normal(size=(T, heads, d)) + 4) * u)
+    r8, k8, v8, w8, a8, u8 = (x.astype(np.float64) for x in (r, k, v, w, au, u))
+    want, state = np.zeros((T, heads, d)), np.zeros((heads, d, d))
+    for i in range(T):
+        z = np.einsum("hk,hkv->hv", u8[i], state)
+        state = w8[i][:, :, None] * state - a8[i][:, :, None] * z[:, None] + k8[i][:, :, None] * v8[i][:, None]
+        want[i] = np.einsum("hk,hkv->hv", r8[i], state)
+    st = Step([(0, 0, T)])
+    st.max_run = T
+    ops_in = [dev(x.reshape(T, heads * d)) for x in (r, k, v, w, au, u)]
+    errors = []
+    for carry in (None, torch.empty(ops.delta_carry_floats(T, 1, heads, d), device=DEV)):
+        o, S = torch.empty(T, heads * d, device=DEV), torch.zeros(1, heads, d, d, device=DEV)
+        ops.delta_scan(*ops_in, o, S, st, heads, d, d, carry=carry)
+        rel = lambda x, y: np.linalg.norm(x.double().cpu().numpy().reshape(-1) - y.reshape(-1)) / np.linalg.norm(y)
+        errors.append((rel(o, want), rel(S, state)))
+    # root mean squares of T x heads x d and of heads x d x d roundings: alike to a few parts in a hundred from one draw to another
+    for walk, chunks in zip(*errors):
+        assert chunks <= 1.05 * walk, errors
