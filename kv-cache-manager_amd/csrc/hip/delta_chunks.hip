@@ -48,16 +48,19 @@ struct DeltaChunkArgs {
   float* state;
   const int *run_start, *seq_start, *state_slots;
   int heads, dk, dv, col_blocks;
-  float* carry;      // per (sequence, chunk of the window, head): M, N [DKP][DKP], Q [C][DKP] in tiles of 16 x 16
-  int first, window, per_group;      // chunks first .. first + window - 1 of every run; chunks a workgroup takes one after the other
+  float* carry;      // per (chunk, head): M, N [DKP][DKP], Q [C][DKP] in tiles of 16 x 16
+  int first, window, per_group, by_row;      // chunks first .. first + window - 1 of every run; chunks a workgroup takes one after the other
 };
 
 __host__ __device__ constexpr int delta_chunk_rows(int dkp) { return dkp == 64 ? 64 : 32; }
 __host__ __device__ constexpr long long delta_chunk_floats(int dkp) { return 2ll * dkp * dkp + delta_chunk_rows(dkp) * dkp; }
 
+// Where chunk p of sequence s lies.  By row, a run's chunks begin at its first row / C + s: a run of n rows has at most n / C chunks and a part of one, so
+// they never meet, and T / C + S places hold any step.  Scratch for fewer holds `window` chunks of every sequence, and the step goes in turns.
 template <int DKP>
-__device__ __forceinline__ float* delta_chunk_place(const DeltaChunkArgs& A, int s, int p, int head) {
-  return A.carry + ((size_t(s) * A.window + (p - A.first)) * A.heads + head) * delta_chunk_floats(DKP);
+__device__ __forceinline__ float* delta_chunk_place(const DeltaChunkArgs& A, int s, int run0, int p, int head) {
+  const size_t place = A.by_row ? size_t(run0 / delta_chunk_rows(DKP)) + s + p : size_t(s) * A.window + (p - A.first);
+  return A.carry + (place * A.heads + head) * delta_chunk_floats(DKP);
 }
 
 // A sum of products a (16 x 16, a row's four values a lane) times b (16 x 16, as an accumulator lies) in four chains, so that 64 terms are added in
@@ -204,7 +207,7 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
   for (int p = p0; p < p1; ++p) {
     const int r0 = run0 + p * C, n = run1 - r0 < C ? run1 - r0 : C;
     float* const tr = ts[(p - p0) % 2];      // (the chunk before may still read its own)
-    float* part = delta_chunk_place<DKP>(A, s, p, head);
+    float* part = delta_chunk_place<DKP>(A, s, run0, p, head);
     // the rows' products of w, and the scaled rows
     double cum[RPT], x = 1.0;
 #pragma unroll
@@ -481,7 +484,7 @@ __global__ void __launch_bounds__((DKP + delta_chunk_rows(DKP)) / 16 * kWave) de
   float4 m[kAhead][KT];
   f32x4 add[kAhead];
   auto request = [&](int p, int into) {
-    const float* part = delta_chunk_place<DKP>(A, s, p, head);
+    const float* part = delta_chunk_place<DKP>(A, s, run0, p, head);
     const float* rows = (keeps ? part : part + 2 * DKP * DKP) + tile * KT * 256 + lane * 4;
 #pragma unroll
     for (int kk = 0; kk < KT; ++kk) m[into][kk] = *reinterpret_cast<const float4*>(rows + kk * 256);
@@ -537,16 +540,18 @@ template <int DKP>
 static int launch_delta_chunks(DeltaChunkArgs A, int S, int T, int max_run, long long carry_floats, hipStream_t s) {
   constexpr int C = delta_chunk_rows(DKP);
   const int chunks = (max_run + C - 1) / C;
-  const long long column = static_cast<long long>(S) * A.heads * delta_chunk_floats(DKP);      // one chunk of every sequence
-  const long long fit = carry_floats / column;
+  const long long place = A.heads * delta_chunk_floats(DKP), rows = T / C + S;      // (the chunks that a step of T rows has at most)
+  const long long fit = carry_floats / (S * place);      // of every sequence
   KVCM_REQUIRE(fit >= 1, "delta_chunks: the scratch is too small");
-  A.window = static_cast<int>(fit < chunks ? fit : chunks);
+  A.by_row = carry_floats / place >= rows;
+  A.window = static_cast<int>(A.by_row || chunks < fit ? chunks : fit);
   // one workgroup a CU: some chunks in a row, whose rows are asked for while the one before is multiplied, once there is more than one a CU
-  const long long most = static_cast<long long>(S) * A.window, rows = T / C + S;      // (chunks of this many rows, a part of one in every sequence)
+  const long long most = static_cast<long long>(S) * A.window;
   const long long turns = (A.heads * (most < rows ? most : rows) + 255) / 256;
   A.per_group = static_cast<int>(turns < 8 ? turns : 8);
+  const int limit = 65535 / S * A.per_group;
+  if (A.window > limit) A.window = limit;
   const long long groups = static_cast<long long>(S) * ((A.window + A.per_group - 1) / A.per_group);
-  KVCM_REQUIRE(groups <= 65535, "delta_chunks: too many sequences and chunks for one launch");
   for (A.first = 0; A.first < chunks; A.first += A.window) {
     delta_chunk_kernel<DKP><<<dim3(A.heads, static_cast<unsigned>(groups)), kDeltaThreads, 0, s>>>(A);
     delta_pass_kernel<DKP><<<dim3(A.heads * A.col_blocks, S), (DKP + C) / 16 * kWave, 0, s>>>(A);
@@ -578,7 +583,7 @@ int kvcm_delta_chunks(const float* r, int ldr, const float* k, int ldk, const fl
   KVCM_REQUIRE(S <= 65535 && heads <= (1 << 20), "delta_chunks: too many sequences or heads for one launch");
   KVCM_REQUIRE(ldr >= heads * dk && ldk >= heads * dk && ldv >= heads * dv && ldo >= heads * dv, "delta_chunks: row strides too small");
   KVCM_REQUIRE(carry && reinterpret_cast<uintptr_t>(carry) % 16 == 0, "delta_chunks: the scratch must be there, 16-byte aligned");
-  DeltaChunkArgs A = {r, k, v, w, au, u, ldr, ldk, ldv, o, ldo, state, run_start, seq_start, state_slots, heads, dk, dv, (dv + 15) / 16, carry, 0, 0, 0};
+  DeltaChunkArgs A = {r, k, v, w, au, u, ldr, ldk, ldv, o, ldo, state, run_start, seq_start, state_slots, heads, dk, dv, (dv + 15) / 16, carry, 0, 0, 0, 0};
   if (dk <= 64) return launch_delta_chunks<64>(A, S, T, max_run, carry_floats, s);
   return launch_delta_chunks<128>(A, S, T, max_run, carry_floats, s);
 }

@@ -100,3 +100,44 @@ def test_keys_that_resemble_each_other(d, mean):
     # root mean squares of T x heads x d and of heads x d x d roundings: alike to a few parts in a hundred from one draw to another
     for walk, chunks in zip(*errors):
         assert chunks <= 1.05 * walk, errors
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,d,dv,runs", [(32, 64, 64, (1100, 700)), (32, 64, 33, (1024, 1)), (40, 48, 48, (509, 100, 509)), (16, 128, 128, (600, 333, 32)),
+                                             (24, 90, 128, (777, 1))])
+def test_chunks_one_after_the_other(heads, d, dv, runs):
+    """More chunks than workgroups at once: outputs and states of steps that take all of the scratch, each run in places of its own, against 64 bits, and
+    bit for bit those of scratch for some chunks of every sequence, which a workgroup's turns do not divide."""
+    from kvcm_amd import ops
+    T, D = sum(runs), heads * d
+    g = torch.Generator(device=DEV).manual_seed(heads + d)
+    r, k, v = (torch.randn(T, heads, c, generator=g, device=DEV) for c in (d, d, dv))
+    u = k / (k.norm(dim=-1, keepdim=True) + 1e-6)
+    w = torch.exp(-0.6065306 * torch.rand(T, heads, d, generator=g, device=DEV) ** 3)
+    au = torch.rand(T, heads, d, generator=g, device=DEV) * u
+    first = torch.randn(len(runs), heads, d, dv, generator=g, device=DEV)
+    r8, k8, v8, w8, a8, u8 = (x.double() for x in (r, k, v, w, au, u))
+    state, want, row = first.double(), torch.empty(T, heads, dv, dtype=torch.float64, device=DEV), 0
+    for s, n in enumerate(runs):
+        for i in range(row, row + n):
+            z = (u8[i].unsqueeze(-1) * state[s]).sum(1, keepdim=True)
+            state[s] = w8[i].unsqueeze(-1) * state[s] - a8[i].unsqueeze(-1) * z + k8[i].unsqueeze(-1) * v8[i].unsqueeze(1)
+            want[i] = (r8[i].unsqueeze(-1) * state[s]).sum(1)
+        row += n
+    st = Step([(i, 5, n) for i, n in enumerate(runs)])
+    st.max_run = max(runs)
+    assert ops.delta_in_chunks(st, heads, d, dv) or 2 * T < len(runs) * max(runs)
+    full, one = ops.delta_carry_floats(T, len(runs), heads, d), int(ops.lib().kvcm_delta_carry_floats(len(runs), 1, heads, d))
+    flat, got = (lambda x: x.reshape(T, -1).contiguous()), []
+    for floats in (full, 5 * one, 3 * one):
+        o, S = torch.full((T, heads * dv), float("nan"), device=DEV), first.clone()
+        carry = torch.full((floats,), float("nan"), device=DEV)
+        a = [flat(x) for x in (r, k, v, w, au, u)]
+        ops._call("kvcm_delta_chunks", ops._ptr(a[0]), D, ops._ptr(a[1]), D, ops._ptr(a[2]), heads * dv, ops._ptr(a[3]), ops._ptr(a[4]), ops._ptr(a[5]),
+                  ops._ptr(o), heads * dv, ops._ptr(S), ops._ptr(st.run_start), ops._ptr(st.seq_start), ops._ptr(st.state_slots), len(runs), heads, d, dv, T,
+                  max(runs), ops._ptr(carry), floats, ops._stream())
+        got.append((o, S))
+        assert torch.equal(o, got[0][0]) and torch.equal(S, got[0][1])
+    # as the walk's: sums of up to 128 keys a row, handed on by a state that forgets
+    for x, y in zip(got[0], (want, state)):
+        assert float((x.double().view_as(y) - y).abs().max()) < 5e-5 * max(1.0, float(y.abs().max()))
