@@ -21,13 +21,14 @@
 // matrix cores (v_mfma_f32_16x16x4_f32) like all the rest.
 //
 // The quotients: w is exp(-exp(-1/2) sigmoid(.)), so 0.545 < w <= 1, W of 64 rows is above 1e-17 and a factor W_i / W_j of a term that is used is at
-// most one and has the relative error of a few roundings.  What lies above the diagonals may be large and is left out by selection.  (What is
-// not finite in a row reaches the rows of its chunk in front of it too.)
+// most one and has the relative error of a few roundings.  What lies above the diagonals may be large and is left out by selection.  A value
+// that is not finite cannot be: the matrix cores multiply it by the diagonal blocks' zeros, and rows in front of it would see it.  A chunk whose X or Y holds one is
+// walked over again row by row (walk_chunk).
 //
 // Errors against 64 bits as parts of the walk's: keys and values with a common mean of 0 to 5 times their spread, rates of removal around 0.05 to 0.98:
 // outputs 0.54 .. 0.86, states 0.64 .. 0.99; in 32 bits, with N and the outputs as the plain differences above, up to 4.2 times the walk's.
-// us, walk / so / with those differences: 32 heads of 64 x 64, 2,048 tokens 291 / 147 / 125, 512 72 / 42 / 37, 192 29.3 / 31.4 / 25.7, 3 of 1,024
-// 332 / 240 / 196; 32 heads of 128 x 128, 2,048 tokens 711 / 359 / 322, 4 of 1,024 1,328 / 721 / 657.
+// us, walk / so / with those differences: 32 heads of 64 x 64, 2,048 tokens 291 / 152 / 125, 512 72 / 43 / 37, 192 29 / 33 / 26, 3 of 1,024
+// 332 / 249 / 196; 32 heads of 128 x 128, 2,048 tokens 711 / 364 / 322, 4 of 1,024 1,328 / 733 / 657.
 //
 // A workgroup of the first kernel is eight waves, one a CU: four matrices of C rows by the keys and four of C by C in LDS, a wave with 16 columns of
 // X or Y in registers throughout, whose accumulators are the next product's second operand as they lie (key 4 g + e of lane group g is element e; the ones of
@@ -124,6 +125,39 @@ __device__ __forceinline__ void turn(f64x4& v) {
 
 constexpr int kDeltaThreads = 512;
 
+// The same M, N, Q and outputs of a chunk by the recurrence itself, started from the identity (M) and from nothing (N): a thread has a column of either
+// and keeps it where the next launch reads it.  (About 2 ms a chunk of 64 rows: for chunks that hold what is not finite.)
+template <int DKP>
+__device__ __forceinline__ void walk_chunk(const DeltaChunkArgs& A, float* part, int head, size_t r0, int n) {
+  constexpr int KT = DKP / 16;
+  if (threadIdx.x >= 2 * DKP) return;
+  const bool of_v = threadIdx.x >= DKP;
+  const int x = threadIdx.x % DKP, dk = A.dk;
+  const size_t D = size_t(A.heads) * dk, kc = size_t(head) * dk;
+  auto m_at = [&](int key) { return (key / 16 * KT + x / 16) * 256 + (x % 16 / 4 * 16 + key % 16) * 4 + x % 4; };
+  float* const Q = part + 2 * DKP * DKP;
+  float* const column = of_v ? part + DKP * DKP + x / 16 * 256 + x % 16 * 4 : part + m_at(0);
+  auto at = [&](int key) -> float& { return column[of_v ? key / 16 * KT * 256 + key % 16 / 4 * 64 + key % 4 : m_at(key) - m_at(0)]; };
+  for (int key = 0; key < DKP; ++key) at(key) = !of_v && key == x ? 1.f : 0.f;
+  for (int i = 0; i < n; ++i) {
+    const size_t row = r0 + i;
+    const float *w = A.w + row * D + kc, *u = A.u + row * D + kc, *au = A.au + row * D + kc, *r = A.r + row * A.ldr + kc, *k = A.k + row * A.ldk + kc;
+    const float v = of_v && x < A.dv ? A.v[row * A.ldv + size_t(head) * A.dv + x] : 0.f;
+    float z = 0.f, o = 0.f;
+#pragma unroll 4
+    for (int key = 0; key < dk; ++key) z = fmaf(u[key], at(key), z);
+#pragma unroll 4
+    for (int key = 0; key < dk; ++key) {
+      float m = fmaf(w[key], at(key), -au[key] * z);
+      if (of_v) m = fmaf(k[key], v, m);
+      at(key) = m;
+      o = fmaf(r[key], m, o);
+    }
+    if (!of_v) Q[m_at(i)] = o;
+    else if (x < A.dv) A.o[row * A.ldo + size_t(head) * A.dv + x] = o;
+  }
+}
+
 template <int DKP>
 __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkArgs A) {
   constexpr int C = delta_chunk_rows(DKP), RT = C / 16, KT = DKP / 16, KP = DKP + 4, PP = C + 4, NW = kDeltaThreads / kWave;
@@ -135,6 +169,7 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
   __shared__ __attribute__((aligned(16))) float Ds[RT][16][20];      // the inverses of (I + L)'s diagonal blocks
   __shared__ __attribute__((aligned(16))) double Dd[RT][16][18];      // the same in 64 bits, the columns in the order 0, 4, 8, 12, 1, ..
   __shared__ __attribute__((aligned(16))) float ts[2][C];      // the rows' t, of this chunk and the next
+  __shared__ int bad;      // the chunk that is not finite
   __shared__ double tot[RG][DKP];
   __shared__ __attribute__((aligned(16))) float Wc[DKP];
   const int head = blockIdx.x, groups = (A.window + A.per_group - 1) / A.per_group;
@@ -203,6 +238,7 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
         }
     }
   };
+  if (tid == 0) bad = -1;
   request(p0);
   for (int p = p0; p < p1; ++p) {
     const int r0 = run0 + p * C, n = run1 - r0 < C ? run1 - r0 : C;
@@ -295,24 +331,21 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
     };
     if (wave < RT) {      // (I + L)^-1 of diagonal block `wave`: X in 32 bits, a column a lane (every sixteen lanes make the same), then X + X (1 - (1 + L) X) in 64
       float (*const inverse)[20] = Ds[wave];
-      float t[16], rate[16];
+      f64x4 l;      // row `col` of L, columns 4 e + g
 #pragma unroll
-      for (int j = 0; j < 16; j += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(&tr[wave * 16 + j]);
-        rate[j] = x.x; rate[j + 1] = x.y; rate[j + 2] = x.z; rate[j + 3] = x.w;
+      for (int e = 0; e < 4; ++e) {
+        const int x = 4 * e + g;
+        l[e] = fma(double(Ps[0][wave * 16 + col][wave * 16 + x]), double(tr[wave * 16 + x]), -double(Ps[1][wave * 16 + col][wave * 16 + x]));
       }
+      float t[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        float lrow[16];
-#pragma unroll
-        for (int j = 0; j < i; j += 4) {
-          const float4 x = *reinterpret_cast<const float4*>(&Ps[0][wave * 16 + i][wave * 16 + j]), y = *reinterpret_cast<const float4*>(&Ps[1][wave * 16 + i][wave * 16 + j]);
-          lrow[j] = fmaf(x.x, rate[j], -y.x); lrow[j + 1] = fmaf(x.y, rate[j + 1], -y.y);
-          lrow[j + 2] = fmaf(x.z, rate[j + 2], -y.z); lrow[j + 3] = fmaf(x.w, rate[j + 3], -y.w);
-        }
         float y = i == col ? 1.f : 0.f;
 #pragma unroll
-        for (int j = 0; j < i; ++j) y = fmaf(-lrow[j], t[j], y);
+        for (int j = 0; j < i; ++j) {      // (L's element is in another lane: one scalar for all)
+          const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(static_cast<float>(l[j / 4])), j % 4 * 16 + i));
+          y = fmaf(-x, t[j], y);
+        }
         t[i] = y;
       }
       if (g == 0) {
@@ -321,13 +354,12 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
       }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       // (as it lies in a product's sum, a matrix is the second operand of the next one)
-      f64x4 left, right, rest, l;
+      f64x4 left, right, rest;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int x = 4 * e + g;
         left[e] = inverse[col][x];
         right[e] = inverse[x][col];
-        l[e] = fma(double(Ps[0][wave * 16 + col][wave * 16 + x]), double(tr[wave * 16 + x]), -double(Ps[1][wave * 16 + col][wave * 16 + x]));
         rest[e] = (x == col ? 1. : 0.) - right[e];
       }
 #pragma unroll
@@ -349,6 +381,7 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
     };
     // row tile t of this wave's columns of M, N or Q: 16 x 16 as the next launch's lanes take them
     auto place = [&](float* m, int t) -> float4& { return *reinterpret_cast<float4*>(m + (t * KT + x0 / 16) * 256 + lane * 4); };
+    bool odd = false;      // (what is not finite, times nothing, is not nothing)
     if (has_y) {
       f32x4 y[RT];
 #pragma unroll
@@ -384,6 +417,8 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
           y[b][e] = static_cast<float>(z[e]);
           vt[b][e] = static_cast<float>(fma(-double(te[e]), z[e], double(vt[b][e])));
         }
+        const f32x4 none = 0.f * y[b] + 0.f * vt[b];
+        odd |= __any((none[0] + none[1]) + (none[2] + none[3]) != 0.f);
       }
       float* N = part + DKP * DKP;
 #pragma unroll 1
@@ -427,6 +462,8 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
         Chains y;
         y.add(*reinterpret_cast<const float4*>(&Ds[b][col][g * 4]), x[b]);
         x[b] = -y.sum();
+        const f32x4 none = 0.f * x[b];
+        odd |= __any((none[0] + none[1]) + (none[2] + none[3]) != 0.f);
       }
 #pragma unroll 1
       for (int t = 0; t < KT; ++t) {
@@ -453,6 +490,9 @@ __global__ void __launch_bounds__(kDeltaThreads) delta_chunk_kernel(DeltaChunkAr
         place(Q, t) = float4{own.x + acc[0], own.y + acc[1], own.z + acc[2], own.w + acc[3]};
       }
     }
+    if (odd && lane == 0) bad = p;
+    __syncthreads();
+    if (bad == p) walk_chunk<DKP>(A, delta_chunk_place<DKP>(A, s, run0, p, head), head, run0 + p * C, n);
   }
 }
 

@@ -1765,9 +1765,9 @@ DELTA_CARRY = 9 << 22        # 32-bit values of scratch that ``delta_scan``'s ma
 def delta_in_chunks(step, heads, dk, dv, one_order=False):
     """Does ``delta_scan``, given scratch for the chunks, take this step's runs in matrix form (csrc/hip/delta_chunks.hip)?  It is worth it
     where the walk waits for its own chain, and while runs are of similar lengths (a single token takes
-    a whole chunk's work).  us, walk / so: 32 heads of 64 x 64, one run of 192 rows 29.3 / 31.4, 256 39 / 33, 512 72 / 42, 2,048 291 / 147, 3 of 1,024
-    332 / 240, one of 1,024 beside a single token 149 / 98; 4 heads, one run of 192 rows 22 / 31, 256 28 / 32, 384 41 / 34; 32 heads of 128 x 128, one run of 128 rows 46 / 38, 2,048 711 / 359,
-    4 of 1,024 1,328 / 721, 8 of 256 604 / 397; 4 heads, one run of 128 rows 25 / 37."""
+    a whole chunk's work).  us, walk / so: 32 heads of 64 x 64, one run of 192 rows 29 / 33, 256 39 / 34, 512 72 / 43, 2,048 291 / 152, 3 of 1,024
+    332 / 249, one of 1,024 beside a single token 149 / 98; 4 heads, one run of 192 rows 22 / 31, 256 28 / 32, 384 41 / 34; 32 heads of 128 x 128, one run of 128 rows 46 / 39, 2,048 711 / 364,
+    4 of 1,024 1,328 / 733, 8 of 256 604 / 401; 4 heads, one run of 128 rows 25 / 37."""
     if (one_order or not 32 < dk <= 128 or dv > (64 if dk <= 64 else 128) or 2 * step.rows < step.seqs * step.max_run
             or int(lib().kvcm_delta_carry_floats(step.seqs, 1, heads, dk)) > DELTA_CARRY):
         return False

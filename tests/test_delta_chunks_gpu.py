@@ -141,3 +141,38 @@ def test_chunks_one_after_the_other(heads, d, dv, runs):
     # as the walk's: sums of up to 128 keys a row, handed on by a state that forgets
     for x, y in zip(got[0], (want, state)):
         assert float((x.double().view_as(y) - y).abs().max()) < 5e-5 * max(1.0, float(y.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["v", "k", "r", "au", "u"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("d", [64, 100])
+def test_what_is_not_finite_stays_behind_its_row(d, value, what):
+    """Rows in front of a value that is not finite are as if it were not there, whatever the place of its row in a chunk; from it on, what the walk says is finite is."""
+    from kvcm_amd import ops
+    heads, runs = 2, (200, 192, 256)
+    T, D = sum(runs), heads * d
+    st = Step([(i, 5, n) for i, n in enumerate(runs)])
+    st.max_run = max(runs)
+    g = torch.Generator(device=DEV).manual_seed(d)
+    a = {x: torch.randn(T, D, generator=g, device=DEV) for x in ("r", "k", "v")}
+    a["w"] = torch.exp(-0.6065306 * torch.rand(T, D, generator=g, device=DEV))
+    a["u"] = a["k"] / d ** 0.5
+    a["au"] = a["u"] * torch.rand(T, D, generator=g, device=DEV)
+    first = torch.randn(len(runs), heads, d, d, generator=g, device=DEV)
+    clean = {x: y.clone() for x, y in a.items()}
+    for row, channel in ((75, 3), (200 + 64 + 30, d + 1), (392 + 37, 20)):      # (in the second head's first run of rows too)
+        a[what][row, channel] = value
+    out = []
+    for q, carry in ((clean, True), (a, True), (a, False)):
+        o, S = torch.full((T, D), 7.0, device=DEV), first.clone()
+        kw = dict(carry=torch.full((ops.delta_carry_floats(T, len(runs), heads, d),), float("nan"), device=DEV)) if carry else {}
+        ops.delta_scan(q["r"], q["k"], q["v"], q["w"], q["au"], q["u"], o, S, st, heads, d, d, **kw)
+        out.append((o, S))
+    (same, state), (o, S), (walk, walked) = out
+    assert torch.isfinite(same).all() and not torch.isfinite(o).all()
+    # where the walk's numbers are finite, ours are, and as near as two orders of the same sums are (as above)
+    for x, y, ref in ((o, walk, same), (S, walked, state)):
+        assert torch.equal(torch.isfinite(x), torch.isfinite(y))
+        ok = torch.isfinite(y)
+        assert float((x[ok] - y[ok]).abs().max()) < 1e-4 * float(ref.abs().max())
