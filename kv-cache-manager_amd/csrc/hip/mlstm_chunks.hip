@@ -18,8 +18,7 @@
 // of 64, 128, 256 rows: 84, 78, 90), 8 of 509 228 / 128, 32 heads of 128 x 128 550 / 197, 64 heads of 16 x 16, 1,024 tokens 153 / 61.
 // Error against 64 bits of outputs and states, the walk / so: 1.1e-6 / 1.0e-6 and 4.5e-7 / 5.0e-7 (2,048 tokens).
 // A workgroup is eight waves on 64 value columns of a head: a row tile of 16 belongs to two waves, which halve its columns.  Key sizes beyond 128
-// do not fit LDS, and 32-bit storage, where a row's result must not depend on where its run began, keeps the walk.  (What is not
-// finite in a row's k or v reaches the rows of its chunk in front of it too.)
+// do not fit LDS, and 32-bit storage, where a row's result must not depend on where its run began, keeps the walk.
 #include "common.h"
 #include "kvcm_hip.h"
 #include "mlstm.h"
@@ -102,6 +101,7 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
   __shared__ float ts[C], ls[C];
   __shared__ float out[C];                   // D(63, j)
   __shared__ __attribute__((aligned(16))) float Ns[DKP];
+  __shared__ int odd;      // the chunk whose values are not all finite
   __shared__ float sums[PARTS ? 1 : 2][C], nq[PARTS ? 1 : C];
   const int head = blockIdx.x / A.col_blocks, c0 = (blockIdx.x % A.col_blocks) * DVT;
   const int s = blockIdx.y / A.pieces_per_seq, p = blockIdx.y % A.pieces_per_seq;
@@ -184,6 +184,7 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
     creg = row < rows ? c : float4{1.f, 0.f, 1.f, 0.f};
   };
 
+  if (tid == 0) odd = -1;
   request(r0);
   for (int t0 = r0; t0 < r1; t0 += C) {
     const int n = r1 - t0 < C ? r1 - t0 : C;
@@ -197,6 +198,10 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
     for (int m = 0; m < VQ; ++m) {
       const int e = tid + m * NT;
       *reinterpret_cast<float4*>(&Vs[e / (DVT / 4)][(e % (DVT / 4)) * 4]) = vreg[m];
+      if constexpr (!PARTS) {      // (what is not finite, times nothing, is not nothing)
+        const float none = 0.f * ((vreg[m].x + vreg[m].y) + (vreg[m].z + vreg[m].w));
+        if (none != 0.f) odd = t0;
+      }
     }
     if (tid < C) {
       ks[tid] = creg.x;
@@ -319,8 +324,9 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
 #pragma unroll
           for (int ct = 0; ct < CT; ++ct) acc[ct][i] *= d;
         }
+        const int whole = __builtin_amdgcn_readfirstlane(odd == t0 ? wave : wave + 1);      // tiles for the matrix cores, which multiply by zeros too
 #pragma unroll 1
-        for (int jt = 0; jt <= wave; ++jt) {
+        for (int jt = 0; jt < whole; ++jt) {
           const float4 pf = *reinterpret_cast<const float4*>(&Ps[wave][col][jt * 16 + g * 4]);
           const float pe[4] = {pf.x, pf.y, pf.z, pf.w};
 #pragma unroll
@@ -328,6 +334,17 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
               acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(pe[e], Vs[jt * 16 + g * 4 + e][cw + ct * 16 + col], acc[ct], 0, 0, 0);
+        }
+        if (whole == wave) {      // rows in front of what is not finite must not see it: the last tile's sums without its zeros
+#pragma unroll 1
+          for (int j = 0; j < 16; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int ct = 0; ct < CT; ++ct) {
+                const float x = Ps[wave][g * 4 + i][wave * 16 + j] * Vs[wave * 16 + j][cw + ct * 16 + col];
+                acc[ct][i] += j <= g * 4 + i ? x : 0.f;
+              }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {

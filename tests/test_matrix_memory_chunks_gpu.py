@@ -68,3 +68,34 @@ def test_the_line_between_the_forms():
     short, long = Step([(0, 0, 255), (1, 0, 3)]), Step([(0, 0, 256), (1, 0, 3)])
     short.max_run, long.max_run = 255, 256
     assert not ops.mlstm_in_chunks(short, 64) and ops.mlstm_in_chunks(long, 128) and not ops.mlstm_in_chunks(long, 129)
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("d,dv", [(64, 64), (100, 20)])
+def test_what_is_not_finite_stays_behind_its_row(d, dv, value, what):
+    """Rows in front of a value that is not finite are as if it were not there, whatever the place of its row in a chunk; from it on, what the walk says is finite is."""
+    from kvcm_amd import ops
+    heads, runs = 2, (300, 200, 256)
+    T = sum(runs)
+    st = Step([(i, 5, n) for i, n in enumerate(runs)])
+    st.max_run = max(runs)
+    g = torch.Generator(device=DEV).manual_seed(d)
+    a = {x: torch.randn(T, heads * c, generator=g, device=DEV).abs() for x, c in (("q", d), ("k", d), ("v", dv))}      # (a divisor without cancellation)
+    gates = torch.randn(2, T, heads, generator=g, device=DEV)
+    first = [torch.rand(len(runs), heads, *c, generator=g, device=DEV) for c in ((d, dv), (d,), ())]
+    clean = {x: y.clone() for x, y in a.items()}
+    for row, channel in ((75, 3), (300 + 64 + 30, heads * (dv if what == "v" else d) - 2), (500 + 37, 9)):
+        a[what][row, channel] = value
+    out = []
+    for q, carry in ((clean, True), (a, True), (a, False)):
+        o, states = torch.full((T, heads * dv), 7.0, device=DEV), [x.clone() for x in first]
+        kw = dict(carry=torch.full((ops.mlstm_carry_floats(T, len(runs), heads, d, dv),), float("nan"), device=DEV)) if carry else {}
+        ops.mlstm_scan(q["q"], q["k"], q["v"], gates[0], gates[1], torch.zeros(heads, device=DEV), torch.full((heads,), 4.0, device=DEV), 15.0, d ** -0.5,
+                       torch.empty(T, 4 * heads, device=DEV), torch.empty(len(runs) * heads * d, device=DEV), o, *states, st, heads, d, dv, **kw)
+        out.append((o, *states))
+    assert all(torch.isfinite(x).all() for x in out[0]) and not torch.isfinite(out[1][0]).all()
+    for ref, x, y in zip(*out):
+        assert torch.equal(torch.isfinite(x), torch.isfinite(y))
+        ok = torch.isfinite(y)
+        assert float((x[ok] - y[ok]).abs().max()) < 6e-5 * float(ref.abs().max())      # both within 3e-5 of the recurrence, as above
