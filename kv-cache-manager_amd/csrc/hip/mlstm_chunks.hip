@@ -16,7 +16,8 @@
 // 32 heads of 64 x 64 (matrix instructions 11, the vectors' bytes 11, vector instructions 13, LDS 8), and the workgroups, two a CU, are all in the same
 // phase: 42 us for the last launch, 14 for the pieces' own parts, 7 between, 15 for the factors.  us, the walk / so: one sequence of 2,048 tokens 300 / 78 (pieces
 // of 64, 128, 256 rows: 84, 78, 90), 8 of 509 228 / 128, 32 heads of 128 x 128 550 / 197, 64 heads of 16 x 16, 1,024 tokens 153 / 61.
-// Error against 64 bits of outputs and states, the walk / so: 1.1e-6 / 1.0e-6 and 4.5e-7 / 5.0e-7 (2,048 tokens).
+// Errors against 64 bits as parts of the walk's (1,024 tokens, 64 heads of 64 and 128, keys and queries with and without a common mean): outputs 0.35 .. 1.0,
+// states 0.99 .. 1.01 (both have the factors' own roundings; with the factors' products in 32 bits 1.03 .. 1.16), normalizers 0.90 .. 0.98.
 // A workgroup is eight waves on 64 value columns of a head: a row tile of 16 belongs to two waves, which halve its columns.  Key sizes beyond 128
 // do not fit LDS, and 32-bit storage, where a row's result must not depend on where its run began, keeps the walk.
 #include "common.h"
@@ -66,14 +67,15 @@ __device__ __forceinline__ float4 row_four(const float* base, int row, int i, in
 }
 
 // lane l: the product of x over lanes l + 1 .. 63
-__device__ __forceinline__ float product_above(float x, int lane) {
+template <typename T>
+__device__ __forceinline__ T product_above(T x, int lane) {
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
-    const float y = __shfl_down(x, d, kWave);
+    const T y = __shfl_down(x, d, kWave);
     x = lane + d < kWave ? x * y : x;
   }
-  const float y = __shfl_down(x, 1, kWave);
-  return lane == kWave - 1 ? 1.f : y;
+  const T y = __shfl_down(x, 1, kWave);
+  return lane == kWave - 1 ? T(1) : y;
 }
 
 __device__ __forceinline__ float first_lane(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
@@ -154,7 +156,7 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
     const float x = PARTS ? 0.f : part[size_t(dk) * dv + (tid < dk ? tid : 0)];
     Ns[tid] = tid < dk ? x : 0.f;
   }
-  float kept = 1.f;
+  double kept = 1.;
 
   constexpr int KQ = C * DKP / 4 / NT, VQ = C * DVT / 4 / NT;
   float4 kreg[KQ], vreg[VQ], qreg[PARTS ? 1 : KS], creg;
@@ -209,9 +211,9 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
       ls[tid] = creg.z;
     }
     // (every wave has the factors of all rows, one a lane)
-    const float above = product_above(creg.x, lane);
-    if (tid < C) out[tid] = creg.y * above;
-    const float through = first_lane(creg.x * above);      // D(63)
+    const double above = product_above(double(creg.x), lane);      // (an error here is every element's of the state: 64 bits)
+    if (tid < C) out[tid] = static_cast<float>(creg.y * above);
+    const float through = first_lane(static_cast<float>(creg.x * above));      // D(63)
     float4 qf[PARTS ? 1 : KS];
     // keep_0 .. keep_(16 wave - 1); lane j: take_j keep_(j+1) .. keep_(16 wave - 1); lane l: keep_(16 wave) .. keep_(16 wave + l % 16)
     float entered = 1.f, before = 1.f, within = 1.f;
@@ -415,7 +417,7 @@ __global__ void __launch_bounds__(kChunkThreads, DKP == 64 ? 4 : 2) mlstm_chunk_
           if (key < dk) ndst[key] = Ns[key];      // (this lane wrote it)
         }
       }
-      if (PARTS && tid == 0) part[size_t(dk) * dv + dk] = kept;
+      if (PARTS && tid == 0) part[size_t(dk) * dv + dk] = static_cast<float>(kept);
     }
   }
 }

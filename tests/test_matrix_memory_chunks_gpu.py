@@ -99,3 +99,52 @@ def test_what_is_not_finite_stays_behind_its_row(d, dv, value, what):
         assert torch.equal(torch.isfinite(x), torch.isfinite(y))
         ok = torch.isfinite(y)
         assert float((x[ok] - y[ok]).abs().max()) < 6e-5 * float(ref.abs().max())      # both within 3e-5 of the recurrence, as above
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_errors_of_long_runs_are_the_walks(d):
+    """Runs of many pieces that are gone on with: outputs, states, normalizers and maxima against 64 bits, with errors as the walk's."""
+    from kvcm_amd import ops
+    heads, parts, cap = 16, ((513, 1025, 1500), (300, 257, 700)), 15.0
+    seqs, total = 3, [813, 1282, 2200]
+    g = torch.Generator(device=DEV).manual_seed(d)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    data = [[draw(n, heads, d) + draw(1, heads, d), draw(n, heads, d) + draw(1, heads, d), draw(n, heads, d), draw(n, heads), draw(n, heads)] for n in total]
+    bi, bf = draw(heads) * 0.1 - 1, torch.linspace(3, 6, heads, device=DEV)
+    want, states = [], []
+    for q, k, v, gi, gf in data:
+        soft = lambda x: cap * torch.tanh(x.double() / cap)
+        li, lf = soft(gi + bi), torch.nn.functional.logsigmoid(soft(gf + bf))
+        S, n, m = (torch.zeros(heads, *x, dtype=torch.float64, device=DEV) for x in ((d, d), (d,), ()))
+        o = torch.empty(q.shape, dtype=torch.float64, device=DEV)
+        q, k, v = q.double() * d ** -0.5, k.double(), v.double()
+        for t in range(q.shape[0]):
+            m1 = torch.maximum(lf[t] + m, li[t])
+            keep, take, m = torch.exp(lf[t] + m - m1), torch.exp(li[t] - m1), m1
+            S = keep[:, None, None] * S + (take[:, None] * k[t]).unsqueeze(2) * v[t].unsqueeze(1)
+            n = keep[:, None] * n + take[:, None] * k[t]
+            o[t] = (q[t].unsqueeze(2) * S).sum(1) / (torch.maximum((n * q[t]).sum(-1).abs(), torch.exp(-m)) + 1e-6)[:, None]
+        want.append(o)
+        states.append((S, n, m))
+    errors = []
+    for chunks in (False, True):
+        S, N, M = (torch.full((seqs, heads, *x), 7.0, device=DEV) for x in ((d, d), (d,), ()))
+        at, outs = [0] * seqs, [[] for _ in range(seqs)]
+        for part in parts:
+            st = Step([(i, at[i], n) for i, n in enumerate(part)])
+            st.max_run = max(part)
+            rows = [torch.cat([x[j][at[i]:at[i] + n].flatten(1) for i, (x, n) in enumerate(zip(data, part))]) for j in range(5)]
+            o = torch.full((st.rows, heads * d), float("nan"), device=DEV)
+            kw = dict(carry=torch.full((ops.mlstm_carry_floats(st.rows, seqs, heads, d, d),), float("nan"), device=DEV)) if chunks else {}
+            assert ops.mlstm_in_chunks(st, d)
+            ops.mlstm_scan(*rows, bi, bf, cap, d ** -0.5, torch.empty(st.rows, 4 * heads, device=DEV), torch.empty(seqs * heads * d, device=DEV), o, S, N, M, st,
+                           heads, d, d, **kw)
+            for i, x in enumerate(o.split(list(part))):
+                outs[i].append(x.view(-1, heads, d))
+                at[i] += part[i]
+        rel = lambda x, y: float((x.double() - y).norm() / y.norm())
+        errors.append((rel(torch.cat([torch.cat(x) for x in outs]), torch.cat(want)), *(rel(x, torch.stack([y[j] for y in states])) for j, x in enumerate((S, N, M)))))
+    walk, chunks = errors
+    assert walk[0] < 3e-5 and max(walk[1:]) < 3e-6, errors      # (the outputs' divisor n . q cancels)
+    # a state's error is that of the factors, which the forms share; what each adds is a few parts in a hundred of it
+    assert all(x <= 1.03 * y for x, y in zip(chunks, walk)), errors
