@@ -117,7 +117,8 @@ __global__ void __launch_bounds__(kWave)
 
 // The same for long runs, whose scan is a chain of tiles of 64 rows (0.85 us each): kMaxWaves waves take a stretch of the run each, put its steps
 // together first (m -> max(m + a, b), as the scan's), and scan it from the maximum that enters it.  2,048 rows of 32 heads: 27 us with one
-// wave, 9 us so.
+// wave, 9 us so.  Not for many runs (32 of 256 rows and 64 heads: 20 us with one wave, 26 so), and not in front of a walk of several: its workgroups of one
+// wave come to lie otherwise after it (32 heads of 128 x 128, 1,024 rows beside 7 single tokens, the walk after one wave 279 us, after this 322).
 constexpr int kMaxWaves = 8;
 __global__ void __launch_bounds__(kMaxWaves* kWave)
     mlstm_max_stretches_kernel(float4* __restrict__ coef, float* __restrict__ m_state, const int* __restrict__ run_start,
@@ -337,12 +338,12 @@ __global__ void __launch_bounds__(256)
 
 void mlstm_factors(const float* ig, int ldi, const float* fg, int ldf, const float* i_bias, const float* f_bias, float cap, float4* coef,
                    float* m_state, const int* run_start, const int* seq_start, const int* state_slots, int S, int heads, int T, int max_run,
-                   int one_order, hipStream_t s) {
+                   int one_order, bool stretches, hipStream_t s) {
   const int logs_first = max_run >= 16 ? 1 : 0;      // long runs: the gates' logarithms of all T rows first, in parallel
   if (logs_first) {
     const long long n = static_cast<long long>(T) * heads;
     mlstm_gate_logs_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(ig, ldi, fg, ldf, i_bias, f_bias, cap, coef, n, heads);
-    if (!one_order && max_run > 2 * kWave) {
+    if (stretches && !one_order && max_run > 2 * kWave) {
       mlstm_max_stretches_kernel<<<S * heads, kMaxWaves * kWave, 0, s>>>(coef, m_state, run_start, seq_start, state_slots, heads);
       return;
     }
@@ -377,7 +378,7 @@ int kvcm_mlstm_scan(const float* q, int ldq, const float* k, int ldk, const floa
   KVCM_REQUIRE(coef && n_new && reinterpret_cast<uintptr_t>(coef) % 16 == 0, "mlstm_scan: the scratch must be there, 16-byte aligned");
   float4* cf = reinterpret_cast<float4*>(coef);
   KVCM_REQUIRE(max_run < 16 || T > 0, "mlstm_scan: the row count is needed for runs of %d", max_run);
-  mlstm_factors(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, S, heads, T, max_run, one_order, s);
+  mlstm_factors(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, S, heads, T, max_run, one_order, S == 1, s);
 #define KVCM_MLSTM_AS(DKP, G, NC, U, NT, HOW)                                                                                    \
   {                                                                                                                          \
     const int col_blocks = (dv + NT / G * NC - 1) / (NT / G * NC);                                                                     \

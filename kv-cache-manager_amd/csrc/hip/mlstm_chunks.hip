@@ -494,7 +494,7 @@ int kvcm_mlstm_chunks(const float* q, int ldq, const float* k, int ldk, const fl
                  (dv + kChunkCols - 1) / kChunkCols, carry, piece, (max_run + piece - 1) / piece};
   KVCM_REQUIRE(static_cast<long long>(S) * A.pieces_per_seq <= 65535 && heads <= 65535 && static_cast<long long>(heads) * A.col_blocks < (1ll << 31),
                "mlstm_chunks: too many sequences and pieces for one launch");
-  mlstm_factors(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, S, heads, T, max_run, 0, s);
+  mlstm_factors(ig, ldi, fg, ldf, i_bias, f_bias, cap, cf, m_state, run_start, seq_start, state_slots, S, heads, T, max_run, 0, static_cast<long long>(S) * heads <= 512, s);
   auto aligned = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
   const bool wide = dk % 4 == 0 && dv % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 && aligned(q) && aligned(k) && aligned(v);
   if (dk <= 64) launch_chunks<64>(A, S, wide, s);

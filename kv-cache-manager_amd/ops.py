@@ -2047,9 +2047,24 @@ MLSTM_PIECE = 128            # rows of a piece of ``mlstm_scan``'s matrix form
 MLSTM_MIN_RUN = 256          # rows of a step's longest run from which that form is worth it (us, 32 heads of 64 x 64, walk / so: 192 rows 38.0 / 40.2, 256 rows 44.9 / 42.3)
 
 
-def mlstm_in_chunks(step, dk, one_order=False):
-    """Does ``mlstm_scan``, given scratch for the pieces, take this step's runs in matrix form (csrc/hip/mlstm_chunks.hip)?"""
-    return not one_order and dk <= 128 and step.max_run >= MLSTM_MIN_RUN and step.seqs * -(-int(step.max_run) // MLSTM_PIECE) <= 65535
+def mlstm_in_chunks(step, dk, one_order=False, heads=1, dv=None):
+    """Does ``mlstm_scan``, given scratch for the pieces, take this step's runs in matrix form (csrc/hip/mlstm_chunks.hip)?  Where the walk's time
+    is the larger, us: the walk's is its longest run's chain (0.15 a token, from 65 keys on 0.2, from 33 on 0.28 once its waves have no
+    SIMD each) or the step's work, the matrix form's its chunks of 64 rows, of which a single token takes a whole one.  Measured, walk / so:
+    32 heads of 64 x 64, one of 256 rows 54 / 49 (so), beside 31 single tokens 94 / 103 (walk), 63 100 / 167 (walk), one of 512 beside 31
+    167 / 110 (so), 32 of 256 335 / 284 (so); 32 heads of 128 x 128, one of 256 90 / 66 (so), beside 7 96 / 110 (walk), 31 143 / 286 (walk), one of
+    1,024 beside 31 318 / 358 (walk), 4 of 256 203 / 124 (so); 64 heads of 16 x 16, 4 of 256 56 / 66 (walk), 32 of 256 107 / 341 (walk), one of
+    1,024 beside 31 172 / 135 (so)."""
+    if one_order or dk > 128 or step.max_run < MLSTM_MIN_RUN or step.seqs * -(-int(step.max_run) // MLSTM_PIECE) > 65535:
+        return False
+    dv, seqs, longest = dv or dk, step.seqs, int(step.max_run)
+    chunks = min(step.rows / 64 + seqs, seqs * -(-longest // 64))
+    if dk <= 64:
+        chain = longest * (0.15 if dk <= 32 or seqs * heads * -(-dv // 8) < 1024 else 0.28)
+    else:
+        chain = longest * (0.2 if -(-step.rows // longest) * heads * -(-dv // 4) <= 1024 else 0.28)
+    work = step.rows * heads * dv / 64 * (0.0002 if dk <= 16 else 0.0005 if dk <= 32 else 0.0013 if dk <= 64 else 0.0028)
+    return 40 + chunks * heads * -(-dv // 64) * (0.03 if dk <= 32 else 0.052 if dk <= 64 else 0.095) < 18 + max(chain, work)
 
 
 def mlstm_carry_floats(rows, seqs, heads, dk, dv):
@@ -2075,7 +2090,7 @@ def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, co
     _f32(n_new, "n_new", step.seqs * heads * dk)
     for t, n, shape in ((s_state, "s_state", (heads, dk, dv)), (n_state, "n_state", (heads, dk)), (m_state, "m_state", (heads,))):
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.is_cuda and tuple(t.shape[1:]) == shape, f"{n} must be float32 [slots, {shape}]")
-    if carry is not None and mlstm_in_chunks(step, dk, one_order):
+    if carry is not None and mlstm_in_chunks(step, dk, one_order, heads, dv):
         _f32(carry, "carry")
         _call("kvcm_mlstm_chunks", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_in), gate_in.stride(0),
               _ptr(gate_keep), gate_keep.stride(0), _ptr(in_bias), _ptr(keep_bias), float(cap), float(q_scale), _ptr(coef), _ptr(o),

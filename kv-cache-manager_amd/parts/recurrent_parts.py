@@ -181,7 +181,7 @@ class MatrixMemoryMixer(_StatefulMixer):
     def carry(self, step, one_order):
         """Scratch for steps whose long runs go in matrix form, sized for the engine's largest step."""
         ops, p, lim = self.ctx.ops, self.params, step.limits
-        if not ops.mlstm_in_chunks(step, p["dim"], one_order):
+        if not ops.mlstm_in_chunks(step, p["dim"], one_order, p["heads"], p["vdim"]):
             return None
         rows, seqs = max(step.rows, lim.max_tokens if lim else 0), max(step.seqs, lim.max_seqs if lim else 0)
         return step.flat("memory_carry", ops.mlstm_carry_floats(rows, seqs, p["heads"], p["dim"], p["vdim"]))

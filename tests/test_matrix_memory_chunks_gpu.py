@@ -148,3 +148,33 @@ def test_errors_of_long_runs_are_the_walks(d):
     assert walk[0] < 3e-5 and max(walk[1:]) < 3e-6, errors      # (the outputs' divisor n . q cancels)
     # a state's error is that of the factors, which the forms share; what each adds is a few parts in a hundred of it
     assert all(x <= 1.03 * y for x, y in zip(chunks, walk)), errors
+
+
+def test_the_line_where_the_walk_is_the_faster():
+    """Single tokens beside a run, heads of few keys, many runs: the form whose measured time is the smaller (us, walk / matrix form)."""
+    from kvcm_amd import ops
+
+    def takes(heads, dk, dv, runs):
+        st = Step([(i, 5, n) for i, n in enumerate(runs)])
+        st.max_run = max(runs)
+        return ops.mlstm_in_chunks(st, dk, False, heads, dv)
+
+    one = [1]
+    for heads, dk, dv, runs, so in ((32, 64, 64, [256], True),                    # 54 / 49
+                                    (32, 64, 64, [256] + 7 * one, True),          # 90 / 63
+                                    (32, 64, 64, [256] + 31 * one, False),        # 94 / 103
+                                    (32, 64, 64, [256] + 63 * one, False),        # 100 / 167
+                                    (32, 64, 64, [1024] + 31 * one, True),        # 311 / 125
+                                    (32, 64, 64, [256] * 32, True),               # 335 / 284
+                                    (32, 128, 128, [256], True),                  # 90 / 66
+                                    (32, 128, 128, [256] + 7 * one, False),       # 96 / 110
+                                    (32, 128, 128, [1024] + 31 * one, False),     # 318 / 358
+                                    (32, 128, 64, [256] + 7 * one, False),        # 73 / 80
+                                    (32, 128, 128, [256] * 4, True),              # 203 / 124
+                                    (64, 16, 16, [256], True),                    # 54 / 44
+                                    (64, 16, 16, [256] * 4, False),               # 57 / 66
+                                    (64, 16, 16, [256] * 32, False),              # 107 / 341
+                                    (64, 16, 16, [1024] + 31 * one, True),        # 172 / 135
+                                    (8, 64, 64, [256] + 63 * one, True),          # 89 / 77
+                                    (32, 32, 32, [256] * 16, False)):             # 88 / 114
+        assert takes(heads, dk, dv, runs) == so, (heads, dk, dv, len(runs), max(runs))
