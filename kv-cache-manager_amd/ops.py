@@ -2044,6 +2044,7 @@ def act_rows(x, out, activation):
 
 
 MLSTM_PIECE = 128            # rows of a piece of ``mlstm_scan``'s matrix form
+MLSTM_CARRY = 9 << 22        # 32-bit values of scratch that it asks for at most, where the states themselves don't take half as much (68 pieces of 32 heads of 128 x 128)
 MLSTM_MIN_RUN = 256          # rows of a step's longest run from which that form is worth it (us, 32 heads of 64 x 64, walk / so: 192 rows 38.0 / 40.2, 256 rows 44.9 / 42.3)
 
 
@@ -2068,8 +2069,21 @@ def mlstm_in_chunks(step, dk, one_order=False, heads=1, dv=None):
 
 
 def mlstm_carry_floats(rows, seqs, heads, dk, dv):
-    """32-bit values of scratch that ``mlstm_scan`` needs to take a step of this shape in matrix form."""
-    return int(lib().kvcm_mlstm_carry_floats(rows, seqs, heads, dk, dv, MLSTM_PIECE))
+    """32-bit values of scratch that ``mlstm_scan`` takes for steps of up to this shape in matrix form: in longer pieces, where those of MLSTM_PIECE rows would
+    take more than MLSTM_CARRY and more than twice what the sequences' own states do (each has a piece at least)."""
+    size, piece = (lambda r: int(lib().kvcm_mlstm_carry_floats(rows, seqs, heads, dk, dv, r))), MLSTM_PIECE
+    most = max(MLSTM_CARRY, int(lib().kvcm_mlstm_carry_floats(0, 2 * seqs, heads, dk, dv, piece)))
+    while size(piece) > most and piece < rows:
+        piece *= 2
+    return size(piece)
+
+
+def mlstm_piece(rows, seqs, heads, dk, dv, floats):
+    """Rows of a piece: MLSTM_PIECE, or as many times two as `floats` values of scratch ask for."""
+    piece = MLSTM_PIECE
+    while piece < rows and int(lib().kvcm_mlstm_carry_floats(rows, seqs, heads, dk, dv, piece)) > floats:
+        piece *= 2
+    return piece
 
 
 def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, coef, n_new, o, s_state, n_state, m_state, step, heads, dk, dv, one_order=False,
@@ -2095,7 +2109,8 @@ def mlstm_scan(q, k, v, gate_in, gate_keep, in_bias, keep_bias, cap, q_scale, co
         _call("kvcm_mlstm_chunks", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_in), gate_in.stride(0),
               _ptr(gate_keep), gate_keep.stride(0), _ptr(in_bias), _ptr(keep_bias), float(cap), float(q_scale), _ptr(coef), _ptr(o),
               o.stride(0), _ptr(s_state), _ptr(n_state), _ptr(m_state), _ptr(step.run_start), _ptr(step.seq_start),
-              _ptr(step.state_slots), step.seqs, heads, dk, dv, T, int(step.max_run), MLSTM_PIECE, _ptr(carry), carry.numel(), _stream())
+              _ptr(step.state_slots), step.seqs, heads, dk, dv, T, int(step.max_run), mlstm_piece(T, step.seqs, heads, dk, dv, carry.numel()), _ptr(carry),
+              carry.numel(), _stream())
         return o
     _call("kvcm_mlstm_scan", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_in), gate_in.stride(0),
           _ptr(gate_keep), gate_keep.stride(0), _ptr(in_bias), _ptr(keep_bias), float(cap), float(q_scale), _ptr(coef), _ptr(n_new), _ptr(o),

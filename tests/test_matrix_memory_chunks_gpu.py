@@ -178,3 +178,34 @@ def test_the_line_where_the_walk_is_the_faster():
                                     (8, 64, 64, [256] + 63 * one, True),          # 89 / 77
                                     (32, 32, 32, [256] * 16, False)):             # 88 / 114
         assert takes(heads, dk, dv, runs) == so, (heads, dk, dv, len(runs), max(runs))
+
+
+def test_scratch_is_bounded_and_longer_pieces_do():
+    from kvcm_amd import ops
+    size = lambda rows, seqs, heads, d, piece: int(ops.lib().kvcm_mlstm_carry_floats(rows, seqs, heads, d, d, piece))
+    for rows, seqs, heads, d in ((2048, 1, 32, 64), (65536, 1, 32, 128), (65536, 256, 32, 128), (1 << 20, 4, 32, 64), (8192, 64, 64, 128)):
+        floats = ops.mlstm_carry_floats(rows, seqs, heads, d, d)
+        assert floats <= max(ops.MLSTM_CARRY, 2 * (seqs + 1) * heads * (d * d + d + 1))
+        assert ops.mlstm_piece(rows, seqs, heads, d, d, floats) >= ops.MLSTM_PIECE and size(rows, seqs, heads, d, ops.mlstm_piece(rows, seqs, heads, d, d, floats)) <= floats
+        assert floats == size(rows, seqs, heads, d, ops.MLSTM_PIECE) or floats < size(rows, seqs, heads, d, ops.MLSTM_PIECE)
+    heads, d, runs = 3, 64, (1100, 300, 513)
+    T = sum(runs)
+    st = Step([(i, 5, n) for i, n in enumerate(runs)])
+    st.max_run = max(runs)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.rand(T, heads * d, generator=g, device=DEV) for _ in range(3))      # (a divisor without cancellation)
+    gates, first, out = torch.randn(2, T, heads, generator=g, device=DEV), [torch.rand(3, heads, *c, generator=g, device=DEV) for c in ((d, d), (d,), ())], []
+    for piece in (128, 256, 512, 2048):
+        floats, o, states = size(T, 3, heads, d, piece), torch.full((T, heads * d), float("nan"), device=DEV), [x.clone() for x in first]
+        assert ops.mlstm_piece(T, 3, heads, d, d, floats) == piece
+        ops.mlstm_scan(q, k, v, gates[0], gates[1], torch.zeros(heads, device=DEV), torch.full((heads,), 4.0, device=DEV), 15.0, d ** -0.5,
+                       torch.empty(T, 4 * heads, device=DEV), torch.empty(3 * heads * d, device=DEV), o, *states, st, heads, d, d,
+                       carry=torch.full((floats,), float("nan"), device=DEV))
+        out.append((o, *states))
+    for got in out[1:]:
+        for x, y in zip(got, out[0]):
+            assert float((x - y).abs().max()) < 6e-5 * float(y.abs().max())      # both within 3e-5 of the recurrence, as above
+    with pytest.raises(RuntimeError):
+        ops.mlstm_scan(q, k, v, gates[0], gates[1], torch.zeros(heads, device=DEV), torch.full((heads,), 4.0, device=DEV), 15.0, d ** -0.5,
+                       torch.empty(T, 4 * heads, device=DEV), torch.empty(3 * heads * d, device=DEV), o, *states, st, heads, d, d,
+                       carry=torch.empty(3 * heads * d * d, device=DEV))
