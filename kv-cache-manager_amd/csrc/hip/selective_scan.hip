@@ -222,13 +222,13 @@ __global__ void __launch_bounds__(kWave)
 }
 
 // The first pass makes the step sizes as it walks and leaves them in place for the second, which makes the gates (a launch of
-// their own read and wrote both, 134 MB of 32-bit rows and 37 us at 2,048 x 4,096).
+// their own read and wrote both, 134 MB of 32-bit rows and 37 us at 2,048 x 4,096), unless they are prepared already.
 template <class T, int N, bool OUT>
 __global__ void __launch_bounds__(256)
     scan_channels_kernel(const T* __restrict__ x, int ldx, float* __restrict__ dt, int lddt, const float* __restrict__ dt_bias,
                          const float* __restrict__ bc, int ldbc, int off_b, int off_c, const float* __restrict__ a_log,
                          const float* __restrict__ dskip, const float* __restrict__ z, int ldz, T* __restrict__ out, int ldo,
-                         const int* __restrict__ run_start, const int* __restrict__ state_slots, int C, int chunk_len,
+                         const int* __restrict__ run_start, const int* __restrict__ state_slots, int C, int prepared, int chunk_len,
                          float* __restrict__ carry, float* __restrict__ dsum) {
   constexpr int U = 4, W = OUT ? 2 * N : N;
   constexpr bool kOneOrder = std::is_same<T, float>::value;      // (32-bit results do not depend on how the states are dealt out)
@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(256)
       const int r = first + u;
       if (r >= r1) break;
       float step = dtv[from][u];
-      if (!OUT) {
+      if (!OUT && !prepared) {
         step = softplus(step + db);
         if (owns) dt[size_t(r) * lddt + c] = step;
       }
@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(256)
       if (OUT && kOneOrder) y = states_sum(ys);
       if (OUT && owns) {
         const float zz = zv[from][u];
-        store_f(out + size_t(r) * ldo + c, fmaf(skip, xv[from][u], y) * (zz / (1.0f + expf(-zz))));
+        store_f(out + size_t(r) * ldo + c, fmaf(skip, xv[from][u], y) * (prepared ? zz : zz / (1.0f + expf(-zz))));
       }
     }
   };
@@ -368,8 +368,8 @@ __global__ void __launch_bounds__(256)
 // lane a channel, 16 states (before the step size's formula above): 256 rows of 1,024 channels 32 / 40, of 2,048 38 / 41, of 4,096 60 / 42; 512 of 1,024 42 / 43, of 2,048 64 / 44;
 // 1,024 of 4,096 183 / 71.  32-bit exponentials take longer, and a wave all of them (pieces of 128): 1 x 2,048 of 1,024 110 / 198, of 2,048
 // 182 / 207, of 4,096 330 / 227, 8 x 512 of 1,024 173 / 203, of 2,048 311 / 220.
-bool scan_by_channels(bool f32, int T, int C, int N) {
-  return (N == 8 || N == 16) && static_cast<long long>(T) * C >= (f32 ? 640ll * kWave * 128 : 1ll << 19);
+bool scan_by_channels(bool f32, int T, int C, int N, int chunk_len) {      // (from about one wave, 64 channels of a piece, a CU on)
+  return (N == 8 || N == 16) && static_cast<long long>(T) * C >= (f32 ? 640ll : 256ll) * kWave * chunk_len;
 }
 
 int prepare_scan(float* dt, int lddt, const float* dt_bias, float* z, int ldz, int T, int C, hipStream_t s) {
@@ -398,12 +398,12 @@ int launch_scan(const void* x, int ldx, float* dt_lin, int lddt, const float* dt
 #undef KVCM_SCAN_SINGLE
     return launch_status("selective_scan");
   }
-  if (phase != 0 && !prepared && scan_by_channels(std::is_same<X, float>::value, T, C, N)) {
+  if (phase != 0 && scan_by_channels(std::is_same<X, float>::value, T, C, N, chunk_len)) {
     const dim3 grid((C + 255) / 256, S, pieces);
 #define KVCM_SCAN_CHANNELS(N, OUT)                                                                                            \
   scan_channels_kernel<X, N, OUT><<<grid, 256, 0, s>>>(static_cast<const X*>(x), ldx, dt_lin, lddt, dt_bias, bc, ldbc, off_b,   \
                                                        off_c, a_log, dskip, z, ldz, static_cast<X*>(out), ldo, run_start,       \
-                                                       state_slots, C, chunk_len, carry, dsum)
+                                                       state_slots, C, prepared, chunk_len, carry, dsum)
     if (N == 8 && phase == 1) KVCM_SCAN_CHANNELS(8, false);
     else if (N == 8) KVCM_SCAN_CHANNELS(8, true);
     else if (phase == 1) KVCM_SCAN_CHANNELS(16, false);
@@ -464,7 +464,7 @@ extern "C" int kvcm_selective_scan(const void* x, int dtype, int ldx, float* dt_
   KVCM_REQUIRE(pieces >= 1 && pieces <= 65535 && carry != nullptr && carry_floats >= slots * C * (N + 1),
                "selective_scan: the scratch for %lld pieces is too small", slots);
   float* dsum = carry + slots * C * N;
-  if (!prepared && !scan_by_channels(dtype == kF32, T, C, N)) {
+  if (!prepared && !scan_by_channels(dtype == kF32, T, C, N, chunk_len)) {
     if (int rc = prepare_scan(dt_lin, lddt, dt_bias, z, ldz, T, C, s)) return rc;
     prepared = 1;
   }
