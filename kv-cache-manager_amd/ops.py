@@ -1703,8 +1703,11 @@ def scan_in_pieces(step, C, N, dtype):
     return step.max_run >= 4 * SCAN_PIECE
 
 
-def selective_scan_carry_floats(rows, seqs, C, N):
-    """32-bit values of scratch that ``selective_scan(..., carry=...)`` needs for steps of up to this shape."""
+def selective_scan_carry_floats(rows, seqs, C, N, piece=None):
+    """32-bit values of scratch that ``selective_scan(..., carry=...)`` takes for steps of up to this shape, in the pieces that it chooses or in pieces of
+    ``piece`` rows (SCAN_PIECE do always: with less than its own pieces need, it takes those)."""
+    if piece is not None:
+        return (rows // piece + seqs + 1) * C * (N + 1)
     short = min(rows // 32, (1 << 19) // C)      # (shorter pieces are no more than that)
     return (max(rows // SCAN_PIECE, short) + seqs + 1) * C * (N + 1)
 
@@ -1713,8 +1716,8 @@ def selective_scan(x, dt_lin, dt_bias, bc, off_b, off_c, a_log, dskip, z, out, s
     """The selective scan of the step's runs (csrc/hip/selective_scan.hip).  x, out [T, C] in the compute dtype;
     dt_lin [T, C], bc rows with B at off_b and C at off_c, z rows: 32-bit; state [slots, C, N].  ``prepare``: the step
     sizes and gates of all rows are made first, in place in dt_lin and z, by a launch of their own (pays for long runs).
-    ``carry`` (float32 scratch of ``selective_scan_carry_floats``; needs ``prepare``): runs are walked in pieces of
-    ``scan_piece`` rows, all pieces at once: each from zero, then the states that enter the pieces (a short walk over the
+    ``carry`` (float32 scratch of ``selective_scan_carry_floats``; needs ``prepare``; dt_lin and z hold what they may of that then): runs are
+    walked in pieces of ``scan_piece`` rows, all pieces at once: each from zero, then the states that enter the pieces (a short walk over the
     pieces' ends), then each again from its entering state.  The sums are the token-by-token ones in another order."""
     C, N = a_log.shape
     _rows2d(x, "x")
@@ -1728,15 +1731,19 @@ def selective_scan(x, dt_lin, dt_bias, bc, off_b, off_c, a_log, dskip, z, out, s
     _f32(dskip, "dskip", C)
     _need(state.dtype == torch.float32 and state.is_contiguous() and state.is_cuda and tuple(state.shape[1:]) == (C, N),
           "state must be float32 [slots, C, N]")
+    piece = 0
     if carry is not None:
+        piece = scan_piece(out.shape[0], C, x.dtype)
+        if carry.numel() < selective_scan_carry_floats(out.shape[0], step.seqs, C, N, piece):
+            piece = SCAN_PIECE
         _need(prepare and carry.dtype == torch.float32 and carry.is_contiguous() and carry.is_cuda
-              and carry.numel() >= selective_scan_carry_floats(out.shape[0], step.seqs, C, N), "the scratch for the pieces is too small")
+              and carry.numel() >= selective_scan_carry_floats(out.shape[0], step.seqs, C, N, piece), "the scratch for the pieces is too small")
     if prepare and carry is None:
         _call("kvcm_scan_prepare", _ptr(dt_lin), dt_lin.stride(0), _ptr(dt_bias), _ptr(z), z.stride(0), out.shape[0], C, _stream())
     _call("kvcm_selective_scan", _ptr(x), _DT[x.dtype], x.stride(0), _ptr(dt_lin), dt_lin.stride(0), _ptr(dt_bias), _ptr(bc),
           bc.stride(0), off_b, off_c, _ptr(a_log), _ptr(dskip), _ptr(z), z.stride(0), _ptr(out), out.stride(0), _ptr(state),
           _ptr(step.run_start), _ptr(step.seq_start), _ptr(step.state_slots), step.seqs, C, N, 1 if prepare and carry is None else 0,
-          scan_piece(out.shape[0], C, x.dtype) if carry is not None else 0, step.max_run, _ptr(carry), carry.numel() if carry is not None else 0,
+          piece, step.max_run, _ptr(carry), carry.numel() if carry is not None else 0,
           out.shape[0], _stream())
     return out
 

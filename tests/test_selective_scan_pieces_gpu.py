@@ -72,6 +72,32 @@ def test_step_sizes_and_gates_that_are_made_already(monkeypatch):
         torch.testing.assert_close(a, b, rtol=0, atol=2.0 ** -8 * float(b.abs().max()))
 
 
+@pytest.mark.gpu
+def test_scratch_for_the_longest_pieces_is_enough():
+    """Scratch sized for pieces of SCAN_PIECE rows is taken where shorter ones would be the choice; less is refused."""
+    from kvcm_amd import ops
+    g = torch.Generator().manual_seed(4)
+    T, C, N = 700, 900, 16
+    x, z, dt = (torch.randn(T, C, generator=g).to(DEV) for _ in range(3))
+    bc, a_log, dsk, db = (torch.randn(*n, generator=g).to(DEV) for n in ((T, 2 * N), (C, N), (C,), (C,)))
+    step, got = Step([(0, 0, T)]), []
+    step.max_run = T
+    assert ops.scan_piece(T, C, torch.bfloat16) < ops.SCAN_PIECE
+    least = ops.selective_scan_carry_floats(T, 1, C, N, ops.SCAN_PIECE)
+    for floats in (ops.selective_scan_carry_floats(T, 1, C, N), least, least - 1):
+        out, state = torch.empty(T, C, dtype=torch.bfloat16, device=DEV), torch.zeros(1, C, N, device=DEV)
+        call = lambda: ops.selective_scan(x.bfloat16(), dt.clone(), db, bc, 0, N, a_log, dsk, z.clone(), out, state, step, prepare=True,
+                                          carry=torch.full((floats,), float("nan"), device=DEV))
+        if floats < least:
+            with pytest.raises(Exception, match="too small"):
+                call()
+        else:
+            call()
+            got.append((out.float(), state))
+    for a, b in zip(*got):      # (half a unit of 8 bits of the largest, each)
+        torch.testing.assert_close(a, b, rtol=0, atol=2.0 ** -8 * float(b.abs().max()))
+
+
 def test_the_scratch_holds_the_pieces_of_every_smaller_step():
     from kvcm_amd import ops
     for C, N, seqs, most in ((4096, 16, 3, 32768), (8192, 16, 1, 5000), (64, 8, 9, 40000), (1, 8, 1, 100), (600000, 8, 1, 700)):
