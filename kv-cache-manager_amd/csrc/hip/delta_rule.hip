@@ -21,27 +21,29 @@
 
 namespace kvcm {
 
-// A wave makes R rows of a head, a workgroup of four those of four heads.  The decay's logit is a two-step projection whose second step
-// runs here in 32-bit: w_lin[c] = sum_j w2[c, j] * tanh(low[j]), low = the first step's output (rank values a row), tanh once for the
-// workgroup's heads; w2 comes transposed, [rank, heads*d], sixteen of a channel's values on their way together: one at a time a
-// step of few rows was a chain of `rank` trips to L2.  us, a wave of its own for every row and head /
-// so, rank 64, 32 heads of 64: 8 rows 5.2 / 4.2, 2,048 rows 66 / 44; of 128 7.4 / 5.6 and 115 / 77 (its bits are the same either way).
-constexpr int kDeltaMaxRank = 256, kDeltaRows = 8;
+// A wave makes R rows of a head, a workgroup those of up to four heads (as many as leave no or one wave idle: of five, three and two).  The decay's logit
+// is a two-step projection whose second step runs here in 32-bit: w_lin[c] = sum_j w2[c, j] * tanh(low[j]), low = the first step's output (rank values
+// a row), tanh once for the workgroup's heads; w2 comes transposed, [rank, heads*d], sixteen of a channel's values on their way together: one at a time a
+// step of few rows was a chain of `rank` trips to L2.  us, a wave of its own for every row and head, its values one at a time /
+// so (the bits are the same either way), heads, size, rank, rows: 32, 64, 64, 8 rows 4.8 / 3.8, 2,048 rows 66 / 42; 32, 128, 64 7.0 / 5.2 and 112 / 73; 32, 64, 8
+// 3.3 / 3.2 and 34 / 30; 5, 64, 64, 2,048 rows 13.0 / 10.4; 1, 64, 64, 2,048 rows 5.3 / 4.9.  Up to 0.8 us slower at a few thousand rows and heads with short ranks (9, 48, 20, 512
+// rows 5.2 / 6.0; 3, 64, 15, 2,048 rows 6.0 / 6.9).
+constexpr int kDeltaMaxRank = 256;
 template <int R>
 __global__ void __launch_bounds__(256)
     delta_prepare_kernel(const float* __restrict__ k, int ldk, const float* __restrict__ a_lin, int lda,
                          const float* __restrict__ a_bias, const float* __restrict__ low, int ldlow,
                          const float* __restrict__ w2t, int rank, const float* __restrict__ w0,
-                         float* __restrict__ w_out, float* __restrict__ au_out, float* __restrict__ u_out, int heads, int d, int T) {
-  constexpr int kWaves = 256 / kWave, kAhead = 16;
+                         float* __restrict__ w_out, float* __restrict__ au_out, float* __restrict__ u_out, int heads, int d, int T,
+                         unsigned row_blocks) {
   __shared__ __attribute__((aligned(16))) float th[kDeltaMaxRank][R];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int row0 = blockIdx.x * R, head = blockIdx.y * kWaves + wave;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, waves = blockDim.x / kWave;
+  const int row0 = static_cast<int>(blockIdx.x % row_blocks) * R, head = static_cast<int>(blockIdx.x / row_blocks) * waves + wave;
   auto row_of = [&](int n) { return size_t(row0 + n < T ? row0 + n : T - 1); };      // (rows beyond the last are left out of the stores)
   if constexpr (R == 1) {
-    for (int j = threadIdx.x; j < rank; j += 256) th[j][0] = tanhf(low[row_of(0) * ldlow + j]);
+    for (int j = threadIdx.x; j < rank; j += blockDim.x) th[j][0] = tanhf(low[row_of(0) * ldlow + j]);
   } else {
-    for (int n = wave; n < R; n += kWaves)
+    for (int n = wave; n < R; n += waves)
       for (int j = lane; j < rank; j += kWave) th[j][n] = tanhf(low[row_of(n) * ldlow + j]);
   }
   __syncthreads();
@@ -65,18 +67,23 @@ __global__ void __launch_bounds__(256)
       ax[n] = a_lin[row_of(n) * lda + col + i];
     }
     int j = 0;
-    for (; j + kAhead <= rank; j += kAhead) {
-      float x[kAhead];
+    auto add = [&](auto ahead, int values) __attribute__((always_inline)) {      // `values` of a channel's from j on, all on their way together
+      constexpr int N = decltype(ahead)::value;
+      float x[N];
 #pragma unroll
-      for (int m = 0; m < kAhead; ++m) x[m] = w2[size_t(j + m) * D];
+      for (int m = 0; m < N; ++m) x[m] = w2[size_t(j + (m < values ? m : values - 1)) * D];
 #pragma unroll
-      for (int m = 0; m < kAhead; ++m)
+      for (int m = 0; m < N; ++m)
+        if (m < values) {
 #pragma unroll
-        for (int n = 0; n < R; ++n) wl[n] = fmaf(x[m], th[j + m][n], wl[n]);
-    }
-    for (; j < rank; ++j)
-#pragma unroll
-      for (int n = 0; n < R; ++n) wl[n] = fmaf(w2[size_t(j) * D], th[j][n], wl[n]);
+          for (int n = 0; n < R; ++n) wl[n] = fmaf(x[m], th[j + m][n], wl[n]);
+        }
+      j += values;
+    };
+    while (j + 16 <= rank) add(std::integral_constant<int, 16>{}, 16);
+    if (j + 8 <= rank) add(std::integral_constant<int, 8>{}, 8);
+    if (j + 4 <= rank) add(std::integral_constant<int, 4>{}, 4);
+    if (j < rank) add(std::integral_constant<int, 3>{}, rank - j);
     const float ab = a_bias[col + i], wb = w0[col + i];
 #pragma unroll
     for (int n = 0; n < R; ++n) {
@@ -245,14 +252,17 @@ int kvcm_delta_prepare(const float* k, int ldk, const float* a_lin, int lda, con
   KVCM_REQUIRE(T > 0 && heads > 0 && d > 0, "delta_prepare: bad sizes T=%d heads=%d d=%d", T, heads, d);
   KVCM_REQUIRE(rank > 0 && rank <= kDeltaMaxRank, "delta_prepare: a rank of %d is not supported (1 to %d)", rank, kDeltaMaxRank);
   KVCM_REQUIRE(ldk >= heads * d && lda >= heads * d && ldlow >= rank, "delta_prepare: row strides too small");
-  const unsigned groups = (heads + 3) / 4;
-  KVCM_REQUIRE(groups <= 65535, "delta_prepare: too many heads");
-  // (a row a wave while eight would leave CUs without work, and where w2 is read soon anyway)
-  if (static_cast<long long>(T) * groups < 256 * kDeltaRows || rank < 16)
-    delta_prepare_kernel<1><<<dim3(T, groups), 256, 0, s>>>(k, ldk, a_lin, lda, a_bias, low, ldlow, w2t, rank, w0, w_out, au_out, u_out, heads, d, T);
-  else
-    delta_prepare_kernel<kDeltaRows><<<dim3((T + kDeltaRows - 1) / kDeltaRows, groups), 256, 0, s>>>(
-        k, ldk, a_lin, lda, a_bias, low, ldlow, w2t, rank, w0, w_out, au_out, u_out, heads, d, T);
+  const int groups = (heads + 3) / 4, threads = (heads + groups - 1) / groups * kWave;
+  // Rows of a wave: as many as leave eight waves a CU, or six of four rows (us, one row / four / eight: 5 heads of 64, rank 64, 2,048 rows 15.7 / 10.4 / 13.9, 2 heads 6.5 / 8.4 / 12.2,
+  // 32 heads of rank 8 55 / - / 30).
+  const long long items = static_cast<long long>(T) * heads;
+  const int rows = items >= 8 * 2048 ? 8 : items >= 4 * 1536 ? 4 : 1;
+  const unsigned row_blocks = static_cast<unsigned>((static_cast<long long>(T) + rows - 1) / rows);
+  const long long blocks = static_cast<long long>(row_blocks) * groups;
+  KVCM_REQUIRE(blocks < (1ll << 31), "delta_prepare: too many rows");
+  auto* kernel = rows == 8 ? delta_prepare_kernel<8> : rows == 4 ? delta_prepare_kernel<4> : delta_prepare_kernel<1>;
+  kernel<<<static_cast<unsigned>(blocks), threads, 0, s>>>(k, ldk, a_lin, lda, a_bias, low, ldlow, w2t, rank, w0, w_out, au_out, u_out, heads, d, T,
+                                                           row_blocks);
   return launch_status("delta_prepare");
 }
 
