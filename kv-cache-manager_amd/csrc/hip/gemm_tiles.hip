@@ -475,8 +475,8 @@ int kvcm_gemm_tiles(const void* X, const void* W, float* partials, void* out, in
 }
 
 // What the library takes for M x wrows x K, us: the fastest of three sizes of tile, each with a constant, a step's chain for every round of 256
-// workgroups and a step's share of the chip, or tiles of 128 x 128 with K cut into up to 16 slices until they are 256; and the results' storing.
-static float library_time(int M, int wrows, int K) {
+// workgroups and a step's share of the chip, or tiles of 128 x 128 with K cut into up to 16 slices until they are 256; and the results' storing, by their bytes.
+static float library_time(int M, int wrows, int K, bool out_f32) {
   struct LibraryTile {
     int size;
     float fixed, chain, share;
@@ -491,7 +491,7 @@ static float library_time(int M, int wrows, int K) {
     if (l.size == 128) part = tiles;
   }
   const float slices = std::fmin(std::fmax(std::floor(1.f / part), 1.f), 16.f), cut = 8.22f + steps * (0.585f / slices + 1.028f * part);
-  return std::fmin(best, cut) + static_cast<float>(M) * static_cast<float>(wrows) * 0.595e-6f;
+  return std::fmin(best, cut) + static_cast<float>(M) * static_cast<float>(wrows) * (out_f32 ? 1.19e-6f : 0.595e-6f);
 }
 
 // Is a product of many rows, in S slices of K that its consumer adds, faster here than by the vendor library (is_gated: than that and
@@ -506,6 +506,8 @@ static float library_time(int M, int wrows, int K) {
 // What the rule picks is 2.1 and 5 % slower than the better of the two, gated (1,197 shapes, 96 to 33,000 rows) 1.2 and 0.6 %.  Against the line and the tiles from before there were
 // tiles of four waves: 0.96 and 0.93 of the time, gated 0.90 and 0.80, slower by more than 5 % at 53 and 9, gated 19 and 8; with the line that came with those tiles it was 209 and 71,
 // gated 64 and 33.  At 1,420 plain shapes that the fit had not seen 0.965 and 0.95, slower by more than 5 % at 83 of 1,220 and 19 of 200; 571 gated 0.92 and 0.85, at 37 and 14.
+// 32-bit results, 900 shapes that the fit had not seen: 1.7 % slower than the better of the two, by more than 5 % at 94; with their storing priced as two bytes 3.3 %, at 159
+// (2048 x 8256 x 2048 75.7 here, 90.6; 2048 x 8192 x 2048 59.3, 63.3).
 // (us, here / library: taken 2048 x 2560 x 2048 25.8 / 29.0, 1040 x 2048 x 2048 17.2 / 23.0, 1024 x 1024 x 512 5.9 / 9.0, 2048 x 2048 x 5632 52.2 / 52.7; 2,048 and 1,024 rows of gate and up,
 // 5632 x 2048, 90 / 92 and 49 / 57; not taken 640 x 64 x 14336 30 / 17, 1040 x 8192 x 2048 44 / 36, 2048 x 8192 x 2048 52 / 50, 384 x 2048 x 5632 whole 27 / 25, 2048 x 256 x 5632 21.7 / 20.6.)
 int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_dtype) {
@@ -513,11 +515,12 @@ int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_
   if (M > 2048 && !is_gated) return 0;
   const float results = static_cast<float>(M) * static_cast<float>(N);
   const int wrows = is_gated ? 2 * N : N;
+  const bool out_f32 = out_dtype == kF32;
   float here = 0.f;
   best_tile(M, wrows, K, S, &here);
-  here += stored_time(M, N, S, out_dtype == kF32) +
+  here += stored_time(M, N, S, out_f32) +
           (S > 1 ? results * (4.f * S - 2.f) / 4.5e6f + static_cast<float>(N) * 4.f * S / 55e3f : 0.f);
-  const float library = library_time(M, wrows, K);
+  const float library = library_time(M, wrows, K, out_f32);
   if (is_gated) return here <= library + 3.4f + results * 6.f / 5e6f;
   const long long tiles = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128);
   const float side = M <= 256 && tiles > 16 ? 1.1f : M > 512 && M <= 1024 && tiles < 116 ? 0.78f : N <= 320 && K >= 5632 ? 0.84f : 0.98f;

@@ -26,6 +26,15 @@ def test_products_of_many_rows_here_or_by_the_library(ops, M, N, K, gated, here)
     assert ops.lib().kvcm_gemm_tiles_preferred(M, N, K, 1, gated, ops._DT[ops.torch.bfloat16]) == here
 
 
+# 32-bit results, whose storing costs the library more: us, here / library, launches one after the other
+@pytest.mark.parametrize("M,N,K,here", [(2048, 8192, 2048, 1),        # 59.3 / 63.3
+                                        (2048, 8256, 2048, 1),        # 75.7 / 90.6
+                                        (2048, 2560, 2048, 1),        # 27.0 / 28.3
+                                        (4072, 2560, 2048, 0)])
+def test_products_with_a_32_bit_result(ops, M, N, K, here):
+    assert ops.lib().kvcm_gemm_tiles_preferred(M, N, K, 1, 0, ops._DT[ops.torch.float32]) == here
+
+
 @pytest.mark.parametrize("M,N,K,S,gated,tile", [(512, 2816, 2048, 1, 1, (128, 96)), (128, 11264, 2048, 2, 0, (128, 96)), (117, 7680, 1600, 4, 0, (128, 128)),
                                                 (64, 2048, 2048, 8, 0, (64, 64)), (2048, 2048, 5632, 1, 0, (128, 128)), (32768, 5632, 2048, 1, 1, (256, 256))])
 def test_tiles_of_products(ops, M, N, K, S, gated, tile):
