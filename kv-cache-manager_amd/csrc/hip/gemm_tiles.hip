@@ -501,7 +501,8 @@ static float library_time(int M, int wrows, int K, bool out_f32) {
 // tile's modelled time, with the slices' reading (4.5 TB/s, and 55 KB a us of one row's through the CU that norms it), against the modelled library's, which was fitted to
 // half of 2,329 plain shapes (1,397 of widths as models have them, the others random; 64 to 32,000 columns, K 256 to 14,336, 96 to 2,048 rows).  It is off by 11 and 18 % a shape: which of
 // its kernels the library picks hangs on more than the sizes (256 x 128 x 5632 9.1 us, x 5120 17.5).  So the line lies a little on its side, and further where it is known to be better
-// than modelled and little is lost by it: 513 to 1,024 rows of fewer than 116 tiles of 128 x 128 (640 x 2048 x 2048 15.5, here 14.2; 768 rows 14.5, 14.4), and few columns of long K;
+// than modelled and little is lost by it: 513 to 1,024 rows of fewer than 116 tiles of 128 x 128 (768 x 2048 x 5632 31.9, here 33.2; at 583 such shapes the pick is 1.1 % slower than the better of the two,
+// 2.0 with a factor of 0.78, 513 x 2048 x 2048 12.8, here 10.8, and 1.9 with 0.98), and few columns of long K;
 // on the tiles' up to 256 rows of more than 16, where it is often far slower than modelled (256 x 5632 x 5632 54, here 37).
 // What the rule picks is 2.1 and 5 % slower than the better of the two, gated (1,197 shapes, 96 to 33,000 rows) 1.2 and 0.6 %.  Against the line and the tiles from before there were
 // tiles of four waves: 0.96 and 0.93 of the time, gated 0.90 and 0.80, slower by more than 5 % at 53 and 9, gated 19 and 8; with the line that came with those tiles it was 209 and 71,
@@ -523,7 +524,7 @@ int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_
   const float library = library_time(M, wrows, K, out_f32);
   if (is_gated) return here <= library + 3.4f + results * 6.f / 5e6f;
   const long long tiles = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128);
-  const float side = M <= 256 && tiles > 16 ? 1.1f : M > 512 && M <= 1024 && tiles < 116 ? 0.78f : N <= 320 && K >= 5632 ? 0.84f : 0.98f;
+  const float side = M <= 256 && tiles > 16 ? 1.1f : M > 512 && M <= 1024 && tiles < 116 ? 0.87f : N <= 320 && K >= 5632 ? 0.84f : 0.98f;
   return here <= side * library;
 }
 
