@@ -21,7 +21,7 @@
 
 namespace kvcm {
 
-// A wave makes R rows of a head, a workgroup those of up to four heads (as many as leave no or one wave idle: of five, three and two).  The decay's logit
+// A wave makes R rows of a head, a workgroup those of up to four heads (of five, three and two).  The decay's logit
 // is a two-step projection whose second step runs here in 32-bit: w_lin[c] = sum_j w2[c, j] * tanh(low[j]), low = the first step's output (rank values
 // a row), tanh once for the workgroup's heads; w2 comes transposed, [rank, heads*d], sixteen of a channel's values on their way together: one at a time a
 // step of few rows was a chain of `rank` trips to L2.  us, a wave of its own for every row and head, its values one at a time /

@@ -323,6 +323,8 @@ __global__ void __launch_bounds__(WM* WN* kWave)
 // 128 x 64 31.9).  From 96 rows on tile_pipe.h's are mostly the faster, but not everywhere: the ring's 128 x 64, 128 x 96 and 128 x 128 stay for short chains and for tiles that just
 // fill the chip (us, the best of tile_pipe.h / so: gate and up of 512 x 2816 x 2048 24.6 / 20.2, 128 x 11264 x 2048 in two slices 17.7 / 15.6, 256 x 8192 x 2048 19.2 / 17.1,
 // 117 x 7680 x 1600 in four 14.2 / 12.0), its 64 x 32 for few columns (48 x 8192 x 2048 10.3 in 32 x 64, 9.6).
+// 16 x 32's constant a round is larger than fitted (0.267): two rounds of it and one of 16 x 64, alike one after the other (9 x 4096 x 14336 in four 21.8 / 22.1; x 8192 14.6 / 13.9), are not
+// in a decode step (22.4 / 21.7).
 // (columns, after the sizes and waves: the stages, and whether the tile is tile_pipe.h's)
 struct Tile {
   int bm, bn;
@@ -330,7 +332,7 @@ struct Tile {
   TileTime time;
 };
 #define KVCM_TILES(T)                                         \
-  T(16, 32, 1, 2, 8, false, 2.786f, 0.121f, 0.654f, 0.267f)   \
+  T(16, 32, 1, 2, 8, false, 2.786f, 0.121f, 0.654f, 0.600f)   \
   T(16, 48, 1, 3, 8, false, 2.807f, 0.137f, 0.742f, 0.631f)   \
   T(16, 64, 1, 4, 8, false, 2.851f, 0.169f, 0.772f, 0.596f)   \
   T(32, 32, 2, 2, 8, false, 2.822f, 0.137f, 0.779f, 0.448f)   \
@@ -507,7 +509,7 @@ static float library_time(int M, int wrows, int K, bool out_f32) {
 // What the rule picks is 2.1 and 5 % slower than the better of the two, gated (1,197 shapes, 96 to 33,000 rows) 1.2 and 0.6 %.  Against the line and the tiles from before there were
 // tiles of four waves: 0.96 and 0.93 of the time, gated 0.90 and 0.80, slower by more than 5 % at 53 and 9, gated 19 and 8; with the line that came with those tiles it was 209 and 71,
 // gated 64 and 33.  At 1,420 plain shapes that the fit had not seen 0.965 and 0.95, slower by more than 5 % at 83 of 1,220 and 19 of 200; 571 gated 0.92 and 0.85, at 37 and 14.
-// 32-bit results, 900 shapes that the fit had not seen: 1.7 % slower than the better of the two, by more than 5 % at 94; with their storing priced as two bytes 3.3 %, at 159
+// 32-bit results, 900 shapes that the fit had not seen: 1.5 % slower than the better of the two, by more than 5 % at 87; with their storing priced as two bytes 3.3 %, at 159
 // (2048 x 8256 x 2048 75.7 here, 90.6; 2048 x 8192 x 2048 59.3, 63.3).
 // (us, here / library: taken 2048 x 2560 x 2048 25.8 / 29.0, 1040 x 2048 x 2048 17.2 / 23.0, 1024 x 1024 x 512 5.9 / 9.0, 2048 x 2048 x 5632 52.2 / 52.7; 2,048 and 1,024 rows of gate and up,
 // 5632 x 2048, 90 / 92 and 49 / 57; not taken 640 x 64 x 14336 30 / 17, 1040 x 8192 x 2048 44 / 36, 2048 x 8192 x 2048 52 / 50, 384 x 2048 x 5632 whole 27 / 25, 2048 x 256 x 5632 21.7 / 20.6.)
