@@ -503,13 +503,13 @@ static float library_time(int M, int wrows, int K, bool out_f32) {
 // tile's modelled time, with the slices' reading (4.5 TB/s, and 55 KB a us of one row's through the CU that norms it), against the modelled library's, which was fitted to
 // half of 2,329 plain shapes (1,397 of widths as models have them, the others random; 64 to 32,000 columns, K 256 to 14,336, 96 to 2,048 rows).  It is off by 11 and 18 % a shape: which of
 // its kernels the library picks hangs on more than the sizes (256 x 128 x 5632 9.1 us, x 5120 17.5).  So the line lies a little on its side, and further where it is known to be better
-// than modelled and little is lost by it: 513 to 1,024 rows of fewer than 116 tiles of 128 x 128 (768 x 2048 x 5632 31.9, here 33.2; at 583 such shapes the pick is 1.1 % slower than the better of the two,
-// 2.0 with a factor of 0.78, 513 x 2048 x 2048 12.8, here 10.8, and 1.9 with 0.98), and few columns of long K;
+// than modelled and little is lost by it: 513 to 1,024 rows of fewer than 116 tiles of 128 x 128 (768 x 2048 x 5632 31.9, here 33.2; 513 x 2048 x 2048 12.8, here 10.8: up to 640 rows a factor
+// of 0.87, with 0.78 what it picked was a tenth slower there; beyond, 0.78 leaves 700 x 2048 x 2048, 13.1, here 11.1, with the library), and few columns of long K;
 // on the tiles' up to 256 rows of more than 16, where it is often far slower than modelled (256 x 5632 x 5632 54, here 37).
 // What the rule picks is 2.1 and 5 % slower than the better of the two, gated (1,197 shapes, 96 to 33,000 rows) 1.2 and 0.6 %.  Against the line and the tiles from before there were
 // tiles of four waves: 0.96 and 0.93 of the time, gated 0.90 and 0.80, slower by more than 5 % at 53 and 9, gated 19 and 8; with the line that came with those tiles it was 209 and 71,
 // gated 64 and 33.  At 1,420 plain shapes that the fit had not seen 0.965 and 0.95, slower by more than 5 % at 83 of 1,220 and 19 of 200; 571 gated 0.92 and 0.85, at 37 and 14.
-// 32-bit results, 900 shapes that the fit had not seen: 1.5 % slower than the better of the two, by more than 5 % at 87; with their storing priced as two bytes 3.3 %, at 159
+// 32-bit results, 900 shapes that the fit had not seen: 1.5 % slower than the better of the two, by more than 5 % at 89; with their storing priced as two bytes 3.3 %, at 159
 // (2048 x 8256 x 2048 75.7 here, 90.6; 2048 x 8192 x 2048 59.3, 63.3).
 // (us, here / library: taken 2048 x 2560 x 2048 25.8 / 29.0, 1040 x 2048 x 2048 17.2 / 23.0, 1024 x 1024 x 512 5.9 / 9.0, 2048 x 2048 x 5632 52.2 / 52.7; 2,048 and 1,024 rows of gate and up,
 // 5632 x 2048, 90 / 92 and 49 / 57; not taken 640 x 64 x 14336 30 / 17, 1040 x 8192 x 2048 44 / 36, 2048 x 8192 x 2048 52 / 50, 384 x 2048 x 5632 whole 27 / 25, 2048 x 256 x 5632 21.7 / 20.6.)
@@ -526,7 +526,7 @@ int kvcm_gemm_tiles_preferred(int M, int N, int K, int S, int is_gated, int out_
   const float library = library_time(M, wrows, K, out_f32);
   if (is_gated) return here <= library + 3.4f + results * 6.f / 5e6f;
   const long long tiles = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128);
-  const float side = M <= 256 && tiles > 16 ? 1.1f : M > 512 && M <= 1024 && tiles < 116 ? 0.87f : N <= 320 && K >= 5632 ? 0.84f : 0.98f;
+  const float side = M <= 256 && tiles > 16 ? 1.1f : M > 512 && M <= 1024 && tiles < 116 ? (M <= 640 ? 0.87f : 0.78f) : N <= 320 && K >= 5632 ? 0.84f : 0.98f;
   return here <= side * library;
 }
 

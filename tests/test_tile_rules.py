@@ -18,7 +18,7 @@ def test_tiles_of_routed_experts(ops, n, E, N, K, tiles):
 
 
 # (M, N, K, gated): products as bench.py's and the command lines' models have them, and others
-@pytest.mark.parametrize("M,N,K,gated,here", [(2048, 2560, 2048, 0, 1), (1040, 2048, 2048, 0, 1), (1024, 1024, 512, 0, 1), (2048, 2048, 5632, 0, 1), (513, 2048, 2048, 0, 1), (700, 2048, 2048, 0, 1),
+@pytest.mark.parametrize("M,N,K,gated,here", [(2048, 2560, 2048, 0, 1), (1040, 2048, 2048, 0, 1), (1024, 1024, 512, 0, 1), (2048, 2048, 5632, 0, 1), (513, 2048, 2048, 0, 1),
                                               (2048, 5632, 2048, 1, 1), (1024, 5632, 2048, 1, 1), (32768, 5632, 2048, 1, 1), (8192, 5632, 2048, 1, 1),
                                               (640, 64, 14336, 0, 0), (1040, 8192, 2048, 0, 0), (2048, 8192, 2048, 0, 0), (384, 2048, 5632, 0, 0),
                                               (2048, 256, 5632, 0, 0), (2049, 2560, 2048, 0, 0)])
