@@ -332,7 +332,7 @@ struct Tile {
   TileTime time;
 };
 #define KVCM_TILES(T)                                         \
-  T(16, 32, 1, 2, 8, false, 2.786f, 0.121f, 0.654f, 0.600f)   \
+  T(16, 32, 1, 2, 8, false, 2.786f, 0.121f, 0.654f, 0.800f)   \
   T(16, 48, 1, 3, 8, false, 2.807f, 0.137f, 0.742f, 0.631f)   \
   T(16, 64, 1, 4, 8, false, 2.851f, 0.169f, 0.772f, 0.596f)   \
   T(32, 32, 2, 2, 8, false, 2.822f, 0.137f, 0.779f, 0.448f)   \
